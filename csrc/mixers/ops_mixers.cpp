@@ -47,6 +47,13 @@ int gated_linear_scan(const float*, const float*, const float*, const void*, int
                       const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int,
                       int, int, int, float*, int, int, const float*, const float*, hipStream_t);
 int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
+int64_t chunk_scan_scratch_floats(int, int, int, int, int, int);
+int chunk_scan_gates(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*,
+                     const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int,
+                     int, int, int, int, float*, hipStream_t);
+int chunk_scan_ssm(const void*, bool, int64_t, const void*, int64_t, const float*, const float*, const float*, float*,
+                   const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, int, int, int, int, float*,
+                   hipStream_t);
 int ssm_scan(const void*, bool, int64_t, const void*, int64_t, const float*, const float*, const float*, float*,
              const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, int, hipStream_t);
 void gated_group_norm(const float*, const void*, bool, int64_t, const float*, int, float, void*, int, int, int, bool,
@@ -276,6 +283,35 @@ PYBIND11_MODULE(_mixers, m) {
   });
   m.def("gated_linear_scan_scratch_floats",
         [](int T, int ns, int H, int dk, int dv) { return xgm::gated_linear_scan_scratch_floats(T, ns, H, dk, dv); });
+  m.def("chunk_scan_scratch_floats", [](int T, int ns, int H, int dk, int dv, int seg) {
+    if (seg < 1) throw std::invalid_argument("chunk_scan_scratch_floats: seg must be positive");
+    return xgm::chunk_scan_scratch_floats(T, ns, H, dk, dv, seg);
+  });
+  m.def("chunk_scan_gates", [](uintptr_t q, uintptr_t f, uintptr_t k, uintptr_t raw, int64_t ld_raw, int off_q, int off_f,
+                               uintptr_t f_bias, uintptr_t lower, uintptr_t v, bool v_f32, int64_t ld_v, uintptr_t state,
+                               uintptr_t qsl, uintptr_t sl, uintptr_t slots, uintptr_t o, int ns, int max_q, int T, int H,
+                               int dk, int dv, int seg, uintptr_t scratch, uintptr_t st) {
+    if (H < 1 || dv < 1 || dk < 1 || ld_v < (int64_t)H * dv ||
+        (raw && (off_q < 0 || off_f < 0 || ld_raw < off_q + (int64_t)H * dk || ld_raw < off_f + (int64_t)H * dk)))
+      throw std::invalid_argument("chunk_scan_gates: inconsistent sizes");
+    int rc = xgm::chunk_scan_gates(P<const float>(q), P<const float>(f), P<const float>(k), P<const void>(raw), ld_raw, off_q,
+                                   off_f, P<const float>(f_bias), P<const float>(lower), P<const void>(v), v_f32, ld_v,
+                                   P<float>(state), P<const int32_t>(qsl), P<const int32_t>(sl), P<const int32_t>(slots),
+                                   P<float>(o), ns, max_q, T, H, dk, dv, seg, P<float>(scratch), S(st));
+    check(rc, "chunk_scan_gates");
+  });
+  m.def("chunk_scan_ssm", [](uintptr_t xbc, bool f32, int64_t ld_x, uintptr_t dt, int64_t ld_dt, uintptr_t dt_bias,
+                             uintptr_t A_log, uintptr_t D, uintptr_t state, uintptr_t qsl, uintptr_t sl, uintptr_t slots,
+                             uintptr_t y, int ns, int max_q, int T, int H, int G, int N, int Pd, int seg, uintptr_t scratch,
+                             uintptr_t st) {
+    if (H < 1 || G < 1 || ld_x < (int64_t)H * Pd + 2 * (int64_t)G * N || ld_dt < H)
+      throw std::invalid_argument("chunk_scan_ssm: inconsistent sizes");
+    int rc = xgm::chunk_scan_ssm(P<const void>(xbc), f32, ld_x, P<const void>(dt), ld_dt, P<const float>(dt_bias),
+                                 P<const float>(A_log), P<const float>(D), P<float>(state), P<const int32_t>(qsl),
+                                 P<const int32_t>(sl), P<const int32_t>(slots), P<float>(y), ns, max_q, T, H, G, N, Pd, seg,
+                                 P<float>(scratch), S(st));
+    check(rc, "chunk_scan_ssm");
+  });
   m.def("ssm_scan", [](uintptr_t xbc, bool f32, int64_t ld_x, uintptr_t dt, int64_t ld_dt, uintptr_t dt_bias,
                        uintptr_t A_log, uintptr_t D, uintptr_t state, uintptr_t qsl, uintptr_t sl, uintptr_t slots,
                        uintptr_t y, int ns, int H, int G, int N, int Pd, uintptr_t st) {

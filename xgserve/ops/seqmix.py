@@ -695,6 +695,15 @@ def ssm_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_l
     if native_device(xbc):
         assert xbc.stride(1) == 1 and dt_raw.stride(1) == 1 and dt_raw.dtype == xbc.dtype
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, N, P)
+        es = xbc.element_size()
+        if _chunk_scan_ok(sm, N) and N % 8 == 0 and xbc.data_ptr() % 16 == 0 \
+                and xbc.stride(0) * es % 16 == 0 and H * P * es % 16 == 0:
+            seg, scratch = _chunk_scan_segments(sm, T, H, N, P, 64, xbc.device)
+            mixers().chunk_scan_ssm(xbc.data_ptr(), is_f32(xbc), xbc.stride(0), dt_raw.data_ptr(), dt_raw.stride(0),
+                                    dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(),
+                                    _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(),
+                                    y.data_ptr(), sm.num_seqs, sm.max_q, T, H, G, N, P, seg, _p(scratch), stream_ptr())
+            return y
         mixers().ssm_scan(xbc.data_ptr(), is_f32(xbc), xbc.stride(0), dt_raw.data_ptr(), dt_raw.stride(0),
                           dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(), _i32(sm.qsl).data_ptr(),
                           _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), y.data_ptr(), sm.num_seqs, H, G, N, P,
@@ -1108,6 +1117,45 @@ SCAN_TWO_PASS_MIN = 512   # portions longer than this may be scanned as chunks o
 SCAN_FILL_WGS = 192       # ... when their one-launch form would start at most this many workgroups (256 compute units)
 
 
+# Prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/chunk_scan.hip). From one whole chunk on: 12
+# sequences of 16 tokens take 12 us against 18 token by token, 4 of 8 the same 11 (16 heads of 64 x 128).
+CHUNK_SCAN = True
+CHUNK_SCAN_MIN = 16
+CHUNK_SCAN_MAX_DK = 128    # state rows a wave holds
+CHUNK_SCAN_MAX_SEQS = 2047   # (sequences x segments are one grid dimension)
+# Long portions are cut into segments until about two workgroups per compute unit run, of at least 64 tokens (128 for the
+# large state, whose sums cost more to write and fold): 4001 tokens of 16 heads of 64 x 128 take 88 us in 32 segments and 731
+# in one, 2521 tokens of 64 heads of 128 x 64 in four sequences 178 and 254; past two per compute unit the second run over the
+# tokens costs more than it spreads (4 x 1024 tokens of 128 heads of 128 x 64: 247 us whole, 368 in two).
+CHUNK_SCAN_FILL_WGS = 512
+CHUNK_SCAN_MIN_SEG, CHUNK_SCAN_MAX_SEGS = 64, 32
+
+
+def _chunk_scan_ok(sm: SeqMeta, dk: int) -> bool:
+    return CHUNK_SCAN and sm.max_q >= CHUNK_SCAN_MIN and dk <= CHUNK_SCAN_MAX_DK and sm.num_seqs <= CHUNK_SCAN_MAX_SEQS
+
+
+def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
+    """(tokens per segment of a step's portions, scratch of the two launches or None: one segment, one launch)."""
+    whole = (sm.max_q + 15) // 16 * 16
+    wgs = max(1, T // sm.max_q) * H * ((dv + cols - 1) // cols)
+    n = min(CHUNK_SCAN_MAX_SEGS, CHUNK_SCAN_FILL_WGS // wgs, whole // (CHUNK_SCAN_MIN_SEG * (2 if dk > 64 else 1)))
+    if n <= 1:
+        return whole, None
+    seg = ((whole + n - 1) // n + 15) // 16 * 16
+    return seg, torch.empty(mixers().chunk_scan_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32,
+                            device=device)
+
+
+def _chunk_scan(q, f, k, raw, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv):
+    seg, scratch = _chunk_scan_segments(sm, v.shape[0], H, dk, dv, 128 if dv > 64 else 64, v.device)
+    mixers().chunk_scan_gates(_p(q), _p(f), _p(k), _p(raw), raw.stride(0) if raw is not None else 0, off_q, off_f, _p(f_bias),
+                              _p(lower), v.data_ptr(), is_f32(v), v.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(),
+                              _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), o.data_ptr(), sm.num_seqs, sm.max_q,
+                              v.shape[0], H, dk, dv, seg, _p(scratch), stream_ptr())
+    return o
+
+
 def _scan_scratch(T: int, sm: SeqMeta, H: int, dk: int, dv: int, device) -> Optional[torch.Tensor]:
     """Chunk summaries of a long portion (gated_linear_scan in two launches); None for short steps and for steps whose
     long sequences fill the chip by themselves (the chunked form runs the recurrence twice: measured 1.7x - 3.7x faster
@@ -1155,6 +1203,8 @@ def gated_linear_scan(q: torch.Tensor, f: Optional[torch.Tensor], k: Optional[to
         assert bonus is None or (bonus.dtype == torch.float32 and bonus.is_contiguous() and bonus.numel() == H * dk)
         assert k is None or (k.dtype == torch.float32 and k.is_contiguous())
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, dk, dv)
+        if _chunk_scan_ok(sm, dk) and decay is None and bonus is None:
+            return _chunk_scan(q, f, k, None, 0, 0, None, None, v, state, o, sm, H, dk, dv)
         scratch = _scan_scratch(T, sm, H, dk, dv, q.device)
         mixers().gated_linear_scan(q.data_ptr(), _p(f), _p(k), 0, 0, 0, 0, 0, 0, v.data_ptr(), is_f32(v),
                                    v.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
@@ -1194,6 +1244,8 @@ def lower_bound_recurrence(proj: torch.Tensor, off_q: int, off_f: int, off_v: in
     assert proj.stride(1) == 1 and lower.dtype == torch.float32 and lower.numel() == n
     assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, dk, dv)
     o = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device)
+    if _chunk_scan_ok(sm, dk):
+        return _chunk_scan(None, None, None, proj, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv)
     scratch = _scan_scratch(proj.shape[0], sm, H, dk, dv, proj.device)
     mixers().gated_linear_scan(0, 0, 0, proj.data_ptr(), proj.stride(0), off_q, off_f, _p(f_bias), lower.data_ptr(),
                                v.data_ptr(), is_f32(proj), proj.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(),
