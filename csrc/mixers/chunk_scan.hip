@@ -31,17 +31,16 @@
 // (sequence s, segment z): q0_s / seg + s + z, distinct for all segments of a step.
 #include <type_traits>
 
-#include "attention_common.h"
+#include "mfma_f32.h"
 
 namespace xgm {
 
-using xgk::f32x4_t;
 using xgk::ld16;
 using xgk::unpack8;
 
 constexpr int kCsRaw = 0, kCsPlain = 1, kCsSsm = 2;
 constexpr int kCsTok = 16;
-constexpr float kCsMaxLog2 = 60.f, kCsMaxIn = 268435456.f;   // 2^28
+constexpr float kCsMaxLog2 = 60.f;
 
 struct ChunkScanArgs {
   const float *q, *f, *k;      // plain: fp32 [T][H dk] (k may be null)
@@ -61,23 +60,6 @@ struct ChunkScanArgs {
   int H, dk, dv, pass, nc, seg;
   float *chA, *chB, *s_in;
 };
-
-__device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-#else
-  return c;
-#endif
-}
-
-__device__ __forceinline__ bool out_of_range(float x) { return !(fabsf(x) < kCsMaxIn); }
-
-// 1 / (1 + e^-x) from the exponential and reciprocal instructions; the product x log2 e in two terms keeps them to 2 ulp
-__device__ __forceinline__ float sigmoid2(float x) {
-  x = x > 100.f ? -100.f : x < -100.f ? 100.f : -x;
-  const float t = x * kLog2e, lo = fmaf(x, kLog2e, -t) + x * 1.9259629e-8f, e = exp2_fast(t);
-  return rcp_fast(1.f + fmaf(e, lo * 0.69314718f, e));
-}
 
 __device__ __forceinline__ float log2_fast(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -1,0 +1,384 @@
+// Generalized delta rule over prompt portions, in chunks of 16 tokens on the fp32 matrix cores (bf16 or fp32 rows, fp32 state):
+//
+//   S_t = diag(w_t) S_(t-1) - b_t (u_t^T S_(t-1)) + k_t v_t^T,   o_t = S_t^T r_t,      b = a u, u = k / |k|, w = e^(-c sigmoid)
+//
+// Token by token this is a chain of two reductions per token (0.45 us). Let L be the running sum of log2 w from the chunk's
+// start and u' = u 2^(L_(t-1)), b' = b 2^(-L_t), k' = k 2^(-L_t), r' = r 2^(L_t) (L loses at most 0.88 a token: 14 bits over a
+// chunk). With M = u' b'^T and N = u' k'^T strictly below the diagonal, P = r' k'^T and Q = r' b'^T up to it and
+// T = (1 + M)^-1, what token t takes out of the state is y = T (u' S + N v), and
+//   y = U S + V,           U = T u', V = T N v,
+//   o = R S + O,           R = r' - Q U, O = P v - Q V,
+//   S <- 2^(L_15) (S + k'^T v - b'^T y).
+// Only the right factors meet the state, so a first launch forms U, V, R, O, k', b' of all chunks at once (one wave per chunk
+// and head; T by forward substitution) and the chain that is left is three matrix products per 16 tokens. All of it is fp32
+// arithmetic.
+//
+// The second launch has one wave per 16 state columns of a (sequence, head). The first writes every operand in the order of the
+// matrix instructions' lanes; the waves bring it in by LDS DMA, three chunks ahead (in registers, two chunks ahead, the compiler
+// parks operands in accumulator registers, which waits for every load: 2.1 us a chunk). A chunk with an input out of range
+// (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
+//
+// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1030 -> 336 us (126 + 210), one sequence of 2048
+// 860 -> 239, 64 tokens 32 -> 20. The first launch is at the memory's rate (it writes 24.6 KB per chunk and head); the second
+// takes 1.6 us a chunk, 0.9 of them its 64 matrix instructions a wave, the rest the way from one to the next: LDS reads behind
+// the barrier, and y, which has to be complete before it goes back in.
+#include "glds.h"
+#include "mfma_f32.h"
+
+namespace xgm {
+
+constexpr int kDcTok = 16;
+constexpr float kDeltaDecayLog2 = -0.6065306597126334f * kLog2e;   // log2 w = this * sigmoid
+
+// floats per (chunk, head): [U | R | k' | -b' | V | O] in lane order, then 2^E per channel, then the flag
+constexpr int dc_stride(int D) { return 6 * kDcTok * D + 256; }
+
+template <typename T, int D>
+__global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __restrict__ proj, int64_t ld, int off_r, int off_k,
+                                                                 int off_v, int off_a, const T* __restrict__ wl,
+                                                                 int64_t ld_wl, const float* __restrict__ a_bias,
+                                                                 const float* __restrict__ w0, const int32_t* __restrict__ qsl,
+                                                                 const int32_t* __restrict__ slots, float* __restrict__ prep,
+                                                                 int H) {
+  constexpr int C = kDcTok, MT = D / 16, QE = D + 4, TPL = C * D / 64;   // (token, channel) pairs per lane
+  constexpr int TG = 64 / D, TT = C / TG;                                // token groups, tokens per lane
+  static_assert(D == 64 || D == 32, "a lane owns one channel");
+  __shared__ __attribute__((aligned(16))) float us[C * QE], rs[C * QE], ks[C * QE], bs[C * QE], ts[C * 20];
+  const int h = blockIdx.x, c = blockIdx.y, s = blockIdx.z;
+  const int q0 = qsl[s], qn = qsl[s + 1] - q0, n = min(C, qn - C * c);
+  if (slots[s] < 0 || n <= 0) return;
+  const int lane = threadIdx.x, g4 = lane >> 4, l16 = lane & 15, d = lane % D, tg = lane / D;
+  float* dst = prep + ((int64_t)(q0 / C + s + c) * H + h) * dc_stride(D);
+  const T* row = proj + (int64_t)(q0 + C * c) * ld + h * D;
+  const T* wrow = wl + (int64_t)(q0 + C * c) * ld_wl + h * D;
+
+  // ---- this lane's channel, tokens tg TT .. (rows past the end repeat the last and are masked)
+  T xr[TT], xk[TT], xa[TT], xw[TT], xv[MT][4];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const uint32_t t = min(TT * tg + i, n - 1), at = t * (uint32_t)ld + d;
+    xk[i] = row[at + off_k], xw[i] = wrow[t * (uint32_t)ld_wl + d];
+    xa[i] = row[at + off_a], xr[i] = row[at + off_r];
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xv[m][t] = row[(uint32_t)min(4 * g4 + t, n - 1) * (uint32_t)ld + off_v + 16 * m + l16];
+  const float ab = a_bias[h * D + d], wb = w0[h * D + d];
+  bool bad = false;
+  float k[TT];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    k[i] = TT * tg + i < n ? ldf(&xk[i]) : 0.f;
+    bad |= out_of_range(k[i]);
+    ks[(TT * tg + i) * QE + d] = k[i];
+  }
+  __syncthreads();
+  float ksq = 0.f;   // |k|^2 of token l16
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    float x[4];
+    ld4(ks + l16 * QE + 16 * m + 4 * g4, x);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ksq = fmaf(x[r], x[r], ksq);
+  }
+  ksq += __shfl_xor(ksq, 16, 64);
+  ksq += __shfl_xor(ksq, 32, 64);
+  const float inv = 1.f / sqrtf(ksq + 1e-6f);
+  float v[MT][4];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      v[m][t] = 4 * g4 + t < n ? ldf(&xv[m][t]) : 0.f;
+      bad |= out_of_range(v[m][t]);
+    }
+  float lw[TT], u[TT], a[TT], r_[TT], run = 0.f;
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const bool on = TT * tg + i < n;
+    u[i] = k[i] * __shfl(inv, TT * tg + i, 64);
+    lw[i] = on ? kDeltaDecayLog2 * sigmoid2(ldf(&xw[i]) + wb) : 0.f;
+    a[i] = on ? sigmoid2(ldf(&xa[i]) + ab) : 0.f;
+    r_[i] = on ? ldf(&xr[i]) : 0.f;
+    bad |= out_of_range(r_[i]) || out_of_range(a[i]) || out_of_range(lw[i]);
+    run += lw[i];
+  }
+  float L = 0.f;   // log decay ahead of this lane's tokens
+  if (TG == 2) {
+    const float up = __shfl_xor(run, D % 64, 64);
+    L = tg ? up : 0.f;
+  }
+  const bool slow = __any(bad);
+  if (lane == 0) dst[6 * C * D + D] = slow ? 1.f : 0.f;
+  if (slow) {   // [w | b | u | k | r] as rows
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      float* to = dst + (TT * tg + i) * D + d;
+      to[0] = exp2f(lw[i]), to[C * D] = a[i] * u[i], to[2 * C * D] = u[i], to[3 * C * D] = k[i], to[4 * C * D] = r_[i];
+    }
+    return;
+  }
+  __syncthreads();   // (ks is rewritten)
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const int at = (TT * tg + i) * QE + d;
+    us[at] = u[i] * exp2_fast(L);
+    L += lw[i];
+    const float e = exp2_fast(L), f = exp2_fast(-L);
+    rs[at] = r_[i] * e, ks[at] = k[i] * f, bs[at] = a[i] * u[i] * f;
+  }
+  if (tg == TG - 1) dst[6 * C * D + d] = exp2_fast(L);
+  __syncthreads();
+
+  // ---- the four 16 x 16 products, transposed: lane holds [token l16][token 4 g4 + r], the A operand of what follows
+  f32x4_t M = {0.f, 0.f, 0.f, 0.f}, N = M, P = M, Q = M;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    float xu[4], xrr[4], xkk[4], xb[4];
+    const int at = l16 * QE + 16 * m + 4 * g4;
+    ld4(us + at, xu), ld4(rs + at, xrr), ld4(ks + at, xkk), ld4(bs + at, xb);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      M = mfma_f32(xb[r], xu[r], M);
+      N = mfma_f32(xkk[r], xu[r], N);
+      P = mfma_f32(xkk[r], xrr[r], P);
+      Q = mfma_f32(xb[r], xrr[r], Q);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int j = 4 * g4 + r;
+    M[r] = j < l16 ? M[r] : 0.f, N[r] = j < l16 ? N[r] : 0.f;
+    P[r] = j <= l16 ? P[r] : 0.f, Q[r] = j <= l16 ? -Q[r] : 0.f;   // (Q enters with its sign)
+  }
+  *reinterpret_cast<float4*>(ts + l16 * 20 + 4 * g4) = make_float4(M[0], M[1], M[2], M[3]);
+  __syncthreads();
+  // ---- T = (1 + M)^-1: lane l16 solves for column l16, x_i = delta - sum_(j < i) M_ij x_j
+  float x[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    float acc = i == l16 ? 1.f : 0.f;
+#pragma unroll
+    for (int j4 = 0; j4 < (i + 3) / 4; ++j4) {
+      float mm[4];
+      ld4(ts + i * 20 + 4 * j4, mm);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * j4 + r < i) acc = fmaf(-mm[r], x[4 * j4 + r], acc);
+    }
+    x[i] = acc;
+  }
+  __syncthreads();
+  if (g4 == 0) {
+#pragma unroll
+    for (int i = 0; i < C; ++i) ts[i * 20 + l16] = x[i];
+  }
+  __syncthreads();
+  float Tf[4];
+  ld4(ts + l16 * 20 + 4 * g4, Tf);   // T[l16][4 g4 + r]
+
+  auto put = [&](int which, int m, f32x4_t y) {
+    *reinterpret_cast<float4*>(dst + which * C * D + 256 * m + 4 * lane) = make_float4(y[0], y[1], y[2], y[3]);
+  };
+  // ---- U (transposed product: token l16, channels 16 m + 4 g4 + r); k' and -b' as the A operands of the state's update
+  f32x4_t U[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    U[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t kk, bb;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int at = (4 * g4 + t) * QE + 16 * m + l16;
+      U[m] = mfma_f32(us[at], Tf[t], U[m]);
+      kk[t] = ks[at], bb[t] = -bs[at];
+    }
+    put(0, m, U[m]), put(2, m, kk), put(3, m, bb);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    *reinterpret_cast<float4*>(us + l16 * QE + 16 * m + 4 * g4) = make_float4(U[m][0], U[m][1], U[m][2], U[m][3]);
+  __syncthreads();
+  // ---- R, then V and O column tile by column tile
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    float r0[4];
+    ld4(rs + l16 * QE + 16 * m + 4 * g4, r0);
+    f32x4_t R = {r0[0], r0[1], r0[2], r0[3]};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) R = mfma_f32(us[(4 * g4 + t) * QE + 16 * m + l16], Q[t], R);
+    put(1, m, R);
+    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, V = y, O = y;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y = mfma_f32(N[t], v[m][t], y), O = mfma_f32(P[t], v[m][t], O);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) V = mfma_f32(Tf[t], y[t], V);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) O = mfma_f32(Q[t], V[t], O);
+    put(4, m, V), put(5, m, O);
+  }
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float* __restrict__ prep, const T* __restrict__ proj,
+                                                                    int64_t ld, int off_v, float* __restrict__ state,
+                                                                    const int32_t* __restrict__ qsl,
+                                                                    const int32_t* __restrict__ seq_lens,
+                                                                    const int32_t* __restrict__ slots, float* __restrict__ o,
+                                                                    int H) {
+  constexpr int C = kDcTok, MT = D / 16, NW = MT, RING = 4;
+  constexpr int FRAG = 6 * C * D * 4, SLOT = FRAG + 1024 + C * D * sizeof(T);   // bytes: [U .. O | 2^E, flag | v rows]
+  constexpr int VL = D * sizeof(T) / 16, VR = C / NW;                            // lanes per v row, v rows per wave
+  constexpr int DMA = 6 * C * D * 4 / 1024 / NW + 2;                             // loads per wave and chunk
+  __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT];
+  const int h = blockIdx.x, s = blockIdx.y;
+  const int q0 = qsl[s], qn = qsl[s + 1] - q0, slot = slots[s];
+  if (slot < 0 || qn <= 0) return;
+  const int ctx = seq_lens[s] - qn;
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = 16 * w + l16;
+  float* Sg = state + ((int64_t)slot * H + h) * D * D + col;
+  f32x4_t S[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[m][r] = ctx > 0 ? Sg[(16 * m + 4 * g4 + r) * D] : 0.f;
+  const int nch = (qn + C - 1) / C;
+  const float* base = prep + ((int64_t)(q0 / C + s) * H + h) * dc_stride(D);
+  const int64_t step = (int64_t)H * dc_stride(D);
+  const T* vb = proj + (int64_t)q0 * ld + off_v + h * D;
+  const int vrow = VR * w + lane / VL;   // (lanes past the wave's rows load nothing)
+
+  auto issue = [&](int c) {   // every wave issues DMA loads, past the last chunk too (its waits count them)
+    char* dst = lds + (c % RING) * SLOT;
+    const char* src = reinterpret_cast<const char*>(base + min(c, nch - 1) * step) + 16 * lane;
+#pragma unroll
+    for (int i = 0; i < DMA - 2; ++i) xgk::glds16(src + 1024 * (NW * i + w), dst + 1024 * (NW * i + w));
+    xgk::glds16(src + FRAG, dst + FRAG);   // (the same bytes from every wave)
+    if (lane < VR * VL)
+      xgk::glds16(vb + (int64_t)min(C * min(c, nch - 1) + vrow, qn - 1) * ld + (lane % VL) * (16 / sizeof(T)),
+                  dst + FRAG + 1024 + VR * w * D * sizeof(T));
+  };
+  for (int c = 0; c < RING - 1; ++c) issue(c);
+  for (int c = 0; c < nch; ++c) {
+    // this chunk's loads have landed (those of the chunks after it are in flight), in every wave; the slot of the chunk
+    // before is free
+    xgk::wait_vmcnt<(RING - 2) * DMA>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    xgk::raw_barrier();
+    issue(c + RING - 1);
+    const char* at = lds + (c % RING) * SLOT;
+    const float* p = reinterpret_cast<const float*>(at);
+    const float4* p4 = reinterpret_cast<const float4*>(at) + lane;
+    const float* pe = reinterpret_cast<const float*>(at + FRAG);
+    const T* pv = reinterpret_cast<const T*>(at + FRAG + 1024) + col;
+    const int n = min(C, qn - C * c);
+    float* ob = o + ((int64_t)(q0 + C * c) * H + h) * D + col;
+    float v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = ldf(pv + (4 * g4 + t) * D);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = 4 * g4 + t < n ? v[t] : 0.f;
+    if (__builtin_amdgcn_readfirstlane(pe[D] != 0.f)) {
+      for (int t = 0; t < n; ++t) {
+        const float vv = ldf(pv + t * D);
+        float uS = 0.f, sum = 0.f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float u[4];
+          ld4(p + 2 * C * D + t * D + 16 * m + 4 * g4, u);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) uS = fmaf(u[r], S[m][r], uS);
+        }
+        uS += __shfl_xor(uS, 16, 64);
+        uS += __shfl_xor(uS, 32, 64);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float wr[4], b[4], k[4], rr[4];
+          const float* x = p + t * D + 16 * m + 4 * g4;
+          ld4(x, wr), ld4(x + C * D, b), ld4(x + 3 * C * D, k), ld4(x + 4 * C * D, rr);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            S[m][r] = wr[r] * S[m][r] - b[r] * uS + k[r] * vv;
+            sum = fmaf(S[m][r], rr[r], sum);
+          }
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        if (g4 == 0) ob[(int64_t)t * H * D] = sum;
+      }
+      continue;
+    }
+    const float4 v0 = p4[64 * (4 * MT + w)], o0 = p4[64 * (5 * MT + w)];
+    f32x4_t y = {v0.x, v0.y, v0.z, v0.w}, out = {o0.x, o0.y, o0.z, o0.w};
+    float4 k[MT], b[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const float4 u = p4[64 * m], r = p4[64 * (MT + m)];
+      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)];
+      y = mfma_f32(u.x, S[m][0], y), out = mfma_f32(r.x, S[m][0], out);
+      y = mfma_f32(u.y, S[m][1], y), out = mfma_f32(r.y, S[m][1], out);
+      y = mfma_f32(u.z, S[m][2], y), out = mfma_f32(r.z, S[m][2], out);
+      y = mfma_f32(u.w, S[m][3], y), out = mfma_f32(r.w, S[m][3], out);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], S[m]);   // (independent of y: behind its last products)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].y, v[1], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].z, v[2], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].w, v[3], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].x, y[0], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].y, y[1], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].z, y[2], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].w, y[3], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      float e[4];
+      ld4(pe + 16 * m + 4 * g4, e);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[m][r] *= e[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * g4 + r < n) ob[(int64_t)(4 * g4 + r) * H * D] = out[r];
+  }
+  xgk::wait_vmcnt<0>();   // (no load may land after the workgroup's LDS is given on)
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Sg[(16 * m + 4 * g4 + r) * D] = S[m][r];
+}
+
+// ================================================================== host launchers
+int64_t delta_chunk_scratch_floats(int T_, int ns, int H, int D) {
+  return (int64_t)(T_ / kDcTok + ns + 1) * H * dc_stride(D);
+}
+
+int delta_chunk(const void* proj, bool f32, int64_t ld, int off_r, int off_k, int off_v, int off_a, const void* wl, int64_t ld_wl,
+                const float* a_bias, const float* w0, float* state, const int32_t* qsl, const int32_t* seq_lens,
+                const int32_t* slots, float* o, int ns, int max_q, int H, int D, float* scratch, hipStream_t st) {
+  if (ns <= 0 || max_q <= 0) return 0;
+  const int nc = (max_q + kDcTok - 1) / kDcTok;
+  const int64_t al = f32 ? 4 : 8;   // (v rows come in 16 bytes at a time)
+  if ((uintptr_t)proj % 16 || ld % al || off_v % al || (uintptr_t)scratch % 16) return -1;
+  if ((D != 32 && D != 64) || H < 1 || !scratch || nc > 65535 || ns > 65535) return -1;
+#define XGM_DC(D)                                                                                                          \
+  XGM_DISPATCH_T(f32, delta_chunk_prep_kernel<T, D><<<dim3(H, nc, ns), 64, 0, st>>>((const T*)proj, ld, off_r, off_k, off_v, \
+                                                                                    off_a, (const T*)wl, ld_wl, a_bias, w0, \
+                                                                                    qsl, slots, scratch, H);                \
+                 delta_chunk_scan_kernel<T, D><<<dim3(H, ns), 4 * D, 0, st>>>(scratch, (const T*)proj, ld, off_v, state, qsl, \
+                                                                              seq_lens, slots, o, H);)                       \
+  return 0;
+  if (D == 32) { XGM_DC(32) }
+  XGM_DC(64)
+#undef XGM_DC
+}
+
+}  // namespace xgm

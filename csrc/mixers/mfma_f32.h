@@ -1,0 +1,34 @@
+// Pieces shared by the chunked fp32 recurrences (chunk_scan.hip, delta_chunk.hip).
+//
+// v_mfma_f32_16x16x4_f32: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 (l / 16) + r][l % 16], r = 0..3. The
+// contraction may run in any order as long as both operands agree: with step r of lane group g standing for index 4 g + r, a D
+// tile is the B operand of the next product as it lies, and D of a transposed product is its A operand.
+#pragma once
+
+#include "attention_common.h"
+
+namespace xgm {
+
+using xgk::f32x4_t;
+
+__device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+#else
+  return c;
+#endif
+}
+
+// inputs past 2^28, infinities and NaN: a chunk that holds one runs token by token (a masked 0 times infinity would reach
+// the tokens before it)
+constexpr float kChunkMaxIn = 268435456.f;
+__device__ __forceinline__ bool out_of_range(float x) { return !(fabsf(x) < kChunkMaxIn); }
+
+// 1 / (1 + e^-x) from the exponential and reciprocal instructions; the product x log2 e in two terms keeps them to 2 ulp
+__device__ __forceinline__ float sigmoid2(float x) {
+  x = x > 100.f ? -100.f : x < -100.f ? 100.f : -x;
+  const float t = x * kLog2e, lo = fmaf(x, kLog2e, -t) + x * 1.9259629e-8f, e = exp2_fast(t);
+  return rcp_fast(1.f + fmaf(e, lo * 0.69314718f, e));
+}
+
+}  // namespace xgm

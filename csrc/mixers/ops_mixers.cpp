@@ -47,6 +47,9 @@ int gated_linear_scan(const float*, const float*, const float*, const void*, int
                       const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int,
                       int, int, int, float*, int, int, const float*, const float*, hipStream_t);
 int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
+int64_t delta_chunk_scratch_floats(int, int, int, int);
+int delta_chunk(const void*, bool, int64_t, int, int, int, int, const void*, int64_t, const float*, const float*, float*,
+                const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, float*, hipStream_t);
 int64_t chunk_scan_scratch_floats(int, int, int, int, int, int);
 int chunk_scan_gates(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*,
                      const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int,
@@ -283,6 +286,21 @@ PYBIND11_MODULE(_mixers, m) {
   });
   m.def("gated_linear_scan_scratch_floats",
         [](int T, int ns, int H, int dk, int dv) { return xgm::gated_linear_scan_scratch_floats(T, ns, H, dk, dv); });
+  m.def("delta_chunk_scratch_floats",
+        [](int T, int ns, int H, int D) { return xgm::delta_chunk_scratch_floats(T, ns, H, D); });
+  m.def("delta_chunk", [](uintptr_t proj, bool f32, int64_t ld, int off_r, int off_k, int off_v, int off_a, uintptr_t wl,
+                          int64_t ld_wl, uintptr_t a_bias, uintptr_t w0, uintptr_t state, uintptr_t qsl, uintptr_t sl,
+                          uintptr_t slots, uintptr_t o, int ns, int max_q, int H, int D, uintptr_t scratch, uintptr_t st) {
+    const int64_t n = (int64_t)H * D;
+    if (H < 1 || D < 1 || off_r < 0 || off_k < 0 || off_v < 0 || off_a < 0 || ld < off_r + n || ld < off_k + n ||
+        ld < off_v + n || ld < off_a + n || ld_wl < n)
+      throw std::invalid_argument("delta_chunk: inconsistent sizes");
+    int rc = xgm::delta_chunk(P<const void>(proj), f32, ld, off_r, off_k, off_v, off_a, P<const void>(wl), ld_wl,
+                              P<const float>(a_bias), P<const float>(w0), P<float>(state), P<const int32_t>(qsl),
+                              P<const int32_t>(sl), P<const int32_t>(slots), P<float>(o), ns, max_q, H, D, P<float>(scratch),
+                              S(st));
+    check(rc, "delta_chunk");
+  });
   m.def("chunk_scan_scratch_floats", [](int T, int ns, int H, int dk, int dv, int seg) {
     if (seg < 1) throw std::invalid_argument("chunk_scan_scratch_floats: seg must be positive");
     return xgm::chunk_scan_scratch_floats(T, ns, H, dk, dv, seg);

@@ -319,6 +319,11 @@ DECAY_SCALE = math.exp(-0.5)
 # XGS_TUNE delta_two_pass=0: the one-pass scan kernel (any head size; A/B and tests)
 DELTA_TWO_PASS = tune.get_bool("delta_two_pass", True)
 UNIT_KEY_EPS = 1e-6
+# prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on: one chunk
+# takes what 16 tokens of the scan take (15.1 against 15.0 us, 32 heads of 64), four take 20 against 32
+DELTA_CHUNK = True
+DELTA_CHUNK_D = (32, 64)
+DELTA_CHUNK_MIN = 32
 
 
 def delta_rule_scan(proj: torch.Tensor, off_r: int, off_k: int, off_v: int, off_a: int, wl: torch.Tensor,
@@ -333,6 +338,16 @@ def delta_rule_scan(proj: torch.Tensor, off_r: int, off_k: int, off_v: int, off_
     if native_device(proj):
         assert proj.stride(1) == 1 and wl.stride(1) == 1 and wl.dtype == proj.dtype
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, D)
+        es = proj.element_size()
+        if DELTA_CHUNK and D in DELTA_CHUNK_D and sm.max_q >= DELTA_CHUNK_MIN and proj.data_ptr() % 16 == 0 \
+                and proj.stride(0) * es % 16 == 0 and off_v * es % 16 == 0:
+            scratch = torch.empty(mixers().delta_chunk_scratch_floats(T, sm.num_seqs, H, D), dtype=torch.float32,
+                                  device=proj.device)
+            mixers().delta_chunk(proj.data_ptr(), is_f32(proj), proj.stride(0), off_r, off_k, off_v, off_a, wl.data_ptr(),
+                                 wl.stride(0), a_bias.data_ptr(), w0.data_ptr(), state.data_ptr(), _i32(sm.qsl).data_ptr(),
+                                 _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), o.data_ptr(), sm.num_seqs, sm.max_q,
+                                 H, D, scratch.data_ptr(), stream_ptr())
+            return o
         # state-independent terms (decay, removal rate, unit key) in a parallel pass of their own
         prep = torch.empty(T * H * 5 * D, dtype=torch.float32, device=proj.device) if DELTA_TWO_PASS else None
         mixers().delta_scan(proj.data_ptr(), is_f32(proj), proj.stride(0), off_r, off_k, off_v, off_a, wl.data_ptr(),
