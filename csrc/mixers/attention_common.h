@@ -55,6 +55,14 @@ struct AttnArgs {
   int keep;
 };
 
+// expanded latents (see prompt_attention.hip)
+struct LatentRows {
+  const bf16 *kn, *v, *lat;
+  const int32_t* koff;
+  const float* rot;
+  int dn, R, rd, rot_dims;
+};
+
 constexpr int kSingleMaxRep = 16;   // query heads per key / value head the single-token kernel takes
 
 // single_attention.hip: steps of single tokens (dk <= 128, dv <= 128 value columns, H / G <= kSingleMaxRep). nsplit > 1:

@@ -106,6 +106,11 @@ int latent_attention(const void*, const void*, bool, int64_t, int, int, const vo
 int latent_attention_mfma(const void*, const void*, int, int, const void*, int64_t, const void*, const int32_t*, int, int,
                           const int32_t*, const int32_t*, const int32_t*, const float*, int, void*, int, int, int, int, int,
                           int, int, float, int, float*, float*, hipStream_t);
+void latent_gather(const void*, const int32_t*, int, int, const int32_t*, const int32_t*, const int32_t*, int, int, int, void*,
+                   int32_t*, int, hipStream_t);
+int latent_prompt_attention(const void*, int, int, int, const void*, const void*, const void*, int, const int32_t*, const void*,
+                            int64_t, const float*, int, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int,
+                            int, int, float, hipStream_t);
 int delta_scan(const void*, bool, int64_t, int, int, int, int, const void*, int64_t, const float*, const float*, float*,
                const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, float*, int, hipStream_t);
 void delta_out(const float*, const float*, const void*, bool, int64_t, float, void*, int, int, int, hipStream_t);
@@ -534,6 +539,23 @@ PYBIND11_MODULE(_mixers, m) {
                                         P<void>(out), T, ns, max_q, H, R, rd, window, scale, nsplit, P<float>(part_o),
                                         P<float>(part_ml), S(st));
     check(rc, "latent_attention_mfma");
+  });
+  m.def("latent_gather", [](uintptr_t cache, uintptr_t bt, int bt_width, int bs, uintptr_t qsl, uintptr_t sl, uintptr_t slots,
+                            int ns, int window, int width, uintptr_t rows, uintptr_t koff, int nk, uintptr_t st) {
+    if (width < 8 || width % 8 || bs < 1 || window < 1) throw std::invalid_argument("latent_gather: inconsistent sizes");
+    xgm::latent_gather(P<const void>(cache), P<const int32_t>(bt), bt_width, bs, P<const int32_t>(qsl), P<const int32_t>(sl),
+                       P<const int32_t>(slots), ns, window, width, P<void>(rows), P<int32_t>(koff), nk, S(st));
+    check(0, "latent_gather");
+  });
+  m.def("latent_prompt_attention", [](uintptr_t q, int dn, int rd, int dv, uintptr_t kn, uintptr_t v, uintptr_t lat, int R,
+                                      uintptr_t koff, uintptr_t gate, int64_t ld_gate, uintptr_t rot, int rot_dims,
+                                      uintptr_t qsl, uintptr_t sl, uintptr_t slots, uintptr_t out, int T, int ns, int max_q,
+                                      int H, int window, float scale, uintptr_t st) {
+    int rc = xgm::latent_prompt_attention(P<const void>(q), dn, rd, dv, P<const void>(kn), P<const void>(v),
+                                          P<const void>(lat), R, P<const int32_t>(koff), P<const void>(gate), ld_gate,
+                                          P<const float>(rot), rot_dims, P<const int32_t>(qsl), P<const int32_t>(sl),
+                                          P<const int32_t>(slots), P<void>(out), T, ns, max_q, H, window, scale, S(st));
+    check(rc, "latent_prompt_attention");
   });
   m.def("delta_scan", [](uintptr_t proj, bool f32, int64_t ld, int off_r, int off_k, int off_v, int off_a, uintptr_t wl,
                          int64_t ld_wl, uintptr_t a_bias, uintptr_t w0, uintptr_t state, uintptr_t qsl, uintptr_t sl,

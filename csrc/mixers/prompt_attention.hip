@@ -12,6 +12,14 @@
 // the last row's own; a tile (or a wave's part of it) that lies wholly inside every row's view skips the per-key tests, one
 // that no row of the wave sees is passed over. 16 keys in a row share a page (block sizes are multiples of 16), so the page
 // index of a wave's DMA rows is one scalar load.
+//
+// LAT: multi-head attention over expanded latents. Every head has keys and values of its own in dense rows: [kn (dn) | the
+// rotated key shared by all heads (rd, read from the latent rows)] and v; key `lo` + i of sequence s is row koff[s] + i, lo the
+// first key its first query row sees. The rotary part of a query is rotated while it is loaded. In latent space (latent_attention)
+// a (query, key) pair costs 2 (2 R + rd) operations per head, here 2 (dn + rd + dv): 3.4 times less at R = 256 and heads of 64,
+// against one product per key row that expands it (4 x 2048 tokens, 32 heads of 64 + 32, window 1024: 950 -> 205 us with the
+// gather and both expansions; heads of 128 + 64, window 4096: 3857 -> 395). Rows of 96 and 192 entries have 12 and 24 chunks: the permutation there
+// stays inside groups of 4 and 8.
 #include "attention_common.h"
 #include "glds.h"
 
@@ -48,19 +56,20 @@ __device__ __forceinline__ void sched_fence() {
 // neighbouring chunks do too
 template <int D>
 __device__ __forceinline__ int xsw(int r) {
-  return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  return D == 96 ? (r >> 2) & 3 : D == 192 ? (r >> 1) & 7 : D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
 
-template <int DK, int DV, int GH, int NSLOT, int WFN>
+template <int DK, int DV, int GH, int NSLOT, int WFN, bool LAT>
 __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_attention_kernel(
     const AttnArgs a, const int32_t* __restrict__ block_tables, const bf16* __restrict__ kcache,
-    const bf16* __restrict__ vcache, int tiles_per_seq, int n_hg) {
+    const bf16* __restrict__ vcache, int tiles_per_seq, int n_hg, const LatentRows lr) {
   constexpr bool sig = WFN == kWeightsSigmoid, capped = WFN == kWeightsBounded || WFN == kWeightsCapped;
   constexpr bool bounded = WFN == kWeightsBounded;
   constexpr int NW = 8, RBLK = NW / GH, BM = 32 * RBLK;
   constexpr int KROW = DK * 2, VROW = DV * 2;            // bytes of a row
   constexpr int KT = kPT * KROW, SLOT = KT + kPT * VROW;  // bytes of a K tile, of a ring slot [K | V]
-  constexpr int KD = DK / 64, VD = DV / 64;               // DMA instructions per wave and tile (8 rows per wave)
+  constexpr int KD = (DK + 63) / 64, VD = DV / 64;        // DMA instructions per wave and tile (8 rows per wave)
+  static_assert(LAT || DK % 64 == 0, "rows of 96 and 192 entries: dense form only");
   __shared__ __attribute__((aligned(1024))) char lds[NSLOT * SLOT];
 
   const int bid = blockIdx.x;
@@ -94,8 +103,29 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
   const int32_t* bt = block_tables + (int64_t)s * a.bt_width;
   auto tile_key = [&](int t) { return t < kt ? t * kPT : kfirst + (t - kt) * kPT; };
 
+  const int lat_lo = first_visible(a.mask, a.size, ctx);   // the sequence's first dense key row
+  const int64_t lat_row = LAT ? (int64_t)lr.koff[s] - lat_lo : 0;
   auto issue = [&](int t) {
     char* dst = lds + (t % NSLOT) * SLOT;
+    if constexpr (LAT) {
+      const int k1 = tile_key(t) + 8 * w;   // (keys in front of the first row are masked: any row will do)
+#pragma unroll
+      for (int i = 0; i < KD; ++i) {
+        const int idx = 64 * i + lane, rr = idx / (DK / 8), d = ((idx % (DK / 8)) ^ xsw<DK>(8 * w + rr)) * 8;
+        const int64_t row = lat_row + max(min(k1 + rr, last), lat_lo);
+        if (idx < DK)   // (8 rows of DK / 8 chunks)
+          xgk::glds16(d < lr.dn ? lr.kn + (row * a.H + head) * lr.dn + d : lr.lat + row * (lr.R + lr.rd) + lr.R + d - lr.dn,
+                      dst + 8 * w * KROW + i * 1024);
+      }
+#pragma unroll
+      for (int i = 0; i < VD; ++i) {
+        const int rr = VD == 2 ? 4 * i + (lane >> 4) : lane >> 3;
+        const int ch = (VD == 2 ? lane & 15 : lane & 7) ^ xsw<DV>(8 * w + rr);
+        const int64_t row = lat_row + max(min(k1 + rr, last), lat_lo);
+        xgk::glds16(lr.v + (row * a.H + head) * DV + ch * 8, dst + KT + (8 * w) * VROW + i * 1024);
+      }
+      return;
+    }
     const int key0 = min(tile_key(t) + 8 * w, last);      // the wave's 8 rows: inside one aligned run of 16 keys
     const int pidx = key0 / a.bs;
     const int64_t prow = (int64_t)bt[pidx] * a.bs - (int64_t)pidx * a.bs;
@@ -121,7 +151,25 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
   {
     const bf16* qp = a.q + ((int64_t)(q0 + min(my_row, qn - 1)) * a.H + head) * DK + 8 * hf;
 #pragma unroll
-    for (int ks = 0; ks < DK / 16; ++ks) qf[ks] = xgk::as_frag(xgk::ld16(qp + 16 * ks));
+    for (int ks = 0; ks < DK / 16; ++ks) {
+      uint4 x = xgk::ld16(qp + 16 * ks);
+      const int i0 = 16 * ks + 8 * hf - lr.dn;   // LAT: pairs (i0, i0 + 1), .. of the rotary part turn by the row's angles
+      if (LAT && i0 >= 0 && i0 < lr.rot_dims) {
+        float f[8];
+        xgk::unpack8(x, f);
+        const float* cs = lr.rot + ((int64_t)min(pos_q, ctx + qn - 1) * (lr.rot_dims >> 1) + (i0 >> 1)) * 2;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          if (i0 + e < lr.rot_dims) {
+            const float c = cs[e], sn = cs[e + 1], u = f[e], v = f[e + 1];
+            f[e] = u * c - v * sn;
+            f[e + 1] = v * c + u * sn;
+          }
+        }
+        x = xgk::pack8(f);
+      }
+      qf[ks] = xgk::as_frag(x);
+    }
   }
   const float cap2 = capped ? a.softcap * kLog2e : 0.f;
   float sc_h = a.scale * (a.temp ? a.temp[head] : 1.f) * (capped ? 2.f / a.softcap : 1.f) * kLog2e;
@@ -158,7 +206,15 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
     // (wave-uniform) nothing of this tile is visible to the wave's rows
     if (!wave_on || base > pos_hi || (base + kPT - 1 < lo_lo && base >= a.keep)) continue;
     const uint32_t slot = (j % NSLOT) * SLOT;
-    const uint32_t k_lane = (slot + r * KROW) ^ ((uint32_t)(hf ^ xsw<DK>(r)) << 4);
+    // chunk 2 ks + hf of row r: KROW a power of two, one xor of the whole address; else xor inside 4 (8) chunks, added on
+    constexpr bool POW2 = DK == 64 || DK == 128;
+    constexpr int KG = DK == 192 ? 4 : 2;   // (pairs of chunks per permuted group)
+    const uint32_t k_lane = POW2 ? (slot + r * KROW) ^ ((uint32_t)(hf ^ xsw<DK>(r)) << 4)
+                                 : slot + r * KROW + ((uint32_t)((hf ^ xsw<DK>(r)) & 1) << 4);
+    uint32_t k_pair[KG];
+#pragma unroll
+    for (int i = 0; i < KG; ++i) k_pair[i] = (uint32_t)(i ^ (xsw<DK>(r) >> 1)) << 5;
+    auto k_at = [&](int ks) { return POW2 ? k_lane ^ (ks << 5) : k_lane + k_pair[ks % KG] + (ks / KG) * (32 * KG); };
     const uint32_t v_row = slot + KT + (4 * hf + tq) * VROW + 8 * (tp & 1);
     const uint32_t v_hi = (uint32_t)(DV == 128 ? tq : tq >> 1) << 6, v_lo = 2 * (tg & 1) + (tp >> 1);
     const uint32_t v_lane0 = (v_row + ((v_lo ^ hf) << 4)) | v_hi;
@@ -171,7 +227,7 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
       for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < DK / 16; ++ks)
-        sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + ((k_lane ^ (ks << 5)) + kb * 32 * KROW))), qf[ks], sacc[kb]);
+        sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + (k_at(ks) + kb * 32 * KROW))), qf[ks], sacc[kb]);
       sched_fence();   // bound the hoisted fragment reads
     }
     // scores in units of ln 2; register e of block kb is key base + 32 kb + 4 hf + (e & 3) + 8 (e >> 2)
@@ -292,7 +348,8 @@ bool prompt_attention(const AttnArgs& a, int max_q, int wfn, hipStream_t st) {
   const int tps = (max_q + bm - 1) / bm, n_hg = a.G * rep / gh;
   const int grid = n_hg * a.ns * tps;
 #define XGM_PA3(DK, DV, GH, WFN)                                                                                      \
-  prompt_attention_kernel<DK, DV, GH, 3, WFN><<<grid, 512, 0, st>>>(a, a.block_tables, a.kcache, a.vcache, tps, n_hg)
+  prompt_attention_kernel<DK, DV, GH, 3, WFN, false><<<grid, 512, 0, st>>>(a, a.block_tables, a.kcache, a.vcache, tps, n_hg, \
+                                                                          LatentRows{})
 #define XGM_PA2(DK, DV, GH)                                  \
   switch (wfn) {                                             \
     case kWeightsSigmoid:                                    \
@@ -329,6 +386,87 @@ bool prompt_attention(const AttnArgs& a, int max_q, int wfn, hipStream_t st) {
 #undef XGM_PA2
 #undef XGM_PA3
   return true;
+}
+
+// ---- dense latent rows of a step's keys: per sequence the cached rows from the first key that its first new token sees to its
+// last; koff[s] = first row of sequence s. One workgroup copies 16 rows.
+constexpr int kGatherRows = 16;
+
+__global__ __launch_bounds__(256) void latent_gather_kernel(const bf16* __restrict__ cache, const int32_t* __restrict__ block_tables,
+                                                            int bt_width, int bs, const int32_t* __restrict__ qsl,
+                                                            const int32_t* __restrict__ seq_lens,
+                                                            const int32_t* __restrict__ slots, int ns, int window, int W8,
+                                                            bf16* __restrict__ rows, int32_t* __restrict__ koff, int nk) {
+  __shared__ int first_s, first_i;
+  const int r0 = blockIdx.x * kGatherRows;
+  if (threadIdx.x == 0) first_s = ns, first_i = 0;
+  __syncthreads();
+  if (threadIdx.x < 64) {   // key counts of 64 sequences at a time, summed up over the wave
+    int before = 0;
+    for (int s0 = 0; s0 < ns; s0 += 64) {
+      const int s = s0 + threadIdx.x;
+      int n = 0;
+      if (s < ns) {
+        const int q = qsl[s + 1] - qsl[s], len = seq_lens[s];
+        n = slots[s] < 0 || q <= 0 ? 0 : len - max(0, len - q - window + 1);
+      }
+      int upto = n;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(upto, o, 64);
+        if (threadIdx.x >= o) upto += up;
+      }
+      const int at = before + upto - n;
+      if (s < ns && blockIdx.x == 0) koff[s] = min(at, nk);
+      if (r0 >= at && r0 < at + n) first_s = s, first_i = r0 - at;
+      before += __shfl(upto, 63, 64);
+    }
+  }
+  __syncthreads();
+  int s = first_s, i = first_i;   // row r0 = key i of sequence s; the rows behind it follow
+  for (int r = r0; r < min(r0 + kGatherRows, nk); ++r, ++i) {
+    int lo = 0, len = 0;
+    for (; s < ns; ++s, i = 0) {
+      const int q = qsl[s + 1] - qsl[s];
+      len = seq_lens[s], lo = max(0, len - q - window + 1);
+      if (slots[s] >= 0 && q > 0 && i < len - lo) break;
+    }
+    if (s >= ns) break;
+    const int key = lo + i;
+    const uint4* src = reinterpret_cast<const uint4*>(cache) +
+                       ((int64_t)block_tables[(int64_t)s * bt_width + key / bs] * bs + key % bs) * W8;
+    for (int c = threadIdx.x; c < W8; c += 256) reinterpret_cast<uint4*>(rows)[(int64_t)r * W8 + c] = src[c];
+  }
+}
+
+void latent_gather(const void* cache, const int32_t* bt, int bt_width, int bs, const int32_t* qsl, const int32_t* seq_lens,
+                   const int32_t* slots, int ns, int window, int width, void* rows, int32_t* koff, int nk, hipStream_t st) {
+  if (ns <= 0 || nk <= 0) return;
+  latent_gather_kernel<<<(nk + kGatherRows - 1) / kGatherRows, 256, 0, st>>>(
+      (const bf16*)cache, bt, bt_width, bs, qsl, seq_lens, slots, ns, window, width / 8, (bf16*)rows, koff, nk);
+}
+
+// q [T][H][dn + rd], out [T][H][dv]; kn [rows][H][dn], v [rows][H][dv], lat [rows][R + rd], koff of latent_gather
+int latent_prompt_attention(const void* q, int dn, int rd, int dv, const void* kn, const void* v, const void* lat, int R,
+                            const int32_t* koff, const void* gate, int64_t ld_gate, const float* rot, int rot_dims,
+                            const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots, void* out, int T_, int ns,
+                            int max_q, int H, int window, float scale, hipStream_t st) {
+  if (ns <= 0 || max_q <= 0) return 0;
+  const int dk = dn + rd;
+  if (dn % 8 || rd % 8 || R % 8 || H < 1 || window < 1 || rot_dims % 2 || rot_dims > rd || !((dk == 96 && dv == 64) ||
+      (dk == 192 && dv == 128)))
+    return -1;
+  AttnArgs a = {};
+  a.q = (const bf16*)q, a.qsl = qsl, a.seq_lens = seq_lens, a.slots = slots, a.out = (bf16*)out;
+  a.T = T_, a.ns = ns, a.H = H, a.G = H, a.dk = dk, a.dv_head = dv, a.mask = kMaskWindow, a.size = window, a.scale = scale;
+  a.gate = (const bf16*)gate, a.ld_gate = ld_gate, a.vmode = kValuesOwn, a.bs = 16;
+  const LatentRows lr = {(const bf16*)kn, (const bf16*)v, (const bf16*)lat, koff, rot, dn, R, rd, rot_dims};
+  const int tps = (max_q + 255) / 256, grid = H * ns * tps;
+  if (dk == 96)
+    prompt_attention_kernel<96, 64, 1, 3, kWeightsSoftmax, true><<<grid, 512, 0, st>>>(a, nullptr, nullptr, nullptr, tps, H, lr);
+  else
+    prompt_attention_kernel<192, 128, 1, 3, kWeightsSoftmax, true><<<grid, 512, 0, st>>>(a, nullptr, nullptr, nullptr, tps, H, lr);
+  return 0;
 }
 
 }  // namespace xgm

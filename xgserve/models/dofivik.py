@@ -75,11 +75,9 @@ class LatentAttentionMixer(nn.Module):
         cq = sq.latent_prep(proj, 0, self.Rq, self.off_kv, self.R, self.rd, self.q_norm, self.kv_norm, self.eps, rot,
                             self.rot_dims, sm, cache_rows)
         q = F.linear(cq, self.uq).view(T, H, dq)
-        qabs = torch.bmm(q[:, :, :self.dn].transpose(0, 1), self.uk.view(H, self.dn, self.R))  # [H, T, R]
-        o_lat = sq.latent_attention(qabs, q, self.dn, proj[:, self.off_g:], cache_rows, rot, self.rot_dims, self.window,
-                                    self.scale, block_size, sm)
-        o = torch.bmm(o_lat, self.uv.view(H, self.dv, self.R).transpose(1, 2))  # [H, T, dv]
-        return F.linear(sq.heads_to_rows(o), self.o)
+        o = sq.latent_attention_heads(q, self.dn, proj[:, self.off_g:], cache_rows, self.uk, self.uv, rot, self.rot_dims,
+                                      self.window, self.scale, block_size, sm)
+        return F.linear(o, self.o)
 
 
 class DeltaRuleMixer(nn.Module):

@@ -304,6 +304,57 @@ def latent_attention(qabs: torch.Tensor, q: torch.Tensor, dn: int, gate: torch.T
     return out
 
 
+# Prompt portions over expanded keys and values (prompt_attention.hip, LAT) instead of in latent space: from 64 tokens on (heads of
+# 64 and 128: 33 -> 30 and 46 -> 35 us alone, 123 -> 61 and 208 -> 89 behind 1024 tokens), however many key rows there are to a
+# token up to the 32 that were measured (128 tokens behind 4000: 722 -> 225 us); 4 x 2048 tokens 950 -> 205 and 3857 -> 395. The
+# rows are bounded because their number is: single tokens of many sequences in the step each count a whole window.
+LATENT_EXPAND = True
+LATENT_EXPAND_MIN = 64
+LATENT_EXPAND_ROWS, LATENT_EXPAND_MAX = 32, 65536   # key rows per token, and in all (1 GB of keys and values at 64 heads' sizes)
+LATENT_EXPAND_SIZES = ((96, 64), (192, 128))        # (dn + rd, dv)
+
+
+def _latent_key_rows(sm: SeqMeta, T: int, window: int, block_size: int) -> int:
+    """At most this many cached rows are seen by a step's portions (the contexts are on the device): the new tokens, and per
+    sequence its window before them or what its page table can hold."""
+    held = sm.num_seqs * sm.block_tables.shape[1] * block_size
+    return T + max(0, min(sm.num_seqs * (window - 1), held - T))
+
+
+def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: torch.Tensor, uk: torch.Tensor,
+                           uv: torch.Tensor, rot: torch.Tensor, rot_dims: int, window: int, scale: float, block_size: int,
+                           sm: SeqMeta) -> torch.Tensor:
+    """Latent attention from the queries to the heads' outputs: q [T, H, dn + rd]; uk [H dn, R] and uv [H dv, R] expand a latent
+    into the heads' unrotated keys and their values. Returns [T, H dv]. Long portions expand the latents they see once and
+    attend over per-head keys and values; otherwise the attention runs in latent space, uk folded into the query and uv behind
+    the softmax."""
+    T, H, dq = q.shape
+    R, dv = uk.shape[1], uv.shape[0] // H
+    if native_device(q) and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN \
+            and (dq, dv) in LATENT_EXPAND_SIZES and dn % 8 == 0 and R % 8 == 0 and rot_dims % 2 == 0:
+        nk = _latent_key_rows(sm, T, window, block_size)
+        if nk <= min(LATENT_EXPAND_ROWS * T, LATENT_EXPAND_MAX):
+            assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
+            assert cache.dtype == gate.dtype == uk.dtype == uv.dtype == q.dtype
+            M, bt = mixers(), _i32(sm.block_tables)
+            lat = torch.empty(nk, R + dq - dn, dtype=q.dtype, device=q.device)
+            koff = torch.empty(sm.num_seqs, dtype=torch.int32, device=q.device)
+            M.latent_gather(cache.data_ptr(), bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(),
+                            _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), sm.num_seqs, int(window), lat.shape[1],
+                            lat.data_ptr(), koff.data_ptr(), nk, stream_ptr())
+            kn = torch.nn.functional.linear(lat[:, :R], uk)
+            v = torch.nn.functional.linear(lat[:, :R], uv)
+            out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+            M.latent_prompt_attention(q.data_ptr(), dn, dq - dn, dv, kn.data_ptr(), v.data_ptr(), lat.data_ptr(), R,
+                                      koff.data_ptr(), gate.data_ptr(), gate.stride(0), rot.data_ptr(), rot_dims,
+                                      sm.qsl.data_ptr(), sm.seq_lens.data_ptr(), sm.slots.data_ptr(), out.data_ptr(), T,
+                                      sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
+            return out
+    qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
+    o_lat = latent_attention(qabs, q, dn, gate, cache, rot, rot_dims, window, scale, block_size, sm)
+    return heads_to_rows(torch.bmm(o_lat, uv.view(H, dv, R).transpose(1, 2)))   # [H, T, dv] -> rows
+
+
 def heads_to_rows(x: torch.Tensor) -> torch.Tensor:
     """[H, T, n] -> [T, H * n]."""
     H, T, n = x.shape
