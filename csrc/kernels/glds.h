@@ -105,4 +105,29 @@ __device__ __forceinline__ void st4_sc1(float* p, float v) {
 #endif
 }
 
+// Every wave drains its stores (write-through), then one relaxed agent-scope
+// ticket; returns in every thread whether this workgroup drew `last_value`. The
+// winner acquires (agent scope: drops this CU's stale L1 lines) before any of its
+// waves reads what the others published, and re-arms the word. `flag` is an LDS
+// word no wave touches concurrently (inside the staging array: ONE __shared__
+// object per kernel, guide §5 "Three .s-level traps" (a)).
+__device__ __forceinline__ bool agent_ticket(int* cnt, int last_value, int* flag) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int prev = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int last = prev == last_value;
+    if (last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *flag = last;
+  }
+  __syncthreads();
+  const bool r = *flag != 0;
+  __syncthreads();
+  return r;
+}
+
 }  // namespace xgk

@@ -14,7 +14,7 @@ int gemm_pf_grouped(const uint16_t*, const int32_t*, const int32_t*, int, int, i
                     uint16_t*, int, int, int, hipStream_t, int, int, float, float);
 }
 namespace xgm {
-void embed_rows(const int32_t*, const void*, bool, float*, int, int, int, const void*, const int32_t*, int, float,
+void embed_rows(const int32_t*, const void*, bool, float*, int, int, int, const void*, const int32_t*, int, float, int*, int,
                 hipStream_t);
 void causal_conv(const void*, bool, int64_t, const float*, const float*, float*, const int32_t*, const int32_t*,
                  const int32_t*, void*, bool, int, int, int, int, bool, bool, hipStream_t);
@@ -47,6 +47,8 @@ int gated_linear_scan(const float*, const float*, const float*, const void*, int
                       const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int,
                       int, int, int, float*, int, int, const float*, const float*, hipStream_t);
 int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
+int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
+                bool, hipStream_t);
 int64_t delta_chunk_scratch_floats(int, int, int, int);
 int delta_chunk(const void*, bool, int64_t, int, int, int, int, const void*, int64_t, const float*, const float*, float*,
                 const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, float*, hipStream_t);
@@ -130,10 +132,10 @@ static void check(int rc, const char* what) {
 
 PYBIND11_MODULE(_mixers, m) {
   m.def("embed_rows", [](uintptr_t ids, uintptr_t table, bool f32, uintptr_t out, int T, int W, int V, uintptr_t pos_table,
-                         uintptr_t positions, int Pn, float scale, uintptr_t st) {
+                         uintptr_t positions, int Pn, float scale, uintptr_t zero, int nzero, uintptr_t st) {
     if (pos_table && !positions) throw std::invalid_argument("embed_rows: a position table needs positions");
     xgm::embed_rows(P<const int32_t>(ids), P<const void>(table), f32, P<float>(out), T, W, V, P<const void>(pos_table),
-                    P<const int32_t>(positions), Pn, scale, S(st));
+                    P<const int32_t>(positions), Pn, scale, P<int>(zero), zero ? nzero : 0, S(st));
     check(0, "embed_rows");
   });
   m.def("causal_conv", [](uintptr_t x, bool in_f32, int64_t ld_in, uintptr_t w, uintptr_t bias, uintptr_t state,
@@ -291,6 +293,13 @@ PYBIND11_MODULE(_mixers, m) {
   });
   m.def("gated_linear_scan_scratch_floats",
         [](int T, int ns, int H, int dk, int dv) { return xgm::gated_linear_scan_scratch_floats(T, ns, H, dk, dv); });
+  m.def("rows_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part,
+                          uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, bool wide,
+                          uintptr_t st) {
+    check(xgm::rows_linear(P<const void>(x), ld_x, P<const void>(w), P<const void>(bias), bias_f32, P<float>(part),
+                           P<void>(out), P<int>(tickets), T, N, K, S_, act, p0, p1, wide, S(st)),
+          "rows_linear");
+  });
   m.def("delta_chunk_scratch_floats",
         [](int T, int ns, int H, int D) { return xgm::delta_chunk_scratch_floats(T, ns, H, D); });
   m.def("delta_chunk", [](uintptr_t proj, bool f32, int64_t ld, int off_r, int off_k, int off_v, int off_a, uintptr_t wl,

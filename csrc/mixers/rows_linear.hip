@@ -1,0 +1,258 @@
+// Products of a few activation rows (decode steps, T <= 64) with a weight matrix, and what follows them:
+//
+//   rows_linear         out [T, N] = act(x [T, K] . w [N, K]^T + bias), or glu(gate, up) of w's two halves
+//
+// The weights are read once and carry the time: 2 N K bytes against T <= 64 rows. A workgroup owns COLS weight rows and
+// one of S equal parts of K; its chunks of x and w come in by LDS-DMA through a ring of NS slots (NS - 1 chunks in
+// flight, so that a CU keeps 40 to 100 KB on the way), every weight row a full 128- or 256-byte line, and the products
+// are 16x16x32 MFMAs with fp32 sums. Rows are staged with their 16-byte granules permuted by the row number, so the
+// fragment reads of 16 rows fall on all banks.
+//
+// S parts of K: the parts of a column tile write fp32 slabs (write-through) and take a ticket; the one that draws the
+// last adds the slabs in order and finishes the tile, so a narrow product still puts a workgroup on every CU and needs
+// no second launch. The tickets are words that are zero before the launch and zero again after it.
+//
+// Measured against the library's product without what follows it, cold weights, us (T = 1 / 17 / 64):
+//   2048 x 2048    5.7 /  7.1 /  8.6 against 11.0 / 11.0 / 11.8      18560 x 4096   28 / 29 / 37 against 67 / 36 / 40
+//   2048 x 8192    9.5 / 11.0 / 13.8 against 12.9 / 13.7 / 22.6      28672 x 4096   39 / 38 / 41 against 64 / 55 / 56
+//   10272 x 2048   9.9 / 10.4 / 13.9 against 16.3 / 14.6 / 15.9      4096 x 14336   21 / 22 / 27 against 26 / 28 / 39
+// (5.8 TB/s of weights at the largest). Small products are bound by latency: the parts' stores, ticket and reads back are
+// 2 us at one row and 4 us at 64 (64 KB to 128 KB of slabs for one workgroup).
+#include "attention_common.h"
+#include "glds.h"
+#include "glu.h"
+
+namespace xgm {
+using xgk::as_frag;
+using xgk::f32x4_t;
+using xgk::glu;
+using xgk::mfma16x16x32;
+
+enum { kActNone = 0, kActXielu = 1, kActRelu2 = 2, kActGlu = 3 };   // kActGlu + kind: glu.h
+
+struct RowsArgs {
+  const bf16 *x, *w;
+  const void* bias;        // [N] fp32 or bf16, or nullptr
+  float* part;             // S > 1: [S, T, N] fp32
+  bf16* out;               // [T, N], or [T, N / 2] for the gated activations
+  int* tickets;            // one zero word per column tile (S > 1)
+  int64_t ld_x;
+  int T, N, K, act;
+  float p0, p1;
+  bool bias_f32;
+};
+
+// act(v + bias) of four neighbouring columns
+__device__ __forceinline__ void rows_finish(const RowsArgs& a, int tok, int col, float (&v)[4]) {
+  if (a.bias) {
+    float b[4];
+    if (a.bias_f32) ld4((const float*)a.bias + col, b);
+    else ld4((const bf16*)a.bias + col, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += b[e];
+  }
+  if (a.act == kActXielu) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float z = v[e];
+      v[e] = z > 0.f ? a.p0 * z * z + 0.5f * z : a.p1 * (expm1f(z) - z) + 0.5f * z;
+    }
+  } else if (a.act == kActRelu2) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float r = v[e] < 0.f ? 0.f : v[e];   // (a NaN stays one)
+      v[e] = r * r;
+    }
+  }
+  st4(a.out + (int64_t)tok * a.N + col, v);
+}
+
+__device__ __forceinline__ void rows_finish_glu(const RowsArgs& a, int tok, int f, const float (&g)[4], const float (&u)[4]) {
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = glu(a.act - kActGlu, g[e], u[e], a.p0, a.p1);
+  st4(a.out + (int64_t)tok * (a.N / 2) + f, v);
+}
+
+// sum of the S slabs at `at` (every read comes from another XCD's workgroup: all S are in flight before the first add)
+template <int S>
+__device__ __forceinline__ void slab_sum(const float* __restrict__ at, int64_t slab, float (&v)[4]) {
+  float p[S][4];
+#pragma unroll
+  for (int s = 0; s < S; ++s) ld4(at + s * slab, p[s]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = p[0][e];
+#pragma unroll
+    for (int s = 1; s < S; ++s) v[e] += p[s][e];
+  }
+}
+
+// the last part of a column tile: columns [c0, c0 + NC) (gated: and as many of the second half) of every row
+template <int NC, int NTHR, int S>
+__device__ __forceinline__ void rows_tail(const RowsArgs& a, int c0, bool gated) {
+  const int64_t slab = (int64_t)a.T * a.N;
+  const int half = a.N / 2;
+#pragma unroll 2
+  for (int i = threadIdx.x; i < a.T * (NC / 4); i += NTHR) {
+    const int tok = i / (NC / 4), col = c0 + 4 * (i % (NC / 4));
+    const float* at = a.part + (int64_t)tok * a.N + col;
+    float v[4];
+    if (gated) {
+      if (col >= half) continue;
+      float u[4];
+      slab_sum<S>(at, slab, v);
+      slab_sum<S>(at + half, slab, u);
+      rows_finish_glu(a, tok, col, v, u);
+    } else {
+      if (col >= a.N) continue;
+      slab_sum<S>(at, slab, v);
+      rows_finish(a, tok, col, v);
+    }
+  }
+}
+
+// Workgroup (tile, part of K): WV waves of NW 16-row weight tiles each, MT 16-row x tiles. A gated launch (NW = 2)
+// gives each wave the same 16 rows of w's first and second half.
+template <int MT, int NW, int WV, int KC, int NS>
+__global__ __launch_bounds__(64 * WV, 1) void rows_linear_kernel(const RowsArgs a) {
+  constexpr int RB = KC * 2, GPR = KC / 8, RPI = 1024 / RB;   // bytes and granules per staged row, rows per DMA instruction
+  constexpr int XROWS = 16 * MT, COLS = 16 * NW * WV;
+  constexpr int XI = XROWS / RPI / WV, WI = 16 * NW / RPI, G = XI + WI;
+  constexpr int SLOT = (XROWS + COLS) * RB;
+  static_assert(XI >= 1 && WI >= 1 && XROWS % (RPI * WV) == 0 && NS * SLOT <= 160 * 1024, "rows_linear geometry");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * SLOT];
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = gridDim.y, part = blockIdx.y, bx = blockIdx.x;
+  const bool gated = NW == 2 && a.act >= kActGlu;
+  const int half = a.N / 2;
+  const int chunks = a.K / KC, c_lo = part * chunks / S, nch = (part + 1) * chunks / S - c_lo;
+  const int n0 = gated ? bx * (COLS / 2) + 16 * wv : bx * COLS + 16 * NW * wv;
+  const int dr = lane / GPR, dj = lane % GPR;
+  const bf16 *ws[WI], *xs[XI];
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    const int r = RPI * i + dr;
+    const int n = gated ? (r < 16 ? min(n0 + r, half - 1) : half + min(n0 + r - 16, half - 1)) : min(n0 + r, a.N - 1);
+    ws[i] = a.w + (int64_t)n * a.K + c_lo * KC + 8 * (dj ^ (r & (GPR - 1)));
+  }
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = RPI * (wv * XI + i) + dr;
+    xs[i] = a.x + min(r, a.T - 1) * a.ld_x + c_lo * KC + 8 * (dj ^ (r & (GPR - 1)));
+  }
+  // few parts: neighbouring tiles start at different chunks, or all of them would ask for the same column of weight rows
+  // 2 K bytes apart (few memory channels) at the same time
+  const int rot = S <= 2 ? (int)((unsigned)bx * 37u % (unsigned)nch) : 0;
+  auto issue = [&](int c) {   // (past the end: the last chunk again, into a slot that nobody reads)
+    uint8_t* slot = lds + (c % NS) * SLOT;
+    int cc = min(c, nch - 1) + rot;
+    cc = cc >= nch ? cc - nch : cc;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) xgk::glds16(xs[i] + cc * KC, slot + RPI * (wv * XI + i) * RB);
+#pragma unroll
+    for (int i = 0; i < WI; ++i) xgk::glds16_nt(ws[i] + cc * KC, slot + (XROWS + 16 * NW * wv) * RB + i * 1024);
+  };
+  f32x4_t acc[NW][MT];
+#pragma unroll
+  for (int n = 0; n < NW; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < NS - 1; ++c) issue(c);
+  for (int c = 0; c < nch; ++c) {
+    xgk::wait_vmcnt<(NS - 2) * G>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    xgk::raw_barrier();
+    issue(c + NS - 1);
+    const uint8_t* xl = lds + (c % NS) * SLOT;
+    const uint8_t* wl = xl + (XROWS + 16 * NW * wv) * RB;
+#pragma unroll
+    for (int t = 0; t < KC / 32; ++t) {
+      const int ph = ((4 * t + g4) ^ (l16 & (GPR - 1))) * 16;
+      uint4 b[MT], w[NW];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) b[m] = *reinterpret_cast<const uint4*>(xl + (16 * m + l16) * RB + ph);
+#pragma unroll
+      for (int n = 0; n < NW; ++n) w[n] = *reinterpret_cast<const uint4*>(wl + (16 * n + l16) * RB + ph);
+#pragma unroll
+      for (int n = 0; n < NW; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[n][m] = mfma16x16x32(as_frag(w[n]), as_frag(b[m]), acc[n][m]);
+    }
+  }
+  xgk::wait_vmcnt<0>();
+  // lane: weight row 4 g4 + r of the tile, token l16
+  if (S == 1) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int tok = 16 * m + l16;
+      if (tok >= a.T) continue;
+      if (gated) {
+        const int f = n0 + 4 * g4;
+        if (f >= half) continue;
+        const float g[4] = {acc[0][m][0], acc[0][m][1], acc[0][m][2], acc[0][m][3]};
+        const float u[4] = {acc[NW - 1][m][0], acc[NW - 1][m][1], acc[NW - 1][m][2], acc[NW - 1][m][3]};
+        rows_finish_glu(a, tok, f, g, u);
+        continue;
+      }
+#pragma unroll
+      for (int n = 0; n < NW; ++n) {
+        const int col = n0 + 16 * n + 4 * g4;
+        if (col >= a.N) continue;
+        float v[4] = {acc[n][m][0], acc[n][m][1], acc[n][m][2], acc[n][m][3]};
+        rows_finish(a, tok, col, v);
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int tok = 16 * m + l16;
+    if (tok >= a.T) continue;
+#pragma unroll
+    for (int n = 0; n < NW; ++n) {
+      const int in = gated ? n0 + 4 * g4 : n0 + 16 * n + 4 * g4;
+      if (in >= (gated ? half : a.N)) continue;
+      xgk::st16_sc1(a.part + ((int64_t)part * a.T + tok) * a.N + in + (gated && n ? half : 0), acc[n][m]);
+    }
+  }
+  if (!xgk::agent_ticket(a.tickets + bx, S - 1, reinterpret_cast<int*>(lds))) return;
+  const int c0 = gated ? bx * (COLS / 2) : bx * COLS;
+#define XGM_TAIL(SS)                                                  \
+  if (S == SS) {                                                      \
+    if (gated) rows_tail<COLS / 2, 64 * WV, SS>(a, c0, true);         \
+    else rows_tail<COLS, 64 * WV, SS>(a, c0, false);                  \
+  }
+  XGM_TAIL(2)
+  XGM_TAIL(4)
+  XGM_TAIL(8)
+#undef XGM_TAIL
+}
+
+// wide: 128 weight rows per workgroup instead of 64 (the gated activations: always). Returns 0, or -1 for sizes outside
+// the contract: 1 <= T <= 64, K % 128 == 0, N % 4 == 0 (gated: N % 8 == 0), S in {1, 2, 4, 8} with at least one chunk of
+// K per part, 16-byte aligned rows.
+int rows_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bool bias_f32, float* part, void* out,
+                int* tickets, int T, int N, int K, int S, int act, float p0, float p1, bool wide, hipStream_t st) {
+  const bool gated = act >= kActGlu;
+  if (T < 1 || T > 64 || N < 1 || K < 128 || K % 128 || N % (gated ? 8 : 4) || ld_x % 8 || (gated && (!wide || bias)) ||
+      act < 0 || (S != 1 && S != 2 && S != 4 && S != 8) || S > K / 128 || (S > 1 && !(part && tickets)) ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part) & 15) || ((uintptr_t)out & 7))
+    return -1;
+  RowsArgs a = {(const bf16*)x, (const bf16*)w, bias, part, (bf16*)out, tickets, ld_x, T, N, K, act, p0, p1, bias_f32};
+  const dim3 grid((N + (wide ? 127 : 63)) / (wide ? 128 : 64), S);
+  if (T <= 16) {
+    if (wide) rows_linear_kernel<1, 2, 4, 128, 4><<<grid, 256, 0, st>>>(a);
+    else rows_linear_kernel<1, 1, 4, 128, 4><<<grid, 256, 0, st>>>(a);
+  } else if (T <= 32) {
+    if (wide) rows_linear_kernel<2, 2, 4, 64, 6><<<grid, 256, 0, st>>>(a);
+    else rows_linear_kernel<2, 1, 4, 64, 6><<<grid, 256, 0, st>>>(a);
+  } else {
+    if (wide) rows_linear_kernel<4, 2, 4, 64, 3><<<grid, 256, 0, st>>>(a);
+    else rows_linear_kernel<4, 1, 4, 64, 4><<<grid, 256, 0, st>>>(a);
+  }
+  return 0;
+}
+}  // namespace xgm

@@ -29,7 +29,6 @@ from typing import Dict, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -59,9 +58,9 @@ class Retention(nn.Module):
         return (self.rot_dims, float(self.rot["base"])) if self.rot_dims else None
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, rot):
-        y = sq.retention(F.linear(h, self.in_proj), self.H, self.dk, self.dv, self.decay, rot, self.rot_dims, self.eps,
+        y = sq.retention(sq.linear(h, self.in_proj, sm), self.H, self.dk, self.dv, self.decay, rot, self.rot_dims, self.eps,
                          lc.gla, sm, self.decay_range)
-        return F.linear(y, self.o)
+        return sq.linear(y, self.o, sm)
 
 
 class WholeNormWindowAttention(nn.Module):
@@ -79,12 +78,12 @@ class WholeNormWindowAttention(nn.Module):
         self.o = _p(torch.empty(width, self.H * self.dv, device=device, dtype=dtype))
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int):
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         q = sq.head_norm_rope_cache(proj, self.H, self.G, self.dk, self.dv, self.q_norm, self.k_norm, self.eps, None, 0, sm,
                                     lc.k, lc.v, h.dtype, whole=True)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, self.mask, self.size, self.scale, None, None,
                                 block_size, sm, gate=proj[:, self.ch:])
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class TimeMix(nn.Module):
@@ -108,11 +107,11 @@ class TimeMix(nn.Module):
         if tile:   # single tokens: the four products in one launch
             r, k, v, g = sq.stacked_linear(mixed[:4], self.rkvg, T)[:, :T].unbind(0)
         else:
-            r, k, v, g = (F.linear(mixed[j], self.rkvg[j]) for j in range(4))
-        z = F.linear(sq.tanh_cols(F.linear(mixed[4][:T], self.w1), 0, self.rank), self.w2)
+            r, k, v, g = (sq.linear(mixed[j], self.rkvg[j], sm) for j in range(4))
+        z = sq.linear(sq.tanh_cols(sq.linear(mixed[4][:T], self.w1, sm), 0, self.rank), self.w2, sm)
         y = sq.time_mix(r, k, v, g, z, self.w0, self.u, self.norm, self.eps, self.H, self.dk, self.dk, lc.gla, sm,
                         dtype)
-        return F.linear(y, self.o)
+        return sq.linear(y, self.o, sm)
 
 
 class ParallelMixer(nn.Module):
@@ -171,7 +170,7 @@ class BazuraxLayer(nn.Module):
             ya, yb = self.mix(x, h, sm, lc, block_size)
             _, h = sq.layer_norm_residual(x, ya, self.norm1, self.eps, dt, y2=yb, scales=self.mix.scales, next_w=nw)
         if not last:
-            y = self.mlp(x, h) if self.moe else self.mlp(h)
+            y = self.mlp(x, h) if self.moe else self.mlp(h, sm)
             _, h = sq.layer_norm_residual(x, y, self.norm2, self.eps, dt, next_w=next_w)
         return h
 
@@ -291,6 +290,9 @@ class BazuraxForCausalLM(nn.Module):
         sm = meta.seq
         if sm is None:
             raise ValueError("Bazurax needs the step's per-sequence metadata (AttnMeta.seq)")
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        if sm.tickets is not None:
+            sm.tickets.zero_()
         x, h = sq.layer_norm_residual(None, self.embed, self.embed_norm, self.cfg.norm_eps, self.dtype, ids=input_ids)
         last, keep = len(self.layers) - 1, self.keep_residuals
         for i, (L, lc) in enumerate(zip(self.layers, cache.layers)):
@@ -302,7 +304,7 @@ class BazuraxForCausalLM(nn.Module):
         return h
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.embed)
+        return sq.linear(h, self.embed)
 
     def set_moe_comm(self, mode: str):
         pass

@@ -27,7 +27,6 @@ from typing import Dict, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -71,13 +70,13 @@ class LatentAttentionMixer(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, cache_rows, rot, block_size):
         T, H, dq = h.shape[0], self.H, self.dn + self.rd
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         cq = sq.latent_prep(proj, 0, self.Rq, self.off_kv, self.R, self.rd, self.q_norm, self.kv_norm, self.eps, rot,
                             self.rot_dims, sm, cache_rows)
-        q = F.linear(cq, self.uq).view(T, H, dq)
+        q = sq.linear(cq, self.uq, sm).view(T, H, dq)
         o = sq.latent_attention_heads(q, self.dn, proj[:, self.off_g:], cache_rows, self.uk, self.uv, rot, self.rot_dims,
                                       self.window, self.scale, block_size, sm)
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class DeltaRuleMixer(nn.Module):
@@ -95,11 +94,11 @@ class DeltaRuleMixer(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, state):
         HD = self.HD
-        proj = F.linear(h, self.in_proj)
-        wl = F.linear(sq.tanh_cols(proj, 5 * HD, self.lr), self.w2)
+        proj = sq.linear(h, self.in_proj, sm)
+        wl = sq.linear(sq.tanh_cols(proj, 5 * HD, self.lr), self.w2, sm)
         o = sq.delta_rule_scan(proj, 0, HD, 2 * HD, 4 * HD, wl, self.a_bias, self.w0, state, self.H, self.D, sm)
         y = sq.delta_rule_out(o, self.norm, proj[:, 3 * HD:4 * HD], self.eps, self.H, self.D, h.dtype)
-        return F.linear(y, self.o)
+        return sq.linear(y, self.o, sm)
 
 
 class XieluMLP(nn.Module):
@@ -116,9 +115,9 @@ class XieluMLP(nn.Module):
         p, q = (float(v) for v in self.act.detach().cpu())
         self.sp, self.cn = _softplus(p), 0.5 + _softplus(q)
 
-    def forward(self, h):
+    def forward(self, h, sm: Optional[sq.SeqMeta] = None):
         """W_down act(W_up h + b_up); the down bias is added by the caller's norm."""
-        return F.linear(sq.xielu(F.linear(h, self.up), self.up_b, self.sp, self.cn), self.down)
+        return sq.linear(sq.linear_xielu(h, self.up, self.up_b, self.sp, self.cn, sm), self.down, sm)
 
 
 class DofivikLayer(nn.Module):
@@ -147,7 +146,7 @@ class DofivikLayer(nn.Module):
         sq.scaled_add_rmsnorm(x, y, self.norm1, self.eps, self.alpha, None, 1.0)
         if self.mlp is not None:
             h = sq.causal_conv_residual(x, self.canon2, lc.conv2, sm, dtype)
-            sq.scaled_add_rmsnorm(x, self.mlp(h), self.norm2, self.eps, self.alpha, self.mlp.down_b, 1.0)
+            sq.scaled_add_rmsnorm(x, self.mlp(h, sm), self.norm2, self.eps, self.alpha, self.mlp.down_b, 1.0)
         return x
 
 
@@ -275,7 +274,8 @@ class DofivikForCausalLM(nn.Module):
         sm = meta.seq
         if sm is None:
             raise ValueError("Dofivik needs the step's per-sequence metadata (AttnMeta.seq)")
-        x = sq.embed_rows(input_ids, self.embed)
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        x = sq.embed_rows(input_ids, self.embed, tickets=sm.tickets)
         for L, lc in zip(self.layers, cache.layers):
             rot = self._rot[(L.mix.rot_dims, L.mix.rot_base)] if L.kind == "latent_attention" else None
             x = L(x, sm, lc, rot, cache.block_size, self.dtype)
@@ -284,7 +284,7 @@ class DofivikForCausalLM(nn.Module):
                                      out_dtype=self.dtype)
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head)
+        return sq.linear(h, self.head)
 
     def set_moe_comm(self, mode: str):
         pass

@@ -31,7 +31,6 @@ from typing import Dict, List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -67,12 +66,12 @@ class ConvRopeAttention(nn.Module):
         return (self.rot_dims, self.rot_base, None if sc is None else tuple(sorted((k, float(v)) for k, v in sc.items())))
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int, rot):
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         q = sq.conv_head_norm_rope_cache(proj, self.conv_w, lc.mix_conv, self.H, self.G, self.dk, self.dv, self.q_norm,
                                          self.k_norm, self.eps, rot, self.rot_dims, sm, lc.k, lc.v)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, sq.MASK_CAUSAL, 0, self.scale, None,
                                 None, block_size, sm, gate=proj[:, self.ch:])
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class TalkingDistanceAttention(nn.Module):
@@ -103,7 +102,7 @@ class TalkingDistanceAttention(nn.Module):
             wide = torch.stack([sq.masked_attention(*args, values=c, **kw).view(-1, H, dv) for c in range(G)], 2)
             wide = wide.reshape(-1, H * G * dv)
         o = sq.talk_mix(wide, self.talk, H, G, dv, gate=proj[:, n:n + H])
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class LowerBoundRecurrence(nn.Module):
@@ -125,7 +124,7 @@ class LowerBoundRecurrence(nn.Module):
         n = self.n
         # the gate's bias is in the projection
         o = sq.lower_bound_recurrence(proj, 0, n, 2 * n, None, self.lower, lc.gla, self.H, self.dk, self.dv, sm)
-        return F.linear(sq.gated_group_norm(o, None, self.norm, self.eps, self.H, proj.dtype), self.o)
+        return sq.linear(sq.gated_group_norm(o, None, self.norm, self.eps, self.H, proj.dtype), self.o, sm)
 
 
 class ParallelMixer(nn.Module):
@@ -139,7 +138,7 @@ class ParallelMixer(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int):
         """The two branch outputs (their norms and mean join the residual update)."""
-        proj = F.linear(h, self.in_proj, self.in_bias)
+        proj = sq.linear(h, self.in_proj, sm, self.in_bias)
         return self.left(proj[:, :self.left.rows], sm, lc, block_size), self.right(proj[:, self.left.rows:], sm, lc)
 
 
@@ -152,9 +151,9 @@ class Relu2MLP(nn.Module):
         self.down = _p(torch.empty(width, self.ff, device=device, dtype=dtype))
         self.down_b = _p(torch.zeros(width, device=device, dtype=torch.float32))
 
-    def forward(self, h):
+    def forward(self, h, sm: Optional[sq.SeqMeta] = None):
         """W_down relu(W_up h + b)^2; the output bias down_b is added by the residual update."""
-        return F.linear(sq.relu2(F.linear(h, self.up), self.up_b), self.down)
+        return sq.linear(sq.linear_relu2(h, self.up, self.up_b, sm), self.down, sm)
 
 
 class LoluzenLayer(nn.Module):
@@ -187,7 +186,7 @@ class LoluzenLayer(nn.Module):
             n = sq.post_norm_residual(x, ya, None, self.norm1b, self.mult, after[0], after[1], self.eps, dt, y2=yb,
                                       pre_w=(self.mix.left.out_norm, self.mix.right.out_norm))
         if not last:
-            n = sq.post_norm_residual(x, self.mlp(n), self.mlp.down_b, self.norm2b, self.mult, extra, next_norm,
+            n = sq.post_norm_residual(x, self.mlp(n, sm), self.mlp.down_b, self.norm2b, self.mult, extra, next_norm,
                                       self.eps, dt)
         return n
 
@@ -325,7 +324,8 @@ class LoluzenForCausalLM(nn.Module):
         if sm is None:
             raise ValueError("Loluzen needs the step's per-sequence metadata (AttnMeta.seq)")
         cfg, eps = self.cfg, self.cfg.norm_eps
-        x = sq.embed_rows(input_ids, self.embed, scale=cfg.embed_scale)
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        x = sq.embed_rows(input_ids, self.embed, scale=cfg.embed_scale, tickets=sm.tickets)
         e = x.clone() if self.pass_starts else None
         n = sq.post_norm_residual(x, None, None, None, 0.0, None, self.layers[self.runs[0]].norm1, eps, self.dtype)
         last = len(self.runs) - 1
@@ -345,7 +345,7 @@ class LoluzenForCausalLM(nn.Module):
         return n
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head)
+        return sq.linear(h, self.head)
 
     def set_moe_comm(self, mode: str):
         pass

@@ -30,7 +30,6 @@ from typing import Dict, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -61,8 +60,8 @@ class MinGRUMixer(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache):
         n = self.n
-        proj = F.linear(h, self.in_proj)
-        return F.linear(sq.mingru_scan(proj, 0, n, 2 * n, n, self.z_b, self.x_b, lc.gru, sm, h.dtype), self.o)
+        proj = sq.linear(h, self.in_proj, sm)
+        return sq.linear(sq.mingru_scan(proj, 0, n, 2 * n, n, self.z_b, self.x_b, lc.gru, sm, h.dtype), self.o, sm)
 
 
 class WindowSinkAttention(nn.Module):
@@ -86,13 +85,13 @@ class WindowSinkAttention(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int, rot, v_first):
         """(output, this layer's own projected values as a view of the fused projection)."""
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         own = proj[:, self.nq + self.nk:self.ch]
         q = sq.head_norm_rope_cache(proj, self.H, self.G, self.dk, self.dv, None, None, 0.0, rot, self.rot_dims, sm, lc.k,
                                     lc.v, h.dtype, half=True, v_first=v_first, v_mix=self.lam if v_first is not None else None)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, self.mask, self.size, self.scale, None,
                                 self.sink, block_size, sm, gate=proj[:, self.ch:], gate_elem=True)
-        return F.linear(o, self.o), own
+        return sq.linear(o, self.o, sm), own
 
 
 class SigmoidAttention(nn.Module):
@@ -119,7 +118,7 @@ class SigmoidAttention(nn.Module):
                                     self.rot_dims, sm, lc.k, lc.v, proj.dtype, whole=True)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, sq.MASK_CAUSAL, 0, self.scale, None, None,
                                 block_size, sm, weights=sq.W_SIGMOID, score_bias=self.pb)
-        return F.linear(o, self.o, self.o_b)
+        return sq.linear(o, self.o, sm, self.o_b)
 
 
 class DecayedLinearAttention(nn.Module):
@@ -141,12 +140,12 @@ class DecayedLinearAttention(nn.Module):
 
     def forward(self, proj, sm: sq.SeqMeta, lc: LayerCache):
         n, nv = self.n, self.nv
-        z = F.linear(proj[:, 2 * n + 2 * nv:], self.a2)
+        z = sq.linear(proj[:, 2 * n + 2 * nv:], self.a2, sm)
         q, f, k = sq.decay_gates(proj, 0, n, n, self.dk ** -0.5, z, self.a2_b, self.tau)
         o = sq.gated_linear_scan(q, f, k, proj[:, 2 * n:2 * n + nv], lc.gla, self.H, self.dk, self.dv, sm)
         y = sq.gated_group_norm(o, proj[:, 2 * n + nv:2 * n + 2 * nv], self.norm, self.eps, self.H, proj.dtype,
                                 gate_after=True)
-        return F.linear(y, self.o)
+        return sq.linear(y, self.o, sm)
 
 
 class ParallelMixer(nn.Module):
@@ -160,7 +159,7 @@ class ParallelMixer(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int, rot):
         """The two branch outputs (their norms and mean join the residual update)."""
-        proj = F.linear(h, self.in_proj, self.in_bias)
+        proj = sq.linear(h, self.in_proj, sm, self.in_bias)
         return (self.left(proj[:, :self.left.rows], sm, lc, block_size, rot),
                 self.right(proj[:, self.left.rows:], sm, lc))
 
@@ -325,7 +324,8 @@ class LotelixForCausalLM(nn.Module):
         if sm is None:
             raise ValueError("Lotelix needs the step's per-sequence metadata (AttnMeta.seq)")
         cfg, eps, groups, dt = self.cfg, self.cfg.norm_eps, self.cfg.norm_groups, self.dtype
-        x = sq.embed_rows(input_ids, self.embed, scale=cfg.embed_scale)
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        x = sq.embed_rows(input_ids, self.embed, scale=cfg.embed_scale, tickets=sm.tickets)
         first = self.layers[0]
         n32, n = sq.residual_norm(x, None, None, None, None, None, first.norm1, eps, dt, False, groups)
         v_first, last, keep = None, len(self.layers) - 1, self.keep_residuals
@@ -354,7 +354,7 @@ class LotelixForCausalLM(nn.Module):
         return n
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head)
+        return sq.linear(h, self.head)
 
     def set_moe_comm(self, mode: str):
         pass

@@ -25,7 +25,6 @@ from typing import Dict, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -66,7 +65,7 @@ class WindowKeepAttention(nn.Module):
         self.o = _p(e(width, self.H * self.dv))
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int, rot):
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         if self.kv_from is None:
             q = sq.head_norm_rope_cache(proj, self.H, self.G, self.dk, self.dv, None, None, 0.0, rot, self.rot_dims, sm,
                                         lc.k, lc.v, h.dtype)
@@ -77,7 +76,7 @@ class WindowKeepAttention(nn.Module):
             q = proj
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, self.mask, self.size, self.scale, None,
                                 None, block_size, sm, softcap=self.softcap, keep_first=self.keep)
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class SoftmaxRouterMoE(nn.Module):
@@ -94,13 +93,13 @@ class SoftmaxRouterMoE(nn.Module):
         # router rows, then (with a shared expert) the row of its gate
         self.router = _p(torch.zeros(self.E + (1 if sh else 0), width, device=device, dtype=torch.float32))
 
-    def forward(self, n32, nact):
+    def forward(self, n32, nact, sm: Optional[sq.SeqMeta] = None):
         """(shared expert's output or None, its gate per token or None, the routed experts' rows)."""
         ids, wts, gate = sq.grouped_router(None, None, self.count, self.keep, self.top, 1.0, rows=n32, router_w=self.router,
                                            score=sq.SCORE_SOFTMAX, rating=sq.RATE_MAX, extra_gate=self.shared is not None,
                                            want_gate=True)
         y3 = sq.routed_experts(nact, self.w13, self.w2, ids, wts, sq.GLU_CLAMPED, self.limit, GLU_ALPHA, combine=False)
-        return (self.shared(nact) if self.shared is not None else None), gate, y3
+        return (self.shared(nact, sm) if self.shared is not None else None), gate, y3
 
 
 class TaritarLayer(nn.Module):
@@ -222,7 +221,8 @@ class TaritarForCausalLM(nn.Module):
         if sm is None:
             raise ValueError("Taritar needs the step's per-sequence metadata (AttnMeta.seq)")
         eps, dt, S, last, keep = self.cfg.norm_eps, self.dtype, self.cfg.streams, len(self.layers) - 1, self.keep_residuals
-        x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions, self.cfg.embed_scale)
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions, self.cfg.embed_scale, tickets=sm.tickets)
         first = self.layers[0]
         x, n32, n = sq.hyper_residual(x, S, None, None, None, None, first.hc1.w_in, first.norm1, eps, dt)
         for i, (L, lc) in enumerate(zip(self.layers, cache.layers)):
@@ -233,7 +233,7 @@ class TaritarForCausalLM(nn.Module):
             x, n32, n = sq.hyper_residual(x, S, y, None, L.hc1.w_out, L.hc1.mix, *after, eps, dt, want_f32=L.moe,
                                           store=L.mlp is not None or i < last or keep is not None)
             if L.mlp is not None:
-                y1, gate, y3 = L.mlp(n32, n) if L.moe else (L.mlp(n), None, None)
+                y1, gate, y3 = L.mlp(n32, n, sm) if L.moe else (L.mlp(n, sm), None, None)
                 x, n32, n = sq.hyper_residual(x, S, y1, y3, L.hc2.w_out, L.hc2.mix, *nxt, eps, dt, y_gate=gate,
                                               store=i < last or keep is not None)
             if keep is not None:
@@ -241,7 +241,7 @@ class TaritarForCausalLM(nn.Module):
         return n
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        logits = F.linear(h, self.head)
+        logits = sq.linear(h, self.head)
         return sq.soft_cap_(logits, self.cfg.logit_softcap) if self.cfg.logit_softcap else logits
 
     def set_moe_comm(self, mode: str):

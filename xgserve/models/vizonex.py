@@ -61,11 +61,11 @@ class ChunkedSinkAttention(nn.Module):
         self.o = _p(e(width, self.H * self.dv))
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int):
-        proj = F.linear(h, self.qkv)
+        proj = sq.linear(h, self.qkv, sm)
         q = sq.qk_norm_cache(proj, self.nq, self.nk, self.nv, self.q_norm, self.k_norm, self.eps, sm, lc.k, lc.v)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, sq.MASK_CHUNK, self.size, self.scale,
                                 self.temp, self.sink, block_size, sm)
-        return F.linear(o, self.o)
+        return sq.linear(o, self.o, sm)
 
 
 class SelectiveStateSpace(nn.Module):
@@ -85,12 +85,12 @@ class SelectiveStateSpace(nn.Module):
 
     def forward(self, h, sm: sq.SeqMeta, lc: LayerCache, block_size: int):
         inner, ch = self.inner, self.ch
-        proj = F.linear(h, self.in_proj)
+        proj = sq.linear(h, self.in_proj, sm)
         xbc = sq.causal_conv(proj[:, inner:inner + ch], self.conv_w, self.conv_b, lc.mix_conv, sm, h.dtype, residual=False,
                              silu=True)
         y = sq.ssm_scan(xbc, proj[:, inner + ch:], self.dt_bias, self.A_log, self.D, lc.ssm, self.H, self.G, self.N,
                         self.P, sm)
-        return F.linear(sq.gated_group_norm(y, proj[:, :inner], self.norm, self.eps, self.ng, h.dtype), self.o)
+        return sq.linear(sq.gated_group_norm(y, proj[:, :inner], self.norm, self.eps, self.ng, h.dtype), self.o, sm)
 
 
 class GatedMLP(nn.Module):
@@ -102,8 +102,8 @@ class GatedMLP(nn.Module):
         self.gate_up = _p(torch.empty(2 * self.ff, width, device=device, dtype=dtype))   # rows [gate | up]
         self.down = _p(torch.empty(width, self.ff, device=device, dtype=dtype))
 
-    def forward(self, h):
-        return F.linear(sq.glu_act(F.linear(h, self.gate_up), self.kind, self.limit, GLU_ALPHA), self.down)
+    def forward(self, h, sm: Optional[sq.SeqMeta] = None):
+        return sq.linear(sq.linear_glu(h, self.gate_up, self.kind, self.limit, GLU_ALPHA, sm), self.down, sm)
 
 
 class GroupedRouterMoE(nn.Module):
@@ -121,12 +121,12 @@ class GroupedRouterMoE(nn.Module):
         sh = mlp.get("shared")
         self.shared = GatedMLP(width, sh["ff"], sq.GLU_CLAMPED, sh["limit"], device, dtype) if sh is not None else None
 
-    def forward(self, n32, nact):
+    def forward(self, n32, nact, sm: Optional[sq.SeqMeta] = None):
         """(shared expert's output as an activation tensor or None, routed sum fp32)."""
         ids, wts = sq.grouped_router(F.linear(n32, self.router), self.correction, self.count, self.keep, self.top,
                                      self.rscale)
         routed = sq.routed_experts(nact, self.w13, self.w2, ids, wts, sq.GLU_CLAMPED, self.limit, GLU_ALPHA)
-        return (self.shared(nact) if self.shared is not None else None), routed
+        return (self.shared(nact, sm) if self.shared is not None else None), routed
 
 
 class VizonexLayer(nn.Module):
@@ -156,9 +156,9 @@ class VizonexLayer(nn.Module):
         y2 = y3 = None
         if self.mlp is not None:
             if self.moe:
-                y2, y3 = self.mlp(n32, nact)
+                y2, y3 = self.mlp(n32, nact, sm)
             else:
-                y2 = self.mlp(nact)
+                y2 = self.mlp(nact, sm)
         n32, nact = sq.residual_norm(x, y1, self.ls1, y2, y3, self.ls2, next_norm, self.eps, nact.dtype, want_f32)
         return x, n32, nact
 
@@ -268,7 +268,8 @@ class VizonexForCausalLM(nn.Module):
         sm = meta.seq
         if sm is None:
             raise ValueError("Vizonex needs the step's per-sequence metadata (AttnMeta.seq)")
-        x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions)
+        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions, tickets=sm.tickets)
         n32, nact = sq.residual_norm(x, None, None, None, None, None, self.layers[0].norm1, self.cfg.norm_eps,
                                      self.dtype, True)
         last = len(self.layers) - 1
@@ -279,7 +280,7 @@ class VizonexForCausalLM(nn.Module):
         return nact
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head)
+        return sq.linear(h, self.head)
 
     def set_moe_comm(self, mode: str):
         pass

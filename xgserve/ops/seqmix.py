@@ -17,6 +17,7 @@ from dataclasses import dataclass
 from typing import Optional
 
 import torch
+import torch.nn.functional as F
 
 from .. import tune
 from ._native import is_f32, mixers, native_device, stream_ptr
@@ -34,6 +35,8 @@ class SeqMeta:
     token_seq: torch.Tensor      # int32 [T]
     positions: torch.Tensor      # int32 [T]
     slot_mapping: torch.Tensor   # int32 [T]
+    # words that are zero between the step's launches, for products whose parts meet (`step_tickets`)
+    tickets: Optional[torch.Tensor] = None
 
 
 def _p(t: Optional[torch.Tensor]) -> int:
@@ -47,9 +50,10 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
 
 # ---------------------------------------------------------------------------- embedding
 def embed_rows(ids: torch.Tensor, table: torch.Tensor, pos_table: Optional[torch.Tensor] = None,
-               positions: Optional[torch.Tensor] = None, scale: float = 1.0) -> torch.Tensor:
+               positions: Optional[torch.Tensor] = None, scale: float = 1.0,
+               tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """fp32 rows table[ids] * scale (zero rows for ids outside the table); with `pos_table` the learned vector
-    pos_table[positions] is added (unscaled)."""
+    pos_table[positions] is added (unscaled). `tickets` (`step_tickets`) are cleared by the same launch."""
     V, W = table.shape
     if not native_device(table):
         ok = (ids >= 0) & (ids < V)
@@ -66,8 +70,105 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, pos_table: Optional[torch
         assert pos_table.dtype == table.dtype and pos_table.shape[1] == W and pos_table.is_contiguous()
     mixers().embed_rows(_i32(ids).data_ptr(), table.data_ptr(), is_f32(table), out.data_ptr(), ids.shape[0], W, V,
                         _p(pos_table), _i32(positions).data_ptr() if pos_table is not None else 0,
-                        pos_table.shape[0] if pos_table is not None else 0, float(scale), stream_ptr())
+                        pos_table.shape[0] if pos_table is not None else 0, float(scale), _p(tickets),
+                        tickets.numel() if tickets is not None else 0, stream_ptr())
     return out
+
+
+# ---------------------------------------------------------------------------- products of a few rows
+ROWS_LINEAR = True
+ROWS_LINEAR_MAX = 64       # rows (four 16-row tiles of x in the registers of a wave)
+# Sizes of a workgroup's share (us, cold weights, 64 rows of x): 64 weight rows while that makes at most one workgroup per
+# compute unit, 128 beyond (14336x4096 25.1 narrow against 35.9 wide, 18560x4096 43.5 against 36.9).
+_ROWS_WGS = 256
+# K in as many parts as keep the grid within _ROWS_WGS, at most 8, each of 512 or more: 2048x2048 12.2 / 10.4 / 8.6 / 9.1 in
+# 1 / 2 / 4 / 8 parts, 2048x8192 39.8 / 25.1 / 17.3 / 13.8, 8192x2048 13.6 / 13.0 / 15.7 in 1 / 2 / 4 (the last part of a
+# tile adds the slabs by itself).
+_ROWS_PARTS, _ROWS_PART_K = 8, 512
+_ROWS_TICKETS = _ROWS_WGS // 2     # column tiles of a product in parts
+
+ACT_NONE, ACT_XIELU, ACT_RELU2, ACT_GLU = 0, 1, 2, 3   # ACT_GLU + GLU_...: the gated activations
+
+
+def step_tickets(like: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
+    """Words for the products of a step of `rows` rows on `like`'s device, uncleared (embed_rows clears them), or None
+    where no product of the step takes them. They belong to the step (SeqMeta.tickets): launches of one stream follow each
+    other, and each leaves the words zero."""
+    if not (ROWS_LINEAR and native_device(like) and like.dtype == torch.bfloat16 and rows <= ROWS_LINEAR_MAX):
+        return None
+    return torch.empty(_ROWS_TICKETS, dtype=torch.int32, device=like.device)
+
+
+def _rows_plan(N: int, K: int, gated: bool):
+    """(wide, parts of K) of an [N, K] product."""
+    wide = gated or N > 64 * _ROWS_WGS
+    tiles, S = -(-N // (128 if wide else 64)), 1
+    while 2 * S * tiles <= _ROWS_WGS and 2 * S <= _ROWS_PARTS and 2 * S * _ROWS_PART_K <= K:
+        S *= 2
+    return wide, S
+
+
+def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool):
+    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
+    pieces, K in whole staged rows, and tickets where K is in parts (clearing them would cost what the parts gain)."""
+    if not (ROWS_LINEAR and native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and 1 <= x.shape[0] <= ROWS_LINEAR_MAX):
+        return None
+    N, K = w.shape
+    if K < 128 or K % 128 or x.shape[1] != K or N < 1 or N % (8 if gated else 4) or not w.is_contiguous() or \
+            x.stride(1) != 1 or x.stride(0) % 8 or (x.data_ptr() | w.data_ptr()) % 16:
+        return None
+    if bias is not None and not (bias.dtype in (torch.float32, torch.bfloat16) and bias.shape == (N,) and
+                                 bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+        return None
+    plan = _rows_plan(N, K, gated)
+    return plan if plan[1] == 1 or (sm is not None and sm.tickets is not None) else None
+
+
+def _rows_linear(plan, x, w, sm, bias, act, p0, p1) -> torch.Tensor:
+    T, (N, K), (wide, S) = x.shape[0], w.shape, plan
+    out = torch.empty(T, N // 2 if act >= ACT_GLU else N, dtype=x.dtype, device=x.device)
+    part = torch.empty(S * T * N, dtype=torch.float32, device=x.device) if S > 1 else None
+    mixers().rows_linear(x.data_ptr(), x.stride(0), w.data_ptr(), _p(bias), bias is not None and is_f32(bias), _p(part),
+                         out.data_ptr(), _p(sm.tickets) if S > 1 else 0, T, N, K, S, act, float(p0), float(p1), wide,
+                         stream_ptr())
+    return out
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None,
+           bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [T, K] . w [N, K]^T + bias."""
+    plan = _rows_plan_of(x, w, sm, bias, False)
+    if plan is not None:
+        return _rows_linear(plan, x, w, sm, bias, ACT_NONE, 0.0, 0.0)
+    return F.linear(x, w, bias)
+
+
+def linear_xielu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], sp: float, cn: float,
+                 sm: Optional[SeqMeta] = None) -> torch.Tensor:
+    """xielu(x . w^T, bias, sp, cn) (bias fp32 per column)."""
+    plan = _rows_plan_of(x, w, sm, bias, False)
+    if plan is not None:
+        return _rows_linear(plan, x, w, sm, bias, ACT_XIELU, sp, cn)
+    return xielu(F.linear(x, w), bias, sp, cn)
+
+
+def linear_relu2(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                 sm: Optional[SeqMeta] = None) -> torch.Tensor:
+    """relu2(x . w^T, bias) (bias fp32 per column)."""
+    plan = _rows_plan_of(x, w, sm, bias, False)
+    if plan is not None:
+        return _rows_linear(plan, x, w, sm, bias, ACT_RELU2, 0.0, 0.0)
+    return relu2(F.linear(x, w), bias)
+
+
+def linear_glu(x: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.702,
+               sm: Optional[SeqMeta] = None) -> torch.Tensor:
+    """glu_act(x . w^T, kind, limit, alpha) of w's rows [gate | up]."""
+    plan = _rows_plan_of(x, w, sm, None, True)
+    if plan is not None:
+        return _rows_linear(plan, x, w, sm, None, ACT_GLU + kind, limit, alpha)
+    return glu_act(F.linear(x, w), kind, limit, alpha)
 
 
 # ---------------------------------------------------------------------------- input convolution
