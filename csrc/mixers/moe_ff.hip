@@ -19,7 +19,7 @@
 //                    gate != nullptr: a logit after the experts' ones, gate[t] = sigmoid(it), takes no part in the
 //                    routing (the gate of an expert that runs for every token).
 //   moe_align        (token, choice) pairs sorted by expert into tiles of `tm` rows (padded with -1); offs: the experts'
-//                    padded starts [E + 1] (what gemm_pf's grouped form walks)
+//                    padded starts [E + 1] (what gemm_pf's grouped form walks); zero[0, nzero) is cleared for later launches
 //   grouped_gemm     per tile: rows x expert weights, in one of three modes:
 //                      kGemmRows    A rows as they lie in the sorted layout -> fp32 rows (the second product)
 //                      kGemmGated   A rows gathered by token; weights [gate | up]; output glu(gate, up)
@@ -233,8 +233,9 @@ __global__ __launch_bounds__(1024) void grouped_router_kernel(const float* __res
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restrict__ ids, int pairs, int E, int cap,
                                                          int kTileM, int32_t* __restrict__ rows,
                                                          int32_t* __restrict__ tile_expert, int32_t* __restrict__ dest,
-                                                         int32_t* __restrict__ offs) {
+                                                         int32_t* __restrict__ offs, int* __restrict__ zero, int nzero) {
   extern __shared__ int si[];
+  for (int i = threadIdx.x; i < nzero; i += blockDim.x) zero[i] = 0;
   int* cnt = si;          // [E]
   int* off = si + E;      // [E + 1] padded starts
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
@@ -331,19 +332,15 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const T* __restrict__
   }
 }
 
-// ---- matrix-core form (bf16; K % 32 == 0, Nout % 16 == 0). A / B fragments come straight from global
-// memory (16 or 32 bytes per lane and step), accumulators are fp32. For steps with few rows per expert (layout
-// tiles of 16 rows). Two shapes of one kernel:
-//   SPLITK = false: a workgroup owns 16 MT rows x 4 x 16 NT columns, each wave 16 NT of the columns over the whole K
-//            (a long loop, four steps' loads in flight);
-//   SPLITK = true:  a workgroup owns 16 rows x 16 NT columns, its four waves a quarter of K each; the partial sums
-//            meet in LDS.
+// ---- matrix-core form for few rows per expert (bf16; K % 32 == 0, Nout % 16 == 0) where K is no multiple of 64
+// (grouped_rows.hip takes the others): a workgroup owns 16 MT rows x 16 NT columns, its four waves a quarter of K each
+// with fragments straight from global memory; the partial sums meet in LDS.
 using xgk::as_frag;
 using xgk::f32x4_t;
 using xgk::ld16;
 using xgk::mfma16x16x32;
 
-template <int MODE, int MT, int NT, bool SPLITK, bool K64>
+template <int MODE, int MT, int NT>
 __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(const bf16* __restrict__ A, int64_t lda,
                                                                 const bf16* __restrict__ Wt,
                                                                 const int32_t* __restrict__ rows,
@@ -353,13 +350,12 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(const bf16* __re
                                                                 const float* __restrict__ row_scale) {
   constexpr bool GATED = MODE == kGemmGated, FIRST = MODE != kGemmRows;
   constexpr int NG = GATED ? NT : 1;
-  __shared__ float red[SPLITK ? 3 : 1][SPLITK ? MT * (NT + NG) : 1][64][4];
+  __shared__ float red[3][MT * (NT + NG)][64][4];
   const int tile = blockIdx.x;          // layout tile of 16 MT rows
   const int e = tile_expert[tile];
   if (e < 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n0 = SPLITK ? blockIdx.y * 16 * NT : (blockIdx.y * 4 + wave) * 16 * NT;
-  if (n0 >= Nout) return;               // (SPLITK: uniform over the workgroup)
+  const int n0 = blockIdx.y * 16 * NT;
   const int l16 = lane & 15, kg = lane >> 4;
   const int64_t wrows = GATED ? 2 * (int64_t)Nout : (int64_t)Nout;
   const bf16* We = Wt + (int64_t)e * wrows * K;
@@ -370,7 +366,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(const bf16* __re
   for (int i = 0; i < MT; ++i) {
     const int pa = rows[rbase + 16 * i + l16];
     aok[i] = pa >= 0;
-    arow[i] = A + (int64_t)(FIRST ? max(pa, 0) / top : rbase + 16 * i + l16) * lda + kg * (K64 ? 16 : 8);
+    arow[i] = A + (int64_t)(FIRST ? max(pa, 0) / top : rbase + 16 * i + l16) * lda + kg * 8;
   }
   f32x4_t acc[MT][NT], accu[MT][NG];
 #pragma unroll
@@ -380,71 +376,58 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(const bf16* __re
 #pragma unroll
     for (int j = 0; j < NG; ++j) accu[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // K64: a lane takes 32 contiguous bytes of a row per step (the four lanes of a row 128 bytes) and feeds them
-  // to two MFMAs. A and B use the same assignment of k to (lane, MFMA), and a sum over k has no order.
-  constexpr int KS = K64 ? 64 : 32, KL = K64 ? 16 : 8;
-  const int kper = SPLITK ? ((K / KS + 3) / 4) * KS : K;
-  const int kbeg = SPLITK ? wave * kper : 0, kend = min(K, kbeg + kper);
-#pragma unroll(SPLITK ? 2 : 4)
-  for (int k0 = kbeg; k0 < kend; k0 += KS) {
-    uint4 av[MT][K64 ? 2 : 1], bv[NT][K64 ? 2 : 1], uv[NG][K64 ? 2 : 1];
+  const int kper = (K / 32 + 3) / 4 * 32, kbeg = wave * kper, kend = min(K, kbeg + kper);
+#pragma unroll 2
+  for (int k0 = kbeg; k0 < kend; k0 += 32) {
+    uint4 av[MT], bv[NT], uv[NG];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int h = 0; h < (K64 ? 2 : 1); ++h)
-        av[i][h] = aok[i] ? ld16(arow[i] + k0 + 8 * h) : make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < MT; ++i) av[i] = aok[i] ? ld16(arow[i] + k0) : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int n = min(n0 + 16 * j, Nout - 16) + l16;  // whole 16-column tiles (Nout % 16 == 0); clamped ones are not stored
-#pragma unroll
-      for (int h = 0; h < (K64 ? 2 : 1); ++h) {
-        bv[j][h] = ld16(We + (int64_t)n * K + k0 + kg * KL + 8 * h);
-        if (GATED) uv[j][h] = ld16(We + (int64_t)(Nout + n) * K + k0 + kg * KL + 8 * h);
-      }
+      bv[j] = ld16(We + (int64_t)n * K + k0 + kg * 8);
+      if (GATED) uv[j] = ld16(We + (int64_t)(Nout + n) * K + k0 + kg * 8);
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        // D = A (rows x k) B (k x cols): accumulator entry r of lane (l16, kg) is row kg * 4 + r, column l16
+        acc[i][j] = mfma16x16x32(as_frag(av[i]), as_frag(bv[j]), acc[i][j]);
+        if (GATED) accu[i][j] = mfma16x16x32(as_frag(av[i]), as_frag(uv[j]), accu[i][j]);
+      }
+  }
+  // waves 1..3 hand their partial sums to wave 0
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int h = 0; h < (K64 ? 2 : 1); ++h) {
-          // D = A (rows x k) B (k x cols): accumulator entry r of lane (l16, kg) is row kg * 4 + r, column l16
-          acc[i][j] = mfma16x16x32(as_frag(av[i][h]), as_frag(bv[j][h]), acc[i][j]);
-          if (GATED) accu[i][j] = mfma16x16x32(as_frag(av[i][h]), as_frag(uv[j][h]), accu[i][j]);
-        }
-  }
-  if (SPLITK) {  // waves 1..3 hand their partial sums to wave 0
-    if (wave > 0) {
+        for (int r = 0; r < 4; ++r) red[wave - 1][i * (NT + NG) + j][lane][r] = acc[i][j][r];
+      if (GATED) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
+        for (int j = 0; j < NG; ++j)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) red[wave - 1][i * (NT + NG) + j][lane][r] = acc[i][j][r];
-        if (GATED) {
-#pragma unroll
-          for (int j = 0; j < NG; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave - 1][i * (NT + NG) + NT + j][lane][r] = accu[i][j][r];
-        }
+          for (int r = 0; r < 4; ++r) red[wave - 1][i * (NT + NG) + NT + j][lane][r] = accu[i][j][r];
       }
     }
-    __syncthreads();
-    if (wave > 0) return;
+  }
+  __syncthreads();
+  if (wave > 0) return;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
+  for (int w = 0; w < 3; ++w) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < MT; ++i) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] += red[w][i * (NT + NG) + j][lane][r];
-        if (GATED) {
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += red[w][i * (NT + NG) + j][lane][r];
+      if (GATED) {
 #pragma unroll
-          for (int j = 0; j < NG; ++j)
+        for (int j = 0; j < NG; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) accu[i][j][r] += red[w][i * (NT + NG) + NT + j][lane][r];
-        }
+          for (int r = 0; r < 4; ++r) accu[i][j][r] += red[w][i * (NT + NG) + NT + j][lane][r];
       }
     }
   }
@@ -592,6 +575,24 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_lds_kernel(const bf16* 
     }
 }
 
+// four columns per thread, T x ceil(W / 1024) workgroups
+__global__ __launch_bounds__(256) void moe_combine4_kernel(const float* __restrict__ y, const int32_t* __restrict__ dest,
+                                                           const float* __restrict__ wts, int top, int W,
+                                                           float* __restrict__ out) {
+  const int t = blockIdx.x, c = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (c >= W) return;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int j = 0; j < top; ++j) {
+    const float w = wts ? wts[(int64_t)t * top + j] : 1.f;
+    float v[4];
+    ld4(y + (int64_t)dest[(int64_t)t * top + j] * W + c, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += w * v[e];
+  }
+  st4(out + (int64_t)t * W + c, acc);
+}
+
 __global__ void moe_combine_kernel(const float* __restrict__ y, const int32_t* __restrict__ dest,
                                    const float* __restrict__ wts, int top, int W, float* __restrict__ out) {
   const int t = blockIdx.x;
@@ -644,13 +645,18 @@ int grouped_router(const float* logits, const float* corr, int T_, int E, int co
 }
 
 int moe_align(const int32_t* ids, int pairs, int E, int cap, int tm, int32_t* rows, int32_t* tile_expert, int32_t* dest,
-              int32_t* offs, hipStream_t st) {
+              int32_t* offs, int* zero, int nzero, hipStream_t st) {
   if (pairs <= 0) return 0;
   if (E < 1 || E > 4096 || tm < 16 || tm % 16 != 0 || cap % tm != 0 || cap < pairs + E * (tm - 1)) return -1;
   moe_align_kernel<<<1, 1024, (2 * E + 1) * sizeof(int), st>>>(ids, pairs, E, cap, tm, rows, tile_expert, dest,
-                                                                   offs);
+                                                                   offs, zero, zero ? nzero : 0);
   return 0;
 }
+
+// grouped_rows.hip
+int grouped_rows(const void* A, int64_t lda, const void* w, const int32_t* rows, const int32_t* tile_expert, int cap, int tm,
+                 int top, int N, int K, int mode, void* out, int kind, float limit, float alpha, const float* row_scale,
+                 hipStream_t st);
 
 int grouped_gemm(const void* A, bool f32, int64_t lda, const void* Wt, const int32_t* rows, const int32_t* tile_expert,
                  int cap, int tm, int top, int Nout, int K, int mode, void* out, int kind, float limit, float alpha,
@@ -661,16 +667,16 @@ int grouped_gemm(const void* A, bool f32, int64_t lda, const void* Wt, const int
       (row_scale && mode != kGemmAct))
     return -1;
   if (!f32 && mfma && K % 32 == 0 && Nout % 16 == 0 && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)Wt % 16 == 0) {
-  // few rows per expert: layout tiles of 16 rows, or of 32 once many experts would fill more than one such tile (an
-  // expert's weights are then streamed once instead of once per 16 rows)
-#define XGM_GG2(MODE, MT, K64)                                                                                      \
-  grouped_gemm_mfma_kernel<MODE, MT, 2, true, K64><<<dim3(cap / tm, (Nout + 31) / 32), 256, 0, st>>>(                \
+    if (tm <= 64 && K % 64 == 0)
+      return grouped_rows(A, lda, Wt, rows, tile_expert, cap, tm, top, Nout, K, mode, out, kind, limit, alpha, row_scale, st);
+#define XGM_GG2(MODE, MT)                                                                           \
+  grouped_gemm_mfma_kernel<MODE, MT, 2><<<dim3(cap / tm, (Nout + 31) / 32), 256, 0, st>>>(          \
       (const bf16*)A, lda, (const bf16*)Wt, rows, tile_expert, top, Nout, K, out, kind, limit, alpha, row_scale);
-#define XGM_GG(MODE, K64)     \
-  if (tm == 32) {             \
-    XGM_GG2(MODE, 2, K64)     \
-  } else {                    \
-    XGM_GG2(MODE, 1, K64)     \
+#define XGM_GG(MODE)     \
+  if (tm == 32) {        \
+    XGM_GG2(MODE, 2)     \
+  } else {               \
+    XGM_GG2(MODE, 1)     \
   }
 #define XGM_GL2(MODE, MT, NT, KS, PF)                                                                                  \
   grouped_gemm_mfma_lds_kernel<MODE, MT, NT, KS, PF>                                                                   \
@@ -686,10 +692,8 @@ int grouped_gemm(const void* A, bool f32, int64_t lda, const void* Wt, const int
       if (mode == kGemmGated) { XGM_GL(kGemmGated, 4, 2) } else if (mode == kGemmAct) { XGM_GL(kGemmAct, 8, 2) } else { XGM_GL(kGemmRows, 8, 2) }
     } else if (tm == 64) {   // gated: 64 x 128; one weight block: 64 x 256
       if (mode == kGemmGated) { XGM_GL(kGemmGated, 4, 2) } else if (mode == kGemmAct) { XGM_GL(kGemmAct, 4, 4) } else { XGM_GL(kGemmRows, 4, 4) }
-    } else if (K % 64 == 0) {
-      if (mode == kGemmGated) { XGM_GG(kGemmGated, true) } else if (mode == kGemmAct) { XGM_GG(kGemmAct, true) } else { XGM_GG(kGemmRows, true) }
     } else {
-      if (mode == kGemmGated) { XGM_GG(kGemmGated, false) } else if (mode == kGemmAct) { XGM_GG(kGemmAct, false) } else { XGM_GG(kGemmRows, false) }
+      if (mode == kGemmGated) { XGM_GG(kGemmGated) } else if (mode == kGemmAct) { XGM_GG(kGemmAct) } else { XGM_GG(kGemmRows) }
     }
 #undef XGM_GL
 #undef XGM_GL2
@@ -709,6 +713,10 @@ int grouped_gemm(const void* A, bool f32, int64_t lda, const void* Wt, const int
 
 void moe_combine(const float* y, const int32_t* dest, const float* wts, int T_, int top, int W, float* out, hipStream_t st) {
   if (T_ <= 0) return;
+  if (W % 4 == 0 && W <= 1024 * 65535 && ((uintptr_t)y | (uintptr_t)out) % 16 == 0) {
+    moe_combine4_kernel<<<dim3(T_, (W / 4 + 255) / 256), 256, 0, st>>>(y, dest, wts, top, W, out);
+    return;
+  }
   moe_combine_kernel<<<T_, 256, 0, st>>>(y, dest, wts, top, W, out);
 }
 

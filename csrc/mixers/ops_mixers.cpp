@@ -70,7 +70,7 @@ int hyper_residual(const float*, bool, float*, int, const void*, int64_t, bool, 
                    const float*, int, const float*, const float*, const float*, const float*, float, float*, void*, bool,
                    int, int, hipStream_t);
 void soft_cap(void*, bool, float, int64_t, hipStream_t);
-int moe_align(const int32_t*, int, int, int, int, int32_t*, int32_t*, int32_t*, int32_t*, hipStream_t);
+int moe_align(const int32_t*, int, int, int, int, int32_t*, int32_t*, int32_t*, int32_t*, int*, int, hipStream_t);
 int grouped_gemm(const void*, bool, int64_t, const void*, const int32_t*, const int32_t*, int, int, int, int, int, int, void*,
                  int, float, float, const float*, bool, hipStream_t);
 int mingru_scan(const void*, bool, int64_t, int, int, int, int, const float*, const float*, float*, const int32_t*,
@@ -377,9 +377,9 @@ PYBIND11_MODULE(_mixers, m) {
     check(rc, "grouped_router");
   });
   m.def("moe_align", [](uintptr_t ids, int pairs, int E, int cap, int tm, uintptr_t rows, uintptr_t tile_expert,
-                        uintptr_t dest, uintptr_t offs, uintptr_t st) {
+                        uintptr_t dest, uintptr_t offs, uintptr_t zero, int nzero, uintptr_t st) {
     int rc = xgm::moe_align(P<const int32_t>(ids), pairs, E, cap, tm, P<int32_t>(rows), P<int32_t>(tile_expert),
-                            P<int32_t>(dest), P<int32_t>(offs), S(st));
+                            P<int32_t>(dest), P<int32_t>(offs), P<int>(zero), nzero, S(st));
     check(rc, "moe_align");
   });
   m.def("grouped_gemm", [](uintptr_t A, bool f32, int64_t lda, uintptr_t Wt, uintptr_t rows, uintptr_t tile_expert, int cap,

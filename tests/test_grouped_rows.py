@@ -1,0 +1,64 @@
+"""Sorted rows times their experts' weights (the grouped GEMM for few rows per expert) against fp64.
+
+Tolerance: products of bf16 inputs are exact in fp32, a sum of K of them errs by at most K 2^-24 of the sum of magnitudes;
+the gated and squared results are rounded once to bf16 (2^-8 of their size), with the activation's slope in front of the sum's
+error."""
+import pytest
+import torch
+
+from xgserve.ops import seqmix as sq
+from xgserve.ops._native import mixers, stream_ptr
+
+pytestmark = pytest.mark.gpu
+
+
+def run(x, w, rows, tile_e, tm, top, N, K, mode, kind=0, limit=0.0, scale=None):
+    out = torch.full((rows.numel(), N), -7.0, device="cuda", dtype=torch.float32 if mode == 0 else torch.bfloat16)
+    mixers().grouped_gemm(x.data_ptr(), False, x.stride(0), w.data_ptr(), rows.data_ptr(), tile_e.data_ptr(), rows.numel(), tm,
+                          top, N, K, mode, out.data_ptr(), kind, limit, 1.702, 0 if scale is None else scale.data_ptr(), True,
+                          stream_ptr())
+    return out
+
+
+@pytest.mark.parametrize("tm", [16, 32, 64])
+@pytest.mark.parametrize("N,K", [(16, 64), (80, 192), (208, 1024), (2064, 320)])
+@pytest.mark.parametrize("T,E,top", [(1, 3, 2), (16, 4, 1), (33, 5, 2), (150, 2, 1)])
+def test_modes(tm, N, K, T, E, top):
+    g = torch.Generator().manual_seed(T + N)
+    h = torch.randn(T, K + 8, generator=g).bfloat16().cuda()[:, :K]           # rows of a wider tensor
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).cuda()
+    if E > 2:
+        ids[ids == E - 1] = 0                                                 # an expert without rows
+    pairs = T * top
+    cap = (pairs + E * (tm - 1) + tm - 1) // tm * tm
+    i32 = dict(dtype=torch.int32, device="cuda")
+    rows, tile_e, dest = torch.empty(cap, **i32), torch.empty(cap // tm, **i32), torch.empty(pairs, **i32)
+    words = torch.full((9,), 5, **i32)
+    mixers().moe_align(ids.data_ptr(), pairs, E, cap, tm, rows.data_ptr(), tile_e.data_ptr(), dest.data_ptr(), 0,
+                       words.data_ptr(), 8, stream_ptr())
+    assert words.tolist() == [0] * 8 + [5]
+    e, d = ids.flatten().long(), dest.long()
+    free = torch.ones(cap, dtype=torch.bool, device="cuda")
+    free[d] = False
+    w13 = (torch.randn(E, 2 * N, K, generator=g) / K ** 0.5).bfloat16().cuda()
+    src = h.double()[torch.arange(pairs, device="cuda") // top]
+    z = torch.stack([w13[a].double() @ v for a, v in zip(e, src)])
+    err = K * 2.0 ** -24 * float(torch.stack([w13[a].double().abs() @ v.abs() for a, v in zip(e, src)]).max()) + 2.0 ** -20
+    top_z = float(z.abs().max())
+
+    def check(out, want, slope, bits):
+        assert bool((out[free] == -7).all())                                  # rows without a pair stay as they were
+        assert bool(((out[d].double() - want).abs() <= slope * err + want.abs() * bits).all())
+
+    a, u = z[:, :N], z[:, N:]
+    check(run(h, w13, rows, tile_e, tm, top, N, K, 1, sq.GLU_SILU), a * torch.sigmoid(a) * u, 3 * top_z + 3, 2.0 ** -8)
+    ac, uc = a.clamp(max=1.0), u.clamp(-1.0, 1.0)
+    check(run(h, w13, rows, tile_e, tm, top, N, K, 1, sq.GLU_CLAMPED, 1.0), ac * torch.sigmoid(1.702 * ac) * (uc + 1),
+          3 * top_z + 3, 2.0 ** -8)
+    w1 = w13[:, :N].contiguous()
+    s = (torch.rand(pairs, generator=g) + 0.5).cuda()
+    check(run(h, w1, rows, tile_e, tm, top, N, K, 2, sq.ACT_RELU2, scale=s), (a * s.double()[:, None]).clamp(min=0) ** 2,
+          6 * top_z + 3, 2.0 ** -8)
+    lay = torch.full((cap, K), float("nan"), device="cuda", dtype=torch.bfloat16)   # padding rows may hold anything
+    lay[d] = h[torch.arange(pairs, device="cuda") // top]
+    check(run(lay, w1, rows, tile_e, tm, top, N, K, 0), a, 1.0, 2.0 ** -22)

@@ -32,7 +32,6 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..ops import seqmix as sq
 from ..parallel.state import get_state
@@ -123,10 +122,14 @@ class GroupedRouterMoE(nn.Module):
 
     def forward(self, n32, nact, sm: Optional[sq.SeqMeta] = None):
         """(shared expert's output as an activation tensor or None, routed sum fp32)."""
-        ids, wts = sq.grouped_router(F.linear(n32, self.router), self.correction, self.count, self.keep, self.top,
-                                     self.rscale)
-        routed = sq.routed_experts(nact, self.w13, self.w2, ids, wts, sq.GLU_CLAMPED, self.limit, GLU_ALPHA)
-        return (self.shared(nact, sm) if self.shared is not None else None), routed
+        ids, wts = sq.grouped_router(None, self.correction, self.count, self.keep, self.top, self.rscale, rows=n32,
+                                     router_w=self.router)
+        step, clear = sm, None
+        if self.shared is not None and (sm is None or sm.tickets is None):
+            clear = sq.step_tickets(nact, nact.shape[0])
+            step = sq.StepTickets(clear)
+        routed = sq.routed_experts(nact, self.w13, self.w2, ids, wts, sq.GLU_CLAMPED, self.limit, GLU_ALPHA, clear=clear)
+        return (self.shared(nact, step) if self.shared is not None else None), routed
 
 
 class VizonexLayer(nn.Module):

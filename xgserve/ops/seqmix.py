@@ -99,6 +99,12 @@ def step_tickets(like: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
     return torch.empty(_ROWS_TICKETS, dtype=torch.int32, device=like.device)
 
 
+@dataclass
+class StepTickets:
+    """Stands for a step's SeqMeta where a product in parts runs without one."""
+    tickets: Optional[torch.Tensor]
+
+
 def _rows_plan(N: int, K: int, gated: bool):
     """(wide, parts of K) of an [N, K] product."""
     wide = gated or N > 64 * _ROWS_WGS
@@ -934,9 +940,13 @@ MOE_MFMA = tune.get_bool("moe_mfma", True)
 # XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on the tiles of csrc/mixers (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
 MOE_PF_MIN = 96   # average rows per expert from which gated experts run on gemm_pf's grouped form
-MOE_TILE_SMALL, MOE_TILES_BIG = 16, (128, 64, 32)   # rows per expert tile of the sorted layout
-MOE_TILE32_MIN = 12   # average rows per expert from which 32-row tiles replace 16-row ones (XGS_TUNE moe_tile32_min)
-MOE_TILE32_MIN = tune.get_int("moe_tile32_min", MOE_TILE32_MIN)
+# Rows per expert tile of the sorted layout, and the average rows per expert from which it is taken. Weight-streaming
+# products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
+# us: tiles of 16 104 / 142 / - / 230 / -, 32 112 / 113 / 115 / 175 / 233, 64 121 / 123 / 123 / 127 / 191; 32 experts of
+# 2 x 1024 x 2048 at 8: 72 / 73 / 79. Tiles of 128 belong to the kernel of prompt-sized steps.
+MOE_TILE32_MIN = tune.get_int("moe_tile32_min", 8)
+MOE_TILE_SMALL, MOE_TILES = 16, ((128, 128), (64, 24), (32, MOE_TILE32_MIN))
+MOE_TILES_GENERAL = ((128, 128), (64, 64), (32, 12))   # the other kernels (float32, K of odd 32s): padding costs more there
 
 
 def _glu_ref(g, u, kind, limit, alpha):
@@ -1040,12 +1050,14 @@ class RoutedRows:
 
 
 def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, kind: int,
-                   limit: float = 0.0, alpha: float = 1.702, scale_input: bool = False, combine: bool = True):
+                   limit: float = 0.0, alpha: float = 1.702, scale_input: bool = False, combine: bool = True,
+                   clear: Optional[torch.Tensor] = None):
     """sum_j wts[t, j] * W2[e] glu(W13[e] h_t), e = ids[t, j]. w13 [E, 2 F, K] holds each expert's gate rows then
     its up rows, w2 [E, W, F]. With an ungated `kind` (ACT_RELU2) w13 is [E, F, K] and the expert is W2 act(W13 h).
     `scale_input`: the weight multiplies the expert's INPUT instead of its output, sum_j expert_e(wts[t, j] h_t); the
     first product being linear, the weight is applied to its fp32 accumulator, act(wts * (W13 h)).
-    Returns fp32 [T, W] (a sum in a fixed order per row), or with combine=False the rows as `RoutedRows`."""
+    Returns fp32 [T, W] (a sum in a fixed order per row), or with combine=False the rows as `RoutedRows`. `clear`
+    (`step_tickets`): cleared on the way."""
     T, K = h.shape
     E = w13.shape[0]
     gated = kind in (GLU_GELU_TANH, GLU_CLAMPED, GLU_SILU)
@@ -1071,9 +1083,9 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     assert h.is_contiguous() and w13.is_contiguous() and w2.is_contiguous() and w13.dtype == w2.dtype == h.dtype
     assert wts.dtype == torch.float32 and wts.is_contiguous()
     pairs = T * top
-    # rows of an expert are padded to whole tiles: 128 / 64-row tiles once the average expert has that many; 32-row
-    # tiles once many experts would need a second 16-row tile (their weights would be streamed twice); else 16
-    tm = next((t for t in MOE_TILES_BIG if pairs >= (t if t > 32 else MOE_TILE32_MIN) * E), MOE_TILE_SMALL)
+    # rows of an expert are padded to whole tiles, so that few experts need a second one (which reads the weights again)
+    streams = MOE_MFMA and h.dtype == torch.bfloat16 and K % 64 == 0 and F_ % 64 == 0
+    tm = next((t for t, least in (MOE_TILES if streams else MOE_TILES_GENERAL) if pairs >= least * E), MOE_TILE_SMALL)
     # ... or run on gemm_pf's grouped form: both operands by LDS DMA, 64-row segments, 256-column tiles
     pf = SEQ_MOE_PF and MOE_MFMA and gated and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E and K % 64 == 0 \
         and F_ % 128 == 0 and W % 256 == 0
@@ -1084,7 +1096,7 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     meta = torch.empty(cap + cap // tm + pairs + E + 1, dtype=torch.int32, device=dev)
     rows, tile_e, dest, offs = meta.split((cap, cap // tm, pairs, E + 1))
     M.moe_align(_i32(ids).data_ptr(), pairs, E, cap, tm, rows.data_ptr(), tile_e.data_ptr(), dest.data_ptr(),
-                offs.data_ptr(), stream_ptr())
+                offs.data_ptr(), _p(clear), clear.numel() if clear is not None else 0, stream_ptr())
     act = torch.empty(cap, F_, dtype=h.dtype, device=dev)
     if pf:
         cfg = _moe_pf_cfg(pairs, E)
