@@ -121,7 +121,93 @@ __global__ void canon_conv_kernel(const TI* __restrict__ x, int64_t ld_in, const
   }
 }
 
-// the carried rows after a step whose sequences were convolved by several tiles
+// The same for 2 to 4 taps and whole quads of channels: a thread owns four neighbouring channels of TT tokens and has all
+// TT + TAPS - 1 rows in flight before it uses the first. The first tile of a sequence, the only one that reads the carried
+// inputs, also writes them back (the last rows are a second read of a few cache lines), so no launch follows.
+// Memory-bound (with silu its arithmetic); against the kernel above without its second launch (5 us), us: 8192 x 2048
+// fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 21.1
+// against 49.0, 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us without silu and loses 5 with it.
+template <typename TI, typename TO, int TAPS, int TT>
+__global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, int64_t ld_in, const float* __restrict__ w,
+                                                    const float* __restrict__ bias, float* __restrict__ state,
+                                                    const int32_t* __restrict__ qsl, const int32_t* __restrict__ seq_lens,
+                                                    const int32_t* __restrict__ slots, TO* __restrict__ out, int W,
+                                                    int residual, int act) {
+  constexpr int NH = TAPS - 1;
+  const int s = blockIdx.z;
+  const int q0 = qsl[s], q = qsl[s + 1] - q0, slot = slots[s];
+  const int t0 = blockIdx.y * TT;
+  if (slot < 0 || t0 >= q) return;
+  const int c = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+  if (c >= W) return;
+  const TI* xc = x + (int64_t)q0 * ld_in + c;
+  float* st = state + (int64_t)slot * NH * W + c;
+  Raw4<TI> in[TT + NH], last[NH];
+  Raw4<float> old[NH], wt[TAPS], b;
+#pragma unroll
+  for (int j = 0; j < TT + NH; ++j) in[j].load(xc + (int64_t)min(max(t0 - NH + j, 0), q - 1) * ld_in);
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) wt[j].load(w + (int64_t)c * TAPS + 4 * j);   // 4 TAPS floats, [channel][tap]
+  b.zero();
+  if (bias) b.load(bias + c);
+  const bool first = t0 == 0;
+  if (first) {
+    const int ctx = seq_lens[s] - q;
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      old[j].zero();
+      if (ctx - NH + j >= 0) old[j].load(st + (int64_t)j * W);
+      last[j].load(xc + (int64_t)max(q - NH + j, 0) * ld_in);
+    }
+  }
+  float wf[4 * TAPS], bf[4], v[TT + NH][4];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) {
+    float f[4];
+    wt[j].get(f);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wf[4 * j + e] = f[e];
+  }
+  b.get(bf);
+#pragma unroll
+  for (int j = 0; j < TT + NH; ++j) in[j].get(v[j]);
+  if (first) {
+    float h[NH][4];
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      old[j].get(h[j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] = h[j][e];
+    }
+    // carried inputs: the last NH of [old | this step's rows]
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      float f[4];
+      last[j].get(f);
+#pragma unroll
+      for (int i = 1; i < NH; ++i)
+        if (q + j == i) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f[e] = h[i][e];
+        }
+      st4(st + (int64_t)j * W, f);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = (residual ? v[t + NH][e] : 0.f) + bf[e];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) o[e] += wf[TAPS * e + j] * v[t + j][e];
+      if (act) o[e] = siluf(o[e]);
+    }
+    if (t0 + t < q) st4(out + (int64_t)(q0 + t0 + t) * W + c, o);   // (no early exit: the loop has to unroll)
+  }
+}
+
+// the carried rows of a step whose sequences were convolved by several tiles of canon_conv_kernel or by another kernel
 template <typename TI>
 __global__ void canon_state_kernel(const TI* __restrict__ x, int64_t ld_in, float* __restrict__ state,
                                    const int32_t* __restrict__ qsl, const int32_t* __restrict__ seq_lens,
@@ -820,6 +906,29 @@ __global__ void delta_out_kernel(const float* __restrict__ o, const float* __res
         row[d] * r * nw[h * D + d] * sigmoidf(ldf(gate + (int64_t)t * gate_stride + h * D + d)));
 }
 
+// D = 4 L with L a power of two: four entries per lane, 64 / L heads per wave. Memory-bound: 8192 x 32 x 64 29.8 us
+// (4.5 TB/s) against 73.6 with a wave per head.
+template <typename T>
+__global__ __launch_bounds__(256) void delta_out4_kernel(const float* __restrict__ o, const float* __restrict__ nw,
+                                                         const T* __restrict__ gate, int64_t gate_stride, float eps,
+                                                         T* __restrict__ out, int64_t quads, int HD, int L) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= quads) return;   // (whole heads: HD is a multiple of 4 L)
+  const int64_t t = 4 * i / HD;
+  const int c = (int)(4 * i - t * HD);
+  float v[4], w[4], g[4];
+  Raw4<T> gr;
+  gr.load(gate + t * gate_stride + c);
+  ld4(nw + c, w);
+  ld4(o + 4 * i, v);
+  const float ss = seg_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], L);
+  const float r = 1.f / sqrtf(ss / (float)(4 * L) + eps);
+  gr.get(g);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * sigmoidf(g[e]);
+  st4(out + 4 * i, v);
+}
+
 // ------------------------------------------------------------------ activations
 // xIELU with sp = softplus(p), cn = 1/2 + softplus(q):
 //   z > 0: sp z^2 + z/2 ;  z <= 0: cn (exp(z) - 1 - z) + z/2
@@ -879,6 +988,29 @@ void causal_conv(const void* x, bool in_f32, int64_t ld_in, const float* w, cons
                  const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots, void* out, bool out_f32, int ns,
                  int max_q, int W, int taps, bool residual, bool act, hipStream_t st) {
   if (ns <= 0 || max_q <= 0) return;
+  const int isz = in_f32 ? 4 : 2, osz = out_f32 ? 4 : 2;
+  if (taps >= 2 && taps <= 4 && W % 4 == 0 && ld_in % 4 == 0 && (max_q + 7) / 8 <= 65535 && ns <= 65535 &&
+      (uintptr_t)x % (4 * isz) == 0 && (uintptr_t)out % (4 * osz) == 0 &&
+      (((uintptr_t)w | (uintptr_t)bias | (uintptr_t)state) & 15) == 0) {
+    // single tokens: a wave per 256 channels, so that few sequences still spread over the chip
+#define XGM_C4(TI, TO, TAPS)                                                                                               \
+  if (max_q == 1)                                                                                                          \
+    conv4_kernel<TI, TO, TAPS, 1><<<dim3((W + 255) / 256, 1, ns), 64, 0, st>>>((const TI*)x, ld_in, w, bias, state, qsl,   \
+                                                                               seq_lens, slots, (TO*)out, W, residual, act); \
+  else                                                                                                                     \
+    conv4_kernel<TI, TO, TAPS, 8><<<dim3((W + 1023) / 1024, (max_q + 7) / 8, ns), 256, 0, st>>>(                        \
+        (const TI*)x, ld_in, w, bias, state, qsl, seq_lens, slots, (TO*)out, W, residual, act);
+#define XGM_C4T(TAPS)                                                       \
+  if (in_f32) {                                                             \
+    if (out_f32) { XGM_C4(float, float, TAPS) } else { XGM_C4(float, bf16, TAPS) } \
+  } else {                                                                  \
+    if (out_f32) { XGM_C4(bf16, float, TAPS) } else { XGM_C4(bf16, bf16, TAPS) }   \
+  }
+    if (taps == 2) { XGM_C4T(2) } else if (taps == 3) { XGM_C4T(3) } else { XGM_C4T(4) }
+#undef XGM_C4T
+#undef XGM_C4
+    return;
+  }
   const int tile = 64;
   const int ntiles = (max_q + tile - 1) / tile;
   dim3 grid((W + 255) / 256, ntiles, ns);
@@ -1076,6 +1208,14 @@ int delta_scan(const void* proj, bool f32, int64_t ld, int off_r, int off_k, int
 void delta_out(const float* o, const float* nw, const void* gate, bool f32, int64_t gate_stride, float eps, void* out,
                int T_, int H, int D, hipStream_t st) {
   if (T_ <= 0) return;
+  const int esz = f32 ? 4 : 2, L = D / 4;
+  const int64_t quads = (int64_t)T_ * H * L;
+  if (D % 4 == 0 && L >= 1 && L <= 64 && (L & (L - 1)) == 0 && gate_stride % 4 == 0 && quads < (1ll << 38) &&
+      (uintptr_t)gate % (4 * esz) == 0 && (((uintptr_t)o | (uintptr_t)nw | (uintptr_t)out) & 15) == 0) {
+    XGM_DISPATCH_T(f32, delta_out4_kernel<T><<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(o, nw, (const T*)gate, gate_stride,
+                                                                                             eps, (T*)out, quads, H * D, L);)
+    return;
+  }
   XGM_DISPATCH_T(f32, delta_out_kernel<T><<<dim3(T_, (H + 3) / 4), 256, 0, st>>>(o, nw, (const T*)gate, gate_stride, eps, (T*)out, H, D);)
 }
 

@@ -38,6 +38,30 @@ __device__ __forceinline__ void st4(bf16* p, const float (&f)[4]) {
   *reinterpret_cast<uint2*>(p) = make_uint2(xgk::pack2(f[0], f[1]), xgk::pack2(f[2], f[3]));
 }
 
+// four elements as they lie in memory: loads of a batch are issued before the first conversion waits for one
+template <typename T> struct Raw4;
+template <> struct Raw4<float> {
+  float4 v;
+  __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void zero() { v = make_float4(0.f, 0.f, 0.f, 0.f); }
+  __device__ __forceinline__ void get(float (&f)[4]) const { f[0] = v.x, f[1] = v.y, f[2] = v.z, f[3] = v.w; }
+};
+template <> struct Raw4<bf16> {
+  uint2 v;
+  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ void zero() { v = make_uint2(0, 0); }
+  __device__ __forceinline__ void get(float (&f)[4]) const {
+    f[0] = __uint_as_float(v.x << 16), f[1] = __uint_as_float(v.x & 0xFFFF0000u);
+    f[2] = __uint_as_float(v.y << 16), f[3] = __uint_as_float(v.y & 0xFFFF0000u);
+  }
+};
+
+// sum over the L lanes (a power of two) of an aligned segment of the wave
+__device__ __forceinline__ float seg_sum(float v, int L) {
+  for (int o = L >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
