@@ -1,0 +1,75 @@
+"""Latent attention of single tokens in shares of the window, with the heads' value expansion, against fp64.
+
+Tolerance: scores of bf16 inputs with fp32 sums (relative to the largest sum of magnitudes, R 2^-24), weights rounded to bf16
+(2^-9), the merged sum rounded to bf16 (2^-9) before the expansion, the result rounded once more (2^-9): the first two move
+every row by at most a share of the largest value, the expansion sums R of them as independent errors."""
+import pytest
+import torch
+
+from xgserve.ops import seqmix as sq
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,dn,rd,dv,R,rot", [(32, 64, 32, 64, 256, 32), (3, 32, 32, 16, 64, 16), (40, 64, 64, 128, 512, 64),
+                                              (16, 16, 64, 80, 128, 0)])
+@pytest.mark.parametrize("lens,window,bs", [([1], 8, 16), ([64, 65, 1], 64, 16), ([300, 1, 129, 1000, 7], 512, 16),
+                                            ([2100, 40], 4096, 1), ([700] * 9, 333, 32)])
+def test_against_fp64(H, dn, rd, dv, R, rot, lens, window, bs):
+    g = torch.Generator().manual_seed(H + len(lens))
+    T, dq = len(lens), dn + rd
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    pages = [-(-n // bs) for n in lens]
+    order = torch.randperm(sum(pages) + 1, generator=g).to(torch.int32)
+    bt, at = torch.zeros(T, max(pages), dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    slots = list(range(T))
+    if T > 2:
+        slots[1] = -1                                                       # a padding row
+    sm = sq.SeqMeta(T, 1, i32(list(range(T + 1))), i32(lens), i32(slots), bt.cuda(), i32(list(range(T))),
+                    i32([n - 1 for n in lens]), i32([0] * T))
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    cache = rnd((sum(pages) + 1) * bs, R + rd).bfloat16()
+    q, gate = rnd(T, H, dq).bfloat16(), rnd(T, H + 8).bfloat16()[:, 8:]
+    uk, uv = (rnd(H * dn, R) / R ** 0.5).bfloat16(), (rnd(H * dv, R) / R ** 0.5).bfloat16()
+    table = sq.build_rot_table(rot, 1e4, max(lens) + 1, "cpu") if rot else torch.zeros(max(lens) + 1, 1, 2)
+    scale = dq ** -0.5
+    dev = [t.cuda() for t in (q, gate, cache, uk, uv, table)]
+    assert sq._latent_shares(dev[0], dev[4], R, rd, dv, window, bs, sm) > 0
+    got = sq.latent_attention_heads(dev[0], dn, dev[1], dev[2], dev[3], dev[4], dev[5], rot, window, scale, bs, sm)
+    # the queries in latent space as the step rounds them
+    qabs = torch.bmm(dev[0][:, :, :dn].transpose(0, 1), dev[3].view(H, dn, R)).cpu().double()
+    for t, n in enumerate(lens):
+        if slots[t] < 0:
+            assert not bool(got[t].any())
+            continue
+        j = torch.arange(max(0, n - window), n)
+        rows = cache[bt[t][j // bs].long() * bs + j % bs].double()
+        qr = q[t, :, dn:].double().clone()
+        if rot:
+            c, s = table[n - 1, :, 0].double(), table[n - 1, :, 1].double()
+            a, b = qr[:, 0:rot:2].clone(), qr[:, 1:rot:2].clone()
+            qr[:, 0:rot:2], qr[:, 1:rot:2] = a * c - b * s, b * c + a * s
+        qr = qr.bfloat16().double()
+        p = torch.softmax((qabs[:, t] @ rows[:, :R].T + qr @ rows[:, R:].T) * scale, -1)
+        lat = (p @ rows[:, :R]) * torch.sigmoid(gate[t, :H].double())[:, None]
+        want = torch.einsum("hr,hdr->hd", lat, uv.view(H, dv, R).double()).reshape(-1)
+        mag = (p @ rows[:, :R].abs()).amax()       # what a weight's rounding is relative to
+        err = (got[t].double().cpu() - want).abs()
+        bound = want.abs() * 2.0 ** -8 + mag * (2.0 ** -9 * 2 + R * 2.0 ** -22) * uv.double().view(H, dv, R).norm(dim=-1).reshape(-1) * 4
+        assert bool((err <= bound).all()), (t, float((err / bound).max()))
+
+
+def test_other_steps_keep_the_general_kernels():
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    sm = sq.SeqMeta(2, 1, i32([0, 1, 2]), i32([5, 9]), i32([0, 1]), i32([[0], [1]]), i32([0, 1]), i32([4, 8]), i32([4, 24]))
+    q, uv = torch.zeros(2, 4, 96, dtype=torch.bfloat16, device="cuda"), torch.zeros(4 * 64, 256, dtype=torch.bfloat16, device="cuda")
+    assert sq._latent_shares(q, uv, 256, 32, 64, 64, 16, sm) == 1
+    assert sq._latent_shares(q.float(), uv, 256, 32, 64, 64, 16, sm) == 0
+    assert sq._latent_shares(q, uv, 240, 32, 64, 64, 16, sm) == 0 and sq._latent_shares(q, uv, 256, 24, 64, 64, 16, sm) == 0
+    sm.block_tables = torch.zeros(2, 1 << 20, dtype=torch.int32, device="cuda")
+    assert sq._latent_shares(q, uv, 256, 32, 64, 1 << 20, 1, sm) == 0       # a share's page table would not fit
+    sm.max_q = 2
+    assert sq._latent_shares(q, uv, 256, 32, 64, 64, 16, sm) == 0

@@ -428,6 +428,27 @@ def _latent_key_rows(sm: SeqMeta, T: int, window: int, block_size: int) -> int:
     return T + max(0, min(sm.num_seqs * (window - 1), held - T))
 
 
+# Steps of single tokens (latent_decode.hip): shares of a window while the grid stays within 256 workgroups, at most 16. From the
+# queries to the heads' outputs, us, 32 heads, in 1 / 2 / 4 / 8 / 16 shares: 64 sequences of 1024 keys, R = 256 43 / 32 / 29 / 31
+# / 42, R = 512 82 / 56 / 48 / 65 / 95; one sequence of 4000 keys, R = 512, in 8 / 16 / 32 / 63 shares 48 / 43 / 49 / 65.
+LATENT_DECODE = True
+LATENT_DECODE_WGS, LATENT_DECODE_SHARES = 256, 16
+LATENT_PAGES = 2048     # page table entries of a share
+
+
+def _latent_shares(q, uv, R: int, rd: int, dv: int, window: int, block_size: int, sm: SeqMeta) -> int:
+    """Shares of the window for latent_decode, 0 where it does not apply."""
+    T, H = q.shape[:2]
+    if not (native_device(q) and LATENT_MFMA and LATENT_DECODE and q.dtype == torch.bfloat16 and sm.max_q == 1
+            and 1 <= T == sm.num_seqs <= 65535 and R in (64, 128, 256, 512) and rd in (32, 64) and dv % 16 == 0
+            and uv.data_ptr() % 16 == 0):
+        return 0
+    tiles = -(-min(window, sm.block_tables.shape[1] * block_size) // 64)
+    groups = T * -(-H // 32)
+    per = -(-tiles // max(1, min(LATENT_DECODE_SHARES, tiles, LATENT_DECODE_WGS // groups)))
+    return -(-tiles // per) if per * 64 <= (LATENT_PAGES - 2) * block_size else 0     # (no share that is always empty)
+
+
 def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: torch.Tensor, uk: torch.Tensor,
                            uv: torch.Tensor, rot: torch.Tensor, rot_dims: int, window: int, scale: float, block_size: int,
                            sm: SeqMeta) -> torch.Tensor:
@@ -458,6 +479,19 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
                                       sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
             return out
     qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
+    shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm)
+    if shares:
+        assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
+        assert cache.dtype == gate.dtype == uv.dtype == q.dtype and uv.is_contiguous()
+        bt = _i32(sm.block_tables)
+        out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+        part = torch.empty(shares * H * T * (R + 2), dtype=torch.float32, device=q.device)
+        mixers().latent_decode(qabs.data_ptr(), q.data_ptr(), dq, dn, gate.data_ptr(), gate.stride(0), cache.data_ptr(),
+                               bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
+                               _i32(sm.slots).data_ptr(), rot.data_ptr(), rot_dims, uv.data_ptr(), out.data_ptr(), T, H, R, dv,
+                               int(window), float(scale), shares, part.data_ptr(),
+                               part.data_ptr() + 4 * shares * H * T * R, stream_ptr())
+        return out
     o_lat = latent_attention(qabs, q, dn, gate, cache, rot, rot_dims, window, scale, block_size, sm)
     return heads_to_rows(torch.bmm(o_lat, uv.view(H, dv, R).transpose(1, 2)))   # [H, T, dv] -> rows
 
