@@ -39,7 +39,11 @@ int conv_head_norm_rope_cache(const void*, bool, int64_t, const float*, int, flo
                               const int32_t*, const int32_t*, int, int, int, int, int, int, const float*, const float*,
                               float, const float*, int, int, const int32_t*, void*, void*, void*, bool, int, hipStream_t);
 int post_norm_residual(float*, const void*, bool, int64_t, const float*, const void*, int64_t, const float*, const float*,
-                       const float*, float, const float*, const float*, float, float, void*, bool, int, int, hipStream_t);
+                       const float*, float, const float*, const float*, float, float, void*, bool, int, int, int, int, int64_t,
+                       hipStream_t);
+int row_update(float*, const void*, int64_t, int64_t, int, const void*, int64_t, int64_t, int, const float*, const float*,
+               const float*, const float*, float, const float*, float, float, bool, float*, void*, const float*, int, float*,
+               const int32_t*, const int32_t*, const int32_t*, void*, int, int, hipStream_t);
 void relu2(const void*, bool, const float*, void*, int64_t, int, hipStream_t);
 void lower_bound_gates(const void*, bool, int64_t, int, int, int, const float*, const float*, float*, float*, int,
                        hipStream_t);
@@ -258,13 +262,24 @@ PYBIND11_MODULE(_mixers, m) {
   m.def("post_norm_residual", [](uintptr_t x, uintptr_t y, bool y_f32, int64_t ldy, uintptr_t y_bias, uintptr_t y2,
                                  int64_t ldy2, uintptr_t pw1, uintptr_t pw2, uintptr_t post_w, float mult, uintptr_t extra,
                                  uintptr_t next_w, float off, float eps, uintptr_t out, bool out_f32, int T, int W,
-                                 uintptr_t st) {
+                                 int n1, int n2, int64_t slab, uintptr_t st) {
     if ((y && ldy < W) || (y2 && ldy2 < W)) throw std::invalid_argument("post_norm_residual: row stride below the width");
     int rc = xgm::post_norm_residual(P<float>(x), P<const void>(y), y_f32, ldy, P<const float>(y_bias), P<const void>(y2),
                                      ldy2, P<const float>(pw1), P<const float>(pw2), P<const float>(post_w), mult,
                                      P<const float>(extra), P<const float>(next_w), off, eps, P<void>(out), out_f32, T, W,
-                                     S(st));
+                                     n1, n2, slab, S(st));
     check(rc, "post_norm_residual");
+  });
+  m.def("row_update", [](uintptr_t x, uintptr_t y1, int64_t ld1, int64_t slab1, int n1, uintptr_t y2, int64_t ld2, int64_t slab2,
+                         int n2, uintptr_t y3, uintptr_t a1, uintptr_t a2, uintptr_t bias, float alpha, uintptr_t g, float off,
+                         float eps, bool keep_norm, uintptr_t n32, uintptr_t nact, uintptr_t cw, int taps, uintptr_t state,
+                         uintptr_t token_seq, uintptr_t seq_lens, uintptr_t slots, uintptr_t h, int T, int W, uintptr_t st) {
+    check(xgm::row_update(P<float>(x), P<const void>(y1), ld1, slab1, n1, P<const void>(y2), ld2, slab2, n2, P<const float>(y3),
+                          P<const float>(a1), P<const float>(a2), P<const float>(bias), alpha, P<const float>(g), off, eps,
+                          keep_norm, P<float>(n32), P<void>(nact), P<const float>(cw), taps, P<float>(state),
+                          P<const int32_t>(token_seq), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<void>(h), T, W,
+                          S(st)),
+          "row_update");
   });
   m.def("relu2", [](uintptr_t in, bool f32, uintptr_t bias, uintptr_t out, int64_t n, int cols, uintptr_t st) {
     if (cols < 1 || n % cols) throw std::invalid_argument("relu2: the element count must be whole rows");

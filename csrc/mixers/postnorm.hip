@@ -77,27 +77,42 @@ __global__ __launch_bounds__(256) void post_norm_residual_kernel(
   for (int c = threadIdx.x; c < W; c += blockDim.x) stf(out + (int64_t)t * W + c, row[c] * rx * (off + next_w[c]));
 }
 
+template <bool PARTS, typename TY>
+__device__ __forceinline__ void row_slabs(const TY* p, int n, int64_t slab, float (&v)[4]) {
+  ld4(p, v);
+  if (!PARTS) return;
+#pragma unroll 4
+  for (int s = 1; s < n; ++s) {
+    float u[4];
+    ld4(p + s * slab, u);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += u[e];
+  }
+}
+
 // The same, for rows of up to 1024 * NV aligned columns: thread t owns columns 4 (t + 256 j) .. + 3, j < NV, in
-// registers; every global load of the row is issued before the first reduction.
-template <typename TY, typename TO, int NV>
-__global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
+// registers; every global load of the row is issued before the first reduction. PARTS (TY = float): y and y2 are n1 and n2
+// slabs of a product in parts, `slab` apart, added here.
+template <typename TY, typename TO, int NV, bool PARTS>
+__global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kernel(
     float* __restrict__ x, const TY* __restrict__ y, int64_t ldy, const float* __restrict__ y_bias,
     const TY* __restrict__ y2, int64_t ldy2, const float* __restrict__ pw1, const float* __restrict__ pw2,
     const float* __restrict__ post_w, float mult, const float* __restrict__ extra, const float* __restrict__ next_w,
-    float off, float eps, TO* __restrict__ out, int W) {
-  __shared__ float red[4];
+    float off, float eps, TO* __restrict__ out, int W, int n1, int n2, int64_t slab) {
+  constexpr int NT = PARTS ? 512 : 256;   // (few rows: more loads of a row in flight)
+  __shared__ float red[NT / 64];
   const int t = blockIdx.x;
   float* xr = x + (int64_t)t * W;
   const float inv_w = 1.f / (float)W;
   float xv[NV][4], u[NV][4], e[NV][4];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + NT * j);
 #pragma unroll
     for (int i = 0; i < 4; ++i) xv[j][i] = u[j][i] = e[j][i] = 0.f;
     if (c < W) {
       ld4(xr + c, xv[j]);
-      if (y) ld4(y + (int64_t)t * ldy + c, u[j]);
+      if (y) row_slabs<PARTS>(y + (int64_t)t * ldy + c, n1, slab, u[j]);
       if (extra) ld4(extra + (int64_t)t * W + c, e[j]);
     }
   }
@@ -108,10 +123,10 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
       float b[NV][4], s1 = 0.f, s2 = 0.f;
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int c = 4 * (threadIdx.x + 256 * j);
+        const int c = 4 * (threadIdx.x + NT * j);
 #pragma unroll
         for (int i = 0; i < 4; ++i) b[j][i] = 0.f;
-        if (c < W) ld4(y2 + (int64_t)t * ldy2 + c, b[j]);
+        if (c < W) row_slabs<PARTS>(y2 + (int64_t)t * ldy2 + c, n2, slab, b[j]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           s1 += u[j][i] * u[j][i];
@@ -122,7 +137,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
       const float rb = 1.f / sqrtf(block_sum(s2, red) * inv_w + eps);
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int c = 4 * (threadIdx.x + 256 * j);
+        const int c = 4 * (threadIdx.x + NT * j);
         if (c < W) {
           float w1[4], w2[4];
           ld4(pw1 + c, w1);
@@ -137,7 +152,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
     } else {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int c = 4 * (threadIdx.x + 256 * j);
+        const int c = 4 * (threadIdx.x + NT * j);
         if (c < W) {
           float bb[4] = {0.f, 0.f, 0.f, 0.f};
           if (y_bias) ld4(y_bias + c, bb);
@@ -152,7 +167,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
     const float ru = mult / sqrtf(block_sum(ssu, red) * inv_w + eps);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int c = 4 * (threadIdx.x + 256 * j);
+      const int c = 4 * (threadIdx.x + NT * j);
       if (c < W) {
         float pw[4];
         ld4(post_w + c, pw);
@@ -167,7 +182,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
   } else {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int c = 4 * (threadIdx.x + 256 * j);
+      const int c = 4 * (threadIdx.x + NT * j);
       if (c < W) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -182,7 +197,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_vec_kernel(
   const float rx = 1.f / sqrtf(block_sum(ssx, red) * inv_w + eps);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + NT * j);
     if (c < W) {
       float nw[4];
       ld4(next_w + c, nw);
@@ -219,7 +234,8 @@ __global__ void relu2_kernel(const T* __restrict__ z, const float* __restrict__ 
 // ================================================================== host launchers
 int post_norm_residual(float* x, const void* y, bool y_f32, int64_t ldy, const float* y_bias, const void* y2, int64_t ldy2,
                        const float* pw1, const float* pw2, const float* post_w, float mult, const float* extra,
-                       const float* next_w, float off, float eps, void* out, bool out_f32, int T_, int W, hipStream_t st) {
+                       const float* next_w, float off, float eps, void* out, bool out_f32, int T_, int W, int n1, int n2,
+                       int64_t slab, hipStream_t st) {
   if (T_ <= 0) return 0;
   if (W < 1 || W > 16000 || (y && !post_w) || (y2 && (!y || !pw1 || !pw2)) || (next_w && !out)) return -1;
   const size_t lds = (size_t)W * sizeof(float);
@@ -227,9 +243,23 @@ int post_norm_residual(float* x, const void* y, bool y_f32, int64_t ldy, const f
   const int ysz = y_f32 ? 4 : 2;
   const bool vec = (W & 3) == 0 && W <= 8192 && (!y || ((ldy & 3) == 0 && (uintptr_t)y % (4 * ysz) == 0)) &&
                    (!y2 || ((ldy2 & 3) == 0 && (uintptr_t)y2 % (4 * ysz) == 0));
+  if (n1 > 1 || n2 > 1) {
+    if (!vec || !y_f32 || slab % 4 || n1 < 1 || (y2 && n2 < 1)) return -2;
+#define XGM_PP(TO, NV)                                                                                                  \
+  post_norm_residual_vec_kernel<float, TO, NV, true><<<T_, 512, 0, st>>>((float*)x, (const float*)y, ldy, y_bias,        \
+                                                                         (const float*)y2, ldy2, pw1, pw2, post_w, mult, \
+                                                                         extra, next_w, off, eps, (TO*)out, W, n1, n2, slab);
+#define XGM_PPN(TO) \
+  if (W <= 2048) { XGM_PP(TO, 1) } else if (W <= 4096) { XGM_PP(TO, 2) } else { XGM_PP(TO, 4) }
+    if (out_f32) { XGM_PPN(float) } else { XGM_PPN(bf16) }
+#undef XGM_PPN
+#undef XGM_PP
+    return 0;
+  }
 #define XGM_PV(TY, TO, NV)                                                                                            \
-  post_norm_residual_vec_kernel<TY, TO, NV><<<T_, 256, 0, st>>>(x, (const TY*)y, ldy, y_bias, (const TY*)y2, ldy2, pw1,  \
-                                                                pw2, post_w, mult, extra, next_w, off, eps, (TO*)out, W);
+  post_norm_residual_vec_kernel<TY, TO, NV, false><<<T_, 256, 0, st>>>(x, (const TY*)y, ldy, y_bias, (const TY*)y2, ldy2, \
+                                                                       pw1, pw2, post_w, mult, extra, next_w, off, eps,  \
+                                                                       (TO*)out, W, 1, 1, 0);
 #define XGM_PN(TY, TO)                                                                                                \
   if (vec && W <= 2048) {                                                                                             \
     XGM_PV(TY, TO, 2)                                                                                                 \

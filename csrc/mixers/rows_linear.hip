@@ -10,7 +10,9 @@
 //
 // S parts of K: the parts of a column tile write fp32 slabs (write-through) and take a ticket; the one that draws the
 // last adds the slabs in order and finishes the tile, so a narrow product still puts a workgroup on every CU and needs
-// no second launch. The tickets are words that are zero before the launch and zero again after it.
+// no second launch. The tickets are words that are zero before the launch and zero again after it. Without tickets the
+// slabs are the result: the next kernel adds them as it reads them (row_update.hip, postnorm.hip), which saves the wait
+// for the last part.
 //
 // Measured against the library's product without what follows it, cold weights, us (T = 1 / 17 / 64):
 //   2048 x 2048    5.7 /  7.1 /  8.6 against 11.0 / 11.0 / 11.8      18560 x 4096   28 / 29 / 37 against 67 / 36 / 40
@@ -35,7 +37,7 @@ struct RowsArgs {
   const void* bias;        // [N] fp32 or bf16, or nullptr
   float* part;             // S > 1: [S, T, N] fp32
   bf16* out;               // [T, N], or [T, N / 2] for the gated activations
-  int* tickets;            // one zero word per column tile (S > 1)
+  int* tickets;            // one zero word per column tile (S > 1), or nullptr: the slabs are the result
   int64_t ld_x;
   int T, N, K, act;
   float p0, p1;
@@ -215,9 +217,12 @@ __global__ __launch_bounds__(64 * WV, 1) void rows_linear_kernel(const RowsArgs 
     for (int n = 0; n < NW; ++n) {
       const int in = gated ? n0 + 4 * g4 : n0 + 16 * n + 4 * g4;
       if (in >= (gated ? half : a.N)) continue;
-      xgk::st16_sc1(a.part + ((int64_t)part * a.T + tok) * a.N + in + (gated && n ? half : 0), acc[n][m]);
+      float* at = a.part + ((int64_t)part * a.T + tok) * a.N + in + (gated && n ? half : 0);
+      if (a.tickets) xgk::st16_sc1(at, acc[n][m]);
+      else *reinterpret_cast<f32x4_t*>(at) = acc[n][m];
     }
   }
+  if (!a.tickets) return;
   if (!xgk::agent_ticket(a.tickets + bx, S - 1, reinterpret_cast<int*>(lds))) return;
   const int c0 = gated ? bx * (COLS / 2) : bx * COLS;
 #define XGM_TAIL(SS)                                                  \
@@ -238,8 +243,10 @@ int rows_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
                 int* tickets, int T, int N, int K, int S, int act, float p0, float p1, bool wide, hipStream_t st) {
   const bool gated = act >= kActGlu;
   if (T < 1 || T > 64 || N < 1 || K < 128 || K % 128 || N % (gated ? 8 : 4) || ld_x % 8 || (gated && (!wide || bias)) ||
-      act < 0 || (S != 1 && S != 2 && S != 4 && S != 8) || S > K / 128 || (S > 1 && !(part && tickets)) ||
-      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part) & 15) || ((uintptr_t)out & 7))
+      act < 0 || (S != 1 && S != 2 && S != 4 && S != 8) || S > K / 128 || (S > 1 && !part) ||
+      (S > 1 && !tickets && (act != kActNone || bias)) ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part) & 15) || ((uintptr_t)out & 7) ||
+      (!out && (S == 1 || tickets)))
     return -1;
   RowsArgs a = {(const bf16*)x, (const bf16*)w, bias, part, (bf16*)out, tickets, ld_x, T, N, K, act, p0, p1, bias_f32};
   const dim3 grid((N + (wide ? 127 : 63)) / (wide ? 128 : 64), S);

@@ -76,7 +76,7 @@ class LatentAttentionMixer(nn.Module):
         q = sq.linear(cq, self.uq, sm).view(T, H, dq)
         o = sq.latent_attention_heads(q, self.dn, proj[:, self.off_g:], cache_rows, self.uk, self.uv, rot, self.rot_dims,
                                       self.window, self.scale, block_size, sm)
-        return sq.linear(o, self.o, sm)
+        return sq.linear_parts(o, self.o, sm)
 
 
 class DeltaRuleMixer(nn.Module):
@@ -98,7 +98,7 @@ class DeltaRuleMixer(nn.Module):
         wl = sq.linear(sq.tanh_cols(proj, 5 * HD, self.lr), self.w2, sm)
         o = sq.delta_rule_scan(proj, 0, HD, 2 * HD, 4 * HD, wl, self.a_bias, self.w0, state, self.H, self.D, sm)
         y = sq.delta_rule_out(o, self.norm, proj[:, 3 * HD:4 * HD], self.eps, self.H, self.D, h.dtype)
-        return sq.linear(y, self.o, sm)
+        return sq.linear_parts(y, self.o, sm)
 
 
 class XieluMLP(nn.Module):
@@ -117,7 +117,7 @@ class XieluMLP(nn.Module):
 
     def forward(self, h, sm: Optional[sq.SeqMeta] = None):
         """W_down act(W_up h + b_up); the down bias is added by the caller's norm."""
-        return sq.linear(sq.linear_xielu(h, self.up, self.up_b, self.sp, self.cn, sm), self.down, sm)
+        return sq.linear_parts(sq.linear_xielu(h, self.up, self.up_b, self.sp, self.cn, sm), self.down, sm)
 
 
 class DofivikLayer(nn.Module):
@@ -137,16 +137,18 @@ class DofivikLayer(nn.Module):
             self.mlp = XieluMLP(W, spec["mlp"]["ff"], device, dtype)
             self.norm2, self.canon2 = _p(f(W)), _p(f(W, taps))
 
-    def forward(self, x, sm: sq.SeqMeta, lc: LayerCache, rot, block_size, dtype):
-        h = sq.causal_conv_residual(x, self.canon1, lc.conv1, sm, dtype)
+    def forward(self, x, conv, sm: sq.SeqMeta, lc: LayerCache, rot, block_size, dtype, next_conv):
+        """x: fp32 residual (updated in place and returned). conv: a list of one, this layer's first convolution of x, replaced
+        by the one that the next layer begins with (next_conv: its weights and state, or None)."""
         if self.kind == "latent_attention":
-            y = self.mix(h, sm, lc.latent, rot, block_size)
+            y = self.mix(conv[0], sm, lc.latent, rot, block_size)
         else:
-            y = self.mix(h, sm, lc.delta)
-        sq.scaled_add_rmsnorm(x, y, self.norm1, self.eps, self.alpha, None, 1.0)
+            y = self.mix(conv[0], sm, lc.delta)
         if self.mlp is not None:
-            h = sq.causal_conv_residual(x, self.canon2, lc.conv2, sm, dtype)
-            sq.scaled_add_rmsnorm(x, self.mlp(h, sm), self.norm2, self.eps, self.alpha, self.mlp.down_b, 1.0)
+            h = sq.norm_conv(x, y, self.norm1, self.eps, self.alpha, None, (self.canon2, lc.conv2), sm, dtype)
+            conv[0] = sq.norm_conv(x, self.mlp(h, sm), self.norm2, self.eps, self.alpha, self.mlp.down_b, next_conv, sm, dtype)
+        else:
+            conv[0] = sq.norm_conv(x, y, self.norm1, self.eps, self.alpha, None, next_conv, sm, dtype)
         return x
 
 
@@ -276,9 +278,12 @@ class DofivikForCausalLM(nn.Module):
             raise ValueError("Dofivik needs the step's per-sequence metadata (AttnMeta.seq)")
         sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
         x = sq.embed_rows(input_ids, self.embed, tickets=sm.tickets)
-        for L, lc in zip(self.layers, cache.layers):
+        sm.parts = sq.step_rows(sm, x, self.dtype, self.cfg.canon_taps)
+        convs = [(L.canon1, lc.conv1) for L, lc in zip(self.layers, cache.layers)] + [None]
+        conv = [sq.causal_conv_residual(x, *convs[0], sm, self.dtype)]
+        for i, (L, lc) in enumerate(zip(self.layers, cache.layers)):
             rot = self._rot[(L.mix.rot_dims, L.mix.rot_base)] if L.kind == "latent_attention" else None
-            x = L(x, sm, lc, rot, cache.block_size, self.dtype)
+            x = L(x, conv, sm, lc, rot, cache.block_size, self.dtype, convs[i + 1])
         self.last_hidden = x
         return sq.scaled_add_rmsnorm(x, None, self.final_norm, self.cfg.norm_eps, 1.0, None, 1.0, inplace=False,
                                      out_dtype=self.dtype)

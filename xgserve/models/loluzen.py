@@ -71,7 +71,7 @@ class ConvRopeAttention(nn.Module):
                                          self.k_norm, self.eps, rot, self.rot_dims, sm, lc.k, lc.v)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, sq.MASK_CAUSAL, 0, self.scale, None,
                                 None, block_size, sm, gate=proj[:, self.ch:])
-        return sq.linear(o, self.o, sm)
+        return sq.linear_parts(o, self.o, sm)
 
 
 class TalkingDistanceAttention(nn.Module):
@@ -102,7 +102,7 @@ class TalkingDistanceAttention(nn.Module):
             wide = torch.stack([sq.masked_attention(*args, values=c, **kw).view(-1, H, dv) for c in range(G)], 2)
             wide = wide.reshape(-1, H * G * dv)
         o = sq.talk_mix(wide, self.talk, H, G, dv, gate=proj[:, n:n + H])
-        return sq.linear(o, self.o, sm)
+        return sq.linear_parts(o, self.o, sm)
 
 
 class LowerBoundRecurrence(nn.Module):
@@ -124,7 +124,7 @@ class LowerBoundRecurrence(nn.Module):
         n = self.n
         # the gate's bias is in the projection
         o = sq.lower_bound_recurrence(proj, 0, n, 2 * n, None, self.lower, lc.gla, self.H, self.dk, self.dv, sm)
-        return sq.linear(sq.gated_group_norm(o, None, self.norm, self.eps, self.H, proj.dtype), self.o, sm)
+        return sq.linear_parts(sq.gated_group_norm(o, None, self.norm, self.eps, self.H, proj.dtype), self.o, sm)
 
 
 class ParallelMixer(nn.Module):
@@ -153,7 +153,7 @@ class Relu2MLP(nn.Module):
 
     def forward(self, h, sm: Optional[sq.SeqMeta] = None):
         """W_down relu(W_up h + b)^2; the output bias down_b is added by the residual update."""
-        return sq.linear(sq.linear_relu2(h, self.up, self.up_b, sm), self.down, sm)
+        return sq.linear_parts(sq.linear_relu2(h, self.up, self.up_b, sm), self.down, sm)
 
 
 class LoluzenLayer(nn.Module):
@@ -326,6 +326,7 @@ class LoluzenForCausalLM(nn.Module):
         cfg, eps = self.cfg, self.cfg.norm_eps
         sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
         x = sq.embed_rows(input_ids, self.embed, scale=cfg.embed_scale, tickets=sm.tickets)
+        sm.parts = sq.step_rows(sm, x, self.dtype)
         e = x.clone() if self.pass_starts else None
         n = sq.post_norm_residual(x, None, None, None, 0.0, None, self.layers[self.runs[0]].norm1, eps, self.dtype)
         last = len(self.runs) - 1

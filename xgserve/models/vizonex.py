@@ -64,7 +64,7 @@ class ChunkedSinkAttention(nn.Module):
         q = sq.qk_norm_cache(proj, self.nq, self.nk, self.nv, self.q_norm, self.k_norm, self.eps, sm, lc.k, lc.v)
         o = sq.masked_attention(q, lc.k, lc.v, self.H, self.G, self.dk, self.dv, sq.MASK_CHUNK, self.size, self.scale,
                                 self.temp, self.sink, block_size, sm)
-        return sq.linear(o, self.o, sm)
+        return sq.linear_parts(o, self.o, sm)
 
 
 class SelectiveStateSpace(nn.Module):
@@ -89,7 +89,7 @@ class SelectiveStateSpace(nn.Module):
                              silu=True)
         y = sq.ssm_scan(xbc, proj[:, inner + ch:], self.dt_bias, self.A_log, self.D, lc.ssm, self.H, self.G, self.N,
                         self.P, sm)
-        return sq.linear(sq.gated_group_norm(y, proj[:, :inner], self.norm, self.eps, self.ng, h.dtype), self.o, sm)
+        return sq.linear_parts(sq.gated_group_norm(y, proj[:, :inner], self.norm, self.eps, self.ng, h.dtype), self.o, sm)
 
 
 class GatedMLP(nn.Module):
@@ -102,7 +102,7 @@ class GatedMLP(nn.Module):
         self.down = _p(torch.empty(width, self.ff, device=device, dtype=dtype))
 
     def forward(self, h, sm: Optional[sq.SeqMeta] = None):
-        return sq.linear(sq.linear_glu(h, self.gate_up, self.kind, self.limit, GLU_ALPHA, sm), self.down, sm)
+        return sq.linear_parts(sq.linear_glu(h, self.gate_up, self.kind, self.limit, GLU_ALPHA, sm), self.down, sm)
 
 
 class GroupedRouterMoE(nn.Module):
@@ -151,10 +151,9 @@ class VizonexLayer(nn.Module):
             self.mlp = GroupedRouterMoE(W, mlp, device, dtype) if self.moe else \
                 GatedMLP(W, mlp["ff"], sq.GLU_GELU_TANH, 0.0, device, dtype)
 
-    def forward(self, x, n32, nact, sm: sq.SeqMeta, lc: LayerCache, block_size: int, next_norm, want_f32: bool):
-        """x: fp32 residual (updated in place); n32 / nact: this block's norm of x. Returns (x, the next
-        norm of x as fp32 or None, and as an activation tensor)."""
-        h = sq.causal_conv(n32, self.canon1, None, lc.conv1, sm, nact.dtype, residual=True)
+    def forward(self, x, h, n32, nact, sm: sq.SeqMeta, lc: LayerCache, block_size: int, next_norm, next_conv, need_f32: bool):
+        """x: fp32 residual (updated in place); n32 / nact: this block's norm of x (fp32 for routers), h: its convolution.
+        Returns (x, the same three of the next block) (next_conv: its convolution's weights and state, or None)."""
         y1 = self.mix(h, sm, lc, block_size)
         y2 = y3 = None
         if self.mlp is not None:
@@ -162,8 +161,9 @@ class VizonexLayer(nn.Module):
                 y2, y3 = self.mlp(n32, nact, sm)
             else:
                 y2 = self.mlp(nact, sm)
-        n32, nact = sq.residual_norm(x, y1, self.ls1, y2, y3, self.ls2, next_norm, self.eps, nact.dtype, want_f32)
-        return x, n32, nact
+        n32, nact, h = sq.residual_norm_conv(x, y1, self.ls1, y2, y3, self.ls2, next_norm, self.eps, nact.dtype, next_conv,
+                                             need_f32, sm)
+        return x, h, n32, nact
 
 
 class VizonexForCausalLM(nn.Module):
@@ -275,10 +275,13 @@ class VizonexForCausalLM(nn.Module):
         x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions, tickets=sm.tickets)
         n32, nact = sq.residual_norm(x, None, None, None, None, None, self.layers[0].norm1, self.cfg.norm_eps,
                                      self.dtype, True)
+        sm.parts = sq.step_rows(sm, x, self.dtype, self.cfg.canon_taps)
         last = len(self.layers) - 1
+        convs = [(L.canon1, lc.conv1) for L, lc in zip(self.layers, cache.layers)] + [None]
+        h = sq.causal_conv(n32, convs[0][0], None, convs[0][1], sm, self.dtype, residual=True)
         for i, (L, lc) in enumerate(zip(self.layers, cache.layers)):
-            nxt = self.layers[i + 1].norm1 if i < last else self.final_norm
-            x, n32, nact = L(x, n32, nact, sm, lc, cache.block_size, nxt, i < last)
+            nxt, need_f32 = (self.layers[i + 1].norm1, self.layers[i + 1].moe) if i < last else (self.final_norm, False)
+            x, h, n32, nact = L(x, h, n32, nact, sm, lc, cache.block_size, nxt, convs[i + 1], need_f32)
         self.last_hidden = x
         return nact
 

@@ -37,6 +37,8 @@ class SeqMeta:
     slot_mapping: torch.Tensor   # int32 [T]
     # words that are zero between the step's launches, for products whose parts meet (`step_tickets`)
     tickets: Optional[torch.Tensor] = None
+    # the step's output products may leave their parts of K unadded (`linear_parts`): what follows them adds the slabs
+    parts: bool = False
 
 
 def _p(t: Optional[torch.Tensor]) -> int:
@@ -103,6 +105,7 @@ def step_tickets(like: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
 class StepTickets:
     """Stands for a step's SeqMeta where a product in parts runs without one."""
     tickets: Optional[torch.Tensor]
+    parts: bool = False
 
 
 def _rows_plan(N: int, K: int, gated: bool):
@@ -114,9 +117,11 @@ def _rows_plan(N: int, K: int, gated: bool):
     return wide, S
 
 
-def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool):
+def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool,
+                  slabs: bool = False):
     """The plan of x . w^T on the kernel of a few rows, or None: bfloat16, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
-    pieces, K in whole staged rows, and tickets where K is in parts (clearing them would cost what the parts gain)."""
+    pieces, K in whole staged rows, and tickets where K is in parts (clearing them would cost what the parts gain) unless the
+    `slabs` are the result."""
     if not (ROWS_LINEAR and native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and 1 <= x.shape[0] <= ROWS_LINEAR_MAX):
         return None
@@ -128,7 +133,7 @@ def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias:
                                  bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return None
     plan = _rows_plan(N, K, gated)
-    return plan if plan[1] == 1 or (sm is not None and sm.tickets is not None) else None
+    return plan if slabs or plan[1] == 1 or (sm is not None and sm.tickets is not None) else None
 
 
 def _rows_linear(plan, x, w, sm, bias, act, p0, p1) -> torch.Tensor:
@@ -148,6 +153,28 @@ def linear(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None,
     if plan is not None:
         return _rows_linear(plan, x, w, sm, bias, ACT_NONE, 0.0, 0.0)
     return F.linear(x, w, bias)
+
+
+@dataclass
+class Parts:
+    """A product whose parts of K have not been added: fp32 [parts, T, N]."""
+    part: torch.Tensor
+
+    def rows(self, dtype: torch.dtype) -> torch.Tensor:
+        return self.part.sum(0).to(dtype)
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None):
+    """x . w^T for a consumer that adds the parts of K itself where the step's SeqMeta says so: `Parts`, or the product."""
+    if sm is not None and sm.parts:
+        plan = _rows_plan_of(x, w, sm, None, False, slabs=True)
+        if plan is not None and plan[1] > 1:
+            T, (N, K), (wide, S) = x.shape[0], w.shape, plan
+            part = torch.empty(S, T, N, dtype=torch.float32, device=x.device)
+            mixers().rows_linear(x.data_ptr(), x.stride(0), w.data_ptr(), 0, False, part.data_ptr(), 0, 0, T, N, K, S, ACT_NONE,
+                                 0.0, 0.0, wide, stream_ptr())
+            return Parts(part)
+    return linear(x, w, sm)
 
 
 def linear_xielu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], sp: float, cn: float,
@@ -278,6 +305,70 @@ def scaled_add_rmsnorm(x: torch.Tensor, y: Optional[torch.Tensor], w: torch.Tens
                                 float(w_offset), float(eps), x.data_ptr() if inplace else 0, _p(out),
                                 is_f32(out) if out is not None else True, T, W, stream_ptr())
     return x if inplace else out
+
+
+# ---------------------------------------------------------------------------- ... and the next convolution, single tokens
+ROW_UPDATE = True
+
+
+def step_rows(sm: SeqMeta, x: torch.Tensor, dtype: torch.dtype, taps: int = 0) -> bool:
+    """Whether a step's residual rows x [T, W] are updated by the kernels of few rows that add the parts of a product
+    (post_norm_residual, and with `taps` row_update, which forms the next convolution of single tokens)."""
+    T, W = x.shape
+    return (ROW_UPDATE and native_device(x) and dtype == torch.bfloat16 and 1 <= T <= ROWS_LINEAR_MAX and W % 4 == 0
+            and W <= 8192 and (taps == 0 or (2 <= taps <= 4 and sm.max_q == 1)))
+
+
+def _row_source(y):
+    """(pointer, row stride, slab stride, slabs) of a bf16 row tensor (0 slabs), `Parts` or None."""
+    if y is None:
+        return 0, 0, 0, 0
+    if isinstance(y, Parts):
+        return y.part.data_ptr(), y.part.stride(1), y.part.stride(0), y.part.shape[0]
+    assert y.dtype == torch.bfloat16 and y.stride(1) == 1
+    return y.data_ptr(), y.stride(0), 0, 0
+
+
+def _row_update(x, y1, y2, y3, a1, a2, bias, alpha, w, off, eps, keep_norm, want_f32, want_act, conv_w, state, sm):
+    T, W = x.shape
+    assert x.dtype == w.dtype == torch.float32 and x.is_contiguous() and sm.max_q == 1
+    assert y3 is None or (y3.dtype == torch.float32 and y3.is_contiguous() and y3.shape == x.shape)
+    n32 = torch.empty_like(x) if want_f32 else None
+    nact = torch.empty(T, W, dtype=torch.bfloat16, device=x.device) if want_act else None
+    h = None
+    if conv_w is not None:
+        assert conv_w.dtype == state.dtype == torch.float32 and conv_w.is_contiguous() and state.is_contiguous()
+        assert conv_w.shape[0] == W and state.shape[1:] == (conv_w.shape[1] - 1, W)
+        h = torch.empty(T, W, dtype=torch.bfloat16, device=x.device)
+    mixers().row_update(x.data_ptr(), *_row_source(y1), *_row_source(y2), _p(y3), _p(a1), _p(a2), _p(bias), float(alpha),
+                        w.data_ptr(), float(off), float(eps), keep_norm, _p(n32), _p(nact), _p(conv_w),
+                        conv_w.shape[1] if conv_w is not None else 0, _p(state) if conv_w is not None else 0,
+                        _i32(sm.token_seq).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), _p(h), T, W,
+                        stream_ptr())
+    return n32, nact, h
+
+
+def norm_conv(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float, bias: Optional[torch.Tensor], conv: Optional[tuple],
+              sm: SeqMeta, dtype: torch.dtype) -> Optional[torch.Tensor]:
+    """x <- rmsnorm(alpha x + y + bias) * (1 + w) in place, then with conv = (weights, state) the residual convolution of the
+    new x (causal_conv_residual). y: an activation tensor, or the `Parts` of a product (sm.parts)."""
+    if sm.parts:
+        return _row_update(x, y, None, None, None, None, bias, alpha, w, 1.0, eps, True, False, False,
+                           *(conv or (None, None)), sm)[2]
+    scaled_add_rmsnorm(x, y, w, eps, alpha, bias, 1.0)
+    return causal_conv_residual(x, conv[0], conv[1], sm, dtype) if conv is not None else None
+
+
+def residual_norm_conv(x: torch.Tensor, y1, a1: Optional[torch.Tensor], y2, y3: Optional[torch.Tensor],
+                       a2: Optional[torch.Tensor], norm_w: torch.Tensor, eps: float, dtype: torch.dtype,
+                       conv: Optional[tuple], need_f32: bool, sm: SeqMeta):
+    """residual_norm (x <- x + a1 y1 + a2 (y2 + y3), n = its norm), then with conv = (weights, state) the residual convolution
+    of n: (n fp32 where `need_f32` or the convolution asks for it, n as `dtype`, convolution or None)."""
+    if sm.parts:
+        return _row_update(x, y1, y2, y3, a1, a2, None, 1.0, norm_w, 0.0, eps, False, need_f32, True, *(conv or (None, None)), sm)
+    n32, n = residual_norm(x, y1, a1, y2, y3, a2, norm_w, eps, dtype, need_f32 or conv is not None)
+    h = causal_conv(n32, conv[0], None, conv[1], sm, dtype, residual=True) if conv is not None else None
+    return n32, n, h
 
 
 # ---------------------------------------------------------------------------- rotation table
@@ -1169,9 +1260,20 @@ def post_norm_residual(x: torch.Tensor, y: Optional[torch.Tensor], y_bias: Optio
         x <- x + mult * N0(u) * (w_offset + post_w) + extra
         n  = N0(x) * (w_offset + next_w)
     with N0(v) = v / sqrt(mean(v^2) + eps). x fp32 [T, W] is updated in place; y / y2 activation tensors or fp32,
-    row-strided; y_bias, the weights fp32 [W]; extra fp32 [T, W]. y None: only `extra` is added. Returns n as
+    row-strided, or the `Parts` of products (SeqMeta.parts); y_bias, the weights fp32 [W]; extra fp32 [T, W]. y None: only `extra` is added. Returns n as
     `out_dtype` (None when next_w is None)."""
     T, W = x.shape
+    n1 = n2 = 1
+    slab = 0
+    if isinstance(y, Parts) or isinstance(y2, Parts):   # slabs of products in parts, added by the kernel
+        if y2 is None or (isinstance(y, Parts) and isinstance(y2, Parts)):
+            n1, slab, y = y.part.shape[0], T * W, y.part
+            if y2 is not None:
+                n2, y2 = y2.part.shape[0], y2.part
+            assert y.is_contiguous() and y.shape[1:] == x.shape and (y2 is None or (y2.is_contiguous() and y2.shape[1:] == x.shape))
+            y, y2 = y[0], (y2[0] if y2 is not None else None)
+        else:   # one branch in parts, the other not
+            y, y2 = (t.rows(out_dtype) if isinstance(t, Parts) else t for t in (y, y2))
 
     def n0(v):
         return v / torch.sqrt(v.pow(2).mean(-1, keepdim=True) + eps)
@@ -1197,7 +1299,7 @@ def post_norm_residual(x: torch.Tensor, y: Optional[torch.Tensor], y_bias: Optio
                                 y2.stride(0) if y2 is not None else 0, _p(pre_w[0]) if pre_w else 0,
                                 _p(pre_w[1]) if pre_w else 0, _p(post_w), float(mult), _p(extra), _p(next_w),
                                 float(w_offset), float(eps), _p(out), is_f32(out) if out is not None else True, T, W,
-                                stream_ptr())
+                                n1, n2, slab, stream_ptr())
     return out
 
 
