@@ -54,6 +54,11 @@ int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
 int latent_decode(const void*, const void*, int, int, const void*, int64_t, const void*, const int32_t*, int, int, const int32_t*,
                   const int32_t*, const int32_t*, const float*, int, const void*, void*, int, int, int, int, int, float, int,
                   float*, float*, hipStream_t);
+int gla_step(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*, const void*,
+             bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, const float*,
+             const float*, hipStream_t);
+int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const void*, const float*, const float*, const float*,
+               float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
 int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
                 bool, hipStream_t);
 int64_t delta_chunk_scratch_floats(int, int, int, int);
@@ -321,6 +326,25 @@ PYBIND11_MODULE(_mixers, m) {
                              P<const void>(uv), P<void>(out), T, H, R, dv, window, scale, shares, P<float>(part_o),
                              P<float>(part_ml), S(st)),
           "latent_decode");
+  });
+  m.def("gla_step", [](uintptr_t q, uintptr_t f, uintptr_t k, uintptr_t raw, int64_t ld_raw, int off_q, int off_f,
+                       uintptr_t f_bias, uintptr_t lower, uintptr_t v, bool v_f32, int64_t ld_v, uintptr_t state, uintptr_t qsl,
+                       uintptr_t seq_lens, uintptr_t slots, uintptr_t o, int ns, int H, int dk, int dv, uintptr_t decay,
+                       uintptr_t bonus, uintptr_t st) {
+    check(xgm::gla_step(P<const float>(q), P<const float>(f), P<const float>(k), P<const void>(raw), ld_raw, off_q, off_f,
+                        P<const float>(f_bias), P<const float>(lower), P<const void>(v), v_f32, ld_v, P<float>(state),
+                        P<const int32_t>(qsl), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<float>(o), ns, H, dk, dv,
+                        P<const float>(decay), P<const float>(bonus), S(st)),
+          "gla_step");
+  });
+  m.def("delta_step", [](uintptr_t proj, int64_t ld, int off_r, int off_k, int off_v, int off_g, int off_a, int off_z, int lr,
+                         uintptr_t w2, uintptr_t a_bias, uintptr_t w0, uintptr_t norm, float eps, uintptr_t state, uintptr_t qsl,
+                         uintptr_t seq_lens, uintptr_t slots, uintptr_t out, int ns, int H, int D, uintptr_t st) {
+    check(xgm::delta_step(P<const void>(proj), ld, off_r, off_k, off_v, off_g, off_a, off_z, lr, P<const void>(w2),
+                          P<const float>(a_bias), P<const float>(w0), P<const float>(norm), eps, P<float>(state),
+                          P<const int32_t>(qsl), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<void>(out), ns, H, D,
+                          S(st)),
+          "delta_step");
   });
   m.def("rows_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part,
                           uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, bool wide,

@@ -93,11 +93,8 @@ class DeltaRuleMixer(nn.Module):
         self.o = _p(e(width, self.HD))
 
     def forward(self, h, sm: sq.SeqMeta, state):
-        HD = self.HD
         proj = sq.linear(h, self.in_proj, sm)
-        wl = sq.linear(sq.tanh_cols(proj, 5 * HD, self.lr), self.w2, sm)
-        o = sq.delta_rule_scan(proj, 0, HD, 2 * HD, 4 * HD, wl, self.a_bias, self.w0, state, self.H, self.D, sm)
-        y = sq.delta_rule_out(o, self.norm, proj[:, 3 * HD:4 * HD], self.eps, self.H, self.D, h.dtype)
+        y = sq.delta_rule_mix(proj, self.w2, self.a_bias, self.w0, self.norm, state, self.eps, self.H, self.D, sm, h.dtype)
         return sq.linear_parts(y, self.o, sm)
 
 

@@ -673,6 +673,26 @@ def delta_rule_out(o: torch.Tensor, norm_w: torch.Tensor, gate: torch.Tensor, ep
     return out
 
 
+def delta_rule_mix(proj: torch.Tensor, w2: torch.Tensor, a_bias: torch.Tensor, w0: torch.Tensor, norm_w: torch.Tensor,
+                   state: torch.Tensor, eps: float, H: int, D: int, sm: SeqMeta, dtype: torch.dtype) -> torch.Tensor:
+    """The delta-rule mixer between its projections: proj's columns [r | k | v | gate | a-logits | low rank], decay logits
+    W2 tanh(low rank), delta_rule_scan, delta_rule_out. Steps of single tokens in one launch."""
+    T, HD, lr = proj.shape[0], H * D, w2.shape[1]
+    if native_device(proj) and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16 \
+            and D in (32, 64, 128) and 8 <= lr <= 256 and lr % 8 == 0 and sm.num_seqs <= 65535 and proj.stride(1) == 1 \
+            and proj.stride(0) % 4 == 0 and proj.data_ptr() % 8 == 0 and w2.is_contiguous() and w2.data_ptr() % 16 == 0:
+        assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, D)
+        y = torch.empty(T, HD, dtype=dtype, device=proj.device)
+        mixers().delta_step(proj.data_ptr(), proj.stride(0), 0, HD, 2 * HD, 3 * HD, 4 * HD, 5 * HD, lr, w2.data_ptr(),
+                            a_bias.data_ptr(), w0.data_ptr(), norm_w.data_ptr(), float(eps), state.data_ptr(),
+                            _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), y.data_ptr(),
+                            sm.num_seqs, H, D, stream_ptr())
+        return y
+    wl = linear(tanh_cols(proj, 5 * HD, lr), w2, sm)
+    o = delta_rule_scan(proj, 0, HD, 2 * HD, 4 * HD, wl, a_bias, w0, state, H, D, sm)
+    return delta_rule_out(o, norm_w, proj[:, 3 * HD:4 * HD], eps, H, D, dtype)
+
+
 # ---------------------------------------------------------------------------- activations
 def xielu(z: torch.Tensor, bias: Optional[torch.Tensor], sp: float, cn: float) -> torch.Tensor:
     """xIELU of z + bias with sp = softplus(p), cn = 1/2 + softplus(q):
@@ -1502,6 +1522,15 @@ def lower_bound_gates(proj: torch.Tensor, off_q: int, off_f: int, n: int, f_bias
     return qf[0], qf[1]
 
 
+# One token per sequence: state_step.hip (a pass over the states); other steps, and states of odd sizes, run as scans
+STATE_STEP = True
+
+
+def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int) -> bool:
+    return (STATE_STEP and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and dk <= 256 and dk * dv <= 16384
+            and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0)
+
+
 def gated_linear_scan(q: torch.Tensor, f: Optional[torch.Tensor], k: Optional[torch.Tensor], v: torch.Tensor,
                       state: torch.Tensor, H: int, dk: int, dv: int, sm: SeqMeta, decay: Optional[torch.Tensor] = None,
                       bonus: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1520,6 +1549,11 @@ def gated_linear_scan(q: torch.Tensor, f: Optional[torch.Tensor], k: Optional[to
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, dk, dv)
         if _chunk_scan_ok(sm, dk) and decay is None and bonus is None:
             return _chunk_scan(q, f, k, None, 0, 0, None, None, v, state, o, sm, H, dk, dv)
+        if _gla_step_ok(v, sm, dk, dv):
+            mixers().gla_step(q.data_ptr(), _p(f), _p(k), 0, 0, 0, 0, 0, 0, v.data_ptr(), is_f32(v), v.stride(0), state.data_ptr(),
+                              _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), o.data_ptr(),
+                              sm.num_seqs, H, dk, dv, _p(decay), _p(bonus), stream_ptr())
+            return o
         scratch = _scan_scratch(T, sm, H, dk, dv, q.device)
         mixers().gated_linear_scan(q.data_ptr(), _p(f), _p(k), 0, 0, 0, 0, 0, 0, v.data_ptr(), is_f32(v),
                                    v.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
@@ -1561,6 +1595,11 @@ def lower_bound_recurrence(proj: torch.Tensor, off_q: int, off_f: int, off_v: in
     o = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device)
     if _chunk_scan_ok(sm, dk):
         return _chunk_scan(None, None, None, proj, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv)
+    if _gla_step_ok(v, sm, dk, dv):
+        mixers().gla_step(0, 0, 0, proj.data_ptr(), proj.stride(0), off_q, off_f, _p(f_bias), lower.data_ptr(), v.data_ptr(),
+                          is_f32(proj), proj.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
+                          _i32(sm.slots).data_ptr(), o.data_ptr(), sm.num_seqs, H, dk, dv, 0, 0, stream_ptr())
+        return o
     scratch = _scan_scratch(proj.shape[0], sm, H, dk, dv, proj.device)
     mixers().gated_linear_scan(0, 0, 0, proj.data_ptr(), proj.stride(0), off_q, off_f, _p(f_bias), lower.data_ptr(),
                                v.data_ptr(), is_f32(proj), proj.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(),
