@@ -56,6 +56,31 @@ template <> struct Raw4<bf16> {
   }
 };
 
+// v += the N - 1 slabs behind the first, all of them in flight
+template <int N>
+__device__ __forceinline__ void add_slabs_n(const float* p, int64_t slab, float (&v)[4]) {
+  float u[N - 1][4];
+#pragma unroll
+  for (int s = 1; s < N; ++s) ld4(p + s * slab, u[s - 1]);
+#pragma unroll
+  for (int s = 1; s < N; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += u[s - 1][e];
+}
+// ... of n (1, 2, 4 or 8 parts are what the products have)
+__device__ __forceinline__ void add_slabs(const float* p, int64_t slab, int n, float (&v)[4]) {
+  if (n == 4) add_slabs_n<4>(p, slab, v);
+  else if (n == 8) add_slabs_n<8>(p, slab, v);
+  else if (n == 2) add_slabs_n<2>(p, slab, v);
+  else
+    for (int s = 1; s < n; ++s) {
+      float u[4];
+      ld4(p + s * slab, u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += u[e];
+    }
+}
+
 // sum over the L lanes (a power of two) of an aligned segment of the wave
 __device__ __forceinline__ float seg_sum(float v, int L) {
   for (int o = L >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -57,6 +57,8 @@ int latent_decode(const void*, const void*, int, int, const void*, int64_t, cons
 int gla_step(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*, const void*,
              bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, const float*,
              const float*, hipStream_t);
+int ssm_step(const void*, bool, int64_t, const void*, int64_t, const float*, const float*, const float*, float*, const int32_t*,
+             const int32_t*, const int32_t*, float*, int, int, int, int, int, hipStream_t);
 int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const void*, const float*, const float*, const float*,
                float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
 int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
@@ -336,6 +338,14 @@ PYBIND11_MODULE(_mixers, m) {
                         P<const int32_t>(qsl), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<float>(o), ns, H, dk, dv,
                         P<const float>(decay), P<const float>(bonus), S(st)),
           "gla_step");
+  });
+  m.def("ssm_step", [](uintptr_t xbc, bool f32, int64_t ld_x, uintptr_t dt_raw, int64_t ld_dt, uintptr_t dt_bias, uintptr_t A_log,
+                       uintptr_t D, uintptr_t state, uintptr_t qsl, uintptr_t seq_lens, uintptr_t slots, uintptr_t y, int ns, int H,
+                       int G, int N, int Pn, uintptr_t st) {
+    check(xgm::ssm_step(P<const void>(xbc), f32, ld_x, P<const void>(dt_raw), ld_dt, P<const float>(dt_bias),
+                        P<const float>(A_log), P<const float>(D), P<float>(state), P<const int32_t>(qsl),
+                        P<const int32_t>(seq_lens), P<const int32_t>(slots), P<float>(y), ns, H, G, N, Pn, S(st)),
+          "ssm_step");
   });
   m.def("delta_step", [](uintptr_t proj, int64_t ld, int off_r, int off_k, int off_v, int off_g, int off_a, int off_z, int lr,
                          uintptr_t w2, uintptr_t a_bias, uintptr_t w0, uintptr_t norm, float eps, uintptr_t state, uintptr_t qsl,

@@ -80,14 +80,7 @@ __global__ __launch_bounds__(256) void post_norm_residual_kernel(
 template <bool PARTS, typename TY>
 __device__ __forceinline__ void row_slabs(const TY* p, int n, int64_t slab, float (&v)[4]) {
   ld4(p, v);
-  if (!PARTS) return;
-#pragma unroll 4
-  for (int s = 1; s < n; ++s) {
-    float u[4];
-    ld4(p + s * slab, u);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += u[e];
-  }
+  if constexpr (PARTS) add_slabs(p, slab, n, v);
 }
 
 // The same, for rows of up to 1024 * NV aligned columns: thread t owns columns 4 (t + 256 j) .. + 3, j < NV, in
@@ -105,12 +98,20 @@ __global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kern
   float* xr = x + (int64_t)t * W;
   const float inv_w = 1.f / (float)W;
   float xv[NV][4], u[NV][4], e[NV][4];
+  // few rows wait for latency alone: the weights are on their way before the first statistic
+  Raw4<float> wpost[PARTS ? NV : 1], wnext[PARTS ? NV : 1], wb1[PARTS ? NV : 1], wb2[PARTS ? NV : 1], wb[PARTS ? NV : 1];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int c = 4 * (threadIdx.x + NT * j);
 #pragma unroll
     for (int i = 0; i < 4; ++i) xv[j][i] = u[j][i] = e[j][i] = 0.f;
     if (c < W) {
+      if constexpr (PARTS) {
+        if (post_w) wpost[j].load(post_w + c);
+        if (next_w) wnext[j].load(next_w + c);
+        if (y2) wb1[j].load(pw1 + c), wb2[j].load(pw2 + c);
+        if (y_bias) wb[j].load(y_bias + c);
+      }
       ld4(xr + c, xv[j]);
       if (y) row_slabs<PARTS>(y + (int64_t)t * ldy + c, n1, slab, u[j]);
       if (extra) ld4(extra + (int64_t)t * W + c, e[j]);
@@ -140,8 +141,8 @@ __global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kern
         const int c = 4 * (threadIdx.x + NT * j);
         if (c < W) {
           float w1[4], w2[4];
-          ld4(pw1 + c, w1);
-          ld4(pw2 + c, w2);
+          if constexpr (PARTS) wb1[j].get(w1), wb2[j].get(w2);
+          else ld4(pw1 + c, w1), ld4(pw2 + c, w2);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             u[j][i] = 0.5f * (u[j][i] * ra * w1[i] + b[j][i] * rb * w2[i]);
@@ -155,7 +156,11 @@ __global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kern
         const int c = 4 * (threadIdx.x + NT * j);
         if (c < W) {
           float bb[4] = {0.f, 0.f, 0.f, 0.f};
-          if (y_bias) ld4(y_bias + c, bb);
+          if constexpr (PARTS) {
+            if (y_bias) wb[j].get(bb);
+          } else if (y_bias) {
+            ld4(y_bias + c, bb);
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             u[j][i] += bb[i];
@@ -170,7 +175,8 @@ __global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kern
       const int c = 4 * (threadIdx.x + NT * j);
       if (c < W) {
         float pw[4];
-        ld4(post_w + c, pw);
+        if constexpr (PARTS) wpost[j].get(pw);
+        else ld4(post_w + c, pw);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           xv[j][i] = xv[j][i] + u[j][i] * ru * (off + pw[i]) + e[j][i];
@@ -200,7 +206,8 @@ __global__ __launch_bounds__(PARTS ? 512 : 256) void post_norm_residual_vec_kern
     const int c = 4 * (threadIdx.x + NT * j);
     if (c < W) {
       float nw[4];
-      ld4(next_w + c, nw);
+      if constexpr (PARTS) wnext[j].get(nw);
+      else ld4(next_w + c, nw);
 #pragma unroll
       for (int i = 0; i < 4; ++i) nw[i] = xv[j][i] * rx * (off + nw[i]);
       st4(out + (int64_t)t * W + c, nw);

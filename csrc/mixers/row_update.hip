@@ -6,8 +6,8 @@
 //   x <- r (keep_norm) or v;  n32, nact <- r;  h <- r + sum_j cw[:, j] (inputs carried in the slot, then r), the slot moves on
 //
 // A workgroup per row; everything the row needs is on its way before the first use. The launches that it replaces take about
-// 4.7 us each whatever they do; the rows are 8 to 24 KB of reads per slab. 64 rows of 2048 (8 slabs): 6.4 us against 4.8 + 4.8
-// and 4 us less in the product; one row of 4096 (two products of 4 slabs): 8.4 us against 7.7 + 4.6.
+// 4.7 us each whatever they do; the rows are 8 to 24 KB of reads per slab. 64 rows of 2048 (8 slabs): 6.1 us against 4.8 + 4.8
+// and 4 us less in the product; one row of 4096 (two products of 4 slabs): 6.5 us against 7.7 + 4.6.
 #include "mixers_common.h"
 
 namespace xgm {
@@ -37,13 +37,7 @@ __device__ __forceinline__ void row_source(const RowSource& y, int t, int c, flo
   }
   const float* p = (const float*)y.p + (int64_t)t * y.ld + c;
   ld4(p, v);
-#pragma unroll 4
-  for (int s = 1; s < y.n; ++s) {
-    float u[4];
-    ld4(p + s * y.slab, u);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += u[e];
-  }
+  add_slabs(p, y.slab, y.n, v);
 }
 
 template <int NV, int TAPS>

@@ -2,6 +2,8 @@
 // everything else that the token needs is formed in the same workgroup.
 //
 //   gla_step     gated linear recurrence (gla.hip) of one token:  S <- diag(f) S + k v^T,  o = S^T q
+//   ssm_step     selective state space (ssm.hip) of one token, the same kernel:  f = exp(-exp(A_log) dt), k = dt B, q = C, v = x,
+//                o = S^T q + D x with dt = softplus(dt_raw + dt_bias)
 //   delta_step   generalized delta rule of one token, from the fused projection row to the mixer's gated output:
 //                  w = exp(-e^(-1/2) sigmoid(W2 tanh(z) + w0)),  a = sigmoid(z_a + a_bias),  u = k / sqrt(|k|^2 + 1e-6)
 //                  S <- diag(w) S - (a u)(u^T S) + k v^T,  o = S^T r,  y = o / rms(o) * norm * sigmoid(gate)
@@ -10,6 +12,7 @@
 // all of its rows in flight while the row vectors are formed in LDS. The scans that serve longer portions give a lane one
 // column (4-byte accesses) and stage tiles of tokens.
 //   gla_step, 17 sequences x 32 heads x 64 x 128 (36 MB in and out): 10.1 us against 34.6
+//   ssm_step, 64 sequences x 64 heads x 128 x 64 (268 MB): 59.7 us against 93.6 (one sequence of 128 heads: 6.6 against 6.7)
 //   delta_step, 64 sequences x 32 heads x 64 x 64 (67 MB): 17.1 us against 40.1 in five launches (tanh 5.0, W2 4.9, row
 //   vectors 5.0, scan 20.4, output norm 4.8)
 #include "mixers_common.h"
@@ -25,6 +28,10 @@ struct GlaStepArgs {
   const int32_t *qsl, *seq_lens, *slots;
   int64_t ld_raw, ld_v;
   int off_q, off_f, H, dk, dv;
+  const void* dt_raw;                // state space: v = raw rows [x (H dv) | B (G dk) | C (G dk)], a row's dt inputs
+  const float *dt_bias, *A_log, *D;
+  int64_t ld_dt;
+  int G;
 };
 
 // NR: rows of a thread; QC = dv / 4 threads side by side, RG = 256 / QC rows at a time
@@ -47,7 +54,15 @@ __global__ __launch_bounds__(256) void gla_step_kernel(const GlaStepArgs a) {
     if (on && old && rg + RG * i < a.dk) sr[i].load(st + (int64_t)(rg + RG * i) * a.dv);
   }
   const int d = threadIdx.x;
-  if (d < a.dk) {
+  float skip = 0.f;
+  if (a.dt_raw) {
+    const float dt = softplusf(ldf((const T*)a.dt_raw + (int64_t)t * a.ld_dt + h) + a.dt_bias[h]);
+    if (d < a.dk) {
+      const T* row = (const T*)a.v + (int64_t)t * a.ld_v + a.H * a.dv + h / (a.H / a.G) * a.dk + d;
+      fs[d] = expf(-expf(a.A_log[h]) * dt), ks[d] = dt * ldf(row), qs[d] = ldf(row + a.G * a.dk);
+    }
+    if (d < a.dv) skip = a.D[h] * ldf((const T*)a.v + (int64_t)t * a.ld_v + h * a.dv + d);
+  } else if (d < a.dk) {
     if (a.raw) {
       const T* row = (const T*)a.raw + (int64_t)t * a.ld_raw + h * a.dk + d;
       const float l = a.lower[h * a.dk + d];
@@ -83,7 +98,7 @@ __global__ __launch_bounds__(256) void gla_step_kernel(const GlaStepArgs a) {
   }
   __syncthreads();
   if (d < a.dv) {
-    float x = 0.f;
+    float x = skip;
     for (int g = 0; g < RG; ++g) x += part[g * a.dv + d];
     a.o[((int64_t)t * a.H + h) * a.dv + d] = x;
   }
@@ -199,6 +214,16 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const DeltaStepArgs a) 
   a.out[((int64_t)t * a.H + h) * D + d] = f2bf(od / sqrtf(ss / (float)D + a.eps) * nd * sigmoidf(gd));
 }
 
+static int launch_gla_step(const GlaStepArgs& a, bool v_f32, int ns, hipStream_t st) {
+  const int RG = 256 / (a.dv / 4), nr = (a.dk + RG - 1) / RG;
+#define XGM_GS(NR) XGM_DISPATCH_T(v_f32, gla_step_kernel<T, NR><<<dim3(a.H, ns), 256, 0, st>>>(a);)
+  if (nr <= 2) { XGM_GS(2) } else if (nr <= 4) { XGM_GS(4) } else if (nr <= 8) { XGM_GS(8) } else if (nr <= 16) { XGM_GS(16) } else {
+    return -1;
+  }
+#undef XGM_GS
+  return 0;
+}
+
 // One token per sequence (max_q == 1). Return -1 for sizes outside the contract: dv a multiple of 4 up to 256, dk up to 256,
 // dk dv up to 16384, aligned rows.
 int gla_step(const float* q, const float* f, const float* k, const void* raw, int64_t ld_raw, int off_q, int off_f,
@@ -211,14 +236,21 @@ int gla_step(const float* q, const float* f, const float* k, const void* raw, in
       ((decay || bonus) && !k))
     return -1;
   const GlaStepArgs a = {q, f, k, raw, f_bias, lower, decay, bonus, v, state, o, qsl, seq_lens, slots, ld_raw, ld_v,
-                         off_q, off_f, H, dk, dv};
-  const int RG = 256 / (dv / 4), nr = (dk + RG - 1) / RG;
-#define XGM_GS(NR) XGM_DISPATCH_T(v_f32, gla_step_kernel<T, NR><<<dim3(H, ns), 256, 0, st>>>(a);)
-  if (nr <= 2) { XGM_GS(2) } else if (nr <= 4) { XGM_GS(4) } else if (nr <= 8) { XGM_GS(8) } else if (nr <= 16) { XGM_GS(16) } else {
+                         off_q, off_f, H, dk, dv, nullptr, nullptr, nullptr, nullptr, 0, 1};
+  return launch_gla_step(a, v_f32, ns, st);
+}
+
+int ssm_step(const void* xbc, bool f32, int64_t ld_x, const void* dt_raw, int64_t ld_dt, const float* dt_bias, const float* A_log,
+             const float* D, float* state, const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots, float* y, int ns,
+             int H, int G, int N, int P, hipStream_t st) {
+  if (ns <= 0) return 0;
+  if (H < 1 || G < 1 || H % G || N < 1 || N > 256 || P < 4 || P > 256 || P % 4 || N * P > 16384 || ns > 65535 || ld_x % 4 ||
+      (uintptr_t)xbc % (f32 ? 16 : 8) || (uintptr_t)state % 16 || !dt_raw)
     return -1;
-  }
-#undef XGM_GS
-  return 0;
+  GlaStepArgs a = {};
+  a.v = xbc, a.ld_v = ld_x, a.state = state, a.o = y, a.qsl = qsl, a.seq_lens = seq_lens, a.slots = slots, a.H = H, a.dk = N, a.dv = P;
+  a.dt_raw = dt_raw, a.ld_dt = ld_dt, a.dt_bias = dt_bias, a.A_log = A_log, a.D = D, a.G = G;
+  return launch_gla_step(a, f32, ns, st);
 }
 
 // One token per sequence, bf16. D 32, 64 or 128, lr (rank of W2 [H D, lr]) a multiple of 8 up to 256; columns of the projection

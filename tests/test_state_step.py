@@ -69,6 +69,35 @@ def test_gated_linear(H, dk, dv, mode, dt):
     assert bool((err <= 40 * 2.0 ** -24 * (want.abs() + float(v.double().abs().max()) * 4)).all())
 
 
+@pytest.mark.parametrize("H,G,N,P", [(1, 1, 1, 4), (4, 2, 128, 64), (6, 2, 33, 20), (2, 1, 256, 64), (2, 2, 16, 256)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_state_space(H, G, N, P, dt):
+    g = torch.Generator().manual_seed(N + P)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    T, sm = len(SLOTS), meta(SLOTS, CTX)
+    xbc, raw = rnd(T, -(-(H * P + 2 * G * N) // 4) * 4).to(dt), rnd(T, H + 3).to(dt)
+    bias, A, D, state = rnd(H), rnd(H), rnd(H), rnd(5, H, N, P)
+    st, xg = state.cuda(), xbc.cuda()
+    assert sq._gla_step_ok(xg, sm, N, P)
+    y = sq.ssm_scan(xg, raw.cuda()[:, 3:], bias.cuda(), A.cuda(), D.cuda(), st, H, G, N, P, sm)
+    z = xbc.double()
+    x = z[:, :H * P].view(T, H, P)
+    B, C = (z[:, H * P + i * G * N:H * P + (i + 1) * G * N].view(T, G, N).repeat_interleave(H // G, 1) for i in (0, 1))
+    step = torch.nn.functional.softplus(raw[:, 3:].double() + bias.double())
+    want = state.double().clone()
+    for t, s in enumerate(SLOTS):
+        if s < 0:
+            continue
+        S = state[s].double() if CTX[t] else torch.zeros(H, N, P, dtype=torch.float64)
+        dec = torch.exp(-torch.exp(A.double()) * step[t])
+        new = dec[:, None, None] * S + (step[t][:, None] * B[t])[:, :, None] * x[t][:, None]
+        out = torch.einsum("hnp,hn->hp", new, C[t]) + D.double()[:, None] * x[t]
+        mag = torch.einsum("hnp,hn->hp", new.abs(), C[t].abs()) + D.double().abs()[:, None] * x[t].abs()
+        assert bool(((y[t].double().cpu().view(H, P) - out).abs() <= (N + 60) * 2.0 ** -24 * (mag + 1) * 4).all())
+        want[s] = new
+    assert bool(((st.double().cpu() - want).abs() <= 200 * 2.0 ** -24 * (want.abs() + 1) * 4).all())
+
+
 @pytest.mark.parametrize("H,D,lr", [(2, 32, 8), (3, 64, 32), (2, 128, 64), (1, 64, 256)])
 def test_delta_rule(H, D, lr):
     g = torch.Generator().manual_seed(D + lr)
