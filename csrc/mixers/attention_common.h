@@ -20,6 +20,15 @@ __device__ __forceinline__ int first_visible(int mask, int size, int pos) {
   return 0;
 }
 
+// log2 of normal numbers
+__device__ __forceinline__ float log2_fast(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_logf(x);
+#else
+  return log2f(x);
+#endif
+}
+
 __device__ __forceinline__ float exp2_fast(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_exp2f(x);

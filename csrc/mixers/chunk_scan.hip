@@ -61,14 +61,6 @@ struct ChunkScanArgs {
   float *chA, *chB, *s_in;
 };
 
-__device__ __forceinline__ float log2_fast(float x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_logf(x);
-#else
-  return log2f(x);
-#endif
-}
-
 // eight elements as loaded
 template <typename T> struct Raw8;
 template <> struct Raw8<bf16> {
