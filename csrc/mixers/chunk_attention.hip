@@ -561,10 +561,11 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(const T* __restrict__ o_a
   const int rep = H / G;
   const T* row = o_all + (int64_t)t * H * G * dv;
   if ((dv & 3) == 0) {  // four value columns per thread
-    for (int e = threadIdx.x; e < H * dv / 4; e += blockDim.x) {
+    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < H * dv / 4; e += gridDim.y * blockDim.x) {
       const int h = e / (dv / 4), d = 4 * (e % (dv / 4));
       const int c = h / rep;
       float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
       for (int g = 0; g < H; ++g) {
         float v[4];
         ld4(row + ((int64_t)g * G + c) * dv + d, v);
@@ -946,7 +947,7 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
     if (!head_slots && max_q > kPromptMinRows && nw_hint == 0 && prompt_attention(args, max_q, wfn, st)) return 0;
     if (head_slots && single_attention(args, wfn, nsplit, part_o, part_ml, st)) {
       if (nsplit > 1)
-        masked_attention_combine_kernel<<<dim3(T_, H), dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit,
+        masked_attention_combine_kernel<<<dim3(T_, H), dv > 128 ? 256 : dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit,
                                                                     (const bf16*)gate, ld_gate, ge, wfn);
       return 0;
     }
@@ -976,7 +977,7 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
     XGM_MK(NKK, NMT, 4)                                                                                               \
   }                                                                                                                   \
   if (nsplit > 1)                                                                                                     \
-    masked_attention_combine_kernel<<<dim3(T_, H), dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit, \
+    masked_attention_combine_kernel<<<dim3(T_, H), dv > 128 ? 256 : dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit, \
                                                                 (const bf16*)gate, ld_gate, ge, wfn);                 \
   return 0;
   if (dk <= 64 && dv <= 64) { XGM_MM(2, 4) }
@@ -991,8 +992,10 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
 void talk_mix(const void* o_all, bool f32, const float* talk, const void* gate, int64_t ld_gate, void* out, int T_, int H,
               int G, int dv, hipStream_t st) {
   if (T_ <= 0) return;
-  XGM_DISPATCH_T(f32, talk_mix_kernel<T><<<T_, 256, 0, st>>>((const T*)o_all, talk, (const T*)gate, ld_gate, (T*)out, H, G,
-                                                              dv);)
+  // few rows: a wave per 256 value columns (17 rows of 16 heads of 128: 7.5 us against 11.7 with a workgroup per row)
+  const int waves = dv % 4 == 0 && T_ <= 256 ? std::min(64, (H * dv / 4 + 63) / 64) : 1;
+  XGM_DISPATCH_T(f32, talk_mix_kernel<T><<<dim3(T_, waves), waves > 1 ? 64 : 256, 0, st>>>((const T*)o_all, talk, (const T*)gate,
+                                                                                           ld_gate, (T*)out, H, G, dv);)
 }
 
 void head_norm_rope_cache(const void* src, bool src_f32, int64_t ld, int H, int G, int dk, int dv, const float* wq,
