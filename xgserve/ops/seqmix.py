@@ -1465,9 +1465,10 @@ CHUNK_SCAN_MIN = 16
 CHUNK_SCAN_MAX_DK = 128    # state rows a wave holds
 CHUNK_SCAN_MAX_SEQS = 2047   # (sequences x segments are one grid dimension)
 # Long portions are cut into segments until about two workgroups per compute unit run, of at least 64 tokens (128 for the
-# large state, whose sums cost more to write and fold): 4001 tokens of 16 heads of 64 x 128 take 88 us in 32 segments and 731
-# in one, 2521 tokens of 64 heads of 128 x 64 in four sequences 178 and 254; past two per compute unit the second run over the
-# tokens costs more than it spreads (4 x 1024 tokens of 128 heads of 128 x 64: 247 us whole, 368 in two).
+# large state, whose sums cost more to write and fold), and into three or more: the second run over the tokens has to be paid
+# for. us whole / in segments: 4001 tokens of 16 heads of 64 x 128 731 / 88 (32), 4 x 2048 of 32 such heads 381 / 266 (4), 8
+# portions of about 650 of 16 136 / 114 (4); in two 16 x 512 of 16 heads 108 / 160, 8 x 650 of 32 137 / 198, 4 x 2048 of 64
+# heads of 128 x 64 337 / 409.
 CHUNK_SCAN_FILL_WGS = 512
 CHUNK_SCAN_MIN_SEG, CHUNK_SCAN_MAX_SEGS = 64, 32
 
@@ -1479,9 +1480,9 @@ def _chunk_scan_ok(sm: SeqMeta, dk: int) -> bool:
 def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
     """(tokens per segment of a step's portions, scratch of the two launches or None: one segment, one launch)."""
     whole = (sm.max_q + 15) // 16 * 16
-    wgs = max(1, T // sm.max_q) * H * ((dv + cols - 1) // cols)
-    n = min(CHUNK_SCAN_MAX_SEGS, CHUNK_SCAN_FILL_WGS // wgs, whole // (CHUNK_SCAN_MIN_SEG * (2 if dk > 64 else 1)))
-    if n <= 1:
+    wgs = max(1.0, T / sm.max_q) * H * ((dv + cols - 1) // cols)   # portions as long as the longest
+    n = min(CHUNK_SCAN_MAX_SEGS, int(CHUNK_SCAN_FILL_WGS / wgs), whole // (CHUNK_SCAN_MIN_SEG * (2 if dk > 64 else 1)))
+    if n < 3:
         return whole, None
     seg = ((whole + n - 1) // n + 15) // 16 * 16
     return seg, torch.empty(mixers().chunk_scan_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32,
