@@ -87,6 +87,28 @@ __device__ __forceinline__ float seg_sum(float v, int L) {
   return v;
 }
 
+// e^z - 1 - z for z <= 0: near zero its power series (z^2 / 2 + .. + z^8 / 8!, the rest is below 2^-24 of it for |z| < 1/2), which
+// also spares the difference of two close numbers; else the exponential itself (the sum is above 0.1 there)
+__device__ __forceinline__ float exp_tail(float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float e = __builtin_amdgcn_exp2f(z * 1.44269504f);
+#else
+  const float e = expf(z);
+#endif
+  float p = fmaf(z, 1.f / 40320.f, 1.f / 5040.f);
+  p = fmaf(z, p, 1.f / 720.f);
+  p = fmaf(z, p, 1.f / 120.f);
+  p = fmaf(z, p, 1.f / 24.f);
+  p = fmaf(z, p, 1.f / 6.f);
+  p = fmaf(z, p, 0.5f);
+  return z > -0.5f ? z * z * p : (e - 1.f) - z;
+}
+
+// xIELU: sp z^2 + z / 2 for z > 0, cn (e^z - 1 - z) + z / 2 else
+__device__ __forceinline__ float xieluf(float z, float sp, float cn) {
+  return z > 0.f ? sp * z * z + 0.5f * z : cn * exp_tail(z) + 0.5f * z;
+}
+
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 

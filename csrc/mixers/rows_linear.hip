@@ -55,10 +55,7 @@ __device__ __forceinline__ void rows_finish(const RowsArgs& a, int tok, int col,
   }
   if (a.act == kActXielu) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float z = v[e];
-      v[e] = z > 0.f ? a.p0 * z * z + 0.5f * z : a.p1 * (expm1f(z) - z) + 0.5f * z;
-    }
+    for (int e = 0; e < 4; ++e) v[e] = xieluf(v[e], a.p0, a.p1);
   } else if (a.act == kActRelu2) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
