@@ -690,8 +690,8 @@ int grouped_gemm(const void* A, bool f32, int64_t lda, const void* Wt, const int
   }
     if (tm == 128) {         // gated: 64 x 128 per workgroup (two accumulator sets); one weight block: 128 x 128
       if (mode == kGemmGated) { XGM_GL(kGemmGated, 4, 2) } else if (mode == kGemmAct) { XGM_GL(kGemmAct, 8, 2) } else { XGM_GL(kGemmRows, 8, 2) }
-    } else if (tm == 64) {   // gated: 64 x 128; one weight block: 64 x 256
-      if (mode == kGemmGated) { XGM_GL(kGemmGated, 4, 2) } else if (mode == kGemmAct) { XGM_GL(kGemmAct, 4, 4) } else { XGM_GL(kGemmRows, 4, 4) }
+    } else if (tm == 64) {   // (K an odd multiple of 32) gated: 64 x 128; one weight block: 64 x 256
+      if (mode == kGemmGated) { XGM_GL2(kGemmGated, 4, 2, 32, false) } else if (mode == kGemmAct) { XGM_GL2(kGemmAct, 4, 4, 32, false) } else { XGM_GL2(kGemmRows, 4, 4, 32, false) }
     } else {
       if (mode == kGemmGated) { XGM_GG(kGemmGated) } else if (mode == kGemmAct) { XGM_GG(kGemmAct) } else { XGM_GG(kGemmRows) }
     }
