@@ -1005,8 +1005,9 @@ void head_norm_rope_cache(const void* src, bool src_f32, int64_t ld, int H, int 
                           const float* v_mix, hipStream_t st) {
   if (T_ <= 0) return;
   // four entries per thread where a head's statistic is a sum over a power of two of lanes (or none is needed: no norm, or
-  // norms over the whole vectors; 4001 rows of 40 heads of 64, fp32: 21 against 51 us) and quads stay whole: head sizes, value rows and strides multiples of 4, rotated pairs inside a quad (2i, 2i + 1) or
-  // a whole number of quads apart (i, i + n / 2), rows aligned to 16 (float) / 8 (bf16) bytes
+  // norms over the whole vectors; 4001 rows of 40 heads of 64, fp32: 21 against 51 us) and quads stay whole: head sizes, value
+  // rows and strides multiples of 4, rotated pairs inside a quad (2i, 2i + 1) or a whole number of quads apart
+  // (i, i + n / 2), rows aligned to 16 (float) / 8 (bf16) bytes
   const int isz = src_f32 ? 4 : 2, osz = out_f32 ? 4 : 2;
   const bool use_rot = rot && rot_dims > 0;
   const int vec = ((!wq && !wk) || whole || (dk <= 256 && (dk & (dk - 1)) == 0)) && dk % 4 == 0 && (G * dv) % 4 == 0 && ld % 4 == 0 &&

@@ -290,7 +290,7 @@ class BazuraxForCausalLM(nn.Module):
         sm = meta.seq
         if sm is None:
             raise ValueError("Bazurax needs the step's per-sequence metadata (AttnMeta.seq)")
-        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        sm.tickets, sm.parts = sq.step_tickets(self.embed, input_ids.shape[0]), False
         if sm.tickets is not None:
             sm.tickets.zero_()
         x, h = sq.layer_norm_residual(None, self.embed, self.embed_norm, self.cfg.norm_eps, self.dtype, ids=input_ids)

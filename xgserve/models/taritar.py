@@ -221,7 +221,7 @@ class TaritarForCausalLM(nn.Module):
         if sm is None:
             raise ValueError("Taritar needs the step's per-sequence metadata (AttnMeta.seq)")
         eps, dt, S, last, keep = self.cfg.norm_eps, self.dtype, self.cfg.streams, len(self.layers) - 1, self.keep_residuals
-        sm.tickets = sq.step_tickets(self.embed, input_ids.shape[0])
+        sm.tickets, sm.parts = sq.step_tickets(self.embed, input_ids.shape[0]), False
         x = sq.embed_rows(input_ids, self.embed, self.pos, sm.positions, self.cfg.embed_scale, tickets=sm.tickets)
         first = self.layers[0]
         x, n32, n = sq.hyper_residual(x, S, None, None, None, None, first.hc1.w_in, first.norm1, eps, dt)
