@@ -54,6 +54,7 @@ int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
 int latent_decode(const void*, const void*, int, int, const void*, int64_t, const void*, const int32_t*, int, int, const int32_t*,
                   const int32_t*, const int32_t*, const float*, int, const void*, void*, int, int, int, int, int, float, int,
                   float*, float*, hipStream_t);
+int gla_step_rows(int, int);
 int gla_step(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*, const void*,
              bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, const float*,
              const float*, hipStream_t);
@@ -329,6 +330,7 @@ PYBIND11_MODULE(_mixers, m) {
                              P<float>(part_ml), S(st)),
           "latent_decode");
   });
+  m.def("gla_step_rows", [](int dk, int dv) { return xgm::gla_step_rows(dk, dv); });
   m.def("gla_step", [](uintptr_t q, uintptr_t f, uintptr_t k, uintptr_t raw, int64_t ld_raw, int off_q, int off_f,
                        uintptr_t f_bias, uintptr_t lower, uintptr_t v, bool v_f32, int64_t ld_v, uintptr_t state, uintptr_t qsl,
                        uintptr_t seq_lens, uintptr_t slots, uintptr_t o, int ns, int H, int dk, int dv, uintptr_t decay,

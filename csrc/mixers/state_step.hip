@@ -214,24 +214,30 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const DeltaStepArgs a) 
   a.out[((int64_t)t * a.H + h) * D + d] = f2bf(od / sqrtf(ss / (float)D + a.eps) * nd * sigmoidf(gd));
 }
 
+// Rows of a [dk, dv] state that a thread of gla_step_kernel holds, 0 for a state that it does not take: dv a multiple of 4 up to
+// 256, dk up to 256, at most 16 rows (a thread's loads in flight). Where dv / 4 does not divide 256 some threads have no
+// column, so the area alone does not bound the rows: 128 x 128 takes 16, 88 x 176 would take 18.
+int gla_step_rows(int dk, int dv) {
+  if (dk < 1 || dk > 256 || dv < 4 || dv > 256 || dv % 4) return 0;
+  const int RG = 256 / (dv / 4), nr = (dk + RG - 1) / RG;
+  return nr <= 16 ? nr : 0;
+}
+
 static int launch_gla_step(const GlaStepArgs& a, bool v_f32, int ns, hipStream_t st) {
-  const int RG = 256 / (a.dv / 4), nr = (a.dk + RG - 1) / RG;
+  const int nr = gla_step_rows(a.dk, a.dv);
 #define XGM_GS(NR) XGM_DISPATCH_T(v_f32, gla_step_kernel<T, NR><<<dim3(a.H, ns), 256, 0, st>>>(a);)
-  if (nr <= 2) { XGM_GS(2) } else if (nr <= 4) { XGM_GS(4) } else if (nr <= 8) { XGM_GS(8) } else if (nr <= 16) { XGM_GS(16) } else {
-    return -1;
-  }
+  if (nr <= 2) { XGM_GS(2) } else if (nr <= 4) { XGM_GS(4) } else if (nr <= 8) { XGM_GS(8) } else { XGM_GS(16) }
 #undef XGM_GS
   return 0;
 }
 
-// One token per sequence (max_q == 1). Return -1 for sizes outside the contract: dv a multiple of 4 up to 256, dk up to 256,
-// dk dv up to 16384, aligned rows.
+// One token per sequence (max_q == 1). Return -1 for states outside gla_step_rows and for rows or states that are not aligned.
 int gla_step(const float* q, const float* f, const float* k, const void* raw, int64_t ld_raw, int off_q, int off_f,
              const float* f_bias, const float* lower, const void* v, bool v_f32, int64_t ld_v, float* state, const int32_t* qsl,
              const int32_t* seq_lens, const int32_t* slots, float* o, int ns, int H, int dk, int dv, const float* decay,
              const float* bonus, hipStream_t st) {
   if (ns <= 0) return 0;
-  if (H < 1 || dk < 1 || dk > 256 || dv < 4 || dv > 256 || dv % 4 || dk * dv > 16384 || ns > 65535 || ld_v % 4 ||
+  if (H < 1 || !gla_step_rows(dk, dv) || ns > 65535 || ld_v % 4 ||
       (uintptr_t)v % (v_f32 ? 16 : 8) || (uintptr_t)state % 16 || (raw ? (!lower || decay || bonus) : (!q || (!f && !decay))) ||
       ((decay || bonus) && !k))
     return -1;
@@ -244,7 +250,7 @@ int ssm_step(const void* xbc, bool f32, int64_t ld_x, const void* dt_raw, int64_
              const float* D, float* state, const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots, float* y, int ns,
              int H, int G, int N, int P, hipStream_t st) {
   if (ns <= 0) return 0;
-  if (H < 1 || G < 1 || H % G || N < 1 || N > 256 || P < 4 || P > 256 || P % 4 || N * P > 16384 || ns > 65535 || ld_x % 4 ||
+  if (H < 1 || G < 1 || H % G || !gla_step_rows(N, P) || ns > 65535 || ld_x % 4 ||
       (uintptr_t)xbc % (f32 ? 16 : 8) || (uintptr_t)state % 16 || !dt_raw)
     return -1;
   GlaStepArgs a = {};

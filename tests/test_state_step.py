@@ -139,3 +139,30 @@ def test_odd_states_run_as_scans():
     assert not sq._gla_step_ok(v, sm, 256, 128)
     sm.max_q = 2
     assert not sq._gla_step_ok(v, sm, 8, 8)
+
+
+@pytest.mark.parametrize("dk,dv", [(88, 176), (168, 96), (120, 136)])
+def test_states_with_too_many_rows_per_thread_run_as_scans(dk, dv):
+    """Sizes within 128 x 128 elements whose columns do not divide the workgroup: one token, through the public ops."""
+    g = torch.Generator().manual_seed(dk)
+    T, H, sm = len(SLOTS), 2, meta(SLOTS, CTX)
+    q, f, k = (torch.rand(T, H * dk, generator=g) for _ in range(3))
+    v, state = torch.randn(T, H * dv, generator=g), torch.randn(5, H, dk, dv, generator=g)
+    xbc = torch.randn(T, H * dv + 2 * dk, generator=g)
+    dt, bias, A, D = torch.randn(T, H, generator=g), torch.randn(H, generator=g), torch.randn(H, generator=g), torch.randn(H, generator=g)
+    st, st2 = state.cuda(), state.cuda()
+    o = sq.gated_linear_scan(q.cuda(), f.cuda(), k.cuda(), v.cuda(), st, H, dk, dv, sm).cpu().double()
+    y = sq.ssm_scan(xbc.cuda(), dt.cuda(), bias.cuda(), A.cuda(), D.cuda(), st2, H, 1, dk, dv, sm).cpu().double()
+    step = torch.nn.functional.softplus(dt.double() + bias.double())
+    for t, s in enumerate(SLOTS):
+        if s < 0:
+            continue
+        S = state[s].double() if CTX[t] else torch.zeros(H, dk, dv, dtype=torch.float64)
+        new = f[t].double().view(H, dk, 1) * S + k[t].double().view(H, dk, 1) * v[t].double().view(H, 1, dv)
+        want = (q[t].double().view(H, dk, 1) * new).sum(1).reshape(-1)
+        assert bool(((o[t] - want).abs() <= (dk + 40) * 2.0 ** -24 * (q[t].double().view(H, dk, 1) * new.abs()).sum(1).reshape(-1) * 4).all())
+        x, B, C = (z.double() for z in xbc[t].split([H * dv, dk, dk]))
+        new = torch.exp(-torch.exp(A.double()) * step[t])[:, None, None] * S + step[t][:, None, None] * B[:, None] * x.view(H, 1, dv)
+        want = (C[:, None] * new).sum(1) + D.double()[:, None] * x.view(H, dv)
+        mag = (C.abs()[:, None] * new.abs()).sum(1) + D.double().abs()[:, None] * x.abs().view(H, dv)
+        assert bool(((y[t].view(H, dv) - want).abs() <= (dk + 60) * 2.0 ** -24 * (mag + 1) * 4).all())

@@ -1534,7 +1534,8 @@ STATE_STEP = True
 
 
 def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int) -> bool:
-    return (STATE_STEP and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and dk <= 256 and dk * dv <= 16384
+    # (sizes: gla_step_rows of state_step.hip, at most 16 rows per thread)
+    return (STATE_STEP and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
             and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0)
 
 
