@@ -5,30 +5,35 @@
 //
 // The inputs are those of gated_linear_scan (fp32 tensors, or raw projection columns whose gates are formed while they are
 // staged) and ssm_scan. Token by token, either scan is a chain of one LDS round trip per token: 0.36 - 0.57 us a token
-// whatever the grid. With L_t the running sum of log2 decays from the chunk's start, a chunk is
-//   P_ij = sum_d q_i 2^(L_i) k_j 2^(-L_j) (j <= i),   o = P v + (q 2^L) S,   S <- 2^E (S + (k 2^-L)^T v)     (E = L_15)
-// and a scalar decay (ssm) factors out of the sums: P_ij = C_i . B_j dt_j 2^(L_i - L_j), no factor above 1 at all. Everything
-// stays fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32, so the results are as exact as the token loop's (operands
-// split into two bf16 terms would not be).
+// whatever the grid. With s_t the product of the decays behind token t up to the chunk's end and E that of all of them, a chunk is
+//   S' = E S,   P_ij = sum_d (q_i / s_i) (k_j s_j) (j <= i),   o = P v + (q / s) S',   S <- S' + (k s)^T v
+// and a scalar decay (ssm) factors out of the sums: P_ij = C_i . B_j dt_j s_j / s_i, no factor above 1 at all. Everything stays
+// fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32 (operands split into two bf16 terms would lose bits) and the products
+// of decays are carried as two floats (Prod). Referred to the chunk's end, the terms that enter the state have one rounding each,
+// as in the token loop; their reciprocals meet the outputs alone.
+// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets): 64 x 128, 1024 tokens, decays around 0.5
+// 6.1e-8 / 6.6e-8 (6.2e-8 / 6.1e-8), 0.95 3.4e-7 / 1.8e-7 (4.3e-7 / 2.1e-7), 0.999 3.5e-6 / 1.3e-6 (4.1e-6 / 1.5e-6); ssm,
+// 128 x 64, A = -0.6 7.4e-8 / 1.1e-7 (7.6e-8 / 1.2e-7), -1.6 6.9e-8 / 9.4e-8 (6.8e-8 / 1.1e-7). Sums of log2 decays in the place
+// of the products gave 3.3e-7 / 1.1e-7 in the first and 6.4e-7 / 2.7e-7 in the last.
 //
 // One workgroup = (sequence, head, 16 NW value columns). A wave keeps 16 columns of the state in accumulator layout, which is
-// also the B operand of (q 2^L) S when the contraction index runs (tile, register, row quad); v comes straight from memory
+// also the B operand of (q / s) S' when the contraction index runs (tile, register, row quad); v comes straight from memory
 // in the layout both products want; P is computed transposed, so that its accumulator layout is the A operand of P v. The
 // waves divide P's contraction and add their shares through LDS: one barrier per chunk, behind which only P v is left.
 // The next chunk is staged and the one after it loaded meanwhile.
 //
-// A chunk whose factors could leave the fp32 range (decays by more than 2^60 or growth by as much, inputs of 2^28 and above,
+// A chunk whose factors could leave the fp32 range (products of decays outside 2^-60 .. 2^60, inputs of 2^28 and above,
 // infinities, NaN) is run token by token in the same layout.
 //
-// Measured (bf16 rows): 4001 tokens of 16 heads of 64 x 128 404 -> 88 us, 4 x 2048 of them 734 -> 147; ssm, 2521 ragged tokens
-// of 64 heads of 128 x 64 781 -> 178, 4 x 1024 of 128 heads 1027 -> 247. What is left is 2.2 us of a compute unit per chunk of
-// the large state, 0.9 of them matrix instructions (68 a wave); the rest is LDS round trips between them. Workgroups of four
-// waves, two to a compute unit, because a lane holds 32 rows of state besides its fragments (184 registers).
+// Measured (bf16 rows): 4001 tokens of 16 heads of 64 x 128 401 -> 91 us, 4 x 2048 of them 734 -> 153; ssm, 2521 ragged tokens
+// of 64 heads of 128 x 64 778 -> 196, 4 x 1024 of 128 heads 1029 -> 270 (log sums: 87, 145, 187, 250). What is left is 2.3 us of
+// a compute unit per chunk of the large state, 0.9 of them matrix instructions (68 a wave); the rest is LDS round trips between
+// them. Workgroups of four waves, two to a compute unit, because a lane holds 32 rows of state besides its fragments (186
+// registers).
 //
 // Long portions of few sequences are cut into segments that run side by side: pass 1 sums every segment up from a zero state
 // (and sets the incoming state aside), a fold turns the sums into each segment's incoming state, pass 2 runs with outputs.
-// Segment slot of
-// (sequence s, segment z): q0_s / seg + s + z, distinct for all segments of a step.
+// Segment slot of (sequence s, segment z): q0_s / seg + s + z, distinct for all segments of a step.
 #include <type_traits>
 
 #include "mfma_f32.h"
@@ -40,7 +45,13 @@ using xgk::unpack8;
 
 constexpr int kCsRaw = 0, kCsPlain = 1, kCsSsm = 2;
 constexpr int kCsTok = 16;
-constexpr float kCsMaxLog2 = 60.f;
+constexpr float kCsMaxProd = 1152921504606846976.f, kCsMinProd = 1.f / kCsMaxProd;   // 2^60
+__device__ __forceinline__ bool prod_out_of_range(float p) { return !(fabsf(p) > kCsMinProd && fabsf(p) < kCsMaxProd); }
+
+// A chunk's tokens lie at these positions of its 16 rows, so that the four matrix steps of the state's update, which take rows
+// t, 4 + t, 8 + t and 12 + t, take tokens 4 t .. 4 t + 3: the terms join in the order of the token loop (ascending where decays
+// are strong; the other order costs the state 16 % of error at decays around 1/2).
+__device__ __forceinline__ int tok_pos(int t) { return (t & 3) << 2 | t >> 2; }
 
 struct ChunkScanArgs {
   const float *q, *f, *k;      // plain: fp32 [T][H dk] (k may be null)
@@ -79,7 +90,8 @@ template <> struct Raw8<float> {
 };
 
 template <typename T, int MODE, int DK, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanArgs a) {
+__global__ __launch_bounds__(64 * NW, NW == 8 && DK == 64 ? 4 : 2) void chunk_scan_kernel(const ChunkScanArgs a) {
+  constexpr bool DENSE = NW == 8 && DK == 64;   // two workgroups of eight waves to a compute unit (one: 4001 tokens 112 us, not 85)
   constexpr int C = kCsTok, MT = DK / 16, NTH = 64 * NW, QE = DK + 4;
   constexpr bool SSM = MODE == kCsSsm;
   constexpr int PT = (MT + NW - 1) / NW;       // 16-channel tiles of P's contraction per wave
@@ -89,9 +101,10 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
   constexpr int UN = (2 * C * DK / 8 + NTH - 1) / NTH;   // ssm: 8-channel units of [C | B] per thread
   __shared__ __attribute__((aligned(16))) float qs[2][C * QE], ks[2][C * QE];
   __shared__ __attribute__((aligned(16))) float ws[SSM ? 1 : 2][SSM ? 4 : C * QE];   // decays of a chunk run token by token
-  __shared__ __attribute__((aligned(16))) float es[SSM ? 1 : 2][SSM ? 4 : DK];       // 2^E per channel
+  __shared__ __attribute__((aligned(16))) float eh[SSM ? 1 : 2][SSM ? 4 : DK], el[SSM ? 1 : 2][SSM ? 4 : DK];   // E per channel
   __shared__ __attribute__((aligned(16))) float ps[2][NW][256];
-  __shared__ __attribute__((aligned(16))) float ls[RING][C], dts[RING][C], ltot[SSM ? 4 : DK];
+  __shared__ __attribute__((aligned(16))) float ri[RING][C], ds[RING][C], dts[RING][C];   // ssm: 1 / s, dt s, dt
+  __shared__ float Eh[RING], El[RING], ptot[SSM ? 4 : DK];   // ssm: E per chunk; gates: decay of the segment per channel
   __shared__ int flags[4][NW];
 
   // workgroups go to the 8 XCDs in turn: heads first, so that short sequences' missing segments empty no XCD, and an XCD
@@ -140,7 +153,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     if (last_seg) return;
   }
   if (!SSM)
-    for (int i = tid; i < DK; i += NTH) ltot[i] = 0.f;
+    for (int i = tid; i < DK; i += NTH) ptot[i] = 1.f;
 
   // ---- loads of a chunk into registers, unconverted (a conversion would wait for them); rows past the end repeat the last
   const T* raw = (const T*)a.raw;
@@ -149,7 +162,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
   using F = std::conditional_t<MODE == kCsPlain, float, T>;
   const int cl = lane % CW, tg = lane / CW, ch = CW * w + cl;   // gates: this lane's channel and tokens tg TL ..
   const uint32_t vcol = min(col, dv - 1), ccol = min(ch, dk - 1);
-  T vraw[4];                                           // v of tokens 4 g4 + r, column col
+  T vraw[4];                                           // v of tokens 4 r + g4 (positions 4 g4 + r), column col
   F rq[TLN], rf[TLN];
   float rk[MODE == kCsPlain ? TLN : 1];
   Raw8<T> un[SSM ? UN : 1];
@@ -159,7 +172,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     const int64_t row0 = q0 + min(t0, c1 - 1);
     const T* vp = vb + row0 * ld_v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) vraw[r] = vp[(uint32_t)min(4 * g4 + r, left) * (uint32_t)ld_v + vcol];
+    for (int r = 0; r < 4; ++r) vraw[r] = vp[(uint32_t)min(4 * r + g4, left) * (uint32_t)ld_v + vcol];
     if constexpr (SSM) {
       const T* rp = raw + row0 * a.ld_raw + gofs;
 #pragma unroll
@@ -184,13 +197,14 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
       }
     }
   };
-  // ---- gates and running log decays of the loaded chunk `ci`; whether it must run token by token
-  const float rate2 = SSM ? expf(a.A_log[h]) * kLog2e : 0.f, dtb = SSM ? a.dt_bias[h] : 0.f;
+  // ---- gates and running decays of the loaded chunk `ci`; whether it must run token by token
+  const float rate = SSM ? expf(a.A_log[h]) : 0.f, dtb = SSM ? a.dt_bias[h] : 0.f;
   float vnew[4];
-  float fq[TLN], ff[TLN], fk[TLN], lg[TLN];   // (lg: running log2 decay)
+  float fq[TLN], ff[TLN], fk[TLN];
+  Prod sg[TLN], E = {1.f, 0.f};
   const float low = MODE == kCsRaw ? a.lower[h * dk + ccol] : 0.f;
   const float fb = MODE == kCsRaw && a.f_bias ? a.f_bias[h * dk + ccol] : 0.f;
-  // ssm: step sizes and log decays of the BLK chunks from chunk `ci` on (a chunk is 16 lanes)
+  // ssm: step sizes and decays of the BLK chunks from chunk `ci` on (a chunk is 16 lanes)
   auto steps = [&](int ci) {
     const int t0 = c0 + C * ci;
     if (t0 >= c1) return;
@@ -199,13 +213,17 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     for (int j = 0; j < BLK * C / NTH; ++j) {
       const int t = tid + NTH * j, left = c1 - t0;
       const float d = t < left ? softplusf(ldf(dp + (int64_t)min(t, left - 1) * a.ld_dt) + dtb) : 0.f;
-      float L = -rate2 * d;
+      Prod p = {out_of_range(d) ? __builtin_nanf("") : expf(-rate * d), 0.f};   // (not a number: the chunk runs token by token)
 #pragma unroll
-      for (int o = 1; o < C; o <<= 1) {
-        const float up = __shfl_up(L, o, C);
-        if (l16 >= o) L += up;
+      for (int o = 1; o < C; o <<= 1) {   // from this token to the chunk's end
+        const Prod dn = {__shfl_down(p.h, o, C), __shfl_down(p.l, o, C)};
+        if (l16 + o < C) p = prod_mul(p, dn);
       }
-      ls[(ci + t / C) % RING][l16] = L, dts[(ci + t / C) % RING][l16] = d;
+      Prod s = {__shfl_down(p.h, 1, C), __shfl_down(p.l, 1, C)};
+      if (l16 == C - 1) s = {1.f, 0.f};
+      const int at = (ci + t / C) % RING, pos = tok_pos(l16);
+      ri[at][pos] = prod_rcp(s), ds[at][pos] = prod_times(s, d), dts[at][pos] = d;
+      if (l16 == 0) Eh[at] = p.h, El[at] = p.l;
     }
   };
   auto gates = [&](int ci, int t0) {
@@ -213,18 +231,17 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     bool bad = false;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      vnew[r] = cok && 4 * g4 + r < n ? ldf(&vraw[r]) : 0.f;
+      vnew[r] = cok && 4 * r + g4 < n ? ldf(&vraw[r]) : 0.f;
       bad |= out_of_range(vnew[r]);
     }
     if constexpr (!SSM) {
-      float run = 0.f;
 #pragma unroll
       for (int i = 0; i < TL; ++i) {
         const bool on = TL * tg + i < n && ch < dk;
         if constexpr (MODE == kCsRaw) {
           const float zq = ldf(&rq[i]);
-          ff[i] = on ? low + (1.f - low) * sigmoid2(ldf(&rf[i]) + fb) : 1.f;
-          fq[i] = on ? zq * sigmoid2(zq) : 0.f;
+          ff[i] = on ? low + (1.f - low) * sigmoidf(ldf(&rf[i]) + fb) : 1.f;
+          fq[i] = on ? siluf(zq) : 0.f;
           fk[i] = 1.f - ff[i];
         } else {
           ff[i] = on ? rf[i] : 1.f;
@@ -232,22 +249,27 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
           fk[i] = a.k ? (on ? rk[i] : 0.f) : 1.f - ff[i];
         }
         bad |= out_of_range(fq[i]) || out_of_range(fk[i]);
-        run += log2_fast(ff[i]);
-        lg[i] = run;
       }
-      float upto = run;   // the groups ahead of this lane's
+      Prod run = {1.f, 0.f};
 #pragma unroll
-      for (int o = 1; o < TG; o <<= 1) {
-        const float up = __shfl_up(upto, o * CW, 64);
-        if (tg >= o) upto += up;
+      for (int i = TL - 1; i >= 0; --i) {
+        sg[i] = run;
+        run = prod_mul(run, ff[i]);
       }
-      float before = __shfl_up(upto, CW, 64);
-      before = tg > 0 ? before : 0.f;
+#pragma unroll
+      for (int o = 1; o < TG; o <<= 1) {   // run: from this lane's group to the chunk's end
+        const Prod dn = {__shfl_down(run.h, o * CW, 64), __shfl_down(run.l, o * CW, 64)};
+        if (tg + o < TG) run = prod_mul(run, dn);
+      }
+      Prod after = {__shfl_down(run.h, CW, 64), __shfl_down(run.l, CW, 64)};
+      if (tg == TG - 1) after = {1.f, 0.f};
 #pragma unroll
       for (int i = 0; i < TL; ++i) {
-        lg[i] += before;
-        bad |= !(fabsf(lg[i]) < kCsMaxLog2);
+        sg[i] = prod_mul(sg[i], after);
+        bad |= prod_out_of_range(sg[i].h);
       }
+      E = run;   // (of the first group's lanes)
+      bad |= prod_out_of_range(E.h);
     }
     const int any = __any(bad);
     if (lane == 0) flags[ci & 3][w] = any;
@@ -256,8 +278,8 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     int f = 0;
 #pragma unroll
     for (int i = 0; i < NW; ++i) f |= flags[ci & 3][i];
-    // (a chunk's last log decay bounds them all)
-    return __builtin_amdgcn_readfirstlane(f | (SSM && !(ls[ci % RING][C - 1] > -kCsMaxLog2))) != 0;
+    // (ssm: a chunk's whole product bounds them all)
+    return __builtin_amdgcn_readfirstlane(f | (SSM && prod_out_of_range(Eh[ci % RING]))) != 0;
   };
   // ---- the loaded chunk's operands into LDS buffer `buf`
   auto stage = [&](int buf, bool slow, int n) {
@@ -269,7 +291,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
           float f[8];
           un[j].get(f);
           const bool on = tok < n && c < dk;
-          float* to = (is_b ? ks[buf] : qs[buf]) + tok * QE + c;
+          float* to = (is_b ? ks[buf] : qs[buf]) + tok_pos(tok) * QE + c;
           *reinterpret_cast<float4*>(to) = on ? make_float4(f[0], f[1], f[2], f[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
           *reinterpret_cast<float4*>(to + 4) = on ? make_float4(f[4], f[5], f[6], f[7]) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -277,20 +299,20 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     } else {
 #pragma unroll
       for (int i = 0; i < TL; ++i) {
-        const int at = (TL * tg + i) * QE + ch;
-        qs[buf][at] = slow ? fq[i] : fq[i] * exp2_fast(lg[i]);
-        ks[buf][at] = slow ? fk[i] : fk[i] * exp2_fast(-lg[i]);
+        const int at = tok_pos(TL * tg + i) * QE + ch;
+        qs[buf][at] = slow ? fq[i] : prod_div(fq[i], sg[i]);
+        ks[buf][at] = slow ? fk[i] : prod_times(sg[i], fk[i]);
         if (slow) ws[buf][at] = ff[i];
       }
-      if (tg == TG - 1) {
-        es[buf][ch] = exp2_fast(lg[TL - 1]);
-        ltot[ch] += lg[TL - 1];
+      if (tg == 0) {
+        eh[buf][ch] = E.h, el[buf][ch] = E.l;
+        ptot[ch] = slow ? ptot[ch] * E.h : prod_times(E, ptot[ch]);
       }
     }
   };
 
   const float skip = SSM ? a.skip[h] : 0.f;
-  float ltot_h = 0.f;   // ssm: log2 decay of the segment
+  float ptot_h = 1.f;   // ssm: decay of the segment
   float v[4];
   // chunk 0 staged, chunk 1 in registers
   fetch(c0);
@@ -313,42 +335,64 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
     for (int r = 0; r < 4; ++r) vn[r] = vnew[r];
     if (t0 + C < c1) stage(buf ^ 1, next_slow, c1 - t0 - C);
     if (more) fetch(t0 + 2 * C);
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};   // o: tokens 4 g4 + r, column col
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};   // o: tokens 4 r + g4, column col
     const float* Q = qs[buf];
     const float* K = ks[buf];
     if (slow) {
 #pragma unroll
-      for (int tg = 0; tg < 4; ++tg)
+      for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          const int t = 4 * tg + tt;
-          if (t < n) {
-            float vv = __shfl(v[tt], 16 * tg + l16, 64), dec = 0.f, sum = 0.f;
+        for (int tg = 0; tg < 4; ++tg) {
+          const int at = 4 * tg + tt;   // token 4 tt + tg
+          if (4 * tt + tg < n) {
+            float vv = __shfl(v[tt], 16 * tg + l16, 64), dec = 0.f, part[4] = {0.f, 0.f, 0.f, 0.f};
             if (SSM) {
-              dec = exp2f(-rate2 * dts[ci % RING][t]);
-              vv *= dts[ci % RING][t];
+              dec = expf(-rate * dts[ci % RING][at]);
+              vv *= dts[ci % RING][at];
+              ptot_h *= dec;
             }
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
               float qr[4], kr[4], wr[4] = {dec, dec, dec, dec};
-              ld4(Q + t * QE + 16 * m + 4 * g4, qr);
-              ld4(K + t * QE + 16 * m + 4 * g4, kr);
-              if (!SSM) ld4(ws[SSM ? 0 : buf] + t * QE + 16 * m + 4 * g4, wr);
+              ld4(Q + at * QE + 16 * m + 4 * g4, qr);
+              ld4(K + at * QE + 16 * m + 4 * g4, kr);
+              if (!SSM) ld4(ws[SSM ? 0 : buf] + at * QE + 16 * m + 4 * g4, wr);
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                S[m][r] = fmaf(wr[r], S[m][r], kr[r] * vv);
-                sum = fmaf(S[m][r], qr[r], sum);
+                S[m][r] = MODE == kCsRaw ? fmaf(wr[r], S[m][r] - vv, vv) : fmaf(wr[r], S[m][r], kr[r] * vv);
+                part[r] = fmaf(S[m][r], qr[r], part[r]);
               }
             }
+            float sum = (part[0] + part[1]) + (part[2] + part[3]);
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
             if (g4 == tg) acc[tt] = sum;
           }
         }
     } else {
+      // the state's own decay first
+      if constexpr (SSM) {
+        const Prod Ec = {Eh[ci % RING], El[ci % RING]};
+        ptot_h = prod_times(Ec, ptot_h);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[m][r] = prod_times(Ec, S[m][r]);
+      } else {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float e[4], f[4];
+          ld4(eh[SSM ? 0 : buf] + 16 * m + 4 * g4, e);
+          ld4(el[SSM ? 0 : buf] + 16 * m + 4 * g4, f);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[m][r] = prod_times({e[r], f[r]}, S[m][r]);
+        }
+      }
       if (pass != 1) {
-        // this wave's share of P^T: rows j = 4 g4 + r, column i = l16
-        f32x4_t pt = {0.f, 0.f, 0.f, 0.f};
+        // this wave's share of P^T: positions j = 4 g4 + r, column i = l16
+        f32x4_t pt[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pt[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int p = 0; p < PT; ++p) {
           const int m = w + NW * p;
@@ -357,92 +401,86 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
             ld4(K + l16 * QE + 16 * m + 4 * g4, kr);
             ld4(Q + l16 * QE + 16 * m + 4 * g4, qr);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pt = mfma_f32(kr[r], qr[r], pt);
+            for (int r = 0; r < 4; ++r) pt[r] = mfma_f32(kr[r], qr[r], pt[r]);
           }
         }
-        *reinterpret_cast<float4*>(&ps[buf][w][4 * lane]) = make_float4(pt[0], pt[1], pt[2], pt[3]);
-        f32x4_t acc2 = {0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<float4*>(&ps[buf][w][4 * lane]) = make_float4(
+            (pt[0][0] + pt[1][0]) + (pt[2][0] + pt[3][0]), (pt[0][1] + pt[1][1]) + (pt[2][1] + pt[3][1]),
+            (pt[0][2] + pt[1][2]) + (pt[2][2] + pt[3][2]), (pt[0][3] + pt[1][3]) + (pt[2][3] + pt[3][3]));
+        // four tiles' fragments in flight; sums side by side for short chains of roundings (two in the form that 128 registers hold)
+        constexpr int MB = MT < 4 ? MT : 4, NP = DENSE ? 2 : MB;
+        f32x4_t part[NP];
 #pragma unroll
-        for (int m0 = 0; m0 < MT; m0 += 4) {   // (four tiles' fragments in flight)
-          constexpr int MB = MT < 4 ? MT : 4;
+        for (int m = 0; m < NP; ++m) part[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m0 = 0; m0 < MT; m0 += 4) {
           float qr[MB][4];
 #pragma unroll
           for (int m = 0; m < MB; ++m) ld4(Q + l16 * QE + 16 * (m0 + m) + 4 * g4, qr[m]);
 #pragma unroll
-          for (int m = 0; m < MB; m += 2)
+          for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              acc = mfma_f32(qr[m][r], S[m0 + m][r], acc);
-              acc2 = mfma_f32(qr[m + 1][r], S[m0 + m + 1][r], acc2);
-            }
+            for (int m = 0; m < MB; ++m) part[m % NP] = mfma_f32(qr[m][r], S[m0 + m][r], part[m % NP]);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] += acc2[r];
+        for (int r = 0; r < 4; ++r) acc[r] = NP == 4 ? (part[0][r] + part[1][r]) + (part[NP - 2][r] + part[NP - 1][r]) : part[0][r] + part[1][r];
         if (SSM) {
-          float L[4];
-          ld4(&ls[ci % RING][4 * g4], L);
+          float x[4];
+          ld4(&ri[ci % RING][4 * g4], x);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[r] *= exp2_fast(L[r]);
+          for (int r = 0; r < 4; ++r) acc[r] *= x[r];
         }
       }
       float vs[4];
-      if constexpr (SSM) {   // the state's own decay first: every factor at most 1
-        float L[4], d[4];
-        ld4(&ls[ci % RING][4 * g4], L);
-        ld4(&dts[ci % RING][4 * g4], d);
-        const float E = ls[ci % RING][C - 1], fe = exp2_fast(E);
+      if constexpr (SSM) {
+        float d[4];
+        ld4(&ds[ci % RING][4 * g4], d);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vs[r] = v[r] * (d[r] * exp2_fast(E - L[r]));
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) S[m][r] *= fe;
+        for (int r = 0; r < 4; ++r) vs[r] = v[r] * d[r];
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) vs[r] = v[r];
       }
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < 4; ++t) S[m] = mfma_f32(K[(4 * g4 + t) * QE + 16 * m + l16], vs[t], S[m]);
-        if constexpr (!SSM) {
-          float e[4];
-          ld4(es[SSM ? 0 : buf] + 16 * m + 4 * g4, e);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) S[m][r] *= e[r];
-        }
-      }
     }
-    if (SSM && pass == 1) ltot_h += ls[ci % RING][C - 1];
     if (more) gates(ci + 2, t0 + 2 * C);
     if (SSM && ci % BLK == BLK / 2) steps(ci + BLK / 2);
     __syncthreads();
     if (pass != 1) {
       if (!slow) {
-        float p[4] = {0.f, 0.f, 0.f, 0.f};
+        constexpr int NP = MT < NW ? MT : NW;   // (2, 4 or 8 shares, added in pairs)
+        float p[4], x[NP][4];
 #pragma unroll
-        for (int i = 0; i < (MT < NW ? MT : NW); ++i) {
-          float x[4];
-          ld4(&ps[buf][i][4 * lane], x);
+        for (int i = 0; i < NP; ++i) ld4(&ps[buf][i][4 * lane], x[i]);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[r] += x[r];
-        }
+        for (int o = NP / 2; o > 0; o >>= 1)
+#pragma unroll
+          for (int i = 0; i < o; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[i][r] += x[i + o][r];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = x[0][r];
         if constexpr (SSM) {
-          float L[4], d[4];
-          ld4(&ls[ci % RING][4 * g4], L);
-          ld4(&dts[ci % RING][4 * g4], d);
-          const float Li = ls[ci % RING][l16];
+          float d[4];
+          ld4(&ds[ci % RING][4 * g4], d);
+          const float x = ri[ci % RING][l16];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[r] *= d[r] * exp2_fast(Li - L[r]);
+          for (int r = 0; r < 4; ++r) p[r] *= d[r] * x;
         }
+        f32x4_t pv = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc = mfma_f32(4 * g4 + r <= l16 ? p[r] : 0.f, v[r], acc);
+        for (int r = 0; r < 4; ++r) pv = mfma_f32(4 * r + g4 <= tok_pos(l16) ? p[r] : 0.f, v[r], pv);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] += pv[r];
       }
       if (cok) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (4 * g4 + r < n)
-            a.o[((int64_t)(q0 + t0 + 4 * g4 + r) * a.H + h) * dv + col] = SSM ? fmaf(skip, v[r], acc[r]) : acc[r];
+          if (4 * r + g4 < n)
+            a.o[((int64_t)(q0 + t0 + 4 * r + g4) * a.H + h) * dv + col] = SSM ? fmaf(skip, v[r], acc[r]) : acc[r];
       }
     }
 #pragma unroll
@@ -461,7 +499,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_scan_kernel(const ChunkScanA
       }
   }
   if (pass == 1 && blockIdx.z == 0)
-    for (int i = tid; i < dk; i += NTH) a.chA[((cs0 + z) * a.H + h) * dk + i] = exp2f(SSM ? ltot_h : ltot[SSM ? 0 : i]);
+    for (int i = tid; i < dk; i += NTH) a.chA[((cs0 + z) * a.H + h) * dk + i] = SSM ? ptot_h : ptot[SSM ? 0 : i];
 }
 
 // ================================================================== host launchers
@@ -491,7 +529,7 @@ __global__ __launch_bounds__(256) void chunk_scan_fold_kernel(const ChunkScanArg
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (z0 + j < nseg) {
-        S = fmaf(f[j], S, b[j]);
+        S = S == 0.f ? b[j] : fmaf(f[j], S, b[j]);   // (a product past fp32 of finite growths leaves a zero zero)
         B[(z0 + j) * stride] = S;
       }
     }

@@ -24,6 +24,31 @@ __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
 constexpr float kChunkMaxIn = 268435456.f;
 __device__ __forceinline__ bool out_of_range(float x) { return !(fabsf(x) < kChunkMaxIn); }
 
+// A running product of decays as the sum of two floats: the rounding of every factor is kept, so that a chunk's 16 steps cost the
+// state one rounding instead of 16. (A sum of logarithms is rounded to 2^-24 of its own size, which is an error of the decay
+// itself: at decays around 1/2 the state's was 5 to 9 times the token loop's.)
+struct Prod {
+  float h, l;
+};
+__device__ __forceinline__ Prod prod_mul(Prod a, float f) {
+  const float h = a.h * f;
+  return {h, fmaf(a.l, f, fmaf(a.h, f, -h))};
+}
+__device__ __forceinline__ Prod prod_mul(Prod a, Prod b) {
+  const float h = a.h * b.h;
+  return {h, fmaf(a.h, b.l, fmaf(a.l, b.h, fmaf(a.h, b.h, -h)))};
+}
+__device__ __forceinline__ float prod_times(Prod p, float x) { return fmaf(p.h, x, p.l * x); }
+// x / p and 1 / p: the reciprocal instruction and one Newton step
+__device__ __forceinline__ float prod_div(float x, Prod p) {
+  const float r = rcp_fast(p.h), t = x * r;
+  return fmaf(fmaf(-p.l, t, fmaf(-p.h, t, x)), r, t);
+}
+__device__ __forceinline__ float prod_rcp(Prod p) {
+  const float r = rcp_fast(p.h);
+  return fmaf(r, fmaf(-p.l, r, fmaf(-p.h, r, 1.f)), r);
+}
+
 // 1 / (1 + e^-x) from the exponential and reciprocal instructions; the product x log2 e in two terms keeps them to 2 ulp
 __device__ __forceinline__ float sigmoid2(float x) {
   x = x > 100.f ? -100.f : x < -100.f ? 100.f : -x;

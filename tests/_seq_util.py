@@ -73,3 +73,19 @@ def seq_meta(device, rows, block_size, tables):
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=device)  # noqa: E731
     return sq.SeqMeta(len(rows), max(r[2] for r in rows), i32(qsl), i32(sl), i32(slots), i32(bt), i32(tseq), i32(pos),
                       i32(smap))
+
+
+def record_native(monkeypatch, module):
+    """The names of the native entry points that `module` calls from here on, in order."""
+    real, names = module.mixers(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            f = getattr(real, name)
+
+            def call(*args):
+                names.append(name)
+                return f(*args)
+            return call
+    monkeypatch.setattr(module, "mixers", Recorder)
+    return names

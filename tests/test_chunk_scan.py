@@ -1,8 +1,9 @@
 """The chunked fp32 form of the outer-product recurrences (csrc/mixers/chunk_scan.hip) against the token loop in fp64.
 
-Tolerance: a chunk's factors are 2^(sum of at most 60 bits of decay); the sum carries 60 x 2^-24 of absolute error, a factor
-ln 2 times that, and a weight is the product of two of them: 60 x 2^-24 x 0.69 x 2 = 5e-6 of each term; 4 times that of the
-output's root mean square bounds the sums seen here. Chunks beyond 60 bits run token by token (2^-24 per step)."""
+Tolerance: a term of the state has one rounding of its factor and at most one of each sum that it is part of, as in the token
+loop, so an entry errs by some 2^-24 of its terms' sizes per token that it remembers; with gates close to one and k = 1 - f the
+rounding of the gate itself is 2^-24 / (1 - f) of a term. 2e-5 of the output's root mean square covers both for the sizes here.
+How the errors compare with the token loop's own is tested apart."""
 import math
 
 import pytest
@@ -10,7 +11,7 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
-from _seq_util import seq_meta
+from _seq_util import record_native, seq_meta
 
 F64 = torch.float64
 TOL = 2e-5
@@ -56,6 +57,7 @@ PORTIONS = [[(0, 16)], [(5, 15), (0, 16), (3, 1)], [(0, 17), (9, 33)], [(0, 300)
 @pytest.mark.parametrize("form", ["raw", "complement", "given"])
 @pytest.mark.parametrize("decay", ["mild", "steep", "zero"])
 def test_gates(portions, H, dk, dv, form, decay, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     monkeypatch.setattr(sq, "CHUNK_SCAN_MIN_SEG", 16)     # the long portion in segments, the short ones whole
     g = torch.Generator().manual_seed(dk * dv + len(portions))
     T, n = sum(p[1] for p in portions), H * dk
@@ -80,6 +82,7 @@ def test_gates(portions, H, dk, dv, form, decay, monkeypatch):
         got = sq.gated_linear_scan(zq.cuda(), f32.cuda(), None if k32 is None else k32.cuda(), v.cuda(), st, H, dk, dv, sm)
         q, f = zq.to(F64), f32.to(F64)
         k = 1 - f if k32 is None else k32.to(F64)
+    assert "chunk_scan_gates" in calls
     at = 0
     for i, (ctx, m) in enumerate(portions):
         S0 = state[i + 1].to(F64) * (ctx > 0)
@@ -97,6 +100,7 @@ def test_gates(portions, H, dk, dv, form, decay, monkeypatch):
 @pytest.mark.parametrize("rate", [0.0, 4.0])               # 4: e^4 of decay per unit of dt, past the chunk form's range
 def test_ssm(portions, H, G, N, P, dtype, rate, monkeypatch):
     monkeypatch.setattr(sq, "CHUNK_SCAN_MIN_SEG", 16)
+    calls = record_native(monkeypatch, sq)
     g = torch.Generator().manual_seed(N * P + len(portions))
     T = sum(p[1] for p in portions)
     sm = layout(portions)
@@ -107,6 +111,8 @@ def test_ssm(portions, H, G, N, P, dtype, rate, monkeypatch):
     state = torch.randn(len(portions) + 1, H, N, P, generator=g)
     st = state.cuda()
     got = sq.ssm_scan(xbc.cuda()[:, :W], dt.cuda(), bias.cuda(), A.cuda(), D.cuda(), st, H, G, N, P, sm)
+    # (B and C that do not lie on 16 bytes keep the token loop)
+    assert ("chunk_scan_ssm" in calls) == (H * P * xbc.element_size() % 16 == 0) and ("ssm_scan" in calls) != ("chunk_scan_ssm" in calls)
     d = torch.nn.functional.softplus(dt.to(F64) + bias.to(F64))
     f = torch.exp(-torch.exp(A.to(F64)) * d)[..., None].expand(T, H, N)
     x = xbc.to(F64)[:, :H * P].view(T, H, P)
@@ -136,3 +142,86 @@ def test_values_out_of_range_reach_what_the_token_loop_lets_them_reach(where, va
     close(got[:bad], ref[:bad].reshape(bad, -1))
     ref = ref.reshape(T, -1).float()   # (what fp32 holds of it)
     assert torch.equal(torch.isfinite(got[bad:]), torch.isfinite(ref[bad:]))
+
+
+def error(got, ref):
+    return float((got.detach().cpu().to(F64) - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("form", ["raw", "given", "ssm"])
+@pytest.mark.parametrize("level", [0, 1, 2, 3])
+@pytest.mark.parametrize("dk,dv,portion", [(64, 128, (3, 400)), (128, 64, (3, 400)), (32, 32, (3, 1500))])
+def test_errors_are_those_of_the_token_loop(form, level, dk, dv, portion, monkeypatch):
+    """The error against fp64 of outputs and of the carried state, beside the token loop's on the same inputs, from decays of
+    about 0.1 a token to 0.999. The chunks have as many roundings of a term as the loop; their order differs, so that either
+    may come out ahead: a tenth is allowed for it, and for an error below 2^-24 what its own rounding makes."""
+    g = torch.Generator().manual_seed(level + dk)
+    H, T = 4, portion[1]
+    sm = layout([portion])
+    state = torch.randn(2, H, dk, dv, generator=g)
+    if form == "ssm":
+        xbc = torch.randn(T, H * dv + 2 * dk, generator=g)
+        dt, bias, D = torch.randn(T, H, generator=g), torch.randn(H, generator=g) * 0.5 - 1, torch.randn(H, generator=g)
+        A = torch.randn(H, generator=g) * 0.3 + (1.0, 0.0, -2.0, -5.0)[level]
+        d = torch.nn.functional.softplus(dt.to(F64) + bias.to(F64))
+        f = torch.exp(-torch.exp(A.to(F64)) * d)[..., None].expand(T, H, dk)
+        x = xbc.to(F64)[:, :H * dv].view(T, H, dv)
+        B, C = (xbc.to(F64)[:, None, H * dv + i * dk:H * dv + (i + 1) * dk].expand(T, H, dk) for i in (0, 1))
+        ref, S = scan(C, f, d[..., None] * B, x, state[1].to(F64))
+        ref = ref + D.to(F64)[:, None] * x
+
+        def run(st):
+            return sq.ssm_scan(xbc.cuda(), dt.cuda(), bias.cuda(), A.cuda(), D.cuda(), st, H, 1, dk, dv, sm)
+    else:
+        n = H * dk
+        z, zq, v = (torch.randn(T, m, generator=g).bfloat16() for m in (n, n, H * dv))
+        z = (z.float() + (-2.0, 0.0, 3.0, 7.0)[level]).bfloat16()
+        f = torch.sigmoid(z.to(F64))
+        if form == "raw":
+            q, k, proj, low = torch.nn.functional.silu(zq.to(F64)), 1 - f, torch.cat([zq, z, v], 1).cuda(), torch.zeros(n).cuda()
+
+            def run(st):
+                return sq.lower_bound_recurrence(proj, 0, n, 2 * n, None, low, st, H, dk, dv, sm)
+        else:
+            f32, q32, k32 = f.float(), zq.float(), torch.randn(T, n, generator=g)
+            f, q, k = f32.to(F64), q32.to(F64), k32.to(F64)
+
+            def run(st):
+                return sq.gated_linear_scan(q32.cuda(), f32.cuda(), k32.cuda(), v.cuda(), st, H, dk, dv, sm)
+        ref, S = scan(*(t.view(T, H, -1) for t in (q, f, k, v.to(F64))), state[1].to(F64))
+    errs = []
+    for chunks in (True, False):
+        with monkeypatch.context() as m:
+            if not chunks:
+                m.setattr(sq, "_chunk_scan_ok", lambda *a: False)
+            calls, st = record_native(m, sq), state.cuda()
+            o = run(st)
+            assert any(c.startswith("chunk_scan_") for c in calls) == chunks
+        errs.append((error(o.view(T, H, dv), ref), error(st[1], S)))
+    (o, s), (o0, s0) = errs
+    assert o <= 1.1 * o0 + 2.0 ** -27 and s <= 1.1 * s0 + 2.0 ** -28, errs
+
+
+@pytest.mark.parametrize("segments", [False, True], ids=["one", "segments"])
+def test_negative_and_growing_decays(segments, monkeypatch):
+    """gated_linear_scan takes any f: signs alternate, factors above one, zeros; whole and in segments."""
+    g = torch.Generator().manual_seed(9)
+    H, dk, dv, T, ctx = 2, 64, 64, 700, 4
+    q, k = torch.randn(T, H * dk, generator=g), torch.randn(T, H * dk, generator=g)
+    f = torch.rand(T, H * dk, generator=g) * 0.9
+    f[torch.rand(T, H * dk, generator=g) < 0.05] *= -1.0
+    f[torch.rand(T, H * dk, generator=g) < 0.02] = 1.5
+    f[torch.rand(T, H * dk, generator=g) < 0.01] = 0.0
+    v, state = torch.randn(T, H * dv, generator=g), torch.randn(2, H, dk, dv, generator=g)
+    state[:, :, ::3] = 0.0
+    sm = layout([(ctx, T)])
+    if not segments:
+        monkeypatch.setattr(sq, "CHUNK_SCAN_MAX_SEGS", 1)
+    assert (sq._chunk_scan_segments(sm, T, H, dk, dv, 64, "cuda")[1] is not None) == segments
+    st = state.cuda()
+    calls = record_native(monkeypatch, sq)
+    got = sq.gated_linear_scan(q.cuda(), f.cuda(), k.cuda(), v.cuda(), st, H, dk, dv, sm)
+    assert "chunk_scan_gates" in calls
+    ref, S = scan(*(t.to(F64).view(T, H, -1) for t in (q, f, k, v)), state[1].to(F64))
+    close(got.view(T, H, dv), ref)
+    close(st[1], S)
