@@ -25,8 +25,8 @@
 // A chunk whose factors could leave the fp32 range (products of decays outside 2^-60 .. 2^60, inputs of 2^28 and above,
 // infinities, NaN) is run token by token in the same layout.
 //
-// Measured (bf16 rows): 4001 tokens of 16 heads of 64 x 128 401 -> 91 us, 4 x 2048 of them 734 -> 153; ssm, 2521 ragged tokens
-// of 64 heads of 128 x 64 778 -> 196, 4 x 1024 of 128 heads 1029 -> 270 (log sums: 87, 145, 187, 250). What is left is 2.3 us of
+// Measured (bf16 rows): 4001 tokens of 16 heads of 64 x 128 401 -> 92 us, 4 x 2048 of them 735 -> 155; ssm, 2521 ragged tokens
+// of 64 heads of 128 x 64 777 -> 199, 4 x 1024 of 128 heads 1030 -> 276 (log sums: 87, 145, 187, 250). What is left is 2.3 us of
 // a compute unit per chunk of the large state, 0.9 of them matrix instructions (68 a wave); the rest is LDS round trips between
 // them. Workgroups of four waves, two to a compute unit, because a lane holds 32 rows of state besides its fragments (186
 // registers).
@@ -78,6 +78,13 @@ template <> struct Raw8<bf16> {
   uint4 v;
   __device__ __forceinline__ void load(const bf16* p) { v = ld16(p); }
   __device__ __forceinline__ void get(float (&f)[8]) const { unpack8(v, f); }
+  __device__ __forceinline__ bool any_out_of_range() const {   // magnitudes order as their bits do, NaN above them all
+    using u16x2 = __attribute__((ext_vector_type(2))) uint16_t;
+    const u16x2 m = __builtin_elementwise_max(
+        __builtin_elementwise_max(__builtin_bit_cast(u16x2, v.x & 0x7FFF7FFFu), __builtin_bit_cast(u16x2, v.y & 0x7FFF7FFFu)),
+        __builtin_elementwise_max(__builtin_bit_cast(u16x2, v.z & 0x7FFF7FFFu), __builtin_bit_cast(u16x2, v.w & 0x7FFF7FFFu)));
+    return max(m.x, m.y) >= (__float_as_uint(kChunkMaxIn) >> 16);
+  }
 };
 template <> struct Raw8<float> {
   float4 a, b;
@@ -86,6 +93,14 @@ template <> struct Raw8<float> {
   }
   __device__ __forceinline__ void get(float (&f)[8]) const {
     f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w, f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
+  }
+  __device__ __forceinline__ bool any_out_of_range() const {
+    float f[8];
+    get(f);
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = max(m, __float_as_uint(f[i]) & 0x7FFFFFFFu);
+    return m >= __float_as_uint(kChunkMaxIn);
   }
 };
 
@@ -234,7 +249,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 && DK == 64 ? 4 : 2) void chunk_sc
       vnew[r] = cok && 4 * r + g4 < n ? ldf(&vraw[r]) : 0.f;
       bad |= out_of_range(vnew[r]);
     }
-    if constexpr (!SSM) {
+    if constexpr (SSM) {   // C . B is formed before dt x joins: large ones would leave the range where the token loop does not
+#pragma unroll
+      for (int j = 0; j < UN; ++j) bad |= un[j].any_out_of_range();
+    } else {
 #pragma unroll
       for (int i = 0; i < TL; ++i) {
         const bool on = TL * tg + i < n && ch < dk;

@@ -225,3 +225,49 @@ def test_negative_and_growing_decays(segments, monkeypatch):
     ref, S = scan(*(t.to(F64).view(T, H, -1) for t in (q, f, k, v)), state[1].to(F64))
     close(got.view(T, H, dv), ref)
     close(st[1], S)
+
+
+@pytest.mark.parametrize("where", ["x", "B", "C", "dt"])
+@pytest.mark.parametrize("value", [math.inf, math.nan, 1e36])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_state_space_values_out_of_range(where, value, dtype, monkeypatch):
+    """One bad input at token 21 of 48: the tokens before it stay what they are, and what is finite in the token loop is finite."""
+    g = torch.Generator().manual_seed(4)
+    H, N, P, T, bad = 1, 64, 64, 48, 21
+    xbc, dt = torch.rand(T, P + 2 * N, generator=g).to(dtype), torch.rand(T, H, generator=g).to(dtype)
+    (dt if where == "dt" else xbc)[bad, {"x": 5, "B": P + 7, "C": P + N + 9, "dt": 0}[where]] = value
+    zero, st = torch.zeros(H), torch.zeros(1, H, N, P).cuda()
+    sm = seq_meta("cuda", [(0, 0, T)], 16, [[0, 1, 2]])
+    calls = record_native(monkeypatch, sq)
+    got = sq.ssm_scan(xbc.cuda(), dt.cuda(), zero.cuda(), zero.cuda(), zero.cuda(), st, H, 1, N, P, sm).cpu()
+    assert "chunk_scan_ssm" in calls
+    d, z = torch.nn.functional.softplus(dt.to(F64)), xbc.to(F64)
+    ref, _ = scan(z[:, None, P + N:], torch.exp(-d)[..., None].expand(T, H, N), d[..., None] * z[:, None, P:P + N], z[:, None, :P],
+                  torch.zeros(H, N, P, dtype=F64))
+    ref = ref.reshape(T, -1)
+    close(got[:bad], ref[:bad])
+    # (+ D x with D = 0: an infinite x is not a number in the sum)
+    ref = (ref + 0.0 * z[:, :P]).float()
+    assert torch.equal(torch.isfinite(got[bad:]), torch.isfinite(ref[bad:]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_state_space_products_that_only_x_keeps_in_range(dtype):
+    """B and C whose product leaves fp32 beside an x that brings it back, and beside an x of 0."""
+    g = torch.Generator().manual_seed(5)
+    H, N, P, T = 2, 128, 64, 64
+    xbc = torch.rand(T, H * P + 2 * N, generator=g)
+    xbc[20:24, H * P:H * P + N] *= 1e30
+    xbc[:, H * P + N:] *= 1e15
+    xbc[20:24, :H * P] *= 1e-28
+    xbc[20:24, :8] = 0.0
+    xbc, dt = xbc.to(dtype), torch.rand(T, H, generator=g).to(dtype)
+    zero, state = torch.zeros(H), torch.randn(2, H, N, P, generator=g)
+    st = state.cuda()
+    got = sq.ssm_scan(xbc.cuda(), dt.cuda(), zero.cuda(), zero.cuda(), zero.cuda(), st, H, 1, N, P, layout([(2, T)]))
+    d, z = torch.nn.functional.softplus(dt.to(F64)), xbc.to(F64)
+    B, C = (z[:, None, H * P + i * N:H * P + (i + 1) * N].expand(T, H, N) for i in (0, 1))
+    ref, S = scan(C, torch.exp(-d)[..., None].expand(T, H, N), d[..., None] * B, z[:, :H * P].view(T, H, P), state[1].to(F64))
+    assert bool(torch.isfinite(ref).all())
+    close(got.view(T, H, P), ref)
+    close(st[1], S)

@@ -1466,9 +1466,9 @@ CHUNK_SCAN_MAX_DK = 128    # state rows a wave holds
 CHUNK_SCAN_MAX_SEQS = 2047   # (sequences x segments are one grid dimension)
 # Long portions are cut into segments until about two workgroups per compute unit run, of at least 64 tokens (128 for the
 # large state, whose sums cost more to write and fold), and into three or more: the second run over the tokens has to be paid
-# for. us whole / in segments: 4001 tokens of 16 heads of 64 x 128 731 / 88 (32), 4 x 2048 of 32 such heads 381 / 266 (4), 8
-# portions of about 650 of 16 136 / 114 (4); in two 16 x 512 of 16 heads 108 / 160, 8 x 650 of 32 137 / 198, 4 x 2048 of 64
-# heads of 128 x 64 337 / 409.
+# for. us whole / in segments: 4001 tokens of 16 heads of 64 x 128 775 / 89 (32), 4 x 2048 of 32 such heads 404 / 281 (4), 8
+# portions of about 650 of 16 133 / 116 (4); in two 16 x 512 of 16 heads 107 / 164, 8 x 650 of 32 135 / 202, 4 x 2048 of 64
+# heads of 128 x 64 372 / 443.
 CHUNK_SCAN_FILL_WGS = 512
 CHUNK_SCAN_MIN_SEG, CHUNK_SCAN_MAX_SEGS = 64, 32
 
