@@ -48,11 +48,6 @@ constexpr int kCsTok = 16;
 constexpr float kCsMaxProd = 1152921504606846976.f, kCsMinProd = 1.f / kCsMaxProd;   // 2^60
 __device__ __forceinline__ bool prod_out_of_range(float p) { return !(fabsf(p) > kCsMinProd && fabsf(p) < kCsMaxProd); }
 
-// A chunk's tokens lie at these positions of its 16 rows, so that the four matrix steps of the state's update, which take rows
-// t, 4 + t, 8 + t and 12 + t, take tokens 4 t .. 4 t + 3: the terms join in the order of the token loop (ascending where decays
-// are strong; the other order costs the state 16 % of error at decays around 1/2).
-__device__ __forceinline__ int tok_pos(int t) { return (t & 3) << 2 | t >> 2; }
-
 struct ChunkScanArgs {
   const float *q, *f, *k;      // plain: fp32 [T][H dk] (k may be null)
   const void* raw;             // raw: projection rows, columns off_q / off_f;  ssm: rows [x (H dv) | B (G dk) | C (G dk)]

@@ -2,35 +2,43 @@
 //
 //   S_t = diag(w_t) S_(t-1) - b_t (u_t^T S_(t-1)) + k_t v_t^T,   o_t = S_t^T r_t,      b = a u, u = k / |k|, w = e^(-c sigmoid)
 //
-// Token by token this is a chain of two reductions per token (0.45 us). Let L be the running sum of log2 w from the chunk's
-// start and u' = u 2^(L_(t-1)), b' = b 2^(-L_t), k' = k 2^(-L_t), r' = r 2^(L_t) (L loses at most 0.88 a token: 14 bits over a
-// chunk). With M = u' b'^T and N = u' k'^T strictly below the diagonal, P = r' k'^T and Q = r' b'^T up to it and
-// T = (1 + M)^-1, what token t takes out of the state is y = T (u' S + N v), and
-//   y = U S + V,           U = T u', V = T N v,
-//   o = R S + O,           R = r' - Q U, O = P v - Q V,
-//   S <- 2^(L_15) (S + k'^T v - b'^T y).
-// Only the right factors meet the state, so a first launch forms U, V, R, O, k', b' of all chunks at once (one wave per chunk
-// and head; T by forward substitution) and the chain that is left is three matrix products per 16 tokens. All of it is fp32
-// arithmetic.
+// Token by token this is a chain of two reductions per token (0.45 us). Let s_t be the product of the decays behind token t up to
+// the chunk's end, E that of all of them, S' = E S, and u' = u / s_(t-1), b' = b s_t, k' = k s_t, r' = r / s_t (a decay is at
+// least 0.545: 2^-14 over a chunk). With M = u' b'^T and N = u' k'^T strictly below the diagonal, P = r' k'^T and Q = r' b'^T up
+// to it and T = (1 + M)^-1, what token t takes out of the state is y = T (u' S' + N v), and
+//   y = (U E) S + V,       U = T u', V = T N v,
+//   o = (R E) S + O,       R = r' - Q U, O = P v - Q V,
+//   S <- E S + k'^T v - b'^T y.
+// Only the right factors meet the state, so a first launch forms U E, V, R E, O, k', b' of all chunks at once (one wave per chunk
+// and head; T by forward substitution: the compact form of a product of rank-one updates, Bischof and Van Loan 1987, as Yang et al.
+// 2024 use it for the delta rule over chunks of a sequence) and the chain that is left is three matrix products per 16 tokens. All of
+// it is fp32 arithmetic, the products of decays two floats each (Prod).
+//
+// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets), 2048 tokens of 32 heads of 64: decays around
+// 0.97 3.2e-7 / 2.2e-7 (3.1e-7 / 2.1e-7), 0.73 6.9e-8 / 6.6e-8 (6.6e-8 / 4.9e-8), 0.55 5.3e-8 / 6.1e-8 (4.6e-8 / 4.5e-8): the
+// output has four roundings of its size where the loop has two. (Sums of log2 decays and one chain per sum gave 1.8e-7 / 2.3e-7 in
+// the second.) That takes the separate sums: k . r has one sign in a trained model, and a chain of 64 rounds at the whole sum's
+// size; what is taken out of the state and of the outputs is summed up by itself before it joins them.
 //
 // The second launch has one wave per 16 state columns of a (sequence, head). The first writes every operand in the order of the
 // matrix instructions' lanes; the waves bring it in by LDS DMA, three chunks ahead (in registers, two chunks ahead, the compiler
 // parks operands in accumulator registers, which waits for every load: 2.1 us a chunk). A chunk with an input out of range
 // (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
 //
-// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1030 -> 336 us (126 + 210), one sequence of 2048
-// 860 -> 239, 64 tokens 32 -> 20. The first launch is at the memory's rate (it writes 24.6 KB per chunk and head); the second
-// takes 1.6 us a chunk, 0.9 of them its 64 matrix instructions a wave, the rest the way from one to the next: LDS reads behind
-// the barrier, and y, which has to be complete before it goes back in.
+// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1030 -> 368 us (147 + 247 in a trace), one sequence of 2048
+// 835 -> 266, 64 tokens 33 -> 23 (log sums in single chains: 325, 236, 21). The first launch writes 24.6 KB per chunk and head and
+// forms three exponentials per token and channel; the second takes 1.8 us a chunk, 0.9 of them its 64 matrix instructions a wave,
+// the rest the way from one to the next: LDS reads behind the barrier, and y, which has to be complete before it goes back in.
+// (E S is formed behind y's products: in front of them it cost 8 us of 280.)
 #include "glds.h"
 #include "mfma_f32.h"
 
 namespace xgm {
 
 constexpr int kDcTok = 16;
-constexpr float kDeltaDecayLog2 = -0.6065306597126334f * kLog2e;   // log2 w = this * sigmoid
+constexpr float kDeltaDecay = -0.6065306597126334f;   // log w = this * sigmoid
 
-// floats per (chunk, head): [U | R | k' | -b' | V | O] in lane order, then 2^E per channel, then the flag
+// floats per (chunk, head): [U E | R E | k' | -b' | V | O] in lane order, then E per channel, then the flag
 constexpr int dc_stride(int D) { return 6 * kDcTok * D + 256; }
 
 template <typename T, int D>
@@ -43,7 +51,7 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   constexpr int C = kDcTok, MT = D / 16, QE = D + 4, TPL = C * D / 64;   // (token, channel) pairs per lane
   constexpr int TG = 64 / D, TT = C / TG;                                // token groups, tokens per lane
   static_assert(D == 64 || D == 32, "a lane owns one channel");
-  __shared__ __attribute__((aligned(16))) float us[C * QE], rs[C * QE], ks[C * QE], bs[C * QE], ts[C * 20];
+  __shared__ __attribute__((aligned(16))) float us[C * QE], rs[C * QE], ks[C * QE], bs[C * QE], ts[C * 20], es[D];
   const int h = blockIdx.x, c = blockIdx.y, s = blockIdx.z;
   const int q0 = qsl[s], qn = qsl[s + 1] - q0, n = min(C, qn - C * c);
   if (slots[s] < 0 || n <= 0) return;
@@ -63,7 +71,7 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) xv[m][t] = row[(uint32_t)min(4 * g4 + t, n - 1) * (uint32_t)ld + off_v + 16 * m + l16];
+    for (int t = 0; t < 4; ++t) xv[m][t] = row[(uint32_t)min(4 * t + g4, n - 1) * (uint32_t)ld + off_v + 16 * m + l16];
   const float ab = a_bias[h * D + d], wb = w0[h * D + d];
   bool bad = false;
   float k[TT];
@@ -71,10 +79,10 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   for (int i = 0; i < TT; ++i) {
     k[i] = TT * tg + i < n ? ldf(&xk[i]) : 0.f;
     bad |= out_of_range(k[i]);
-    ks[(TT * tg + i) * QE + d] = k[i];
+    ks[tok_pos(TT * tg + i) * QE + d] = k[i];
   }
   __syncthreads();
-  float ksq = 0.f;   // |k|^2 of token l16
+  float ksq = 0.f;   // |k|^2 of the token at position l16
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     float x[4];
@@ -90,24 +98,18 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      v[m][t] = 4 * g4 + t < n ? ldf(&xv[m][t]) : 0.f;
+      v[m][t] = 4 * t + g4 < n ? ldf(&xv[m][t]) : 0.f;
       bad |= out_of_range(v[m][t]);
     }
-  float lw[TT], u[TT], a[TT], r_[TT], run = 0.f;
+  float wt[TT], u[TT], a[TT], r_[TT];
 #pragma unroll
   for (int i = 0; i < TT; ++i) {
     const bool on = TT * tg + i < n;
-    u[i] = k[i] * __shfl(inv, TT * tg + i, 64);
-    lw[i] = on ? kDeltaDecayLog2 * sigmoid2(ldf(&xw[i]) + wb) : 0.f;
-    a[i] = on ? sigmoid2(ldf(&xa[i]) + ab) : 0.f;
+    u[i] = k[i] * __shfl(inv, tok_pos(TT * tg + i), 64);
+    wt[i] = on ? expf(kDeltaDecay * sigmoidf(ldf(&xw[i]) + wb)) : 1.f;
+    a[i] = on ? sigmoidf(ldf(&xa[i]) + ab) : 0.f;
     r_[i] = on ? ldf(&xr[i]) : 0.f;
-    bad |= out_of_range(r_[i]) || out_of_range(a[i]) || out_of_range(lw[i]);
-    run += lw[i];
-  }
-  float L = 0.f;   // log decay ahead of this lane's tokens
-  if (TG == 2) {
-    const float up = __shfl_xor(run, D % 64, 64);
-    L = tg ? up : 0.f;
+    bad |= out_of_range(r_[i]) || out_of_range(a[i]) || out_of_range(wt[i]);
   }
   const bool slow = __any(bad);
   if (lane == 0) dst[6 * C * D + D] = slow ? 1.f : 0.f;
@@ -115,24 +117,33 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
 #pragma unroll
     for (int i = 0; i < TT; ++i) {
       float* to = dst + (TT * tg + i) * D + d;
-      to[0] = exp2f(lw[i]), to[C * D] = a[i] * u[i], to[2 * C * D] = u[i], to[3 * C * D] = k[i], to[4 * C * D] = r_[i];
+      to[0] = wt[i], to[C * D] = a[i] * u[i], to[2 * C * D] = u[i], to[3 * C * D] = k[i], to[4 * C * D] = r_[i];
     }
     return;
   }
   __syncthreads();   // (ks is rewritten)
+  Prod run = {1.f, 0.f};   // from the token behind this one to the chunk's end
+  if (TG == 2) {
 #pragma unroll
-  for (int i = 0; i < TT; ++i) {
-    const int at = (TT * tg + i) * QE + d;
-    us[at] = u[i] * exp2_fast(L);
-    L += lw[i];
-    const float e = exp2_fast(L), f = exp2_fast(-L);
-    rs[at] = r_[i] * e, ks[at] = k[i] * f, bs[at] = a[i] * u[i] * f;
+    for (int i = 0; i < TT; ++i) run = prod_mul(run, wt[i]);
+    const Prod up = {__shfl_xor(run.h, D % 64, 64), __shfl_xor(run.l, D % 64, 64)};
+    run = tg ? Prod{1.f, 0.f} : up;
   }
-  if (tg == TG - 1) dst[6 * C * D + d] = exp2_fast(L);
+#pragma unroll
+  for (int i = TT - 1; i >= 0; --i) {
+    const int at = tok_pos(TT * tg + i) * QE + d;
+    rs[at] = prod_div(r_[i], run), ks[at] = prod_times(run, k[i]), bs[at] = prod_times(run, a[i] * u[i]);
+    run = prod_mul(run, wt[i]);
+    us[at] = prod_div(u[i], run);
+  }
+  if (tg == 0) es[d] = dst[6 * C * D + d] = run.h + run.l;
   __syncthreads();
 
-  // ---- the four 16 x 16 products, transposed: lane holds [token l16][token 4 g4 + r], the A operand of what follows
-  f32x4_t M = {0.f, 0.f, 0.f, 0.f}, N = M, P = M, Q = M;
+  // ---- the four 16 x 16 products, transposed: lane holds [position l16][position 4 g4 + r], the A operand of what follows. Each is
+  // the sum of four chains (k . r of a trained model has one sign: a chain of 64 would round at the size of the whole sum).
+  f32x4_t Mc[4], Nc[4], Pc[4], Qc[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) Mc[r] = Nc[r] = Pc[r] = Qc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     float xu[4], xrr[4], xkk[4], xb[4];
@@ -140,39 +151,45 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
     ld4(us + at, xu), ld4(rs + at, xrr), ld4(ks + at, xkk), ld4(bs + at, xb);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      M = mfma_f32(xb[r], xu[r], M);
-      N = mfma_f32(xkk[r], xu[r], N);
-      P = mfma_f32(xkk[r], xrr[r], P);
-      Q = mfma_f32(xb[r], xrr[r], Q);
+      Mc[r] = mfma_f32(xb[r], xu[r], Mc[r]);
+      Nc[r] = mfma_f32(xkk[r], xu[r], Nc[r]);
+      Pc[r] = mfma_f32(xkk[r], xrr[r], Pc[r]);
+      Qc[r] = mfma_f32(xb[r], xrr[r], Qc[r]);
     }
   }
+  float M[4], N[4], P[4], Q[4];
+  const int ti = tok_pos(l16);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int j = 4 * g4 + r;
-    M[r] = j < l16 ? M[r] : 0.f, N[r] = j < l16 ? N[r] : 0.f;
-    P[r] = j <= l16 ? P[r] : 0.f, Q[r] = j <= l16 ? -Q[r] : 0.f;   // (Q enters with its sign)
+    const int j = 4 * r + g4;   // the token at position 4 g4 + r
+    M[r] = j < ti ? (Mc[0][r] + Mc[1][r]) + (Mc[2][r] + Mc[3][r]) : 0.f;
+    N[r] = j < ti ? (Nc[0][r] + Nc[1][r]) + (Nc[2][r] + Nc[3][r]) : 0.f;
+    P[r] = j <= ti ? (Pc[0][r] + Pc[1][r]) + (Pc[2][r] + Pc[3][r]) : 0.f;
+    Q[r] = j <= ti ? -((Qc[0][r] + Qc[1][r]) + (Qc[2][r] + Qc[3][r])) : 0.f;   // (Q enters with its sign)
   }
   *reinterpret_cast<float4*>(ts + l16 * 20 + 4 * g4) = make_float4(M[0], M[1], M[2], M[3]);
   __syncthreads();
-  // ---- T = (1 + M)^-1: lane l16 solves for column l16, x_i = delta - sum_(j < i) M_ij x_j
+  // ---- T = (1 + M)^-1: lane l16 solves for token l16's column, x_i = delta - sum_(j < i) M_ij x_j
   float x[C];
 #pragma unroll
   for (int i = 0; i < C; ++i) {
     float acc = i == l16 ? 1.f : 0.f;
 #pragma unroll
-    for (int j4 = 0; j4 < (i + 3) / 4; ++j4) {
-      float mm[4];
-      ld4(ts + i * 20 + 4 * j4, mm);
+    for (int a = 0; a < 4; ++a) {
+      if (a < i) {
+        float mm[4];   // tokens a, a + 4, a + 8, a + 12
+        ld4(ts + tok_pos(i) * 20 + 4 * a, mm);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (4 * j4 + r < i) acc = fmaf(-mm[r], x[4 * j4 + r], acc);
+        for (int r = 0; r < 4; ++r)
+          if (a + 4 * r < i) acc = fmaf(-mm[r], x[a + 4 * r], acc);
+      }
     }
     x[i] = acc;
   }
   __syncthreads();
   if (g4 == 0) {
 #pragma unroll
-    for (int i = 0; i < C; ++i) ts[i * 20 + l16] = x[i];
+    for (int i = 0; i < C; ++i) ts[tok_pos(i) * 20 + tok_pos(l16)] = x[i];
   }
   __syncthreads();
   float Tf[4];
@@ -181,7 +198,7 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   auto put = [&](int which, int m, f32x4_t y) {
     *reinterpret_cast<float4*>(dst + which * C * D + 256 * m + 4 * lane) = make_float4(y[0], y[1], y[2], y[3]);
   };
-  // ---- U (transposed product: token l16, channels 16 m + 4 g4 + r); k' and -b' as the A operands of the state's update
+  // ---- U (transposed product: position l16, channels 16 m + 4 g4 + r); k' and -b' as the A operands of the state's update
   f32x4_t U[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -193,7 +210,9 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
       U[m] = mfma_f32(us[at], Tf[t], U[m]);
       kk[t] = ks[at], bb[t] = -bs[at];
     }
-    put(0, m, U[m]), put(2, m, kk), put(3, m, bb);
+    float e[4];
+    ld4(es + 16 * m + 4 * g4, e);
+    put(0, m, f32x4_t{U[m][0] * e[0], U[m][1] * e[1], U[m][2] * e[2], U[m][3] * e[3]}), put(2, m, kk), put(3, m, bb);
   }
   __syncthreads();
 #pragma unroll
@@ -205,17 +224,20 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   for (int m = 0; m < MT; ++m) {
     float r0[4];
     ld4(rs + l16 * QE + 16 * m + 4 * g4, r0);
-    f32x4_t R = {r0[0], r0[1], r0[2], r0[3]};
+    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, V = y, O = y, R = y, QV = y;   // (what is taken out is summed up by itself: no roundings of the whole)
 #pragma unroll
     for (int t = 0; t < 4; ++t) R = mfma_f32(us[(4 * g4 + t) * QE + 16 * m + l16], Q[t], R);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) R[t] = (R[t] + r0[t]) * es[16 * m + 4 * g4 + t];
     put(1, m, R);
-    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, V = y, O = y;
 #pragma unroll
     for (int t = 0; t < 4; ++t) y = mfma_f32(N[t], v[m][t], y), O = mfma_f32(P[t], v[m][t], O);
 #pragma unroll
     for (int t = 0; t < 4; ++t) V = mfma_f32(Tf[t], y[t], V);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) O = mfma_f32(Q[t], V[t], O);
+    for (int t = 0; t < 4; ++t) QV = mfma_f32(Q[t], V[t], QV);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) O[t] += QV[t];
     put(4, m, V), put(5, m, O);
   }
 }
@@ -228,7 +250,7 @@ __global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float*
                                                                     const int32_t* __restrict__ slots, float* __restrict__ o,
                                                                     int H) {
   constexpr int C = kDcTok, MT = D / 16, NW = MT, RING = 4;
-  constexpr int FRAG = 6 * C * D * 4, SLOT = FRAG + 1024 + C * D * sizeof(T);   // bytes: [U .. O | 2^E, flag | v rows]
+  constexpr int FRAG = 6 * C * D * 4, SLOT = FRAG + 1024 + C * D * sizeof(T);   // bytes: [U .. O | E, flag | v rows]
   constexpr int VL = D * sizeof(T) / 16, VR = C / NW;                            // lanes per v row, v rows per wave
   constexpr int DMA = 6 * C * D * 4 / 1024 / NW + 2;                             // loads per wave and chunk
   __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT];
@@ -277,9 +299,9 @@ __global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float*
     float* ob = o + ((int64_t)(q0 + C * c) * H + h) * D + col;
     float v[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = ldf(pv + (4 * g4 + t) * D);
+    for (int t = 0; t < 4; ++t) v[t] = ldf(pv + (4 * t + g4) * D);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = 4 * g4 + t < n ? v[t] : 0.f;
+    for (int t = 0; t < 4; ++t) v[t] = 4 * t + g4 < n ? v[t] : 0.f;
     if (__builtin_amdgcn_readfirstlane(pe[D] != 0.f)) {
       for (int t = 0; t < n; ++t) {
         const float vv = ldf(pv + t * D);
@@ -311,43 +333,47 @@ __global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float*
       continue;
     }
     const float4 v0 = p4[64 * (4 * MT + w)], o0 = p4[64 * (5 * MT + w)];
-    f32x4_t y = {v0.x, v0.y, v0.z, v0.w}, out = {o0.x, o0.y, o0.z, o0.w};
     float4 k[MT], b[MT];
+    float e[MT][4];
+    f32x4_t yc[2], oc[2];   // two chains each: even and odd 16s of the state's rows
+    yc[0] = yc[1] = oc[0] = oc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const float4 u = p4[64 * m], r = p4[64 * (MT + m)];
-      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)];
-      y = mfma_f32(u.x, S[m][0], y), out = mfma_f32(r.x, S[m][0], out);
-      y = mfma_f32(u.y, S[m][1], y), out = mfma_f32(r.y, S[m][1], out);
-      y = mfma_f32(u.z, S[m][2], y), out = mfma_f32(r.z, S[m][2], out);
-      y = mfma_f32(u.w, S[m][3], y), out = mfma_f32(r.w, S[m][3], out);
+      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)], ld4(pe + 16 * m + 4 * g4, e[m]);
+      yc[m % 2] = mfma_f32(u.x, S[m][0], yc[m % 2]), oc[m % 2] = mfma_f32(r.x, S[m][0], oc[m % 2]);
+      yc[m % 2] = mfma_f32(u.y, S[m][1], yc[m % 2]), oc[m % 2] = mfma_f32(r.y, S[m][1], oc[m % 2]);
+      yc[m % 2] = mfma_f32(u.z, S[m][2], yc[m % 2]), oc[m % 2] = mfma_f32(r.z, S[m][2], oc[m % 2]);
+      yc[m % 2] = mfma_f32(u.w, S[m][3], yc[m % 2]), oc[m % 2] = mfma_f32(r.w, S[m][3], oc[m % 2]);
     }
+    // E S + k' v behind y's last products; what is taken out is summed up by itself
+    f32x4_t by[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], S[m]);   // (independent of y: behind its last products)
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], f32x4_t{e[m][0] * S[m][0], e[m][1] * S[m][1], e[m][2] * S[m][2], e[m][3] * S[m][3]});
 #pragma unroll
     for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].y, v[1], S[m]);
 #pragma unroll
     for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].z, v[2], S[m]);
 #pragma unroll
     for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].w, v[3], S[m]);
+    const float y[4] = {yc[0][0] + yc[1][0] + v0.x, yc[0][1] + yc[1][1] + v0.y, yc[0][2] + yc[1][2] + v0.z, yc[0][3] + yc[1][3] + v0.w};
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].x, y[0], S[m]);
+    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].x, y[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].y, y[1], S[m]);
+    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].y, y[1], by[m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].z, y[2], S[m]);
+    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].z, y[2], by[m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(b[m].w, y[3], S[m]);
+    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].w, y[3], by[m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      float e[4];
-      ld4(pe + 16 * m + 4 * g4, e);
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[m][r] *= e[r];
-    }
+      for (int r = 0; r < 4; ++r) S[m][r] += by[m][r];
+    const float out[4] = {oc[0][0] + oc[1][0] + o0.x, oc[0][1] + oc[1][1] + o0.y, oc[0][2] + oc[1][2] + o0.z,
+                          oc[0][3] + oc[1][3] + o0.w};
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (4 * g4 + r < n) ob[(int64_t)(4 * g4 + r) * H * D] = out[r];
+      if (4 * r + g4 < n) ob[(int64_t)(4 * r + g4) * H * D] = out[r];
   }
   xgk::wait_vmcnt<0>();   // (no load may land after the workgroup's LDS is given on)
 #pragma unroll

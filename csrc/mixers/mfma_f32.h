@@ -19,6 +19,11 @@ __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
 #endif
 }
 
+// A chunk's tokens lie at these positions of its 16 rows (an involution), so that the four matrix steps of the state's update, which
+// take rows t, 4 + t, 8 + t and 12 + t, take tokens 4 t .. 4 t + 3: the terms join in the order of the token loop (ascending where
+// decays are strong; the other order costs the state 16 % of error at decays around 1/2).
+__device__ __forceinline__ constexpr int tok_pos(int t) { return (t & 3) << 2 | t >> 2; }
+
 // inputs past 2^28, infinities and NaN: a chunk that holds one runs token by token (a masked 0 times infinity would reach
 // the tokens before it)
 constexpr float kChunkMaxIn = 268435456.f;
@@ -47,13 +52,6 @@ __device__ __forceinline__ float prod_div(float x, Prod p) {
 __device__ __forceinline__ float prod_rcp(Prod p) {
   const float r = rcp_fast(p.h);
   return fmaf(r, fmaf(-p.l, r, fmaf(-p.h, r, 1.f)), r);
-}
-
-// 1 / (1 + e^-x) from the exponential and reciprocal instructions; the product x log2 e in two terms keeps them to 2 ulp
-__device__ __forceinline__ float sigmoid2(float x) {
-  x = x > 100.f ? -100.f : x < -100.f ? 100.f : -x;
-  const float t = x * kLog2e, lo = fmaf(x, kLog2e, -t) + x * 1.9259629e-8f, e = exp2_fast(t);
-  return rcp_fast(1.f + fmaf(e, lo * 0.69314718f, e));
 }
 
 }  // namespace xgm

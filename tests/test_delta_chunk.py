@@ -1,7 +1,8 @@
 """The chunked form of the generalized delta rule (csrc/mixers/delta_chunk.hip) against the token loop in fp64.
 
-Tolerance: a chunk's factors are 2^(up to 14 bits of decay) whose exponents carry 14 x 2^-24 of absolute error: 14 x 2^-24 x 0.69
-x 2 = 1.2e-6 of a term, two products deep, over sums of up to 64 terms of either sign: 2e-5 of the output's root mean square."""
+Tolerance: a term has one rounding of each factor and one of each sum that it is part of, some 2^-24 of its size per token that the
+state remembers; keys that repeat make the terms larger than their sum. 2e-5 of the output's root mean square covers the sizes
+here. How the errors compare with the token loop's own is tested apart."""
 import math
 
 import pytest
@@ -9,8 +10,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
-from _seq_util import seq_meta
-from test_chunk_scan import close, layout
+from _seq_util import record_native
+from test_chunk_scan import close, error, layout
 
 F64 = torch.float64
 pytestmark = pytest.mark.gpu
@@ -48,7 +49,7 @@ def case(portions, H, D, dtype, g, tweak=lambda x: None):
 @pytest.mark.parametrize("H,D", [(3, 32), (2, 64), (5, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("keys", ["random", "repeated", "none"])
-def test_portions(portions, H, D, dtype, keys):
+def test_portions(portions, H, D, dtype, keys, monkeypatch):
     """repeated: every token removes what the last one wrote (the triangular system at its fullest); none: zero keys."""
     def tweak(x):
         if keys == "repeated":
@@ -56,7 +57,9 @@ def test_portions(portions, H, D, dtype, keys):
             x["a"] += 6.0
         elif keys == "none":
             x["k"][::2] = 0.0
+    calls = record_native(monkeypatch, sq)
     got, st, state, t = case(portions, H, D, dtype, torch.Generator().manual_seed(H * D + len(portions)), tweak)
+    assert calls.count("delta_chunk") == 1 and "delta_scan" not in calls
     at = 0
     for i, (ctx, m) in enumerate(portions):
         r = slice(at, at + m)
@@ -76,3 +79,26 @@ def test_values_out_of_range_reach_what_the_token_loop_lets_them_reach(where, va
     ref, _ = reference(t, state[1].to(F64) * 0)
     close(got[:21], ref[:21])
     assert torch.equal(torch.isfinite(got[21:].cpu()), torch.isfinite(ref[21:].float()))
+
+
+@pytest.mark.parametrize("mid", [-4.0, 0.0, 4.0])
+@pytest.mark.parametrize("H,D", [(4, 32), (4, 64)])
+def test_errors_are_those_of_the_token_loop(mid, H, D, monkeypatch):
+    """Errors against fp64 beside the token loop's on the same inputs, decays around 0.97, 0.73 and 0.55. A state's terms have as
+    many roundings as in the loop (in another order: a fifth is allowed); an output is the sum of four parts of its size, each
+    rounded, where the loop's has two: its error may be 2^(1/2) times as large (and a tenth for chance)."""
+    def tweak(x):
+        x["w"] += mid
+        x["r"] = 0.8 * x["r"] + 0.6 * x["k"]
+    errs = []
+    for chunks in (True, False):
+        with monkeypatch.context() as m:
+            if not chunks:
+                m.setattr(sq, "DELTA_CHUNK_MIN", 1 << 30)
+            calls = record_native(m, sq)
+            got, st, state, t = case([(3, 700)], H, D, torch.bfloat16, torch.Generator().manual_seed(D), tweak)
+            assert ("delta_chunk" in calls) == chunks
+        o, S = reference(t, state[1].to(F64))
+        errs.append((error(got, o), error(st[1], S)))
+    (o, s), (o0, s0) = errs
+    assert o <= 1.55 * o0 and s <= 1.2 * s0, errs

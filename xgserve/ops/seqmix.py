@@ -602,8 +602,8 @@ DECAY_SCALE = math.exp(-0.5)
 # XGS_TUNE delta_two_pass=0: the one-pass scan kernel (any head size; A/B and tests)
 DELTA_TWO_PASS = tune.get_bool("delta_two_pass", True)
 UNIT_KEY_EPS = 1e-6
-# prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on: one chunk
-# takes what 16 tokens of the scan take (15.1 against 15.0 us, 32 heads of 64), four take 20 against 32
+# prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on, which take what
+# 32 tokens of the scan take (19.7 against 19.8 us, 32 heads of 64): one takes 17.9 against 14.2, four 23 against 33
 DELTA_CHUNK = True
 DELTA_CHUNK_D = (32, 64)
 DELTA_CHUNK_MIN = 32
