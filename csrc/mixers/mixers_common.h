@@ -87,26 +87,28 @@ __device__ __forceinline__ float seg_sum(float v, int L) {
   return v;
 }
 
-// e^z - 1 - z for z <= 0: near zero its power series (z^2 / 2 + .. + z^8 / 8!, the rest is below 2^-24 of it for |z| < 1/2), which
-// also spares the difference of two close numbers; else the exponential itself (the sum is above 0.1 there)
+// e^z - 1 - z for z <= 0. Above -1, z^2 times the polynomial that interpolates the quotient at the 7 Chebyshev points of [-1, 0]
+// (1e-8 of it off), which spares the difference of close numbers; else the exponential itself (the difference is above 1/3).
 __device__ __forceinline__ float exp_tail(float z) {
+  float p = fmaf(z, 1.6928126569837332e-05f, 0.00018832476052921265f);
+  p = fmaf(z, p, 0.0013822416076436639f);
+  p = fmaf(z, p, 0.008331050164997578f);
+  p = fmaf(z, p, 0.041666291654109955f);
+  p = fmaf(z, p, 0.166666641831398f);
+  p = fmaf(z, p, 0.5f);
 #if defined(__HIP_DEVICE_COMPILE__)
   const float e = __builtin_amdgcn_exp2f(z * 1.44269504f);
 #else
   const float e = expf(z);
 #endif
-  float p = fmaf(z, 1.f / 40320.f, 1.f / 5040.f);
-  p = fmaf(z, p, 1.f / 720.f);
-  p = fmaf(z, p, 1.f / 120.f);
-  p = fmaf(z, p, 1.f / 24.f);
-  p = fmaf(z, p, 1.f / 6.f);
-  p = fmaf(z, p, 0.5f);
-  return z > -0.5f ? z * z * p : (e - 1.f) - z;
+  return z > -1.f ? z * z * p : (e - 1.f) - z;
 }
 
-// xIELU: sp z^2 + z / 2 for z > 0, cn (e^z - 1 - z) + z / 2 else
+// xIELU: sp z^2 + z / 2 for z > 0, cn (e^z - 1 - z) + z / 2 else. z / 2 is exact, so it joins in the last multiply-add.
+// Error of the fp32 result against fp64 (2-norm over a range of z; in brackets with expm1f and every operation rounded): above
+// -1/2 3.4e-8 (1.0e-7), -1 to -1/2 1.2e-7 (1.8e-7), -2 to -1 1.8e-7 (2.1e-7), 0 to 5 3.3e-8 (4.0e-8).
 __device__ __forceinline__ float xieluf(float z, float sp, float cn) {
-  return z > 0.f ? sp * z * z + 0.5f * z : cn * exp_tail(z) + 0.5f * z;
+  return fmaf(z > 0.f ? sp * z : cn, z > 0.f ? z : exp_tail(z), 0.5f * z);
 }
 
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }

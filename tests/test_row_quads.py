@@ -151,3 +151,24 @@ def test_head_norm(dk, rot_dims, half, dt):
         if s >= 0:
             close(k[s], want[t], dk / 2 + 16, float(want.abs().max()))
             assert torch.equal(v[s].cpu(), src[t, (H + G) * dk:].to(dt))
+
+
+@pytest.mark.parametrize("lo,hi", [(-0.5, 0.0), (-1.0, -0.5), (-2.0, -1.0), (-30.0, -2.0), (0.0, 6.0)])
+@pytest.mark.parametrize("F", [4096, 30])
+def test_xielu_keeps_fp32_accuracy(lo, hi, F):
+    """fp32 in and out: e^z - 1 - z to three roundings of its size, the sum with z / 2 to one (both forms of the kernel)."""
+    g = torch.Generator().manual_seed(1)
+    sp, cn = torch.tensor(0.7), torch.tensor(1.2)
+    z = torch.rand(512, F, generator=g) * (hi - lo) + lo
+    got = sq.xielu(z.cuda(), None, float(sp), float(cn)).cpu().double()
+    zd = z.double()
+    part = torch.where(zd > 0, sp.double() * zd * zd, cn.double() * (torch.expm1(zd.clamp(max=0)) - zd))
+    want = part + 0.5 * zd
+    assert bool(((got - want).abs() <= 2.0 ** -24 * (3 * part + want.abs()) + 1e-30).all())
+
+
+def test_xielu_of_extremes():
+    z = torch.tensor([[float("inf"), float("-inf"), float("nan"), -3e38, -1e30, 1e30, 0.0, -0.0]])
+    got = sq.xielu(z.cuda(), None, 0.7, 0.6).cpu()[0]
+    assert got[0] == float("inf") and got[1].isnan() and got[2].isnan() and got[5] == float("inf") and not got[6:].any()
+    torch.testing.assert_close(got[3:5].double(), 0.1 * -z[0, 3:5].double(), rtol=1e-5, atol=0)
