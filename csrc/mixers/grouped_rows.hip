@@ -21,11 +21,6 @@ using xgk::f32x4_t;
 using xgk::glu;
 using xgk::mfma16x16x32;
 
-__device__ __forceinline__ float act1(float z) {
-  const float r = z < 0.f ? 0.f : z;
-  return r * r;
-}
-
 struct GroupedArgs {
   const bf16 *A, *w;
   const int32_t *rows, *tile_expert;
@@ -122,7 +117,7 @@ __global__ __launch_bounds__(64 * WV, 1) void grouped_rows_kernel(const GroupedA
       for (int j = 0; j < 4; ++j) {
         v[j] = acc[n][m][j];
         if (MODE == 1) v[j] = glu(a.kind, v[j], acc[(GATED ? NW / 2 : 0) + n][m][j], a.limit, a.alpha);
-        if (MODE == 2) v[j] = act1(v[j] * (a.row_scale ? a.row_scale[pr] : 1.f));
+        if (MODE == 2) v[j] = relu2f(v[j] * (a.row_scale ? a.row_scale[pr] : 1.f));
       }
       if (FIRST) st4((bf16*)a.out + (int64_t)r * a.N + col, v);
       else st4((float*)a.out + (int64_t)r * a.N + col, v);

@@ -111,6 +111,11 @@ __device__ __forceinline__ float xieluf(float z, float sp, float cn) {
   return fmaf(z > 0.f ? sp * z : cn, z > 0.f ? z : exp_tail(z), 0.5f * z);
 }
 
+// max(z, 0)^2; a NaN stays one (fmaxf would make it 0)
+__device__ __forceinline__ float relu2f(float z) {
+  const float r = z < 0.f ? 0.f : z;
+  return r * r;
+}
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 

@@ -43,12 +43,6 @@ using xgk::kGluGeluTanh;
 constexpr int kActRelu2 = 2;
 constexpr int kGemmRows = 0, kGemmGated = 1, kGemmAct = 2;
 
-__device__ __forceinline__ float act1(int kind, float z) {
-  (void)kind;  // kActRelu2
-  const float r = fmaxf(z, 0.f);
-  return r * r;
-}
-
 template <typename T>
 __global__ void glu_act_kernel(const T* __restrict__ in, int64_t ld, T* __restrict__ out, int F, int64_t total, int kind,
                                float limit, float alpha) {
@@ -327,7 +321,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const T* __restrict__
     const int n = n0 + tc + 16 * j;
     if (n >= Nout) continue;
     if (GATED) stf((T*)out + (int64_t)r * Nout + n, glu(kind, acc[j], accu[j], limit, alpha));
-    else if (FIRST) stf((T*)out + (int64_t)r * Nout + n, act1(kind, acc[j] * (row_scale ? row_scale[pr] : 1.f)));
+    else if (FIRST) stf((T*)out + (int64_t)r * Nout + n, relu2f(acc[j] * (row_scale ? row_scale[pr] : 1.f)));
     else ((float*)out)[(int64_t)r * Nout + n] = acc[j];
   }
 }
@@ -443,7 +437,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(const bf16* __re
         const int pr = rows[rr];
         if (pr < 0) continue;
         if (GATED) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(glu(kind, acc[i][j][r], accu[i][GATED ? j : 0][r], limit, alpha));
-        else if (FIRST) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(act1(kind, acc[i][j][r] * (row_scale ? row_scale[pr] : 1.f)));
+        else if (FIRST) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(relu2f(acc[i][j][r] * (row_scale ? row_scale[pr] : 1.f)));
         else ((float*)out)[(int64_t)rr * Nout + n] = acc[i][j][r];
       }
     }
@@ -569,7 +563,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_lds_kernel(const bf16* 
         const int pr = rows[rr];
         if (pr < 0) continue;
         if (GATED) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(glu(kind, acc[i][j][r], accu[i][GATED ? j : 0][r], limit, alpha));
-        else if (FIRST) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(act1(kind, acc[i][j][r] * (row_scale ? row_scale[pr] : 1.f)));
+        else if (FIRST) ((bf16*)out)[(int64_t)rr * Nout + n] = f2bf(relu2f(acc[i][j][r] * (row_scale ? row_scale[pr] : 1.f)));
         else ((float*)out)[(int64_t)rr * Nout + n] = acc[i][j][r];
       }
     }

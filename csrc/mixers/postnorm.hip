@@ -225,16 +225,10 @@ __global__ void relu2_kernel(const T* __restrict__ z, const float* __restrict__ 
     ld4(z + i, v);
     if (bias) ld4(bias + (int)(i % cols), b);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float a = fmaxf(v[e] + b[e], 0.f);
-      v[e] = a * a;
-    }
+    for (int e = 0; e < 4; ++e) v[e] = relu2f(v[e] + b[e]);
     st4(out + i, v);
   } else {
-    for (int64_t j = i; j < n && j < i + 4; ++j) {
-      const float a = fmaxf(ldf(z + j) + (bias ? bias[j % cols] : 0.f), 0.f);
-      stf(out + j, a * a);
-    }
+    for (int64_t j = i; j < n && j < i + 4; ++j) stf(out + j, relu2f(ldf(z + j) + (bias ? bias[j % cols] : 0.f)));
   }
 }
 

@@ -58,10 +58,7 @@ __device__ __forceinline__ void rows_finish(const RowsArgs& a, int tok, int col,
     for (int e = 0; e < 4; ++e) v[e] = xieluf(v[e], a.p0, a.p1);
   } else if (a.act == kActRelu2) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float r = v[e] < 0.f ? 0.f : v[e];   // (a NaN stays one)
-      v[e] = r * r;
-    }
+    for (int e = 0; e < 4; ++e) v[e] = relu2f(v[e]);
   }
   st4(a.out + (int64_t)tok * a.N + col, v);
 }

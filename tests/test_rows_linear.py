@@ -134,3 +134,25 @@ def test_embed_clears_the_words_and_replays_agree():
         torch.cuda.synchronize()
         assert torch.equal(a, want) and torch.equal(b, want)
         torch.full((64, 1024), 3.0, device="cuda").sum().item()
+
+
+@gpu
+@pytest.mark.parametrize("T", [17, 64, 65, 200])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_nan_through_the_squared_relu_whatever_the_rows(T, dtype):
+    """As torch.relu keeps it: in the product's epilogue (up to 64 rows), in a launch of its own, and between expert products."""
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(T, 256, generator=g).to(dtype).cuda(), (torch.randn(128, 256, generator=g) / 16).to(dtype).cuda()
+    x[5, 7] = float("nan")
+    rows = torch.arange(T, device="cuda") != 5
+    y = sq.linear_relu2(x, w, None, types.SimpleNamespace(tickets=None))
+    assert bool(y[5].isnan().all()) and bool(y[rows].isfinite().all())
+    z = sq.relu2(torch.randn(T, 30, generator=g).to(dtype).cuda().index_fill(0, torch.tensor([5], device="cuda"), float("nan")))
+    assert bool(z[5].isnan().all()) and bool(z[rows].isfinite().all())
+    for E, K in ((1, 256), (1, 96), (4, 256)):
+        h = torch.randn(T, K, generator=g).to(dtype).cuda()
+        h[5, 7] = float("nan")
+        up, down = (torch.randn(E, *s, generator=g).to(dtype).cuda() / 16 for s in ((64, K), (K, 64)))
+        ids = (torch.arange(T, device="cuda") % E).to(torch.int32)[:, None].contiguous()
+        o = sq.routed_experts(h, up, down, ids, torch.ones(T, 1, device="cuda"), sq.ACT_RELU2)
+        assert bool(o[5].isnan().all()) and bool(o[rows].isfinite().all()), (E, K)
