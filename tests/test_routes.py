@@ -18,3 +18,41 @@ def test_single_token_states_are_those_the_kernel_takes():
             assert sq._gla_step_ok(v, sm, dk, dv) == (rows(dk, dv) > 0), (dk, dv)
     for dk, dv in ((88, 176), (168, 96), (152, 104), (136, 120), (72, 208)):   # 17 or 18 rows within 128 x 128 elements
         assert dk * dv <= 128 * 128 and not sq._gla_step_ok(v, sm, dk, dv)
+
+
+@pytest.fixture
+def as_if_native(monkeypatch):
+    """CPU tensors pass for the device's (rules only: no kernel is called)."""
+    monkeypatch.setattr(sq, "native_device", lambda t: t.device.type in ("cpu", "cuda"))
+
+
+def test_products_that_torch_refuses_or_differentiates_stay_with_it(as_if_native):
+    x, w, b = torch.randn(3, 256).bfloat16(), torch.randn(64, 256).bfloat16(), torch.randn(64).bfloat16()
+    sm = types.SimpleNamespace(tickets=torch.zeros(128, dtype=torch.int32))
+
+    def plan(x, w, b=None):
+        return sq._rows_plan_of(x, w, sm, b, False)
+    assert plan(x, w) is not None and plan(x, w, b) is not None and plan(x, w, b.float()) is not None
+    # another device: F.linear raises, a kernel would read a pointer of the other device
+    meta = dict(device="meta", dtype=torch.bfloat16)
+    assert plan(x, torch.empty(64, 256, **meta)) is None and plan(x, w, torch.empty(64, **meta)) is None
+    assert plan(x, w[None]) is None and plan(x, w[0]) is None and plan(x[None], w) is None
+    with pytest.raises(RuntimeError):
+        sq.linear(x, w, sm, b.float())                      # a bias of another type than the rows
+    # something that follows the values
+    xg, wg = x.clone().requires_grad_(), w.clone().requires_grad_()
+    assert plan(xg, w) is None and plan(x, wg) is None and plan(x, w, b.clone().requires_grad_()) is None
+    y = sq.linear(xg, w, sm)
+    y.float().sum().backward()
+    torch.testing.assert_close(xg.grad.float(), w.float().sum(0).expand(3, 256), rtol=2e-2, atol=0.1)
+    with torch.no_grad():
+        assert plan(xg, wg) is not None
+    ref = torch.nn.functional.linear(x.expand(2, 3, 256), w)
+    torch.testing.assert_close(torch.func.vmap(lambda h: sq.linear(h, w, sm))(x.expand(2, 3, 256)), ref)
+    _, tangent = torch.func.jvp(lambda h: sq.linear(h, w, sm), (x,), (torch.ones_like(x),))
+    torch.testing.assert_close(tangent, torch.nn.functional.linear(torch.ones_like(x), w))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        out = torch.autograd.forward_ad.unpack_dual(sq.linear(dual, w, sm)).tangent
+        torch.testing.assert_close(out, torch.nn.functional.linear(torch.ones_like(x), w))
+    assert plan(x, w) is not None

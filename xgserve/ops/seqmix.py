@@ -17,7 +17,9 @@ from dataclasses import dataclass
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as _fwd_ad
 import torch.nn.functional as F
+from torch._C._functorch import is_functorch_wrapped_tensor as _is_transformed
 
 from .. import tune
 from ._native import is_f32, mixers, native_device, stream_ptr
@@ -117,20 +119,28 @@ def _rows_plan(N: int, K: int, gated: bool):
     return wide, S
 
 
+def _forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform. (A product on a kernel
+    of this library has no derivative; torch's has.)"""
+    if _fwd_ad._current_level >= 0 or _is_transformed(x) or _is_transformed(w) or (bias is not None and _is_transformed(bias)):
+        return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))
+
+
 def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool,
                   slabs: bool = False):
-    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
-    pieces, K in whole staged rows, and tickets where K is in parts (clearing them would cost what the parts gain) unless the
-    `slabs` are the result."""
+    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16 on one device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
+    pieces, K in whole staged rows, nothing that wants a derivative, and tickets where K is in parts (clearing them would cost
+    what the parts gain) unless the `slabs` are the result. What is refused here goes to torch, which refuses what it cannot do."""
     if not (ROWS_LINEAR and native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and 1 <= x.shape[0] <= ROWS_LINEAR_MAX):
+            and w.device == x.device and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX and _forward_only(x, w, bias)):
         return None
     N, K = w.shape
     if K < 128 or K % 128 or x.shape[1] != K or N < 1 or N % (8 if gated else 4) or not w.is_contiguous() or \
             x.stride(1) != 1 or x.stride(0) % 8 or (x.data_ptr() | w.data_ptr()) % 16:
         return None
-    if bias is not None and not (bias.dtype in (torch.float32, torch.bfloat16) and bias.shape == (N,) and
-                                 bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+    if bias is not None and not (bias.device == x.device and bias.dtype in (torch.float32, torch.bfloat16) and bias.shape == (N,)
+                                 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return None
     plan = _rows_plan(N, K, gated)
     return plan if slabs or plan[1] == 1 or (sm is not None and sm.tickets is not None) else None
@@ -149,7 +159,7 @@ def _rows_linear(plan, x, w, sm, bias, act, p0, p1) -> torch.Tensor:
 def linear(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [T, K] . w [N, K]^T + bias."""
-    plan = _rows_plan_of(x, w, sm, bias, False)
+    plan = _rows_plan_of(x, w, sm, bias, False) if bias is None or bias.dtype == x.dtype else None
     if plan is not None:
         return _rows_linear(plan, x, w, sm, bias, ACT_NONE, 0.0, 0.0)
     return F.linear(x, w, bias)
