@@ -56,3 +56,24 @@ def test_products_that_torch_refuses_or_differentiates_stay_with_it(as_if_native
         out = torch.autograd.forward_ad.unpack_dual(sq.linear(dual, w, sm)).tangent
         torch.testing.assert_close(out, torch.nn.functional.linear(torch.ones_like(x), w))
     assert plan(x, w) is not None
+
+
+def test_tensors_that_lie_off_16_bytes_keep_the_general_kernels(as_if_native):
+    """The wide kernels refuse them, which would raise; the general ones take them."""
+    sm = types.SimpleNamespace(max_q=1, num_seqs=2, block_tables=torch.zeros(2, 4, dtype=torch.int32))
+
+    def off(*shape, dtype=torch.float32):
+        n = torch.Size(shape).numel()
+        return torch.zeros(n + 1, dtype=dtype)[1:].view(shape)
+    v, state = torch.zeros(2, 64), torch.zeros(2, 1, 64, 64)
+    assert sq._gla_step_ok(v, sm, 64, 64, state) and not sq._gla_step_ok(v, sm, 64, 64, off(2, 1, 64, 64))
+    proj, w2 = torch.zeros(2, 5 * 64 + 8).bfloat16(), torch.zeros(64, 8).bfloat16()
+    assert sq._delta_step_ok(proj, w2, state, 64, sm, torch.bfloat16)
+    assert not sq._delta_step_ok(proj, w2, off(2, 1, 64, 64), 64, sm, torch.bfloat16)
+    q, uv, cache = torch.zeros(2, 4, 96).bfloat16(), torch.zeros(256, 256).bfloat16(), torch.zeros(8, 288).bfloat16()
+    assert sq._latent_shares(q, uv, 256, 32, 64, 64, 16, sm, cache) == 1
+    assert sq._latent_shares(q, uv, 256, 32, 64, 64, 16, sm, off(8, 288, dtype=torch.bfloat16)) == 0
+    x, y, w = torch.zeros(2, 64), torch.zeros(2, 64).bfloat16(), torch.zeros(64)
+    assert sq._rows_aligned(y, None, x, w, None) and sq._rows_aligned(sq.Parts(torch.zeros(2, 2, 64)), y, x)
+    assert not sq._rows_aligned(y, None, x, off(64)) and not sq._rows_aligned(y, off(2, 64, dtype=torch.bfloat16), x)
+    assert not sq._rows_aligned(torch.zeros(2, 66).bfloat16()[:, :64], None, x)

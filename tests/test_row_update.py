@@ -128,3 +128,25 @@ def test_products_stay_in_parts_where_the_step_says_so():
     sm.max_q = 2
     assert not sq.step_rows(sm, x.float(), torch.bfloat16, 4) and sq.step_rows(sm, x.float(), torch.bfloat16)
     assert not sq.step_rows(sm, x.float(), torch.float32)
+
+
+def test_weights_off_16_bytes_take_the_separate_kernels():
+    """Parameters and states that are slices of a larger buffer: the same results, by launches that take them."""
+    g = torch.Generator().manual_seed(2)
+    T, W, taps, slots, ctx = 3, 64, 4, [2, 0, 1], [7, 0, 2]
+    sm = meta(T, slots, ctx)
+    x, w, a1, a2 = torch.randn(T, W, generator=g), *(torch.randn(W, generator=g) for _ in range(3))
+    cw, state = torch.randn(W, taps, generator=g), torch.randn(3, taps - 1, W, generator=g)
+    y, z = (sq.Parts(torch.randn(2, T, W, generator=g).cuda()) for _ in range(2))
+
+    def off(t):
+        return torch.cat([torch.zeros(1), t.flatten()]).cuda()[1:].view(t.shape)
+    outs = []
+    for place in (lambda t: t.cuda(), off):
+        xg, st = x.cuda(), place(state)
+        h = sq.norm_conv(xg, y, place(w), 1e-5, 0.7, None, (place(cw), st), sm, torch.bfloat16)
+        x2, st2 = x.cuda(), place(state)
+        rest = sq.residual_norm_conv(x2, y, place(a1), z, None, place(a2), place(w), 1e-5, torch.bfloat16, (place(cw), st2), True, sm)
+        outs.append([xg, st, h, x2, st2, *rest])
+    for a, b in zip(*outs):   # (the product's sum is rounded to bf16 there)
+        torch.testing.assert_close(a.float(), b.float(), rtol=2e-2, atol=4e-2)

@@ -329,6 +329,18 @@ def step_rows(sm: SeqMeta, x: torch.Tensor, dtype: torch.dtype, taps: int = 0) -
             and W <= 8192 and (taps == 0 or (2 <= taps <= 4 and sm.max_q == 1)))
 
 
+def _rows_aligned(y1, y2, *tensors: Optional[torch.Tensor]) -> bool:
+    """Whether the kernels of few rows can take these rows (activation tensors, `Parts` or None) and fp32 tensors."""
+    for y in (y1, y2):
+        if isinstance(y, torch.Tensor) and (y.stride(1) != 1 or y.stride(0) % 4 or y.data_ptr() % 8):
+            return False
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _added(y, dtype: torch.dtype):
+    return y.rows(dtype) if isinstance(y, Parts) else y
+
+
 def _row_source(y):
     """(pointer, row stride, slab stride, slabs) of a bf16 row tensor (0 slabs), `Parts` or None."""
     if y is None:
@@ -362,10 +374,10 @@ def norm_conv(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float, bia
               sm: SeqMeta, dtype: torch.dtype) -> Optional[torch.Tensor]:
     """x <- rmsnorm(alpha x + y + bias) * (1 + w) in place, then with conv = (weights, state) the residual convolution of the
     new x (causal_conv_residual). y: an activation tensor, or the `Parts` of a product (sm.parts)."""
-    if sm.parts:
+    if sm.parts and _rows_aligned(y, None, x, w, bias, *(conv or ())):
         return _row_update(x, y, None, None, None, None, bias, alpha, w, 1.0, eps, True, False, False,
                            *(conv or (None, None)), sm)[2]
-    scaled_add_rmsnorm(x, y, w, eps, alpha, bias, 1.0)
+    scaled_add_rmsnorm(x, _added(y, dtype), w, eps, alpha, bias, 1.0)
     return causal_conv_residual(x, conv[0], conv[1], sm, dtype) if conv is not None else None
 
 
@@ -374,9 +386,9 @@ def residual_norm_conv(x: torch.Tensor, y1, a1: Optional[torch.Tensor], y2, y3: 
                        conv: Optional[tuple], need_f32: bool, sm: SeqMeta):
     """residual_norm (x <- x + a1 y1 + a2 (y2 + y3), n = its norm), then with conv = (weights, state) the residual convolution
     of n: (n fp32 where `need_f32` or the convolution asks for it, n as `dtype`, convolution or None)."""
-    if sm.parts:
+    if sm.parts and _rows_aligned(y1, y2, x, y3, a1, a2, norm_w, *(conv or ())):
         return _row_update(x, y1, y2, y3, a1, a2, None, 1.0, norm_w, 0.0, eps, False, need_f32, True, *(conv or (None, None)), sm)
-    n32, n = residual_norm(x, y1, a1, y2, y3, a2, norm_w, eps, dtype, need_f32 or conv is not None)
+    n32, n = residual_norm(x, _added(y1, dtype), a1, _added(y2, dtype), y3, a2, norm_w, eps, dtype, need_f32 or conv is not None)
     h = causal_conv(n32, conv[0], None, conv[1], sm, dtype, residual=True) if conv is not None else None
     return n32, n, h
 
@@ -537,12 +549,12 @@ LATENT_DECODE_WGS, LATENT_DECODE_SHARES = 256, 16
 LATENT_PAGES = 2048     # page table entries of a share
 
 
-def _latent_shares(q, uv, R: int, rd: int, dv: int, window: int, block_size: int, sm: SeqMeta) -> int:
+def _latent_shares(q, uv, R: int, rd: int, dv: int, window: int, block_size: int, sm: SeqMeta, cache=None) -> int:
     """Shares of the window for latent_decode, 0 where it does not apply."""
     T, H = q.shape[:2]
     if not (native_device(q) and LATENT_MFMA and LATENT_DECODE and q.dtype == torch.bfloat16 and sm.max_q == 1
             and 1 <= T == sm.num_seqs <= 65535 and R in (64, 128, 256, 512) and rd in (32, 64) and dv % 16 == 0
-            and uv.data_ptr() % 16 == 0):
+            and uv.data_ptr() % 16 == 0 and (cache is None or cache.data_ptr() % 16 == 0)):
         return 0
     tiles = -(-min(window, sm.block_tables.shape[1] * block_size) // 64)
     groups = T * -(-H // 32)
@@ -580,7 +592,7 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
                                       sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
             return out
     qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
-    shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm)
+    shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm, cache)
     if shares:
         assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
         assert cache.dtype == gate.dtype == uv.dtype == q.dtype and uv.is_contiguous()
@@ -632,7 +644,7 @@ def delta_rule_scan(proj: torch.Tensor, off_r: int, off_k: int, off_v: int, off_
         assert proj.stride(1) == 1 and wl.stride(1) == 1 and wl.dtype == proj.dtype
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, D)
         es = proj.element_size()
-        if DELTA_CHUNK and D in DELTA_CHUNK_D and sm.max_q >= DELTA_CHUNK_MIN and proj.data_ptr() % 16 == 0 \
+        if DELTA_CHUNK and D in DELTA_CHUNK_D and DELTA_CHUNK_MIN <= sm.max_q <= 65535 * 16 and sm.num_seqs <= 65535 and proj.data_ptr() % 16 == 0 \
                 and proj.stride(0) * es % 16 == 0 and off_v * es % 16 == 0:
             scratch = torch.empty(mixers().delta_chunk_scratch_floats(T, sm.num_seqs, H, D), dtype=torch.float32,
                                   device=proj.device)
@@ -683,14 +695,20 @@ def delta_rule_out(o: torch.Tensor, norm_w: torch.Tensor, gate: torch.Tensor, ep
     return out
 
 
+def _delta_step_ok(proj: torch.Tensor, w2: torch.Tensor, state: torch.Tensor, D: int, sm: SeqMeta, dtype: torch.dtype) -> bool:
+    lr = w2.shape[1]
+    return (native_device(proj) and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16
+            and D in (32, 64, 128) and 8 <= lr <= 256 and lr % 8 == 0 and sm.num_seqs <= 65535 and proj.stride(1) == 1
+            and proj.stride(0) % 4 == 0 and proj.data_ptr() % 8 == 0 and w2.is_contiguous() and w2.data_ptr() % 16 == 0
+            and state.data_ptr() % 16 == 0)
+
+
 def delta_rule_mix(proj: torch.Tensor, w2: torch.Tensor, a_bias: torch.Tensor, w0: torch.Tensor, norm_w: torch.Tensor,
                    state: torch.Tensor, eps: float, H: int, D: int, sm: SeqMeta, dtype: torch.dtype) -> torch.Tensor:
     """The delta-rule mixer between its projections: proj's columns [r | k | v | gate | a-logits | low rank], decay logits
     W2 tanh(low rank), delta_rule_scan, delta_rule_out. Steps of single tokens in one launch."""
     T, HD, lr = proj.shape[0], H * D, w2.shape[1]
-    if native_device(proj) and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16 \
-            and D in (32, 64, 128) and 8 <= lr <= 256 and lr % 8 == 0 and sm.num_seqs <= 65535 and proj.stride(1) == 1 \
-            and proj.stride(0) % 4 == 0 and proj.data_ptr() % 8 == 0 and w2.is_contiguous() and w2.data_ptr() % 16 == 0:
+    if _delta_step_ok(proj, w2, state, D, sm, dtype):
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, D)
         y = torch.empty(T, HD, dtype=dtype, device=proj.device)
         mixers().delta_step(proj.data_ptr(), proj.stride(0), 0, HD, 2 * HD, 3 * HD, 4 * HD, 5 * HD, lr, w2.data_ptr(),
@@ -1032,7 +1050,7 @@ def ssm_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_l
                                     _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(),
                                     y.data_ptr(), sm.num_seqs, sm.max_q, T, H, G, N, P, seg, _p(scratch), stream_ptr())
             return y
-        if _gla_step_ok(xbc, sm, N, P):
+        if _gla_step_ok(xbc, sm, N, P, state):
             mixers().ssm_step(xbc.data_ptr(), is_f32(xbc), xbc.stride(0), dt_raw.data_ptr(), dt_raw.stride(0),
                               dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(), _i32(sm.qsl).data_ptr(),
                               _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), y.data_ptr(), sm.num_seqs, H, G, N, P,
@@ -1543,10 +1561,11 @@ def lower_bound_gates(proj: torch.Tensor, off_q: int, off_f: int, n: int, f_bias
 STATE_STEP = True
 
 
-def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int) -> bool:
+def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int, state: Optional[torch.Tensor] = None) -> bool:
     # (sizes: gla_step_rows of state_step.hip, at most 16 rows per thread)
     return (STATE_STEP and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
-            and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0)
+            and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0
+            and (state is None or state.data_ptr() % 16 == 0))
 
 
 def gated_linear_scan(q: torch.Tensor, f: Optional[torch.Tensor], k: Optional[torch.Tensor], v: torch.Tensor,
@@ -1567,7 +1586,7 @@ def gated_linear_scan(q: torch.Tensor, f: Optional[torch.Tensor], k: Optional[to
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, dk, dv)
         if _chunk_scan_ok(sm, dk) and decay is None and bonus is None:
             return _chunk_scan(q, f, k, None, 0, 0, None, None, v, state, o, sm, H, dk, dv)
-        if _gla_step_ok(v, sm, dk, dv):
+        if _gla_step_ok(v, sm, dk, dv, state):
             mixers().gla_step(q.data_ptr(), _p(f), _p(k), 0, 0, 0, 0, 0, 0, v.data_ptr(), is_f32(v), v.stride(0), state.data_ptr(),
                               _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), o.data_ptr(),
                               sm.num_seqs, H, dk, dv, _p(decay), _p(bonus), stream_ptr())
@@ -1613,7 +1632,7 @@ def lower_bound_recurrence(proj: torch.Tensor, off_q: int, off_f: int, off_v: in
     o = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device)
     if _chunk_scan_ok(sm, dk):
         return _chunk_scan(None, None, None, proj, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv)
-    if _gla_step_ok(v, sm, dk, dv):
+    if _gla_step_ok(v, sm, dk, dv, state):
         mixers().gla_step(0, 0, 0, proj.data_ptr(), proj.stride(0), off_q, off_f, _p(f_bias), lower.data_ptr(), v.data_ptr(),
                           is_f32(proj), proj.stride(0), state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
                           _i32(sm.slots).data_ptr(), o.data_ptr(), sm.num_seqs, H, dk, dv, 0, 0, stream_ptr())
