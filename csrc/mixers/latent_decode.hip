@@ -41,12 +41,12 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
   int32_t* pages = reinterpret_cast<int32_t*>(lds + 2 * SLOT);
   const int s = blockIdx.y, share = blockIdx.x, lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ht = wave & 1, kg = wave >> 1;
-  const int head = blockIdx.z * 32 + 16 * ht + li;
-  if (a.slots[s] < 0 || a.qsl[s + 1] - a.qsl[s] <= 0) return;
+  const int head = blockIdx.z * 32 + 16 * ht + li, t = a.qsl[s];   // the sequence's row (sequences without a token have none)
+  if (a.slots[s] < 0 || a.qsl[s + 1] - t <= 0) return;
   const int pos = a.seq_lens[s] - 1, first = max(0, pos - a.window + 1);
   const int tiles_all = (pos - first + 64) / 64, per = (tiles_all + a.shares - 1) / a.shares;
   const int k0 = first + 64 * per * share, k1 = min(pos, k0 + 64 * per - 1);   // this share's keys [k0, k1]
-  const int64_t row = ((int64_t)share * a.H + head) * a.T + s;
+  const int64_t row = ((int64_t)share * a.H + head) * a.T + t;
   if (k0 > pos) {   // an empty share
     if (kg == 0 && g == 0 && head < a.H) a.part_ml[2 * row] = -INFINITY, a.part_ml[2 * row + 1] = 0.f;
     return;
@@ -69,11 +69,11 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
   const int hq = min(head, a.H - 1), half = a.rot_dims >> 1;
   uint4 qr[NKK];
 #pragma unroll
-  for (int kk = 0; kk < NR; ++kk) qr[kk] = xgk::ld16(a.qabs + ((int64_t)hq * a.T + s) * R + 32 * kk + 8 * g);
+  for (int kk = 0; kk < NR; ++kk) qr[kk] = xgk::ld16(a.qabs + ((int64_t)hq * a.T + t) * R + 32 * kk + 8 * g);
 #pragma unroll
   for (int kk = 0; kk < ND; ++kk) {
     const int i0 = 32 * kk + 8 * g;
-    const bf16* src = a.q + ((int64_t)s * a.H + hq) * a.dq + a.dn + i0;
+    const bf16* src = a.q + ((int64_t)t * a.H + hq) * a.dq + a.dn + i0;
     float f[8];
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
@@ -183,8 +183,9 @@ template <int NR>
 __global__ __launch_bounds__(256) void latent_out_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                          const bf16* __restrict__ gate, int64_t gate_stride,
                                                          const bf16* __restrict__ uv, const int32_t* __restrict__ slots,
-                                                         const int32_t* __restrict__ qsl, bf16* __restrict__ out, int T, int H,
-                                                         int dv, int shares) {
+                                                         const int32_t* __restrict__ qsl,
+                                                         const int32_t* __restrict__ token_seq, bf16* __restrict__ out, int T,
+                                                         int H, int dv, int shares) {
   constexpr int R = 32 * NR, LD = R + 8, TOK = 8;
   __shared__ __attribute__((aligned(16))) uint16_t lat[TOK * LD];
   __shared__ float wt[TOK][64];   // a share's weight: e^(m_s - M) gate / L (shares <= 64)
@@ -199,7 +200,8 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const float* __restrict
   for (int i = wave; i < TOK; i += 4) {
     const int t = t0 + i;
     float x = 0.f;
-    if (t < T && slots[t] >= 0 && qsl[t + 1] > qsl[t]) {
+    const int s = t < T ? token_seq[t] : -1;
+    if (s >= 0 && s < T && slots[s] >= 0 && qsl[s] == t && qsl[s + 1] > t) {   // (T sequences)
       const int64_t r = 2 * (((int64_t)min(lane, shares - 1) * H + h) * T + t);
       const float m = lane < shares ? part_ml[r] : -INFINITY, l = part_ml[r + 1];
       const float M = wave_max(m), e = m == -INFINITY ? 0.f : __expf(m - M);
@@ -244,11 +246,11 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const float* __restrict
   }
 }
 
-// One token per sequence (row t is sequence t). Returns 0, or -1 for sizes that it does not take: R 64, 128, 256 or 512, rd 32 or
+// At most one token per sequence, as many rows as sequences (rows behind the last token are zero). Returns 0, or -1 for sizes that it does not take: R 64, 128, 256 or 512, rd 32 or
 // 64, dv a multiple of 16, 1 to 64 shares, a share's keys within kLatentPages pages.
 int latent_decode(const void* qabs, const void* q, int dq, int dn, const void* gate, int64_t gate_stride, const void* cache,
                   const int32_t* bt, int bt_width, int bs, const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots,
-                  const float* rot, int rot_dims, const void* uv, void* out, int T, int H, int R, int dv, int window, float scale,
+                  const int32_t* token_seq, const float* rot, int rot_dims, const void* uv, void* out, int T, int H, int R, int dv, int window, float scale,
                   int shares, float* part_o, float* part_ml, hipStream_t st) {
   if (T <= 0) return 0;
   const int rd = dq - dn, nr = R / 32;
@@ -265,7 +267,8 @@ int latent_decode(const void* qabs, const void* q, int dq, int dn, const void* g
     if (rd == 32) latent_decode_kernel<NR, 1><<<grid, 256, 0, st>>>(a);                                                     \
     else latent_decode_kernel<NR, 2><<<grid, 256, 0, st>>>(a);                                                              \
     latent_out_kernel<NR><<<dim3(H, (T + 7) / 8), 256, 0, st>>>(part_o, part_ml, (const bf16*)gate, gate_stride,            \
-                                                                (const bf16*)uv, slots, qsl, (bf16*)out, T, H, dv, shares); \
+                                                                (const bf16*)uv, slots, qsl, token_seq, (bf16*)out, T, H,   \
+                                                                dv, shares);                                                \
     return 0;                                                                                                               \
   }
   XGM_LD(2)

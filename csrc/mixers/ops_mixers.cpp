@@ -52,7 +52,7 @@ int gated_linear_scan(const float*, const float*, const float*, const void*, int
                       int, int, int, float*, int, int, const float*, const float*, hipStream_t);
 int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
 int latent_decode(const void*, const void*, int, int, const void*, int64_t, const void*, const int32_t*, int, int, const int32_t*,
-                  const int32_t*, const int32_t*, const float*, int, const void*, void*, int, int, int, int, int, float, int,
+                  const int32_t*, const int32_t*, const int32_t*, const float*, int, const void*, void*, int, int, int, int, int, float, int,
                   float*, float*, hipStream_t);
 int gla_step_rows(int, int);
 int gla_step(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*, const void*,
@@ -321,12 +321,13 @@ PYBIND11_MODULE(_mixers, m) {
         [](int T, int ns, int H, int dk, int dv) { return xgm::gated_linear_scan_scratch_floats(T, ns, H, dk, dv); });
   m.def("latent_decode", [](uintptr_t qabs, uintptr_t q, int dq, int dn, uintptr_t gate, int64_t gate_stride, uintptr_t cache,
                             uintptr_t bt, int bt_width, int bs, uintptr_t qsl, uintptr_t seq_lens, uintptr_t slots,
-                            uintptr_t rot, int rot_dims, uintptr_t uv, uintptr_t out, int T, int H, int R, int dv, int window,
+                            uintptr_t token_seq, uintptr_t rot, int rot_dims, uintptr_t uv, uintptr_t out, int T, int H, int R, int dv, int window,
                             float scale, int shares, uintptr_t part_o, uintptr_t part_ml, uintptr_t st) {
     check(xgm::latent_decode(P<const void>(qabs), P<const void>(q), dq, dn, P<const void>(gate), gate_stride,
                              P<const void>(cache), P<const int32_t>(bt), bt_width, bs, P<const int32_t>(qsl),
-                             P<const int32_t>(seq_lens), P<const int32_t>(slots), P<const float>(rot), rot_dims,
-                             P<const void>(uv), P<void>(out), T, H, R, dv, window, scale, shares, P<float>(part_o),
+                             P<const int32_t>(seq_lens), P<const int32_t>(slots), P<const int32_t>(token_seq),
+                             P<const float>(rot), rot_dims, P<const void>(uv), P<void>(out), T, H, R, dv, window, scale, shares,
+                             P<float>(part_o),
                              P<float>(part_ml), S(st)),
           "latent_decode");
   });

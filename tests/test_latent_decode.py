@@ -73,3 +73,32 @@ def test_other_steps_keep_the_general_kernels():
     assert sq._latent_shares(q, uv, 256, 32, 64, 1 << 20, 1, sm) == 0       # a share's page table would not fit
     sm.max_q = 2
     assert sq._latent_shares(q, uv, 256, 32, 64, 64, 16, sm) == 0
+
+
+def test_sequences_without_a_token():
+    """A sequence that waits (no token in the step) between others, and a row behind the last token: rows follow the sequences."""
+    g = torch.Generator().manual_seed(7)
+    H, dn, rd, dv, R, bs, window = 4, 64, 32, 64, 256, 16, 64
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    lens, qsl, token_seq = [40, 9, 100, 23], [0, 1, 1, 2, 3], [0, 2, 3, -1]
+    bt, at = torch.zeros(4, 7, dtype=torch.int32), 0
+    for i, n in enumerate(lens):
+        m = -(-n // bs)
+        bt[i, :m] = torch.arange(at, at + m)
+        at += m
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()  # noqa: E731
+    cache, q, gate = rnd(at * bs, R + rd), rnd(4, H, dn + rd), rnd(4, H)
+    uk, uv = rnd(H * dn, R) / 16, rnd(H * dv, R) / 16
+    rot = sq.build_rot_table(rd, 1e4, 101, "cpu").cuda()
+
+    def attend(rows, seqs):
+        """The same sequences, each with its token."""
+        k = len(seqs)
+        sm = sq.SeqMeta(k, 1, i32(list(range(k + 1))), i32([lens[s] for s in seqs]), i32(list(range(k))), bt[seqs].cuda(),
+                        i32(list(range(k))), i32([lens[s] - 1 for s in seqs]), i32([0] * k))
+        return sq.latent_attention_heads(q[rows].contiguous(), dn, gate[rows].contiguous(), cache, uk, uv, rot, rd, window, 0.1, bs, sm)
+    want = attend([0, 1, 2], [0, 2, 3])
+    sm = sq.SeqMeta(4, 1, i32(qsl), i32(lens), i32([0, 1, 2, 3]), bt.cuda(), i32(token_seq), i32([39, 99, 22, 0]), i32([0] * 4))
+    assert sq._latent_shares(q, uv, R, rd, dv, window, bs, sm, cache) > 0
+    got = sq.latent_attention_heads(q, dn, gate, cache, uk, uv, rot, rd, window, 0.1, bs, sm)
+    assert torch.equal(got[:3], want) and not bool(got[3].any())

@@ -601,8 +601,8 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
         part = torch.empty(shares * H * T * (R + 2), dtype=torch.float32, device=q.device)
         mixers().latent_decode(qabs.data_ptr(), q.data_ptr(), dq, dn, gate.data_ptr(), gate.stride(0), cache.data_ptr(),
                                bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
-                               _i32(sm.slots).data_ptr(), rot.data_ptr(), rot_dims, uv.data_ptr(), out.data_ptr(), T, H, R, dv,
-                               int(window), float(scale), shares, part.data_ptr(),
+                               _i32(sm.slots).data_ptr(), _i32(sm.token_seq).data_ptr(), rot.data_ptr(), rot_dims,
+                               uv.data_ptr(), out.data_ptr(), T, H, R, dv, int(window), float(scale), shares, part.data_ptr(),
                                part.data_ptr() + 4 * shares * H * T * R, stream_ptr())
         return out
     o_lat = latent_attention(qabs, q, dn, gate, cache, rot, rot_dims, window, scale, block_size, sm)
