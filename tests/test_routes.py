@@ -77,3 +77,20 @@ def test_tensors_that_lie_off_16_bytes_keep_the_general_kernels(as_if_native):
     assert sq._rows_aligned(y, None, x, w, None) and sq._rows_aligned(sq.Parts(torch.zeros(2, 2, 64)), y, x)
     assert not sq._rows_aligned(y, None, x, off(64)) and not sq._rows_aligned(y, off(2, 64, dtype=torch.bfloat16), x)
     assert not sq._rows_aligned(torch.zeros(2, 66).bfloat16()[:, :64], None, x)
+
+
+@pytest.mark.parametrize("H,dn,rd,dv,R", [(32, 64, 32, 64, 256), (64, 128, 64, 128, 512), (128, 128, 64, 128, 512), (256, 128, 64, 128, 512)])
+def test_expanded_latents_stay_within_their_bytes(as_if_native, H, dn, rd, dv, R):
+    """Portions behind long contexts: the expansion is chosen only while keys, values and gathered rows stay within 1 GiB, which
+    the cache's sizing leaves free. (Rows alone let 64 heads of 128 + 128 take 2.1 GB and 128 heads 4.3 GB.)"""
+    chosen = []
+    for T, ctx in ((64, 0), (2048, 30000), (2100, 65000), (4096, 65536), (8192, 57344), (8192, 200000)):
+        q = torch.empty(1, H, dn + rd, dtype=torch.bfloat16).expand(T, -1, -1)
+        cache = torch.empty(8, R + rd, dtype=torch.bfloat16)
+        sm = types.SimpleNamespace(max_q=T, num_seqs=1, block_tables=torch.zeros(1, -(-(T + ctx) // 16), dtype=torch.int32))
+        nk = sq._latent_expands(q, dn, R, dv, rd, 1 << 20, 16, sm, cache)
+        keys = sq._latent_key_rows(sm, T, 1 << 20, 16)
+        size = keys * (H * (dn + dv) + R + rd) * 2
+        assert nk == (keys if keys <= 32 * T and size <= 1 << 30 else 0)
+        chosen.append(nk > 0)
+    assert chosen[0] and not chosen[-1]

@@ -530,7 +530,7 @@ def latent_attention(qabs: torch.Tensor, q: torch.Tensor, dn: int, gate: torch.T
 # rows are bounded because their number is: single tokens of many sequences in the step each count a whole window.
 LATENT_EXPAND = True
 LATENT_EXPAND_MIN = 64
-LATENT_EXPAND_ROWS, LATENT_EXPAND_MAX = 32, 65536   # key rows per token, and in all (1 GB of keys and values at 64 heads' sizes)
+LATENT_EXPAND_ROWS, LATENT_EXPAND_BYTES = 32, 1 << 30   # key rows per token, and what all of them take expanded (and gathered)
 LATENT_EXPAND_SIZES = ((96, 64), (192, 128))        # (dn + rd, dv)
 
 
@@ -539,6 +539,18 @@ def _latent_key_rows(sm: SeqMeta, T: int, window: int, block_size: int) -> int:
     sequence its window before them or what its page table can hold."""
     held = sm.num_seqs * sm.block_tables.shape[1] * block_size
     return T + max(0, min(sm.num_seqs * (window - 1), held - T))
+
+
+def _latent_expands(q, dn: int, R: int, dv: int, rot_dims: int, window: int, block_size: int, sm: SeqMeta, cache) -> int:
+    """Key rows that a step's portions are expanded over, 0 where the attention stays in latent space."""
+    T, H, dq = q.shape
+    if not (native_device(q) and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN
+            and (dq, dv) in LATENT_EXPAND_SIZES and dn % 8 == 0 and R % 8 == 0 and rot_dims % 2 == 0
+            and cache.data_ptr() % 16 == 0):
+        return 0
+    nk = _latent_key_rows(sm, T, window, block_size)
+    fits = nk * (H * (dn + dv) + R + dq - dn) * q.element_size() <= LATENT_EXPAND_BYTES
+    return nk if nk <= LATENT_EXPAND_ROWS * T and fits else 0
 
 
 # Steps of single tokens (latent_decode.hip): shares of a window while the grid stays within 256 workgroups, at most 16. From the
@@ -571,26 +583,24 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
     the softmax."""
     T, H, dq = q.shape
     R, dv = uk.shape[1], uv.shape[0] // H
-    if native_device(q) and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN \
-            and (dq, dv) in LATENT_EXPAND_SIZES and dn % 8 == 0 and R % 8 == 0 and rot_dims % 2 == 0:
-        nk = _latent_key_rows(sm, T, window, block_size)
-        if nk <= min(LATENT_EXPAND_ROWS * T, LATENT_EXPAND_MAX):
-            assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
-            assert cache.dtype == gate.dtype == uk.dtype == uv.dtype == q.dtype
-            M, bt = mixers(), _i32(sm.block_tables)
-            lat = torch.empty(nk, R + dq - dn, dtype=q.dtype, device=q.device)
-            koff = torch.empty(sm.num_seqs, dtype=torch.int32, device=q.device)
-            M.latent_gather(cache.data_ptr(), bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(),
-                            _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), sm.num_seqs, int(window), lat.shape[1],
-                            lat.data_ptr(), koff.data_ptr(), nk, stream_ptr())
-            kn = torch.nn.functional.linear(lat[:, :R], uk)
-            v = torch.nn.functional.linear(lat[:, :R], uv)
-            out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
-            M.latent_prompt_attention(q.data_ptr(), dn, dq - dn, dv, kn.data_ptr(), v.data_ptr(), lat.data_ptr(), R,
-                                      koff.data_ptr(), gate.data_ptr(), gate.stride(0), rot.data_ptr(), rot_dims,
-                                      sm.qsl.data_ptr(), sm.seq_lens.data_ptr(), sm.slots.data_ptr(), out.data_ptr(), T,
-                                      sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
-            return out
+    nk = _latent_expands(q, dn, R, dv, rot_dims, window, block_size, sm, cache)
+    if nk:
+        assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
+        assert cache.dtype == gate.dtype == uk.dtype == uv.dtype == q.dtype
+        M, bt = mixers(), _i32(sm.block_tables)
+        lat = torch.empty(nk, R + dq - dn, dtype=q.dtype, device=q.device)
+        koff = torch.empty(sm.num_seqs, dtype=torch.int32, device=q.device)
+        M.latent_gather(cache.data_ptr(), bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(),
+                        _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), sm.num_seqs, int(window), lat.shape[1],
+                        lat.data_ptr(), koff.data_ptr(), nk, stream_ptr())
+        kn = torch.nn.functional.linear(lat[:, :R], uk)
+        v = torch.nn.functional.linear(lat[:, :R], uv)
+        out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+        M.latent_prompt_attention(q.data_ptr(), dn, dq - dn, dv, kn.data_ptr(), v.data_ptr(), lat.data_ptr(), R,
+                                  koff.data_ptr(), gate.data_ptr(), gate.stride(0), rot.data_ptr(), rot_dims,
+                                  sm.qsl.data_ptr(), sm.seq_lens.data_ptr(), sm.slots.data_ptr(), out.data_ptr(), T,
+                                  sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
+        return out
     qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
     shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm, cache)
     if shares:
