@@ -1,5 +1,8 @@
 """Which kernel a call takes: the rules in Python against the kernels' own contracts, over all that they accept. No GPU is needed
 (a rule looks at sizes, strides, types and alignment; CPU tensors stand for the device's)."""
+import os
+import subprocess
+import sys
 import types
 
 import pytest
@@ -7,6 +10,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 from xgserve.ops._native import mixers
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def test_single_token_states_are_those_the_kernel_takes():
@@ -94,3 +99,37 @@ def test_expanded_latents_stay_within_their_bytes(as_if_native, H, dn, rd, dv, R
         assert nk == (keys if keys <= 32 * T and size <= 1 << 30 else 0)
         chosen.append(nk > 0)
     assert chosen[0] and not chosen[-1]
+
+
+def test_tuning_keys_choose_the_kernels_that_they_name(as_if_native, monkeypatch):
+    """latent_mfma, delta_two_pass, scan_cols and scan_two_pass ask for the kernels they asked for before the chunked, expanded
+    and one-token forms came in front of them."""
+    step, prompt = types.SimpleNamespace(max_q=1, num_seqs=2, block_tables=torch.zeros(2, 4, dtype=torch.int32)), \
+        types.SimpleNamespace(max_q=4001, num_seqs=1, block_tables=torch.zeros(1, 256, dtype=torch.int32))
+    q, uv, cache = torch.zeros(2, 4, 96).bfloat16(), torch.zeros(256, 256).bfloat16(), torch.zeros(8, 288).bfloat16()
+    qp = torch.zeros(1, 4, 96).bfloat16().expand(4001, -1, -1)
+    proj, w2, state = torch.zeros(2, 5 * 64 + 8).bfloat16(), torch.zeros(64, 8).bfloat16(), torch.zeros(2, 1, 64, 64)
+    v = torch.zeros(2, 64)
+
+    def routes():
+        return {"latent step": sq._latent_shares(q, uv, 256, 32, 64, 64, 16, step, cache) > 0,
+                "latent prompt": sq._latent_expands(qp, 64, 256, 64, 32, 1024, 16, prompt, cache) > 0,
+                "delta step": sq._delta_step_ok(proj, w2, state, 64, step, torch.bfloat16),
+                "delta prompt": sq._delta_chunk_ok(proj, 0, 64, prompt),
+                "scan step": sq._gla_step_ok(v, step, 64, 64, state), "scan prompt": sq._chunk_scan_ok(prompt, 64),
+                "segments": sq._chunk_scan_segments(prompt, 4001, 16, 64, 128, 128, "cpu")[1] is not None}
+    assert all(routes().values())
+    for key, value, off in (("LATENT_MFMA", False, {"latent step", "latent prompt"}), ("DELTA_TWO_PASS", False, {"delta step", "delta prompt"}),
+                            ("SCAN_COLS", 32, {"scan step", "scan prompt"}), ("SCAN_TWO_PASS", False, {"segments"})):
+        with monkeypatch.context() as m:
+            m.setattr(sq, key, value)
+            assert {k for k, on in routes().items() if not on} == off, key
+
+
+def test_the_32_row_tiles_follow_their_key():
+    """moe_tile32_min reaches every kind of expert."""
+    code = "from xgserve.ops import seqmix as sq; print(dict(sq.MOE_TILES)[32], dict(sq.MOE_TILES_GENERAL)[32])"
+    for spec, want in (("", "8 12"), ("moe_tile32_min=20", "20 20")):
+        out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, XGS_TUNE=spec), cwd=ROOT, capture_output=True,
+                             text=True, check=True)
+        assert out.stdout.split() == want.split()

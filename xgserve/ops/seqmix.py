@@ -544,7 +544,7 @@ def _latent_key_rows(sm: SeqMeta, T: int, window: int, block_size: int) -> int:
 def _latent_expands(q, dn: int, R: int, dv: int, rot_dims: int, window: int, block_size: int, sm: SeqMeta, cache) -> int:
     """Key rows that a step's portions are expanded over, 0 where the attention stays in latent space."""
     T, H, dq = q.shape
-    if not (native_device(q) and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN
+    if not (native_device(q) and LATENT_MFMA and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN
             and (dq, dv) in LATENT_EXPAND_SIZES and dn % 8 == 0 and R % 8 == 0 and rot_dims % 2 == 0
             and cache.data_ptr() % 16 == 0):
         return 0
@@ -631,7 +631,7 @@ def heads_to_rows(x: torch.Tensor) -> torch.Tensor:
 
 # ---------------------------------------------------------------------------- generalized delta rule
 DECAY_SCALE = math.exp(-0.5)
-# XGS_TUNE delta_two_pass=0: the one-pass scan kernel (any head size; A/B and tests)
+# XGS_TUNE delta_two_pass=0: the one-pass scan kernel for every step (any head size; A/B and tests)
 DELTA_TWO_PASS = tune.get_bool("delta_two_pass", True)
 UNIT_KEY_EPS = 1e-6
 # prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on, which take what
@@ -639,6 +639,12 @@ UNIT_KEY_EPS = 1e-6
 DELTA_CHUNK = True
 DELTA_CHUNK_D = (32, 64)
 DELTA_CHUNK_MIN = 32
+
+
+def _delta_chunk_ok(proj: torch.Tensor, off_v: int, D: int, sm: SeqMeta) -> bool:
+    es = proj.element_size()
+    return (DELTA_TWO_PASS and DELTA_CHUNK and D in DELTA_CHUNK_D and DELTA_CHUNK_MIN <= sm.max_q <= 65535 * 16
+            and sm.num_seqs <= 65535 and proj.data_ptr() % 16 == 0 and proj.stride(0) * es % 16 == 0 and off_v * es % 16 == 0)
 
 
 def delta_rule_scan(proj: torch.Tensor, off_r: int, off_k: int, off_v: int, off_a: int, wl: torch.Tensor,
@@ -653,9 +659,7 @@ def delta_rule_scan(proj: torch.Tensor, off_r: int, off_k: int, off_v: int, off_
     if native_device(proj):
         assert proj.stride(1) == 1 and wl.stride(1) == 1 and wl.dtype == proj.dtype
         assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, D)
-        es = proj.element_size()
-        if DELTA_CHUNK and D in DELTA_CHUNK_D and DELTA_CHUNK_MIN <= sm.max_q <= 65535 * 16 and sm.num_seqs <= 65535 and proj.data_ptr() % 16 == 0 \
-                and proj.stride(0) * es % 16 == 0 and off_v * es % 16 == 0:
+        if _delta_chunk_ok(proj, off_v, D, sm):
             scratch = torch.empty(mixers().delta_chunk_scratch_floats(T, sm.num_seqs, H, D), dtype=torch.float32,
                                   device=proj.device)
             mixers().delta_chunk(proj.data_ptr(), is_f32(proj), proj.stride(0), off_r, off_k, off_v, off_a, wl.data_ptr(),
@@ -707,7 +711,7 @@ def delta_rule_out(o: torch.Tensor, norm_w: torch.Tensor, gate: torch.Tensor, ep
 
 def _delta_step_ok(proj: torch.Tensor, w2: torch.Tensor, state: torch.Tensor, D: int, sm: SeqMeta, dtype: torch.dtype) -> bool:
     lr = w2.shape[1]
-    return (native_device(proj) and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16
+    return (native_device(proj) and DELTA_TWO_PASS and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16
             and D in (32, 64, 128) and 8 <= lr <= 256 and lr % 8 == 0 and sm.num_seqs <= 65535 and proj.stride(1) == 1
             and proj.stride(0) % 4 == 0 and proj.data_ptr() % 8 == 0 and w2.is_contiguous() and w2.data_ptr() % 16 == 0
             and state.data_ptr() % 16 == 0)
@@ -1133,9 +1137,10 @@ MOE_PF_MIN = 96   # average rows per expert from which gated experts run on gemm
 # products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
 # us: tiles of 16 104 / 142 / - / 230 / -, 32 112 / 113 / 115 / 175 / 233, 64 121 / 123 / 123 / 127 / 191; 32 experts of
 # 2 x 1024 x 2048 at 8: 72 / 73 / 79. Tiles of 128 belong to the kernel of prompt-sized steps.
-MOE_TILE32_MIN = tune.get_int("moe_tile32_min", 8)
-MOE_TILE_SMALL, MOE_TILES = 16, ((128, 128), (64, 24), (32, MOE_TILE32_MIN))
-MOE_TILES_GENERAL = ((128, 128), (64, 64), (32, 12))   # the other kernels (float32, K of odd 32s): padding costs more there
+# XGS_TUNE moe_tile32_min=N: average rows per expert from which 32-row tiles replace 16-row ones, whatever the kernel
+MOE_TILE_SMALL, MOE_TILES = 16, ((128, 128), (64, 24), (32, tune.get_int("moe_tile32_min", 8)))
+# the other kernels (float32, K of odd 32s): padding costs more there
+MOE_TILES_GENERAL = ((128, 128), (64, 64), (32, tune.get_int("moe_tile32_min", 12)))
 
 
 def _glu_ref(g, u, kind, limit, alpha):
@@ -1488,7 +1493,8 @@ def talk_mix(o_all: torch.Tensor, talk: torch.Tensor, H: int, G: int, dv: int,
 
 
 # ---------------------------------------------------------------------------- gated linear recurrence
-# XGS_TUNE scan_cols=32|64: state columns per workgroup of the gated linear scan (0: by the size of the step)
+# XGS_TUNE scan_cols=32|64: the gated linear scan, token by token, with that many state columns per workgroup (0: the kernel and
+# the columns by the size of the step)
 SCAN_COLS = tune.get_int("scan_cols", 0)
 # XGS_TUNE scan_two_pass=0: every portion in one workgroup per (sequence, head, column block) (A/B and tests)
 SCAN_TWO_PASS = tune.get_bool("scan_two_pass", True)
@@ -1512,7 +1518,7 @@ CHUNK_SCAN_MIN_SEG, CHUNK_SCAN_MAX_SEGS = 64, 32
 
 
 def _chunk_scan_ok(sm: SeqMeta, dk: int) -> bool:
-    return CHUNK_SCAN and sm.max_q >= CHUNK_SCAN_MIN and dk <= CHUNK_SCAN_MAX_DK and sm.num_seqs <= CHUNK_SCAN_MAX_SEQS
+    return CHUNK_SCAN and not SCAN_COLS and sm.max_q >= CHUNK_SCAN_MIN and dk <= CHUNK_SCAN_MAX_DK and sm.num_seqs <= CHUNK_SCAN_MAX_SEQS
 
 
 def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
@@ -1520,7 +1526,7 @@ def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: in
     whole = (sm.max_q + 15) // 16 * 16
     wgs = max(1.0, T / sm.max_q) * H * ((dv + cols - 1) // cols)   # portions as long as the longest
     n = min(CHUNK_SCAN_MAX_SEGS, int(CHUNK_SCAN_FILL_WGS / wgs), whole // (CHUNK_SCAN_MIN_SEG * (2 if dk > 64 else 1)))
-    if n < 3:
+    if n < 3 or not SCAN_TWO_PASS:
         return whole, None
     seg = ((whole + n - 1) // n + 15) // 16 * 16
     return seg, torch.empty(mixers().chunk_scan_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32,
@@ -1573,7 +1579,7 @@ STATE_STEP = True
 
 def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int, state: Optional[torch.Tensor] = None) -> bool:
     # (sizes: gla_step_rows of state_step.hip, at most 16 rows per thread)
-    return (STATE_STEP and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
+    return (STATE_STEP and not SCAN_COLS and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
             and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0
             and (state is None or state.data_ptr() % 16 == 0))
 
