@@ -80,7 +80,6 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, pos_table: Optional[torch
 
 
 # ---------------------------------------------------------------------------- products of a few rows
-ROWS_LINEAR = True
 ROWS_LINEAR_MAX = 64       # rows (four 16-row tiles of x in the registers of a wave)
 # Sizes of a workgroup's share (us, cold weights, 64 rows of x): 64 weight rows while that makes at most one workgroup per
 # compute unit, 128 beyond (14336x4096 25.1 narrow against 35.9 wide, 18560x4096 43.5 against 36.9).
@@ -98,7 +97,7 @@ def step_tickets(like: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
     """Words for the products of a step of `rows` rows on `like`'s device, uncleared (embed_rows clears them), or None
     where no product of the step takes them. They belong to the step (SeqMeta.tickets): launches of one stream follow each
     other, and each leaves the words zero."""
-    if not (ROWS_LINEAR and native_device(like) and like.dtype == torch.bfloat16 and rows <= ROWS_LINEAR_MAX):
+    if not (native_device(like) and like.dtype == torch.bfloat16 and rows <= ROWS_LINEAR_MAX):
         return None
     return torch.empty(_ROWS_TICKETS, dtype=torch.int32, device=like.device)
 
@@ -132,7 +131,7 @@ def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias:
     """The plan of x . w^T on the kernel of a few rows, or None: bfloat16 on one device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
     pieces, K in whole staged rows, nothing that wants a derivative, and tickets where K is in parts (clearing them would cost
     what the parts gain) unless the `slabs` are the result. What is refused here goes to torch, which refuses what it cannot do."""
-    if not (ROWS_LINEAR and native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+    if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and w.device == x.device and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX and _forward_only(x, w, bias)):
         return None
     N, K = w.shape
@@ -318,14 +317,11 @@ def scaled_add_rmsnorm(x: torch.Tensor, y: Optional[torch.Tensor], w: torch.Tens
 
 
 # ---------------------------------------------------------------------------- ... and the next convolution, single tokens
-ROW_UPDATE = True
-
-
 def step_rows(sm: SeqMeta, x: torch.Tensor, dtype: torch.dtype, taps: int = 0) -> bool:
     """Whether a step's residual rows x [T, W] are updated by the kernels of few rows that add the parts of a product
     (post_norm_residual, and with `taps` row_update, which forms the next convolution of single tokens)."""
     T, W = x.shape
-    return (ROW_UPDATE and native_device(x) and dtype == torch.bfloat16 and 1 <= T <= ROWS_LINEAR_MAX and W % 4 == 0
+    return (native_device(x) and dtype == torch.bfloat16 and 1 <= T <= ROWS_LINEAR_MAX and W % 4 == 0
             and W <= 8192 and (taps == 0 or (2 <= taps <= 4 and sm.max_q == 1)))
 
 
@@ -528,7 +524,6 @@ def latent_attention(qabs: torch.Tensor, q: torch.Tensor, dn: int, gate: torch.T
 # 64 and 128: 33 -> 30 and 46 -> 35 us alone, 123 -> 61 and 208 -> 89 behind 1024 tokens), however many key rows there are to a
 # token up to the 32 that were measured (128 tokens behind 4000: 722 -> 225 us); 4 x 2048 tokens 950 -> 205 and 3857 -> 395. The
 # rows are bounded because their number is: single tokens of many sequences in the step each count a whole window.
-LATENT_EXPAND = True
 LATENT_EXPAND_MIN = 64
 LATENT_EXPAND_ROWS, LATENT_EXPAND_BYTES = 32, 1 << 30   # key rows per token, and what all of them take expanded (and gathered)
 LATENT_EXPAND_SIZES = ((96, 64), (192, 128))        # (dn + rd, dv)
@@ -544,7 +539,7 @@ def _latent_key_rows(sm: SeqMeta, T: int, window: int, block_size: int) -> int:
 def _latent_expands(q, dn: int, R: int, dv: int, rot_dims: int, window: int, block_size: int, sm: SeqMeta, cache) -> int:
     """Key rows that a step's portions are expanded over, 0 where the attention stays in latent space."""
     T, H, dq = q.shape
-    if not (native_device(q) and LATENT_MFMA and LATENT_EXPAND and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN
+    if not (native_device(q) and LATENT_MFMA and q.dtype == torch.bfloat16 and sm.max_q >= LATENT_EXPAND_MIN
             and (dq, dv) in LATENT_EXPAND_SIZES and dn % 8 == 0 and R % 8 == 0 and rot_dims % 2 == 0
             and cache.data_ptr() % 16 == 0):
         return 0
@@ -556,7 +551,6 @@ def _latent_expands(q, dn: int, R: int, dv: int, rot_dims: int, window: int, blo
 # Steps of single tokens (latent_decode.hip): shares of a window while the grid stays within 256 workgroups, at most 16. From the
 # queries to the heads' outputs, us, 32 heads, in 1 / 2 / 4 / 8 / 16 shares: 64 sequences of 1024 keys, R = 256 43 / 32 / 29 / 31
 # / 42, R = 512 82 / 56 / 48 / 65 / 95; one sequence of 4000 keys, R = 512, in 8 / 16 / 32 / 63 shares 48 / 43 / 49 / 65.
-LATENT_DECODE = True
 LATENT_DECODE_WGS, LATENT_DECODE_SHARES = 256, 16
 LATENT_PAGES = 2048     # page table entries of a share
 
@@ -564,7 +558,7 @@ LATENT_PAGES = 2048     # page table entries of a share
 def _latent_shares(q, uv, R: int, rd: int, dv: int, window: int, block_size: int, sm: SeqMeta, cache=None) -> int:
     """Shares of the window for latent_decode, 0 where it does not apply."""
     T, H = q.shape[:2]
-    if not (native_device(q) and LATENT_MFMA and LATENT_DECODE and q.dtype == torch.bfloat16 and sm.max_q == 1
+    if not (native_device(q) and LATENT_MFMA and q.dtype == torch.bfloat16 and sm.max_q == 1
             and 1 <= T == sm.num_seqs <= 65535 and R in (64, 128, 256, 512) and rd in (32, 64) and dv % 16 == 0
             and uv.data_ptr() % 16 == 0 and (cache is None or cache.data_ptr() % 16 == 0)):
         return 0
@@ -636,14 +630,13 @@ DELTA_TWO_PASS = tune.get_bool("delta_two_pass", True)
 UNIT_KEY_EPS = 1e-6
 # prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on, which take what
 # 32 tokens of the scan take (19.7 against 19.8 us, 32 heads of 64): one takes 17.9 against 14.2, four 23 against 33
-DELTA_CHUNK = True
 DELTA_CHUNK_D = (32, 64)
 DELTA_CHUNK_MIN = 32
 
 
 def _delta_chunk_ok(proj: torch.Tensor, off_v: int, D: int, sm: SeqMeta) -> bool:
     es = proj.element_size()
-    return (DELTA_TWO_PASS and DELTA_CHUNK and D in DELTA_CHUNK_D and DELTA_CHUNK_MIN <= sm.max_q <= 65535 * 16
+    return (DELTA_TWO_PASS and D in DELTA_CHUNK_D and DELTA_CHUNK_MIN <= sm.max_q <= 65535 * 16
             and sm.num_seqs <= 65535 and proj.data_ptr() % 16 == 0 and proj.stride(0) * es % 16 == 0 and off_v * es % 16 == 0)
 
 
@@ -711,7 +704,7 @@ def delta_rule_out(o: torch.Tensor, norm_w: torch.Tensor, gate: torch.Tensor, ep
 
 def _delta_step_ok(proj: torch.Tensor, w2: torch.Tensor, state: torch.Tensor, D: int, sm: SeqMeta, dtype: torch.dtype) -> bool:
     lr = w2.shape[1]
-    return (native_device(proj) and DELTA_TWO_PASS and STATE_STEP and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16
+    return (native_device(proj) and DELTA_TWO_PASS and sm.max_q == 1 and proj.dtype == w2.dtype == dtype == torch.bfloat16
             and D in (32, 64, 128) and 8 <= lr <= 256 and lr % 8 == 0 and sm.num_seqs <= 65535 and proj.stride(1) == 1
             and proj.stride(0) % 4 == 0 and proj.data_ptr() % 8 == 0 and w2.is_contiguous() and w2.data_ptr() % 16 == 0
             and state.data_ptr() % 16 == 0)
@@ -1504,7 +1497,6 @@ SCAN_FILL_WGS = 192       # ... when their one-launch form would start at most t
 
 # Prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/chunk_scan.hip). From one whole chunk on: 12
 # sequences of 16 tokens take 12 us against 18 token by token, 4 of 8 the same 11 (16 heads of 64 x 128).
-CHUNK_SCAN = True
 CHUNK_SCAN_MIN = 16
 CHUNK_SCAN_MAX_DK = 128    # state rows a wave holds
 CHUNK_SCAN_MAX_SEQS = 2047   # (sequences x segments are one grid dimension)
@@ -1518,7 +1510,7 @@ CHUNK_SCAN_MIN_SEG, CHUNK_SCAN_MAX_SEGS = 64, 32
 
 
 def _chunk_scan_ok(sm: SeqMeta, dk: int) -> bool:
-    return CHUNK_SCAN and not SCAN_COLS and sm.max_q >= CHUNK_SCAN_MIN and dk <= CHUNK_SCAN_MAX_DK and sm.num_seqs <= CHUNK_SCAN_MAX_SEQS
+    return not SCAN_COLS and sm.max_q >= CHUNK_SCAN_MIN and dk <= CHUNK_SCAN_MAX_DK and sm.num_seqs <= CHUNK_SCAN_MAX_SEQS
 
 
 def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
@@ -1574,12 +1566,9 @@ def lower_bound_gates(proj: torch.Tensor, off_q: int, off_f: int, n: int, f_bias
 
 
 # One token per sequence: state_step.hip (a pass over the states); other steps, and states of odd sizes, run as scans
-STATE_STEP = True
-
-
 def _gla_step_ok(v: torch.Tensor, sm: SeqMeta, dk: int, dv: int, state: Optional[torch.Tensor] = None) -> bool:
     # (sizes: gla_step_rows of state_step.hip, at most 16 rows per thread)
-    return (STATE_STEP and not SCAN_COLS and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
+    return (not SCAN_COLS and sm.max_q == 1 and dv % 4 == 0 and 4 <= dv <= 256 and 1 <= dk <= 256 and -(-dk // (256 // (dv // 4))) <= 16
             and sm.num_seqs <= 65535 and v.stride(0) % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0
             and (state is None or state.data_ptr() % 16 == 0))
 
