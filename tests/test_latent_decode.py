@@ -8,6 +8,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
+from _seq_util import record_native
+
 pytestmark = pytest.mark.gpu
 
 
@@ -15,7 +17,7 @@ pytestmark = pytest.mark.gpu
                                               (16, 16, 64, 80, 128, 0)])
 @pytest.mark.parametrize("lens,window,bs", [([1], 8, 16), ([64, 65, 1], 64, 16), ([300, 1, 129, 1000, 7], 512, 16),
                                             ([2100, 40], 4096, 1), ([700] * 9, 333, 32)])
-def test_against_fp64(H, dn, rd, dv, R, rot, lens, window, bs):
+def test_against_fp64(H, dn, rd, dv, R, rot, lens, window, bs, monkeypatch):
     g = torch.Generator().manual_seed(H + len(lens))
     T, dq = len(lens), dn + rd
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
@@ -38,7 +40,9 @@ def test_against_fp64(H, dn, rd, dv, R, rot, lens, window, bs):
     scale = dq ** -0.5
     dev = [t.cuda() for t in (q, gate, cache, uk, uv, table)]
     assert sq._latent_shares(dev[0], dev[4], R, rd, dv, window, bs, sm) > 0
+    calls = record_native(monkeypatch, sq)
     got = sq.latent_attention_heads(dev[0], dn, dev[1], dev[2], dev[3], dev[4], dev[5], rot, window, scale, bs, sm)
+    assert calls == ["latent_decode"]
     # the queries in latent space as the step rounds them
     qabs = torch.bmm(dev[0][:, :, :dn].transpose(0, 1), dev[3].view(H, dn, R)).cpu().double()
     for t, n in enumerate(lens):

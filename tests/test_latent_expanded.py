@@ -9,6 +9,7 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
+from _seq_util import record_native
 from test_chunk_scan import layout
 
 F64 = torch.float64
@@ -40,8 +41,10 @@ def test_against_fp64(H, dn, rd, dv, R, rot_dims, portions, window, monkeypatch)
     max_pos = int(sm.seq_lens.max())
     rot = sq.build_rot_table(rot_dims, 100.0, max_pos + 1).cuda()
     scale = (dn + rd) ** -0.5
+    calls = record_native(monkeypatch, sq)
     got = sq.latent_attention_heads(q.cuda(), dn, gate.cuda(), cache.cuda(), uk.cuda(), uv.cuda(), rot, rot_dims, window, scale, bs, sm)
     # the expanded form, with every key row counted
+    assert calls == ["latent_gather", "latent_prompt_attention"]
     assert routed and 32 * T >= routed[0] >= sum(n + min(c, window - 1) for c, n in portions)
     at, out = 0, []
     for i, (ctx, n) in enumerate(portions):

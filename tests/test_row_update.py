@@ -8,6 +8,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
+from _seq_util import record_native
+
 pytestmark = pytest.mark.gpu
 
 
@@ -49,7 +51,8 @@ def conv(r, w, state, slots, ctx):
 @pytest.mark.parametrize("W,taps", [(4, 4), (2048, 4), (2052, 3), (4100, 2), (8192, 4)])
 @pytest.mark.parametrize("S1,S2", [(0, 0), (1, 2), (4, 0), (8, 3)])
 @pytest.mark.parametrize("T", [1, 5])
-def test_norms_and_convolution(W, taps, S1, S2, T):
+def test_norms_and_convolution(W, taps, S1, S2, T, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     g = torch.Generator().manual_seed(W + S1)
     slots, ctx = [3, -1, 0, 4, 2][:T], [7, 0, 0, 1, 2][:T]
     sm = meta(T, slots, ctx)
@@ -90,6 +93,7 @@ def test_norms_and_convolution(W, taps, S1, S2, T):
             close(n32, r, W / 2 + 16, big)
         close(h[live], want_h[live], W / 2 + 40, big * 8)
         close(st, want_st, W / 2 + 16, max(big, 5.0))
+    assert calls == ["row_update"] * 5
 
 
 @pytest.mark.parametrize("W", [4, 2048, 4096, 4100])

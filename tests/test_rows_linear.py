@@ -10,6 +10,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
+from _seq_util import record_native
+
 gpu = pytest.mark.gpu
 # rows on both sides of the tiles of 16; columns and K on both sides of a workgroup's share and of the parts of K
 ROWS = (1, 16, 17, 33, 64)
@@ -52,7 +54,8 @@ def check(got, want, scale, K, slope):
 @gpu
 @pytest.mark.parametrize("N,K", SHAPES)
 @pytest.mark.parametrize("T", ROWS)
-def test_products(T, N, K):
+def test_products(T, N, K, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     g, x, w, sm = data(T, N, K)
     z, mag = x.double() @ w.double().t(), float((x.double().abs() @ w.double().abs().t()).max())
     assert sq._rows_plan_of(x, w, sm, None, False) is not None
@@ -66,6 +69,7 @@ def test_products(T, N, K):
     neg = 0.9 * (torch.expm1(v.clamp(max=0)) - v) + 0.5 * v
     check(sq.linear_xielu(x, w, b, 0.6, 0.9, sm), torch.where(v > 0, 0.6 * v * v + 0.5 * v, neg), mag + 8, K, slope)
     assert not bool(sm.tickets.any())                      # every launch leaves the words zero
+    assert calls == ["rows_linear"] * 4
     # rows of a wider activation tensor
     wide = torch.full((T, K + 16), float("nan"), device="cuda", dtype=torch.bfloat16)
     wide[:, 8:8 + K] = x
@@ -75,7 +79,8 @@ def test_products(T, N, K):
 @gpu
 @pytest.mark.parametrize("N,K", [(8, 128), (136, 1024), (2048, 2048), (16400, 256)])
 @pytest.mark.parametrize("T", ROWS)
-def test_gated_products(T, N, K):
+def test_gated_products(T, N, K, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     _, x, w, sm = data(T, N, K, 1)
     z, mag = x.double() @ w.double().t(), float((x.double().abs() @ w.double().abs().t()).max())
     a, u = z[:, :N // 2], z[:, N // 2:]
@@ -86,6 +91,7 @@ def test_gated_products(T, N, K):
     check(sq.linear_glu(x, w, sq.GLU_GELU_TANH, sm=sm), 0.5 * a * (1 + tanh) * u, mag, K, slope)
     ac, uc = a.clamp(max=2.0), u.clamp(-2.0, 2.0)
     check(sq.linear_glu(x, w, sq.GLU_CLAMPED, 2.0, 1.702, sm), ac * torch.sigmoid(1.702 * ac) * (uc + 1), mag, K, slope)
+    assert calls == ["rows_linear"] * 3
 
 
 @gpu

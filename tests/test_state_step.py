@@ -7,6 +7,8 @@ import torch
 
 from xgserve.ops import seqmix as sq
 
+from _seq_util import record_native
+
 pytestmark = pytest.mark.gpu
 
 
@@ -23,7 +25,8 @@ SLOTS, CTX = [2, -1, 0, 4], [5, 3, 0, 1]
 @pytest.mark.parametrize("H,dk,dv", [(1, 1, 4), (3, 64, 128), (2, 128, 128), (2, 256, 64), (3, 33, 20), (2, 16, 256)])
 @pytest.mark.parametrize("mode", ["plain", "complement", "raw", "decay", "bonus"])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-def test_gated_linear(H, dk, dv, mode, dt):
+def test_gated_linear(H, dk, dv, mode, dt, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     g = torch.Generator().manual_seed(dk + dv)
     rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
     T, n, sm = len(SLOTS), H * dk, meta(SLOTS, CTX)
@@ -52,6 +55,7 @@ def test_gated_linear(H, dk, dv, mode, dt):
         fd = decay.double().repeat_interleave(dk).expand(T, n) if mode == "decay" else f.double()
         if mode == "complement":
             kd = 1 - fd
+    assert "gla_step" in calls and "gated_linear_scan" not in calls
     want = state.double().clone()
     for t, s in enumerate(SLOTS):
         if s < 0:
@@ -71,7 +75,8 @@ def test_gated_linear(H, dk, dv, mode, dt):
 
 @pytest.mark.parametrize("H,G,N,P", [(1, 1, 1, 4), (4, 2, 128, 64), (6, 2, 33, 20), (2, 1, 256, 64), (2, 2, 16, 256)])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-def test_state_space(H, G, N, P, dt):
+def test_state_space(H, G, N, P, dt, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     g = torch.Generator().manual_seed(N + P)
     rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
     T, sm = len(SLOTS), meta(SLOTS, CTX)
@@ -80,6 +85,7 @@ def test_state_space(H, G, N, P, dt):
     st, xg = state.cuda(), xbc.cuda()
     assert sq._gla_step_ok(xg, sm, N, P)
     y = sq.ssm_scan(xg, raw.cuda()[:, 3:], bias.cuda(), A.cuda(), D.cuda(), st, H, G, N, P, sm)
+    assert calls == ["ssm_step"]
     z = xbc.double()
     x = z[:, :H * P].view(T, H, P)
     B, C = (z[:, H * P + i * G * N:H * P + (i + 1) * G * N].view(T, G, N).repeat_interleave(H // G, 1) for i in (0, 1))
@@ -99,7 +105,8 @@ def test_state_space(H, G, N, P, dt):
 
 
 @pytest.mark.parametrize("H,D,lr", [(2, 32, 8), (3, 64, 32), (2, 128, 64), (1, 64, 256)])
-def test_delta_rule(H, D, lr):
+def test_delta_rule(H, D, lr, monkeypatch):
+    calls = record_native(monkeypatch, sq)
     g = torch.Generator().manual_seed(D + lr)
     rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
     T, HD, sm = len(SLOTS), H * D, meta(SLOTS, CTX)
@@ -108,6 +115,7 @@ def test_delta_rule(H, D, lr):
     a_bias, w0, norm, state = rnd(HD), rnd(HD), rnd(HD), rnd(5, H, D, D)
     st = state.cuda()
     y = sq.delta_rule_mix(proj.cuda(), w2.cuda(), a_bias.cuda(), w0.cuda(), norm.cuda(), st, 1e-5, H, D, sm, torch.bfloat16)
+    assert calls == ["delta_step"]
     p = proj.double()
     r, k, v, gate, za = (p[:, i * HD:(i + 1) * HD].view(T, H, D) for i in range(5))
     wl = torch.tanh(p[:, 5 * HD:]) @ w2.double().T
@@ -142,7 +150,7 @@ def test_odd_states_run_as_scans():
 
 
 @pytest.mark.parametrize("dk,dv", [(88, 176), (168, 96), (120, 136)])
-def test_states_with_too_many_rows_per_thread_run_as_scans(dk, dv):
+def test_states_with_too_many_rows_per_thread_run_as_scans(dk, dv, monkeypatch):
     """Sizes within 128 x 128 elements whose columns do not divide the workgroup: one token, through the public ops."""
     g = torch.Generator().manual_seed(dk)
     T, H, sm = len(SLOTS), 2, meta(SLOTS, CTX)
@@ -151,8 +159,10 @@ def test_states_with_too_many_rows_per_thread_run_as_scans(dk, dv):
     xbc = torch.randn(T, H * dv + 2 * dk, generator=g)
     dt, bias, A, D = torch.randn(T, H, generator=g), torch.randn(H, generator=g), torch.randn(H, generator=g), torch.randn(H, generator=g)
     st, st2 = state.cuda(), state.cuda()
+    calls = record_native(monkeypatch, sq)
     o = sq.gated_linear_scan(q.cuda(), f.cuda(), k.cuda(), v.cuda(), st, H, dk, dv, sm).cpu().double()
     y = sq.ssm_scan(xbc.cuda(), dt.cuda(), bias.cuda(), A.cuda(), D.cuda(), st2, H, 1, dk, dv, sm).cpu().double()
+    assert calls == ["gated_linear_scan", "ssm_scan"]
     step = torch.nn.functional.softplus(dt.double() + bias.double())
     for t, s in enumerate(SLOTS):
         if s < 0:
