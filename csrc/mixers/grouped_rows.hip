@@ -6,11 +6,17 @@
 //
 // Measured on 8 experts of 2 x 3584 x 4096 (gated) and 4096 x 3584, cold weights, us, against fragments read straight from
 // global memory by four waves with a quarter of K each:
-//   64 tokens, top 2 (tiles of 32)    73.7 + 39.2 against 140.7 + 70.9   (6.3 TB/s of weights)
+//   64 tokens, top 2 (tiles of 32)    73.7 + 39.2 against 140.7 + 70.9   (6.4 and 6.0 TB/s of weights; in a step, between other
+//                                     launches, 78.8 + 45.7 against 152 + 82: 6.0 and 5.1)
 //   150 tokens (64)                   79.3 + 47.6 against 175.8 + 105.6 (its 32-row tiles)
 //   4 tokens, 1 token (16)            53.7 + 28.5, 22.1 + 12.1 against 88.3 + 40.7, 68.7 + 34.0
-// Several small workgroups per compute unit (40 to 60 KB of LDS) hide that the grid seldom is a multiple of 256: one
-// workgroup of 144 KB per unit took 88.6 for the first.
+// and against tiles of 64 x 128 (gated) and 64 x 256 columns staged in LDS, which had the experts of 64 rows and more; sorting
+// and both products:
+//   64 / 80 / 95 rows on average, gated               202 / 248 / 246 against 367 / 397 / 557
+//   64 / 95 / 112 / 127 rows, one weight block        165 / 194 / 195 / 233 against 318 / 357 / 380 / 405
+//   32 experts of 1024 x 2048, 64 / 95 rows           141 / 169 against 193 / 228 (gated), 114 / 138 against 163 / 177
+// Two to four workgroups share a compute unit (40 KB of LDS in the gated form for 16 rows, 48 to 61 for 32, 64 and 72 for 64), which
+// hides that the grid seldom is a multiple of 256: one workgroup of 144 KB per unit took 88.6 for the first.
 #include "attention_common.h"
 #include "glds.h"
 #include "glu.h"

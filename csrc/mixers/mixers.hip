@@ -944,7 +944,7 @@ __global__ void xielu_kernel(const T* __restrict__ in, const float* __restrict__
 }
 
 // four neighbouring columns per thread, a row (grid.y) at a time, so that no column is a remainder; bound by the bytes (8192 x 8192:
-// 48.6 us, 68 with a 64-bit remainder and the general expm1)
+// 43.5 us in a step, 65.7 with a 64-bit remainder and the general expm1)
 template <typename T>
 __global__ __launch_bounds__(256) void xielu_vec_kernel(const T* __restrict__ in, const float* __restrict__ bias, float sp, float cn,
                                                         T* __restrict__ out, int64_t rows, int F) {

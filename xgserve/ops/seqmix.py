@@ -1129,7 +1129,9 @@ MOE_PF_MIN = 96   # average rows per expert from which gated experts run on gemm
 # Rows per expert tile of the sorted layout, and the average rows per expert from which it is taken. Weight-streaming
 # products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
 # us: tiles of 16 104 / 142 / - / 230 / -, 32 112 / 113 / 115 / 175 / 233, 64 121 / 123 / 123 / 127 / 191; 32 experts of
-# 2 x 1024 x 2048 at 8: 72 / 73 / 79. Tiles of 128 belong to the kernel of prompt-sized steps.
+# 2 x 1024 x 2048 at 8: 72 / 73 / 79. Tiles of 64 serve up to 127 rows (grouped_rows.hip has the times of the kernel that they took
+# the place of: 1.3 to 2.3 times as long); tiles of 128 belong to the kernel of prompt-sized steps, which a 127-row average on
+# tiles of 64 still beats (233 us against 313 at 128 rows, 8 experts of 3584 x 4096, one weight block).
 # XGS_TUNE moe_tile32_min=N: average rows per expert from which 32-row tiles replace 16-row ones, whatever the kernel
 MOE_TILE_SMALL, MOE_TILES = 16, ((128, 128), (64, 24), (32, tune.get_int("moe_tile32_min", 8)))
 # the other kernels (float32, K of odd 32s): padding costs more there
