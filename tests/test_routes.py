@@ -63,6 +63,27 @@ def test_products_that_torch_refuses_or_differentiates_stay_with_it(as_if_native
     assert plan(x, w) is not None
 
 
+def test_products_that_are_recorded_stay_with_torch(as_if_native):
+    """A tracer, a dispatch mode or a tensor type of its own sees torch's operator (a kernel's result would be a constant to it)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w = torch.randn(3, 256).bfloat16(), torch.randn(64, 256).bfloat16()
+    sm = types.SimpleNamespace(tickets=torch.zeros(128, dtype=torch.int32))
+    want = torch.nn.functional.linear(2 * x, w)
+    traced = torch.jit.trace(lambda h: sq.linear(h, w, sm), (x,), check_trace=False)
+    torch.testing.assert_close(traced(2 * x), want)
+    torch.testing.assert_close(make_fx(lambda h: sq.linear(h, w, sm))(x)(2 * x), want)
+    with FlopCounterMode(display=False) as count:
+        sq.linear(x, w, sm)
+    assert count.get_total_flops() == 2 * 3 * 256 * 64
+    with FakeTensorMode() as mode:
+        assert sq.linear(mode.from_tensor(x), mode.from_tensor(w), sm).shape == (3, 64)
+    fake = mode.from_tensor(x), mode.from_tensor(w)
+    assert sq.linear(*fake, sm).shape == (3, 64)
+    assert sq._rows_plan_of(x, torch.nn.Parameter(w, requires_grad=False), sm, None, False) is not None
+
+
 def test_tensors_that_lie_off_16_bytes_keep_the_general_kernels(as_if_native):
     """The wide kernels refuse them, which would raise; the general ones take them."""
     sm = types.SimpleNamespace(max_q=1, num_seqs=2, block_tables=torch.zeros(2, 4, dtype=torch.int32))

@@ -119,10 +119,15 @@ def _rows_plan(N: int, K: int, gated: bool):
 
 
 def _forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
-    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform. (A product on a kernel
-    of this library has no derivative; torch's has.)"""
-    if _fwd_ad._current_level >= 0 or _is_transformed(x) or _is_transformed(w) or (bias is not None and _is_transformed(bias)):
+    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform, no tracing or dispatch
+    mode, no tensor type of its own. (A product on a kernel of this library has no derivative and no operator to record; torch's
+    has.)"""
+    if _fwd_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing() \
+            or torch.compiler.is_compiling():
         return False
+    for t in (x, w, bias):
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or _is_transformed(t)):
+            return False
     return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))
 
 
