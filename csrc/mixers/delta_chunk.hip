@@ -9,27 +9,29 @@
 //   y = (U E) S + V,       U = T u', V = T N v,
 //   o = (R E) S + O,       R = r' - Q U, O = P v - Q V,
 //   S <- E S + k'^T v - b'^T y.
+// (U E and R E are formed from u and r times the decays before them, R E = r E / s - Q U E: one rounding less for each factor.)
 // Only the right factors meet the state, so a first launch forms U E, V, R E, O, k', b' of all chunks at once (one wave per chunk
 // and head; T by forward substitution: the compact form of a product of rank-one updates, Bischof and Van Loan 1987, as Yang et al.
 // 2024 use it for the delta rule over chunks of a sequence) and the chain that is left is three matrix products per 16 tokens. All of
 // it is fp32 arithmetic, the products of decays two floats each (Prod).
 //
-// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets), 2048 tokens of 32 heads of 64: decays around
-// 0.97 3.2e-7 / 2.2e-7 (3.1e-7 / 2.1e-7), 0.73 6.9e-8 / 6.6e-8 (6.6e-8 / 4.9e-8), 0.55 5.3e-8 / 6.1e-8 (4.6e-8 / 4.5e-8): the
-// output has four roundings of its size where the loop has two. (Sums of log2 decays and one chain per sum gave 1.8e-7 / 2.3e-7 in
-// the second.) That takes the separate sums: k . r has one sign in a trained model, and a chain of 64 rounds at the whole sum's
-// size; what is taken out of the state and of the outputs is summed up by itself before it joins them.
+// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets), 497 to 1024 tokens of 32 heads of 64, r with
+// a share of k: decays around 0.97 3.03e-7 / 1.99e-7 (3.03e-7 / 1.97e-7), 0.73 6.6e-8 / 4.9e-8 (6.6e-8 / 4.9e-8), 0.55 4.7e-8 /
+// 4.3e-8 (4.6e-8 / 4.5e-8); heads of 32 0.92 to 1.03 of the loop's. (Sums of log2 decays and one chain per sum gave 1.8e-7 / 2.3e-7
+// in the second.) That takes: separate sums, because k . r has one sign in a trained model and a chain of 64 rounds at the
+// whole sum's size, and P in two floats (4.9e-8 in the second; 6.1e-8 in one, from half as many chains); what is taken out of the state and of the
+// outputs summed up by itself and before the tokens' own terms, the latest and largest of them last; E in two floats.
 //
 // The second launch has one wave per 16 state columns of a (sequence, head). The first writes every operand in the order of the
 // matrix instructions' lanes; the waves bring it in by LDS DMA, three chunks ahead (in registers, two chunks ahead, the compiler
 // parks operands in accumulator registers, which waits for every load: 2.1 us a chunk). A chunk with an input out of range
 // (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
 //
-// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1030 -> 368 us (147 + 247 in a trace), one sequence of 2048
-// 835 -> 266, 64 tokens 33 -> 23 (log sums in single chains: 325, 236, 21). The first launch writes 24.6 KB per chunk and head and
-// forms three exponentials per token and channel; the second takes 1.8 us a chunk, 0.9 of them its 64 matrix instructions a wave,
-// the rest the way from one to the next: LDS reads behind the barrier, and y, which has to be complete before it goes back in.
-// (E S is formed behind y's products: in front of them it cost 8 us of 280.)
+// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1019 -> 380 us (172 + 258 in a step's trace), one sequence of
+// 2048 838 -> 273, 64 tokens 32 -> 23 (log sums in single chains: 325, 236, 21). The first launch writes 24.6 KB per chunk and head
+// and forms three exponentials per token and channel; the second takes 1.9 us a chunk, 0.9 of them its 64 matrix instructions a
+// wave, the rest the way from one to the next: LDS reads behind the barrier, and y, which has to be complete before it goes back
+// in. (E S is formed behind y's products: in front of them it cost 8 us of 280. k' v behind y instead of beside it: 380 against 394.)
 #include "glds.h"
 #include "mfma_f32.h"
 
@@ -38,7 +40,7 @@ namespace xgm {
 constexpr int kDcTok = 16;
 constexpr float kDeltaDecay = -0.6065306597126334f;   // log w = this * sigmoid
 
-// floats per (chunk, head): [U E | R E | k' | -b' | V | O] in lane order, then E per channel, then the flag
+// floats per (chunk, head): [U E | R E | k' | -b' | V | O] in lane order, then E per channel (at 0 and 2 D), the flag at D
 constexpr int dc_stride(int D) { return 6 * kDcTok * D + 256; }
 
 template <typename T, int D>
@@ -51,7 +53,7 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   constexpr int C = kDcTok, MT = D / 16, QE = D + 4, TPL = C * D / 64;   // (token, channel) pairs per lane
   constexpr int TG = 64 / D, TT = C / TG;                                // token groups, tokens per lane
   static_assert(D == 64 || D == 32, "a lane owns one channel");
-  __shared__ __attribute__((aligned(16))) float us[C * QE], rs[C * QE], ks[C * QE], bs[C * QE], ts[C * 20], es[D];
+  __shared__ __attribute__((aligned(16))) float us[C * QE], rs[C * QE], ks[C * QE], bs[C * QE], ts[C * 20];
   const int h = blockIdx.x, c = blockIdx.y, s = blockIdx.z;
   const int q0 = qsl[s], qn = qsl[s + 1] - q0, n = min(C, qn - C * c);
   if (slots[s] < 0 || n <= 0) return;
@@ -122,12 +124,13 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
     return;
   }
   __syncthreads();   // (ks is rewritten)
-  Prod run = {1.f, 0.f};   // from the token behind this one to the chunk's end
+  Prod run = {1.f, 0.f}, pre = run;   // from the token behind this one to the chunk's end, from the chunk's start to this one
   if (TG == 2) {
 #pragma unroll
     for (int i = 0; i < TT; ++i) run = prod_mul(run, wt[i]);
     const Prod up = {__shfl_xor(run.h, D % 64, 64), __shfl_xor(run.l, D % 64, 64)};
     run = tg ? Prod{1.f, 0.f} : up;
+    pre = tg ? up : Prod{1.f, 0.f};
   }
 #pragma unroll
   for (int i = TT - 1; i >= 0; --i) {
@@ -136,14 +139,22 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
     run = prod_mul(run, wt[i]);
     us[at] = prod_div(u[i], run);
   }
-  if (tg == 0) es[d] = dst[6 * C * D + d] = run.h + run.l;
+  if (tg == 0) dst[6 * C * D + d] = run.h, dst[6 * C * D + 2 * D + d] = run.l;
+  // u and r referred to the chunk's start, one rounding each: what U E and R E are made of
+  float ue[TT], re[TT];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    ue[i] = prod_times(pre, u[i]);
+    pre = prod_mul(pre, wt[i]);
+    re[i] = prod_times(pre, r_[i]);
+  }
   __syncthreads();
 
   // ---- the four 16 x 16 products, transposed: lane holds [position l16][position 4 g4 + r], the A operand of what follows. Each is
   // the sum of four chains (k . r of a trained model has one sign: a chain of 64 would round at the size of the whole sum).
-  f32x4_t Mc[4], Nc[4], Pc[4], Qc[4];
+  f32x4_t Mc[4], Nc[4], Pc[8], Qc[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) Mc[r] = Nc[r] = Pc[r] = Qc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < 4; ++r) Mc[r] = Nc[r] = Pc[r] = Pc[4 + r] = Qc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     float xu[4], xrr[4], xkk[4], xb[4];
@@ -153,22 +164,29 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
     for (int r = 0; r < 4; ++r) {
       Mc[r] = mfma_f32(xb[r], xu[r], Mc[r]);
       Nc[r] = mfma_f32(xkk[r], xu[r], Nc[r]);
-      Pc[r] = mfma_f32(xkk[r], xrr[r], Pc[r]);
+      Pc[4 * (m % 2) + r] = mfma_f32(xkk[r], xrr[r], Pc[4 * (m % 2) + r]);
       Qc[r] = mfma_f32(xb[r], xrr[r], Qc[r]);
     }
   }
-  float M[4], N[4], P[4], Q[4];
+  float M[4], N[4], P[4], Pl[4], Q[4];   // P as two floats: its part of an output is the output's size
   const int ti = tok_pos(l16);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int j = 4 * r + g4;   // the token at position 4 g4 + r
     M[r] = j < ti ? (Mc[0][r] + Mc[1][r]) + (Mc[2][r] + Mc[3][r]) : 0.f;
     N[r] = j < ti ? (Nc[0][r] + Nc[1][r]) + (Nc[2][r] + Nc[3][r]) : 0.f;
-    P[r] = j <= ti ? (Pc[0][r] + Pc[1][r]) + (Pc[2][r] + Pc[3][r]) : 0.f;
+    const Prod p0 = two_sum(Pc[0][r] + Pc[1][r], Pc[2][r] + Pc[3][r]), p1 = two_sum(Pc[4][r] + Pc[5][r], Pc[6][r] + Pc[7][r]);
+    const Prod p = two_sum(p0.h, p1.h);
+    P[r] = j <= ti ? p.h : 0.f, Pl[r] = j <= ti ? p.l + (p0.l + p1.l) : 0.f;
     Q[r] = j <= ti ? -((Qc[0][r] + Qc[1][r]) + (Qc[2][r] + Qc[3][r])) : 0.f;   // (Q enters with its sign)
   }
   *reinterpret_cast<float4*>(ts + l16 * 20 + 4 * g4) = make_float4(M[0], M[1], M[2], M[3]);
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const int at = tok_pos(TT * tg + i) * QE + d;
+    us[at] = ue[i], rs[at] = re[i];
+  }
   // ---- T = (1 + M)^-1: lane l16 solves for token l16's column, x_i = delta - sum_(j < i) M_ij x_j
   float x[C];
 #pragma unroll
@@ -198,7 +216,7 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   auto put = [&](int which, int m, f32x4_t y) {
     *reinterpret_cast<float4*>(dst + which * C * D + 256 * m + 4 * lane) = make_float4(y[0], y[1], y[2], y[3]);
   };
-  // ---- U (transposed product: position l16, channels 16 m + 4 g4 + r); k' and -b' as the A operands of the state's update
+  // ---- U E (transposed product: position l16, channels 16 m + 4 g4 + r); k' and -b' as the A operands of the state's update
   f32x4_t U[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -210,34 +228,34 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
       U[m] = mfma_f32(us[at], Tf[t], U[m]);
       kk[t] = ks[at], bb[t] = -bs[at];
     }
-    float e[4];
-    ld4(es + 16 * m + 4 * g4, e);
-    put(0, m, f32x4_t{U[m][0] * e[0], U[m][1] * e[1], U[m][2] * e[2], U[m][3] * e[3]}), put(2, m, kk), put(3, m, bb);
+    put(0, m, U[m]), put(2, m, kk), put(3, m, bb);
   }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < MT; ++m)
     *reinterpret_cast<float4*>(us + l16 * QE + 16 * m + 4 * g4) = make_float4(U[m][0], U[m][1], U[m][2], U[m][3]);
   __syncthreads();
-  // ---- R, then V and O column tile by column tile
+  // ---- R E, then V and O column tile by column tile
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     float r0[4];
     ld4(rs + l16 * QE + 16 * m + 4 * g4, r0);
-    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, V = y, O = y, R = y, QV = y;   // (what is taken out is summed up by itself: no roundings of the whole)
+    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, V = y, O = y, R = y;   // (what is taken out is summed up first: fewer roundings of the whole)
 #pragma unroll
     for (int t = 0; t < 4; ++t) R = mfma_f32(us[(4 * g4 + t) * QE + 16 * m + l16], Q[t], R);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) R[t] = (R[t] + r0[t]) * es[16 * m + 4 * g4 + t];
+    for (int t = 0; t < 4; ++t) R[t] += r0[t];
     put(1, m, R);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) y = mfma_f32(N[t], v[m][t], y), O = mfma_f32(P[t], v[m][t], O);
+    for (int t = 0; t < 4; ++t) y = mfma_f32(N[t], v[m][t], y);
 #pragma unroll
     for (int t = 0; t < 4; ++t) V = mfma_f32(Tf[t], y[t], V);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) QV = mfma_f32(Q[t], V[t], QV);
+    for (int t = 0; t < 4; ++t) O = mfma_f32(Q[t], V[t], O);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) O[t] += QV[t];
+    for (int t = 0; t < 4; ++t) O = mfma_f32(Pl[t], v[m][t], O);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) O = mfma_f32(P[t], v[m][t], O);
     put(4, m, V), put(5, m, O);
   }
 }
@@ -334,29 +352,25 @@ __global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float*
     }
     const float4 v0 = p4[64 * (4 * MT + w)], o0 = p4[64 * (5 * MT + w)];
     float4 k[MT], b[MT];
-    float e[MT][4];
+    float e[MT][4], el[MT][4];
     f32x4_t yc[2], oc[2];   // two chains each: even and odd 16s of the state's rows
     yc[0] = yc[1] = oc[0] = oc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const float4 u = p4[64 * m], r = p4[64 * (MT + m)];
-      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)], ld4(pe + 16 * m + 4 * g4, e[m]);
+      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)], ld4(pe + 16 * m + 4 * g4, e[m]), ld4(pe + 2 * D + 16 * m + 4 * g4, el[m]);
       yc[m % 2] = mfma_f32(u.x, S[m][0], yc[m % 2]), oc[m % 2] = mfma_f32(r.x, S[m][0], oc[m % 2]);
       yc[m % 2] = mfma_f32(u.y, S[m][1], yc[m % 2]), oc[m % 2] = mfma_f32(r.y, S[m][1], oc[m % 2]);
       yc[m % 2] = mfma_f32(u.z, S[m][2], yc[m % 2]), oc[m % 2] = mfma_f32(r.z, S[m][2], oc[m % 2]);
       yc[m % 2] = mfma_f32(u.w, S[m][3], yc[m % 2]), oc[m % 2] = mfma_f32(r.w, S[m][3], oc[m % 2]);
     }
-    // E S + k' v behind y's last products; what is taken out is summed up by itself
-    f32x4_t by[MT];
+    // E S behind y's last products; then what is taken out, summed up by itself, then the tokens' terms in their order
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], f32x4_t{e[m][0] * S[m][0], e[m][1] * S[m][1], e[m][2] * S[m][2], e[m][3] * S[m][3]});
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].y, v[1], S[m]);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].z, v[2], S[m]);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].w, v[3], S[m]);
+      for (int r = 0; r < 4; ++r) S[m][r] = prod_times({e[m][r], el[m][r]}, S[m][r]);
     const float y[4] = {yc[0][0] + yc[1][0] + v0.x, yc[0][1] + yc[1][1] + v0.y, yc[0][2] + yc[1][2] + v0.z, yc[0][3] + yc[1][3] + v0.w};
+    f32x4_t by[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].x, y[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
@@ -366,9 +380,13 @@ __global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float*
 #pragma unroll
     for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].w, y[3], by[m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], S[m] + by[m]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[m][r] += by[m][r];
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].y, v[1], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].z, v[2], S[m]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].w, v[3], S[m]);
     const float out[4] = {oc[0][0] + oc[1][0] + o0.x, oc[0][1] + oc[1][1] + o0.y, oc[0][2] + oc[1][2] + o0.z,
                           oc[0][3] + oc[1][3] + o0.w};
 #pragma unroll

@@ -44,6 +44,11 @@ __device__ __forceinline__ Prod prod_mul(Prod a, Prod b) {
   return {h, fmaf(a.h, b.l, fmaf(a.l, b.h, fmaf(a.h, b.h, -h)))};
 }
 __device__ __forceinline__ float prod_times(Prod p, float x) { return fmaf(p.h, x, p.l * x); }
+// a + b and what its rounding left out
+__device__ __forceinline__ Prod two_sum(float a, float b) {
+  const float s = a + b, bb = s - a;
+  return {s, (a - (s - bb)) + (b - bb)};
+}
 // x / p and 1 / p: the reciprocal instruction and one Newton step
 __device__ __forceinline__ float prod_div(float x, Prod p) {
   const float r = rcp_fast(p.h), t = x * r;

@@ -84,9 +84,8 @@ def test_values_out_of_range_reach_what_the_token_loop_lets_them_reach(where, va
 @pytest.mark.parametrize("mid", [-4.0, 0.0, 4.0])
 @pytest.mark.parametrize("H,D", [(4, 32), (4, 64)])
 def test_errors_are_those_of_the_token_loop(mid, H, D, monkeypatch):
-    """Errors against fp64 beside the token loop's on the same inputs, decays around 0.97, 0.73 and 0.55. A state's terms have as
-    many roundings as in the loop (in another order: a fifth is allowed); an output is the sum of four parts of its size, each
-    rounded, where the loop's has two: its error may be 2^(1/2) times as large (and a tenth for chance)."""
+    """Errors against fp64 beside the token loop's on the same inputs, decays around 0.97, 0.73 and 0.55. State and outputs have as
+    many roundings of their size as in the loop; the order differs, so that either may come out ahead: a tenth is allowed for it."""
     def tweak(x):
         x["w"] += mid
         x["r"] = 0.8 * x["r"] + 0.6 * x["k"]
@@ -101,4 +100,4 @@ def test_errors_are_those_of_the_token_loop(mid, H, D, monkeypatch):
         o, S = reference(t, state[1].to(F64))
         errs.append((error(got, o), error(st[1], S)))
     (o, s), (o0, s0) = errs
-    assert o <= 1.55 * o0 and s <= 1.2 * s0, errs
+    assert o <= 1.1 * o0 and s <= 1.1 * s0, errs

@@ -634,7 +634,7 @@ DECAY_SCALE = math.exp(-0.5)
 DELTA_TWO_PASS = tune.get_bool("delta_two_pass", True)
 UNIT_KEY_EPS = 1e-6
 # prompt portions in chunks of 16 tokens on the fp32 matrix cores (csrc/mixers/delta_chunk.hip); from two chunks on, which take what
-# 32 tokens of the scan take (19.7 against 19.8 us, 32 heads of 64): one takes 17.9 against 14.2, four 23 against 33
+# 32 tokens of the scan take (20.0 against 20.5 us, 32 heads of 64): one takes 18.2 against 18.5, three 21.4 against 25.6
 DELTA_CHUNK_D = (32, 64)
 DELTA_CHUNK_MIN = 32
 
