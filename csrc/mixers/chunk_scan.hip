@@ -10,11 +10,12 @@
 // and a scalar decay (ssm) factors out of the sums: P_ij = C_i . B_j dt_j s_j / s_i, no factor above 1 at all. Everything stays
 // fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32 (operands split into two bf16 terms would lose bits) and the products
 // of decays are carried as two floats (Prod). Referred to the chunk's end, the terms that enter the state have one rounding each,
-// as in the token loop; their reciprocals meet the outputs alone.
-// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets): 64 x 128, 1024 tokens, decays around 0.5
-// 6.1e-8 / 6.6e-8 (6.2e-8 / 6.1e-8), 0.95 3.4e-7 / 1.8e-7 (4.3e-7 / 2.1e-7), 0.999 3.5e-6 / 1.3e-6 (4.1e-6 / 1.5e-6); ssm,
-// 128 x 64, A = -0.6 7.4e-8 / 1.1e-7 (7.6e-8 / 1.2e-7), -1.6 6.9e-8 / 9.4e-8 (6.8e-8 / 1.1e-7). Sums of log2 decays in the place
-// of the products gave 3.3e-7 / 1.1e-7 in the first and 6.4e-7 / 2.7e-7 in the last.
+// as in the token loop; their reciprocals meet the outputs alone, where what came in goes first and the chunk's terms follow in
+// their order (summed apart and added, decays around 0.5 had 1.05 to 1.17 times the loop's error, so 0.97 to 1.10).
+// Error against fp64 (2-norm, carried state / outputs, the token loop's in brackets): 64 x 128, 400 tokens, decays around 0.5
+// 6.0e-8 / 6.1e-8 (6.0e-8 / 6.1e-8), 0.95 3.6e-7 / 1.8e-7 (4.5e-7 / 2.1e-7), 0.999 1.5e-6 / 8.5e-7 (1.8e-6 / 1.0e-6); ssm,
+// 128 x 64, A around -1 7.3e-8 / 1.2e-7 (7.7e-8 / 1.2e-7), -2.7 8.2e-8 / 1.0e-7 (7.6e-8 / 1.1e-7). Sums of log2 decays in the place
+// of the products gave 3.3e-7 / 1.1e-7 in the first.
 //
 // One workgroup = (sequence, head, 16 NW value columns). A wave keeps 16 columns of the state in accumulator layout, which is
 // also the B operand of (q / s) S' when the contraction index runs (tile, register, row quad); v comes straight from memory
@@ -483,11 +484,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 && DK == 64 ? 4 : 2) void chunk_sc
 #pragma unroll
           for (int r = 0; r < 4; ++r) p[r] *= d[r] * x;
         }
-        f32x4_t pv = {0.f, 0.f, 0.f, 0.f};
+        // (what came in, then the chunk's terms in their order: one rounding of the whole)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pv = mfma_f32(4 * r + g4 <= tok_pos(l16) ? p[r] : 0.f, v[r], pv);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] += pv[r];
+        for (int r = 0; r < 4; ++r) acc = mfma_f32(4 * r + g4 <= tok_pos(l16) ? p[r] : 0.f, v[r], acc);
       }
       if (cok) {
 #pragma unroll
