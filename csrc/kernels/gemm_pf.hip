@@ -3,7 +3,7 @@
 //
 //   out[M, N] = x[M, K] . W[N, K]^T        (bf16 in, fp32 accumulate)
 //
-// Replaces the library GEMM of the mixed step (VERDICT r4 "next round" #1): at
+// Replaces the library GEMM of the mixed step: at
 // M ~ 575 the four projections of a Llama-3-8B layer are ~250 GFLOP, compute-
 // bound, so the kernel is built around keeping the matrix pipe busy
 // (cdna_hip_programming.md §5 "The 256² 8-phase template", §5.5 T1-T5):

@@ -19,8 +19,9 @@
 // a share of k: decays around 0.97 3.03e-7 / 1.99e-7 (3.03e-7 / 1.97e-7), 0.73 6.6e-8 / 4.9e-8 (6.6e-8 / 4.9e-8), 0.55 4.7e-8 /
 // 4.3e-8 (4.6e-8 / 4.5e-8); heads of 32 0.92 to 1.03 of the loop's. (Sums of log2 decays and one chain per sum gave 1.8e-7 / 2.3e-7
 // in the second.) That takes: separate sums, because k . r has one sign in a trained model and a chain of 64 rounds at the
-// whole sum's size, and P in two floats (4.9e-8 in the second; 6.1e-8 in one, from half as many chains); what is taken out of the state and of the
-// outputs summed up by itself and before the tokens' own terms, the latest and largest of them last; E in two floats.
+// whole sum's size, and P in two floats (4.9e-8 in the second; 6.1e-8 in one, from half as many chains); what is taken out of the
+// state and of the outputs summed up by itself and before the tokens' own terms, the latest and largest of them last; E in two
+// floats.
 //
 // The second launch has one wave per 16 state columns of a (sequence, head). The first writes every operand in the order of the
 // matrix instructions' lanes; the waves bring it in by LDS DMA, three chunks ahead (in registers, two chunks ahead, the compiler

@@ -280,8 +280,7 @@ class LlamaLayer(nn.Module):
         (half the bytes of the all-reduce) straight into this rank's rows, whose
         post-attention norm feeds the expert dispatch, and the combined expert output
         stays sliced. Per layer: all_gather(h) + reduce_scatter(o) + 2 all_to_all,
-        against all_reduce(o) + 2 all_to_all + all_gather(out) in the replicated form
-        (VERDICT r2 #8)."""
+        against all_reduce(o) + 2 all_to_all + all_gather(out) in the replicated form."""
         eps = self.cfg.norm_eps
         Ts = max(0, min(T, (self.rank + 1) * per) - self.rank * per)
         if residual is None:

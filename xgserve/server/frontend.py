@@ -80,7 +80,7 @@ class _Conn:
     what the kernel takes and leaves the rest to a loop writer callback, so a peer
     that is itself busy writing (both ends flushing batches larger than the socket
     buffer) can never block this loop -- each side keeps reading while its own
-    bytes wait (ADVICE r3: blocking send_bytes on both ends could deadlock)."""
+    bytes wait (blocking send_bytes on both ends could deadlock)."""
 
     READ_CHUNK = 1 << 20
 
