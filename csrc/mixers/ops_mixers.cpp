@@ -62,6 +62,8 @@ int ssm_step(const void*, bool, int64_t, const void*, int64_t, const float*, con
              const int32_t*, const int32_t*, float*, int, int, int, int, int, hipStream_t);
 int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const void*, const float*, const float*, const float*,
                float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
+int tile_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int, int, int, int, int, int, float, float,
+                int, int, int, hipStream_t);
 int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
                 bool, hipStream_t);
 int64_t delta_chunk_scratch_floats(int, int, int, int);
@@ -358,6 +360,12 @@ PYBIND11_MODULE(_mixers, m) {
                           P<const int32_t>(qsl), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<void>(out), ns, H, D,
                           S(st)),
           "delta_step");
+  });
+  m.def("tile_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part, uintptr_t out,
+                          int M, int N, int K, int S_, int act, int pairs, float p0, float p1, int fm, int fn, int cus, uintptr_t st) {
+    check(xgm::tile_linear(P<const void>(x), ld_x, P<const void>(w), P<const void>(bias), bias_f32, P<float>(part), P<void>(out),
+                           M, N, K, S_, act, pairs, p0, p1, fm, fn, cus, S(st)),
+          "tile_linear");
   });
   m.def("rows_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part,
                           uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, bool wide,

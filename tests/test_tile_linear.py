@@ -1,0 +1,87 @@
+"""Products of many rows (csrc/mixers/tile_linear.hip): every tile at its edges, parts of K, what follows the product."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from xgserve.ops import seqmix as sq
+from xgserve.ops import tile_linear as tl
+
+
+def test_plans_fit_the_kernel():
+    for M in (65, 66, 127, 200, 401, 1000, 2601, 8192):
+        for N, K in ((8, 64), (40, 4096), (1088, 2048), (2048, 8192), (28672, 4096), (4096, 14336)):
+            fm, fn, S = tl.tile_plan(M, N, K)
+            assert (fm, fn) in tl._TILES and 1 <= S <= K // 64
+            assert S == 1 or -(-M // (32 * fm)) * -(-N // (32 * fn)) * S <= tl._SPLIT_TILES
+
+
+def test_refused_products_stay_with_torch():
+    x, w = torch.zeros(128, 64, dtype=torch.bfloat16), torch.zeros(256, 64, dtype=torch.bfloat16)
+    assert tl.tile_plan_of(x, w) is None                     # not on the GPU
+    assert torch.equal(sq.linear(x, w), F.linear(x, w))
+    assert tl.library_better(300, 2048, 2048) and tl.library_better(4096, 4096, 4096)
+    assert not tl.library_better(300, 4096, 14336) and not tl.library_better(4001, 10304, 2048)
+
+
+def _close(y, ref, K):
+    # one rounding to bf16 (2^-9 of the value) and fp32 sums of K products: K 2^-24 of the sum of the products' sizes (about
+    # sqrt(K) times a result of unit variance) at most
+    assert torch.isfinite(y.float()).all()
+    err = (y.double() - ref).abs()
+    assert (err <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * K ** 0.5 + 1e-6).all(), float(err.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("M,N,K,S", [(1, 8, 64, 1), (33, 264, 128, 1), (257, 520, 192, 3), (300, 1096, 320, 2), (513, 384, 640, 4)])
+def test_tiles_at_their_edges(tile, M, N, K, S):
+    g = torch.Generator("cuda").manual_seed(M + N)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").to(torch.bfloat16)[:, :K]     # rows with a stride of their own
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device="cuda")
+    ref = x.double() @ w.double().t()
+    for parts in (1, S):
+        plan = (*tile, parts)
+        _close(tl.tile_linear(plan, x, w), ref, K)
+        _close(tl.tile_linear(plan, x, w, b.to(torch.bfloat16)), ref + b.to(torch.bfloat16).double(), K)
+        z = ref + b.double()
+        # the square doubles the sum's relative error and takes its size
+        y = tl.tile_linear(plan, x, w, b, sq.ACT_RELU2).double()
+        assert ((y - z.clamp(min=0) ** 2).abs() <= 2.0 ** -8 * z ** 2 + 2 * z.abs() * K ** 1.5 * 2.0 ** -24 + 1e-6).all()
+        y = tl.tile_linear(plan, x, w, b, sq.ACT_XIELU, 0.7, 0.9).double()
+        r = torch.where(z > 0, 0.7 * z * z, 0.9 * (torch.expm1(z.clamp(max=0)) - z)) + 0.5 * z
+        # (its slope is at most 1.4 z + 0.5 above zero and 1.4 below)
+        assert ((y - r).abs() <= 2.0 ** -8 * r.abs() + (1.4 * z.abs() + 1.4) * (K ** 1.5 * 2.0 ** -24 + 2.0 ** -22) + 1e-6).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("M,F_,K,S", [(1, 8, 64, 1), (70, 132, 128, 2), (270, 528, 192, 3)])
+@pytest.mark.parametrize("kind", [sq.GLU_GELU_TANH, sq.GLU_CLAMPED, sq.GLU_SILU])
+def test_gated_tiles(tile, M, F_, K, S, kind):
+    g = torch.Generator("cuda").manual_seed(M + F_)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(2 * F_, K, generator=g, device="cuda") * 3 * K ** -0.5).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    ref = sq._glu_ref(z[:, :F_], z[:, F_:], kind, 2.0, 1.702)
+    forms = [(w, tl.PAIR_HALVES)]
+    if F_ % 16 == 0:
+        forms.append((torch.stack([w[:F_].view(-1, 16, K), w[F_:].view(-1, 16, K)], 1).reshape(2 * F_, K), tl.PAIR_BLOCKS))
+    for ww, pairs in forms:
+        for parts in (1, S):
+            y = tl.tile_linear((*tile, parts), x, ww, None, sq.ACT_GLU + kind, 2.0, 1.702, pairs).double()
+            # slopes of the gate up to 1.2 and of the other factor 1, each times the other side
+            room = (1.5 * z[:, F_:].abs() + 1.5 * z[:, :F_].abs() + 2) * (3 * K ** 1.5 * 2.0 ** -24 + 2.0 ** -22)
+            assert ((y - ref).abs() <= 2.0 ** -8 * ref.abs() + room).all()
+
+
+@pytest.mark.gpu
+def test_prompt_products_take_the_tiles():
+    x = torch.randn(300, 2048, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(10304, 2048, device="cuda", dtype=torch.bfloat16) * 2048 ** -0.5
+    assert tl.tile_plan_of(x, w, plain=True) is not None and tl.tile_plan_of(x[:64], w) is None
+    assert tl.tile_plan_of(x, torch.nn.Parameter(w)) is None            # a derivative is torch's
+    with torch.no_grad():
+        assert tl.tile_plan_of(x, torch.nn.Parameter(w)) is not None
+    assert tl.tile_plan_of(x.t().contiguous().t(), w) is None and tl.tile_plan_of(x[:, 1:], w[:, 1:]) is None
+    _close(sq.linear(x, w), x.double() @ w.double().t(), 2048)

@@ -17,13 +17,12 @@ from dataclasses import dataclass
 from typing import Optional
 
 import torch
-import torch.autograd.forward_ad as _fwd_ad
 import torch.nn.functional as F
-from torch._C._functorch import is_functorch_wrapped_tensor as _is_transformed
 
 from .. import tune
 from ._native import is_f32, mixers, native_device, stream_ptr
 from .moe import _moe_pf_cfg
+from .tile_linear import PAIR_HALVES, forward_only as _forward_only, tile_linear, tile_plan_of
 
 
 @dataclass
@@ -90,6 +89,11 @@ _ROWS_WGS = 256
 _ROWS_PARTS, _ROWS_PART_K = 8, 512
 _ROWS_TICKETS = _ROWS_WGS // 2     # column tiles of a product in parts
 
+# xIELU behind the product of prompt rows up to here: its 25 instructions an element run on four waves there and on a full chip in a
+# launch of their own (8192 x 2048, us, behind / by itself: 300 rows 20.6 / 24.3, 1000 rows 42.5 / 42.2, 8192 rows 275 / 259). The
+# squared ReLU and the gated activations always go behind (8192 rows: 216 / 253; gated 16384 x 2048, 2521 rows 147 / 193).
+XIELU_BEHIND_MAX = 512
+
 ACT_NONE, ACT_XIELU, ACT_RELU2, ACT_GLU = 0, 1, 2, 3   # ACT_GLU + GLU_...: the gated activations
 
 
@@ -116,19 +120,6 @@ def _rows_plan(N: int, K: int, gated: bool):
     while 2 * S * tiles <= _ROWS_WGS and 2 * S <= _ROWS_PARTS and 2 * S * _ROWS_PART_K <= K:
         S *= 2
     return wide, S
-
-
-def _forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
-    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform, no tracing or dispatch
-    mode, no tensor type of its own. (A product on a kernel of this library has no derivative and no operator to record; torch's
-    has.)"""
-    if _fwd_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing() \
-            or torch.compiler.is_compiling():
-        return False
-    for t in (x, w, bias):
-        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or _is_transformed(t)):
-            return False
-    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))
 
 
 def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool,
@@ -160,13 +151,18 @@ def _rows_linear(plan, x, w, sm, bias, act, p0, p1) -> torch.Tensor:
     return out
 
 
+def _prompt_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    plan = tile_plan_of(x, w, bias, plain=True)
+    return tile_linear(plan, x, w, bias) if plan is not None else F.linear(x, w, bias)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [T, K] . w [N, K]^T + bias."""
     plan = _rows_plan_of(x, w, sm, bias, False) if bias is None or bias.dtype == x.dtype else None
     if plan is not None:
         return _rows_linear(plan, x, w, sm, bias, ACT_NONE, 0.0, 0.0)
-    return F.linear(x, w, bias)
+    return _prompt_linear(x, w, bias) if bias is None or bias.dtype == x.dtype else F.linear(x, w, bias)
 
 
 @dataclass
@@ -197,7 +193,10 @@ def linear_xielu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     plan = _rows_plan_of(x, w, sm, bias, False)
     if plan is not None:
         return _rows_linear(plan, x, w, sm, bias, ACT_XIELU, sp, cn)
-    return xielu(F.linear(x, w), bias, sp, cn)
+    plan = tile_plan_of(x, w, bias) if x.shape[0] <= XIELU_BEHIND_MAX else None
+    if plan is not None:
+        return tile_linear(plan, x, w, bias, ACT_XIELU, sp, cn)
+    return xielu(linear(x, w), bias, sp, cn)
 
 
 def linear_relu2(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -206,6 +205,9 @@ def linear_relu2(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     plan = _rows_plan_of(x, w, sm, bias, False)
     if plan is not None:
         return _rows_linear(plan, x, w, sm, bias, ACT_RELU2, 0.0, 0.0)
+    plan = tile_plan_of(x, w, bias)
+    if plan is not None:
+        return tile_linear(plan, x, w, bias, ACT_RELU2)
     return relu2(F.linear(x, w), bias)
 
 
@@ -215,6 +217,9 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
     plan = _rows_plan_of(x, w, sm, None, True)
     if plan is not None:
         return _rows_linear(plan, x, w, sm, None, ACT_GLU + kind, limit, alpha)
+    plan = tile_plan_of(x, w, None, PAIR_HALVES)
+    if plan is not None:
+        return tile_linear(plan, x, w, None, ACT_GLU + kind, limit, alpha, PAIR_HALVES)
     return glu_act(F.linear(x, w), kind, limit, alpha)
 
 
@@ -592,8 +597,7 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
         M.latent_gather(cache.data_ptr(), bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(),
                         _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(), sm.num_seqs, int(window), lat.shape[1],
                         lat.data_ptr(), koff.data_ptr(), nk, stream_ptr())
-        kn = torch.nn.functional.linear(lat[:, :R], uk)
-        v = torch.nn.functional.linear(lat[:, :R], uv)
+        kn, v = _prompt_linear(lat[:, :R], uk), _prompt_linear(lat[:, :R], uv)
         out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
         M.latent_prompt_attention(q.data_ptr(), dn, dq - dn, dv, kn.data_ptr(), v.data_ptr(), lat.data_ptr(), R,
                                   koff.data_ptr(), gate.data_ptr(), gate.stride(0), rot.data_ptr(), rot_dims,

@@ -1,0 +1,119 @@
+"""Products of many rows (prompt steps) on csrc/mixers/tile_linear.hip: the sizes they run at, and where the library's stay.
+
+`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 1 200 timings on an MI355X (15 weights
+of 768 to 14336 in K and 1088 to 28672 in N, 65 to 8192 rows, cold weights); over these its choice is 1 % slower than the fastest
+of the kernel's forms in the mean and 13 % at most.
+"""
+from __future__ import annotations
+
+import functools
+from typing import Optional
+
+import torch
+import torch.autograd.forward_ad as _fwd_ad
+from torch._C._functorch import is_functorch_wrapped_tensor as _is_transformed
+
+from ._native import is_f32, mixers, native_device, stream_ptr
+from .linear import PendingSum, cu_count
+
+# rows and columns of a workgroup's tile / 32 -> us per 64 of K and per tile
+_TILES = {(8, 8): (1.098, 0.02), (7, 8): (0.995, 0.63), (6, 8): (0.868, 0.86), (4, 8): (0.694, 1.11), (8, 4): (0.667, 1.18),
+          (6, 4): (0.527, 1.55), (4, 4): (0.401, 1.88), (3, 4): (0.331, 1.95), (4, 2): (0.274, 1.23), (3, 2): (0.249, 0.09)}
+_LAUNCH, _SUM = 2.2, 3.7                    # us of the launch, and of the one that adds the parts
+_W_BYTES, _PART_BYTES, _OUT_BYTES = 6.1e6, 2.5e6, 3.0e6   # bytes per us: weights, fp32 parts (there and back), the result
+_OVERLAP = 0.29                             # share of the shorter of products and weight stream that stays visible
+_SPLITS = (1, 2, 3, 4, 6, 8, 12, 16)
+_SPLIT_K, _SPLIT_TILES = 256, 540           # a part's least K; parts of all tiles at most (a bound on the slabs: 2.1 tiles per CU)
+
+PAIR_NONE, PAIR_HALVES, PAIR_BLOCKS = 0, 1, 2   # rows of a gated weight: [gate | up], or 16 gate rows, 16 up rows, ...
+TILE_ROWS_MIN = 65                          # (up to 64 rows the weights are streamed past them: rows_linear)
+
+
+@functools.lru_cache(maxsize=8192)
+def tile_plan(M: int, N: int, K: int, cus: int = 256):
+    """(rows / 32, columns / 32, parts of K) of an [M, K] . [N, K]^T product."""
+    best = None
+    for (fm, fn), (kt, per) in _TILES.items():
+        # measured up to 400 and 2600 rows only: many small tiles read the weights and rows more often than this counts
+        if 32 * fm >= 2 * M + 64 or (fn == 2 and M > 400) or (fm <= 4 and fn == 4 and M > 2600):
+            continue
+        tiles = -(-M // (32 * fm)) * -(-N // (32 * fn))
+        for S in _SPLITS:
+            if S > 1 and (K // S < _SPLIT_K or tiles * S > _SPLIT_TILES):
+                break
+            work = -(-tiles * S // cus) * (-(-(K // 64) // S) * kt + per)
+            load = 2 * N * K / _W_BYTES
+            t = _LAUNCH + max(work, load) + _OVERLAP * min(work, load)
+            t += _SUM + 4 * M * N * S / _PART_BYTES if S > 1 else 2 * M * N / _OUT_BYTES
+            if best is None or t < best[0]:
+                best = (t, fm, fn, S)
+    return best[1:]
+
+
+def library_better(M: int, N: int, K: int) -> bool:
+    """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel).
+
+    Small: narrow products below 3.3 G multiply-adds start fewer workgroups than there are compute units (2048x2048, 512 rows 11.5
+    against 15.2; 1088x2048, 700 rows 11.4 against 16.4; beyond the line 2048x2048, 1536 rows 18.8 against 16.6). Long: both run at
+    the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
+    4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81; up to 1792 rows 4096x14336, 1536 rows 168 against 140;
+    6144x4096, 700 rows 45 against 41), as long as no columns are left over beside its tiles of 256 (10304x2048, 4001 rows 168 against
+    129; 18560x4096, 2048 rows 344 against 257)."""
+    if N <= 3072 and K >= 1024 and M * N * K < 3.3e9:
+        return True
+    return N % 256 == 0 and M > 1792
+
+
+def forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform, no tracing or dispatch
+    mode, no tensor type of its own. (A product on a kernel of this library has no derivative and no operator to record; torch's
+    has.)"""
+    if _fwd_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing() \
+            or torch.compiler.is_compiling():
+        return False
+    for t in (x, w, bias):
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or _is_transformed(t)):
+            return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))
+
+
+def tile_plan_of(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, pairs: int = PAIR_NONE,
+                 plain: bool = False):
+    """The plan of x . w^T on the tile kernel, or None: bfloat16 on one device, more than 64 rows of whole 16-byte pieces, K in
+    whole steps of 64, whole groups of columns, nothing that wants a derivative; `plain` products only where the library's is not
+    faster. What is refused here goes to torch, which refuses what it cannot do."""
+    if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and w.device == x.device and w.dim() == 2 and x.shape[0] >= TILE_ROWS_MIN and forward_only(x, w, bias)):
+        return None
+    (M, ldk), (N, K) = x.shape, w.shape
+    if ldk != K or K < 64 or K % 64 or N < 8 or N % (32 if pairs == PAIR_BLOCKS else 8) or not w.is_contiguous() or \
+            x.stride(1) != 1 or x.stride(0) < K or x.stride(0) % 8 or (x.data_ptr() | w.data_ptr()) % 16:
+        return None
+    # (a lane's offsets are 32 bits: of the whole weight, and of a tile's rows; tiles are counted in an int)
+    if 2 * N * K >= 1 << 32 or 512 * x.stride(0) >= 1 << 32 or M * N >= 1 << 40:
+        return None
+    if bias is not None and not (pairs == PAIR_NONE and bias.device == x.device and bias.dtype in (torch.float32, torch.bfloat16)
+                                 and bias.shape == (N,) and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+        return None
+    return None if plain and library_better(M, N, K) else tile_plan(M, N, K, cu_count(x.device))
+
+
+def tile_linear(plan, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = 0, p0: float = 0.0,
+                p1: float = 0.0, pairs: int = PAIR_NONE) -> torch.Tensor:
+    """act(x . w^T + bias) on `plan` (`tile_plan_of`); act: ops.seqmix's ACT_..., gated ones with `pairs`."""
+    M, (N, K), (fm, fn, S) = x.shape[0], w.shape, plan
+    out = torch.empty(M, N // 2 if pairs else N, dtype=x.dtype, device=x.device)
+    part = torch.empty(S * M * N, dtype=torch.float32, device=x.device) if S > 1 else None
+    mixers().tile_linear(x.data_ptr(), x.stride(0), w.data_ptr(), 0 if bias is None else bias.data_ptr(),
+                         bias is not None and is_f32(bias), 0 if part is None else part.data_ptr(), out.data_ptr(), M, N, K, S, act,
+                         pairs, float(p0), float(p1), fm, fn, cu_count(x.device), stream_ptr())
+    return out
+
+
+def tile_parts(plan, x: torch.Tensor, w: torch.Tensor) -> PendingSum:
+    """x . w^T on a `plan` with K in parts, which the next kernel adds."""
+    M, (N, K), (fm, fn, S) = x.shape[0], w.shape, plan
+    part = torch.empty(S, M, N, dtype=torch.float32, device=x.device)
+    mixers().tile_linear(x.data_ptr(), x.stride(0), w.data_ptr(), 0, False, part.data_ptr(), 0, M, N, K, S, 0, PAIR_NONE, 0.0, 0.0,
+                         fm, fn, cu_count(x.device), stream_ptr())
+    return PendingSum(part, S)
