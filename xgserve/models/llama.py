@@ -40,6 +40,8 @@ from ..ops.linear import (MODE_PARTIAL, MODE_SILU, MW_MAX_M, W8_MAX_M, W8_MIN_EL
                           mw_linear, mw_plan, pf_linear, pf_plan, pick_split,
                           quantize_fp8, quantize_weight, skinny_linear, splitk_linear, splitk_prefill_ok, w8_linear,
                           w8_plan, WQ_FORMATS)
+from ..ops.seqmix import ACT_GLU, GLU_SILU
+from ..ops.tile_linear import PAIR_BLOCKS, tile_linear, tile_parts, tile_plan_of
 from .base import AttnMeta, PagedAttention, init_weight, kv_head_range, local_heads, shard
 from .config import ModelConfig
 
@@ -67,9 +69,9 @@ MW_MAX_TOKENS = min(MW_MAX_M, tune.get_int("mw_max_tokens", MW_MAX_M))
 # tuned library GEMM (profiles/r6/r6p_pf_vs_library.md, cold weights, the engine's
 # library forms) -- QKV / O / down as split-K partials into their consumers, gate_up
 # with the SiLU gate in its epilogue:
-#   gate_up 448-576 rows: 4-5 % ahead of the library's GEMM + SiLU-gate pair at 448 / 512
-#     rows, 22 % at 575 -- its tile-quantisation cliff (GEMM 103 us at 512 rows, 135 at
-#     575), where two 288-row tiles cover the step; within +-1 % or behind elsewhere;
+#   gate_up 513-576 rows: two 288-row tiles cover the step (121 us at 575 rows, where two
+#     rounds of the 192-row tiles of ops.tile_linear take 138); up to 512 rows two 256-row
+#     tiles of that kernel do (104 us against 109 here);
 #   down 513-576 rows: 5-11 % ahead of the library's split-4 GEMM in isolation at every
 #     measured size from 320 to 576 rows, but its 8 fp32 slabs (vs the library's 4) cost
 #     the consumer more than that below 513: 447-row steps (--prompt-len 384) ran 11,603
@@ -78,7 +80,7 @@ MW_MAX_TOKENS = min(MW_MAX_M, tune.get_int("mw_max_tokens", MW_MAX_M))
 #     to their consumers (r5: -0.5 % end to end with every projection on pf).
 # XGS_TUNE pf: "1" = these windows, "0" = library everywhere, or a comma list of
 # projections to allow; pf_windows overrides the table ("gate_up:513-576/down:321-576").
-PF_WINDOWS_DEFAULT = "gate_up:448-576/down:513-576"
+PF_WINDOWS_DEFAULT = "gate_up:513-576/down:513-576"
 
 
 def _parse_pf_windows(spec: str):
@@ -102,6 +104,22 @@ PF_MAX_M = max([hi for ws in PF_WINDOWS.values() for _, hi in ws] or [0])
 def pf_projections(T: int) -> frozenset:
     """The projections that run on gemm_pf at a T-token step."""
     return frozenset(k for k, ws in PF_WINDOWS.items() if any(lo <= T <= hi for lo, hi in ws))
+
+
+def _product(x: torch.Tensor, w: torch.Tensor, parts: bool = False):
+    """x . w^T of a prompt-sized step, on the tile kernel or the library's; parts: a PendingSum where K is in parts."""
+    plan = tile_plan_of(x, w, plain=True)
+    if plan is None:
+        return F.linear(x, w)
+    return tile_parts(plan, x, w) if parts and plan[2] > 1 else tile_linear(plan, x, w)
+
+
+def _silu_gate(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of a block-16 interleaved gate|up weight."""
+    plan = tile_plan_of(x, w, None, PAIR_BLOCKS)
+    if plan is None:
+        return ops.silu_and_mul(F.linear(x, w), interleave16=True)
+    return tile_linear(plan, x, w, None, ACT_GLU + GLU_SILU, pairs=PAIR_BLOCKS)
 
 
 # TP > 1 prefill-sized steps: the row-parallel all-reduces are pipelined over this
@@ -320,11 +338,20 @@ class LlamaLayer(nn.Module):
             if self.tp > 1 and self._moe_use_alltoall(h):
                 return self._moe_alltoall(h)
             return self._moe_allreduce(h)
-        gu = F.linear(h, self.gate_up)
-        a = ops.silu_and_mul(gu, interleave16=True)
-        if self.tp == 1 and splitk_prefill_ok(a, self.down):
-            return splitk_linear(a, self.down, linear_mod.SPLITK_PREFILL_S)  # reduced by the next add + norm
-        return self._ar(F.linear(a, self.down))
+        a = _silu_gate(h, self.gate_up)
+        if self.tp > 1:
+            return self._ar(_product(a, self.down))
+        return self._down(a)
+
+    def _down(self, a: torch.Tensor):
+        """The down projection of a prompt-sized step on one GPU; parts of K are added by the next add + norm."""
+        if tile_plan_of(a, self.down, plain=True) is None and splitk_prefill_ok(a, self.down):
+            return splitk_linear(a, self.down, linear_mod.SPLITK_PREFILL_S)
+        return _product(a, self.down, parts=True)
+
+    def _attend_prompt(self, h: torch.Tensor, meta: AttnMeta, kv, cos_sin) -> torch.Tensor:
+        qkv = _product(h, self.qkv, parts=True)
+        return (self.attn.from_partials if isinstance(qkv, linear_mod.PendingSum) else self.attn)(qkv, meta, kv, cos_sin)
 
     def _row_parallel_fast(self, a: torch.Tensor, w: torch.Tensor, split: int):
         pend = skinny_linear(a, w, None, MODE_PARTIAL)
@@ -409,20 +436,18 @@ class LlamaLayer(nn.Module):
             if "qkv" in use_pf:
                 a = self.attn.from_partials(pf_linear(h, self.qkv, MODE_PARTIAL), meta, kv, cos_sin)
             else:
-                a = self.attn(F.linear(h, self.qkv), meta, kv, cos_sin)
-            o = pf_linear(a, self.o, MODE_PARTIAL) if "o" in use_pf else F.linear(a, self.o)
+                a = self._attend_prompt(h, meta, kv, cos_sin)
+            o = pf_linear(a, self.o, MODE_PARTIAL) if "o" in use_pf else _product(a, self.o, parts=True)
             h, residual = ops.fused_add_rmsnorm(o, residual, self.post_norm, eps)
             if self.moe:
                 return self.mlp(h), residual
             if "gate_up" in use_pf:
                 act = pf_linear(h, self.gate_up, MODE_SILU)
             else:
-                act = ops.silu_and_mul(F.linear(h, self.gate_up), interleave16=True)
+                act = _silu_gate(h, self.gate_up)
             if "down" in use_pf:
                 return pf_linear(act, self.down, MODE_PARTIAL), residual
-            if splitk_prefill_ok(act, self.down):
-                return splitk_linear(act, self.down, linear_mod.SPLITK_PREFILL_S), residual
-            return F.linear(act, self.down), residual
+            return self._down(act), residual
         if self.fast_ok and T <= FAST_M_SLAB:
             # 16 < M <= 64: measured per shape on MI355X -- only the O projection
             # (N = H) is faster on the LDS-slab kernel; its split-K partials are
@@ -432,10 +457,10 @@ class LlamaLayer(nn.Module):
             o = self._row_parallel_fast(a, self.o, self.split_o)
             h, residual = ops.fused_add_rmsnorm(o, residual, self.post_norm, eps)
             return self.mlp(h), residual
-        a = self.attn(F.linear(h, self.qkv), meta, kv, cos_sin)
+        a = self._attend_prompt(h, meta, kv, cos_sin)
         if self.tp > 1 and not self.moe and T >= TP_OVERLAP_MIN_TOKENS and TP_OVERLAP_CHUNKS > 1:
             return self._forward_tp_overlap(a, residual)
-        o = self._ar(F.linear(a, self.o))
+        o = _product(a, self.o, parts=True) if self.tp == 1 else self._ar(_product(a, self.o))
         h, residual = ops.fused_add_rmsnorm(o, residual, self.post_norm, eps)
         return self.mlp(h), residual
 
