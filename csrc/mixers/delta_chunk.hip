@@ -23,16 +23,17 @@
 // state and of the outputs summed up by itself and before the tokens' own terms, the latest and largest of them last; E in two
 // floats.
 //
-// The second launch has one wave per 16 state columns of a (sequence, head). The first writes every operand in the order of the
-// matrix instructions' lanes; the waves bring it in by LDS DMA, three chunks ahead (in registers, two chunks ahead, the compiler
-// parks operands in accumulator registers, which waits for every load: 2.1 us a chunk). A chunk with an input out of range
-// (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
+// The second launch has two waves per 16 state columns of a (sequence, head), one for the even and one for the odd 16s of the state's
+// rows, which are the two chains that y and the outputs are summed in anyway: they hand each other y (and the outputs' sums) through
+// LDS at the one barrier of a chunk, so each has half of the matrix instructions. A workgroup takes 32 columns, so a head of 64 has
+// two and 32 heads of 4 sequences fill the chip. The first launch writes every operand in the order of the matrix instructions' lanes;
+// the waves bring it in by LDS DMA, five chunks ahead, and read a chunk's operands while the one before it still adds to the state.
+// A chunk with an input out of range (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
 //
-// Measured, bf16 rows, both launches: 4 x 2048 tokens of 32 heads of 64 1019 -> 380 us (172 + 258 in a step's trace), one sequence of
-// 2048 838 -> 273, 64 tokens 32 -> 23 (log sums in single chains: 325, 236, 21). The first launch writes 24.6 KB per chunk and head
-// and forms three exponentials per token and channel; the second takes 1.9 us a chunk, 0.9 of them its 64 matrix instructions a
-// wave, the rest the way from one to the next: LDS reads behind the barrier, and y, which has to be complete before it goes back
-// in. (E S is formed behind y's products: in front of them it cost 8 us of 280. k' v behind y instead of beside it: 380 against 394.)
+// Measured, bf16 rows, 4 x 2048 tokens of 32 heads of 64 in a step: the first launch 162 us (it writes 24.6 KB per chunk and head and
+// forms three exponentials per token and channel), the second 169, 1.3 us a chunk (one wave per 16 columns 238 to 258; two, operands
+// read at a chunk's head 184, loads behind the barrier instead of between y's products 173). What is left of a chunk is the way from
+// one matrix instruction to the next, 0.45 us of it the instructions: with every load from the same 25 KB it takes as long.
 #include "glds.h"
 #include "mfma_f32.h"
 
@@ -262,143 +263,214 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
 }
 
 template <typename T, int D>
-__global__ __launch_bounds__(4 * D, 1) void delta_chunk_scan_kernel(const float* __restrict__ prep, const T* __restrict__ proj,
-                                                                    int64_t ld, int off_v, float* __restrict__ state,
-                                                                    const int32_t* __restrict__ qsl,
-                                                                    const int32_t* __restrict__ seq_lens,
-                                                                    const int32_t* __restrict__ slots, float* __restrict__ o,
-                                                                    int H) {
-  constexpr int C = kDcTok, MT = D / 16, NW = MT, RING = 4;
-  constexpr int FRAG = 6 * C * D * 4, SLOT = FRAG + 1024 + C * D * sizeof(T);   // bytes: [U .. O | E, flag | v rows]
-  constexpr int VL = D * sizeof(T) / 16, VR = C / NW;                            // lanes per v row, v rows per wave
-  constexpr int DMA = 6 * C * D * 4 / 1024 / NW + 2;                             // loads per wave and chunk
-  __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT];
-  const int h = blockIdx.x, s = blockIdx.y;
+__global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(const float* __restrict__ prep, const T* __restrict__ proj,
+                                                                  int64_t ld, int off_v, float* __restrict__ state,
+                                                                  const int32_t* __restrict__ qsl,
+                                                                  const int32_t* __restrict__ seq_lens,
+                                                                  const int32_t* __restrict__ slots, float* __restrict__ o,
+                                                                  int H) {
+  constexpr int C = kDcTok, MT = D / 16, MH = MT / 2, RING = 6;
+  constexpr int OPS = 4 * C * D * 4, VO = 2 * C * 32 * 4, FRAG = OPS + VO;   // bytes: [U | R | k' | -b'], this half's [V | O]
+  constexpr int VROWS = C * 32 * sizeof(T), SLOT = FRAG + 1024 + VROWS;      // ... [E, flag | v rows]
+  constexpr int PIECES = FRAG / 1024 / 4, VD = VROWS / 1024, DMA = PIECES + 1 + VD;   // loads per wave and chunk
+  constexpr int kEx = 2 * (4 + 2) * 1024;                                    // handed over: y of four waves, outputs of two
+  constexpr int VL = 32 * sizeof(T) / 16;                                    // lanes per v row
+  static_assert(RING * SLOT + kEx <= 160 * 1024 && (RING - 2) * DMA < 64, "delta_chunk_scan geometry");
+  __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT + kEx];
+  const int h = blockIdx.x, s = blockIdx.y, half = blockIdx.z;
   const int q0 = qsl[s], qn = qsl[s + 1] - q0, slot = slots[s];
   if (slot < 0 || qn <= 0) return;
   const int ctx = seq_lens[s] - qn;
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = 16 * w + l16;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ct = w >> 1, par = w & 1;
+  const int col = 32 * half + 16 * ct + l16;
   float* Sg = state + ((int64_t)slot * H + h) * D * D + col;
-  f32x4_t S[MT];
+  f32x4_t S[MH];   // rows 16 (2 i + par) ..
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int i = 0; i < MH; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[m][r] = ctx > 0 ? Sg[(16 * m + 4 * g4 + r) * D] : 0.f;
+    for (int r = 0; r < 4; ++r) S[i][r] = ctx > 0 ? Sg[(16 * (2 * i + par) + 4 * g4 + r) * D] : 0.f;
   const int nch = (qn + C - 1) / C;
   const float* base = prep + ((int64_t)(q0 / C + s) * H + h) * dc_stride(D);
   const int64_t step = (int64_t)H * dc_stride(D);
-  const T* vb = proj + (int64_t)q0 * ld + off_v + h * D;
-  const int vrow = VR * w + lane / VL;   // (lanes past the wave's rows load nothing)
+  const T* vb = proj + (int64_t)q0 * ld + off_v + h * D + 32 * half;
 
-  auto issue = [&](int c) {   // every wave issues DMA loads, past the last chunk too (its waits count them)
+  // every wave issues DMA loads, past the last chunk too (its waits count them): i-th of DMA of chunk c
+  const T* vrow = vb + (lane % VL) * (16 / sizeof(T));
+  auto issue1 = [&](int c, int i) __attribute__((always_inline)) {
     char* dst = lds + (c % RING) * SLOT;
-    const char* src = reinterpret_cast<const char*>(base + min(c, nch - 1) * step) + 16 * lane;
+    const int cc = min(c, nch - 1);
+    const char* src = reinterpret_cast<const char*>(base + cc * step) + 16 * lane;
+    if (i < PIECES) {
+      const int pc = PIECES * w + i, vo = pc - OPS / 1024;   // (V and O: two of their MT kilobytes each)
+      const int from = vo < 0 ? pc : OPS / 1024 + (vo >> 1) * MT + 2 * half + (vo & 1);
+      xgk::glds16(src + 1024 * from, dst + 1024 * pc);
+    } else if (i == PIECES) {
+      xgk::glds16(src + 6 * C * D * 4, dst + FRAG);   // (the same bytes from every wave, and so the v rows)
+    } else {
+      const int j = i - PIECES - 1;
+      xgk::glds16(vrow + (int64_t)min(C * cc + j * (64 / VL) + lane / VL, qn - 1) * ld, dst + FRAG + 1024 + 1024 * j);
+    }
+  };
+  auto issue = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < DMA - 2; ++i) xgk::glds16(src + 1024 * (NW * i + w), dst + 1024 * (NW * i + w));
-    xgk::glds16(src + FRAG, dst + FRAG);   // (the same bytes from every wave)
-    if (lane < VR * VL)
-      xgk::glds16(vb + (int64_t)min(C * min(c, nch - 1) + vrow, qn - 1) * ld + (lane % VL) * (16 / sizeof(T)),
-                  dst + FRAG + 1024 + VR * w * D * sizeof(T));
+    for (int i = 0; i < DMA; ++i) issue1(c, i);
   };
   for (int c = 0; c < RING - 1; ++c) issue(c);
-  for (int c = 0; c < nch; ++c) {
-    // this chunk's loads have landed (those of the chunks after it are in flight), in every wave; the slot of the chunk
-    // before is free
-    xgk::wait_vmcnt<(RING - 2) * DMA>();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    xgk::raw_barrier();
-    issue(c + RING - 1);
+#pragma unroll
+  for (int i = 0; i < MH; ++i) asm volatile("" : "+v"(S[i]));   // (the state is here: its loads are not waited for inside the loop)
+  xgk::wait_vmcnt<(RING - 2) * DMA>();
+  xgk::raw_barrier();
+  // A chunk's operands in registers: read while the chunk before it still adds to the state, so that the first product waits for
+  // nothing (18 reads of four waves at the head of a chunk were 0.3 us of it).
+  struct Ops {
+    float4 u[MH], r[MH], k[MH], b[MH], e[MH], el[MH], v0, o0;
+    T v[4];
+    float flag;
+  };
+  auto load = [&](int c, Ops& x) __attribute__((always_inline)) {
     const char* at = lds + (c % RING) * SLOT;
-    const float* p = reinterpret_cast<const float*>(at);
     const float4* p4 = reinterpret_cast<const float4*>(at) + lane;
     const float* pe = reinterpret_cast<const float*>(at + FRAG);
-    const T* pv = reinterpret_cast<const T*>(at + FRAG + 1024) + col;
+    const T* pv = reinterpret_cast<const T*>(at + FRAG + 1024) + 16 * ct + l16;
+#pragma unroll
+    for (int i = 0; i < MH; ++i) x.u[i] = p4[64 * (2 * i + par)];
+#pragma unroll
+    for (int i = 0; i < MH; ++i) x.r[i] = p4[64 * (MT + 2 * i + par)];
+#pragma unroll
+    for (int i = 0; i < MH; ++i) {
+      const int m = 2 * i + par;
+      x.e[i] = *reinterpret_cast<const float4*>(pe + 16 * m + 4 * g4);
+      x.el[i] = *reinterpret_cast<const float4*>(pe + 2 * D + 16 * m + 4 * g4);
+      x.k[i] = p4[64 * (2 * MT + m)], x.b[i] = p4[64 * (3 * MT + m)];
+    }
+    x.v0 = p4[64 * (4 * MT + ct)], x.o0 = p4[64 * (4 * MT + 2 + ct)];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x.v[t] = pv[(4 * t + g4) * 32];
+    x.flag = pe[D];
+  };
+  auto chunk = [&](int c, Ops& x, Ops& next) __attribute__((always_inline)) {
     const int n = min(C, qn - C * c);
     float* ob = o + ((int64_t)(q0 + C * c) * H + h) * D + col;
-    float v[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = ldf(pv + (4 * t + g4) * D);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = 4 * t + g4 < n ? v[t] : 0.f;
-    if (__builtin_amdgcn_readfirstlane(pe[D] != 0.f)) {
+    // what the two waves of a column tile hand each other, two buffers in turn: y, and the outputs' sums
+    float4* ex = reinterpret_cast<float4*>(lds + RING * SLOT + (c & 1) * (kEx / 2)) + lane;
+    float4* exo = ex + 256;
+    auto meet = [&]() __attribute__((always_inline)) {   // the next chunk has landed, in every wave
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      xgk::wait_vmcnt<(RING - 2) * DMA>();
+      xgk::raw_barrier();
+    };
+    if (__builtin_amdgcn_readfirstlane(x.flag != 0.f)) {
+      const float* p = reinterpret_cast<const float*>(lds + (c % RING) * SLOT);
+      __syncthreads();   // (what the chunk before handed over has been read)
+      float* xs = reinterpret_cast<float*>(lds + RING * SLOT);   // [wave][lane], sums into the state, then the outputs'
+      const float* rr0 = base + c * step + 4 * C * D;            // (r lies where V would: only half of that is in LDS)
+      const T* pv = reinterpret_cast<const T*>(lds + (c % RING) * SLOT + FRAG + 1024) + 16 * ct + l16;
       for (int t = 0; t < n; ++t) {
-        const float vv = ldf(pv + t * D);
+        const float vv = ldf(pv + t * 32);
         float uS = 0.f, sum = 0.f;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
+        for (int i = 0; i < MH; ++i) {
           float u[4];
-          ld4(p + 2 * C * D + t * D + 16 * m + 4 * g4, u);
+          ld4(p + 2 * C * D + t * D + 16 * (2 * i + par) + 4 * g4, u);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) uS = fmaf(u[r], S[m][r], uS);
+          for (int r = 0; r < 4; ++r) uS = fmaf(u[r], S[i][r], uS);
         }
         uS += __shfl_xor(uS, 16, 64);
         uS += __shfl_xor(uS, 32, 64);
+        xs[64 * w + lane] = uS;
+        __syncthreads();
+        uS += xs[64 * (w ^ 1) + lane];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
+        for (int i = 0; i < MH; ++i) {
           float wr[4], b[4], k[4], rr[4];
-          const float* x = p + t * D + 16 * m + 4 * g4;
-          ld4(x, wr), ld4(x + C * D, b), ld4(x + 3 * C * D, k), ld4(x + 4 * C * D, rr);
+          const int ch = t * D + 16 * (2 * i + par) + 4 * g4;
+          ld4(p + ch, wr), ld4(p + ch + C * D, b), ld4(p + ch + 3 * C * D, k), ld4(rr0 + ch, rr);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            S[m][r] = wr[r] * S[m][r] - b[r] * uS + k[r] * vv;
-            sum = fmaf(S[m][r], rr[r], sum);
+            S[i][r] = wr[r] * S[i][r] - b[r] * uS + k[r] * vv;
+            sum = fmaf(S[i][r], rr[r], sum);
           }
         }
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
-        if (g4 == 0) ob[(int64_t)t * H * D] = sum;
+        xs[256 + 64 * w + lane] = sum;
+        __syncthreads();
+        sum += xs[256 + 64 * (w ^ 1) + lane];
+        if (par == 0 && g4 == 0) ob[(int64_t)t * H * D] = sum;
       }
-      continue;
+      issue(c + RING - 1);
+      meet();
+      load(c + 1, next);
+      return;
     }
-    const float4 v0 = p4[64 * (4 * MT + w)], o0 = p4[64 * (5 * MT + w)];
-    float4 k[MT], b[MT];
-    float e[MT][4], el[MT][4];
-    f32x4_t yc[2], oc[2];   // two chains each: even and odd 16s of the state's rows
-    yc[0] = yc[1] = oc[0] = oc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // one chain each over this wave's 16s of the state's rows (the even ones, or the odd ones)
+    // (between its products the loads of the chunk RING - 1 on, into the slot of the chunk before, which every wave is past)
+    f32x4_t yc = {0.f, 0.f, 0.f, 0.f}, oc = yc;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const float4 u = p4[64 * m], r = p4[64 * (MT + m)];
-      k[m] = p4[64 * (2 * MT + m)], b[m] = p4[64 * (3 * MT + m)], ld4(pe + 16 * m + 4 * g4, e[m]), ld4(pe + 2 * D + 16 * m + 4 * g4, el[m]);
-      yc[m % 2] = mfma_f32(u.x, S[m][0], yc[m % 2]), oc[m % 2] = mfma_f32(r.x, S[m][0], oc[m % 2]);
-      yc[m % 2] = mfma_f32(u.y, S[m][1], yc[m % 2]), oc[m % 2] = mfma_f32(r.y, S[m][1], oc[m % 2]);
-      yc[m % 2] = mfma_f32(u.z, S[m][2], yc[m % 2]), oc[m % 2] = mfma_f32(r.z, S[m][2], oc[m % 2]);
-      yc[m % 2] = mfma_f32(u.w, S[m][3], yc[m % 2]), oc[m % 2] = mfma_f32(r.w, S[m][3], oc[m % 2]);
+    for (int q = 0; q < 4 * MH; ++q) {
+      const float4 u = x.u[q / 4];
+      yc = mfma_f32(q % 4 == 0 ? u.x : q % 4 == 1 ? u.y : q % 4 == 2 ? u.z : u.w, S[q / 4][q % 4], yc);
+#pragma unroll
+      for (int i = q * DMA / (4 * MH); i < (q + 1) * DMA / (4 * MH); ++i) issue1(c + RING - 1, i);
     }
-    // E S behind y's last products; then what is taken out, summed up by itself, then the tokens' terms in their order
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int i = 0; i < MH; ++i) {
+      oc = mfma_f32(x.r[i].x, S[i][0], oc), oc = mfma_f32(x.r[i].y, S[i][1], oc);
+      oc = mfma_f32(x.r[i].z, S[i][2], oc), oc = mfma_f32(x.r[i].w, S[i][3], oc);
+    }
+    ex[64 * w] = make_float4(yc[0], yc[1], yc[2], yc[3]);
+    // E S behind the products with S; then what is taken out, summed up by itself, then the tokens' terms in their order
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[m][r] = prod_times({e[m][r], el[m][r]}, S[m][r]);
-    const float y[4] = {yc[0][0] + yc[1][0] + v0.x, yc[0][1] + yc[1][1] + v0.y, yc[0][2] + yc[1][2] + v0.z, yc[0][3] + yc[1][3] + v0.w};
-    f32x4_t by[MT];
+    for (int i = 0; i < MH; ++i) {
+      S[i][0] = prod_times({x.e[i].x, x.el[i].x}, S[i][0]), S[i][1] = prod_times({x.e[i].y, x.el[i].y}, S[i][1]);
+      S[i][2] = prod_times({x.e[i].z, x.el[i].z}, S[i][2]), S[i][3] = prod_times({x.e[i].w, x.el[i].w}, S[i][3]);
+    }
+    if (par) exo[64 * ct] = make_float4(oc[0], oc[1], oc[2], oc[3]);
+    float v[4];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].x, y[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
+    for (int t = 0; t < 4; ++t) v[t] = ldf(&x.v[t]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].y, y[1], by[m]);
+    for (int t = 0; t < 4; ++t) v[t] = 4 * t + g4 < n ? v[t] : 0.f;
+    meet();
+    const float4 yo = ex[64 * (w ^ 1)], oo = exo[64 * ct];
+    load(c + 1, next);
+    const float y[4] = {yc[0] + yo.x + x.v0.x, yc[1] + yo.y + x.v0.y, yc[2] + yo.z + x.v0.z, yc[3] + yo.w + x.v0.w};
+    f32x4_t by[MH];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].z, y[2], by[m]);
+    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].x, y[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int m = 0; m < MT; ++m) by[m] = mfma_f32(b[m].w, y[3], by[m]);
+    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].y, y[1], by[i]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].x, v[0], S[m] + by[m]);
+    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].z, y[2], by[i]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].y, v[1], S[m]);
+    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].w, y[3], by[i]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].z, v[2], S[m]);
+    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].x, v[0], S[i] + by[i]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_f32(k[m].w, v[3], S[m]);
-    const float out[4] = {oc[0][0] + oc[1][0] + o0.x, oc[0][1] + oc[1][1] + o0.y, oc[0][2] + oc[1][2] + o0.z,
-                          oc[0][3] + oc[1][3] + o0.w};
+    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].y, v[1], S[i]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (4 * r + g4 < n) ob[(int64_t)(4 * r + g4) * H * D] = out[r];
+    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].z, v[2], S[i]);
+#pragma unroll
+    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].w, v[3], S[i]);
+    if (par == 0) {
+      const float out[4] = {oc[0] + oo.x + x.o0.x, oc[1] + oo.y + x.o0.y, oc[2] + oo.z + x.o0.z, oc[3] + oo.w + x.o0.w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * r + g4 < n) ob[(int64_t)(4 * r + g4) * H * D] = out[r];
+    }
+  };
+  Ops x0, x1;
+  load(0, x0);
+  for (int c = 0; c < nch; c += 2) {
+    chunk(c, x0, x1);
+    if (c + 1 < nch) chunk(c + 1, x1, x0);
   }
   xgk::wait_vmcnt<0>();   // (no load may land after the workgroup's LDS is given on)
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int i = 0; i < MH; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Sg[(16 * m + 4 * g4 + r) * D] = S[m][r];
+    for (int r = 0; r < 4; ++r) Sg[(16 * (2 * i + par) + 4 * g4 + r) * D] = S[i][r];
 }
 
 // ================================================================== host launchers
@@ -418,7 +490,7 @@ int delta_chunk(const void* proj, bool f32, int64_t ld, int off_r, int off_k, in
   XGM_DISPATCH_T(f32, delta_chunk_prep_kernel<T, D><<<dim3(H, nc, ns), 64, 0, st>>>((const T*)proj, ld, off_r, off_k, off_v, \
                                                                                     off_a, (const T*)wl, ld_wl, a_bias, w0, \
                                                                                     qsl, slots, scratch, H);                \
-                 delta_chunk_scan_kernel<T, D><<<dim3(H, ns), 4 * D, 0, st>>>(scratch, (const T*)proj, ld, off_v, state, qsl, \
+                 delta_chunk_scan_kernel<T, D><<<dim3(H, ns, D / 32), 256, 0, st>>>(scratch, (const T*)proj, ld, off_v, state, qsl, \
                                                                               seq_lens, slots, o, H);)                       \
   return 0;
   if (D == 32) { XGM_DC(32) }
