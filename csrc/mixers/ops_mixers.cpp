@@ -64,6 +64,8 @@ int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const vo
                float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
 int tile_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int, int, int, int, int, int, float, float,
                 int, int, int, hipStream_t);
+int tile_grouped(const void*, int64_t, int, const int32_t*, const int32_t*, int, int, const void*, float*, void*, int, int, int, int, float,
+                 float, int, int, int, hipStream_t);
 int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
                 bool, hipStream_t);
 int64_t delta_chunk_scratch_floats(int, int, int, int);
@@ -366,6 +368,13 @@ PYBIND11_MODULE(_mixers, m) {
     check(xgm::tile_linear(P<const void>(x), ld_x, P<const void>(w), P<const void>(bias), bias_f32, P<float>(part), P<void>(out),
                            M, N, K, S_, act, pairs, p0, p1, fm, fn, cus, S(st)),
           "tile_linear");
+  });
+  m.def("tile_grouped", [](uintptr_t x, int64_t ld_x, int x_rows, uintptr_t rows, uintptr_t offs, int E, int top, uintptr_t w,
+                           uintptr_t y, uintptr_t out, int M, int N, int K, int act, float p0, float p1, int fm, int fn, int cus,
+                           uintptr_t st) {
+    check(xgm::tile_grouped(P<const void>(x), ld_x, x_rows, P<const int32_t>(rows), P<const int32_t>(offs), E, top, P<const void>(w),
+                            P<float>(y), P<void>(out), M, N, K, act, p0, p1, fm, fn, cus, S(st)),
+          "tile_grouped");
   });
   m.def("rows_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part,
                           uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, bool wide,

@@ -17,6 +17,11 @@
 // Workgroups stay and take tile after tile: the next tile's first loads go out ahead of a tile's stores (8192 x 8192 x 2048: 229 us with
 // a workgroup per tile, 200 so). S parts of K fill the chip where the tiles are few; their slabs are added by a second launch.
 //
+// The grouped form (tile_grouped) walks the tiles of all experts' sorted rows one expert after the other, with the rows of x gathered
+// through the sort; a tile ends where its expert's rows do. Both products of 8 experts with sorting and sum, us, against 64-row tiles of
+// grouped_rows.hip or 192 to 288-row ones of gemm_pf (tokens, two experts each): 2 x 3584 x 4096 300 240 -> 170, 700 242 -> 210, 4000
+// 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 300 76 -> 48, 1000 129 -> 93; 32 experts of 2 x 1024 x 2048, four each, 2000 239 -> 196.
+//
 // Measured, cold weights, us, against the library's product without what follows (M x N x K): 128 x 4096 x 14336 34 against 72;
 // 512 x 4096 x 14336 64 against 86; 300 x 10304 x 2048 20 against 24; 2521 x 10304 x 2048 88 against 96; 4001 x 18560 x 4096 438 against 554;
 // gated, 2521 x 16384 x 2048 147 against 193 with its activation, 8192 x 28672 x 4096 1403 against 1402; 8192 x 4096 x 14336 645 against 599
@@ -38,12 +43,17 @@ enum { kPairNone = 0, kPairHalves = 1, kPairBlocks = 2 };               // w's r
 struct TileArgs {
   const bf16 *x, *w;
   const void* bias;        // [N] fp32 or bf16, or nullptr
-  float* part;             // S > 1: [S, M, N] fp32 (gated: [gate | up] whatever the rows' order)
-  bf16* out;               // [M, N], or [M, N / 2] for the gated activations
+  float* part;             // [S, M, N] fp32 (gated: [gate | up] whatever the rows' order), or nullptr: the result is `out`
+  bf16* out;               // [M, N], or [M, N / 2] for the gated activations (S > 1: what the slabs' sum is written to)
   int64_t ld_x;
   int M, N, K, S, act, pairs;
   float p0, p1;
   bool bias_f32;
+  // grouped: row p of the experts' sorted rows is row rows[p] / top of x (rows nullptr: p; pads below 0: any), expert e's are
+  // offs[e] .. offs[e + 1], its weights w + e w_stride
+  const int32_t *rows, *offs;
+  int E, top;
+  int64_t w_stride;
 };
 
 // LDS DMA of 16 bytes a lane from a uniform base and a lane's byte offset
@@ -58,12 +68,6 @@ __device__ __forceinline__ void tile_dma(const void* base, uint32_t off, uint32_
 __device__ __forceinline__ void tile_mfma(f32x4_t& acc, bf16x8_t w, bf16x8_t x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-#endif
-}
-// ... and in vector registers, for what the 256 accumulation registers do not hold
-__device__ __forceinline__ void tile_mfma_v(f32x4_t& acc, bf16x8_t w, bf16x8_t x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w), "v"(x));
 #endif
 }
 
@@ -105,7 +109,7 @@ __device__ __forceinline__ void tile_by_act(const TileArgs& a, F f) {
   }
 }
 
-template <int FM, int FN, int RA, int RW, int OCC, bool PAIR>
+template <int FM, int FN, int RA, int RW, int OCC, bool PAIR, bool GRP>
 __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a) {
   constexpr int BM = 32 * FM, BN = 32 * FN, ASZ = BM * 128, WSZ = BN * 128;
   constexpr int LD = FM + FN;                      // fragment reads of a step, and DMA instructions of a K tile, per wave
@@ -120,9 +124,15 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wv >> 1, wn = wv & 1;
 
-  const int TM = (a.M + BM - 1) / BM, TN = (a.N + BN - 1) / BN, total = TM * TN * a.S;
+  const int TN = (a.N + BN - 1) / BN;
+  int total = (a.M + BM - 1) / BM * TN * a.S;
+  if constexpr (GRP) {
+    total = 0;
+    for (int e = 0; e < a.E; ++e) total += (a.offs[e + 1] - a.offs[e] + BM - 1) / BM * TN;
+    if ((int)blockIdx.x >= total) return;
+  }
   const int nk_all = a.K / 64, half = a.N / 2, dr = lane >> 3, dj = lane & 7;
-  int m0, n0, s, nk;
+  int m0, m_hi = a.M, n0, s, nk;
   uint32_t ao[FM], wo[FN];
   const char *xb, *wb;
   // the tile at place `at` of the order: neighbours on one XCD, columns of up to 8 row tiles next to each other. And what this
@@ -130,16 +140,27 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
   auto place = [&](int done) __attribute__((always_inline)) {
     const int nb = min((int)gridDim.x, total - done), bid = blockIdx.x, q8 = nb >> 3, r8 = nb & 7, xcd = bid & 7;
     const int v = done + (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
-    s = v / (TM * TN);
-    const int u = v - s * TM * TN, GM = TM < 8 ? TM : 8, gid = u / (GM * TN), first = gid * GM;
+    int TM = (a.M + BM - 1) / BM, u = v, lo = 0, e = 0;
+    if constexpr (GRP) {   // the experts' tiles one expert after the other
+      for (;; ++e) {
+        lo = a.offs[e], m_hi = a.offs[e + 1], TM = (m_hi - lo + BM - 1) / BM;
+        if (u < TM * TN) break;
+        u -= TM * TN;
+      }
+      s = 0;
+    } else {
+      s = v / (TM * TN), u = v - s * TM * TN;
+    }
+    const int GM = TM < 8 ? TM : 8, gid = u / (GM * TN), first = gid * GM;
     const int gm = TM - first < GM ? TM - first : GM, ug = u - gid * GM * TN;
-    m0 = (first + ug % gm) * BM, n0 = (ug / gm) * BN;
+    m0 = lo + (first + ug % gm) * BM, n0 = (ug / gm) * BN;
     const int kt_lo = s * nk_all / a.S;
     nk = (s + 1) * nk_all / a.S - kt_lo;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int r = min(8 * (wv * FM + i) + dr, a.M - 1 - m0);
-      ao[i] = (uint32_t)r * (uint32_t)(2 * a.ld_x) + 16 * (dj ^ dr);
+      int r = min(m0 + 8 * (wv * FM + i) + dr, m_hi - 1);
+      if (GRP && a.rows) r = max(a.rows[r], 0) / a.top;
+      ao[i] = (uint32_t)(GRP ? r : r - m0) * (uint32_t)(2 * a.ld_x) + 16 * (dj ^ dr);
     }
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
@@ -153,8 +174,8 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
       }
       wo[i] = (uint32_t)r * (uint32_t)(2 * a.K) + 16 * (dj ^ ((dr & 3) | ((p & 1) << 2)));
     }
-    xb = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ld_x + kt_lo * 64);
-    wb = reinterpret_cast<const char*>(a.w + kt_lo * 64);
+    xb = reinterpret_cast<const char*>(a.x + (GRP ? 0 : (int64_t)m0 * a.ld_x) + kt_lo * 64);
+    wb = reinterpret_cast<const char*>(a.w + (GRP ? e * a.w_stride : 0) + kt_lo * 64);
   };
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t) reinterpret_cast<uintptr_t>((xgk::lds_void_t*)lds));
   auto dma = [&](int i, int t, int sa, int sw) __attribute__((always_inline)) {   // i-th of tile t's loads: A of tile t, or W of tile t
@@ -200,8 +221,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
 #pragma unroll
     for (int q = 0; q < FM * FN; ++q) {
       const int m = FM >= FN ? q / FN : q % FM, n = FM >= FN ? q % FN : q / FM;
-      if (m * FN + n < 64) tile_mfma(acc[m][n], wf[KS][n], af[KS][m]);
-      else tile_mfma_v(acc[m][n], wf[KS][n], af[KS][m]);
+      tile_mfma(acc[m][n], wf[KS][n], af[KS][m]);
       if (q % RS == 0 && q / RS < LD) read(q / RS, KS ^ 1, ra, rw);
       if (KS == 1 && q % DS == DS / 2 && q / DS < LD) {
         const int j = q / DS;
@@ -246,7 +266,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
     for (int i = 0; i < LD; ++i) read(i, 0, 0, 0);
     const int col0 = PAIR ? n0 / 2 + wn * 8 * FN + 4 * g4 : n0 + wn * 16 * FN + 8 * g4, cols = PAIR ? half : a.N;
     // (the biases ahead of the loop, whose last tiles wait for all loads anyway: a load between the stores would wait for those)
-    const bool biased = !PAIR && a.bias && a.S == 1;
+    const bool biased = !PAIR && a.bias && !a.part;
     float b[FN / 2][8];
     if (!PAIR) {
 #pragma unroll
@@ -263,8 +283,8 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
 
     // ---- a lane holds 8 neighbouring columns of a row (two fragments), or 4 gate and 4 up columns. The next tile's first loads go
     // ahead of the stores (every wave is past its reads of this one since the last barrier).
-    const int row0 = m0 + wm * 16 * FM + l16, part = s;
-    behind = m0 + BM <= a.M && n0 + BN <= a.N;
+    const int row0 = m0 + wm * 16 * FM + l16, part = s, end = m_hi;
+    behind = m0 + BM <= m_hi && n0 + BN <= a.N;
     done += gridDim.x;
     const bool more = done + (int)blockIdx.x < total;
     if (more) place(done), prologue();
@@ -273,7 +293,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
 #pragma unroll
       for (int m = 0; m < FM; ++m) {
         const int row = row0 + 16 * m;
-        if (row >= a.M) continue;
+        if (row >= end) continue;
 #pragma unroll
         for (int j = 0; j < FN / 2; ++j) {
           const int col = col0 + (PAIR ? 16 : 32) * j;
@@ -281,7 +301,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
         }
       }
     };
-    if (a.S > 1) {
+    if (a.part) {
       each([&](int row, int col, int j, f32x4_t lo, f32x4_t hi) __attribute__((always_inline)) {
         float* at = a.part + ((int64_t)part * a.M + row) * a.N + col;
         *reinterpret_cast<f32x4_t*>(at) = lo;
@@ -341,8 +361,16 @@ template <int FM, int FN, int RA, int RW, int OCC>
 static void tile_launch(const TileArgs& a, int cus, hipStream_t st) {
   const int tiles = ((a.M + 32 * FM - 1) / (32 * FM)) * ((a.N + 32 * FN - 1) / (32 * FN));
   const int grid = tiles * a.S < cus * OCC ? tiles * a.S : cus * OCC;
-  if (a.pairs) tile_linear_kernel<FM, FN, RA, RW, OCC, true><<<grid, 256, 0, st>>>(a);
-  else tile_linear_kernel<FM, FN, RA, RW, OCC, false><<<grid, 256, 0, st>>>(a);
+  if (a.pairs) tile_linear_kernel<FM, FN, RA, RW, OCC, true, false><<<grid, 256, 0, st>>>(a);
+  else tile_linear_kernel<FM, FN, RA, RW, OCC, false, false><<<grid, 256, 0, st>>>(a);
+}
+
+template <int FM, int FN, int RA, int RW>
+static void tile_launch_grouped(const TileArgs& a, int cus, hipStream_t st) {
+  const int64_t tiles = (int64_t)(a.M / (32 * FM) + a.E) * ((a.N + 32 * FN - 1) / (32 * FN));   // at most
+  const int grid = tiles < cus ? (int)tiles : cus;
+  if (a.pairs) tile_linear_kernel<FM, FN, RA, RW, 1, true, true><<<grid, 256, 0, st>>>(a);
+  else tile_linear_kernel<FM, FN, RA, RW, 1, false, true><<<grid, 256, 0, st>>>(a);
 }
 
 int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bool bias_f32, float* part, void* out, int M,
@@ -354,7 +382,8 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part | (uintptr_t)out) & 15) ||
       (int64_t)N * K * 2 >= (1LL << 32) || 256 * ld_x * 2 >= (1LL << 32))
     return -1;
-  TileArgs a = {(const bf16*)x, (const bf16*)w, bias, part, (bf16*)out, ld_x, M, N, K, S, act, pairs, p0, p1, bias_f32};
+  TileArgs a = {(const bf16*)x, (const bf16*)w, bias, S > 1 ? part : nullptr, (bf16*)out, ld_x, M, N, K, S, act, pairs, p0, p1, bias_f32,
+                nullptr, nullptr, 0, 1, 0};
 #define XGM_TILE(FM, FN, RA, RW, OCC) else if (fm == FM && fn == FN) tile_launch<FM, FN, RA, RW, OCC>(a, cus, st);
   if (false) {}
   XGM_TILE(8, 8, 2, 3, 1)
@@ -375,6 +404,33 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
     if (gated) tile_linear_sum_kernel<true><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
     else tile_linear_sum_kernel<false><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a);
   }
+  return 0;
+}
+
+// Products of the experts' sorted rows (moe_align, moe_ff.hip) with their expert's weights w [E, N, K]: gated (act >= kTileGlu) `out`
+// [M, N / 2] bf16 of w's rows [gate | up], or fp32 `y` [M, N]. rows[p] / top is row p's row of x (nullptr: p), x_rows of them. Rows of
+// no expert are not written; a segment's pads (rows below 0) hold something finite.
+int tile_grouped(const void* x, int64_t ld_x, int x_rows, const int32_t* rows, const int32_t* offs, int E, int top, const void* w,
+                 float* y, void* out, int M, int N, int K, int act, float p0, float p1, int fm, int fn, int cus, hipStream_t st) {
+  const bool gated = act >= kTileGlu;
+  if (M < 1 || E < 1 || top < 1 || x_rows < 1 || N < 8 || N % 8 || K < 64 || K % 64 || ld_x < K || ld_x % 8 || !offs || cus < 1 ||
+      (gated ? !out || y : !y || out || act != kTileNone) || (!rows && x_rows < M) ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)out) & 15) || (int64_t)N * K * 2 >= (1LL << 32) ||
+      x_rows * ld_x * 2 >= (1LL << 32))
+    return -1;
+  TileArgs a = {(const bf16*)x, (const bf16*)w, nullptr, y, (bf16*)out, ld_x, M, N, K, 1, act, gated ? kPairHalves : kPairNone, p0, p1,
+                false, rows, offs, E, top, (int64_t)N * K};
+#define XGM_TILE(FM, FN, RA, RW) else if (fm == FM && fn == FN) tile_launch_grouped<FM, FN, RA, RW>(a, cus, st);
+  if (false) {}
+  XGM_TILE(8, 8, 2, 3)
+  XGM_TILE(7, 8, 2, 3)
+  XGM_TILE(6, 8, 2, 3)
+  XGM_TILE(4, 8, 3, 3)
+  XGM_TILE(6, 4, 4, 4)
+  XGM_TILE(4, 4, 5, 5)
+  XGM_TILE(3, 4, 5, 5)
+  else return -1;
+#undef XGM_TILE
   return 0;
 }
 }  // namespace xgm

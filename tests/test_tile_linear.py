@@ -6,6 +6,8 @@ import torch.nn.functional as F
 from xgserve.ops import seqmix as sq
 from xgserve.ops import tile_linear as tl
 
+from _seq_util import record_native
+
 
 def test_plans_fit_the_kernel():
     for M in (65, 66, 127, 200, 401, 1000, 2601, 8192):
@@ -85,3 +87,41 @@ def test_prompt_products_take_the_tiles():
         assert tl.tile_plan_of(x, torch.nn.Parameter(w)) is not None
     assert tl.tile_plan_of(x.t().contiguous().t(), w) is None and tl.tile_plan_of(x[:, 1:], w[:, 1:]) is None
     _close(sq.linear(x, w), x.double() @ w.double().t(), 2048)
+
+
+def test_grouped_plans_are_the_kernels():
+    for pairs, E, N, K in ((56, 1, 8, 64), (450, 8, 7168, 4096), (16384, 8, 4096, 3584), (100000, 64, 2048, 1024)):
+        assert tl.grouped_plan(pairs, E, N, K) in tl._GROUPED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tl._GROUPED)
+@pytest.mark.parametrize("kind", [sq.GLU_GELU_TANH, sq.GLU_CLAMPED, sq.GLU_SILU])
+def test_grouped_tiles(tile, kind, monkeypatch):
+    """Shares of every size: no row, one, a tile's worth and one more, several tiles; columns left over."""
+    K, F_, W, top = 128, 192, 136, 2
+    share = [0, 1, 32 * tile[0], 32 * tile[0] + 1, 7, 0, 2 * 32 * tile[0] - 5, 500]
+    E, g = len(share), torch.Generator().manual_seed(tile[0])
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(share))
+    if ids.numel() % 2:
+        ids = torch.cat([ids, ids[-1:]])
+    ids = ids[torch.randperm(ids.numel(), generator=g)].view(-1, top).to(torch.int32)
+    T = ids.shape[0]
+    h = torch.randn(T, K, generator=g).to(torch.bfloat16)
+    w13 = (torch.randn(E, 2 * F_, K, generator=g) * 3 * K ** -0.5).to(torch.bfloat16)
+    w2 = (torch.randn(E, W, F_, generator=g) * F_ ** -0.5).to(torch.bfloat16)
+    wts = torch.rand(T, top, generator=g)
+    monkeypatch.setattr(sq, "grouped_plan", lambda *a: tile)
+    calls = record_native(monkeypatch, sq)
+    got = sq.routed_experts(h.cuda(), w13.cuda(), w2.cuda(), ids.cuda(), wts.cuda(), kind, 2.0, 1.702).cpu().double()
+    assert calls.count("tile_grouped") == 2
+    ref = torch.zeros(T, W, dtype=torch.float64)
+    size = torch.zeros(T, W, dtype=torch.float64)
+    for e in range(E):
+        t, j = torch.nonzero(ids == e, as_tuple=True)
+        z = h[t].double() @ w13[e].double().t()
+        a = sq._glu_ref(z[:, :F_], z[:, F_:], kind, 2.0, 1.702)
+        ref.index_add_(0, t, wts[t, j, None].double() * (a @ w2[e].double().t()))
+        size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
+    # the activations are rounded to bf16 (2^-9 of each term of the second product), the sums are fp32
+    assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())

@@ -21,8 +21,9 @@ import torch.nn.functional as F
 
 from .. import tune
 from ._native import is_f32, mixers, native_device, stream_ptr
+from .linear import cu_count
 from .moe import _moe_pf_cfg
-from .tile_linear import PAIR_HALVES, forward_only as _forward_only, tile_linear, tile_plan_of
+from .tile_linear import GROUPED_EXPERTS_MAX, PAIR_HALVES, forward_only as _forward_only, grouped_plan, tile_linear, tile_plan_of
 
 
 @dataclass
@@ -1134,7 +1135,11 @@ ACT_RELU2 = 2   # routed_experts(kind=...): an expert without a gate, W_down rel
 MOE_MFMA = tune.get_bool("moe_mfma", True)
 # XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on the tiles of csrc/mixers (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
-MOE_PF_MIN = 96   # average rows per expert from which gated experts run on gemm_pf's grouped form
+# Average rows per expert from which gated experts run on the tiles of tile_linear.hip: up to there most segments fit one tile of 64
+# rows of the weight-streaming products. Both products with the sum, 8 experts of 2 x 3584 x 4096, us, streamed / tiles: average 50
+# 147 / 163, 75 240 / 170, 100 224 / 179; of 2 x 2048 x 2048 53 / 47, 76 / 48, 96 / 52.
+MOE_TILED_MIN = 56
+MOE_PF_MIN = 96   # ... and more experts than those tiles take on gemm_pf's grouped form
 # Rows per expert tile of the sorted layout, and the average rows per expert from which it is taken. Weight-streaming
 # products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
 # us: tiles of 16 104 / 142 / - / 230 / -, 32 112 / 113 / 115 / 175 / 233, 64 121 / 123 / 123 / 127 / 191; 32 experts of
@@ -1287,8 +1292,11 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     # ... or run on gemm_pf's grouped form: both operands by LDS DMA, 64-row segments, 256-column tiles
     pf = SEQ_MOE_PF and MOE_MFMA and gated and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E and K % 64 == 0 \
         and F_ % 128 == 0 and W % 256 == 0
-    if pf:
-        tm = 64
+    tiled = SEQ_MOE_PF and streams and gated and not scale_input and pairs >= MOE_TILED_MIN * E and E <= GROUPED_EXPERTS_MAX \
+        and W % 8 == 0 and max(T * K, 2 * F_ * K, W * F_, (pairs + 16 * E) * F_) < 1 << 31 \
+        and (h.data_ptr() | w13.data_ptr() | w2.data_ptr()) % 16 == 0
+    if pf or tiled:
+        tm = 16 if tiled else 64   # (rows of an expert's last tile: the tiles end where the segment does)
     cap = (pairs + E * (tm - 1) + tm - 1) // tm * tm
     dev = h.device
     meta = torch.empty(cap + cap // tm + pairs + E + 1, dtype=torch.int32, device=dev)
@@ -1296,6 +1304,14 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     M.moe_align(_i32(ids).data_ptr(), pairs, E, cap, tm, rows.data_ptr(), tile_e.data_ptr(), dest.data_ptr(),
                 offs.data_ptr(), _p(clear), clear.numel() if clear is not None else 0, stream_ptr())
     act = torch.empty(cap, F_, dtype=h.dtype, device=dev)
+    if tiled:
+        cus = cu_count(dev)
+        y = torch.empty(cap, W, dtype=torch.float32, device=dev)
+        M.tile_grouped(h.data_ptr(), K, T, rows.data_ptr(), offs.data_ptr(), E, top, w13.data_ptr(), 0, act.data_ptr(), cap, 2 * F_, K,
+                       ACT_GLU + kind, float(limit), float(alpha), *grouped_plan(pairs, E, 2 * F_, K, cus), cus, stream_ptr())
+        M.tile_grouped(act.data_ptr(), F_, cap, 0, offs.data_ptr(), E, 1, w2.data_ptr(), y.data_ptr(), 0, cap, W, F_, ACT_NONE, 0.0, 0.0,
+                       *grouped_plan(pairs, E, W, F_, cus), cus, stream_ptr())
+        return _routed_sum(M, y, dest, wts, T, top, W, combine)
     if pf:
         cfg = _moe_pf_cfg(pairs, E)
         y = torch.empty(cap, W, dtype=torch.float32, device=dev)

@@ -7,6 +7,7 @@ of the kernel's forms in the mean and 13 % at most.
 from __future__ import annotations
 
 import functools
+import math
 from typing import Optional
 
 import torch
@@ -47,6 +48,26 @@ def tile_plan(M: int, N: int, K: int, cus: int = 256):
             t += _SUM + 4 * M * N * S / _PART_BYTES if S > 1 else 2 * M * N / _OUT_BYTES
             if best is None or t < best[0]:
                 best = (t, fm, fn, S)
+    return best[1:]
+
+
+# Tiles of the experts' products; offsets of all experts are looked through for a tile's, so there is a bound on their number
+_GROUPED, GROUPED_EXPERTS_MAX = ((8, 8), (7, 8), (6, 8), (4, 8), (6, 4), (4, 4), (3, 4)), 64
+
+
+@functools.lru_cache(maxsize=4096)
+def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
+    """(rows / 32, columns / 32) for `pairs` rows shared out among E experts' [N, K] weights at random: `tile_plan`'s prices, the
+    tiles counted at six quantiles of an expert's rows."""
+    avg, best = pairs / E, None
+    for fm, fn in _GROUPED:
+        kt, per = _TILES[fm, fn]
+        rows = [max(1.0, avg + z * math.sqrt(avg)) for z in (-1.3, -0.7, -0.25, 0.25, 0.7, 1.3)]
+        tiles = E * sum(-(-r // (32 * fm)) for r in rows) / len(rows) * -(-N // (32 * fn))
+        work, load = -(-tiles // cus) * (K / 64 * kt + per), 2 * E * N * K / _W_BYTES
+        t = max(work, load) + _OVERLAP * min(work, load)
+        if best is None or t < best[0]:
+            best = (t, fm, fn)
     return best[1:]
 
 
