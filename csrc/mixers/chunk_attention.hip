@@ -592,6 +592,51 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(const T* __restrict__ o_a
   }
 }
 
+// The same from the shares that the keys of single tokens were divided into (masked_attention_combine's, vmode all): merged and mixed
+// in one launch, the merged rows in LDS and fp32. A workgroup has 16 value columns of a token, which belong to one key/value head.
+// Both launches it stands for are latency alone: 17 tokens of 16 heads, 2 x 128 value columns, 5.2 + 7.6 us.
+__global__ __launch_bounds__(256) void talk_mix_parts_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                             const int32_t* __restrict__ slots, const float* __restrict__ talk,
+                                                             const bf16* __restrict__ gate, int64_t ld_gate,
+                                                             bf16* __restrict__ out, int Ttot, int H, int G, int dv, int nsplit) {
+  __shared__ float ws[64][65], inv[64], o[64][17];
+  const int t = blockIdx.x, nd = dv / 16, c = blockIdx.y / nd, d0 = 16 * (blockIdx.y % nd), rep = H / G;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  bf16* row = out + ((int64_t)t * H + c * rep) * dv + d0;
+  if (slots[t] < 0) {
+    for (int i = threadIdx.x; i < rep * 16; i += 256) row[(i / 16) * dv + i % 16] = 0;
+    return;
+  }
+  const int64_t step = (int64_t)Ttot * H, row0 = (int64_t)t * H;
+  for (int g = wid; g < H; g += 4) {
+    const float ms = lane < nsplit ? part_ml[2 * (row0 + g + lane * step)] : -INFINITY;
+    const float ls = lane < nsplit ? part_ml[2 * (row0 + g + lane * step) + 1] : 0.f;
+    const float M = wave_max(ms);
+    const float w = ms == -INFINITY ? 0.f : exp2_fast(ms - M);
+    const float L = wave_sum(w * ls);
+    ws[g][lane] = w;
+    if (lane == 0) inv[g] = L > 0.f ? 1.f / L : 0.f;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < H * 16; i += 256) {
+    const int g = i / 16, d = i % 16;
+    const float* p = part_o + (row0 + g) * G * dv + c * dv + d0 + d;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int sp = 0; sp < nsplit; ++sp) acc += ws[g][sp] * p[sp * step * G * dv];   // (a share without keys holds zeros)
+    o[g][d] = acc * inv[g];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < rep * 16; i += 256) {
+    const int h = c * rep + i / 16, d = i % 16;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int g = 0; g < H; ++g) acc += talk[h * H + g] * o[g][d];
+    if (gate) acc *= sigmoidf(bf2f(gate[(int64_t)t * ld_gate + h]));
+    row[(i / 16) * dv + d] = f2bf(acc);
+  }
+}
+
 // ------------------------------------------------------------------ q / k norm + rotation -> q, cache rows
 // One workgroup per token; a wave takes the heads (H query heads, then G key heads) round robin. A lane owns the
 // entries d = lane, lane + 64, ... of a head; the partner of a rotated entry is re-read (it is in the same row).
@@ -916,7 +961,7 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
                           const float* sink, void* out, int T_, int ns, int max_q, int H, int G, int dk, int dv_head,
                           int mask, int size, float scale, int nsplit, float* part_o, float* part_ml, const void* gate,
                           int64_t ld_gate, const float* r1, const float* r2, int vmode, int nw_hint, bool gate_elem,
-                          int wfn, const float* hbias, float softcap, int keep, hipStream_t st) {
+                          int wfn, const float* hbias, float softcap, int keep, bool merge, hipStream_t st) {
   if (T_ <= 0 || ns <= 0 || max_q <= 0) return 0;
   const int dv = vmode == kValuesAll ? G * dv_head : dv_head;
   if (G <= 0 || H % G != 0 || dk % 32 != 0 || dv % 16 != 0 || dk > 128 || dv > 256 || mask < 0 || mask > 2 ||
@@ -946,7 +991,7 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
                         ld_gate, r1, r2, vmode, ge, hbias, softcap, keep};
     if (!head_slots && max_q > kPromptMinRows && nw_hint == 0 && prompt_attention(args, max_q, wfn, st)) return 0;
     if (head_slots && single_attention(args, wfn, nsplit, part_o, part_ml, st)) {
-      if (nsplit > 1)
+      if (nsplit > 1 && merge)
         masked_attention_combine_kernel<<<dim3(T_, H), dv > 128 ? 256 : dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit,
                                                                     (const bf16*)gate, ld_gate, ge, wfn);
       return 0;
@@ -976,7 +1021,7 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
   } else {                                                                                                            \
     XGM_MK(NKK, NMT, 4)                                                                                               \
   }                                                                                                                   \
-  if (nsplit > 1)                                                                                                     \
+  if (nsplit > 1 && merge)                                                                                            \
     masked_attention_combine_kernel<<<dim3(T_, H), dv > 128 ? 256 : dv > 64 ? 128 : 64, 0, st>>>(part_o, part_ml, slots, (bf16*)out, T_, H, dv, nsplit, \
                                                                 (const bf16*)gate, ld_gate, ge, wfn);                 \
   return 0;
@@ -987,6 +1032,15 @@ int masked_attention_mfma(const void* q, const void* kcache, const void* vcache,
 #undef XGM_MM
 #undef XGM_MK
 #undef XGM_MK2
+}
+
+int talk_mix_parts(const float* part_o, const float* part_ml, const int32_t* slots, const float* talk, const void* gate,
+                   int64_t ld_gate, void* out, int T_, int H, int G, int dv, int nsplit, hipStream_t st) {
+  if (T_ <= 0) return 0;
+  if (H < 1 || H > 64 || G < 1 || H % G || dv < 16 || dv % 16 || nsplit < 1 || nsplit > 64 || (int64_t)G * dv / 16 > 65535) return -1;
+  talk_mix_parts_kernel<<<dim3(T_, G * (dv / 16)), 256, 0, st>>>(part_o, part_ml, slots, talk, (const bf16*)gate, ld_gate, (bf16*)out,
+                                                                 T_, H, G, dv, nsplit);
+  return 0;
 }
 
 void talk_mix(const void* o_all, bool f32, const float* talk, const void* gate, int64_t ld_gate, void* out, int T_, int H,

@@ -30,7 +30,9 @@ int masked_attention(const void*, bool, const void*, const void*, const int32_t*
 int masked_attention_mfma(const void*, const void*, const void*, const int32_t*, int, int, const int32_t*, const int32_t*,
                           const int32_t*, const float*, const float*, void*, int, int, int, int, int, int, int, int, int,
                           float, int, float*, float*, const void*, int64_t, const float*, const float*, int, int, bool, int,
-                          const float*, float, int, hipStream_t);
+                          const float*, float, int, bool, hipStream_t);
+int talk_mix_parts(const float*, const float*, const int32_t*, const float*, const void*, int64_t, void*, int, int, int, int, int,
+                   hipStream_t);
 void talk_mix(const void*, bool, const float*, const void*, int64_t, void*, int, int, int, int, hipStream_t);
 void head_norm_rope_cache(const void*, bool, int64_t, int, int, int, int, const float*, const float*, float, const float*,
                           int, int, const int32_t*, const int32_t*, void*, void*, void*, bool, int, bool, bool, const void*,
@@ -222,7 +224,7 @@ PYBIND11_MODULE(_mixers, m) {
                                     int size, float scale, int nsplit, uintptr_t part_o, uintptr_t part_ml,
                                     uintptr_t gate, int64_t ld_gate, uintptr_t r1, uintptr_t r2, int vmode, int nw_hint,
                                     bool gate_elem, int wfn, uintptr_t hbias, float softcap, int keep_first,
-                                    uintptr_t st) {
+                                    bool merge, uintptr_t st) {
     if (bs < 1 || bt_width < 1 || nsplit < 1 || (gate && ld_gate < (gate_elem ? (int64_t)H * dv : H)))
       throw std::invalid_argument("masked_attention_mfma: inconsistent sizes");
     int rc = xgm::masked_attention_mfma(P<const void>(q), P<const void>(kc), P<const void>(vc), P<const int32_t>(bt),
@@ -230,8 +232,15 @@ PYBIND11_MODULE(_mixers, m) {
                                         P<const float>(temp), P<const float>(sink), P<void>(out), T, ns, max_q, H, G, dk,
                                         dv, mask, size, scale, nsplit, P<float>(part_o), P<float>(part_ml),
                                         P<const void>(gate), ld_gate, P<const float>(r1), P<const float>(r2), vmode,
-                                        nw_hint, gate_elem, wfn, P<const float>(hbias), softcap, keep_first, S(st));
+                                        nw_hint, gate_elem, wfn, P<const float>(hbias), softcap, keep_first, merge, S(st));
     check(rc, "masked_attention_mfma");
+  });
+  m.def("talk_mix_parts", [](uintptr_t part_o, uintptr_t part_ml, uintptr_t slots, uintptr_t talk, uintptr_t gate, int64_t ld_gate,
+                             uintptr_t out, int T, int H, int G, int dv, int nsplit, uintptr_t st) {
+    if (gate && ld_gate < H) throw std::invalid_argument("talk_mix_parts: inconsistent sizes");
+    check(xgm::talk_mix_parts(P<const float>(part_o), P<const float>(part_ml), P<const int32_t>(slots), P<const float>(talk),
+                              P<const void>(gate), ld_gate, P<void>(out), T, H, G, dv, nsplit, S(st)),
+          "talk_mix_parts");
   });
   m.def("talk_mix", [](uintptr_t o_all, bool f32, uintptr_t talk, uintptr_t gate, int64_t ld_gate, uintptr_t out, int T,
                        int H, int G, int dv, uintptr_t st) {

@@ -96,12 +96,12 @@ class TalkingDistanceAttention(nn.Module):
         q = sq.qk_norm_cache(proj[:, :n], self.nq, self.nk, self.nv, None, None, 0.0, sm, lc.k, lc.v)
         kw = dict(gate=None, dist=(self.r1, self.r2))
         args = (q, lc.k, lc.v, H, G, self.dk, dv, sq.MASK_CAUSAL, 0, self.scale, None, None, block_size, sm)
+        gate = proj[:, n:n + H]
         if G * dv <= sq.V_ALL_MAX:
-            wide = sq.masked_attention(*args, values=sq.V_ALL, **kw)
+            o = sq.masked_attention(*args, values=sq.V_ALL, talk=(self.talk, gate), **kw)
         else:   # one pass per value head
             wide = torch.stack([sq.masked_attention(*args, values=c, **kw).view(-1, H, dv) for c in range(G)], 2)
-            wide = wide.reshape(-1, H * G * dv)
-        o = sq.talk_mix(wide, self.talk, H, G, dv, gate=proj[:, n:n + H])
+            o = sq.talk_mix(wide.reshape(-1, H * G * dv), self.talk, H, G, dv, gate=gate)
         return sq.linear_parts(o, self.o, sm)
 
 

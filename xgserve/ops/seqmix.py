@@ -947,12 +947,46 @@ V_ALL_MAX = 256         # ... V_ALL serves up to this many value columns (G * dv
 W_SOFTMAX, W_SIGMOID = 0, 1   # masked_attention(weights=...): how scores become weights
 
 
+def _key_shares(T: int, G: int, mask: int, size: int, keep_first: int = 0) -> int:
+    """Workgroups that share the visible keys of a single token's key/value head."""
+    tiles = (size + keep_first + 63) // 64 if mask != MASK_CAUSAL else ATTN_MAX_SPLITS
+    return max(1, min(ATTN_MAX_SPLITS, tiles, ATTN_SPLIT_WGS // max(1, T * G)))
+
+
+def _talking_attention(q, kcache, vcache, H, G, dk, dv, mask, size, scale, temp, sink, block_size, sm, dist, talk):
+    """masked_attention(values=V_ALL) and talk_mix of its result; the shares of single tokens' keys are merged by the mixing launch."""
+    T, (mix, gate) = q.shape[0], talk
+    nsplit = _key_shares(T, G, mask, size)
+    if not (native_device(q) and ATTN_MFMA and q.dtype == torch.bfloat16 and sm.max_q == 1 and T == sm.num_seqs and nsplit > 1
+            and dk % 32 == 0 and dk <= 128 and dv % 16 == 0 and G * dv <= 256 and H // G <= 64 and H <= 64
+            and (gate is None or (gate.dtype == q.dtype and gate.stride(1) == 1 and gate.shape[1] >= H))):
+        wide = masked_attention(q, kcache, vcache, H, G, dk, dv, mask, size, scale, temp, sink, block_size, sm, dist=dist,
+                                values=V_ALL)
+        return talk_mix(wide, mix, H, G, dv, gate=gate)
+    assert q.is_contiguous() and kcache.is_contiguous() and vcache.is_contiguous() and kcache.dtype == vcache.dtype == q.dtype
+    assert mix.dtype == torch.float32 and mix.is_contiguous() and mix.shape == (H, H)
+    r1, r2 = dist if dist is not None else (None, None)
+    bt, slots = _i32(sm.block_tables), _i32(sm.slots)
+    wide = torch.empty(T, H * G * dv, dtype=q.dtype, device=q.device)   # (rows of no sequence are cleared there, no others written)
+    part_o = torch.empty(nsplit * T * H * G * dv, dtype=torch.float32, device=q.device)
+    part_ml = torch.empty(nsplit * T * H * 2, dtype=torch.float32, device=q.device)
+    mixers().masked_attention_mfma(q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), bt.data_ptr(), bt.shape[1], block_size,
+                                   _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), slots.data_ptr(), _p(temp), _p(sink),
+                                   wide.data_ptr(), T, sm.num_seqs, 1, H, G, dk, dv, int(mask), int(size), float(scale), nsplit,
+                                   part_o.data_ptr(), part_ml.data_ptr(), 0, 0, _p(r1), _p(r2), V_ALL, ATTN_WAVES, False,
+                                   W_SOFTMAX, 0, 0.0, 0, False, stream_ptr())
+    out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+    mixers().talk_mix_parts(part_o.data_ptr(), part_ml.data_ptr(), slots.data_ptr(), mix.data_ptr(), _p(gate),
+                            gate.stride(0) if gate is not None else 0, out.data_ptr(), T, H, G, dv, nsplit, stream_ptr())
+    return out
+
+
 def masked_attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, H: int, G: int, dk: int, dv: int,
                      mask: int, size: int, scale: float, temp: Optional[torch.Tensor], sink: Optional[torch.Tensor],
                      block_size: int, sm: SeqMeta, gate: Optional[torch.Tensor] = None,
                      dist: Optional[tuple] = None, values: int = V_OWN, gate_elem: bool = False,
                      weights: int = W_SOFTMAX, score_bias: Optional[torch.Tensor] = None, softcap: float = 0.0,
-                     keep_first: int = 0) -> torch.Tensor:
+                     keep_first: int = 0, talk: Optional[tuple] = None) -> torch.Tensor:
     """Softmax attention of H query heads over G cached key/value heads (query head h reads head h // (H / G)).
     A query at position i sees keys first_visible(mask, size, i) .. i of its own sequence, and with `keep_first` (sliding
     windows) also the sequence's first keep_first keys up to its own position. score = (q . k) * scale * temp[h], with
@@ -964,8 +998,12 @@ def masked_attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor
     0), not normalised over the keys (no sink).
     `values`: V_OWN: head h weighs the values of its own key/value head, returns [T, H * dv]; V_ALL: the values of
     all G heads concatenated, returns [T, H * G * dv] (what mixing of the heads' weight maps needs);
-    c >= 0: the values of head c for every query head.
+    c >= 0: the values of head c for every query head. With `talk` = (weights [H, H], gate or None), V_ALL alone: what
+    talk_mix makes of the result.
     q [T, H * dk]; caches [rows, G * dk] / [rows, G * dv]."""
+    if talk is not None:
+        assert values == V_ALL and gate is None
+        return _talking_attention(q, kcache, vcache, H, G, dk, dv, mask, size, scale, temp, sink, block_size, sm, dist, talk)
     T = q.shape[0]
     dvo = G * dv if values == V_ALL else dv           # value columns per query head
     out = torch.empty(T, H * dvo, dtype=q.dtype, device=q.device)
@@ -988,8 +1026,7 @@ def masked_attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor
             # single tokens as the query heads of one key/value head per wave
             nsplit, part_o, part_ml = 1, None, None
             if single:  # divide the visible key tiles over several workgroups (merged by a second launch)
-                tiles = (size + keep_first + 63) // 64 if mask != MASK_CAUSAL else ATTN_MAX_SPLITS
-                nsplit = max(1, min(ATTN_MAX_SPLITS, tiles, ATTN_SPLIT_WGS // max(1, T * G)))
+                nsplit = _key_shares(T, G, mask, size, keep_first)
                 if nsplit > 1:
                     part_o = torch.empty(nsplit * T * H * dvo, dtype=torch.float32, device=q.device)
                     part_ml = torch.empty(nsplit * T * H * 2, dtype=torch.float32, device=q.device)
@@ -999,7 +1036,7 @@ def masked_attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor
                                            sm.max_q, H, G, dk, dv, int(mask), int(size), float(scale), nsplit,
                                            _p(part_o), _p(part_ml), _p(gate), gate.stride(0) if gate is not None else 0,
                                            _p(r1), _p(r2), int(values), ATTN_WAVES, bool(gate_elem), int(weights),
-                                           _p(score_bias), float(softcap), int(keep_first), stream_ptr())
+                                           _p(score_bias), float(softcap), int(keep_first), True, stream_ptr())
             return out
         mixers().masked_attention(q.data_ptr(), is_f32(q), kcache.data_ptr(), vcache.data_ptr(), bt.data_ptr(),
                                   bt.shape[1], block_size, _i32(sm.positions).data_ptr(), _i32(sm.token_seq).data_ptr(),
