@@ -35,10 +35,11 @@ def tile_plan(M: int, N: int, K: int, cus: int = 256):
     """(rows / 32, columns / 32, parts of K) of an [M, K] . [N, K]^T product."""
     best = None
     for (fm, fn), (kt, per) in _TILES.items():
-        # measured up to 400 and 2600 rows only: many small tiles read the weights and rows more often than this counts
-        if 32 * fm >= 2 * M + 64 or (fn == 2 and M > 400) or (fm <= 4 and fn == 4 and M > 2600):
-            continue
+        # (many small tiles read the weights and rows more often than this counts: those of 64 columns only while the chip holds
+        # them all, 512 x 2048 x 2048 11.7 us against 15.6 with 128 columns)
         tiles = -(-M // (32 * fm)) * -(-N // (32 * fn))
+        if 32 * fm >= 2 * M + 64 or (fn == 2 and M > 400 and tiles > cus) or (fm <= 4 and fn == 4 and M > 2600):
+            continue
         for S in _SPLITS:
             if S > 1 and (K // S < _SPLIT_K or tiles * S > _SPLIT_TILES):
                 break
@@ -74,13 +75,14 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
 def library_better(M: int, N: int, K: int) -> bool:
     """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel).
 
-    Small: narrow products below 3.3 G multiply-adds start fewer workgroups than there are compute units (2048x2048, 512 rows 11.5
-    against 15.2; 1088x2048, 700 rows 11.4 against 16.4; beyond the line 2048x2048, 1536 rows 18.8 against 16.6). Long: both run at
+    Small: narrow products of few rows start fewer workgroups than there are compute units, and what adds their parts is a launch
+    (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4; 2048x4096, 128 rows 11.0 against 12.6; 1088x2048, 192 rows 8.5
+    against 10.0; beyond the line 2048x4096, 320 rows 18.0 against 16.7; 2048x8192, 65 rows 18.3 against 13.5). Long: both run at
     the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
     4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81; up to 1792 rows 4096x14336, 1536 rows 168 against 140;
     6144x4096, 700 rows 45 against 41), as long as no columns are left over beside its tiles of 256 (10304x2048, 4001 rows 168 against
     129; 18560x4096, 2048 rows 344 against 257)."""
-    if N <= 3072 and K >= 1024 and M * N * K < 3.3e9:
+    if N <= 2304 and 1024 <= K <= 4096 and M * N * K < 2.2e9:
         return True
     return N % 256 == 0 and M > 1792
 
