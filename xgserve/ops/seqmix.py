@@ -92,7 +92,7 @@ _ROWS_TICKETS = _ROWS_WGS // 2     # column tiles of a product in parts
 
 # xIELU behind the product of prompt rows up to here: its 25 instructions an element run on four waves there and on a full chip in a
 # launch of their own (8192 x 2048, us, behind / by itself: 300 rows 20.6 / 24.3, 1000 rows 42.5 / 42.2, 8192 rows 275 / 259). The
-# squared ReLU and the gated activations always go behind (8192 rows: 216 / 253; gated 16384 x 2048, 2521 rows 147 / 193).
+# squared ReLU and the gated activations always go behind (8192 rows: 216 / 253; gated 16384 x 2048, 2521 rows 141 / 192).
 XIELU_BEHIND_MAX = 512
 
 ACT_NONE, ACT_XIELU, ACT_RELU2, ACT_GLU = 0, 1, 2, 3   # ACT_GLU + GLU_...: the gated activations
