@@ -56,7 +56,7 @@ def mixers():
 
 def native_device(t: torch.Tensor) -> bool:
     """True when `t` lives on the GPU: its ops run on the HIP kernels or raise."""
-    return t.device.type == "cuda"
+    return t.is_cuda
 
 
 def is_f32(t: torch.Tensor) -> bool:
@@ -85,7 +85,9 @@ def use_native(t: torch.Tensor) -> bool:
 
 
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device. (torch.cuda.current_stream() makes a Stream object of it, 3 us of a launch's host
+    time; small prompt steps wait for the host.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(t) -> int:

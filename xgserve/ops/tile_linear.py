@@ -73,17 +73,13 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
 
 
 def library_better(M: int, N: int, K: int) -> bool:
-    """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel).
-
-    Small: narrow products of few rows start fewer workgroups than there are compute units, and what adds their parts is a launch
-    (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4; 2048x4096, 128 rows 11.0 against 12.6; 1088x2048, 192 rows 8.5
-    against 10.0; beyond the line 2048x4096, 320 rows 18.0 against 16.7; 2048x8192, 65 rows 18.3 against 13.5). Long: both run at
-    the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
-    4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81; up to 1792 rows 4096x14336, 1536 rows 168 against 140;
-    6144x4096, 700 rows 45 against 41; below 150 tiles of 256 x 256 2048x8192, 2521 rows 77 to 81 against 75), as long as no columns are left over beside its tiles of 256 (10304x2048, 4001 rows 168 against
-    129; 18560x4096, 2048 rows 344 against 257)."""
-    if N <= 2304 and 1024 <= K <= 4096 and M * N * K < 2.2e9:
-        return True
+    """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel): long ones, which run
+    at the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
+    4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81), as long as no columns are left over beside its tiles of
+    256 (10304x2048, 4001 rows 168 against 129; 18560x4096, 2048 rows 344 against 257) and there are 150 such tiles (2048x8192, 2521
+    rows 77 to 81 against 75; up to 1792 rows 4096x14336, 1536 rows 168 against 140; 6144x4096, 700 rows 45 against 41). Its narrow
+    products of few rows are 1 to 2 us faster on the card (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4), but such
+    steps wait for the host, of which the library's call takes 31 us and this kernel's 10."""
     return N % 256 == 0 and M > 1792 and -(-M // 256) * (N // 256) >= 150
 
 
