@@ -19,8 +19,8 @@
 //
 // The grouped form (tile_grouped) walks the tiles of all experts' sorted rows one expert after the other, with the rows of x gathered
 // through the sort; a tile ends where its expert's rows do. Both products of 8 experts with sorting and sum, us, against 64-row tiles of
-// grouped_rows.hip or 192 to 288-row ones of gemm_pf (tokens, two experts each): 2 x 3584 x 4096 300 240 -> 170, 700 242 -> 210, 4000
-// 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 300 76 -> 48, 1000 129 -> 93; 32 experts of 2 x 1024 x 2048, four each, 2000 239 -> 196.
+// grouped_rows.hip or 192 to 288-row ones of gemm_pf (tokens, two experts each): 2 x 3584 x 4096 300 240 -> 152, 700 242 -> 189, 4000
+// 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 300 76 -> 48, 1000 129 -> 85; 32 experts of 2 x 1024 x 2048, four each, 500 130 -> 108.
 //
 // Measured, cold weights, us, against the library's product without what follows (M x N x K): 128 x 4096 x 14336 34 against 72;
 // 512 x 4096 x 14336 64 against 86; 300 x 10304 x 2048 20 against 24; 2521 x 10304 x 2048 88 against 96; 4001 x 18560 x 4096 438 against 554;
@@ -39,6 +39,13 @@ using xgk::f32x4_t;
 enum { kTileNone = 0, kTileXielu = 1, kTileRelu2 = 2, kTileGlu = 3 };   // kTileGlu + kind: glu.h
 enum { kPairNone = 0, kPairHalves = 1, kPairBlocks = 2 };               // w's rows: [gate | up], or 16 gate, 16 up, ...
 
+// Up to so many rows (grouped: per expert) neighbouring column tiles start at different places in K: else all of them ask for the same
+// column of weight rows 2 K bytes apart, which few memory channels hold, at the same time. With more rows the workgroups of one row tile
+// gain more from reading its rows together. us without / with: 128 x 28672 x 4096 57 / 50, 128 x 18560 x 4096 50 / 46, 192 x 4096 x 8192 31 /
+// 29, 400 x 18560 x 4096 73 / 77, 1024 x 2048 x 8192 45 / 80; both products of 8 experts of 2 x 3584 x 4096 with 75 rows each 176 / 152,
+// with 250 290 / 270.
+constexpr int kRotateRows = 256;
+
 struct TileArgs {
   const bf16 *x, *w;
   const void* bias;        // [N] fp32 or bf16, or nullptr
@@ -53,6 +60,7 @@ struct TileArgs {
   const int32_t *rows, *offs;
   int E, top;
   int64_t w_stride;
+  bool rotate;             // column tiles start at different K tiles
 };
 
 // LDS DMA of 16 bytes a lane from a uniform base and a lane's byte offset
@@ -143,7 +151,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
     if ((int)blockIdx.x >= total) return;
   }
   const int nk_all = a.K / 64, half = a.N / 2, dr = lane >> 3, dj = lane & 7;
-  int m0, m_hi = a.M, n0, s, nk;
+  int m0, m_hi = a.M, n0, s, nk, rot;
   uint32_t ao[FM], wo[FN];
   const char *xb, *wb;
   // the tile at place `at` of the order: neighbours on one XCD, columns of up to 8 row tiles next to each other. And what this
@@ -167,6 +175,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
     m0 = lo + (first + ug % gm) * BM, n0 = (ug / gm) * BN;
     const int kt_lo = s * nk_all / a.S;
     nk = (s + 1) * nk_all / a.S - kt_lo;
+    rot = a.rotate ? (int)((unsigned)(ug / gm) * 37u % (unsigned)nk) : 0;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       int r = min(m0 + 8 * (wv * FM + i) + dr, m_hi - 1);
@@ -190,8 +199,10 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
   };
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t) reinterpret_cast<uintptr_t>((xgk::lds_void_t*)lds));
   auto dma = [&](int i, int t, int sa, int sw) __attribute__((always_inline)) {   // i-th of tile t's loads: A of tile t, or W of tile t
-    if (i < FM) tile_dma(xb + (int64_t)t * 128, ao[i], lds0 + sa * ASZ + (wv * FM + i) * 1024);
-    else tile_dma(wb + (int64_t)t * 128, wo[i - FM], lds0 + RA * ASZ + sw * WSZ + (wv * FN + i - FM) * 1024);
+    int kt = t + rot;
+    kt = kt >= nk ? kt - nk : kt;
+    if (i < FM) tile_dma(xb + (int64_t)kt * 128, ao[i], lds0 + sa * ASZ + (wv * FM + i) * 1024);
+    else tile_dma(wb + (int64_t)kt * 128, wo[i - FM], lds0 + RA * ASZ + sw * WSZ + (wv * FN + i - FM) * 1024);
   };
 
   // ---- fragment reads: x row 16 i + l16, W row 32 (i / 2) + 8 (l16 / 4) + l16 % 4 + 4 (i % 2); K half ks
@@ -398,7 +409,7 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
       (int64_t)N * K * 2 >= (1LL << 32) || 256 * ld_x * 2 >= (1LL << 32))
     return -1;
   TileArgs a = {(const bf16*)x, (const bf16*)w, bias, S > 1 ? part : nullptr, (bf16*)out, ld_x, M, N, K, S, act, pairs, p0, p1, bias_f32,
-                nullptr, nullptr, 0, 1, 0};
+                nullptr, nullptr, 0, 1, 0, M <= kRotateRows};
 #define XGM_TILE(FM, FN, RA, RW, OCC) else if (fm == FM && fn == FN) tile_launch<FM, FN, RA, RW, OCC>(a, cus, st);
   if (false) {}
   XGM_TILE(8, 8, 2, 3, 1)
@@ -408,7 +419,6 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
   XGM_TILE(8, 4, 3, 4, 1)
   XGM_TILE(6, 4, 4, 4, 1)
   XGM_TILE(4, 4, 5, 5, 1)
-  else if (fm == 104 && fn == 4) tile_launch<4, 4, 2, 2, 2>(a, cus, st);
   XGM_TILE(3, 4, 5, 5, 1)
   XGM_TILE(4, 2, 6, 6, 1)
   XGM_TILE(3, 2, 3, 3, 2)
@@ -434,7 +444,7 @@ int tile_grouped(const void* x, int64_t ld_x, int x_rows, const int32_t* rows, c
       x_rows * ld_x * 2 >= (1LL << 32))
     return -1;
   TileArgs a = {(const bf16*)x, (const bf16*)w, nullptr, y, (bf16*)out, ld_x, M, N, K, 1, act, gated ? kPairHalves : kPairNone, p0, p1,
-                false, rows, offs, E, top, (int64_t)N * K};
+                false, rows, offs, E, top, (int64_t)N * K, M <= (int64_t)kRotateRows * E};
 #define XGM_TILE(FM, FN, RA, RW) else if (fm == FM && fn == FN) tile_launch_grouped<FM, FN, RA, RW>(a, cus, st);
   if (false) {}
   XGM_TILE(8, 8, 2, 3)

@@ -1173,9 +1173,9 @@ MOE_MFMA = tune.get_bool("moe_mfma", True)
 # XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on the tiles of csrc/mixers (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
 # Average rows per expert from which gated experts run on the tiles of tile_linear.hip: up to there most segments fit one tile of 64
-# rows of the weight-streaming products. Both products with the sum, 8 experts of 2 x 3584 x 4096, us, streamed / tiles: average 50
-# 147 / 163, 75 240 / 170, 100 224 / 179; of 2 x 2048 x 2048 53 / 47, 76 / 48, 96 / 52.
-MOE_TILED_MIN = 56
+# rows of the weight-streaming products. Both products with the sum, us, streamed / tiles: 8 experts of 2 x 3584 x 4096, average 37
+# 138 / 141, 50 147 / 145, 75 244 / 152; of 2 x 2048 x 2048 50 / 46, 51 / 47, 74 / 48; 32 of 2 x 1024 x 2048 95 / 103, 113 / 106, - / -.
+MOE_TILED_MIN = 45
 MOE_PF_MIN = 96   # ... and more experts than those tiles take on gemm_pf's grouped form
 # Rows per expert tile of the sorted layout, and the average rows per expert from which it is taken. Weight-streaming
 # products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
