@@ -20,7 +20,7 @@
 // The grouped form (tile_grouped) walks the tiles of all experts' sorted rows one expert after the other, with the rows of x gathered
 // through the sort; a tile ends where its expert's rows do. Both products of 8 experts with sorting and sum, us, against 64-row tiles of
 // grouped_rows.hip or 192 to 288-row ones of gemm_pf (tokens, two experts each): 2 x 3584 x 4096 300 240 -> 152, 700 242 -> 189, 4000
-// 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 300 76 -> 48, 1000 129 -> 85; 32 experts of 2 x 1024 x 2048, four each, 500 130 -> 108.
+// 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 1000 129 -> 85; 32 experts of 2 x 1024 x 2048, four each, 2000 239 -> 194.
 //
 // Measured, cold weights, us, against the library's product without what follows (M x N x K): 128 x 4096 x 14336 34 against 72;
 // 512 x 4096 x 14336 64 against 86; 300 x 10304 x 2048 20 against 24; 2521 x 10304 x 2048 88 against 96; 4001 x 18560 x 4096 438 against 554;

@@ -125,3 +125,28 @@ def test_grouped_tiles(tile, kind, monkeypatch):
         size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
     # the activations are rounded to bf16 (2^-9 of each term of the second product), the sums are fp32
     assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("F_,K,T,tiled", [(4096, 2048, 179, False), (4096, 2048, 180, True),      # 45 rows an expert: 16 M weights each
+                                          (256, 128, 383, False), (256, 128, 384, True)])         # 96: smaller experts
+def test_which_experts_take_the_tiles(F_, K, T, tiled, monkeypatch):
+    E, W, top = 8, 256, 2
+    g = torch.Generator("cuda").manual_seed(T)
+    h = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16)
+    w13 = (torch.randn(E, 2 * F_, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    w2 = (torch.randn(E, W, F_, generator=g, device="cuda") * F_ ** -0.5).to(torch.bfloat16)
+    ids = (torch.arange(T * top, device="cuda", dtype=torch.int32) % E).view(T, top)
+    wts = torch.rand(T, top, generator=g, device="cuda")
+    calls = record_native(monkeypatch, sq)
+    got = sq.routed_experts(h, w13, w2, ids, wts, sq.GLU_SILU).double()
+    assert calls.count("tile_grouped") == (2 if tiled else 0)
+    ref, size = torch.zeros(T, W, dtype=torch.float64, device="cuda"), torch.zeros(T, W, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        t, j = torch.nonzero(ids == e, as_tuple=True)
+        z = h[t].double() @ w13[e].double().t()
+        a = sq._glu_ref(z[:, :F_], z[:, F_:], sq.GLU_SILU, 0.0, 0.0)
+        ref.index_add_(0, t, wts[t, j, None].double() * (a @ w2[e].double().t()))
+        size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
+    # activations in bf16 (2^-9 of each term), sums in fp32
+    assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())

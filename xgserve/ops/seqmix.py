@@ -1173,9 +1173,10 @@ MOE_MFMA = tune.get_bool("moe_mfma", True)
 # XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on the tiles of csrc/mixers (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
 # Average rows per expert from which gated experts run on the tiles of tile_linear.hip: up to there most segments fit one tile of 64
-# rows of the weight-streaming products. Both products with the sum, us, streamed / tiles: 8 experts of 2 x 3584 x 4096, average 37
-# 138 / 141, 50 147 / 145, 75 244 / 152; of 2 x 2048 x 2048 50 / 46, 51 / 47, 74 / 48; 32 of 2 x 1024 x 2048 95 / 103, 113 / 106, - / -.
-MOE_TILED_MIN = 45
+# rows of the weight-streaming products, and experts of less than MOE_TILED_ELEMS gate and up weights stay on those up to where
+# gemm_pf's form would begin. Cold weights, with router and shared expert, us, streamed / tiles: 8 experts of 2 x 3584 x 4096, average
+# 45 228 / 210, 57 246 / 217, 75 290 / 241; of 2 x 2048 x 2048 101 / 104, 103 / 108, 116 / 124, 100 167 / 127.
+MOE_TILED_MIN, MOE_TILED_ELEMS = 45, 16 << 20
 MOE_PF_MIN = 96   # ... and more experts than those tiles take on gemm_pf's grouped form
 # Rows per expert tile of the sorted layout, and the average rows per expert from which it is taken. Weight-streaming
 # products (csrc/mixers/grouped_rows.hip), both of 8 experts of 2 x 3584 x 4096 at an average of 4 / 16 / 25 / 38 / 64 rows,
@@ -1329,7 +1330,8 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     # ... or run on gemm_pf's grouped form: both operands by LDS DMA, 64-row segments, 256-column tiles
     pf = SEQ_MOE_PF and MOE_MFMA and gated and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E and K % 64 == 0 \
         and F_ % 128 == 0 and W % 256 == 0
-    tiled = SEQ_MOE_PF and streams and gated and not scale_input and pairs >= MOE_TILED_MIN * E and E <= GROUPED_EXPERTS_MAX \
+    tiled_min = MOE_TILED_MIN if 2 * F_ * K >= MOE_TILED_ELEMS else max(MOE_TILED_MIN, MOE_PF_MIN)
+    tiled = SEQ_MOE_PF and streams and gated and not scale_input and pairs >= tiled_min * E and E <= GROUPED_EXPERTS_MAX \
         and W % 8 == 0 and max(T * K, 2 * F_ * K, W * F_, (pairs + 16 * E) * F_) < 1 << 31 \
         and (h.data_ptr() | w13.data_ptr() | w2.data_ptr()) % 16 == 0
     if pf or tiled:
