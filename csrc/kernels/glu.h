@@ -7,6 +7,7 @@
 namespace xgk {
 
 constexpr int kGluGeluTanh = 0, kGluClamped = 1, kGluSilu = 3;   // (2: an ungated activation of the expert products)
+constexpr bool glu_known(int kind) { return kind == kGluGeluTanh || kind == kGluClamped || kind == kGluSilu; }
 
 //   kGluGeluTanh   0.5 g (1 + tanh(sqrt(2 / pi) (g + 0.044715 g^3))) * u, as g sigmoid(2 sqrt(2 / pi) ...) * u: the same number
 //                  without the difference of 1 and a tanh close to -1, in half the instructions

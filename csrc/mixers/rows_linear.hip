@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * WV, 1) void rows_linear_kernel(const RowsArgs 
 int rows_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bool bias_f32, float* part, void* out,
                 int* tickets, int T, int N, int K, int S, int act, float p0, float p1, bool wide, hipStream_t st) {
   const bool gated = act >= kActGlu;
-  if (T < 1 || T > 64 || N < 1 || K < 128 || K % 128 || N % (gated ? 8 : 4) || ld_x % 8 || (gated && (!wide || bias)) ||
+  if (T < 1 || T > 64 || N < 1 || K < 128 || K % 128 || N % (gated ? 8 : 4) || ld_x % 8 || (gated && (!wide || bias || !xgk::glu_known(act - kActGlu))) ||
       act < 0 || (S != 1 && S != 2 && S != 4 && S != 8) || S > K / 128 || (S > 1 && !part) ||
       (S > 1 && !tickets && (act != kActNone || bias)) ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part) & 15) || ((uintptr_t)out & 7) ||

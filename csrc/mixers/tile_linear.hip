@@ -403,7 +403,7 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
                 int N, int K, int S, int act, int pairs, float p0, float p1, int fm, int fn, int cus, hipStream_t st) {
   const bool gated = act >= kTileGlu;
   if (M < 1 || N < 8 || N % 8 || K < 64 || K % 64 || ld_x < K || ld_x % 8 || S < 1 || S > K / 64 || act < 0 || gated != (pairs != 0) ||
-      pairs < 0 || pairs > 2 || (gated && (bias || N % (pairs == kPairBlocks ? 32 : 8))) || (S > 1 && !part) ||
+      (gated && !xgk::glu_known(act - kTileGlu)) || cus < 1 || pairs < 0 || pairs > 2 || (gated && (bias || N % (pairs == kPairBlocks ? 32 : 8))) || (S > 1 && !part) ||
       (!out && (S == 1 || act != kTileNone || bias)) ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)part | (uintptr_t)out) & 15) ||
       (int64_t)N * K * 2 >= (1LL << 32) || 256 * ld_x * 2 >= (1LL << 32))
@@ -439,7 +439,7 @@ int tile_grouped(const void* x, int64_t ld_x, int x_rows, const int32_t* rows, c
                  float* y, void* out, int M, int N, int K, int act, float p0, float p1, int fm, int fn, int cus, hipStream_t st) {
   const bool gated = act >= kTileGlu;
   if (M < 1 || E < 1 || top < 1 || x_rows < 1 || N < 8 || N % 8 || K < 64 || K % 64 || ld_x < K || ld_x % 8 || !offs || cus < 1 ||
-      (gated ? !out || y : !y || out || act != kTileNone) || (!rows && x_rows < M) ||
+      (gated ? !out || y || !xgk::glu_known(act - kTileGlu) : !y || out || act != kTileNone) || (!rows && x_rows < M) ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)out) & 15) || (int64_t)N * K * 2 >= (1LL << 32) ||
       x_rows * ld_x * 2 >= (1LL << 32))
     return -1;

@@ -150,3 +150,25 @@ def test_which_experts_take_the_tiles(F_, K, T, tiled, monkeypatch):
         size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
     # activations in bf16 (2^-9 of each term), sums in fp32
     assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())
+
+
+@pytest.mark.parametrize("rows", [8, 128])
+@pytest.mark.parametrize("kind", [-1, 2, 4])
+def test_unknown_gates_go_to_the_activation_that_refuses_them(rows, kind, monkeypatch):
+    seen = []
+    monkeypatch.setattr(sq, "_rows_plan_of", lambda *a, **k: (True, 1))
+    monkeypatch.setattr(sq, "tile_plan_of", lambda *a, **k: (3, 2, 1))
+    monkeypatch.setattr(sq, "_rows_linear", lambda *a: seen.append("rows"))
+    monkeypatch.setattr(sq, "tile_linear", lambda *a: seen.append("tiles"))
+    monkeypatch.setattr(sq, "glu_act", lambda z, k, *a: seen.append(k))
+    sq.linear_glu(torch.zeros(rows, 128), torch.zeros(256, 128), kind)
+    assert seen == [kind]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [8, 128])
+@pytest.mark.parametrize("kind", [-1, 2, 4])
+def test_unknown_gates_are_refused(rows, kind):
+    x, w = torch.zeros(rows, 128, device="cuda", dtype=torch.bfloat16), torch.zeros(256, 128, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        sq.linear_glu(x, w, kind)

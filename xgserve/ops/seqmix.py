@@ -215,10 +215,11 @@ def linear_relu2(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
 def linear_glu(x: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.702,
                sm: Optional[SeqMeta] = None) -> torch.Tensor:
     """glu_act(x . w^T, kind, limit, alpha) of w's rows [gate | up]."""
-    plan = _rows_plan_of(x, w, sm, None, True)
+    known = kind in (GLU_GELU_TANH, GLU_CLAMPED, GLU_SILU)   # (glu_act refuses others)
+    plan = _rows_plan_of(x, w, sm, None, True) if known else None
     if plan is not None:
         return _rows_linear(plan, x, w, sm, None, ACT_GLU + kind, limit, alpha)
-    plan = tile_plan_of(x, w, None, PAIR_HALVES)
+    plan = tile_plan_of(x, w, None, PAIR_HALVES) if known else None
     if plan is not None:
         return tile_linear(plan, x, w, None, ACT_GLU + kind, limit, alpha, PAIR_HALVES)
     return glu_act(F.linear(x, w), kind, limit, alpha)
