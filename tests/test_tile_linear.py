@@ -172,3 +172,17 @@ def test_unknown_gates_are_refused(rows, kind):
     x, w = torch.zeros(rows, 128, device="cuda", dtype=torch.bfloat16), torch.zeros(256, 128, device="cuda", dtype=torch.bfloat16)
     with pytest.raises(ValueError):
         sq.linear_glu(x, w, kind)
+
+
+@pytest.mark.parametrize("rows", [8, 128])
+def test_products_on_another_device_stay_with_torch(rows, monkeypatch):
+    """Launches go to the current device's stream; torch's products run where their tensors are."""
+    x, w = torch.zeros(rows, 256, dtype=torch.bfloat16), torch.zeros(64, 256, dtype=torch.bfloat16)
+    for m in (sq, tl):
+        monkeypatch.setattr(m, "native_device", lambda t: True)
+    monkeypatch.setattr(tl, "cu_count", lambda d: 256)
+    plan = (lambda: sq._rows_plan_of(x, w, None, None, False)) if rows <= 64 else (lambda: tl.tile_plan_of(x, w))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device(), raising=False)
+    assert plan() is not None
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device() + 1, raising=False)
+    assert plan() is None

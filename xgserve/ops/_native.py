@@ -59,6 +59,11 @@ def native_device(t: torch.Tensor) -> bool:
     return t.is_cuda
 
 
+def on_current_device(t: torch.Tensor) -> bool:
+    """Whether a GPU tensor lies on the device whose stream launches go to (`stream_ptr`)."""
+    return t.get_device() == torch._C._cuda_getDevice()
+
+
 def is_f32(t: torch.Tensor) -> bool:
     if t.dtype == torch.float32:
         return True

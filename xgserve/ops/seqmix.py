@@ -20,7 +20,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import tune
-from ._native import is_f32, mixers, native_device, stream_ptr
+from ._native import is_f32, mixers, native_device, on_current_device, stream_ptr
 from .linear import cu_count
 from .moe import _moe_pf_cfg
 from .tile_linear import GROUPED_EXPERTS_MAX, PAIR_HALVES, forward_only as _forward_only, grouped_plan, tile_linear, tile_plan_of
@@ -125,11 +125,12 @@ def _rows_plan(N: int, K: int, gated: bool):
 
 def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool,
                   slabs: bool = False):
-    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16 on one device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
+    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16 on the current device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
     pieces, K in whole staged rows, nothing that wants a derivative, and tickets where K is in parts (clearing them would cost
     what the parts gain) unless the `slabs` are the result. What is refused here goes to torch, which refuses what it cannot do."""
     if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.device == x.device and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX and _forward_only(x, w, bias)):
+            and w.device == x.device and on_current_device(x) and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX
+            and _forward_only(x, w, bias)):
         return None
     N, K = w.shape
     if K < 128 or K % 128 or x.shape[1] != K or N < 1 or N % (8 if gated else 4) or not w.is_contiguous() or \

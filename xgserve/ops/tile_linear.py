@@ -13,7 +13,7 @@ import torch
 import torch.autograd.forward_ad as _fwd_ad
 from torch._C._functorch import is_functorch_wrapped_tensor as _is_transformed
 
-from ._native import is_f32, mixers, native_device, stream_ptr
+from ._native import is_f32, mixers, native_device, on_current_device, stream_ptr
 from .linear import PendingSum, cu_count
 
 # rows and columns of a workgroup's tile / 32 -> us per 64 of K and per tile
@@ -100,11 +100,12 @@ def forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor])
 
 def tile_plan_of(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, pairs: int = PAIR_NONE,
                  plain: bool = False):
-    """The plan of x . w^T on the tile kernel, or None: bfloat16 on one device, more than 64 rows of whole 16-byte pieces, K in
+    """The plan of x . w^T on the tile kernel, or None: bfloat16 on the current device, more than 64 rows of whole 16-byte pieces, K in
     whole steps of 64, whole groups of columns, nothing that wants a derivative; `plain` products only where the library's is not
     faster. What is refused here goes to torch, which refuses what it cannot do."""
     if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.device == x.device and w.dim() == 2 and x.shape[0] >= TILE_ROWS_MIN and forward_only(x, w, bias)):
+            and w.device == x.device and on_current_device(x) and w.dim() == 2 and x.shape[0] >= TILE_ROWS_MIN
+            and forward_only(x, w, bias)):
         return None
     (M, ldk), (N, K) = x.shape, w.shape
     if ldk != K or K < 64 or K % 64 or N < 8 or N % (32 if pairs == PAIR_BLOCKS else 8) or not w.is_contiguous() or \
