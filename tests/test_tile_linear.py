@@ -186,3 +186,33 @@ def test_products_on_another_device_stay_with_torch(rows, monkeypatch):
     assert plan() is not None
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device() + 1, raising=False)
     assert plan() is None
+
+
+class _Seen(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def test_modes_that_choose_or_see_a_product_keep_it_with_torch():
+    x, w = torch.zeros(128, 64, dtype=torch.bfloat16), torch.zeros(256, 64, dtype=torch.bfloat16)
+    assert tl.forward_only(x, w, None)
+    with torch.autocast("cpu", dtype=torch.float16):
+        assert not tl.forward_only(x, w, None)
+        with torch.autocast("cpu", enabled=False):
+            assert tl.forward_only(x, w, None)
+    with _Seen():
+        assert not tl.forward_only(x, w, None)
+    with torch.device("cpu"):
+        assert tl.forward_only(x, w, None)
+        with _Seen():
+            assert not tl.forward_only(x, w, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [8, 128])
+def test_autocast_chooses_the_type(rows):
+    x, w = torch.ones(rows, 128, device="cuda", dtype=torch.bfloat16), torch.ones(256, 128, device="cuda", dtype=torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.float16):
+        y = sq.linear(x, w)
+    assert y.dtype == torch.float16 and bool((y == 128).all())
+    assert sq.linear(x, w).dtype == torch.bfloat16

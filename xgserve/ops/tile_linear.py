@@ -12,6 +12,8 @@ from typing import Optional
 import torch
 import torch.autograd.forward_ad as _fwd_ad
 from torch._C._functorch import is_functorch_wrapped_tensor as _is_transformed
+from torch.overrides import _get_current_function_mode_stack as _function_modes
+from torch.utils._device import DeviceContext
 
 from ._native import is_f32, mixers, native_device, on_current_device, stream_ptr
 from .linear import PendingSum, cu_count
@@ -86,11 +88,13 @@ def library_better(M: int, N: int, K: int) -> bool:
 
 
 def forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
-    """Whether nothing follows these tensors through the call: no graph, no tangents, no function transform, no tracing or dispatch
-    mode, no tensor type of its own. (A product on a kernel of this library has no derivative and no operator to record; torch's
-    has.)"""
+    """Whether nothing follows these tensors through the call or stands before it: no graph, no tangents, no function transform, no
+    tracing, function or dispatch mode (a default device alone is none: it makes tensors), no autocast, which chooses the product's
+    type, no tensor type of its own. (A product on a kernel of this library has no derivative and no operator to record; torch's has.)"""
     if _fwd_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing() \
-            or torch.compiler.is_compiling():
+            or torch.compiler.is_compiling() or torch.is_autocast_enabled(x.device.type):
+        return False
+    if torch._C._len_torch_function_stack() > 0 and any(type(m) is not DeviceContext for m in _function_modes()):
         return False
     for t in (x, w, bias):
         if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or _is_transformed(t)):
