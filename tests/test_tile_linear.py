@@ -216,3 +216,13 @@ def test_autocast_chooses_the_type(rows):
         y = sq.linear(x, w)
     assert y.dtype == torch.float16 and bool((y == 128).all())
     assert sq.linear(x, w).dtype == torch.bfloat16
+
+
+def test_grouped_sizes_end_where_the_kernel_refuses():
+    """Activations of 2^31 elements in the sorted layout (one expert: up to 30 rows more than there are pairs) are past a lane's
+    offset: pairs just below stay on the streamed products."""
+    F_ = 2048
+    for pairs in range((1 << 20) - 40, (1 << 20) + 2):
+        cap = sq._sorted_rows(pairs, 1, 16)
+        assert sq._experts_on_tiles(pairs, 1, 64, F_, 64, pairs) == (cap * F_ < 1 << 31)
+    assert not sq._experts_on_tiles((1 << 20) - 17, 1, 64, F_, 64, (1 << 20) - 17)   # 2^20 rows

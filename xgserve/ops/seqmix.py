@@ -1292,6 +1292,19 @@ class RoutedRows:
     wts: Optional[torch.Tensor] = None
 
 
+def _sorted_rows(pairs: int, E: int, tm: int) -> int:
+    """Rows of the sorted layout, each expert's padded to whole tiles of tm, at most."""
+    return (pairs + E * (tm - 1) + tm - 1) // tm * tm
+
+
+def _experts_on_tiles(pairs: int, E: int, K: int, F_: int, W: int, T: int) -> bool:
+    """Whether gated experts of these sizes run on tile_linear's grouped form: enough rows per expert, whole column groups, and what a
+    lane's 32-bit byte offset reaches (the rows, an expert's weights, the activations in their sorted layout)."""
+    least = MOE_TILED_MIN if 2 * F_ * K >= MOE_TILED_ELEMS else max(MOE_TILED_MIN, MOE_PF_MIN)
+    return pairs >= least * E and E <= GROUPED_EXPERTS_MAX and W % 8 == 0 \
+        and max(T * K, 2 * F_ * K, W * F_, _sorted_rows(pairs, E, 16) * F_) < 1 << 31
+
+
 def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, kind: int,
                    limit: float = 0.0, alpha: float = 1.702, scale_input: bool = False, combine: bool = True,
                    clear: Optional[torch.Tensor] = None):
@@ -1332,13 +1345,11 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     # ... or run on gemm_pf's grouped form: both operands by LDS DMA, 64-row segments, 256-column tiles
     pf = SEQ_MOE_PF and MOE_MFMA and gated and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E and K % 64 == 0 \
         and F_ % 128 == 0 and W % 256 == 0
-    tiled_min = MOE_TILED_MIN if 2 * F_ * K >= MOE_TILED_ELEMS else max(MOE_TILED_MIN, MOE_PF_MIN)
-    tiled = SEQ_MOE_PF and streams and gated and not scale_input and pairs >= tiled_min * E and E <= GROUPED_EXPERTS_MAX \
-        and W % 8 == 0 and max(T * K, 2 * F_ * K, W * F_, (pairs + 16 * E) * F_) < 1 << 31 \
+    tiled = streams and gated and not scale_input and SEQ_MOE_PF and _experts_on_tiles(pairs, E, K, F_, W, T) \
         and (h.data_ptr() | w13.data_ptr() | w2.data_ptr()) % 16 == 0
     if pf or tiled:
         tm = 16 if tiled else 64   # (rows of an expert's last tile: the tiles end where the segment does)
-    cap = (pairs + E * (tm - 1) + tm - 1) // tm * tm
+    cap = _sorted_rows(pairs, E, tm)
     dev = h.device
     meta = torch.empty(cap + cap // tm + pairs + E + 1, dtype=torch.int32, device=dev)
     rows, tile_e, dest, offs = meta.split((cap, cap // tm, pairs, E + 1))
