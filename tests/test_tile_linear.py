@@ -182,9 +182,10 @@ def test_products_on_another_device_stay_with_torch(rows, monkeypatch):
         monkeypatch.setattr(m, "native_device", lambda t: True)
     monkeypatch.setattr(tl, "cu_count", lambda d: 256)
     plan = (lambda: sq._rows_plan_of(x, w, None, None, False)) if rows <= 64 else (lambda: tl.tile_plan_of(x, w))
-    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device(), raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 1, raising=False)
+    monkeypatch.setattr(torch.Tensor, "get_device", lambda t: 1)
     assert plan() is not None
-    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device() + 1, raising=False)
+    monkeypatch.setattr(torch.Tensor, "get_device", lambda t: 0)
     assert plan() is None
 
 

@@ -60,8 +60,9 @@ def native_device(t: torch.Tensor) -> bool:
 
 
 def on_current_device(t: torch.Tensor) -> bool:
-    """Whether a GPU tensor lies on the device whose stream launches go to (`stream_ptr`)."""
-    return t.get_device() == torch._C._cuda_getDevice()
+    """Whether a GPU tensor lies on the device whose stream launches go to (`stream_ptr`); a host tensor (-1) lies on no other."""
+    index = t.get_device()
+    return index < 0 or index == torch._C._cuda_getDevice()
 
 
 def is_f32(t: torch.Tensor) -> bool:

@@ -129,8 +129,8 @@ def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias:
     pieces, K in whole staged rows, nothing that wants a derivative, and tickets where K is in parts (clearing them would cost
     what the parts gain) unless the `slabs` are the result. What is refused here goes to torch, which refuses what it cannot do."""
     if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.device == x.device and on_current_device(x) and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX
-            and _forward_only(x, w, bias)):
+            and w.device == x.device and w.dim() == 2 and 1 <= x.shape[0] <= ROWS_LINEAR_MAX and _forward_only(x, w, bias)
+            and on_current_device(x)):
         return None
     N, K = w.shape
     if K < 128 or K % 128 or x.shape[1] != K or N < 1 or N % (8 if gated else 4) or not w.is_contiguous() or \

@@ -108,8 +108,8 @@ def tile_plan_of(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     whole steps of 64, whole groups of columns, nothing that wants a derivative; `plain` products only where the library's is not
     faster. What is refused here goes to torch, which refuses what it cannot do."""
     if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-            and w.device == x.device and on_current_device(x) and w.dim() == 2 and x.shape[0] >= TILE_ROWS_MIN
-            and forward_only(x, w, bias)):
+            and w.device == x.device and w.dim() == 2 and x.shape[0] >= TILE_ROWS_MIN and forward_only(x, w, bias)
+            and on_current_device(x)):
         return None
     (M, ldk), (N, K) = x.shape, w.shape
     if ldk != K or K < 64 or K % 64 or N < 8 or N % (32 if pairs == PAIR_BLOCKS else 8) or not w.is_contiguous() or \
