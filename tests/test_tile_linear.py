@@ -227,3 +227,13 @@ def test_grouped_sizes_end_where_the_kernel_refuses():
         cap = sq._sorted_rows(pairs, 1, 16)
         assert sq._experts_on_tiles(pairs, 1, 64, F_, 64, pairs) == (cap * F_ < 1 << 31)
     assert not sq._experts_on_tiles((1 << 20) - 17, 1, 64, F_, 64, (1 << 20) - 17)   # 2^20 rows
+
+
+def test_llama_products_run_in_torch_where_the_kernels_are_missing(monkeypatch):
+    """XGS_ALLOW_TORCH_FALLBACK=1 without a built library: no plan is asked for, torch's products run."""
+    from xgserve.models import llama
+    monkeypatch.setattr(llama, "use_native", lambda t: False, raising=False)
+    monkeypatch.setattr(llama, "tile_plan_of", lambda *a, **k: pytest.fail("a plan without kernels"))
+    x, w = torch.randn(128, 64).bfloat16(), torch.randn(256, 64).bfloat16()
+    assert torch.equal(llama._product(x, w, parts=True), F.linear(x, w))
+    assert llama._silu_gate(x, w).shape == (128, 128)

@@ -40,6 +40,7 @@ from ..ops.linear import (MODE_PARTIAL, MODE_SILU, MW_MAX_M, W8_MAX_M, W8_MIN_EL
                           mw_linear, mw_plan, pf_linear, pf_plan, pick_split,
                           quantize_fp8, quantize_weight, skinny_linear, splitk_linear, splitk_prefill_ok, w8_linear,
                           w8_plan, WQ_FORMATS)
+from ..ops._native import use_native
 from ..ops.seqmix import ACT_GLU, GLU_SILU
 from ..ops.tile_linear import PAIR_BLOCKS, tile_linear, tile_parts, tile_plan_of
 from .base import AttnMeta, PagedAttention, init_weight, kv_head_range, local_heads, shard
@@ -106,9 +107,13 @@ def pf_projections(T: int) -> frozenset:
     return frozenset(k for k, ws in PF_WINDOWS.items() if any(lo <= T <= hi for lo, hi in ws))
 
 
+def _tile_plan(x: torch.Tensor, w: torch.Tensor, **kw):
+    return tile_plan_of(x, w, **kw) if use_native(x) else None
+
+
 def _product(x: torch.Tensor, w: torch.Tensor, parts: bool = False):
     """x . w^T of a prompt-sized step, on the tile kernel or the library's; parts: a PendingSum where K is in parts."""
-    plan = tile_plan_of(x, w, plain=True)
+    plan = _tile_plan(x, w, plain=True)
     if plan is None:
         return F.linear(x, w)
     return tile_parts(plan, x, w) if parts and plan[2] > 1 else tile_linear(plan, x, w)
@@ -116,7 +121,7 @@ def _product(x: torch.Tensor, w: torch.Tensor, parts: bool = False):
 
 def _silu_gate(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up of a block-16 interleaved gate|up weight."""
-    plan = tile_plan_of(x, w, None, PAIR_BLOCKS)
+    plan = _tile_plan(x, w, pairs=PAIR_BLOCKS)
     if plan is None:
         return ops.silu_and_mul(F.linear(x, w), interleave16=True)
     return tile_linear(plan, x, w, None, ACT_GLU + GLU_SILU, pairs=PAIR_BLOCKS)
@@ -345,7 +350,7 @@ class LlamaLayer(nn.Module):
 
     def _down(self, a: torch.Tensor):
         """The down projection of a prompt-sized step on one GPU; parts of K are added by the next add + norm."""
-        if tile_plan_of(a, self.down, plain=True) is None and splitk_prefill_ok(a, self.down):
+        if _tile_plan(a, self.down, plain=True) is None and splitk_prefill_ok(a, self.down):
             return splitk_linear(a, self.down, linear_mod.SPLITK_PREFILL_S)
         return _product(a, self.down, parts=True)
 
