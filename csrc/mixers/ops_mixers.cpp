@@ -64,6 +64,8 @@ int ssm_step(const void*, bool, int64_t, const void*, int64_t, const float*, con
              const int32_t*, const int32_t*, float*, int, int, int, int, int, hipStream_t);
 int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const void*, const float*, const float*, const float*,
                float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
+int tile_plan(const double*, int, const int*, int, const double*, int64_t, int64_t, int64_t, int, int*);
+int grouped_plan(const double*, int, const double*, int, const double*, int64_t, int64_t, int64_t, int64_t, int, int*);
 int tile_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int, int, int, int, int, int, float, float,
                 int, int, int, hipStream_t);
 int tile_grouped(const void*, int64_t, int, const int32_t*, const int32_t*, int, int, const void*, float*, void*, int, int, int, int, float,
@@ -371,6 +373,19 @@ PYBIND11_MODULE(_mixers, m) {
                           P<const int32_t>(qsl), P<const int32_t>(seq_lens), P<const int32_t>(slots), P<void>(out), ns, H, D,
                           S(st)),
           "delta_step");
+  });
+  m.def("tile_plan", [](uintptr_t tiles, int n, uintptr_t splits, int n_splits, uintptr_t prices, int64_t M, int64_t N, int64_t K, int cus) {
+    int best[3];
+    if (xgm::tile_plan(P<const double>(tiles), n, P<const int>(splits), n_splits, P<const double>(prices), M, N, K, cus, best))
+      throw std::invalid_argument("tile_plan: no tile for these sizes");
+    return py::make_tuple(best[0], best[1], best[2]);
+  });
+  m.def("grouped_plan", [](uintptr_t tiles, int n, uintptr_t quantiles, int n_q, uintptr_t prices, int64_t pairs, int64_t E, int64_t N,
+                           int64_t K, int cus) {
+    int best[2];
+    if (xgm::grouped_plan(P<const double>(tiles), n, P<const double>(quantiles), n_q, P<const double>(prices), pairs, E, N, K, cus, best))
+      throw std::invalid_argument("grouped_plan: no tile for these sizes");
+    return py::make_tuple(best[0], best[1]);
   });
   m.def("tile_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part, uintptr_t out,
                           int M, int N, int K, int S_, int act, int pairs, float p0, float p1, int fm, int fn, int cus, uintptr_t st) {

@@ -237,3 +237,44 @@ def test_llama_products_run_in_torch_where_the_kernels_are_missing(monkeypatch):
     x, w = torch.randn(128, 64).bfloat16(), torch.randn(256, 64).bfloat16()
     assert torch.equal(llama._product(x, w, parts=True), F.linear(x, w))
     assert llama._silu_gate(x, w).shape == (128, 128)
+
+
+def _priced(M, N, K, cus):
+    """The cheapest tile and parts of K by the prices, counted out plainly (the first of equals)."""
+    out = []
+    for (fm, fn), (kt, per) in tl._TILES.items():
+        tiles = -(-M // (32 * fm)) * -(-N // (32 * fn))
+        if 32 * fm >= 2 * M + 64 or (fn == 2 and M > 400 and tiles > cus) or (fm <= 4 and fn == 4 and M > 2600):
+            continue
+        for S in tl._SPLITS:
+            if S > 1 and (K // S < tl._SPLIT_K or tiles * S > tl._SPLIT_TILES):
+                continue
+            both = sorted((-(-tiles * S // cus) * (-(-(K // 64) // S) * kt + per), 2 * N * K / tl._W_BYTES))
+            last = tl._SUM + 4 * M * N * S / tl._PART_BYTES if S > 1 else 2 * M * N / tl._OUT_BYTES
+            out.append((tl._LAUNCH + (both[1] + tl._OVERLAP * both[0]) + last, fm, fn, S))
+    return min(out, key=lambda c: c[0])[1:]
+
+
+def test_the_native_search_finds_the_cheapest_plan():
+    for M in (65, 96, 97, 400, 401, 1000, 2600, 2601, 8191):
+        for N, K in ((8, 64), (1088, 2048), (4096, 14336), (18560, 4096)):
+            for cus in (8, 256):
+                assert tl.tile_plan(M, N, K, cus) == _priced(M, N, K, cus)
+    with pytest.raises(ValueError):
+        tl.tile_plan(128, 256, 0)
+
+
+def test_a_new_row_count_costs_no_search_in_python():
+    """A server's prompt steps have another token count nearly every time: a plan that was not asked for before is some microseconds
+    (in Python 20 to 140)."""
+    def cost(plan, *args):
+        import time
+        best = 1.0
+        for _ in range(5):
+            t = time.perf_counter()
+            for M in range(500, 700):
+                plan.__wrapped__(M, *args)
+            best = min(best, (time.perf_counter() - t) / 200)
+        return best
+    assert cost(tl.tile_plan, 4096, 4096) < 12e-6
+    assert cost(tl.grouped_plan, 8, 4096, 4096) < 12e-6

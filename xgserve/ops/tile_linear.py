@@ -6,6 +6,7 @@ of the kernel's forms in the mean and 13 % at most.
 """
 from __future__ import annotations
 
+import array
 import functools
 from typing import Optional
 
@@ -31,30 +32,31 @@ PAIR_NONE, PAIR_HALVES, PAIR_BLOCKS = 0, 1, 2   # rows of a gated weight: [gate 
 TILE_ROWS_MIN = 65                          # (up to 64 rows the weights are streamed past them: rows_linear)
 
 
-@functools.lru_cache(maxsize=8192)
+def _table(kind: str, *rows):
+    """(address, entries) of numbers that stay for the process, for the native search."""
+    a = array.array(kind, [v for r in rows for v in r])
+    _KEPT.append(a)
+    return a.buffer_info()
+
+
+_KEPT: list = []
+_PRICES = _table("d", (_LAUNCH, _SUM, _W_BYTES, _PART_BYTES, _OUT_BYTES, _OVERLAP, _SPLIT_K, _SPLIT_TILES))[0]
+_TILE_ROWS = _table("d", *(t + p for t, p in _TILES.items()))[0]
+_SPLIT_ROWS = _table("i", _SPLITS)[0]
+
+
+@functools.lru_cache(maxsize=8192)   # (csrc/mixers/tile_plan.cpp: 2 us for a new size, 60 in Python)
 def tile_plan(M: int, N: int, K: int, cus: int = 256):
     """(rows / 32, columns / 32, parts of K) of an [M, K] . [N, K]^T product."""
-    best = None
-    for (fm, fn), (kt, per) in _TILES.items():
-        # (many small tiles read the weights and rows more often than this counts: those of 64 columns only while the chip holds
-        # them all, 512 x 2048 x 2048 11.7 us against 15.6 with 128 columns)
-        tiles = -(-M // (32 * fm)) * -(-N // (32 * fn))
-        if 32 * fm >= 2 * M + 64 or (fn == 2 and M > 400 and tiles > cus) or (fm <= 4 and fn == 4 and M > 2600):
-            continue
-        for S in _SPLITS:
-            if S > 1 and (K // S < _SPLIT_K or tiles * S > _SPLIT_TILES):
-                break
-            work = -(-tiles * S // cus) * (-(-(K // 64) // S) * kt + per)
-            load = 2 * N * K / _W_BYTES
-            t = _LAUNCH + max(work, load) + _OVERLAP * min(work, load)
-            t += _SUM + 4 * M * N * S / _PART_BYTES if S > 1 else 2 * M * N / _OUT_BYTES
-            if best is None or t < best[0]:
-                best = (t, fm, fn, S)
-    return best[1:]
+    return mixers().tile_plan(_TILE_ROWS, len(_TILES), _SPLIT_ROWS, len(_SPLITS), _PRICES, M, N, K, cus)
 
 
 # Tiles of the experts' products; offsets of all experts are looked through for a tile's, so there is a bound on their number
 _GROUPED, GROUPED_EXPERTS_MAX = ((8, 8), (7, 8), (6, 8), (4, 8), (6, 4), (4, 4), (3, 4)), 64
+_SHARES = (-1.2, -0.9, -0.6, -0.2, 0.2, 0.6, 0.9, 1.4)   # eight quantiles of an expert's rows, in units of their spread ...
+_SPREAD = 0.55                                            # ... from the mean, in units of the mean
+_GROUPED_ROWS = _table("d", *(t + _TILES[t] for t in _GROUPED))[0]
+_QUANTILES = _table("d", [z * _SPREAD for z in _SHARES])[0]
 
 
 @functools.lru_cache(maxsize=4096)
@@ -64,16 +66,7 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
     of the mean instead, tiles that just hold the mean were taken, and the larger experts' second ones made a round of their own. Cold
     weights, both products, router and shared expert, us: 8 experts of 2 x 2048 x 2048, 300 tokens 131 -> 124; of 2 x 3584 x 4096 256 ->
     241, 400 tokens 290 -> 276 (either product's change alone)."""
-    avg, best = pairs / E, None
-    for fm, fn in _GROUPED:
-        kt, per = _TILES[fm, fn]
-        rows = [max(1.0, avg + z * 0.55 * avg) for z in (-1.2, -0.9, -0.6, -0.2, 0.2, 0.6, 0.9, 1.4)]
-        tiles = E * sum(-(-r // (32 * fm)) for r in rows) / len(rows) * -(-N // (32 * fn))
-        work, load = -(-tiles // cus) * (K / 64 * kt + per), 2 * E * N * K / _W_BYTES
-        t = max(work, load) + _OVERLAP * min(work, load)
-        if best is None or t < best[0]:
-            best = (t, fm, fn)
-    return best[1:]
+    return mixers().grouped_plan(_GROUPED_ROWS, len(_GROUPED), _QUANTILES, len(_SHARES), _PRICES, pairs, E, N, K, cus)
 
 
 def library_better(M: int, N: int, K: int) -> bool:
