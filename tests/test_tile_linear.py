@@ -278,3 +278,18 @@ def test_a_new_row_count_costs_no_search_in_python():
         return best
     assert cost(tl.tile_plan, 4096, 4096) < 12e-6
     assert cost(tl.grouped_plan, 8, 4096, 4096) < 12e-6
+
+
+@pytest.mark.parametrize("plan,split,want", [((3, 2, 4), True, "parts"), ((8, 8, 1), True, "tiles"), (None, True, "split"),
+                                             (None, False, "torch")])
+def test_llama_down_asks_for_one_plan(plan, split, want, monkeypatch):
+    from xgserve.models import llama
+    asked, layer = [], llama.LlamaLayer.__new__(llama.LlamaLayer)
+    torch.nn.Module.__init__(layer)
+    layer.down = torch.zeros(64, 128)
+    monkeypatch.setattr(llama, "_tile_plan", lambda *a, **k: asked.append(k) or plan)
+    monkeypatch.setattr(llama, "splitk_prefill_ok", lambda *a: split)
+    for name, tag in (("tile_parts", "parts"), ("tile_linear", "tiles"), ("splitk_linear", "split")):
+        monkeypatch.setattr(llama, name, lambda *a, tag=tag: tag)
+    monkeypatch.setattr(llama.F, "linear", lambda *a: "torch")
+    assert layer._down(torch.zeros(70, 128)) == want and asked == [dict(plain=True)]

@@ -113,7 +113,10 @@ def _tile_plan(x: torch.Tensor, w: torch.Tensor, **kw):
 
 def _product(x: torch.Tensor, w: torch.Tensor, parts: bool = False):
     """x . w^T of a prompt-sized step, on the tile kernel or the library's; parts: a PendingSum where K is in parts."""
-    plan = _tile_plan(x, w, plain=True)
+    return _planned(_tile_plan(x, w, plain=True), x, w, parts)
+
+
+def _planned(plan, x: torch.Tensor, w: torch.Tensor, parts: bool):
     if plan is None:
         return F.linear(x, w)
     return tile_parts(plan, x, w) if parts and plan[2] > 1 else tile_linear(plan, x, w)
@@ -349,10 +352,12 @@ class LlamaLayer(nn.Module):
         return self._down(a)
 
     def _down(self, a: torch.Tensor):
-        """The down projection of a prompt-sized step on one GPU; parts of K are added by the next add + norm."""
-        if _tile_plan(a, self.down, plain=True) is None and splitk_prefill_ok(a, self.down):
+        """The down projection of a prompt-sized step on one GPU; parts of K are added by the next add + norm. Products that the tile
+        kernel leaves to torch (`forward_only`) run as torch's batched one over parts of K."""
+        plan = _tile_plan(a, self.down, plain=True)
+        if plan is None and splitk_prefill_ok(a, self.down):
             return splitk_linear(a, self.down, linear_mod.SPLITK_PREFILL_S)
-        return _product(a, self.down, parts=True)
+        return _planned(plan, a, self.down, parts=True)
 
     def _attend_prompt(self, h: torch.Tensor, meta: AttnMeta, kv, cos_sin) -> torch.Tensor:
         qkv = _product(h, self.qkv, parts=True)
