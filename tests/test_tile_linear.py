@@ -293,3 +293,78 @@ def test_llama_down_asks_for_one_plan(plan, split, want, monkeypatch):
         monkeypatch.setattr(llama, name, lambda *a, tag=tag: tag)
     monkeypatch.setattr(llama.F, "linear", lambda *a: "torch")
     assert layer._down(torch.zeros(70, 128)) == want and asked == [dict(plain=True)]
+
+
+# ---- workgroups that take tile after tile: the next tile's loads go out ahead of a whole tile's stores, which the waits then count.
+# A launch told of 3 compute units has several rounds at small sizes. K tiles of 64: fewer than a ring has slots, as many, more.
+_ROUNDS_K = (64, 192, 256, 384, 832)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("rotated", [False, True])     # (up to 256 rows column tiles start at different places in K)
+@pytest.mark.parametrize("K", _ROUNDS_K)
+def test_a_workgroup_takes_several_tiles(tile, rotated, K, monkeypatch):
+    monkeypatch.setattr(tl, "cu_count", lambda d: 3)
+    fm, fn = tile
+    M, N = 256 if rotated else max(32 * fm * 3, 288) + 5, 32 * fn * 7 + 8
+    assert -(-M // (32 * fm)) * -(-N // (32 * fn)) >= 8 and (M <= 256) == rotated
+    g = torch.Generator("cuda").manual_seed(K + fm)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device="cuda")
+    ref = x.double() @ w.double().t()
+    for S in (1, 2) if K >= 128 else (1,):
+        _close(tl.tile_linear((*tile, S), x, w), ref, K)
+        _close(tl.tile_linear((*tile, S), x, w, b), ref + b.double(), K)
+        if S > 1:
+            part = tl.tile_parts((*tile, S), x, w).part
+            # fp32 sums of K products (see _close)
+            assert ((part.double().sum(0) - ref).abs() <= K * 2.0 ** -24 * K ** 0.5 + 1e-6).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("rotated", [False, True])
+@pytest.mark.parametrize("K", _ROUNDS_K)
+def test_a_workgroup_takes_several_gated_tiles(tile, rotated, K, monkeypatch):
+    monkeypatch.setattr(tl, "cu_count", lambda d: 3)
+    fm, fn = tile
+    M, F_ = 256 if rotated else max(32 * fm * 3, 288) + 5, 16 * fn * 7 + 16
+    g = torch.Generator("cuda").manual_seed(K + fn)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(2 * F_, K, generator=g, device="cuda") * 3 * K ** -0.5).to(torch.bfloat16)
+    blocks = torch.stack([w[:F_].view(-1, 16, K), w[F_:].view(-1, 16, K)], 1).reshape(2 * F_, K)
+    z = x.double() @ w.double().t()
+    ref = sq._glu_ref(z[:, :F_], z[:, F_:], sq.GLU_SILU, 0.0, 0.0)
+    room = (1.5 * z[:, F_:].abs() + 1.5 * z[:, :F_].abs() + 2) * (3 * K ** 1.5 * 2.0 ** -24 + 2.0 ** -22)   # (as in test_gated_tiles)
+    for S in (1, 2) if K >= 128 else (1,):
+        for ww, pairs in ((w, tl.PAIR_HALVES), (blocks, tl.PAIR_BLOCKS)):
+            y = tl.tile_linear((*tile, S), x, ww, None, sq.ACT_GLU + sq.GLU_SILU, pairs=pairs).double()
+            assert ((y - ref).abs() <= 2.0 ** -8 * ref.abs() + room).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tl._GROUPED)
+@pytest.mark.parametrize("idle", [0, 9])     # experts without rows: with them 256 rows an expert are not reached, and columns rotate
+def test_grouped_workgroups_take_several_tiles(tile, idle, monkeypatch):
+    K, F_, W, top = 512, 512, 264, 1
+    share = [700, 32 * tile[0] * 2, 32 * tile[0], 300] + [0] * idle
+    E, T, g = len(share), sum(share), torch.Generator().manual_seed(tile[1])
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(share))[torch.randperm(T, generator=g)].view(T, 1).to(torch.int32)
+    assert (T > 256 * E) == (idle == 0)
+    h = torch.randn(T, K, generator=g).to(torch.bfloat16)
+    w13 = (torch.randn(E, 2 * F_, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    w2 = (torch.randn(E, W, F_, generator=g) * F_ ** -0.5).to(torch.bfloat16)
+    wts = torch.rand(T, top, generator=g)
+    monkeypatch.setattr(sq, "grouped_plan", lambda *a: tile)
+    monkeypatch.setattr(sq, "cu_count", lambda d: 3)
+    calls = record_native(monkeypatch, sq)
+    got = sq.routed_experts(h.cuda(), w13.cuda(), w2.cuda(), ids.cuda(), wts.cuda(), sq.GLU_SILU).cpu().double()
+    assert calls.count("tile_grouped") == 2
+    for e in range(4):
+        t = torch.nonzero(ids[:, 0] == e).view(-1)
+        z = h[t].double() @ w13[e].double().t()
+        a = sq._glu_ref(z[:, :F_], z[:, F_:], sq.GLU_SILU, 0.0, 0.0)
+        ref, size = wts[t].double() * (a @ w2[e].double().t()), wts[t].double() * (a.abs() @ w2[e].double().abs().t())
+        assert ((got[t] - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all()   # (as in test_grouped_tiles)
