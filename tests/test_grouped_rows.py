@@ -62,3 +62,12 @@ def test_modes(tm, N, K, T, E, top):
     lay = torch.full((cap, K), float("nan"), device="cuda", dtype=torch.bfloat16)   # padding rows may hold anything
     lay[d] = h[torch.arange(pairs, device="cuda") // top]
     check(run(lay, w1, rows, tile_e, tm, top, N, K, 0), a, 1.0, 2.0 ** -22)
+
+
+@pytest.mark.parametrize("T", [8, 200])
+def test_weights_in_front_of_a_gate_are_refused(T):
+    """Whatever the rows per expert: no gated form multiplies the product by the row's weight."""
+    h, w13 = torch.zeros(T, 128, device="cuda").bfloat16(), torch.zeros(2, 256, 128, device="cuda").bfloat16()
+    w2, ids = torch.zeros(2, 256, 128, device="cuda").bfloat16(), torch.zeros(T, 1, device="cuda", dtype=torch.int32)
+    with pytest.raises((ValueError, RuntimeError)):
+        sq.routed_experts(h, w13, w2, ids, torch.full((T, 1), 0.5, device="cuda"), sq.GLU_SILU, scale_input=True)

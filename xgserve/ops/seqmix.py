@@ -1343,8 +1343,9 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     streams = MOE_MFMA and h.dtype == torch.bfloat16 and K % 64 == 0 and F_ % 64 == 0
     tm = next((t for t, least in (MOE_TILES if streams else MOE_TILES_GENERAL) if pairs >= least * E), MOE_TILE_SMALL)
     # ... or run on gemm_pf's grouped form: both operands by LDS DMA, 64-row segments, 256-column tiles
-    pf = SEQ_MOE_PF and MOE_MFMA and gated and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E and K % 64 == 0 \
-        and F_ % 128 == 0 and W % 256 == 0
+    # (neither form weighs the rows in front of a gate: grouped_gemm refuses that)
+    pf = SEQ_MOE_PF and MOE_MFMA and gated and not scale_input and h.dtype == torch.bfloat16 and pairs >= MOE_PF_MIN * E \
+        and K % 64 == 0 and F_ % 128 == 0 and W % 256 == 0
     tiled = streams and gated and not scale_input and SEQ_MOE_PF and _experts_on_tiles(pairs, E, K, F_, W, T) \
         and (h.data_ptr() | w13.data_ptr() | w2.data_ptr()) % 16 == 0
     if pf or tiled:
@@ -1371,7 +1372,7 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
                           act.data_ptr(), 3, cfg, top, int(kind), float(limit), float(alpha), stream_ptr())
         M.gemm_pf_grouped(act.data_ptr(), 0, offs.data_ptr(), E, cap, F_, w2.data_ptr(), W, pairs, y.data_ptr(), 0, 1, cfg,
                           1, 0, 0.0, 0.0, stream_ptr())
-        return _routed_sum(M, y, dest, None if scale_input else wts, T, top, W, combine)
+        return _routed_sum(M, y, dest, wts, T, top, W, combine)
     M.grouped_gemm(h.data_ptr(), is_f32(h), h.stride(0), w13.data_ptr(), rows.data_ptr(), tile_e.data_ptr(), cap, tm, top,
                    F_, K, 1 if gated else 2, act.data_ptr(), int(kind), float(limit), float(alpha),
                    wts.data_ptr() if scale_input else 0, MOE_MFMA, stream_ptr())
