@@ -664,8 +664,8 @@ def test_router_softmax_over_the_chosen(device, T, E, top, W):
 @pytest.mark.parametrize("T,E,top,K,F_", [(7, 5, 2, 40, 24), (50, 1, 1, 32, 16), (300, 3, 3, 64, 48), (700, 4, 1, 96, 64),
                                           (1300, 4, 2, 128, 32), (64, 12, 1, 24, 10), (260, 2, 2, 256, 128)])
 def test_silu_gated_experts_and_their_sum(device, dtype, T, E, top, K, F_):
-    """Every grouped-GEMM path (16, 32, 64 and 128-row tiles, matrix-core, general, the prompt-sized form) against the dense
-    form, and the weighted sum of the chosen rows inside the layer-norm update."""
+    """Tiles of 16, 32, 64 and 128 rows, matrix-core, general and tile_linear's grouped form (by the rows per expert and the widths)
+    against the dense form, and the weighted sum of the chosen rows inside the layer-norm update."""
     dt = getattr(torch, dtype)
     g = torch.Generator().manual_seed(T + E)
     mlp = {"router": {"experts": E, "top": top}, "expert": {"ff": F_}}

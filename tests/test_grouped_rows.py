@@ -71,3 +71,33 @@ def test_weights_in_front_of_a_gate_are_refused(T):
     w2, ids = torch.zeros(2, 256, 128, device="cuda").bfloat16(), torch.zeros(T, 1, device="cuda", dtype=torch.int32)
     with pytest.raises((ValueError, RuntimeError)):
         sq.routed_experts(h, w13, w2, ids, torch.full((T, 1), 0.5, device="cuda"), sq.GLU_SILU, scale_input=True)
+
+
+@pytest.mark.parametrize("kind", [sq.GLU_GELU_TANH, sq.GLU_CLAMPED, sq.GLU_SILU])
+@pytest.mark.parametrize("E,top,K,F_,W,form", [(4, 2, 256, 128, 256, "gemm_pf_grouped"), (5, 1, 512, 384, 512, "gemm_pf_grouped"),
+                                               (66, 4, 128, 128, 256, "gemm_pf_grouped"),     # more experts than the tiles take
+                                               (4, 2, 256, 192, 128, "grouped_gemm"), (66, 4, 128, 64, 96, "grouped_gemm")])
+def test_gated_experts_that_the_tiles_do_not_take(kind, E, top, K, F_, W, form, monkeypatch):
+    """Many rows per expert on gemm_pf's grouped form and on the 128-row tiles, against fp64."""
+    from _seq_util import record_native
+    if E <= 64:
+        monkeypatch.setattr(sq, "GROUPED_EXPERTS_MAX", 0)
+    T = -(-140 * E // top)
+    g = torch.Generator("cuda").manual_seed(E + F_)
+    h = torch.randn(T, K, generator=g, device="cuda").bfloat16()
+    w13 = (torch.randn(E, 2 * F_, K, generator=g, device="cuda") * 2 * K ** -0.5).bfloat16()
+    w2 = (torch.randn(E, W, F_, generator=g, device="cuda") * F_ ** -0.5).bfloat16()
+    ids = torch.rand(T, E, generator=g, device="cuda").topk(top, -1).indices.to(torch.int32)
+    wts = torch.rand(T, top, generator=g, device="cuda")
+    calls = record_native(monkeypatch, sq)
+    got = sq.routed_experts(h, w13, w2, ids, wts, kind, 2.0, 1.702).double()
+    assert calls.count(form) == 2 and "tile_grouped" not in calls
+    ref, size = torch.zeros_like(got), torch.zeros_like(got)
+    for e in range(E):
+        t, j = torch.nonzero(ids == e, as_tuple=True)
+        z = h[t].double() @ w13[e].double().t()
+        a = sq._glu_ref(z[:, :F_], z[:, F_:], kind, 2.0, 1.702)
+        ref.index_add_(0, t, wts[t, j, None].double() * (a @ w2[e].double().t()))
+        size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
+    # activations in bf16 (2^-9 of each term), sums in fp32
+    assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())

@@ -624,7 +624,8 @@ def test_clamped_gate_of_dense_layers(device, dtype, T, ff, limit):
                                           (700, 4, 1, 96, 64), (1300, 4, 2, 128, 32), (64, 12, 1, 24, 10),
                                           (900, 4, 2, 256, 128), (300, 3, 3, 256, 256), (2100, 5, 1, 512, 384)])
 def test_routed_experts_with_a_clamped_gate(device, dtype, T, E, top, K, F_):
-    """Every grouped-GEMM path; softmax weights at the output; the sum over choices inside the residual write."""
+    """Tiles of 16 to 128 rows, general kernels and tile_linear's grouped form (by the rows per expert and the widths); softmax weights
+    at the output; the sum over choices inside the residual write."""
     dt = getattr(torch, dtype)
     g = torch.Generator().manual_seed(T + E)
     mlp = {"router": {"experts": E, "top": top}, "expert": {"ff": F_, "limit": 0.8}}
