@@ -5,7 +5,8 @@
 //
 // Bound by the matrix cores from some 400 rows on, by the weights' bytes below. A workgroup of four waves, one per SIMD, owns a tile
 // of 32 FM rows and 32 FN weight rows, 2 x 2 waves of 16 FM x 16 FN: with 128 x 128 products a wave reads 32 fragments from LDS per
-// 128 matrix instructions, half of what eight waves read for the same tile, and its accumulators fill the 256 accumulation registers.
+// 128 matrix instructions (the tile 64 per 32 of K; eight waves of 128 x 64 read 96), and its accumulators fill the 256 accumulation
+// registers.
 // x and w come in by LDS DMA, 64 of K at a time, into a ring of RA and RW slots (160 KB for the large tiles: two of x, three of w,
 // whose first reader waits for HBM). A K tile is two steps, one per 32 of K. Between the products of a step the other step's fragments
 // are read (into the registers that the step before has used up) and, once the K tile's slots are free, the tiles RA and RW further on
@@ -71,7 +72,10 @@ __device__ __forceinline__ void tile_dma(const void* base, uint32_t off, uint32_
 }
 
 // acc += w . x^T in accumulation registers. (From the builtin hipcc moves accumulators between the two register files inside the
-// loop, some 100 moves per 64 products. No product here reads what one of the 12 before it writes; what follows the loop waits.)
+// loop, some 100 moves per 64 products. It puts no waits between these: an accumulator is read again by the same instruction on the
+// same registers, which takes two wait states at most, and FM FN - 1 other products lie between, kMfmaApart at least; what follows the
+// loop waits.)
+constexpr int kMfmaApart = 5;
 __device__ __forceinline__ void tile_mfma(f32x4_t& acc, bf16x8_t w, bf16x8_t x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
@@ -102,8 +106,8 @@ template <int ACT>
 __device__ __forceinline__ float tile_act(const TileArgs& a, float v) {
   return ACT == kTileXielu ? xieluf(v, a.p0, a.p1) : ACT == kTileRelu2 ? relu2f(v) : v;
 }
-// glu.h's gates for a bf16 result, whose rounding is 2^-9: the exponential and reciprocal instructions (2^-23 each) instead of expf and a
-// division, 20 instructions an output instead of 45. A tile's gates run on four waves while its matrix cores wait: 8192 x 16384 x 2048
+// glu.h's gates for a bf16 result, whose rounding is 2^-9: the exponential and reciprocal instructions (2^-23 each, and 2^-24 of the
+// exponent from its rounding) instead of expf and a division, 20 instructions an output instead of 45. A tile's gates run on four waves while its matrix cores wait: 8192 x 16384 x 2048
 // 440 -> 405 us, 2521 rows 152 -> 141, 8192 x 28672 x 4096 1381 -> 1319. Error of the result against fp64 over gates and factors of spread
 // 0.3, 1 and 3: 1.649554e-3, 1.660321e-3, 1.654740e-3 (tanh-GELU; the others likewise), the same to seven digits as with those.
 template <int KIND>
@@ -135,6 +139,7 @@ __global__ __launch_bounds__(256, OCC) void tile_linear_kernel(const TileArgs a)
   constexpr int ST = FM * FN / 2;   // stores of a whole tile (fp32 parts: twice that)
   constexpr int RS = FM * FN >= 2 * LD ? 3 * FM * FN / 4 / LD : 1, DS = FM * FN / LD;   // products between two reads (the last has a quarter to land), two loads
   static_assert(RS >= 1 && DS >= 1, "a step's reads and loads fit between its products");
+  static_assert(FM * FN > kMfmaApart, "products on the same accumulators keep their distance");
   // loads behind the last one that the next tile needs (A of RA tiles ahead and then W of RW tiles ahead are asked for per tile)
   constexpr int CA = FN + (RA - 2) * LD, CW = (RW - 2) * LD, CNT = CA < CW ? CA : CW;
   constexpr int CA0 = FN + (RA - 1) * LD, CW0 = (RW - 1) * LD, CNT0 = CA0 < CW0 ? CA0 : CW0;   // ... and that tile 0 needs

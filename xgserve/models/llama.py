@@ -63,13 +63,13 @@ FUSED_DECODE = tune.get_bool("fused_decode", True)
 # 64 < T <= this many tokens (the mixed step: decode rows + one bounded prefill chunk)
 # run every projection on gemm_mw (csrc/kernels/gemm_mw.hip): weight-stream-bound
 # MFMA GEMMs whose split-K partials go to the consumers, SiLU-gate in gate_up.
-# 0 = hipBLASLt for every step above 64 tokens.
+# 0 = prompt-sized forms (ops.tile_linear or the library) for every step above 64 tokens.
 MW_MAX_TOKENS = min(MW_MAX_M, tune.get_int("mw_max_tokens", MW_MAX_M))
 # Prompt-sized mixed steps on TP = 1: each projection takes gemm_pf
-# (csrc/kernels/gemm_pf.hip) for the step sizes where it measured faster than the
-# tuned library GEMM (profiles/r6/r6p_pf_vs_library.md, cold weights, the engine's
-# library forms) -- QKV / O / down as split-K partials into their consumers, gate_up
-# with the SiLU gate in its epilogue:
+# (csrc/kernels/gemm_pf.hip) for the step sizes where it measured faster than
+# ops.tile_linear (gate_up) or the tuned library GEMM (profiles/r6/r6p_pf_vs_library.md,
+# cold weights, the engine's library forms) -- QKV / O / down as split-K partials into
+# their consumers, gate_up with the SiLU gate in its epilogue:
 #   gate_up 513-576 rows: two 288-row tiles cover the step (121 us at 575 rows, where two
 #     rounds of the 192-row tiles of ops.tile_linear take 138); up to 512 rows two 256-row
 #     tiles of that kernel do (104 us against 109 here);
@@ -79,7 +79,7 @@ MW_MAX_TOKENS = min(MW_MAX_M, tune.get_int("mw_max_tokens", MW_MAX_M))
 #     vs 11,694 tok/s with down on pf (r6p_pf_vs_library.md);
 #   QKV / O: never -- pf's isolated lead is smaller than the fp32 partial slabs it adds
 #     to their consumers (r5: -0.5 % end to end with every projection on pf).
-# XGS_TUNE pf: "1" = these windows, "0" = library everywhere, or a comma list of
+# XGS_TUNE pf: "1" = these windows, "0" = gemm_pf nowhere, or a comma list of
 # projections to allow; pf_windows overrides the table ("gate_up:513-576/down:321-576").
 PF_WINDOWS_DEFAULT = "gate_up:513-576/down:513-576"
 
@@ -442,7 +442,7 @@ class LlamaLayer(nn.Module):
         if use_pf:
             # prompt-sized mixed steps: gemm_pf for the projections whose measured window
             # holds T (split-K partials into the consumers: rope_cache_partials / add +
-            # rmsnorm; the SiLU gate in the gate_up epilogue), the library GEMMs for the others
+            # rmsnorm; the SiLU gate in the gate_up epilogue), tile_linear or the library for the others
             if "qkv" in use_pf:
                 a = self.attn.from_partials(pf_linear(h, self.qkv, MODE_PARTIAL), meta, kv, cos_sin)
             else:
@@ -480,7 +480,8 @@ class LlamaLayer(nn.Module):
         the following chunk: O GEMM(c) -> AR(c) async; then per chunk: wait AR(c)
         -> add + post-norm -> gate_up -> SiLU-gate -> down(c) -> AR(c) async. Only
         the last chunk's down all-reduce is exposed. Everything after attention is
-        per-token, so the chunked result equals the unchunked one exactly."""
+        per-token; the products are torch's (into the all-reduce's buffers), the unchunked
+        step's ops.tile_linear's where that is faster, so both agree to their rounding."""
         T, H = residual.shape
         eps = self.cfg.norm_eps
         n = TP_OVERLAP_CHUNKS

@@ -1172,7 +1172,7 @@ GLU_GELU_TANH, GLU_CLAMPED, GLU_SILU = 0, 1, 3
 ACT_RELU2 = 2   # routed_experts(kind=...): an expert without a gate, W_down relu(W_up h)^2
 # XGS_TUNE moe_mfma=0: the general grouped GEMM for bf16 too (A/B and tests)
 MOE_MFMA = tune.get_bool("moe_mfma", True)
-# XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on the tiles of csrc/mixers (A/B and tests)
+# XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on grouped_gemm (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
 # Average rows per expert from which gated experts run on the tiles of tile_linear.hip: up to there most segments fit one tile of 64
 # rows of the weight-streaming products, and experts of less than MOE_TILED_ELEMS gate and up weights stay on those up to where

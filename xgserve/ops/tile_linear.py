@@ -75,8 +75,11 @@ def library_better(M: int, N: int, K: int) -> bool:
     4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81), as long as no columns are left over beside its tiles of
     256 (10304x2048, 4001 rows 168 against 129; 18560x4096, 2048 rows 344 against 257) and there are 150 such tiles (2048x8192, 2521
     rows 77 to 81 against 75; up to 1792 rows 4096x14336, 1536 rows 168 against 140; 6144x4096, 700 rows 45 against 41). Its narrow
-    products of few rows are 1 to 2 us faster on the card (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4), but such
-    steps wait for the host, of which the library's call takes 31 us and this kernel's 10."""
+    products of few rows are 1 to 2 us faster on the card (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4; 4096x4096,
+    256 rows 23.1 against 27.8), and some of middle size by 2 to 9 (6144x4096, 512 rows 38.2 against 40.8; 18560x4096, 400 rows 71
+    against 80), but not in steps. Eager ones of few rows wait for the host, of which the library's call takes 31 us and this kernel's
+    10: with the faster of both for every product, 96 rows, Vizonex "1b" 868 -> 1159 us, Dofivik 1300 -> 1507; from 400 rows on within
+    1 %. Replayed ones of 96 and 160 rows are up to 2 % slower with it, of 256 rows up to 2 % faster."""
     return N % 256 == 0 and M > 1792 and -(-M // 256) * (N // 256) >= 150
 
 
