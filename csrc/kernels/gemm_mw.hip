@@ -41,7 +41,7 @@ int k_rotation(int S);  // gemm_m64g.hip
 
 enum : int { MW_BF16 = 0, MW_PARTIAL = 1, MW_SILU = 2 };
 
-// PR: anatomy-probe code paths of round 4 (profiles/r4_mw_probe.md), now always 0:
+// PR: anatomy-probe code paths (profiles/r4_mw_probe.md), now always 0:
 // PR & 7 selects compiled-out pipeline parts, PR & 8 forces K rotation.
 template <int WN, int NWT, int MTW, int D, bool NT, int PR = 0>
 __global__ void __launch_bounds__(512, 1) gemm_mw_kernel(const uint16_t* __restrict__ x, int M, int K,
@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(512, 1) gemm_mw_kernel(const uint16_t* __restr
   }
 }
 
-// (Measured and removed in round 5 -- records kept in profiles/: the split-role rings
+// (Measured and removed -- records kept in profiles/: the split-role rings
 // "gemm_mw2" (waves 0-3 weights, 4-7 x; r4_mw_sweep.md, r4_mw2_sweep.jsonl) and the
 // software-pipelined "gemm_mw3" (one ring of whole chunks, reads of chunk c + 1 under
 // chunk c's MFMAs; r4_mw_sweep_v1.jsonl) never beat the kernel above on a default plan,

@@ -34,7 +34,7 @@ def _run(nproc, *args, launcher=True):
     if launcher:
         cmd = [sys.executable, "-m", "torch.distributed.run", "--nnodes=1", f"--nproc-per-node={nproc}",
                "--master-addr", "127.0.0.1", "--master-port", str(_free_port()), str(ROOT / "bench.py")]
-    else:  # bench.py spawns its own ranks (the driver's `python bench.py --gpus N` form)
+    else:  # bench.py spawns its own ranks (the `python bench.py --gpus N` form)
         cmd = [sys.executable, str(ROOT / "bench.py")]
     cmd += ["--gpus", str(nproc), *SMALL, *args]
     p = subprocess.run(cmd, cwd=ROOT, env=_env(), capture_output=True, text=True, timeout=240)
@@ -49,7 +49,7 @@ def _run(nproc, *args, launcher=True):
 def test_bench_multi_rank_json_contract(nproc, tp, model, par):
     r = _run(nproc, "--tp", str(tp), "--model", model, *(["--allow-rccl-decode"] if tp > 1 else []))
     _check_contract(r, nproc, model, par, tp)
-    # pre-flight evidence (VERDICT r4 #4): the communicator formed at world N and summed
+    # pre-flight evidence: the communicator formed at world N and summed
     # correctly, the TP groups, and which library carried the TP decode all-reduce
     assert r["rccl_world"] == nproc
     assert r["tp_groups"] == [list(range(g, g + tp)) for g in range(0, nproc, tp)]

@@ -1,4 +1,4 @@
-"""The round-3 serving fixes, end to end:
+"""Serving fixes, end to end:
 
 * an HTTP/1.0 client asking for `stream: true` gets a clean close-delimited SSE
   body (no chunk-size lines: the pre-framed HTTP/1.1 wire path is only for chunked

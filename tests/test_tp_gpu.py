@@ -1,5 +1,5 @@
 """Tensor parallelism on the MI355X kernels: TP=2 as two processes sharing the one
-GPU of a gpurun box (per-rank shards of real Llama-3-8B layer shapes loaded from
+GPU of a machine (per-rank shards of real Llama-3-8B layer shapes loaded from
 a safetensors checkpoint; gloo carries the plan broadcast and the RCCL-shaped
 collectives, the one-shot IPC all-reduce carries the decode all-reduces).
 

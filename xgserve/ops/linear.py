@@ -103,7 +103,7 @@ M64G_SMALL_ONLY = (8, 9, 10)
 # down 22.9 -> 19.2 us); the rest keep the skinny kernel.
 _M64_TUNED = {
     # Llama-3-8B / Mixtral attention, TP1
-    # 16 / 32 re-swept with K rotation in round 4 (profiles/r4_m64g_sweep_m1.jsonl; 64: r4_m64g_sweep_rot.jsonl)
+    # 16 / 32 re-swept with K rotation (profiles/r4_m64g_sweep_m1.jsonl; 64: r4_m64g_sweep_rot.jsonl)
     (6144, 4096, MODE_PARTIAL): {64: (2, 5, 3), 32: (1, 5, 7), 16: (1, 2, 9)},
     (4096, 4096, MODE_PARTIAL): {64: (1, 4, 0), 32: (1, 4, 0), 16: (1, 3, 0)},
     # bucket 16: the fused (row-scaled) form's sweep, r6/r6_fused_plans.md (batch 1 +3 %)
@@ -116,7 +116,7 @@ _M64_TUNED = {
     (8192, 8192, MODE_PARTIAL): {64: (1, 2, 1), 32: (2, 8, 7), 16: (1, 1, 9)},  # 8-wave tile: 23.3 vs 24.8-25.7 us
     (57344, 8192, MODE_SILU): {64: (2, 1, 7), 32: (2, 1, 7), 16: (2, 1, 7)},  # 8-wave tile: 148 vs 166-178 us
     (8192, 28672, MODE_PARTIAL): {64: (2, 4, 1), 16: (1, 2, 1)},
-    # 70B shards re-swept with K rotation in round 4 at M = 1 / 64 (profiles/r4_m64g_sweep_tp.jsonl)
+    # 70B shards re-swept with K rotation at M = 1 / 64 (profiles/r4_m64g_sweep_tp.jsonl)
     # TP shards (Llama-3-8B / Mixtral attention TP2/4/8, Llama-3-70B TP2/4/8), re-swept at
     # M = 1 / 16 (bucket 16: best sum), 32, 64 (profiles/r2_tp_shard_sweep.jsonl); gate_up
     # shards with split-K SiLU (S > 1) and the 8-wave cfg 7: profiles/r2_silu_split_sweep.jsonl
@@ -242,8 +242,8 @@ def m64_linear(x: torch.Tensor, w: torch.Tensor, mode: int = MODE_PARTIAL, split
 # by LDS-DMA, split-K partials for grids that would not fill the chip.
 # cfg -> (columns per workgroup, weight ring depth, non-temporal weight DMA)
 # (0-4: 4 x 2 waves as N x M; 5-6: 2 x 4 waves -- fewer LDS fragment reads per MFMA.
-# The split-role and software-pipelined families of round 4 (cfg 7-21) never won a
-# default plan and were removed in round 5; their sweeps stay in profiles/r4_mw*.)
+# The split-role and software-pipelined families (cfg 7-21) never won a
+# default plan and were removed; their sweeps stay in profiles/r4_mw*.)
 MW_CFGS = {0: (256, 2, True), 1: (128, 3, True), 2: (128, 2, True), 3: (256, 2, False), 4: (128, 3, False),
            5: (128, 3, True), 6: (256, 2, True)}
 MW_MAX_M = 320   # M > 256 (a 320-row x tile) fits the LDS on cfg 2 only
