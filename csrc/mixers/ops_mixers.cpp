@@ -71,7 +71,7 @@ int tile_linear(const void*, int64_t, const void*, const void*, bool, float*, vo
 int tile_grouped(const void*, int64_t, int, const int32_t*, const int32_t*, int, int, const void*, float*, void*, int, int, int, int, float,
                  float, int, int, int, hipStream_t);
 int rows_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int*, int, int, int, int, int, float, float,
-                bool, hipStream_t);
+                int, hipStream_t);
 int64_t delta_chunk_scratch_floats(int, int, int, int);
 int delta_chunk(const void*, bool, int64_t, int, int, int, int, const void*, int64_t, const float*, const float*, float*,
                 const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, float*, hipStream_t);
@@ -401,10 +401,10 @@ PYBIND11_MODULE(_mixers, m) {
           "tile_grouped");
   });
   m.def("rows_linear", [](uintptr_t x, int64_t ld_x, uintptr_t w, uintptr_t bias, bool bias_f32, uintptr_t part,
-                          uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, bool wide,
+                          uintptr_t out, uintptr_t tickets, int T, int N, int K, int S_, int act, float p0, float p1, int cols,
                           uintptr_t st) {
     check(xgm::rows_linear(P<const void>(x), ld_x, P<const void>(w), P<const void>(bias), bias_f32, P<float>(part),
-                           P<void>(out), P<int>(tickets), T, N, K, S_, act, p0, p1, wide, S(st)),
+                           P<void>(out), P<int>(tickets), T, N, K, S_, act, p0, p1, cols, S(st)),
           "rows_linear");
   });
   m.def("delta_chunk_scratch_floats",

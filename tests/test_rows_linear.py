@@ -162,3 +162,37 @@ def test_nan_through_the_squared_relu_whatever_the_rows(T, dtype):
         ids = (torch.arange(T, device="cuda") % E).to(torch.int32)[:, None].contiguous()
         o = sq.routed_experts(h, up, down, ids, torch.ones(T, 1, device="cuda"), sq.ACT_RELU2)
         assert bool(o[5].isnan().all()) and bool(o[rows].isfinite().all()), (E, K)
+
+
+def test_whole_tiles_fit_one_round_and_parts_stay_where_they_cost_less():
+    for T in (1, 16, 17, 33, 49, 64):
+        for N in [*range(8, 20000, 56), 32000, 128256]:
+            for K in (128, 768, 2048, 4096, 8192, 14336):
+                for gated in (False, True):
+                    wide, S = sq._rows_plan(N, K, gated)
+                    cols = sq._rows_cols(T, N, K, gated, wide, S)
+                    assert cols == (128 if wide else 64) or (cols in ((32, 64) if gated else (16, 32, 48)) and -(-N // cols) <= 256)
+    assert [sq._rows_cols(T, 2048, K, False, *sq._rows_plan(2048, K, False)) for T, K in ((64, 2048), (64, 8192), (1, 2048))] == \
+        [16, 64, 16]
+
+
+@gpu
+@pytest.mark.parametrize("N,K,cols", [(4, 128, 16), (2052, 1152, 16), (4092, 640, 16), (4100, 256, 32), (8188, 640, 32), (8196, 128, 48),
+                                      (12284, 384, 48), (8, 256, -32), (2056, 1152, -32), (8184, 128, -32), (8200, 640, -64),
+                                      (16376, 128, -64)])
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 48, 49, 64])
+def test_whole_tiles(T, N, K, cols, monkeypatch):
+    """Tiles of 16 to 64 weight rows over the whole K (cols < 0: gated): partial tiles, fewer chunks than the ring, more than it."""
+    calls = record_native(monkeypatch, sq)
+    g, x, w, sm = data(T, N, K, N + T)
+    z, mag = x.double() @ w.double().t(), float((x.double().abs() @ w.double().abs().t()).max())
+    assert sq._rows_plan_of(x, w, sm, None, cols < 0) == (abs(cols), 1)
+    if cols < 0:
+        a, u = z[:, :N // 2], z[:, N // 2:]
+        check(sq.linear_glu(x, w, sq.GLU_SILU, sm=sm), a * torch.sigmoid(a) * u, mag, K, 3 * float(z.abs().max()) + 3)
+    else:
+        check(sq.linear(x, w, sm), z, mag, K, 1.0)
+        b = torch.randn(N, generator=g).cuda()
+        v = z + b.double()
+        check(sq.linear_relu2(x, w, b, sm), v.clamp(min=0) ** 2, mag + 8, K, 2 * float(v.abs().max()) + 2)
+    assert calls == ["rows_linear"] * (1 if cols < 0 else 2)

@@ -123,9 +123,21 @@ def _rows_plan(N: int, K: int, gated: bool):
     return wide, S
 
 
+def _rows_cols(T: int, N: int, K: int, gated: bool, wide: bool, S: int) -> int:
+    """Weight rows of a workgroup: 128 (`wide`) or 64 of one of S parts of K, or fewer of the whole K. Costs of a workgroup as
+    rows_linear.hip has them, 6.5e-5 us each: (0.4 rows of x + columns) K, and for parts that meet 15000 + 25000 a tile of 16
+    rows (measured 1.5 us at one row, 3.5 to 5 at 64). Tiles that leave one round of workgroups only: a second one doubles the time."""
+    x, tiles = 0.4 * 16 * -(-T // 16), -(-T // 16)
+    parts = (x + (128 if wide else 64)) * K / S + (15000 + 25000 * tiles if S > 1 else 0)
+    for cols in ((32, 64) if gated else (16, 32, 48)):
+        if -(-N // cols) <= _ROWS_WGS:
+            return cols if (x + cols) * K < parts else 128 if wide else 64
+    return 128 if wide else 64
+
+
 def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias: Optional[torch.Tensor], gated: bool,
                   slabs: bool = False):
-    """The plan of x . w^T on the kernel of a few rows, or None: bfloat16 on the current device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
+    """(weight rows of a workgroup, parts of K) of x . w^T on the kernels of a few rows, or None: bfloat16 on the current device, 1 to ROWS_LINEAR_MAX rows of whole 16-byte
     pieces, K in whole staged rows, nothing that wants a derivative, and tickets where K is in parts (clearing them would cost
     what the parts gain) unless the `slabs` are the result. What is refused here goes to torch, which refuses what it cannot do."""
     if not (native_device(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
@@ -139,16 +151,21 @@ def _rows_plan_of(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta], bias:
     if bias is not None and not (bias.device == x.device and bias.dtype in (torch.float32, torch.bfloat16) and bias.shape == (N,)
                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return None
-    plan = _rows_plan(N, K, gated)
-    return plan if slabs or plan[1] == 1 or (sm is not None and sm.tickets is not None) else None
+    wide, S = _rows_plan(N, K, gated)
+    if slabs:
+        return 128 if wide else 64, S
+    if S > 1 and (sm is None or sm.tickets is None):
+        return None
+    cols = _rows_cols(x.shape[0], N, K, gated, wide, S)
+    return cols, 1 if cols < (128 if gated else 64) else S
 
 
 def _rows_linear(plan, x, w, sm, bias, act, p0, p1) -> torch.Tensor:
-    T, (N, K), (wide, S) = x.shape[0], w.shape, plan
+    T, (N, K), (cols, S) = x.shape[0], w.shape, plan
     out = torch.empty(T, N // 2 if act >= ACT_GLU else N, dtype=x.dtype, device=x.device)
     part = torch.empty(S * T * N, dtype=torch.float32, device=x.device) if S > 1 else None
     mixers().rows_linear(x.data_ptr(), x.stride(0), w.data_ptr(), _p(bias), bias is not None and is_f32(bias), _p(part),
-                         out.data_ptr(), _p(sm.tickets) if S > 1 else 0, T, N, K, S, act, float(p0), float(p1), wide,
+                         out.data_ptr(), _p(sm.tickets) if S > 1 else 0, T, N, K, S, act, float(p0), float(p1), cols,
                          stream_ptr())
     return out
 
@@ -181,10 +198,10 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None)
     if sm is not None and sm.parts:
         plan = _rows_plan_of(x, w, sm, None, False, slabs=True)
         if plan is not None and plan[1] > 1:
-            T, (N, K), (wide, S) = x.shape[0], w.shape, plan
+            T, (N, K), (cols, S) = x.shape[0], w.shape, plan
             part = torch.empty(S, T, N, dtype=torch.float32, device=x.device)
             mixers().rows_linear(x.data_ptr(), x.stride(0), w.data_ptr(), 0, False, part.data_ptr(), 0, 0, T, N, K, S, ACT_NONE,
-                                 0.0, 0.0, wide, stream_ptr())
+                                 0.0, 0.0, cols, stream_ptr())
             return Parts(part)
     return linear(x, w, sm)
 
