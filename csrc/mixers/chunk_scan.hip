@@ -8,7 +8,7 @@
 // whatever the grid. With s_t the product of the decays behind token t up to the chunk's end and E that of all of them, a chunk is
 //   S' = E S,   P_ij = sum_d (q_i / s_i) (k_j s_j) (j <= i),   o = P v + (q / s) S',   S <- S' + (k s)^T v
 // and a scalar decay (ssm) factors out of the sums: P_ij = C_i . B_j dt_j s_j / s_i, no factor above 1 at all. Everything stays
-// fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32 (operands split into two bf16 terms would lose bits) and the products
+// fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32 (bf16 rows of the second run in ssm_chunk.hip) and the products
 // of decays are carried as two floats (Prod). Referred to the chunk's end, the terms that enter the state have one rounding each,
 // as in the token loop; their reciprocals meet the outputs alone, where what came in goes first and the chunk's terms follow in
 // their order (summed apart and added, decays around 0.5 had 1.05 to 1.17 times the loop's error, so 0.97 to 1.10).

@@ -79,6 +79,9 @@ int64_t chunk_scan_scratch_floats(int, int, int, int, int, int);
 int chunk_scan_gates(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*,
                      const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int,
                      int, int, int, int, float*, hipStream_t);
+int64_t ssm_chunk_scratch_floats(int, int, int, int, int, int);
+int ssm_chunk(const void*, int64_t, const void*, int64_t, const float*, const float*, const float*, float*, const int32_t*,
+              const int32_t*, const int32_t*, float*, int, int, int, int, int, int, int, int, float*, hipStream_t);
 int chunk_scan_ssm(const void*, bool, int64_t, const void*, int64_t, const float*, const float*, const float*, float*,
                    const int32_t*, const int32_t*, const int32_t*, float*, int, int, int, int, int, int, int, int, float*,
                    hipStream_t);
@@ -439,13 +442,21 @@ PYBIND11_MODULE(_mixers, m) {
                                    P<float>(o), ns, max_q, T, H, dk, dv, seg, P<float>(scratch), S(st));
     check(rc, "chunk_scan_gates");
   });
+  m.def("ssm_chunk_scratch_floats", [](int T, int ns, int H, int N, int Pd, int seg) {
+    if (seg < 1) throw std::invalid_argument("ssm_chunk_scratch_floats: seg must be positive");
+    return xgm::ssm_chunk_scratch_floats(T, ns, H, N, Pd, seg);
+  });
   m.def("chunk_scan_ssm", [](uintptr_t xbc, bool f32, int64_t ld_x, uintptr_t dt, int64_t ld_dt, uintptr_t dt_bias,
                              uintptr_t A_log, uintptr_t D, uintptr_t state, uintptr_t qsl, uintptr_t sl, uintptr_t slots,
                              uintptr_t y, int ns, int max_q, int T, int H, int G, int N, int Pd, int seg, uintptr_t scratch,
-                             uintptr_t st) {
+                             bool split, uintptr_t st) {
     if (H < 1 || G < 1 || ld_x < (int64_t)H * Pd + 2 * (int64_t)G * N || ld_dt < H)
       throw std::invalid_argument("chunk_scan_ssm: inconsistent sizes");
-    int rc = xgm::chunk_scan_ssm(P<const void>(xbc), f32, ld_x, P<const void>(dt), ld_dt, P<const float>(dt_bias),
+    if (split && f32) throw std::invalid_argument("chunk_scan_ssm: chunks of 64 tokens take bfloat16 rows");
+    int rc = split ? xgm::ssm_chunk(P<const void>(xbc), ld_x, P<const void>(dt), ld_dt, P<const float>(dt_bias), P<const float>(A_log),
+                                    P<const float>(D), P<float>(state), P<const int32_t>(qsl), P<const int32_t>(sl),
+                                    P<const int32_t>(slots), P<float>(y), ns, max_q, T, H, G, N, Pd, seg, P<float>(scratch), S(st))
+                   : xgm::chunk_scan_ssm(P<const void>(xbc), f32, ld_x, P<const void>(dt), ld_dt, P<const float>(dt_bias),
                                  P<const float>(A_log), P<const float>(D), P<float>(state), P<const int32_t>(qsl),
                                  P<const int32_t>(sl), P<const int32_t>(slots), P<float>(y), ns, max_q, T, H, G, N, Pd, seg,
                                  P<float>(scratch), S(st));

@@ -1,0 +1,100 @@
+"""State-space chunks of 64 tokens (csrc/mixers/ssm_chunk.hip) against the token loop in fp64.
+
+Tolerance: as in test_chunk_scan.py, 2e-5 of the output's root mean square for some 2^-24 of a term's size per token that it
+remembers. How the errors compare with the fp32 token loop's own is tested apart, with a tenth for another order of the sums."""
+import math
+
+import pytest
+import torch
+
+from xgserve.ops import seqmix as sq
+
+from _seq_util import record_native
+from test_chunk_scan import F64, close, error, layout, scan
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(portions, H, G, N, P, level, seed):
+    g = torch.Generator().manual_seed(seed)
+    T = sum(n for _, n in portions)
+    xbc = torch.nn.functional.silu(torch.randn(T, H * P + 2 * G * N, generator=g)).bfloat16()
+    dt = torch.randn(T, H, generator=g).bfloat16()
+    return (xbc, dt, torch.randn(H, generator=g) * 0.5 - 1, torch.randn(H, generator=g) * 0.3 + level, torch.randn(H, generator=g),
+            torch.randn(len(portions) + 1, H, N, P, generator=g))
+
+
+def run(args, portions, H, G, N, P):
+    xbc, dt, bias, A, D, state = (t.cuda() for t in args)
+    out = sq.ssm_scan(xbc, dt, bias, A, D, state, H, G, N, P, layout(portions))
+    return out, state
+
+
+def reference(args, portions, H, G, N, P):
+    xbc, dt, bias, A, D, state = args
+    T = xbc.shape[0]
+    d = torch.nn.functional.softplus(dt.to(F64) + bias.to(F64))
+    f = torch.exp(-torch.exp(A.to(F64)) * d)[..., None].expand(T, H, N)
+    z = xbc.to(F64)
+    x = z[:, :H * P].view(T, H, P)
+    B, C = (z[:, H * P + i * G * N:H * P + (i + 1) * G * N].view(T, G, N).repeat_interleave(H // G, 1) for i in (0, 1))
+    out, states, at = [], [], 0
+    for i, (ctx, n) in enumerate(portions):
+        r = slice(at, at + n)
+        o, S = scan(C[r], f[r], d[r][..., None] * B[r], x[r], state[i + 1].to(F64) * (ctx > 0))
+        out.append(o + D.to(F64)[:, None] * x[r])
+        states.append(S)
+        at += n
+    return torch.cat(out).reshape(T, H * P), states
+
+
+@pytest.mark.parametrize("portions", [[(0, 16)], [(3, 63), (0, 64)], [(0, 65), (9, 1), (2, 31)], [(5, 127), (0, 129), (1, 17)],
+                                      [(0, 700), (40, 300), (7, 64)]], ids=str)
+@pytest.mark.parametrize("H,G,N,P", [(8, 2, 128, 64), (3, 3, 64, 16), (4, 1, 64, 80), (2, 2, 128, 128)])
+@pytest.mark.parametrize("level", [-0.5, 2.5])   # 2.5: some sub-chunks past 2^-90, which run token by token
+@pytest.mark.parametrize("two_pass", [True, False])
+def test_chunks(portions, H, G, N, P, level, two_pass, monkeypatch):
+    monkeypatch.setattr(sq, "SCAN_TWO_PASS", two_pass)
+    calls = record_native(monkeypatch, sq)
+    args = inputs(portions, H, G, N, P, level, N + P + len(portions))
+    got, state = run(args, portions, H, G, N, P)
+    assert "chunk_scan_ssm" in calls and ("ssm_chunk_scratch_floats" in calls) == (two_pass and portions[0][1] == 700)
+    want, states = reference(args, portions, H, G, N, P)
+    close(got, want)
+    for i, S in enumerate(states):
+        close(state[i + 1], S)
+    assert torch.equal(state[0].cpu(), args[-1][0])
+
+
+@pytest.mark.parametrize("level", [0.0, -0.5, -2.0, -5.0])
+@pytest.mark.parametrize("N,P,T", [(128, 64, 300), (64, 64, 200)])
+def test_errors_are_those_of_the_token_loop(level, N, P, T, monkeypatch):
+    """The mean of six draws: where decays are strong, a carried state is a few tokens and one draw a few dozen roundings."""
+    portions, H, G, errs = [(3, T)], 8, 2, []
+    for seed in range(6):
+        args = inputs(portions, H, G, N, P, level, seed)
+        want, states = reference(args, portions, H, G, N, P)
+        for chunks in (True, False):
+            with monkeypatch.context() as m:
+                if not chunks:
+                    m.setattr(sq, "_chunk_scan_ok", lambda *a: False)
+                out, state = run(args, portions, H, G, N, P)
+            errs += [error(out, want), error(state[1], states[0])]
+    o, s, o0, s0 = (sum(errs[i::4]) / 6 for i in range(4))
+    assert o <= 1.1 * o0 and s <= 1.1 * s0, (o, s, o0, s0)
+
+
+@pytest.mark.parametrize("value", [3e37, math.inf, math.nan])
+def test_states_that_cannot_be_split(value):
+    """One entry of the incoming state: its column goes the way of the token loop, the others do not see it."""
+    portions, H, G, N, P = [(3, 150)], 2, 1, 128, 64
+    args = inputs(portions, H, G, N, P, -6.0, 5)
+    ref, _ = run(args, portions, H, G, N, P)
+    args[-1][1, 1, 40, 21] = value
+    got, state = run(args, portions, H, G, N, P)
+    keep = torch.ones(H * P, dtype=torch.bool)
+    keep[P + 21] = False
+    torch.testing.assert_close(got[:, keep], ref[:, keep], rtol=1e-4, atol=1e-4)
+    want, states = reference(args, portions, H, G, N, P)
+    close(got[:, ~keep].float(), want[:, ~keep].float().to(F64))
+    close(state[1, 1, :, 21].float(), states[0][1, :, 21].float().to(F64))

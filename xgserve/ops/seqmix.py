@@ -1117,11 +1117,12 @@ def ssm_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_l
         es = xbc.element_size()
         if _chunk_scan_ok(sm, N) and N % 8 == 0 and xbc.data_ptr() % 16 == 0 \
                 and xbc.stride(0) * es % 16 == 0 and H * P * es % 16 == 0:
-            seg, scratch = _chunk_scan_segments(sm, T, H, N, P, 64, xbc.device)
+            split = xbc.dtype == torch.bfloat16 and N in (64, 128) and P % 16 == 0 and xbc.stride(0) < 1 << 25
+            seg, scratch = (_ssm_chunk_segments if split else _chunk_scan_segments)(sm, T, H, N, P, 64, xbc.device)
             mixers().chunk_scan_ssm(xbc.data_ptr(), is_f32(xbc), xbc.stride(0), dt_raw.data_ptr(), dt_raw.stride(0),
                                     dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(),
                                     _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(), _i32(sm.slots).data_ptr(),
-                                    y.data_ptr(), sm.num_seqs, sm.max_q, T, H, G, N, P, seg, _p(scratch), stream_ptr())
+                                    y.data_ptr(), sm.num_seqs, sm.max_q, T, H, G, N, P, seg, _p(scratch), split, stream_ptr())
             return y
         if _gla_step_ok(xbc, sm, N, P, state):
             mixers().ssm_step(xbc.data_ptr(), is_f32(xbc), xbc.stride(0), dt_raw.data_ptr(), dt_raw.stride(0),
@@ -1620,6 +1621,19 @@ def _chunk_scan_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: in
     seg = ((whole + n - 1) // n + 15) // 16 * 16
     return seg, torch.empty(mixers().chunk_scan_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32,
                             device=device)
+
+
+def _ssm_chunk_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
+    """The same for the state-space chunks of 64 tokens (csrc/mixers/ssm_chunk.hip): four to eight segments where at most a workgroup
+    per compute unit would run. us whole / in segments, heads of 128 x 64: 4001 tokens of 64 heads 324 / 96 (8), of 128 328 / 179 (4),
+    1531 + 700 + 257 + 33 of 64 130 / 75, 512 of 64 44 / 27; 1500 + 900 of 128 130 / 124, but 300 + 200 36 / 46 and 3 x 800 of 128 102 / 118."""
+    chunks = -(-sm.max_q // 64)
+    wgs = max(1.0, T / sm.max_q) * H * ((dv + cols - 1) // cols)
+    n = min(8, max(4, int(CHUNK_SCAN_FILL_WGS / wgs)), chunks)
+    if wgs > 256 or chunks < (4 if wgs <= 128 else 8) or not SCAN_TWO_PASS:
+        return 64 * chunks, None
+    seg = 64 * -(-chunks // n)
+    return seg, torch.empty(mixers().ssm_chunk_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32, device=device)
 
 
 def _chunk_scan(q, f, k, raw, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv):
