@@ -18,14 +18,22 @@
 // first key its first query row sees. The rotary part of a query is rotated while it is loaded. In latent space (latent_attention)
 // a (query, key) pair costs 2 (2 R + rd) operations per head, here 2 (dn + rd + dv): 3.4 times less at R = 256 and heads of 64,
 // against one product per key row that expands it (4 x 2048 tokens, 32 heads of 64 + 32, window 1024: 950 -> 205 us with the
-// gather and both expansions; heads of 128 + 64, window 4096: 3857 -> 395). Rows of 96 and 192 entries have 12 and 24 chunks: the permutation there
+// gather and both expansions, the attention 155 of them, since then 125; heads of 128 + 64, window 4096: 3857 -> 395). Rows of 96 and 192 entries have 12 and 24 chunks: the permutation there
 // stays inside groups of 4 and 8.
+//
+// Vector work and matrix instructions bound it together: 4001 tokens, 32 heads of 64 + 64, took 275 vector instructions a tile and
+// wave beside 16 matrix ones (156 and 64 of 266 thousand clocks), 118 to 124 us. Scores that stay products up to the exponential, a
+// reference that seldom moves, masks by edge (compares and selects, no branches), addresses as a uniform base and a lane's
+// constant: 195 instructions, 100 to 109 us; 16 heads of 64 + 128 with a distance penalty 132 -> 115, 2 x 1800 tokens of 32 heads
+// of 128 + 128 96 -> 89, expanded latents (64 + 32) + 64 of 4 x 2048 tokens 156 -> 125, (128 + 64) + 128 of 2 x 1300 97 -> 82.
+// (Both blocks of 32 keys in turn, so that two chains of matrix instructions run; waves' priorities and two sums for l change nothing.)
 #include "attention_common.h"
 #include "glds.h"
 
 namespace xgm {
 
 constexpr int kPT = 64;   // keys per tile
+constexpr float kLag = 8.f;   // see `m` below
 
 typedef xgk::f32x16_t f32x16_t;
 
@@ -60,7 +68,7 @@ __device__ __forceinline__ int xsw(int r) {
 }
 
 template <int DK, int DV, int GH, int NSLOT, int WFN, bool LAT>
-__global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_attention_kernel(
+__global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_attention_kernel(
     const AttnArgs a, const int32_t* __restrict__ block_tables, const bf16* __restrict__ kcache,
     const bf16* __restrict__ vcache, int tiles_per_seq, int n_hg, const LatentRows lr) {
   constexpr bool sig = WFN == kWeightsSigmoid, capped = WFN == kWeightsBounded || WFN == kWeightsCapped;
@@ -118,46 +126,62 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
   const int32_t* bt = block_tables + (int64_t)s * a.bt_width;
   auto tile_key = [&](int t) { return t < kt ? t * kPT : kfirst + (t - kt) * kPT; };
 
+  const bool pages_pow2 = (a.bs & (a.bs - 1)) == 0;
+  const int page_shift = __builtin_ctz(a.bs);
   const int lat_lo = first_visible(a.mask, a.size, ctx);   // the sequence's first dense key row
   const int64_t lat_row = LAT ? (int64_t)lr.koff[s] - lat_lo : 0;
+  // what a lane's DMA loads add to the tile's first row of the wave (elements); LAT: the address for key 0 and the bytes of a key's row
+  uint32_t k_off[KD], v_off[VD], k_row[LAT ? KD : 1];
+  const bf16* k_from[LAT ? KD : 1];
+#pragma unroll
+  for (int i = 0; i < KD; ++i) {
+    if constexpr (LAT) {
+      const int idx = min(64 * i + lane, DK - 1), rr = idx / (DK / 8), d = ((idx % (DK / 8)) ^ xsw<DK>(8 * w + rr)) * 8;
+      k_off[i] = rr, k_row[i] = 2 * (d < lr.dn ? a.H * lr.dn : lr.R + lr.rd);
+      k_from[i] = d < lr.dn ? lr.kn + (lat_row * a.H + head) * lr.dn + d : lr.lat + lat_row * (lr.R + lr.rd) + lr.R + d - lr.dn;
+    } else {
+      const int rr = KD == 2 ? 4 * i + (lane >> 4) : lane >> 3;
+      k_off[i] = rr * (uint32_t)krow + g * DK + 8 * ((KD == 2 ? lane & 15 : lane & 7) ^ xsw<DK>(8 * w + rr));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < VD; ++i) {
+    const int rr = VD == 2 ? 4 * i + (lane >> 4) : lane >> 3, ch = (VD == 2 ? lane & 15 : lane & 7) ^ xsw<DV>(8 * w + rr);
+    v_off[i] = LAT ? rr * (uint32_t)(a.H * DV) + ch * 8 : rr * (uint32_t)vrow + voff + ch * 8;
+  }
   auto issue = [&](int t) {
     char* dst = lds + (t % NSLOT) * SLOT;
-    if constexpr (LAT) {
-      const int k1 = tile_key(t) + 8 * w;   // (keys in front of the first row are masked: any row will do)
+    const int k1 = tile_key(t) + 8 * w;   // the wave's 8 rows: inside one aligned run of 16 keys
+    const bool whole = k1 + 7 <= last;    // (else the last row again)
+    if constexpr (LAT) {   // (keys in front of the first row are masked: any row will do)
+      const bool in = whole && k1 >= lat_lo;
 #pragma unroll
       for (int i = 0; i < KD; ++i) {
-        const int idx = 64 * i + lane, rr = idx / (DK / 8), d = ((idx % (DK / 8)) ^ xsw<DK>(8 * w + rr)) * 8;
-        const int64_t row = lat_row + max(min(k1 + rr, last), lat_lo);
-        if (idx < DK)   // (8 rows of DK / 8 chunks)
-          xgk::glds16(d < lr.dn ? lr.kn + (row * a.H + head) * lr.dn + d : lr.lat + row * (lr.R + lr.rd) + lr.R + d - lr.dn,
-                      dst + 8 * w * KROW + i * 1024);
+        const uint32_t key = in ? k1 + k_off[i] : max(min(k1 + (int)k_off[i], last), lat_lo);
+        if (64 * i + lane < DK)   // (8 rows of DK / 8 chunks)
+          xgk::glds16(reinterpret_cast<const char*>(k_from[i]) + (uint64_t)key * k_row[i], dst + 8 * w * KROW + i * 1024);
       }
+      const bf16* vp = lr.v + ((lat_row + k1) * a.H + head) * DV;
 #pragma unroll
       for (int i = 0; i < VD; ++i) {
         const int rr = VD == 2 ? 4 * i + (lane >> 4) : lane >> 3;
-        const int ch = (VD == 2 ? lane & 15 : lane & 7) ^ xsw<DV>(8 * w + rr);
-        const int64_t row = lat_row + max(min(k1 + rr, last), lat_lo);
-        xgk::glds16(lr.v + (row * a.H + head) * DV + ch * 8, dst + KT + (8 * w) * VROW + i * 1024);
+        const int64_t at = in ? v_off[i] : (int64_t)v_off[i] + (int64_t)(max(min(k1 + rr, last), lat_lo) - k1 - rr) * (a.H * DV);
+        xgk::glds16(vp + at, dst + KT + (8 * w) * VROW + i * 1024);
       }
       return;
     }
-    const int key0 = min(tile_key(t) + 8 * w, last);      // the wave's 8 rows: inside one aligned run of 16 keys
-    const int pidx = key0 / a.bs;
-    const int64_t prow = (int64_t)bt[pidx] * a.bs - (int64_t)pidx * a.bs;
-    const int k1 = tile_key(t) + 8 * w;
+    const int key0 = min(k1, last), pidx = pages_pow2 ? key0 >> page_shift : key0 / a.bs;
+    const int64_t row = (int64_t)bt[pidx] * a.bs - (int64_t)pidx * a.bs + k1;
+    const bf16 *kp = kcache + row * krow, *vp = vcache + row * vrow;
 #pragma unroll
     for (int i = 0; i < KD; ++i) {
       const int rr = KD == 2 ? 4 * i + (lane >> 4) : lane >> 3;
-      const int ch = (KD == 2 ? lane & 15 : lane & 7) ^ xsw<DK>(8 * w + rr);
-      const int64_t row = prow + min(k1 + rr, last);
-      xgk::glds16(kcache + row * krow + g * DK + ch * 8, dst + (8 * w) * KROW + i * 1024);
+      xgk::glds16(kp + (whole ? (int64_t)k_off[i] : k_off[i] + (min(k1 + rr, last) - k1 - rr) * krow), dst + (8 * w) * KROW + i * 1024);
     }
 #pragma unroll
     for (int i = 0; i < VD; ++i) {
       const int rr = VD == 2 ? 4 * i + (lane >> 4) : lane >> 3;
-      const int ch = (VD == 2 ? lane & 15 : lane & 7) ^ xsw<DV>(8 * w + rr);
-      const int64_t row = prow + min(k1 + rr, last);
-      xgk::glds16(vcache + row * vrow + voff + ch * 8, dst + KT + (8 * w) * VROW + i * 1024);
+      xgk::glds16(vp + (whole ? (int64_t)v_off[i] : v_off[i] + (min(k1 + rr, last) - k1 - rr) * vrow), dst + KT + (8 * w) * VROW + i * 1024);
     }
   };
 
@@ -187,9 +211,19 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
     }
   }
   const float cap2 = capped ? a.softcap * kLog2e : 0.f;
+  auto uniform = [](float x) {   // (the same in all lanes: a scalar register)
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+  };
   float sc_h = a.scale * (a.temp ? a.temp[head] : 1.f) * (capped ? 2.f / a.softcap : 1.f) * kLog2e;
-  float pen1 = a.r1 ? a.r1[head] : 0.f, pen2 = a.r1 ? a.r2[head] : 0.f;
-  float sbias = (sig && a.hbias) ? a.hbias[head] * kLog2e : 0.f;
+  const float pen1 = uniform(a.r1 ? a.r1[head] : 0.f), pen2 = uniform(a.r1 ? a.r2[head] : 0.f);
+  const float sbias = uniform((sig && a.hbias) ? a.hbias[head] * kLog2e : 0.f);
+  // Scores stay products until they are exponentials: one multiply-add takes them to their distance from the row's reference m (sc1;
+  // 1 where a bound or a penalty has made them scores already). The sign of the scale is the query's, so that the largest
+  // product is the largest score; a scale of 0 is the smallest number instead (0 would make a masked one not a number).
+  const bool scaled = capped || sig || a.r1;
+  const uint32_t flip = !scaled && sc_h < 0.f ? 0x80008000u : 0u;
+  sc_h = uniform(scaled ? sc_h : sc_h == 0.f ? 1.1754944e-38f : fabsf(sc_h));
+  const float sc1 = scaled ? 1.f : sc_h;
   float m = bounded ? 0.f : a.sink ? a.sink[head] * kLog2e : -INFINITY;
   float l = (a.sink && hf == 0) ? 1.f : 0.f;   // each half of a row's two lanes sums its own keys
   f32x16_t o[DV / 32];
@@ -199,8 +233,13 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
     for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
   // everything loaded so far is complete before the first DMA: from here on vmcnt counts the DMAs alone
 #pragma unroll
-  for (int ks = 0; ks < DK / 16; ++ks) asm volatile("" : "+v"(qf[ks]));
-  asm volatile("" : "+v"(sc_h), "+v"(pen1), "+v"(pen2), "+v"(sbias), "+v"(m));
+  for (int ks = 0; ks < DK / 16; ++ks) {
+    uint4 x = __builtin_bit_cast(uint4, qf[ks]);
+    x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
+    qf[ks] = xgk::as_frag(x);
+    asm volatile("" : "+v"(qf[ks]));
+  }
+  asm volatile("" : "+v"(m));
   xgk::wait_vmcnt<0>();
 #pragma unroll
   for (int p = 0; p < NSLOT - 1; ++p)
@@ -237,26 +276,29 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
 
     f32x16_t sacc[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
 #pragma unroll
-      for (int ks = 0; ks < DK / 16; ++ks)
+    for (int ks = 0; ks < DK / 16; ++ks) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
         sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + (k_at(ks) + kb * 32 * KROW))), qf[ks], sacc[kb]);
-      sched_fence();   // bound the hoisted fragment reads
+      if (ks % 2) sched_fence();   // bound the hoisted fragment reads
     }
     // scores in units of ln 2; register e of block kb is key base + 32 kb + 4 hf + (e & 3) + 8 (e >> 2)
     const bool full = base + kPT - 1 <= pos_lo && (base >= lo_hi || base + kPT <= a.keep);
     const int vis_hi = pos_q - base - 4 * hf, vis_lo = lo_q - base - 4 * hf, vis_keep = a.keep - base - 4 * hf;
-    float mx = -INFINITY;
+    if (scaled) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        float v = sacc[kb][e] * sc_h;
-        if constexpr (capped) v = cap2 - 2.f * cap2 * rcp_fast(1.f + exp2_fast(v));
-        sacc[kb][e] = v;
-      }
+        for (int e = 0; e < 16; ++e) {
+          float v = sacc[kb][e] * sc_h;
+          if constexpr (capped) v = cap2 - 2.f * cap2 * rcp_fast(1.f + exp2_fast(v));
+          sacc[kb][e] = v;
+        }
+    }
     if (a.r1) {
       // (distances are exact in fp32; those of keys behind the query may have no logarithm and are masked below; 138 -> 130 us
       // against an integer distance and the general logarithm)
@@ -267,14 +309,22 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
         for (int e = 0; e < 16; ++e)
           sacc[kb][e] -= pen1 * log2_fast(fmaf(pen2, dist - (float)(kb * 32 + (e & 3) + 8 * (e >> 2)), 1.f));
     }
-    if (!full) {
+    if (!full) {   // (wave-uniform: a tile mostly has one of the two edges)
+      if (base + kPT - 1 > pos_lo) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int c = kb * 32 + (e & 3) + 8 * (e >> 2);
-          if (c > vis_hi || (c < vis_lo && c >= vis_keep)) sacc[kb][e] = -INFINITY;
-        }
+          for (int e = 0; e < 16; ++e) sacc[kb][e] = kb * 32 + (e & 3) + 8 * (e >> 2) > vis_hi ? -INFINITY : sacc[kb][e];
+      }
+      if (base < lo_hi && base + kPT > a.keep) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int c = kb * 32 + (e & 3) + 8 * (e >> 2);
+            sacc[kb][e] = (int)(c < vis_lo) & (int)(c >= vis_keep) ? -INFINITY : sacc[kb][e];
+          }
+      }
     }
     if constexpr (sig) {
 #pragma unroll
@@ -284,16 +334,15 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
     } else {
       float nm = 0.f;
       if constexpr (!bounded) {
+        float mx = -INFINITY;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
-        mx = xor32_max(mx);
-        const float m_new = fmaxf(m, mx);
-        nm = m_new == -INFINITY ? 0.f : -m_new;
-        // no row of the wave raised its maximum: nothing to rescale
-        if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
-          const float alpha = m == -INFINITY ? 0.f : exp2_fast(m + nm);
+        mx = xor32_max(mx) * sc1;
+        // the reference follows the maximum only when that is 2^kLag ahead of it: sums and outputs are rarely rescaled
+        if (__builtin_amdgcn_ballot_w64(mx > m + kLag) != 0) {
+          const float m_new = mx > m + kLag ? mx : m, alpha = m == -INFINITY ? 0.f : exp2_fast(m - m_new);
           l *= alpha;
 #pragma unroll
           for (int db = 0; db < DV / 32; ++db)
@@ -301,12 +350,13 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
             for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
           m = m_new;
         }
+        nm = m == -INFINITY ? 0.f : -m;
       }
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const float p = exp2_fast(bounded ? sacc[kb][e] : sacc[kb][e] + nm);
+          const float p = exp2_fast(bounded ? sacc[kb][e] : fmaf(sacc[kb][e], sc1, nm));
           sacc[kb][e] = p;
           l += p;
         }
@@ -330,7 +380,7 @@ __global__ __launch_bounds__(512, (DK == 64 && DV == 64) ? 4 : 2) void prompt_at
           const xgk::bf16x8_t vf = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
           o[db] = mfma32x32x16(vf, pf, o[db]);
         }
-        sched_fence();
+        if (ss) sched_fence();
       }
   }
   l += __shfl_xor(l, 32, 64);

@@ -50,3 +50,32 @@ def test_causal_prompts(H, G, dk, dv, lens, ctx, dist):
             # independent roundings of the weights: at most 2^-9 of the root of their squares, 6 sigma
             bound = want.abs() * 2.0 ** -8 + 6 * 2.0 ** -9 * p.pow(2).sum(-1, keepdim=True).sqrt() * vv.abs().max() + 1e-5
             assert bool((err <= bound).all()), (s, h, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("mask,size", [(sq.MASK_CAUSAL, 0), (sq.MASK_WINDOW, 90), (sq.MASK_CHUNK, 100)])
+@pytest.mark.parametrize("sink", [False, True])
+def test_scales_of_any_sign_and_growing_scores(dk, dv, mask, size, sink):
+    """Scales of either sign, 0 and large (some keys far above all before them, the reference catches up), with and without a sink, on
+    pages of 48 keys. Same tolerance; a score errs by 2^-23 of its size and a weight by as much of itself."""
+    g = torch.Generator().manual_seed(dk + size)
+    H, n, bs = 4, 330, 48
+    q, k, v = (torch.randn(n, H * d, generator=g).bfloat16() for d in (dk, dk, dv))
+    k[::37] *= 8.0
+    temp, sinks = torch.tensor([1.0, -1.3, 0.0, 25.0]), torch.randn(H, generator=g) * 2
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    sm = sq.SeqMeta(1, n, i32([0, n]), i32([n]), i32([0]), i32([list(range(-(-n // bs)))]), i32([0] * n), i32(list(range(n))), i32(list(range(n))))
+    cache = [torch.cat([t, torch.zeros(-n % bs, t.shape[1])]).bfloat16().cuda() for t in (k, v)]
+    got = sq.masked_attention(q.cuda(), *cache, H, H, dk, dv, mask, size, dk ** -0.5, temp.cuda(), sinks.cuda() if sink else None, bs, sm)
+    i, j = torch.arange(n)[:, None], torch.arange(n)[None]
+    seen = (j <= i) & (i - j < size if mask == sq.MASK_WINDOW else i // size == j // size if mask == sq.MASK_CHUNK else j <= i)
+    for h in range(H):
+        sc = (q[:, h * dk:(h + 1) * dk].double() @ k[:, h * dk:(h + 1) * dk].double().T * dk ** -0.5 * temp[h].double()).masked_fill(~seen, float("-inf"))
+        full = torch.cat([sc, sinks[h].double().expand(n, 1)], 1) if sink else sc
+        p = torch.softmax(full, -1)[:, :n]
+        vv = v[:, h * dv:(h + 1) * dv].double()
+        want = p @ vv
+        err = (got[:, h * dv:(h + 1) * dv].double().cpu() - want).abs()
+        big = sc.masked_fill(~seen, 0).abs().amax(-1, keepdim=True)
+        bound = want.abs() * 2.0 ** -8 + (6 * 2.0 ** -9 * p.pow(2).sum(-1, keepdim=True).sqrt() + big * 2.0 ** -22) * vv.abs().max() + 1e-5
+        assert bool((err <= bound).all()), (h, float((err / bound).max()))
