@@ -13,7 +13,9 @@
 //
 // 64 sequences of 1024 keys, 32 heads, R = 256, rd = 32: 17.6 us (37.7 MB of rows) and 8.1 us against 30.6 and, for merge,
 // expansion product and transpose in three launches, 25.7. The kernel before had one 64-key tile to a workgroup (16 shares),
-// nothing in flight behind it, 33 MB of fp32 shares written and read back, and half of its waves without heads.
+// nothing in flight behind it, 33 MB of fp32 shares written and read back, and half of its waves without heads. (R = 512, rd = 64: 30.9
+// where every tile rescaled its 128 accumulators, 28.5 since only those that raise the maximum do. Four slots, or two tiles at a
+// time on eight waves: no faster, one tile takes 7.5 us, most of it one memory latency behind the other.)
 #include "attention_common.h"
 #include "glds.h"
 
@@ -32,6 +34,17 @@ struct LatentDecodeArgs {
   int dq, dn, bt_width, bs, rot_dims, T, H, window, shares;
   float scale;
 };
+
+// maximum over the four lanes that share a column
+__device__ __forceinline__ float column_max(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+#endif
+  return x;
+}
 
 template <int NR, int ND>
 __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecodeArgs a) {
@@ -90,7 +103,7 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
   f32x4_t o[NMT];
 #pragma unroll
   for (int mt = 0; mt < NMT; ++mt) o[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, l = 0.f;   // the column's reference; this lane's share of its sum
   // the queries have to be here before the second tile is asked for: the wait for them would cover it too
 #pragma unroll
   for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(qr[kk].x), "+v"(qr[kk].y), "+v"(qr[kk].z), "+v"(qr[kk].w));
@@ -120,20 +133,23 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
         sc[n][r] = k > k1 ? -INFINITY : sc[n][r] * a.scale;
         mx = fmaxf(mx, sc[n][r]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx), alpha = mn == -INFINITY ? 1.f : __expf(m - mn);
-    float rs = 0.f;
+    mx = column_max(mx);
+    // (the reference follows the maximum only when that is e^5 ahead: the sums are rarely rescaled)
+    if (__builtin_amdgcn_ballot_w64(mx > m + 5.f) != 0) {
+      const float mn = mx > m + 5.f ? mx : m, alpha = m == -INFINITY ? 0.f : __expf(m - mn);
+      l *= alpha, m = mn;
+#pragma unroll
+      for (int mt = 0; mt < NMT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[mt][r] *= alpha;
+    }
 #pragma unroll
     for (int n = 0; n < 2; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        sc[n][r] = mn == -INFINITY ? 0.f : __expf(sc[n][r] - mn);
-        rs += sc[n][r];
+        sc[n][r] = m == -INFINITY ? 0.f : __expf(sc[n][r] - m);
+        l += sc[n][r];
       }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l = l * alpha + rs, m = mn;
     uint4 pb;
     pb.x = xgk::pack2(sc[0][0], sc[0][1]), pb.y = xgk::pack2(sc[0][2], sc[0][3]);
     pb.z = xgk::pack2(sc[1][0], sc[1][1]), pb.w = xgk::pack2(sc[1][2], sc[1][3]);
@@ -144,13 +160,13 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
       const xgk::bf16x4_t a0 = xgk::lds_read_tr16(reinterpret_cast<const uint16_t*>(v));
       const xgk::bf16x4_t a1 = xgk::lds_read_tr16(reinterpret_cast<const uint16_t*>(v + NKK * 1024));
       const xgk::bf16x8_t vf = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[mt][r] *= alpha;
       o[mt] = mfma16x16x32(vf, as_frag(pb), o[mt]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     xgk::raw_barrier();
   }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
   xgk::wait_vmcnt<0>();
   __syncthreads();   // (a slower wave's last rows are still on their way into a slot)
   // the second half of the keys joins the first
@@ -177,16 +193,18 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
   }
 }
 
-// Workgroup = (head, 8 tokens): out[t][h dv + j] = sum_d lat[t][d] W_uv[h dv + j][d], lat the merged and gated latent sum, rounded
-// to bf16. The columns of a 16-token product beyond the 8 repeat them (more workgroups; the products cost nothing here).
-template <int NR>
+// Workgroup = (head, TOK tokens): out[t][h dv + j] = sum_d lat[t][d] W_uv[h dv + j][d], lat the merged and gated latent sum, rounded
+// to bf16. The columns of a 16-token product beyond TOK repeat them (more workgroups; the products cost nothing here): so few tokens
+// that about a workgroup per compute unit runs (32 heads, 8 tokens each / as here, us: 9 tokens, 16 shares, R = 512 26.9 / 8.8, one token,
+// 10 shares 12.2 / 7.0, 17 tokens, 15 shares, R = 256 10.4 / 7.1).
+template <int NR, int TOK>
 __global__ __launch_bounds__(256) void latent_out_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                          const bf16* __restrict__ gate, int64_t gate_stride,
                                                          const bf16* __restrict__ uv, const int32_t* __restrict__ slots,
                                                          const int32_t* __restrict__ qsl,
                                                          const int32_t* __restrict__ token_seq, bf16* __restrict__ out, int T,
                                                          int H, int dv, int shares) {
-  constexpr int R = 32 * NR, LD = R + 8, TOK = 8;
+  constexpr int R = 32 * NR, LD = R + 8;
   __shared__ __attribute__((aligned(16))) uint16_t lat[TOK * LD];
   __shared__ float wt[TOK][64];   // a share's weight: e^(m_s - M) gate / L (shares <= 64)
   const int h = blockIdx.x, t0 = blockIdx.y * TOK, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -230,7 +248,7 @@ __global__ __launch_bounds__(256) void latent_out_kernel(const float* __restrict
   __syncthreads();
   uint4 b[NR];
 #pragma unroll
-  for (int kk = 0; kk < NR; ++kk) b[kk] = *reinterpret_cast<const uint4*>(lat + (li & 7) * LD + 32 * kk + 8 * g);
+  for (int kk = 0; kk < NR; ++kk) b[kk] = *reinterpret_cast<const uint4*>(lat + (li & (TOK - 1)) * LD + 32 * kk + 8 * g);
   for (int j = wave; 16 * j < dv; j += 4) {
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -262,13 +280,17 @@ int latent_decode(const void* qabs, const void* q, int dq, int dn, const void* g
   const LatentDecodeArgs a = {(const bf16*)qabs, (const bf16*)q, (const bf16*)cache, bt, qsl, seq_lens, slots, rot, part_o, part_ml,
                               dq, dn, bt_width, bs, rot_dims, T, H, window, shares, scale};
   const dim3 grid(shares, T, (H + 31) / 32);
+#define XGM_LO(NR, TOK)                                                                                                     \
+  {                                                                                                                         \
+    latent_out_kernel<NR, TOK><<<dim3(H, (T + TOK - 1) / TOK), 256, 0, st>>>(part_o, part_ml, (const bf16*)gate, gate_stride, \
+                                                                             (const bf16*)uv, slots, qsl, token_seq,        \
+                                                                             (bf16*)out, T, H, dv, shares);                 \
+  }
 #define XGM_LD(NR)                                                                                                          \
   if (nr == NR) {                                                                                                           \
     if (rd == 32) latent_decode_kernel<NR, 1><<<grid, 256, 0, st>>>(a);                                                     \
     else latent_decode_kernel<NR, 2><<<grid, 256, 0, st>>>(a);                                                              \
-    latent_out_kernel<NR><<<dim3(H, (T + 7) / 8), 256, 0, st>>>(part_o, part_ml, (const bf16*)gate, gate_stride,            \
-                                                                (const bf16*)uv, slots, qsl, token_seq, (bf16*)out, T, H,   \
-                                                                dv, shares);                                                \
+    if (H * T > 1024) XGM_LO(NR, 8) else if (H * T > 512) XGM_LO(NR, 4) else if (H * T > 256) XGM_LO(NR, 2) else XGM_LO(NR, 1) \
     return 0;                                                                                                               \
   }
   XGM_LD(2)
@@ -276,6 +298,7 @@ int latent_decode(const void* qabs, const void* q, int dq, int dn, const void* g
   XGM_LD(8)
   XGM_LD(16)
 #undef XGM_LD
+#undef XGM_LO
   return -1;
 }
 }  // namespace xgm
