@@ -368,3 +368,11 @@ def test_grouped_workgroups_take_several_tiles(tile, idle, monkeypatch):
         a = sq._glu_ref(z[:, :F_], z[:, F_:], sq.GLU_SILU, 0.0, 0.0)
         ref, size = wts[t].double() * (a @ w2[e].double().t()), wts[t].double() * (a.abs() @ w2[e].double().abs().t())
         assert ((got[t] - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all()   # (as in test_grouped_tiles)
+
+
+@pytest.mark.parametrize("M,N,K,library", [(2048, 16384, 2048, True), (6144, 2048, 2048, True),       # 512 and 192 of the library's tiles
+                                           (2049, 16384, 2048, True), (5889, 2048, 2048, True),       # 576 of 768 and 192: three quarters
+                                           (2560, 4096, 4096, False), (3100, 6144, 4096, False),      # 160 of 256, 312 of 512
+                                           (1792, 16384, 2048, False), (8192, 10304, 2048, False)])
+def test_the_library_keeps_full_rounds(M, N, K, library):
+    assert tl.library_better(M, N, K) is library

@@ -1,8 +1,11 @@
 """Products of many rows (prompt steps) on csrc/mixers/tile_linear.hip: the sizes they run at, and where the library's stay.
 
-`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 1 200 timings on an MI355X (15 weights
+`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 4 500 timings on an MI355X (15 weights
 of 768 to 14336 in K and 1088 to 28672 in N, 65 to 8192 rows, cold weights); over these its choice is 1 % slower than the fastest
-of the kernel's forms in the mean and 13 % at most.
+of the kernel's forms in the mean and 13 % at most. A product's time steps up with every round of tiles that is begun, so there are
+many sizes: (5, 8), (8, 6), (7, 6), (6, 6), (7, 4) and (5, 4) beside the ten that were there take 2 % off the mean of 144 products of 80 to
+5000 rows, and, us, cold weights: 2521 x 4096 x 14336 243 -> 213 (256 tiles of 160 x 256, where 192 x 256 left 32 of 256 workgroups out),
+2521 x 2048 x 8192 79 -> 74, 3100 x 6144 x 4096 139 -> 126, 1024 x 18560 x 4096 148 -> 130, 700 x 6144 x 4096 43 -> 38.
 """
 from __future__ import annotations
 
@@ -20,11 +23,13 @@ from ._native import is_f32, mixers, native_device, on_current_device, stream_pt
 from .linear import PendingSum, cu_count
 
 # rows and columns of a workgroup's tile / 32 -> us per 64 of K and per tile
-_TILES = {(8, 8): (1.098, 0.02), (7, 8): (0.995, 0.63), (6, 8): (0.868, 0.86), (4, 8): (0.694, 1.11), (8, 4): (0.667, 1.18),
-          (6, 4): (0.527, 1.55), (4, 4): (0.401, 1.88), (3, 4): (0.331, 1.95), (4, 2): (0.274, 1.23), (3, 2): (0.249, 0.09)}
-_LAUNCH, _SUM = 2.2, 3.7                    # us of the launch, and of the one that adds the parts
-_W_BYTES, _PART_BYTES, _OUT_BYTES = 6.1e6, 2.5e6, 3.0e6   # bytes per us: weights, fp32 parts (there and back), the result
-_OVERLAP = 0.29                             # share of the shorter of products and weight stream that stays visible
+_TILES = {(8, 8): (1.135, 0.02), (7, 8): (1.036, 0.02), (6, 8): (0.901, 0.02), (5, 8): (0.816, 0.02), (4, 8): (0.721, 0.02),
+          (8, 6): (0.937, 0.02), (7, 6): (0.819, 0.61), (6, 6): (0.708, 0.98), (8, 4): (0.705, 0.10), (7, 4): (0.627, 1.11),
+          (6, 4): (0.540, 1.13), (5, 4): (0.480, 1.19), (4, 4): (0.399, 1.62), (3, 4): (0.327, 1.90), (4, 2): (0.254, 1.57),
+          (3, 2): (0.229, 0.46)}
+_LAUNCH, _SUM = 2.19, 3.35                  # us of the launch, and of the one that adds the parts
+_W_BYTES, _PART_BYTES, _OUT_BYTES = 6.25e6, 2.56e6, 2.55e6   # bytes per us: weights, fp32 parts (there and back), the result
+_OVERLAP = 0.31                             # share of the shorter of products and weight stream that stays visible
 _SPLITS = (1, 2, 3, 4, 6, 8, 12, 16)
 _SPLIT_K, _SPLIT_TILES = 256, 540           # a part's least K; parts of all tiles at most (a bound on the slabs: 2.1 tiles per CU)
 
@@ -52,10 +57,13 @@ def tile_plan(M: int, N: int, K: int, cus: int = 256):
 
 
 # Tiles of the experts' products; offsets of all experts are looked through for a tile's, so there is a bound on their number
-_GROUPED, GROUPED_EXPERTS_MAX = ((8, 8), (7, 8), (6, 8), (4, 8), (6, 4), (4, 4), (3, 4)), 64
+# (their prices are a fit of their own: rows are gathered, and most experts end in a part of a tile)
+_GROUPED = {(8, 8): (1.098, 0.02), (7, 8): (0.995, 0.63), (6, 8): (0.868, 0.86), (4, 8): (0.694, 1.11), (6, 4): (0.527, 1.55),
+            (4, 4): (0.401, 1.88), (3, 4): (0.331, 1.95)}
+GROUPED_EXPERTS_MAX = 64
 _SHARES = (-1.2, -0.9, -0.6, -0.2, 0.2, 0.6, 0.9, 1.4)   # eight quantiles of an expert's rows, in units of their spread ...
 _SPREAD = 0.55                                            # ... from the mean, in units of the mean
-_GROUPED_ROWS = _table("d", *(t + _TILES[t] for t in _GROUPED))[0]
+_GROUPED_ROWS = _table("d", *(t + p for t, p in _GROUPED.items()))[0]
 _QUANTILES = _table("d", [z * _SPREAD for z in _SHARES])[0]
 
 
@@ -72,15 +80,17 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
 def library_better(M: int, N: int, K: int) -> bool:
     """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel): long ones, which run
     at the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
-    4001 rows 89 against 93; 8192x2048, 2521 rows 70 to 74 against 72 to 81), as long as no columns are left over beside its tiles of
-    256 (10304x2048, 4001 rows 168 against 129; 18560x4096, 2048 rows 344 against 257) and there are 150 such tiles (2048x8192, 2521
-    rows 77 to 81 against 75; up to 1792 rows 4096x14336, 1536 rows 168 against 140; 6144x4096, 700 rows 45 against 41). Its narrow
+    4001 rows 91 against 98; 16384x2048, 2048 rows 103 against 117), as long as no columns are left over beside its tiles of 256
+    (10304x2048, 4001 rows 168 against 129; 18560x4096, 2048 rows 344 against 257) and these fill their rounds of the chip to three
+    quarters (0.81 to 1: -14 to 10 %; below, at 0.6, 6144x4096, 3100 rows 169 against 126; 4096x14336, 2521 rows 226 against 213;
+    4096x4096, 5000 rows 137 against 132; up to 1792 rows 4096x14336, 1536 rows 168 against 140; 6144x4096, 700 rows 45 against 38). Its narrow
     products of few rows are 1 to 2 us faster on the card (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4; 4096x4096,
     256 rows 23.1 against 27.8), and some of middle size by 2 to 9 (6144x4096, 512 rows 38.2 against 40.8; 18560x4096, 400 rows 71
     against 80), but not in steps. Eager ones of few rows wait for the host, of which the library's call takes 31 us and this kernel's
     10: with the faster of both for every product, 96 rows, Vizonex "1b" 868 -> 1159 us, Dofivik 1300 -> 1507; from 400 rows on within
     1 %. Replayed ones of 96 and 160 rows are up to 2 % slower with it, of 256 rows up to 2 % faster."""
-    return N % 256 == 0 and M > 1792 and -(-M // 256) * (N // 256) >= 150
+    tiles = -(-M // 256) * (N // 256)
+    return N % 256 == 0 and M > 1792 and 4 * tiles >= 3 * 256 * -(-tiles // 256)
 
 
 def forward_only(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
