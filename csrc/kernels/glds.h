@@ -32,6 +32,29 @@ __device__ __forceinline__ void glds16(const void* src, void* lds_base) {
 #endif
 }
 
+// The same from a base that all lanes share and a lane's offset to an LDS byte address that all lanes share. (s_nop 4: a base that a
+// vector instruction has just written, where the compiler moved it through one.)
+__device__ __forceinline__ void glds16_at(const void* base, uint32_t offset, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_nop 4\n\t"
+      "global_load_lds_dwordx4 %0, %1"
+      :
+      : "v"(offset), "s"(base), "{m0}"(lds)
+      : "memory");
+#endif
+}
+__device__ __forceinline__ void glds16_v(const void* src, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "{m0}"(lds)
+      : "memory");
+#endif
+}
+
 // non-temporal weight stream (read once per step: keeps the activations in L2)
 __device__ __forceinline__ void glds16_nt(const void* src, void* lds_base) {
 #if defined(__HIP_DEVICE_COMPILE__)

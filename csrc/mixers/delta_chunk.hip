@@ -23,17 +23,20 @@
 // state and of the outputs summed up by itself and before the tokens' own terms, the latest and largest of them last; E in two
 // floats.
 //
-// The second launch has two waves per 16 state columns of a (sequence, head), one for the even and one for the odd 16s of the state's
-// rows, which are the two chains that y and the outputs are summed in anyway: they hand each other y (and the outputs' sums) through
-// LDS at the one barrier of a chunk, so each has half of the matrix instructions. A workgroup takes 32 columns, so a head of 64 has
-// two and 32 heads of 4 sequences fill the chip. The first launch writes every operand in the order of the matrix instructions' lanes;
-// the waves bring it in by LDS DMA, five chunks ahead, and read a chunk's operands while the one before it still adds to the state.
-// A chunk with an input out of range (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
+// The second launch has a wave per 16 x 16 of the state: the waves of a column tile (four for heads of 64) sum y and the outputs over
+// their rows and hand each other the sums through LDS, y at the one barrier of a chunk and the outputs' behind it, to be added and
+// stored behind the next. A workgroup takes 32 columns, so a head of 64 has two and 32 heads of 4 sequences fill the chip, two waves to
+// a SIMD. The first launch writes every operand in the order of the matrix instructions' lanes; the waves bring it in by LDS DMA, four
+// chunks ahead, and read a chunk's operands while the one before it still adds to the state. A chunk with an input out of range
+// (infinities, NaN, 2^28 and above) is stored as w, b, u, k, r and run token by token.
 //
-// Measured, bf16 rows, 4 x 2048 tokens of 32 heads of 64 in a step: the first launch 162 us (it writes 24.6 KB per chunk and head and
-// forms three exponentials per token and channel), the second 169, 1.3 us a chunk (one wave per 16 columns 238 to 258; two, operands
-// read at a chunk's head 184, loads behind the barrier instead of between y's products 173). What is left of a chunk is the way from
-// one matrix instruction to the next, 0.45 us of it the instructions: with every load from the same 25 KB it takes as long.
+// Measured, bf16 rows, 4 x 2048 tokens of 32 heads of 64 in a step, us: the first launch 186 -> 169 (in one trace; it writes 24.6 KB per chunk and head,
+// 570 MB with its reads; three exponentials per token and channel, which a branch per token kept from overlapping, and 80 addresses
+// formed lane by lane were the difference), the second 168 -> 138, 1.1 us a chunk. It was two waves per 16 columns and one to a
+// SIMD, which waited for each of its instructions: with DMA addresses kept instead of formed (a third of 260 instructions a chunk)
+// and the outputs' products behind y's 146, with four waves 144, with no branches between the products 138. What is left of a chunk is the
+// way from one matrix instruction to the next and through LDS, 0.43 us of it the instructions: with every load from the same 25 KB
+// it takes 137, with nothing stored 133.
 #include "glds.h"
 #include "mfma_f32.h"
 
@@ -66,16 +69,21 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
 
   // ---- this lane's channel, tokens tg TT .. (rows past the end repeat the last and are masked)
   T xr[TT], xk[TT], xa[TT], xw[TT], xv[MT][4];
+  const int t0 = TG == 1 ? 0 : min(TT * tg, n - 1);   // (heads of 64: the same for all lanes, and so the rows' addresses)
+  const T *at = row + t0 * ld, *wat = wrow + t0 * ld_wl;
 #pragma unroll
   for (int i = 0; i < TT; ++i) {
-    const uint32_t t = min(TT * tg + i, n - 1), at = t * (uint32_t)ld + d;
-    xk[i] = row[at + off_k], xw[i] = wrow[t * (uint32_t)ld_wl + d];
-    xa[i] = row[at + off_a], xr[i] = row[at + off_r];
+    xk[i] = (at + off_k)[(uint32_t)d], xw[i] = wat[(uint32_t)d];
+    xa[i] = (at + off_a)[(uint32_t)d], xr[i] = (at + off_r)[(uint32_t)d];
+    const bool more = (TG == 1 ? 0 : TT * tg) + i + 1 < n;
+    at += more ? ld : 0, wat += more ? ld_wl : 0;
   }
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int t = 0; t < 4; ++t) {
+    const T* at = row + off_v + l16 + (int64_t)min(4 * t + g4, n - 1) * ld;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) xv[m][t] = row[(uint32_t)min(4 * t + g4, n - 1) * (uint32_t)ld + off_v + 16 * m + l16];
+    for (int m = 0; m < MT; ++m) xv[m][t] = at[16 * m];
+  }
   const float ab = a_bias[h * D + d], wb = w0[h * D + d];
   bool bad = false;
   float k[TT];
@@ -110,8 +118,10 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
   for (int i = 0; i < TT; ++i) {
     const bool on = TT * tg + i < n;
     u[i] = k[i] * __shfl(inv, tok_pos(TT * tg + i), 64);
-    wt[i] = on ? expf(kDeltaDecay * sigmoidf(ldf(&xw[i]) + wb)) : 1.f;
-    a[i] = on ? sigmoidf(ldf(&xa[i]) + ab) : 0.f;
+    // (formed for the repeated rows too: a branch per token keeps one token's exponentials waiting for the other's)
+    wt[i] = expf(kDeltaDecay * sigmoidf(ldf(&xw[i]) + wb)), a[i] = sigmoidf(ldf(&xa[i]) + ab);
+    asm volatile("" : "+v"(wt[i]), "+v"(a[i]));
+    wt[i] = on ? wt[i] : 1.f, a[i] = on ? a[i] : 0.f;
     r_[i] = on ? ldf(&xr[i]) : 0.f;
     bad |= out_of_range(r_[i]) || out_of_range(a[i]) || out_of_range(wt[i]);
   }
@@ -263,98 +273,138 @@ __global__ __launch_bounds__(64, 2) void delta_chunk_prep_kernel(const T* __rest
 }
 
 template <typename T, int D>
-__global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(const float* __restrict__ prep, const T* __restrict__ proj,
-                                                                  int64_t ld, int off_v, float* __restrict__ state,
-                                                                  const int32_t* __restrict__ qsl,
-                                                                  const int32_t* __restrict__ seq_lens,
-                                                                  const int32_t* __restrict__ slots, float* __restrict__ o,
-                                                                  int H) {
-  constexpr int C = kDcTok, MT = D / 16, MH = MT / 2, RING = 6;
+__global__ __launch_bounds__(8 * D, 1) void delta_chunk_scan_kernel(const float* __restrict__ prep, const T* __restrict__ proj,
+                                                                    int64_t ld, int off_v, float* __restrict__ state,
+                                                                    const int32_t* __restrict__ qsl,
+                                                                    const int32_t* __restrict__ seq_lens,
+                                                                    const int32_t* __restrict__ slots, float* __restrict__ o,
+                                                                    int H) {
+  constexpr int C = kDcTok, MT = D / 16, W = 2 * MT, RING = D == 64 ? 5 : 6;
   constexpr int OPS = 4 * C * D * 4, VO = 2 * C * 32 * 4, FRAG = OPS + VO;   // bytes: [U | R | k' | -b'], this half's [V | O]
   constexpr int VROWS = C * 32 * sizeof(T), SLOT = FRAG + 1024 + VROWS;      // ... [E, flag | v rows]
-  constexpr int PIECES = FRAG / 1024 / 4, VD = VROWS / 1024, DMA = PIECES + 1 + VD;   // loads per wave and chunk
-  constexpr int kEx = 2 * (4 + 2) * 1024;                                    // handed over: y of four waves, outputs of two
+  constexpr int NE = FRAG / 1024, NP = NE + 1 + VROWS / 1024, DMA = (NP + W - 1) / W;   // kilobytes of a chunk, loads per wave
+  constexpr int HAND = 2 * W * 1024;                                         // handed over: y of all waves, then their outputs' sums
   constexpr int VL = 32 * sizeof(T) / 16;                                    // lanes per v row
-  static_assert(RING * SLOT + kEx <= 160 * 1024 && (RING - 2) * DMA < 64, "delta_chunk_scan geometry");
-  __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT + kEx];
+  constexpr int NO = 4 / MT;                                                 // of a lane's four output rows the wave's share
+  static_assert(RING * SLOT + 2 * HAND <= 160 * 1024 && (RING - 2) * DMA < 64 && W * (DMA - 1) <= NE, "delta_chunk_scan geometry");
+  __shared__ __attribute__((aligned(1024))) char lds[RING * SLOT + 2 * HAND];
   const int h = blockIdx.x, s = blockIdx.y, half = blockIdx.z;
   const int q0 = qsl[s], qn = qsl[s + 1] - q0, slot = slots[s];
   if (slot < 0 || qn <= 0) return;
   const int ctx = seq_lens[s] - qn;
   const int lane = threadIdx.x & 63, g4 = lane >> 4, l16 = lane & 15;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ct = w >> 1, par = w & 1;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ct = w / MT, par = w % MT;
   const int col = 32 * half + 16 * ct + l16;
-  float* Sg = state + ((int64_t)slot * H + h) * D * D + col;
-  f32x4_t S[MH];   // rows 16 (2 i + par) ..
+  float* Sg = state + ((int64_t)slot * H + h) * D * D + (16 * par + 4 * g4) * D + col;
+  f32x4_t S;   // rows 16 par + 4 g4 ..
 #pragma unroll
-  for (int i = 0; i < MH; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) S[i][r] = ctx > 0 ? Sg[(16 * (2 * i + par) + 4 * g4 + r) * D] : 0.f;
+  for (int r = 0; r < 4; ++r) S[r] = ctx > 0 ? Sg[r * D] : 0.f;
   const int nch = (qn + C - 1) / C;
   const float* base = prep + ((int64_t)(q0 / C + s) * H + h) * dc_stride(D);
-  const int64_t step = (int64_t)H * dc_stride(D);
-  const T* vb = proj + (int64_t)q0 * ld + off_v + h * D + 32 * half;
+  const int64_t step = (int64_t)H * dc_stride(D) * 4;
 
-  // every wave issues DMA loads, past the last chunk too (its waits count them): i-th of DMA of chunk c
-  const T* vrow = vb + (lane % VL) * (16 / sizeof(T));
-  auto issue1 = [&](int c, int i) __attribute__((always_inline)) {
-    char* dst = lds + (c % RING) * SLOT;
-    const int cc = min(c, nch - 1);
-    const char* src = reinterpret_cast<const char*>(base + cc * step) + 16 * lane;
-    if (i < PIECES) {
-      const int pc = PIECES * w + i, vo = pc - OPS / 1024;   // (V and O: two of their MT kilobytes each)
-      const int from = vo < 0 ? pc : OPS / 1024 + (vo >> 1) * MT + 2 * half + (vo & 1);
-      xgk::glds16(src + 1024 * from, dst + 1024 * pc);
-    } else if (i == PIECES) {
-      xgk::glds16(src + 6 * C * D * 4, dst + FRAG);   // (the same bytes from every wave, and so the v rows)
-    } else {
-      const int j = i - PIECES - 1;
-      xgk::glds16(vrow + (int64_t)min(C * cc + j * (64 / VL) + lane / VL, qn - 1) * ld, dst + FRAG + 1024 + 1024 * j);
-    }
-  };
-  auto issue = [&](int c) __attribute__((always_inline)) {
+  // Every wave issues DMA loads, past the last chunk too (its waits count them, and the last chunk is brought in again; so is a slot's
+  // last kilobyte where the waves have more loads than there are). An address is the chunk's, the same for all lanes, plus what a
+  // lane keeps: formed anew for every load, these were a third of the loop's instructions. The last of a wave's loads, which may be
+  // v's, goes from a pointer of the lane's.
+  uint32_t from[DMA];
 #pragma unroll
-    for (int i = 0; i < DMA; ++i) issue1(c, i);
+  for (int i = 0; i < DMA; ++i) {
+    const int kb = W * i + w, vo = kb - OPS / 1024;   // (V and O: two of their MT kilobytes each)
+    from[i] = 16 * lane + 1024 * (kb == NE ? 6 * C * D / 256 : vo < 0 ? kb : OPS / 1024 + (vo >> 1) * MT + 2 * half + (vo & 1));
+  }
+  const int kb_last = min(W * (DMA - 1) + w, NP - 1);
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const char *p_last = reinterpret_cast<const char*>(base) + from[DMA - 1], *p_end = p_last + (nch - 1) * step;
+  int64_t p_step = step;
+  if (kb_last > NE) {
+    const int r = (kb_last - NE - 1) * (64 / VL) + lane / VL;
+    const T* at = proj + (int64_t)q0 * ld + off_v + h * D + 32 * half + (lane % VL) * (16 / sizeof(T));
+    p_last = reinterpret_cast<const char*>(at + min(r, qn - 1) * ld);
+    p_end = reinterpret_cast<const char*>(at + min(C * (nch - 1) + r, qn - 1) * ld);
+    p_step = C * ld * sizeof(T);
+  }
+  int c_in = 0;              // the chunk that is asked for next,
+  uint32_t at_in = ring;     // and its slot
+  auto operands = [&]() __attribute__((always_inline)) {
+    const uint64_t at = (uint64_t)(uintptr_t)base + (uint64_t)c_in * step;   // (said to be one for all lanes, which it is)
+    return (const char*)(uintptr_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
+                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)at));
   };
-  for (int c = 0; c < RING - 1; ++c) issue(c);
+  auto issue1 = [&](int i, const char* ahead) __attribute__((always_inline)) {
+    if (i < DMA - 1)
+      xgk::glds16_at(ahead, from[i], at_in + 1024 * (W * i + w));
+    else
+      xgk::glds16_v(p_last, at_in + 1024 * kb_last);
+  };
+  auto issued = [&]() __attribute__((always_inline)) {   // (all of them: on to the next)
+    c_in = min(c_in + 1, nch - 1);
+    p_last = c_in == nch - 1 ? p_end : p_last + p_step;
+    at_in = at_in == ring + (RING - 1) * SLOT ? ring : at_in + SLOT;
+  };
+  auto issue = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < MH; ++i) asm volatile("" : "+v"(S[i]));   // (the state is here: its loads are not waited for inside the loop)
+    for (int i = 0; i < DMA; ++i) issue1(i, operands());
+    issued();
+  };
+  for (int c = 0; c < RING - 1; ++c) issue();
+  asm volatile("" : "+v"(S));   // (the state is here: its loads are not waited for inside the loop)
   xgk::wait_vmcnt<(RING - 2) * DMA>();
   xgk::raw_barrier();
-  // A chunk's operands in registers: read while the chunk before it still adds to the state, so that the first product waits for
-  // nothing (18 reads of four waves at the head of a chunk were 0.3 us of it).
+  // A chunk's operands in registers: read while the chunk before it still adds to the state, in the order they are wanted, so that
+  // the first product waits for nothing.
   struct Ops {
-    float4 u[MH], r[MH], k[MH], b[MH], e[MH], el[MH], v0, o0;
+    float4 u, r, e, el, k, b, v0;
+    float o0[NO], flag;
     T v[4];
-    float flag;
   };
-  auto load = [&](int c, Ops& x) __attribute__((always_inline)) {
-    const char* at = lds + (c % RING) * SLOT;
+  uint32_t at_out = 0;   // the slot of the chunk that is read next
+  auto load = [&](Ops& x, int part) __attribute__((always_inline)) {
+    const char* at = lds + at_out;
     const float4* p4 = reinterpret_cast<const float4*>(at) + lane;
     const float* pe = reinterpret_cast<const float*>(at + FRAG);
-    const T* pv = reinterpret_cast<const T*>(at + FRAG + 1024) + 16 * ct + l16;
+    if (part == 0) x.flag = pe[D], x.u = p4[64 * par], x.e = *reinterpret_cast<const float4*>(pe + 16 * par + 4 * g4);
+    if (part == 1) x.el = *reinterpret_cast<const float4*>(pe + 2 * D + 16 * par + 4 * g4), x.r = p4[64 * (MT + par)];
+    if (part == 2) {
+      const T* pv = reinterpret_cast<const T*>(at + FRAG + 1024) + 16 * ct + l16;
 #pragma unroll
-    for (int i = 0; i < MH; ++i) x.u[i] = p4[64 * (2 * i + par)];
-#pragma unroll
-    for (int i = 0; i < MH; ++i) x.r[i] = p4[64 * (MT + 2 * i + par)];
-#pragma unroll
-    for (int i = 0; i < MH; ++i) {
-      const int m = 2 * i + par;
-      x.e[i] = *reinterpret_cast<const float4*>(pe + 16 * m + 4 * g4);
-      x.el[i] = *reinterpret_cast<const float4*>(pe + 2 * D + 16 * m + 4 * g4);
-      x.k[i] = p4[64 * (2 * MT + m)], x.b[i] = p4[64 * (3 * MT + m)];
+      for (int t = 0; t < 4; ++t) x.v[t] = pv[(4 * t + g4) * 32];
+      x.v0 = p4[64 * (4 * MT + ct)], x.b = p4[64 * (3 * MT + par)];
     }
-    x.v0 = p4[64 * (4 * MT + ct)], x.o0 = p4[64 * (4 * MT + 2 + ct)];
+    if (part == 3) {
+      x.k = p4[64 * (2 * MT + par)];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) x.v[t] = pv[(4 * t + g4) * 32];
-    x.flag = pe[D];
+      for (int i = 0; i < NO; ++i) x.o0[i] = reinterpret_cast<const float*>(p4 + 64 * (4 * MT + 2 + ct))[par + MT * i];
+      at_out = at_out == (RING - 1) * SLOT ? 0 : at_out + SLOT;
+    }
+  };
+  auto load_all = [&](Ops& x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load(x, i);
+  };
+  // The waves of a column tile hand each other y before a chunk's barrier, and the outputs' sums behind it: those are read, added and
+  // stored behind the next one, a part of the rows by each wave. Two buffers, in turn.
+  char* const hand = lds + RING * SLOT;
+  float o0_was[NO];   // of the chunk before, whose outputs are not stored yet: this wave's part of O,
+  int n_was = 0;      // and its rows
+  float* ob = o + ((int64_t)q0 * H + h) * D + col + (int64_t)(4 * par + g4) * H * D;   // (the next one to be stored)
+  auto sums = [&](const char* at, float* out) __attribute__((always_inline)) {   // the outputs' sums of the column tile's waves
+    const float* p = reinterpret_cast<const float*>(at + (W + MT * ct) * 1024) + 64 * par + lane;
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      out[i] = p[64 * MT * i] + p[256 + 64 * MT * i];
+      if (MT == 4) out[i] += p[512] + p[768];
+    }
+  };
+  auto store = [&](const float* out) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NO; ++i)
+      if (4 * (par + MT * i) + g4 < n_was) ob[(int64_t)(4 * MT * i) * H * D] = out[i] + o0_was[i];
+    ob += (int64_t)C * H * D;
   };
   auto chunk = [&](int c, Ops& x, Ops& next) __attribute__((always_inline)) {
     const int n = min(C, qn - C * c);
-    float* ob = o + ((int64_t)(q0 + C * c) * H + h) * D + col;
-    // what the two waves of a column tile hand each other, two buffers in turn: y, and the outputs' sums
-    float4* ex = reinterpret_cast<float4*>(lds + RING * SLOT + (c & 1) * (kEx / 2)) + lane;
-    float4* exo = ex + 256;
+    char *now = hand + (c & 1) * HAND, *was = hand + (~c & 1) * HAND;
     auto meet = [&]() __attribute__((always_inline)) {   // the next chunk has landed, in every wave
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       xgk::wait_vmcnt<(RING - 2) * DMA>();
@@ -362,115 +412,122 @@ __global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(const float* _
     };
     if (__builtin_amdgcn_readfirstlane(x.flag != 0.f)) {
       const float* p = reinterpret_cast<const float*>(lds + (c % RING) * SLOT);
-      __syncthreads();   // (what the chunk before handed over has been read)
-      float* xs = reinterpret_cast<float*>(lds + RING * SLOT);   // [wave][lane], sums into the state, then the outputs'
-      const float* rr0 = base + c * step + 4 * C * D;            // (r lies where V would: only half of that is in LDS)
+      __syncthreads();   // (what the chunk before handed over is there, and y has been read)
+      if (n_was) {
+        float out[NO];
+        sums(was, out);
+        store(out);
+      }
+      n_was = 0;
+      float* xs = reinterpret_cast<float*>(hand);                // [wave][lane], sums into the state, then the outputs' (below `sums`)
+      const float* rr0 = base + c * (step / 4) + 4 * C * D;      // (r lies where V would: only half of that is in LDS)
       const T* pv = reinterpret_cast<const T*>(lds + (c % RING) * SLOT + FRAG + 1024) + 16 * ct + l16;
+      float* to = ob - (int64_t)(4 * par + g4) * H * D;
+      auto tile_sum = [&](float* xs, float y) __attribute__((always_inline)) {
+        y += __shfl_xor(y, 16, 64);
+        y += __shfl_xor(y, 32, 64);
+        xs[64 * w + lane] = y;
+        __syncthreads();
+        y += xs[64 * (w ^ 1) + lane];
+        return MT == 4 ? y + (xs[64 * (w ^ 2) + lane] + xs[64 * (w ^ 3) + lane]) : y;
+      };
       for (int t = 0; t < n; ++t) {
         const float vv = ldf(pv + t * 32);
-        float uS = 0.f, sum = 0.f;
+        const int ch = t * D + 16 * par + 4 * g4;
+        float u[4], wr[4], b[4], k[4], rr[4], uS = 0.f, sum = 0.f;
+        ld4(p + 2 * C * D + ch, u);
 #pragma unroll
-        for (int i = 0; i < MH; ++i) {
-          float u[4];
-          ld4(p + 2 * C * D + t * D + 16 * (2 * i + par) + 4 * g4, u);
+        for (int r = 0; r < 4; ++r) uS = fmaf(u[r], S[r], uS);
+        uS = tile_sum(xs, uS);
+        ld4(p + ch, wr), ld4(p + ch + C * D, b), ld4(p + ch + 3 * C * D, k), ld4(rr0 + ch, rr);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) uS = fmaf(u[r], S[i][r], uS);
+        for (int r = 0; r < 4; ++r) {
+          S[r] = wr[r] * S[r] - b[r] * uS + k[r] * vv;
+          sum = fmaf(S[r], rr[r], sum);
         }
-        uS += __shfl_xor(uS, 16, 64);
-        uS += __shfl_xor(uS, 32, 64);
-        xs[64 * w + lane] = uS;
-        __syncthreads();
-        uS += xs[64 * (w ^ 1) + lane];
-#pragma unroll
-        for (int i = 0; i < MH; ++i) {
-          float wr[4], b[4], k[4], rr[4];
-          const int ch = t * D + 16 * (2 * i + par) + 4 * g4;
-          ld4(p + ch, wr), ld4(p + ch + C * D, b), ld4(p + ch + 3 * C * D, k), ld4(rr0 + ch, rr);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            S[i][r] = wr[r] * S[i][r] - b[r] * uS + k[r] * vv;
-            sum = fmaf(S[i][r], rr[r], sum);
-          }
-        }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        xs[256 + 64 * w + lane] = sum;
-        __syncthreads();
-        sum += xs[256 + 64 * (w ^ 1) + lane];
-        if (par == 0 && g4 == 0) ob[(int64_t)t * H * D] = sum;
+        sum = tile_sum(xs + 64 * W, sum);
+        if (par == 0 && g4 == 0) to[(int64_t)t * H * D] = sum;
       }
-      issue(c + RING - 1);
+      ob += (int64_t)C * H * D;
+      issue();
       meet();
-      load(c + 1, next);
+      load_all(next);
       return;
     }
-    // one chain each over this wave's 16s of the state's rows (the even ones, or the odd ones)
-    // (between its products the loads of the chunk RING - 1 on, into the slot of the chunk before, which every wave is past)
-    f32x4_t yc = {0.f, 0.f, 0.f, 0.f}, oc = yc;
+    // one chain over this wave's 16 of the state's rows; between its products the loads of the chunk RING - 1 on, into the slot of the
+    // chunk before, which every wave is past, and E S
+    f32x4_t yc = {0.f, 0.f, 0.f, 0.f}, oc = yc, ES;
+    auto mul = [&](const float4& a, const f32x4_t& y, int q, f32x4_t z) __attribute__((always_inline)) {
+      return mfma_f32(q == 0 ? a.x : q == 1 ? a.y : q == 2 ? a.z : a.w, y[q], z);
+    };
+    const char* ahead = operands();
 #pragma unroll
-    for (int q = 0; q < 4 * MH; ++q) {
-      const float4 u = x.u[q / 4];
-      yc = mfma_f32(q % 4 == 0 ? u.x : q % 4 == 1 ? u.y : q % 4 == 2 ? u.z : u.w, S[q / 4][q % 4], yc);
+    for (int q = 0; q < 4; ++q) {
+      yc = mul(x.u, S, q, yc);
 #pragma unroll
-      for (int i = q * DMA / (4 * MH); i < (q + 1) * DMA / (4 * MH); ++i) issue1(c + RING - 1, i);
+      for (int i = q * DMA / 4; i < (q + 1) * DMA / 4; ++i) issue1(i, ahead);
     }
-#pragma unroll
-    for (int i = 0; i < MH; ++i) {
-      oc = mfma_f32(x.r[i].x, S[i][0], oc), oc = mfma_f32(x.r[i].y, S[i][1], oc);
-      oc = mfma_f32(x.r[i].z, S[i][2], oc), oc = mfma_f32(x.r[i].w, S[i][3], oc);
-    }
+    issued();
+    ES = f32x4_t{prod_times({x.e.x, x.el.x}, S[0]), prod_times({x.e.y, x.el.y}, S[1]), prod_times({x.e.z, x.el.z}, S[2]),
+                 prod_times({x.e.w, x.el.w}, S[3])};
+    asm volatile("" : "+v"(ES));   // (formed here, beside the products, and not where it is used)
+    float4* ex = reinterpret_cast<float4*>(now) + lane;
     ex[64 * w] = make_float4(yc[0], yc[1], yc[2], yc[3]);
-    // E S behind the products with S; then what is taken out, summed up by itself, then the tokens' terms in their order
+    // the outputs' products with S: one half while y is on its way to the other waves, one while theirs is on its way here
+    oc = mul(x.r, S, 0, oc), oc = mul(x.r, S, 1, oc);
+    f32x4_t v;
 #pragma unroll
-    for (int i = 0; i < MH; ++i) {
-      S[i][0] = prod_times({x.e[i].x, x.el[i].x}, S[i][0]), S[i][1] = prod_times({x.e[i].y, x.el[i].y}, S[i][1]);
-      S[i][2] = prod_times({x.e[i].z, x.el[i].z}, S[i][2]), S[i][3] = prod_times({x.e[i].w, x.el[i].w}, S[i][3]);
-    }
-    if (par) exo[64 * ct] = make_float4(oc[0], oc[1], oc[2], oc[3]);
-    float v[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = ldf(&x.v[t]);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = 4 * t + g4 < n ? v[t] : 0.f;
+    for (int t = 0; t < 4; ++t) v[t] = 4 * t + g4 < n ? ldf(&x.v[t]) : 0.f;
+    __builtin_amdgcn_sched_barrier(0);
     meet();
-    const float4 yo = ex[64 * (w ^ 1)], oo = exo[64 * ct];
-    load(c + 1, next);
-    const float y[4] = {yc[0] + yo.x + x.v0.x, yc[1] + yo.y + x.v0.y, yc[2] + yo.z + x.v0.z, yc[3] + yo.w + x.v0.w};
-    f32x4_t by[MH];
+    const float4 y1 = ex[64 * (w ^ 1)];
+    float4 y2 = make_float4(0.f, 0.f, 0.f, 0.f), y3 = y2;
+    if (MT == 4) y2 = ex[64 * (w ^ 2)], y3 = ex[64 * (w ^ 3)];
+    float out[NO];
+    sums(was, out);
+    __builtin_amdgcn_sched_barrier(0);
+    oc = mul(x.r, S, 2, oc), oc = mul(x.r, S, 3, oc);
+    // what is taken out, summed up by itself, then the tokens' terms in their order; the next chunk is read meanwhile
+    const f32x4_t y = {((yc[0] + y1.x) + (y2.x + y3.x)) + x.v0.x, ((yc[1] + y1.y) + (y2.y + y3.y)) + x.v0.y,
+                       ((yc[2] + y1.z) + (y2.z + y3.z)) + x.v0.z, ((yc[3] + y1.w) + (y2.w + y3.w)) + x.v0.w};
+    f32x4_t by = mul(x.b, y, 0, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    __builtin_amdgcn_sched_barrier(0);
+    load(next, 0);
+    by = mul(x.b, y, 1, by);
+    __builtin_amdgcn_sched_barrier(0);
+    load(next, 1);
+    by = mul(x.b, y, 2, by);
+    __builtin_amdgcn_sched_barrier(0);
+    load(next, 2);
+    by = mul(x.b, y, 3, by);
+    __builtin_amdgcn_sched_barrier(0);
+    load(next, 3);
+    float* exo = reinterpret_cast<float*>(now) + 256 * (W + w) + lane;   // (row by row: a wave reads one of the four, or two)
+    exo[0] = oc[0], exo[64] = oc[1], exo[128] = oc[2], exo[192] = oc[3];
+    S = mul(x.k, v, 0, ES + by);
+    S = mul(x.k, v, 1, S);
+    if (n_was) store(out);
+    S = mul(x.k, v, 2, S);
+    S = mul(x.k, v, 3, S);
 #pragma unroll
-    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].x, y[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].y, y[1], by[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].z, y[2], by[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) by[i] = mfma_f32(x.b[i].w, y[3], by[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].x, v[0], S[i] + by[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].y, v[1], S[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].z, v[2], S[i]);
-#pragma unroll
-    for (int i = 0; i < MH; ++i) S[i] = mfma_f32(x.k[i].w, v[3], S[i]);
-    if (par == 0) {
-      const float out[4] = {oc[0] + oo.x + x.o0.x, oc[1] + oo.y + x.o0.y, oc[2] + oo.z + x.o0.z, oc[3] + oo.w + x.o0.w};
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (4 * r + g4 < n) ob[(int64_t)(4 * r + g4) * H * D] = out[r];
-    }
+    for (int i = 0; i < NO; ++i) o0_was[i] = x.o0[i];
+    n_was = n;
   };
   Ops x0, x1;
-  load(0, x0);
+  load_all(x0);
   for (int c = 0; c < nch; c += 2) {
     chunk(c, x0, x1);
     if (c + 1 < nch) chunk(c + 1, x1, x0);
   }
   xgk::wait_vmcnt<0>();   // (no load may land after the workgroup's LDS is given on)
+  __syncthreads();
+  if (n_was) {
+    float out[NO];
+    sums(hand + (~nch & 1) * HAND, out);
+    store(out);
+  }
 #pragma unroll
-  for (int i = 0; i < MH; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) Sg[(16 * (2 * i + par) + 4 * g4 + r) * D] = S[i][r];
+  for (int r = 0; r < 4; ++r) Sg[r * D] = S[r];
 }
 
 // ================================================================== host launchers
@@ -490,7 +547,7 @@ int delta_chunk(const void* proj, bool f32, int64_t ld, int off_r, int off_k, in
   XGM_DISPATCH_T(f32, delta_chunk_prep_kernel<T, D><<<dim3(H, nc, ns), 64, 0, st>>>((const T*)proj, ld, off_r, off_k, off_v, \
                                                                                     off_a, (const T*)wl, ld_wl, a_bias, w0, \
                                                                                     qsl, slots, scratch, H);                \
-                 delta_chunk_scan_kernel<T, D><<<dim3(H, ns, D / 32), 256, 0, st>>>(scratch, (const T*)proj, ld, off_v, state, qsl, \
+                 delta_chunk_scan_kernel<T, D><<<dim3(H, ns, D / 32), 8 * D, 0, st>>>(scratch, (const T*)proj, ld, off_v, state, qsl, \
                                                                               seq_lens, slots, o, H);)                       \
   return 0;
   if (D == 32) { XGM_DC(32) }

@@ -81,6 +81,21 @@ def test_values_out_of_range_reach_what_the_token_loop_lets_them_reach(where, va
     assert torch.equal(torch.isfinite(got[21:].cpu()), torch.isfinite(ref[21:].float()))
 
 
+@pytest.mark.parametrize("by_token", [[0], [6], [2, 3], [0, 2, 4, 6], [1, 3, 5], list(range(7))], ids=str)
+@pytest.mark.parametrize("D", [32, 64])
+def test_chunks_run_token_by_token_between_others(by_token, D):
+    """A chunk's outputs are stored by the one that follows it: either may be one that runs token by token (an r of 2^29)."""
+    large = [min(16 * c + 5 * c % 13, 99) for c in by_token]
+    def tweak(x):
+        x["r"][large, 3::D] = 2.0 ** 29
+    got, st, state, t = case([(7, 100)], 2, D, torch.bfloat16, torch.Generator().manual_seed(D + len(by_token)), tweak)
+    o, S = reference(t, state[1].to(F64))
+    rest = [i for i in range(100) if i not in large]
+    close(got[rest], o[rest])
+    close(got[large], o[large])
+    close(st[1], S)
+
+
 @pytest.mark.parametrize("mid", [-4.0, 0.0, 4.0])
 @pytest.mark.parametrize("H,D", [(4, 32), (4, 64)])
 def test_errors_are_those_of_the_token_loop(mid, H, D, monkeypatch):
