@@ -258,7 +258,13 @@ __global__ void __launch_bounds__(256 * GH) prefill_attn_kernel(
 //     halving the serial tile chain of the heaviest (last) row tile;
 //   * softmax in base 2 with the scale folded into one FMA, row max / sum across the
 //     two lane halves by v_permlane32_swap, and the O rescale skipped exactly when no
-//     row of the wave raised its max (ballot).
+//     row of the wave raised its max (ballot);
+//   * 8 waves of one key phase: the second four run one barrier behind the first, so that
+//     a SIMD's two waves are never both at their products or both at their softmax.
+// Bound by the two pipes' work of a tile, 1020 clocks a wave of matrix products and 1000 of vector instructions, and the power limit.
+// us before / now (all waves in step; 32 query heads, 8 kv heads): 4 x 2048 tokens 195 / 185, 8192 572 / 525, 2048 52 / 50, 512
+// (two key phases, in step) 15.3 / 14.9, 4 x 512 behind 1500 83 / 80. In pairs of waves or every second one behind instead, which
+// share no SIMD: 217 and 640 for the first two.
 // NW waves = GH query heads (one GQA group slice) x NW/GH/KS 32-row blocks x KS.
 // ---------------------------------------------------------------------------
 template <int NW, int GH, int KS, int NSLOT>
@@ -272,6 +278,8 @@ struct Pf2Cfg {
   static constexpr int NDMA = WROWS / 4;        // 1-KiB DMAs per wave per slot, each of K and V
   static constexpr int TILE = BN * D * 2;       // bytes of one K (or V) 64-key tile
   static constexpr int SLOT = 2 * KS * TILE;    // [K phase 0 .. KS-1][V phase 0 .. KS-1]
+  static constexpr bool PP = NW == 8 && KS == 1;  // two halves of the waves, one barrier apart
+  static_assert(!PP || NSLOT == 4, "tiles j - 1 .. j + 2 in the ring");
   static_assert(NW % (GH * KS) == 0 && WROWS % 4 == 0 && WROWS <= 16 && NSLOT >= 2 && NSLOT <= 4, "wave layout");
   static_assert(NSLOT * SLOT <= 160 * 1024, "LDS");
 };
@@ -310,6 +318,28 @@ __device__ __forceinline__ float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 #else
   return x;
+#endif
+}
+
+// o *= a unless `rows` is 0, in o's registers and one basic block: around a branch hipcc keeps the accumulators twice, and copies
+// them in every round that passes it. Not within 16 matrix instructions of the one that wrote o (hipcc's hazard pass does not look
+// into the statement).
+__device__ __forceinline__ void scale_if(uint64_t rows, f32x16_t& o, float a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  float x0 = o[0], x1 = o[1], x2 = o[2], x3 = o[3], x4 = o[4], x5 = o[5], x6 = o[6], x7 = o[7], x8 = o[8], x9 = o[9], x10 = o[10],
+        x11 = o[11], x12 = o[12], x13 = o[13], x14 = o[14], x15 = o[15];
+  asm volatile(
+      "s_cmp_eq_u64 %17, 0\n\ts_cbranch_scc1 .Lkeep%=\n\t"
+      "v_mul_f32 %0, %16, %0\n\tv_mul_f32 %1, %16, %1\n\tv_mul_f32 %2, %16, %2\n\tv_mul_f32 %3, %16, %3\n\t"
+      "v_mul_f32 %4, %16, %4\n\tv_mul_f32 %5, %16, %5\n\tv_mul_f32 %6, %16, %6\n\tv_mul_f32 %7, %16, %7\n\t"
+      "v_mul_f32 %8, %16, %8\n\tv_mul_f32 %9, %16, %9\n\tv_mul_f32 %10, %16, %10\n\tv_mul_f32 %11, %16, %11\n\t"
+      "v_mul_f32 %12, %16, %12\n\tv_mul_f32 %13, %16, %13\n\tv_mul_f32 %14, %16, %14\n\tv_mul_f32 %15, %16, %15\n"
+      ".Lkeep%=:"
+      : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3), "+v"(x4), "+v"(x5), "+v"(x6), "+v"(x7), "+v"(x8), "+v"(x9), "+v"(x10), "+v"(x11),
+        "+v"(x12), "+v"(x13), "+v"(x14), "+v"(x15)
+      : "v"(a), "s"(rows)
+      : "scc");
+  o = f32x16_t{x0, x1, x2, x3, x4, x5, x6, x7, x8, x9, x10, x11, x12, x13, x14, x15};
 #endif
 }
 
@@ -372,22 +402,25 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
   const int nslots = (ntiles + KS - 1) / KS;               // ring fills (super-tiles)
   const int32_t* btr = block_tables + static_cast<int64_t>(s) * bt_stride;
 
-  auto issue = [&](int t) {  // super-tile t: keys [t * SK, + SK)
-    char* kb = lds + (t % NSLOT) * C::SLOT;
-    const int key0 = min(t * C::SK + w * C::WROWS, L - 1);
+  const uint32_t ring = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)lds));
+  uint32_t from[C::NDMA], rel[C::NDMA];  // this lane's share of the wave's DMAs: bytes within a row, and the row
+#pragma unroll
+  for (int i = 0; i < C::NDMA; ++i) {
+    rel[i] = 4 * i + (lane >> 4);
+    from[i] = ((lane & 15) ^ pf2_xsw((w * C::WROWS + rel[i]) & 63)) * 16;
+  }
+  auto issue = [&](int t) __attribute__((always_inline)) {  // super-tile t: keys [t * SK, + SK)
+    const int key0 = min(t * C::SK + w * C::WROWS, L - 1), last = L - 1 - key0;
     const int pidx = key0 / bs;
     const int pg = btr[pidx];  // wave-uniform: scalar load
-    const int64_t pbase = (static_cast<int64_t>(pg) * Hkv + kvh) * bs - static_cast<int64_t>(pidx) * bs;
+    const int64_t at = ((static_cast<int64_t>(pg) * Hkv + kvh) * bs + (key0 - pidx * bs)) * (D * 2);
+    // phase srow / 64, row srow % 64 of its tile
+    const uint32_t dst = ring + (t % NSLOT) * C::SLOT + (w * C::WROWS >> 6) * C::TILE + (w * C::WROWS & 63) * 256;
 #pragma unroll
     for (int i = 0; i < C::NDMA; ++i) {
-      const int srow = w * C::WROWS + 4 * i + (lane >> 4);  // row in the super-tile
-      const int kabs = min(t * C::SK + srow, L - 1);
-      const int ch = (lane & 15) ^ pf2_xsw(srow & 63);
-      const int64_t off = (pbase + kabs) * D + ch * 8;  // kabs lies in page pidx
-      // phase srow / 64, row srow % 64 of its tile
-      char* dst = kb + (srow >> 6) * C::TILE + ((w * C::WROWS + 4 * i) & 63) * 256;
-      glds16(kc + off, dst);
-      glds16(vc + off, dst + KS * C::TILE);
+      const uint32_t off = min(static_cast<int>(rel[i]), last) * (D * 2) + from[i];
+      glds16_at(reinterpret_cast<const char*>(kc) + at, off, dst + i * 1024);
+      glds16_at(reinterpret_cast<const char*>(vc) + at, off, dst + i * 1024 + KS * C::TILE);
     }
   };
 
@@ -398,125 +431,196 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
     for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
   float m = -INFINITY, l = 0.f;  // m in raw score units (scale applied inside exp2)
 
-  wait_vmcnt<0>();  // Q fragments landed; from here on only the DMAs are counted
-#pragma unroll
-  for (int p = 0; p < NSLOT - 1; ++p)
-    if (p < nslots) issue(p);
-
+  // lane byte offsets into a tile (image (b)); per-read parts are one XOR with a
+  // constant: K chunk 2 ks + hf -> ^ (ks << 5); V chunk 4 db + .. -> ^ (db << 6)
   const int g = lane >> 4, gi = lane & 15;
   const int tq = gi >> 2, tp = gi & 3;
-  for (int j = 0; j < nslots; ++j) {
-    // own DMAs of super-tile j done (later ones may stay in flight), then everyone's
-    {
-      const int ahead = min(NSLOT - 2, nslots - 1 - j);  // later super-tiles issued so far
-      if constexpr (NSLOT >= 4) {
-        if (ahead >= 2) wait_vmcnt<4 * C::NDMA>();
-        else if (ahead == 1) wait_vmcnt<2 * C::NDMA>();
-        else wait_vmcnt<0>();
-      } else if constexpr (NSLOT == 3) {
-        if (ahead >= 1) wait_vmcnt<2 * C::NDMA>();
-        else wait_vmcnt<0>();
-      } else {
-        wait_vmcnt<0>();
-      }
+  const uint32_t k_lane = (r * 256) ^ (static_cast<uint32_t>(hf ^ pf2_xsw(r)) << 4);
+  const uint32_t v_row = KS * C::TILE + (4 * hf + tq) * 256 + 8 * (tp & 1);
+  const uint32_t v_lane0 = (v_row + ((((2 * (g & 1) + (tp >> 1)) ^ (hf & 3)) << 4))) | (tq << 6);
+  const uint32_t v_lane1 = (v_row + 8 * 256 + ((((2 * (g & 1) + (tp >> 1)) ^ ((hf + 2) & 3)) << 4))) | (tq << 6);
+  f32x16_t sacc[2];  // S^T of a tile: two 32-key blocks
+  uint4 pb[4];       // its P^T as bf16: k-step (kb, ss) = accumulator registers 8 ss .. 8 ss + 7 of block kb
+  auto read_k = [&](uint32_t at, int kb, uint4* kf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) kf[ks] = *reinterpret_cast<const uint4*>(lds + at + (k_lane ^ (ks << 5)) + kb * 8192);
+  };
+  auto mul_k = [&](int kb, const uint4* kf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) sacc[kb] = mfma32x32x16(as_frag(kf[ks]), qf[ks], sacc[kb]);
+  };
+  auto read_v = [&](uint32_t at, int step, bf16x8_t* vf) __attribute__((always_inline)) {
+    // rows kb*32 + 16 ss + 4 hf + tq (elements 0..3) and + 8 (elements 4..7); step = 2 kb + ss
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) {
+      const uint32_t ro = at + step * 16 * 256;
+      const bf16x4_t a0 = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds + ((v_lane0 ^ (db << 6)) + ro)));
+      const bf16x4_t a1 = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds + ((v_lane1 ^ (db << 6)) + ro)));
+      vf[db] = bf16x8_t{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
     }
-    raw_barrier();
-    if (j + NSLOT - 1 < nslots) issue(j + NSLOT - 1);
-    const int tile = j * KS + kp;
+  };
+  auto mul_v = [&](int step, const bf16x8_t* vf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) o[db] = mfma32x32x16(vf[db], as_frag(pb[step]), o[db]);
+  };
+  // online softmax (base 2, scale folded into one FMA) of tile `tile` on this lane's query row. The reference is the maximum itself:
+  // the largest weight, 1, is then exact in bf16 (a reference that lags behind costs 2 to 20 % of the result's error at scores of spread 1 to
+  // 3, and gains 2 %)
+  auto softmax = [&](int tile) __attribute__((always_inline)) {
     const int kv0 = tile * C::BN;
-    if (tile >= ntiles || kv0 > wave_hi) continue;  // wave-uniform: nothing of this tile is visible
-    // lane byte offsets into the tile (image (b)); per-read parts are one XOR with a
-    // constant: K chunk 2 ks + hf -> ^ (ks << 5); V chunk 4 db + .. -> ^ (db << 6)
-    const uint32_t kt_off = (j % NSLOT) * C::SLOT + kp * C::TILE;
-    const uint32_t k_lane = (kt_off + r * 256) ^ (static_cast<uint32_t>(hf ^ pf2_xsw(r)) << 4);
-    const uint32_t v_row = kt_off + KS * C::TILE + (4 * hf + tq) * 256 + 8 * (tp & 1);
-    const uint32_t v_lane0 = (v_row + ((((2 * (g & 1) + (tp >> 1)) ^ (hf & 3)) << 4))) | (tq << 6);
-    const uint32_t v_lane1 = (v_row + 8 * 256 + ((((2 * (g & 1) + (tp >> 1)) ^ ((hf + 2) & 3)) << 4))) | (tq << 6);
-
-    // ---- S^T = K . Q^T: two 32-key blocks
-    f32x16_t sacc[2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        const uint4 kf = *reinterpret_cast<const uint4*>(lds + ((k_lane ^ (ks << 5)) + kb * 8192));
-        sacc[kb] = mfma32x32x16(as_frag(kf), qf[ks], sacc[kb]);
-      }
-      sched_fence();  // bound the hoisted fragment reads (registers)
-    }
-    // ---- online softmax (base 2, scale folded into one FMA) on this lane's query row
     const bool need_mask = kv0 + C::BN - 1 > wave_lo || kv0 + C::BN > L;
-    float mx = -INFINITY;
     if (need_mask) {
       // key kv0 + 4 hf + c (c a per-register constant) is visible iff c <= lim - kv0 - 4 hf
       const int vis = lim - kv0 - 4 * hf;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
+        for (int e = 0; e < 16; ++e)
           if (kb * 32 + (e & 3) + 8 * (e >> 2) > vis) sacc[kb][e] = -INFINITY;
-          mx = fmaxf(mx, sacc[kb][e]);
-        }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
     }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
     mx = xor32_max(mx);
+    const uint64_t raised = __builtin_amdgcn_ballot_w64(mx > m);
     const float m_new = fmaxf(m, mx);
-    const float nms = m_new == -INFINITY ? 0.f : -m_new * scale_log2;
-    // exact rescale skip: no row of the wave raised its max -> alpha = 1 everywhere
-    if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
-      const float alpha = fast_exp2(fmaf(m, scale_log2, nms));  // m = -inf -> 0
-      l *= alpha;
+    const float alpha = mx > m ? fast_exp2((m - m_new) * scale_log2) : 1.f;  // m = -inf -> 0
+    l *= alpha;
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
-      m = m_new;
-    }
-    // pairwise: the fma / add pairs issue as packed v_pk_fma_f32 / v_pk_add_f32
-    f32x2v_t rs2 = {0.f, 0.f};
-    const f32x2v_t sc2 = {scale_log2, scale_log2}, nm2 = {nms, nms};
+    for (int db = 0; db < D / 32; ++db) scale_if(raised, o[db], alpha);
+    m = m_new;
+    const float nms = m == -INFINITY ? 0.f : -m * scale_log2;
+    float rs[2] = {0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
-        f32x2v_t x = {sacc[kb][e], sacc[kb][e + 1]};
-        x = x * sc2 + nm2;
-        x[0] = fast_exp2(x[0]);
-        x[1] = fast_exp2(x[1]);
-        sacc[kb][e] = x[0];
-        sacc[kb][e + 1] = x[1];
-        rs2 += x;
+        const float x0 = fast_exp2(fmaf(sacc[kb][e], scale_log2, nms)), x1 = fast_exp2(fmaf(sacc[kb][e + 1], scale_log2, nms));
+        rs[0] += x0, rs[1] += x1;
+        reinterpret_cast<uint32_t*>(&pb[2 * kb + (e >> 3)])[(e & 7) >> 1] = pack2(x0, x1);
       }
-    l += xor32_sum(rs2[0] + rs2[1]);
+    l += xor32_sum(rs[0] + rs[1]);
+  };
 
-    // ---- O^T += V^T . P^T: k-step (kb, ss) takes accumulator registers 8 ss .. 8 ss + 7
+  wait_vmcnt<0>();  // Q fragments landed; from here on only the DMAs are counted
+  if constexpr (C::PP) {
+    // Waves w and w + 4 share a SIMD. In step with each other, their products and their softmax met on one pipe while the other
+    // idled; so the second four run one barrier behind: one half's products are the other half's softmax. Between barriers 2 j and
+    // 2 j + 1 the first four add tile j - 1's P^T V^T and form tile j's scores, then, up to 2 j + 2, that tile's P^T. Tile j has landed
+    // at barrier 2 j for every wave, and its slot is free behind 2 j + 4.
+    auto landed = [&](int t) __attribute__((always_inline)) {  // own DMAs of tile t (those up to t + 1 have been issued)
+      if (t + 1 < nslots) wait_vmcnt<2 * C::NDMA>();
+      else wait_vmcnt<0>();
+    };
+    const int n_vis = min(ntiles, wave_hi / C::BN + 1);  // tiles with a key that some row of the wave sees
+    bf16x8_t vf[2][D / 32];  // the next products' first fragments
+    auto scores = [&](uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb) {
+        uint4 kf[D / 16];
+        read_k(at, kb, kf);
+        mul_k(kb, kf);
+        sched_fence();  // bound the hoisted fragment reads (registers)
+      }
+    };
+    auto ask = [&](int j) __attribute__((always_inline)) {
+      if (j + 2 < nslots) issue(j + 2);
+    };
+    auto pass = [&](int j, bool mine) __attribute__((always_inline)) {
+      if (mine && j + 1 < nslots) landed(j + 1);
+      raw_barrier();
+    };
+    auto weights = [&](int j) __attribute__((always_inline)) {
+      softmax(j);
 #pragma unroll
-      for (int ss = 0; ss < 2; ++ss) {
-        uint4 pb;
-        pb.x = pack2(sacc[kb][8 * ss + 0], sacc[kb][8 * ss + 1]);
-        pb.y = pack2(sacc[kb][8 * ss + 2], sacc[kb][8 * ss + 3]);
-        pb.z = pack2(sacc[kb][8 * ss + 4], sacc[kb][8 * ss + 5]);
-        pb.w = pack2(sacc[kb][8 * ss + 6], sacc[kb][8 * ss + 7]);
-        const bf16x8_t pf = as_frag(pb);
-        // rows kb*32 + 16 ss + 4 hf + tq (elements 0..3) and + 8 (elements 4..7)
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(pb[i].x), "+v"(pb[i].y), "+v"(pb[i].z), "+v"(pb[i].w));  // (here, not behind the barrier)
+      sched_fence();
+      const uint32_t at = (j % NSLOT) * C::SLOT;
+      read_v(at, 0, vf[0]), read_v(at, 1, vf[1]);
+    };
+    const bool late = w >= 4;
+    issue(0);
+    if (nslots > 1) issue(1);
+    landed(0);
+    raw_barrier();
+    if (late) raw_barrier();
+    ask(0);
+    scores(0);
+    pass(0, late);
+    weights(0);
+    pass(0, !late);
+    for (int j = 1; j < n_vis; ++j) {
+      ask(j);
+      const uint32_t at = (j % NSLOT) * C::SLOT, was = ((j + NSLOT - 1) % NSLOT) * C::SLOT;
+      {
+        bf16x8_t vg[D / 32];
+        uint4 kf[D / 16];
+        __builtin_amdgcn_s_setprio(1);  // (the matrix pipe is fed first: the other half's softmax has the slots between)
+        mul_v(0, vf[0]);
+        read_v(was, 2, vf[0]);
+        sched_fence();
+        mul_v(1, vf[1]);
+        read_v(was, 3, vg);
+        sched_fence();
+        mul_v(2, vf[0]);
+        read_k(at, 0, kf);
+        sched_fence();
+        mul_v(3, vg);
+        sched_fence();
+        mul_k(0, kf);
+        read_k(at, 1, kf);
+        mul_k(1, kf);
+        __builtin_amdgcn_s_setprio(0);
+      }
+      pass(j, late);
+      weights(j);
+      pass(j, !late);
+    }
+    ask(n_vis);
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) {
-          const uint32_t ro = (kb * 32 + 16 * ss) * 256;
-          const bf16x4_t a0 = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds + ((v_lane0 ^ (db << 6)) + ro)));
-          const bf16x4_t a1 = lds_read_tr16(reinterpret_cast<const uint16_t*>(lds + ((v_lane1 ^ (db << 6)) + ro)));
-          const bf16x8_t vf = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-          o[db] = mfma32x32x16(vf, pf, o[db]);
-        }
+    for (int step = 0; step < 4; ++step) {
+      if (step >= 2) read_v(((n_vis - 1) % NSLOT) * C::SLOT, step, vf[step & 1]);
+      mul_v(step, vf[step & 1]);
+    }
+    for (int j = n_vis; j < nslots; ++j) {  // nothing of these tiles is visible
+      if (j > n_vis) ask(j);
+      pass(j, late);
+      pass(j, !late);
+    }
+    if (!late) raw_barrier();
+  } else {
+#pragma unroll
+    for (int p = 0; p < NSLOT - 1; ++p)
+      if (p < nslots) issue(p);
+    for (int j = 0; j < nslots; ++j) {
+      // own DMAs of super-tile j done (later ones may stay in flight), then everyone's
+      if (NSLOT == 3 && j + 1 < nslots) wait_vmcnt<2 * C::NDMA>();
+      else wait_vmcnt<0>();
+      raw_barrier();
+      if (j + NSLOT - 1 < nslots) issue(j + NSLOT - 1);
+      const int tile = j * KS + kp;
+      if (tile >= ntiles || tile * C::BN > wave_hi) continue;  // wave-uniform: nothing of this tile is visible
+      const uint32_t at = (j % NSLOT) * C::SLOT + kp * C::TILE;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        uint4 kf[D / 16];
+        read_k(at, kb, kf);
+        mul_k(kb, kf);
+        sched_fence();  // bound the hoisted fragment reads (registers)
+      }
+      softmax(tile);
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        bf16x8_t vf[D / 32];
+        read_v(at, step, vf);
+        mul_v(step, vf);
         sched_fence();
       }
+    }
   }
 
   if constexpr (KS > 1) {
@@ -601,7 +705,7 @@ int prefill_attention(const uint16_t* q, int64_t q_stride, const uint16_t* kc, c
       nw = 8;
       ks = wg8 >= 512 ? 1 : 2;
     }
-    if (ns == 0) ns = ks == 2 ? 2 : (nw == 8 ? 3 : 2);
+    if (ns == 0 || (ns == 3 && nw == 8)) ns = nw == 8 && ks == 1 ? 4 : 2;  // (three slots of 8 waves: four, what they run on)
     if (G % ghh != 0 || nw % (ghh * ks) != 0) return -1;
     const int bm = 32 * (nw / ghh / ks);
     const int tps = (max_q_len + bm - 1) / bm;
@@ -613,10 +717,10 @@ int prefill_attention(const uint16_t* q, int64_t q_stride, const uint16_t* kc, c
                      bt_stride, qsl, seq_lens, out, out_stride, num_seqs, Hq, Hkv, bs, sl2, tps, n_hg)
     const int code = ((ks * 10 + ns) * 10 + nw) * 10 + ghh;
     switch (code) {
-      case 1384: XGK_PF2(8, 4, 1, 3); break;
-      case 1382: XGK_PF2(8, 2, 1, 3); break;
-      case 1381: XGK_PF2(8, 1, 1, 3); break;
-      case 1388: XGK_PF2(8, 8, 1, 3); break;
+      case 1484: XGK_PF2(8, 4, 1, 4); break;
+      case 1482: XGK_PF2(8, 2, 1, 4); break;
+      case 1481: XGK_PF2(8, 1, 1, 4); break;
+      case 1488: XGK_PF2(8, 8, 1, 4); break;
       case 1244: XGK_PF2(4, 4, 1, 2); break;
       case 1242: XGK_PF2(4, 2, 1, 2); break;
       case 1241: XGK_PF2(4, 1, 1, 2); break;

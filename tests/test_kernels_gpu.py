@@ -208,6 +208,27 @@ def test_prefill_attention_spike_forces_rescale():
     torch.testing.assert_close(out.cpu().float(), ref.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("gh", [-82, -81, -88, -382, -1282, -42])
+@pytest.mark.parametrize("growth", [0.2, 3.0])   # of a row's largest score from one tile of 64 keys to the next, in powers of two
+@pytest.mark.parametrize("L", [1, 63, 64, 65, 128, 129, 193, 449])
+def test_prefill_attention_growing_scores(gh, growth, L):
+    """Maxima that grow slowly and quickly from tile to tile, at tile edges (every weight and sum is rescaled, or nearly none).
+    Against fp64: probabilities and outputs rounded to bf16, 2^-9 each, of the largest |V|."""
+    D, Hq, Hkv, ctx = 128, 8, 1, 70
+    kc, vc, bt = _paged([L + ctx], Hkv, D, 16)
+    q = rnd(L, Hq, D)
+    q[..., 0] = 8.0
+    for key in range(L + ctx):
+        kc[bt[0, key // 16], 0, key % 16, 0] = growth * (key // 64) * math.log(2.0) * math.sqrt(D) / 8.0
+    qsl, sl = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([0, L], [L + ctx]))
+    out = ops.prefill_attention(q, kc, vc, bt, qsl, sl, L, 1.0 / math.sqrt(D), gh=gh).cpu().double()
+    pages = bt[0].long().cpu()
+    k, v = (c.cpu()[pages, 0].reshape(-1, D)[:L + ctx].double() for c in (kc, vc))
+    s = q.cpu().double() @ k.t() / math.sqrt(D)
+    s.masked_fill_(torch.arange(L + ctx) > torch.arange(ctx, L + ctx)[:, None, None], -math.inf)
+    assert (out - s.softmax(-1) @ v).abs().max() <= 2 * 2.0 ** -9 * float(v.abs().max())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("V", [128256, 50257, 32000, 1000, 16387])
 def test_argmax_logprob(dtype, V):
