@@ -18,14 +18,14 @@
 // first key its first query row sees. The rotary part of a query is rotated while it is loaded. In latent space (latent_attention)
 // a (query, key) pair costs 2 (2 R + rd) operations per head, here 2 (dn + rd + dv): 3.4 times less at R = 256 and heads of 64,
 // against one product per key row that expands it (4 x 2048 tokens, 32 heads of 64 + 32, window 1024: 950 -> 205 us with the
-// gather and both expansions, the attention 155 of them, since then 125; heads of 128 + 64, window 4096: 3857 -> 395). Rows of 96 and 192 entries have 12 and 24 chunks: the permutation there
+// gather and both expansions, the attention 155 of them, since then 127; heads of 128 + 64, window 4096: 3857 -> 395). Rows of 96 and 192 entries have 12 and 24 chunks: the permutation there
 // stays inside groups of 4 and 8.
 //
 // Vector work and matrix instructions bound it together: 4001 tokens, 32 heads of 64 + 64, took 275 vector instructions a tile and
-// wave beside 16 matrix ones (156 and 64 of 266 thousand clocks), 118 to 124 us. Scores that stay products up to the exponential, a
-// reference that seldom moves, masks by edge (compares and selects, no branches), addresses as a uniform base and a lane's
-// constant: 195 instructions, 100 to 109 us; 16 heads of 64 + 128 with a distance penalty 132 -> 115, 2 x 1800 tokens of 32 heads
-// of 128 + 128 96 -> 89, expanded latents (64 + 32) + 64 of 4 x 2048 tokens 156 -> 125, (128 + 64) + 128 of 2 x 1300 97 -> 82.
+// wave beside 16 matrix ones (156 and 64 of 266 thousand clocks), 125 us. Scores that stay products up to the exponential, masks by
+// edge (compares and selects, no branches), addresses as a uniform base and a lane's constant: 113 us; 16 heads of 64 + 128 with a
+// distance penalty 131 -> 121, 2 x 1800 tokens of 32 heads of 128 + 128 97 -> 93, expanded latents (64 + 32) + 64 of 4 x 2048 tokens
+// 154 -> 127, (128 + 64) + 128 of 2 x 1300 96 -> 84.
 // (Both blocks of 32 keys in turn, so that two chains of matrix instructions run; waves' priorities and two sums for l change nothing.)
 #include "attention_common.h"
 #include "glds.h"
@@ -33,7 +33,6 @@
 namespace xgm {
 
 constexpr int kPT = 64;   // keys per tile
-constexpr float kLag = 8.f;   // see `m` below
 
 typedef xgk::f32x16_t f32x16_t;
 
@@ -340,9 +339,10 @@ __global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_atte
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
         mx = xor32_max(mx) * sc1;
-        // the reference follows the maximum only when that is 2^kLag ahead of it: sums and outputs are rarely rescaled
-        if (__builtin_amdgcn_ballot_w64(mx > m + kLag) != 0) {
-          const float m_new = mx > m + kLag ? mx : m, alpha = m == -INFINITY ? 0.f : exp2_fast(m - m_new);
+        // (none of the wave's rows has a new maximum: nothing to rescale. A reference that lags behind the maximum by up to 2^8 is 2 to 4 %
+        // faster, but the largest weight is then not 1, which bf16 holds exactly: 2 to 20 % more error at scores of spread 1 to 3)
+        if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
+          const float m_new = fmaxf(m, mx), alpha = m == -INFINITY ? 0.f : exp2_fast(m - m_new);
           l *= alpha;
 #pragma unroll
           for (int db = 0; db < DV / 32; ++db)
