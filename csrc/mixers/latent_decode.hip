@@ -134,9 +134,9 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(const LatentDecod
         mx = fmaxf(mx, sc[n][r]);
       }
     mx = column_max(mx);
-    // (the reference follows the maximum only when that is e^5 ahead: the sums are rarely rescaled)
-    if (__builtin_amdgcn_ballot_w64(mx > m + 5.f) != 0) {
-      const float mn = mx > m + 5.f ? mx : m, alpha = m == -INFINITY ? 0.f : __expf(m - mn);
+    // (no column of the wave has a new maximum: nothing to rescale. The reference is the maximum itself: the largest weight, 1, is exact in bf16)
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
+      const float mn = fmaxf(m, mx), alpha = m == -INFINITY ? 0.f : __expf(m - mn);
       l *= alpha, m = mn;
 #pragma unroll
       for (int mt = 0; mt < NMT; ++mt)
