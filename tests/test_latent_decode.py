@@ -66,6 +66,12 @@ def test_against_fp64(H, dn, rd, dv, R, rot, lens, window, bs, monkeypatch):
         assert bool((err <= bound).all()), (t, float((err / bound).max()))
 
 
+@pytest.mark.parametrize("T", [8, 9, 16, 17, 32, 33])
+def test_tokens_to_a_workgroup(T, monkeypatch):
+    """32 heads of 8, 16 and 32 tokens are where the value expansion takes one, two, four and eight tokens to a workgroup."""
+    test_against_fp64(32, 64, 32, 64, 256, 32, [20 + 7 * i % 45 for i in range(T)], 64, 16, monkeypatch)
+
+
 def test_other_steps_keep_the_general_kernels():
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
     sm = sq.SeqMeta(2, 1, i32([0, 1, 2]), i32([5, 9]), i32([0, 1]), i32([[0], [1]]), i32([0, 1]), i32([4, 8]), i32([4, 24]))
