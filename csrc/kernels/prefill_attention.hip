@@ -705,7 +705,7 @@ int prefill_attention(const uint16_t* q, int64_t q_stride, const uint16_t* kc, c
       nw = 8;
       ks = wg8 >= 512 ? 1 : 2;
     }
-    if (ns == 0 || (ns == 3 && nw == 8)) ns = nw == 8 && ks == 1 ? 4 : 2;  // (three slots of 8 waves: four, what they run on)
+    if (ns == 0 || (ns == 3 && nw == 8 && ks == 1)) ns = nw == 8 && ks == 1 ? 4 : 2;  // (three slots of 8 waves: four, what they run on)
     if (G % ghh != 0 || nw % (ghh * ks) != 0) return -1;
     const int bm = 32 * (nw / ghh / ks);
     const int tps = (max_q_len + bm - 1) / bm;
