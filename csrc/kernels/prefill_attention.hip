@@ -488,12 +488,12 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
     mx = xor32_max(mx);
     const uint64_t raised = __builtin_amdgcn_ballot_w64(mx > m);
     const float m_new = fmaxf(m, mx);
-    const float alpha = mx > m ? fast_exp2((m - m_new) * scale_log2) : 1.f;  // m = -inf -> 0
+    const float nms = m_new == -INFINITY ? 0.f : -m_new * scale_log2;
+    const float alpha = raised ? fast_exp2(fmaf(m, scale_log2, nms)) : 1.f;  // m = -inf -> 0
     l *= alpha;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) scale_if(raised, o[db], alpha);
     m = m_new;
-    const float nms = m == -INFINITY ? 0.f : -m * scale_log2;
     float rs[2] = {0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
