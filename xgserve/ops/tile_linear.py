@@ -23,7 +23,7 @@ from ._native import is_f32, mixers, native_device, on_current_device, stream_pt
 from .linear import PendingSum, cu_count
 
 # rows and columns of a workgroup's tile / 32 -> us per 64 of K and per tile
-_TILES = {(8, 8): (1.135, 0.02), (7, 8): (1.036, 0.02), (6, 8): (0.901, 0.02), (5, 8): (0.816, 0.02), (4, 8): (0.721, 0.02),
+_TILES = {(8, 8): (1.135, 0.02), (7, 8): (1.036, 0.02), (6, 8): (0.910, 0.02), (5, 8): (0.816, 0.02), (4, 8): (0.721, 0.02),
           (8, 6): (0.937, 0.02), (7, 6): (0.819, 0.61), (6, 6): (0.708, 0.98), (8, 4): (0.705, 0.10), (7, 4): (0.627, 1.11),
           (6, 4): (0.540, 1.13), (5, 4): (0.480, 1.19), (4, 4): (0.399, 1.62), (3, 4): (0.327, 1.90), (4, 2): (0.254, 1.57),
           (3, 2): (0.229, 0.46)}
