@@ -12,8 +12,9 @@
 // sub-chunk's own reciprocals (above 2^-90) is ever above 1. G is formed once per workgroup, three of its twelve 16 x 16 tiles a wave,
 // split, and handed on through LDS in the order of the lanes. State row 32 i + 8 g + 4 k + r is register r of lane group g in tile
 // 2 i + k, so that two tiles' registers are the B operand of C S as they lie; B^T and x come from LDS by transposed reads.
-// A chunk with an input out of range (2^28 and above, infinities, NaN), a sub-chunk below 2^-90, or a state above 1e36 runs
-// token by token.
+// A chunk with an input out of range (2^28 and above, infinities, NaN) or a sub-chunk below 2^-90 runs token by token, and so does a
+// wave whose state is too large for C S, which meets the decays only after its sum: above 2^92 it could leave fp32 (128 terms, C below
+// 2^28), above 2^40 what it leaves behind decays that underflow within the chunk could count.
 //
 // Error against fp64 (2-norm, outputs / carried state; chunks of 16 tokens in fp32 in brackets, then the token loop), 400 tokens of 8
 // heads of 128 x 64, A_log about 0 8.4e-8 / 6.3e-8 (8.8e-8 / 5.8e-8; 8.7e-8 / 6.2e-8), -0.5 8.4e-8 / 6.6e-8 (9.2e-8 / 6.9e-8; 8.8e-8 /
@@ -38,6 +39,7 @@ using xgk::mfma16x16x32;
 
 constexpr int kSsTok = 64, kSsSub = 16, kSsRing = 8;   // tokens per chunk and sub-chunk; chunks whose step sizes are held
 constexpr float kSsMinProd = 8.077935669463161e-28f;   // 2^-90
+constexpr float kSsMinChunk = 7.888609052210118e-31f, kSsMaxState = 4.951760157141521e27f, kSsMaxFaded = 1099511627776.f;   // 2^-100, 2^92, 2^40
 
 struct SsmChunkArgs {
   const bf16* rows;            // [x (H P) | B (G N) | C (G N)]
@@ -321,11 +323,11 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
     if (ci % 4 == 2) steps(ci + 2);
     __syncthreads();
     const bool slow = __builtin_amdgcn_readfirstlane(flags[ci & 1][0] | flags[ci & 1][1] | flags[ci & 1][2] | flags[ci & 1][3] | bad_step[rg]) != 0;
-    // a state that has left the range cannot be split: its wave goes token by token (a NaN stays one either way)
+    // (a NaN goes token by token too; a chunk's whole decay bounds all of its own)
     float top = 0.f;
 #pragma unroll
     for (int m = 0; m < MT; ++m) top = fmaxf(fmaxf(fabsf(S[m][0]), fabsf(S[m][1])), fmaxf(top, fmaxf(fabsf(S[m][2]), fabsf(S[m][3]))));
-    const bool wslow = slow || __any(!(top < 1e36f));
+    const bool wslow = slow || __any(!(top < (Eh[rg] >= kSsMinChunk ? kSsMaxState : kSsMaxFaded)));
     if (!SUMS && !slow) {
       // G^T of three of the twelve tiles: rows j = 32 q + 8 (i / 4) + 4 half + i % 4, columns token 16 b + l16
 #pragma unroll

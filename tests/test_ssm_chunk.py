@@ -98,3 +98,25 @@ def test_states_that_cannot_be_split(value):
     want, states = reference(args, portions, H, G, N, P)
     close(got[:, ~keep].float(), want[:, ~keep].float().to(F64))
     close(state[1, 1, :, 21].float(), states[0][1, :, 21].float().to(F64))
+
+
+@pytest.mark.parametrize("level", [0.6, 1.4])   # a chunk's decay is 2^-86 and 2^-192, no sub-chunk's past 2^-90
+@pytest.mark.parametrize("large", [1e28, 1e31, 9e35])
+def test_large_states_that_fade_before_large_rows_read_them(level, large):
+    """C S of a whole chunk would leave fp32 (or what is left of the state, its decays), where a token's own sum does not. Tokens from 8
+    on write nothing, so that every output is what is left of the state; C is 500 from token 24 on."""
+    portions, H, G, N, P = [(3, 150)], 2, 1, 128, 64
+    xbc, dt, bias, A, D, state = inputs(portions, H, G, N, P, level, 5)
+    dt[:], bias[:], A[:], D[:] = -0.4, 0.0, level, 0.0   # steps of 0.513: decays of e^-0.93 and e^-2.08
+    xbc[8:, :H * P] = 0
+    xbc[24:, H * P + N + 40] = 500.0
+    state[1, 1, :, 21] = 0
+    state[1, 1, 40, 21] = large
+    args = (xbc, dt, bias, A, D, state)
+    got, after = run(args, portions, H, G, N, P)
+    want, states = reference(args, portions, H, G, N, P)
+    assert bool(torch.isfinite(got).all()) and bool(torch.isfinite(after).all())
+    col, ref = got[:, P + 21].cpu().to(F64), want[:, P + 21]
+    seen = ref.abs() > 1e-30   # (a state's entry is a product of up to 150 roundings of decays, 2^-23 each with the step's own)
+    assert int(seen.sum()) > 40 and float(((col - ref).abs() / ref.abs())[seen].max()) < 150 * 2.0 ** -22
+    assert float((after[1].cpu().to(F64) - states[0]).abs().max()) <= 150 * 2.0 ** -22 * float(states[0].abs().max()) + 1e-37
