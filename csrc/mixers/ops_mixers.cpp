@@ -79,7 +79,7 @@ int64_t chunk_scan_scratch_floats(int, int, int, int, int, int);
 int chunk_scan_gates(const float*, const float*, const float*, const void*, int64_t, int, int, const float*, const float*,
                      const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int, int,
                      int, int, int, int, float*, hipStream_t);
-int64_t ssm_chunk_scratch_floats(int, int, int, int, int, int);
+int64_t ssm_chunk_scratch_floats(int, int, int, int, int);
 int ssm_chunk(const void*, int64_t, const void*, int64_t, const float*, const float*, const float*, float*, const int32_t*,
               const int32_t*, const int32_t*, float*, int, int, int, int, int, int, int, int, float*, hipStream_t);
 int chunk_scan_ssm(const void*, bool, int64_t, const void*, int64_t, const float*, const float*, const float*, float*,
@@ -442,9 +442,9 @@ PYBIND11_MODULE(_mixers, m) {
                                    P<float>(o), ns, max_q, T, H, dk, dv, seg, P<float>(scratch), S(st));
     check(rc, "chunk_scan_gates");
   });
-  m.def("ssm_chunk_scratch_floats", [](int T, int ns, int H, int N, int Pd, int seg) {
+  m.def("ssm_chunk_scratch_floats", [](int T, int H, int N, int Pd, int seg) {
     if (seg < 1) throw std::invalid_argument("ssm_chunk_scratch_floats: seg must be positive");
-    return xgm::ssm_chunk_scratch_floats(T, ns, H, N, Pd, seg);
+    return xgm::ssm_chunk_scratch_floats(T, H, N, Pd, seg);
   });
   m.def("chunk_scan_ssm", [](uintptr_t xbc, bool f32, int64_t ld_x, uintptr_t dt, int64_t ld_dt, uintptr_t dt_bias,
                              uintptr_t A_log, uintptr_t D, uintptr_t state, uintptr_t qsl, uintptr_t sl, uintptr_t slots,

@@ -22,9 +22,14 @@
 // parts below the first summed up by themselves, the chunk's terms added to E S as one sum, dt itself on G's diagonal, and the
 // leading bits of post x (top4).
 //
-// Long portions of few sequences run in segments side by side: a first launch sums every segment but the last up from a zero state (and
-// sets the incoming state aside), the second puts its state together from those in front of it and runs with outputs. Segment
-// slot of (sequence s, segment z): q0_s / seg + s + z, distinct for all segments of a step.
+// Long portions of few sequences run in segments side by side: a first launch sums every segment but the last up from a zero state, the
+// second puts its state together from those in front of it and runs with outputs. Segment z of a sequence of more than one has slot
+// 2 (q0 / seg) + z, which no other has: the next such sequence begins floor(q / seg) >= 1 segments on at least, and ceil(q / seg) is at
+// most twice that. Token (slot / 2 + 1) seg - 1 is one of the sequence's (z seg of its q tokens are in front of segment z), so a
+// workgroup of a slot finds its sequence. The incoming state, which the last segment's workgroup replaces, is set aside in the place
+// of that segment's sum, which nobody reads. Sequences of one segment (single tokens beside a prompt) have no part in the first
+// launch and their states are read in place. (With a workgroup per sequence and possible segment, and every sequence's state set aside,
+// 200 single tokens beside 256 of 64 heads took 448 us and 0.9 GB of scratch, now 290 and 34 MB.)
 //
 // Measured, heads of 128 x 64: 2521 ragged tokens of 64 heads 199 -> 75 us, 4 x 1024 of 128 276 -> 122, 4001 of 64 96. A chunk of one
 // workgroup is 5 us by itself, 3.9 where two share a unit: 1.9 of vector work (splitting, scales, range checks: 1100 instructions a
@@ -50,9 +55,8 @@ struct SsmChunkArgs {
   float* state;                // [slots, H, N, P]
   const int32_t *qsl, *seq_lens, *slots;
   float* o;                    // [T, H P]
-  int H, G, P, pass, nc, seg;
-  float *decay, *sums;         // per (segment, head): its whole decay; its sum in the order of the lanes (S of a zero state)
-  float* s_in;                 // per (sequence, head): the incoming state, likewise
+  int ns, H, G, P, pass, seg, slots_seg;   // slots_seg: slots of segments, in front of the sequences in the grid (0 in one pass)
+  float *decay, *sums;         // per (segment, head): its whole decay; its sum in the order of the lanes (S of a zero state; incoming S)
 };
 
 // granule (16 bytes) of a staged row: rows of 256 bytes and of 128; reads of 16 rows and transposed reads of 4 x 4 granules
@@ -136,13 +140,22 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
   __shared__ float Eh[kSsRing], El[kSsRing];
   __shared__ int bad_step[kSsRing], flags[2][4];
 
-  const int s = blockIdx.y / a.nc, z = blockIdx.y % a.nc, hx = blockIdx.x;
+  const int hx = blockIdx.x;
+  int s = (int)blockIdx.y - a.slots_seg, z = 0;
+  if (s < 0) {   // the sequence of the slot's token
+    const int tok = (blockIdx.y / 2 + 1) * a.seg - 1, l = threadIdx.x & 63;
+    s = 0;
+    for (int i = 0; i < a.ns; i += 64) s += __popcll(__ballot(i + l < a.ns && a.qsl[min(i + l, a.ns - 1) + 1] <= tok));
+    if (s >= a.ns) return;
+    z = blockIdx.y - 2 * (a.qsl[s] / a.seg);
+  }
   const int h = a.H % 8 == 0 ? (hx % 8) * (a.H / 8) + hx / 8 : hx;   // (an XCD takes neighbouring heads, which share B and C)
   const int q0 = a.qsl[s], qn = a.qsl[s + 1] - q0, slot = a.slots[s];
   const int c0 = z * a.seg, c1 = min(qn, c0 + a.seg), pass = SUMS ? 1 : a.pass;
-  if (slot < 0 || c0 >= qn) return;
-  const bool last_seg = c1 == qn;
-  if (SUMS && last_seg && z > 0) return;   // nobody reads its sum
+  if (slot < 0 || c0 < 0 || c0 >= qn) return;
+  const bool last_seg = c1 == qn, whole = qn <= a.seg;
+  if (a.slots_seg && whole == ((int)blockIdx.y < a.slots_seg)) return;   // (a slot's token of a sequence of one segment, and the other way round)
+  if (SUMS && last_seg) return;   // nobody reads its sum
   const int ctx = a.seq_lens[s] - qn;
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, l16 = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -152,29 +165,27 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
   float* Sg = a.state + ((int64_t)slot * a.H + h) * (int64_t)N * a.P + (int64_t)(8 * g4) * a.P + min(col, a.P - 1);
   const int64_t lane_tile = (int64_t)gridDim.z * 4 * MT * 64;   // float4s of a state in lane order
   const int64_t mine = ((int64_t)blockIdx.z * 4 + w) * MT * 64 + lane;
-  const int64_t cs0 = q0 / a.seg + s;
-  float4* s_in = reinterpret_cast<float4*>(a.s_in) + ((int64_t)s * a.H + h) * lane_tile + mine;
+  const int64_t cs0 = 2 * (q0 / a.seg);
   float4* sums = reinterpret_cast<float4*>(a.sums) + (cs0 * a.H + h) * lane_tile + mine;
   const int64_t seg_step = (int64_t)a.H * lane_tile;
+  float4* s_in = sums + (qn - 1) / a.seg * seg_step;
 
   f32x4_t S[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) S[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto row_at = [&](int m, int r) { return (int64_t)(32 * (m >> 1) + 4 * (m & 1) + r) * a.P; };
-  if (SUMS || pass != 2) {
-    if (on && ctx > 0)
+  if (SUMS || pass != 2 || whole) {
+    if (on && ctx > 0 && z == 0)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[m][r] = Sg[row_at(m, r)];
-    if (SUMS) {   // segments are summed up from zero; the incoming state is set aside
+    if (SUMS && z == 0)   // segments are summed up from zero; the incoming state is set aside
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        if (z == 0) s_in[64 * m] = make_float4(S[m][0], S[m][1], S[m][2], S[m][3]);
+        s_in[64 * m] = make_float4(S[m][0], S[m][1], S[m][2], S[m][3]);
         S[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
-      if (last_seg) return;
-    }
   } else {   // the state in front of this segment: what came in, and the sums of the segments before
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -519,10 +530,11 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
 }
 
 // ================================================================== host launchers
-// floats: per segment and head its decay and sum, per sequence and head the incoming state (columns in blocks of 64)
-int64_t ssm_chunk_scratch_floats(int T_, int ns, int H, int N, int P, int seg) {
-  const int64_t tile = (int64_t)N * ((P + 63) / 64 * 64), cslots = T_ / seg + ns + 1;
-  return (cslots * H + 3) / 4 * 4 + (cslots + ns) * H * tile;
+// floats: per segment and head its decay and sum (columns in blocks of 64)
+static int64_t ssm_chunk_slots(int T_, int seg) { return 2 * (int64_t)(T_ / seg) + 2; }
+int64_t ssm_chunk_scratch_floats(int T_, int H, int N, int P, int seg) {
+  const int64_t tile = (int64_t)N * ((P + 63) / 64 * 64), cslots = ssm_chunk_slots(T_, seg);
+  return (cslots * H + 3) / 4 * 4 + cslots * H * tile;
 }
 
 int ssm_chunk(const void* xbc, int64_t ld_x, const void* dt_raw, int64_t ld_dt, const float* dt_bias, const float* A_log,
@@ -536,15 +548,13 @@ int ssm_chunk(const void* xbc, int64_t ld_x, const void* dt_raw, int64_t ld_dt, 
   SsmChunkArgs a = {};
   a.rows = (const bf16*)xbc, a.ld = ld_x, a.dt = (const bf16*)dt_raw, a.ld_dt = ld_dt, a.dt_bias = dt_bias, a.A_log = A_log;
   a.skip = Dskip, a.state = state, a.qsl = qsl, a.seq_lens = seq_lens, a.slots = slots, a.o = y, a.H = H, a.G = G, a.P = P;
-  a.seg = seg, a.nc = (max_q + seg - 1) / seg;
-  if (a.nc > 1 && !scratch) return -1;
-  if ((int64_t)ns * a.nc > 65535) return -1;
-  if (scratch) {
-    const int64_t cslots = T_ / seg + ns + 1, tile = (int64_t)N * ((P + 63) / 64 * 64);
-    a.decay = scratch, a.sums = scratch + (cslots * H + 3) / 4 * 4, a.s_in = a.sums + cslots * H * tile;
-  }
-  const dim3 grid(H, ns * a.nc, (P + 63) / 64);
-  for (int pass = a.nc > 1 ? 1 : 0; pass < (a.nc > 1 ? 3 : 1); ++pass) {
+  const bool two = max_q > seg;
+  const int64_t n_slots = two ? ssm_chunk_slots(T_, seg) : 0;
+  if ((two && !scratch) || ns + n_slots > 65535) return -1;
+  a.ns = ns, a.seg = seg, a.slots_seg = (int)n_slots;
+  if (scratch) a.decay = scratch, a.sums = scratch + (ssm_chunk_slots(T_, seg) * H + 3) / 4 * 4;
+  for (int pass = two ? 1 : 0; pass < (two ? 3 : 1); ++pass) {
+    const dim3 grid(H, n_slots + (pass == 1 ? 0 : ns), (P + 63) / 64);
     a.pass = pass;
     if (N == 128 && pass == 1) ssm_chunk_kernel<128, true><<<grid, 256, 0, st>>>(a);
     else if (N == 128) ssm_chunk_kernel<128, false><<<grid, 256, 0, st>>>(a);

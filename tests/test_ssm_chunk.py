@@ -120,3 +120,48 @@ def test_large_states_that_fade_before_large_rows_read_them(level, large):
     seen = ref.abs() > 1e-30   # (a state's entry is a product of up to 150 roundings of decays, 2^-23 each with the step's own)
     assert int(seen.sum()) > 40 and float(((col - ref).abs() / ref.abs())[seen].max()) < 150 * 2.0 ** -22
     assert float((after[1].cpu().to(F64) - states[0]).abs().max()) <= 150 * 2.0 ** -22 * float(states[0].abs().max()) + 1e-37
+
+
+@pytest.mark.parametrize("portions", [[(9, 1)] * 5 + [(4, 700)] + [(0, 1), (3, 64), (5, 300), (0, 65)], [(0, 256)] + [(2, 1)] * 70,
+                                      [(1, 100), (0, 257), (6, 1), (2, 513), (0, 128), (7, 129)], [(3, 1)] * 67 + [(0, 400), (5, 2)]], ids=len)
+@pytest.mark.parametrize("H,G,N,P", [(8, 2, 128, 64), (2, 1, 64, 80)])
+def test_sequences_of_one_and_of_several_segments(portions, H, G, N, P, monkeypatch):
+    """Their order, single tokens of more than 64 sequences in front, lengths around whole segments; states with and without a past."""
+    calls = record_native(monkeypatch, sq)
+    args = inputs(portions, H, G, N, P, -0.5, N + len(portions))
+    got, state = run(args, portions, H, G, N, P)
+    assert "ssm_chunk_scratch_floats" in calls
+    want, states = reference(args, portions, H, G, N, P)
+    close(got, want)
+    for i, S in enumerate(states):
+        close(state[i + 1], S)
+    assert torch.equal(state[0].cpu(), args[-1][0])
+
+
+def test_scratch_does_not_grow_with_single_tokens():
+    H, N, P = 8, 128, 64
+    for singles in (0, 200):
+        portions = [(3, 1)] * singles + [(0, 256)]
+        seg, scratch = sq._ssm_chunk_segments(layout(portions), 256 + singles, H, N, P, 64, "cuda")
+        assert seg < 256 and scratch.numel() <= (2 * ((256 + singles) // seg) + 2) * H * (N * P + 1) + 4
+
+
+@pytest.mark.parametrize("where", ["x", "B", "C", "dt"])
+@pytest.mark.parametrize("value", [2.0 ** 29, math.inf, math.nan])
+def test_values_out_of_range_in_a_segment_between_others(where, value):
+    """One bad input at token 300 of 700: what lies before it stays what it is, what follows is what the token loop makes of it."""
+    portions, H, G, N, P, bad = [(3, 1), (4, 700)], 2, 1, 128, 64, 301
+    args = inputs(portions, H, G, N, P, -4.0, 7)
+    if where == "dt":
+        args[1][bad, 1] = value
+    else:
+        args[0][bad, {"x": 21, "B": H * P + 40, "C": H * P + N + 40}[where]] = value
+    got, state = run(args, portions, H, G, N, P)
+    want, states = reference(args, portions, H, G, N, P)
+    close(got[:bad], want[:bad])
+    finite = torch.isfinite(want[bad:].float())
+    assert torch.equal(torch.isfinite(got[bad:].cpu()), finite)
+    # (a column's terms are of its largest output's size; 400 tokens' roundings of 2^-24, the step's among them twice)
+    err = (torch.where(finite, got[bad:].cpu().to(F64) - want[bad:], 0.0)).abs()
+    assert bool((err <= 400 * 2.0 ** -23 * torch.where(finite, want[bad:], 0.0).abs().amax(0) + 1e-5).all())
+    assert torch.equal(torch.isfinite(state[2].cpu()), torch.isfinite(states[1].float()))

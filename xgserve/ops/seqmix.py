@@ -1633,7 +1633,7 @@ def _ssm_chunk_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int
     if wgs > 256 or chunks < (4 if wgs <= 128 else 8) or not SCAN_TWO_PASS:
         return 64 * chunks, None
     seg = 64 * -(-chunks // n)
-    return seg, torch.empty(mixers().ssm_chunk_scratch_floats(T, sm.num_seqs, H, dk, dv, seg), dtype=torch.float32, device=device)
+    return seg, torch.empty(mixers().ssm_chunk_scratch_floats(T, H, dk, dv, seg), dtype=torch.float32, device=device)
 
 
 def _chunk_scan(q, f, k, raw, off_q, off_f, f_bias, lower, v, state, o, sm, H, dk, dv):
