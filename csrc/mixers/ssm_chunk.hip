@@ -15,6 +15,8 @@
 // A chunk with an input out of range (2^28 and above, infinities, NaN) or a sub-chunk below 2^-90 runs token by token, and so does a
 // wave whose state is too large for C S, which meets the decays only after its sum: above 2^92 it could leave fp32 (128 terms, C below
 // 2^28), above 2^40 what it leaves behind decays that underflow within the chunk could count.
+// Chunks of up to four tokens (single tokens beside a prompt, remainders) run token by token for speed: 60 x 1 + 16 tokens of 64 heads 90 ->
+// 63 us, 60 x 1 + 512 102 -> 76, 40 sequences of 2 / 3 / 4 tokens beside 100 70.5 -> 57 / 61 / 64, of 6 70 either way.
 //
 // Error against fp64 (2-norm, outputs / carried state; chunks of 16 tokens in fp32 in brackets, then the token loop), 400 tokens of 8
 // heads of 128 x 64, A_log about 0 8.4e-8 / 6.3e-8 (8.8e-8 / 5.8e-8; 8.7e-8 / 6.2e-8), -0.5 8.4e-8 / 6.6e-8 (9.2e-8 / 6.9e-8; 8.8e-8 /
@@ -29,7 +31,7 @@
 // workgroup of a slot finds its sequence. The incoming state, which the last segment's workgroup replaces, is set aside in the place
 // of that segment's sum, which nobody reads. Sequences of one segment (single tokens beside a prompt) have no part in the first
 // launch and their states are read in place. (With a workgroup per sequence and possible segment, and every sequence's state set aside,
-// 200 single tokens beside 256 of 64 heads took 448 us and 0.9 GB of scratch, now 290 and 34 MB.)
+// 200 single tokens beside 256 of 64 heads took 448 us and 0.9 GB of scratch, now 208 and 34 MB.)
 //
 // Measured, heads of 128 x 64: 2521 ragged tokens of 64 heads 199 -> 75 us, 4 x 1024 of 128 276 -> 122, 4001 of 64 96. A chunk of one
 // workgroup is 5 us by itself, 3.9 where two share a unit: 1.9 of vector work (splitting, scales, range checks: 1100 instructions a
@@ -43,6 +45,7 @@ using xgk::ld16;
 using xgk::mfma16x16x32;
 
 constexpr int kSsTok = 64, kSsSub = 16, kSsRing = 8;   // tokens per chunk and sub-chunk; chunks whose step sizes are held
+constexpr int kSsFew = 4;                                    // tokens of a chunk that run one by one
 constexpr float kSsMinProd = 8.077935669463161e-28f;   // 2^-90
 constexpr float kSsMinChunk = 7.888609052210118e-31f, kSsMaxState = 4.951760157141521e27f, kSsMaxFaded = 1099511627776.f;   // 2^-100, 2^92, 2^40
 
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
     if (ci % 4 == 1) dt_load(ci + 3);
     if (ci % 4 == 2) steps(ci + 2);
     __syncthreads();
-    const bool slow = __builtin_amdgcn_readfirstlane(flags[ci & 1][0] | flags[ci & 1][1] | flags[ci & 1][2] | flags[ci & 1][3] | bad_step[rg]) != 0;
+    const bool slow = n <= kSsFew || __builtin_amdgcn_readfirstlane(flags[ci & 1][0] | flags[ci & 1][1] | flags[ci & 1][2] | flags[ci & 1][3] | bad_step[rg]) != 0;
     // (a NaN goes token by token too; a chunk's whole decay bounds all of its own)
     float top = 0.f;
 #pragma unroll

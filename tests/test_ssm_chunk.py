@@ -165,3 +165,17 @@ def test_values_out_of_range_in_a_segment_between_others(where, value):
     err = (torch.where(finite, got[bad:].cpu().to(F64) - want[bad:], 0.0)).abs()
     assert bool((err <= 400 * 2.0 ** -23 * torch.where(finite, want[bad:], 0.0).abs().amax(0) + 1e-5).all())
     assert torch.equal(torch.isfinite(state[2].cpu()), torch.isfinite(states[1].float()))
+
+
+@pytest.mark.parametrize("two_pass", [True, False])
+@pytest.mark.parametrize("H,G,N,P", [(8, 2, 128, 64), (2, 1, 64, 80)])
+def test_chunks_of_few_tokens(H, G, N, P, two_pass, monkeypatch):
+    """Sequences and remainders of one to six tokens, of which up to four run one by one."""
+    monkeypatch.setattr(sq, "SCAN_TWO_PASS", two_pass)
+    portions = [(9 * (n % 2), n) for n in range(1, 7)] + [(0, 65), (3, 66), (0, 68), (2, 69), (4, 259), (0, 4), (0, 324)]
+    args = inputs(portions, H, G, N, P, -0.5, P)
+    got, state = run(args, portions, H, G, N, P)
+    want, states = reference(args, portions, H, G, N, P)
+    close(got, want)
+    for i, S in enumerate(states):
+        close(state[i + 1], S)
