@@ -179,3 +179,9 @@ def test_chunks_of_few_tokens(H, G, N, P, two_pass, monkeypatch):
     close(got, want)
     for i, S in enumerate(states):
         close(state[i + 1], S)
+
+
+def test_few_heads_run_in_more_segments():
+    for H, n in ((4, 16), (16, 16), (32, 16), (64, 8), (128, 4)):
+        seg, _ = sq._ssm_chunk_segments(layout([(0, 4001)]), 4001, H, 128, 64, 64, "cuda")
+        assert -(-4001 // seg) == n, H
