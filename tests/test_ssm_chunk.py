@@ -181,6 +181,25 @@ def test_chunks_of_few_tokens(H, G, N, P, two_pass, monkeypatch):
         close(state[i + 1], S)
 
 
+@pytest.mark.parametrize("portions,chunk", [([(0, 16)] * 12, 16), ([(0, 16)], 16), ([(5, 8)] * 20 + [(0, 16)] * 20, 16), ([(0, 17)] * 12, 64),
+                                            ([(5, 1)] * 20 + [(0, 16)] * 20, 64), ([(5, 1)] * 60 + [(0, 16)], 64), ([(0, 16)] * 6 + [(0, 33)], 64)],
+                         ids=lambda v: str(v)[:20])
+def test_portions_that_fill_a_chunk_of_16_alone_keep_it(portions, chunk, monkeypatch):
+    H, G, N, P = 2, 1, 128, 64
+    real, split = sq.mixers(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            return (lambda *a: (split.append(a[-2]), real.chunk_scan_ssm(*a))) if name == "chunk_scan_ssm" else getattr(real, name)
+    monkeypatch.setattr(sq, "mixers", Recorder)
+    args = inputs(portions, H, G, N, P, -0.5, len(portions))
+    got, state = run(args, portions, H, G, N, P)
+    assert split == [chunk == 64]
+    want, states = reference(args, portions, H, G, N, P)
+    close(got, want)
+    close(state[1:], torch.stack(states))
+
+
 def test_few_heads_run_in_more_segments():
     for H, n in ((4, 16), (16, 16), (32, 16), (64, 8), (128, 4)):
         seg, _ = sq._ssm_chunk_segments(layout([(0, 4001)]), 4001, H, 128, 64, 64, "cuda")
