@@ -264,7 +264,10 @@ __global__ void __launch_bounds__(256 * GH) prefill_attn_kernel(
 // Bound by the two pipes' work of a tile, 1020 clocks a wave of matrix products and 1000 of vector instructions, and the power limit.
 // us before / now (all waves in step; 32 query heads, 8 kv heads): 4 x 2048 tokens 195 / 185, 8192 572 / 525, 2048 52 / 50, 512
 // (two key phases, in step) 15.3 / 14.9, 4 x 512 behind 1500 83 / 80. In pairs of waves or every second one behind instead, which
-// share no SIMD: 217 and 640 for the first two.
+// share no SIMD: 217 and 640 for the first two. Up to six tiles of keys all waves stay in step: with few rounds, two barriers a tile
+// and a start and an end of their own cost more than they give (staggered / in step: 50 x 77 tokens 44.6 / 37.6, 32 x 128 34.5 / 31.4, 20 x
+// 200 43.3 / 37.9, 16 x 384 59.3 / 57.2; 28 heads on 4: 52.6 / 39.2, 44.8 / 36.0, 49.2 / 46.0, 72.8 / 64.6). A wave without a row of its own
+// (prompts that end early in their last block of rows) leaves its SIMD to the other: 32 x 64 tokens behind 2000 143 -> 125 us.
 // NW waves = GH query heads (one GQA group slice) x NW/GH/KS 32-row blocks x KS.
 // ---------------------------------------------------------------------------
 template <int NW, int GH, int KS, int NSLOT>
@@ -279,6 +282,7 @@ struct Pf2Cfg {
   static constexpr int TILE = BN * D * 2;       // bytes of one K (or V) 64-key tile
   static constexpr int SLOT = 2 * KS * TILE;    // [K phase 0 .. KS-1][V phase 0 .. KS-1]
   static constexpr bool PP = NW == 8 && KS == 1;  // two halves of the waves, one barrier apart
+  static constexpr int IN_STEP = 6;               // ... from more tiles of keys on
   static_assert(!PP || NSLOT == 4, "tiles j - 1 .. j + 2 in the ring");
   static_assert(NW % (GH * KS) == 0 && WROWS % 4 == 0 && WROWS <= 16 && NSLOT >= 2 && NSLOT <= 4, "wave layout");
   static_assert(NSLOT * SLOT <= 160 * 1024, "LDS");
@@ -507,7 +511,38 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
   };
 
   wait_vmcnt<0>();  // Q fragments landed; from here on only the DMAs are counted
-  if constexpr (C::PP) {
+  const bool idle = i0 + rb * 32 >= qlen;  // none of the wave's rows is one of the prompt's: it loads and meets the others
+  if (!C::PP || nslots <= C::IN_STEP) {
+#pragma unroll
+    for (int p = 0; p < NSLOT - 1; ++p)
+      if (p < nslots) issue(p);
+    for (int j = 0; j < nslots; ++j) {
+      // own DMAs of super-tile j done (later ones may stay in flight), then everyone's
+      if (NSLOT == 4 && j + 2 < nslots) wait_vmcnt<4 * C::NDMA>();
+      else if (NSLOT == 4 && j + 1 < nslots) wait_vmcnt<2 * C::NDMA>();
+      else wait_vmcnt<0>();
+      raw_barrier();
+      if (j + NSLOT - 1 < nslots) issue(j + NSLOT - 1);
+      const int tile = j * KS + kp;
+      if (idle || tile >= ntiles || tile * C::BN > wave_hi) continue;  // wave-uniform: nothing of this tile is visible
+      const uint32_t at = (j % NSLOT) * C::SLOT + kp * C::TILE;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        uint4 kf[D / 16];
+        read_k(at, kb, kf);
+        mul_k(kb, kf);
+        sched_fence();  // bound the hoisted fragment reads (registers)
+      }
+      softmax(tile);
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        bf16x8_t vf[D / 32];
+        read_v(at, step, vf);
+        mul_v(step, vf);
+        sched_fence();
+      }
+    }
+  } else if constexpr (C::PP) {
     // Waves w and w + 4 share a SIMD. In step with each other, their products and their softmax met on one pipe while the other
     // idled; so the second four run one barrier behind: one half's products are the other half's softmax. Between barriers 2 j and
     // 2 j + 1 the first four add tile j - 1's P^T V^T and form tile j's scores, then, up to 2 j + 2, that tile's P^T. Tile j has landed
@@ -516,7 +551,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
       if (t + 1 < nslots) wait_vmcnt<2 * C::NDMA>();
       else wait_vmcnt<0>();
     };
-    const int n_vis = min(ntiles, wave_hi / C::BN + 1);  // tiles with a key that some row of the wave sees
+    const int n_vis = idle ? 1 : min(ntiles, wave_hi / C::BN + 1);  // tiles with a key that some row of the wave sees
     bf16x8_t vf[2][D / 32];  // the next products' first fragments
     auto scores = [&](uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
@@ -549,9 +584,9 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
     raw_barrier();
     if (late) raw_barrier();
     ask(0);
-    scores(0);
+    if (!idle) scores(0);
     pass(0, late);
-    weights(0);
+    if (!idle) weights(0);
     pass(0, !late);
     for (int j = 1; j < n_vis; ++j) {
       ask(j);
@@ -582,7 +617,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
     }
     ask(n_vis);
 #pragma unroll
-    for (int step = 0; step < 4; ++step) {
+    for (int step = 0; step < 4 && !idle; ++step) {
       if (step >= 2) read_v(((n_vis - 1) % NSLOT) * C::SLOT, step, vf[step & 1]);
       mul_v(step, vf[step & 1]);
     }
@@ -592,35 +627,6 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
       pass(j, !late);
     }
     if (!late) raw_barrier();
-  } else {
-#pragma unroll
-    for (int p = 0; p < NSLOT - 1; ++p)
-      if (p < nslots) issue(p);
-    for (int j = 0; j < nslots; ++j) {
-      // own DMAs of super-tile j done (later ones may stay in flight), then everyone's
-      if (NSLOT == 3 && j + 1 < nslots) wait_vmcnt<2 * C::NDMA>();
-      else wait_vmcnt<0>();
-      raw_barrier();
-      if (j + NSLOT - 1 < nslots) issue(j + NSLOT - 1);
-      const int tile = j * KS + kp;
-      if (tile >= ntiles || tile * C::BN > wave_hi) continue;  // wave-uniform: nothing of this tile is visible
-      const uint32_t at = (j % NSLOT) * C::SLOT + kp * C::TILE;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        uint4 kf[D / 16];
-        read_k(at, kb, kf);
-        mul_k(kb, kf);
-        sched_fence();  // bound the hoisted fragment reads (registers)
-      }
-      softmax(tile);
-#pragma unroll
-      for (int step = 0; step < 4; ++step) {
-        bf16x8_t vf[D / 32];
-        read_v(at, step, vf);
-        mul_v(step, vf);
-        sched_fence();
-      }
-    }
   }
 
   if constexpr (KS > 1) {

@@ -210,7 +210,7 @@ def test_prefill_attention_spike_forces_rescale():
 
 @pytest.mark.parametrize("gh", [-82, -81, -88, -382, -1282, -42])
 @pytest.mark.parametrize("growth", [0.2, 3.0])   # of a row's largest score from one tile of 64 keys to the next, in powers of two
-@pytest.mark.parametrize("L", [1, 63, 64, 65, 128, 129, 193, 449])
+@pytest.mark.parametrize("L", [1, 63, 64, 65, 128, 129, 193, 314, 315, 449])   # (314: the last of six tiles of keys full)
 def test_prefill_attention_growing_scores(gh, growth, L):
     """Maxima that grow slowly and quickly from tile to tile, at tile edges (every weight and sum is rescaled, or nearly none).
     Against fp64: probabilities and outputs rounded to bf16, 2^-9 each, of the largest |V|."""
