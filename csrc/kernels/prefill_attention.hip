@@ -621,6 +621,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
       if (step >= 2) read_v(((n_vis - 1) % NSLOT) * C::SLOT, step, vf[step & 1]);
       mul_v(step, vf[step & 1]);
     }
+    sched_fence();  // (the last fragments are here, in front of the barrier that frees their slot)
     for (int j = n_vis; j < nslots; ++j) {  // nothing of these tiles is visible
       if (j > n_vis) ask(j);
       pass(j, late);
