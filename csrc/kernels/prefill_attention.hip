@@ -284,7 +284,7 @@ struct Pf2Cfg {
   static constexpr bool PP = NW == 8 && KS == 1;  // two halves of the waves, one barrier apart
   static constexpr int IN_STEP = 6;               // ... from more tiles of keys on
   static_assert(!PP || NSLOT == 4, "tiles j - 1 .. j + 2 in the ring");
-  static_assert(NW % (GH * KS) == 0 && WROWS % 4 == 0 && WROWS <= 16 && NSLOT >= 2 && NSLOT <= 4, "wave layout");
+  static_assert(NW % (GH * KS) == 0 && WROWS % 4 == 0 && WROWS <= 16 && (NSLOT == 2 || NSLOT == 4), "wave layout");
   static_assert(NSLOT * SLOT <= 160 * 1024, "LDS");
 };
 
@@ -326,8 +326,9 @@ __device__ __forceinline__ float xor32_sum(float x) {
 }
 
 // o *= a unless `rows` is 0, in o's registers and one basic block: around a branch hipcc keeps the accumulators twice, and copies
-// them in every round that passes it. Not within 16 matrix instructions of the one that wrote o (hipcc's hazard pass does not look
-// into the statement).
+// them in every round that passes it. hipcc's hazard pass does not look into the statement, so no product into o may still be under way:
+// `rows` comes from products that a sched_fence keeps behind the last of those, and matrix instructions end in their order. (Waiting
+// inside, 19 states where it rescales: 5 to 7 % slower; a read of o that hipcc sees in front of it: 1 %.)
 __device__ __forceinline__ void scale_if(uint64_t rows, f32x16_t& o, float a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   float x0 = o[0], x1 = o[1], x2 = o[2], x3 = o[3], x4 = o[4], x5 = o[5], x6 = o[6], x7 = o[7], x8 = o[8], x9 = o[9], x10 = o[10],
@@ -539,7 +540,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
         bf16x8_t vf[D / 32];
         read_v(at, step, vf);
         mul_v(step, vf);
-        sched_fence();
+        sched_fence();  // (and the next tile's scores behind the products into o: scale_if)
       }
     }
   } else if constexpr (C::PP) {
@@ -605,7 +606,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && NSLOT <= 2 ? 2 : 1)) pref
         read_k(at, 0, kf);
         sched_fence();
         mul_v(3, vg);
-        sched_fence();
+        sched_fence();  // (the scores behind the products into o: scale_if)
         mul_k(0, kf);
         read_k(at, 1, kf);
         mul_k(1, kf);
@@ -694,7 +695,8 @@ int prefill_attention(const uint16_t* q, int64_t q_stride, const uint16_t* kc, c
   if (bs % 16 != 0 || Hq % Hkv != 0) return -1;
   const int G = Hq / Hkv;
   // D = 128: prefill_attn2_kernel. gh == 0 picks the configuration; gh < 0 forces
-  // -gh = 10 * NW + GH (A/B and tests); gh > 0 selects the 16-row kernel above.
+  // -gh = 10 * NW + GH (A/B and tests); gh > 0 selects the 16-row kernel above. Ring slots are two, and four for 8 waves of one key
+  // phase, whose forced codes say 0 or, as when their ring had that many, 3.
   if (D == 128 && gh <= 0) {
     int nw = 0, ghh = 0, ns = 0, ks = 1;
     if (gh < 0) {  // -gh = 1000 * (KS - 1) + 100 * NSLOT + 10 * NW + GH (NSLOT 0: default)
@@ -712,8 +714,10 @@ int prefill_attention(const uint16_t* q, int64_t q_stride, const uint16_t* kc, c
       nw = 8;
       ks = wg8 >= 512 ? 1 : 2;
     }
-    if (ns == 0 || (ns == 3 && nw == 8 && ks == 1)) ns = nw == 8 && ks == 1 ? 4 : 2;  // (three slots of 8 waves: four, what they run on)
-    if (G % ghh != 0 || nw % (ghh * ks) != 0) return -1;
+    const bool apart = nw == 8 && ks == 1;
+    if (ns != 0 && ns != (apart ? 3 : 2)) return -1;
+    ns = apart ? 4 : 2;
+    if ((nw != 4 && nw != 8) || ghh < 1 || G % ghh != 0 || nw % (ghh * ks) != 0) return -1;
     const int bm = 32 * (nw / ghh / ks);
     const int tps = (max_q_len + bm - 1) / bm;
     const int n_hg = Hq / ghh;

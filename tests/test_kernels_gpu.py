@@ -208,7 +208,21 @@ def test_prefill_attention_spike_forces_rescale():
     torch.testing.assert_close(out.cpu().float(), ref.float(), atol=2e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("gh", [-82, -81, -88, -382, -1282, -42])
+def test_prefill_attention_forced_codes():
+    """Each form has one ring: a code names it as 0 or by the slots it had (8 waves of one key phase: 3), any other count is refused."""
+    Hq, Hkv, D = 8, 1, 128
+    kc, vc, bt = _paged([500], Hkv, D, 16)
+    q = rnd(500, Hq, D)
+    qsl, sl = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([0, 500], [500]))
+    run = lambda gh: ops.prefill_attention(q, kc, vc, bt, qsl, sl, 500, 0.088, gh=gh)  # noqa: E731
+    for code, same in ((-382, -82), (-388, -88), (-242, -42), (-1282, -1082)):
+        assert torch.equal(run(code), run(same))
+    for code in (-482, -282, -342, -442, -1382, -1482, -83, -80, -2, -22):
+        with pytest.raises(ValueError):
+            run(code)
+
+
+@pytest.mark.parametrize("gh", [-82, -81, -88, -1282, -42])
 @pytest.mark.parametrize("growth", [0.2, 3.0])   # of a row's largest score from one tile of 64 keys to the next, in powers of two
 @pytest.mark.parametrize("L", [1, 63, 64, 65, 128, 129, 193, 314, 315, 449])   # (314: the last of six tiles of keys full)
 def test_prefill_attention_growing_scores(gh, growth, L):

@@ -154,7 +154,8 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     gh (tests / A/B sweeps; None = the kernel's own choice): > 0 runs the 16-row
     kernel with gh query heads per workgroup; < 0 forces a D = 128 prefill_attn2_kernel
     configuration -gh = 1000 (KS - 1) + 100 NSLOT + 10 NW + GH (key phases, ring
-    slots, waves, heads per workgroup; NSLOT 0 = default), e.g. -82 or -1284."""
+    slots, waves, heads per workgroup; NSLOT 0 = default), e.g. -82 or -1284. (Each has one ring
+    now: NSLOT 3 of 8 waves and one key phase, once a form of its own, is the default's.)"""
     if not use_native(q):
         r = prefill_attention_ref(q, k_cache, v_cache, block_tables, query_start_loc, seq_lens, scale)
         if out is not None:
