@@ -16,7 +16,7 @@
 //
 // That meeting costs 1.5 us at one row and 3.5 to 5 at 64: store, ticket, reads back, one behind the other. rows_whole_kernel
 // takes narrower tiles over the whole K instead. A CU has about 105 requests of 128 bytes under way, each for some 1000
-// clocks where it goes to memory (w) and 400 where it hits L2 (x, which every workgroup reads), so a workgroup costs
+// clocks where it goes to memory (w) and 400 where it hits L2 (x, which every workgroup reads), so a workgroup costs about
 // (0.4 rows + columns) K whatever the ring holds, and the caller takes the form that costs less (ops.seqmix._rows_cols). Its
 // waves divide K, not the columns: each byte is read from LDS once, where four waves over the columns read x four times, which at
 // 64 rows was 670 clocks for every 64 of K. us, cold weights, T = 1 / 17 / 40 / 64, parts with tickets (or whole tiles of 64) before:

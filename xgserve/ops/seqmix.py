@@ -124,14 +124,21 @@ def _rows_plan(N: int, K: int, gated: bool):
 
 
 def _rows_cols(T: int, N: int, K: int, gated: bool, wide: bool, S: int) -> int:
-    """Weight rows of a workgroup: 128 (`wide`) or 64 of one of S parts of K, or fewer of the whole K. Costs of a workgroup as
-    rows_linear.hip has them, 6.5e-5 us each: (0.4 rows of x + columns) K, and for parts that meet 15000 + 25000 a tile of 16
-    rows (measured 1.5 us at one row, 3.5 to 5 at 64). Tiles that leave one round of workgroups only: a second one doubles the time."""
-    x, tiles = 0.4 * 16 * -(-T // 16), -(-T // 16)
-    parts = (x + (128 if wide else 64)) * K / S + (15000 + 25000 * tiles if S > 1 else 0)
+    """Weight rows of a workgroup: 128 (`wide`) or 64 of one of S parts of K, or fewer of the whole K, whichever costs less, in units
+    of some 6.5e-5 us: (0.36 rows of x + columns) K and 3600 for the sums of whole ones, rows at 0.14 in wider ones, and for parts that meet
+    38000 + (7000 + 650 S) a tile of 16 rows. Fitted to 1 700 products of 512 to 16384 x 128 to 14336 and up to 64 rows: 0.2 % slower than the faster of
+    both in the mean, 5.5 at most than parts. (Rows at 0.4 in both and 15000 + 25000 a tile: 0.7 %, 20 at most, 3072 x 5120, 64 rows, 17.4
+    us against 14.5.) From K = 12288 on the whole of it gains 4 % at most. Gated products, whose parts are of 128 rows, keep those other prices: whole
+    ones are 0.4 % slower at most and up to 40 % faster. Tiles that leave one round of workgroups only: a second one doubles the time."""
+    tiles = -(-T // 16)
+    if gated:
+        whole, parts = 6.4 * tiles, (6.4 * tiles + 128) * K / S + (15000 + 25000 * tiles if S > 1 else 0)
+    else:
+        whole = 0.36 * T + 3600 / K
+        parts = (0.14 * T + (128 if wide else 64)) * K / S + (38000 + (7000 + 650 * S) * tiles if S > 1 else 0)
     for cols in ((32, 64) if gated else (16, 32, 48)):
-        if -(-N // cols) <= _ROWS_WGS:
-            return cols if (x + cols) * K < parts else 128 if wide else 64
+        if -(-N // cols) <= _ROWS_WGS and (gated or S == 1 or K <= 12288):
+            return cols if (whole + cols) * K < parts else 128 if wide else 64
     return 128 if wide else 64
 
 
