@@ -201,6 +201,6 @@ def test_portions_that_fill_a_chunk_of_16_alone_keep_it(portions, chunk, monkeyp
 
 
 def test_few_heads_run_in_more_segments():
-    for H, n in ((4, 16), (16, 16), (32, 16), (64, 8), (128, 4)):
-        seg, _ = sq._ssm_chunk_segments(layout([(0, 4001)]), 4001, H, 128, 64, 64, "cuda")
-        assert -(-4001 // seg) == n, H
+    for T, H, n in ((4001, 4, 32), (4001, 16, 32), (4001, 32, 16), (4001, 64, 8), (4001, 128, 4), (2000, 8, 16), (700, 8, 11)):
+        seg, _ = sq._ssm_chunk_segments(layout([(0, T)]), T, H, 128, 64, 64, "cuda")
+        assert -(-T // seg) == n, (T, H)

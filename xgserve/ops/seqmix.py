@@ -1638,12 +1638,12 @@ def _ssm_chunks_fill(sm: SeqMeta, T: int) -> bool:
 
 def _ssm_chunk_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
     """The same for the state-space chunks of 64 tokens (csrc/mixers/ssm_chunk.hip): four to sixteen segments where at most a workgroup
-    per compute unit would run. us whole / in segments, heads of 128 x 64: 4001 tokens of 64 heads 367 / 103 (8), of 128 370 / 191 (4), of 8
-    363 / 49 (16; 8: 77), 1531 + 700 + 257 + 33 of 64 145 / 79, 512 of 64 50 / 29; 60 x 1 + 1931 of 16 195 / 43 (16; 8: 48); 1500 + 900 of 128
+    per compute unit would run, up to 32 of two chunks each. us whole / in segments, heads of 128 x 64: 4001 tokens of 64 heads 367 / 103 (8), of 128 370 / 191 (4), of 8
+    363 / 42 (32; 16: 48, 8: 75), of 8 whose decays are so strong that tokens run one by one 151 (32; 16: 265; 217 in chunks of 16 tokens), 1531 + 700 + 257 + 33 of 64 145 / 79, 512 of 64 50 / 29; 60 x 1 + 1931 of 16 195 / 43 (16; 8: 48); 1500 + 900 of 128
     130 / 124, but 300 + 200 36 / 46 and 3 x 800 of 128 102 / 118."""
     chunks = -(-sm.max_q // 64)
     wgs = max(1.0, T / sm.max_q) * H * ((dv + cols - 1) // cols)
-    n = min(16, max(4, int(CHUNK_SCAN_FILL_WGS / wgs)), chunks)
+    n = min(32, max(4, int(CHUNK_SCAN_FILL_WGS / wgs)), max(16, (chunks + 1) // 2), chunks)
     if wgs > 256 or chunks < (4 if wgs <= 128 else 8) or not SCAN_TWO_PASS:
         return 64 * chunks, None
     seg = 64 * -(-chunks // n)
