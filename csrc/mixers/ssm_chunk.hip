@@ -35,7 +35,9 @@
 //
 // Measured, heads of 128 x 64: 2521 ragged tokens of 64 heads 199 -> 75 us, 4 x 1024 of 128 276 -> 122, 4001 of 64 96. A chunk of one
 // workgroup is 5 us by itself, 3.9 where two share a unit: 1.9 of vector work (splitting, scales, range checks: 1100 instructions a
-// wave), 0.95 of matrix instructions, 1.2 of LDS reads, the rest waits between its three barriers.
+// wave), 0.95 of matrix instructions, 1.2 of LDS reads, the rest waits between its three barriers. A token by itself is 200 vector
+// instructions and one LDS latency (its eight reads go out at once; one behind the other 64 heads, 4001 such tokens 631 -> 605, 8 heads, 257
+// 75 -> 73). No register of a lane is spilled; some 40 scalars that the loop does not hold are lane reads, 2 % of a chunk's instructions.
 #include "mfma_f32.h"
 
 namespace xgm {
@@ -44,7 +46,7 @@ using xgk::as_frag;
 using xgk::ld16;
 using xgk::mfma16x16x32;
 
-constexpr int kSsTok = 64, kSsSub = 16, kSsRing = 8;   // tokens per chunk and sub-chunk; chunks whose step sizes are held
+constexpr int kSsTok = 64, kSsRing = 8;   // tokens per chunk; chunks whose step sizes are held
 constexpr int kSsFew = 4;                                    // tokens of a chunk that run one by one
 constexpr float kSsMinProd = 8.077935669463161e-28f;   // 2^-90
 constexpr float kSsMinChunk = 7.888609052210118e-31f, kSsMaxState = 4.951760157141521e27f, kSsMaxFaded = 1099511627776.f;   // 2^-100, 2^92, 2^40
@@ -336,12 +338,14 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
     if (ci % 4 == 1) dt_load(ci + 3);
     if (ci % 4 == 2) steps(ci + 2);
     __syncthreads();
-    const bool slow = n <= kSsFew || __builtin_amdgcn_readfirstlane(flags[ci & 1][0] | flags[ci & 1][1] | flags[ci & 1][2] | flags[ci & 1][3] | bad_step[rg]) != 0;
+    const float most = Eh[rg] >= kSsMinChunk ? kSsMaxState : kSsMaxFaded;
+    const int odd = flags[ci & 1][0] | flags[ci & 1][1] | flags[ci & 1][2] | flags[ci & 1][3] | bad_step[rg];
+    const bool slow = (n <= kSsFew) | (__builtin_amdgcn_readfirstlane(odd) != 0);
     // (a NaN goes token by token too; a chunk's whole decay bounds all of its own)
     float top = 0.f;
 #pragma unroll
     for (int m = 0; m < MT; ++m) top = fmaxf(fmaxf(fabsf(S[m][0]), fabsf(S[m][1])), fmaxf(top, fmaxf(fabsf(S[m][2]), fabsf(S[m][3]))));
-    const bool wslow = slow || __any(!(top < (Eh[rg] >= kSsMinChunk ? kSsMaxState : kSsMaxFaded)));
+    const bool wslow = slow | (__any(!(top < most)) != 0);
     if (!SUMS && !slow) {
       // G^T of three of the twelve tiles: rows j = 32 q + 8 (i / 4) + 4 half + i % 4, columns token 16 b + l16
 #pragma unroll
@@ -490,12 +494,19 @@ __global__ __launch_bounds__(256, 2) void ssm_chunk_kernel(const SsmChunkArgs a)
         const int c = 2 * w + (l16 >> 3);
         const float vv = bf2f(*reinterpret_cast<const bf16*>(xs + t * 128 + 16 * (c ^ ss_swz8(t)) + 2 * (l16 & 7))), vd = vv * dts[rg][t];
         float part[4] = {0.f, 0.f, 0.f, 0.f};
+        uint4 bu[KS], cu[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           const int at = t * RB + 16 * ((4 * ks + g4) ^ (GR == 16 ? ss_swz16(t) : ss_swz8(t)));
+          bu[ks] = *reinterpret_cast<const uint4*>(bs + at);
+          if (!SUMS) cu[ks] = *reinterpret_cast<const uint4*>(cs + at);
+        }
+        ss_fence();   // (all of a token's reads under way at once)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
           float bb[8], cc[8];
-          xgk::unpack8(*reinterpret_cast<const uint4*>(bs + at), bb);
-          if (!SUMS) xgk::unpack8(*reinterpret_cast<const uint4*>(cs + at), cc);
+          xgk::unpack8(bu[ks], bb);
+          if (!SUMS) xgk::unpack8(cu[ks], cc);
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             float& v = reinterpret_cast<float(&)[4]>(S[2 * ks + (e >> 2)])[e & 3];
