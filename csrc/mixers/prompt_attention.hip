@@ -25,8 +25,10 @@
 // wave beside 16 matrix ones (156 and 64 of 266 thousand clocks), 125 us. Scores that stay products up to the exponential, masks by
 // edge (compares and selects, no branches), addresses as a uniform base and a lane's constant: 113 us; 16 heads of 64 + 128 with a
 // distance penalty 131 -> 121, 2 x 1800 tokens of 32 heads of 128 + 128 97 -> 93, expanded latents (64 + 32) + 64 of 4 x 2048 tokens
-// 154 -> 127, (128 + 64) + 128 of 2 x 1300 96 -> 84.
-// (Both blocks of 32 keys in turn, so that two chains of matrix instructions run; waves' priorities and two sums for l change nothing.)
+// 154 -> 127, (128 + 64) + 128 of 2 x 1300 96 -> 84. A distance penalty in units of products (no product with the scale in front of it),
+// and heads of 128 with one block of 32 keys behind the other: 4001 tokens of 32 heads of 128 + 128 with a penalty 229 -> 214, of 16 of
+// 64 + 64 105 -> 101; heads of 128 + 64 with bounded scores 116 -> 111, of 128 + 128 without either 187 -> 182.
+// (Heads of 64: both blocks of 32 keys in turn, so that two chains of matrix instructions run; waves' priorities and two sums for l change nothing.)
 #include "attention_common.h"
 #include "glds.h"
 
@@ -217,12 +219,15 @@ __global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_atte
   const float pen1 = uniform(a.r1 ? a.r1[head] : 0.f), pen2 = uniform(a.r1 ? a.r2[head] : 0.f);
   const float sbias = uniform((sig && a.hbias) ? a.hbias[head] * kLog2e : 0.f);
   // Scores stay products until they are exponentials: one multiply-add takes them to their distance from the row's reference m (sc1;
-  // 1 where a bound or a penalty has made them scores already). The sign of the scale is the query's, so that the largest
-  // product is the largest score; a scale of 0 is the smallest number instead (0 would make a masked one not a number).
-  const bool scaled = capped || sig || a.r1;
+  // 1 where a bound has made them scores already, or a penalty that in units of products would leave fp32). The sign of the scale is the
+  // query's, so that the largest product is the largest score; a scale of 0 is the smallest number instead (0 would make a masked one not
+  // a number).
+  const float pen_f = pen1 / fabsf(sc_h);   // the penalty in units of products
+  const bool scaled = capped || sig || (a.r1 && !(fabsf(pen_f) < 1e30f && fabsf(sc_h) > 1e-30f));
   const uint32_t flip = !scaled && sc_h < 0.f ? 0x80008000u : 0u;
   sc_h = uniform(scaled ? sc_h : sc_h == 0.f ? 1.1754944e-38f : fabsf(sc_h));
   const float sc1 = scaled ? 1.f : sc_h;
+  const float pen = uniform(scaled ? pen1 : pen_f);
   float m = bounded ? 0.f : a.sink ? a.sink[head] * kLog2e : -INFINITY;
   float l = (a.sink && hf == 0) ? 1.f : 0.f;   // each half of a row's two lanes sums its own keys
   f32x16_t o[DV / 32];
@@ -278,12 +283,22 @@ __global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_atte
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
+    if constexpr (DK == 128) {   // (turns as below: as fast without a bound or penalty, 2 to 5 % slower with)
 #pragma unroll
-    for (int ks = 0; ks < DK / 16; ++ks) {
+      for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + (k_at(ks) + kb * 32 * KROW))), qf[ks], sacc[kb]);
-      if (ks % 2) sched_fence();   // bound the hoisted fragment reads
+        for (int ks = 0; ks < DK / 16; ++ks)
+          sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + (k_at(ks) + kb * 32 * KROW))), qf[ks], sacc[kb]);
+        sched_fence();   // bound the hoisted fragment reads
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < DK / 16; ++ks) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          sacc[kb] = mfma32x32x16(xgk::as_frag(xgk::ld16(lds + (k_at(ks) + kb * 32 * KROW))), qf[ks], sacc[kb]);
+        if (ks % 2) sched_fence();
+      }
     }
     // scores in units of ln 2; register e of block kb is key base + 32 kb + 4 hf + (e & 3) + 8 (e >> 2)
     const bool full = base + kPT - 1 <= pos_lo && (base >= lo_hi || base + kPT <= a.keep);
@@ -306,7 +321,7 @@ __global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_atte
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          sacc[kb][e] -= pen1 * log2_fast(fmaf(pen2, dist - (float)(kb * 32 + (e & 3) + 8 * (e >> 2)), 1.f));
+          sacc[kb][e] -= pen * log2_fast(fmaf(pen2, dist - (float)(kb * 32 + (e & 3) + 8 * (e >> 2)), 1.f));
     }
     if (!full) {   // (wave-uniform: a tile mostly has one of the two edges)
       if (base + kPT - 1 > pos_lo) {
@@ -315,13 +330,15 @@ __global__ __launch_bounds__(512, DK == 64 && DV == 64 ? 4 : 2) void prompt_atte
 #pragma unroll
           for (int e = 0; e < 16; ++e) sacc[kb][e] = kb * 32 + (e & 3) + 8 * (e >> 2) > vis_hi ? -INFINITY : sacc[kb][e];
       }
-      if (base < lo_hi && base + kPT > a.keep) {
+      if (base < lo_hi && base + kPT > a.keep) {   // keys from vis_keep on, up to vis_lo
+        const uint32_t hidden = max(vis_lo - vis_keep, 0);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
             const int c = kb * 32 + (e & 3) + 8 * (e >> 2);
-            sacc[kb][e] = (int)(c < vis_lo) & (int)(c >= vis_keep) ? -INFINITY : sacc[kb][e];
+            const bool out = DK == 128 ? (uint32_t)(c - vis_keep) < hidden : (bool)((int)(c < vis_lo) & (int)(c >= vis_keep));
+            sacc[kb][e] = out ? -INFINITY : sacc[kb][e];
           }
       }
     }

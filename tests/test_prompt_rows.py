@@ -79,3 +79,36 @@ def test_scales_of_any_sign_and_growing_scores(dk, dv, mask, size, sink):
         big = sc.masked_fill(~seen, 0).abs().amax(-1, keepdim=True)
         bound = want.abs() * 2.0 ** -8 + (6 * 2.0 ** -9 * p.pow(2).sum(-1, keepdim=True).sqrt() + big * 2.0 ** -22) * vv.abs().max() + 1e-5
         assert bool((err <= bound).all()), (h, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (64, 128)])
+@pytest.mark.parametrize("sink", [False, True])
+def test_penalties_beside_scales_of_any_size(dk, dv, sink):
+    """A penalty is taken in units of products, except where those would leave fp32: scales of either sign, 0, 1e-20 and 1e-36, penalties
+    that come to nothing, small, so large that a row's own key is all it sees, and negative. Same tolerance."""
+    g = torch.Generator().manual_seed(dk + dv)
+    H, n, bs = 8, 330, 16
+    q, k, v = (torch.randn(n, H * d, generator=g).bfloat16() for d in (dk, dk, dv))
+    temp = torch.tensor([1.0, -1.3, 0.0, 1e-20, 1e-36, 4.0, -1e-25, 1.0])
+    r1 = torch.tensor([0.7, 1.1, 0.4, 0.9, 0.6, 1e6, 1e12, -0.2])
+    r2, sinks = torch.rand(H, generator=g) + 0.1, torch.randn(H, generator=g)
+    r2[5] = 0.0   # (a large penalty of nothing)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    sm = sq.SeqMeta(1, n, i32([0, n]), i32([n]), i32([0]), i32([list(range(-(-n // bs)))]), i32([0] * n), i32(list(range(n))), i32(list(range(n))))
+    cache = [torch.cat([t, torch.zeros(-n % bs, t.shape[1])]).bfloat16().cuda() for t in (k, v)]
+    got = sq.masked_attention(q.cuda(), *cache, H, H, dk, dv, sq.MASK_CAUSAL, 0, dk ** -0.5, temp.cuda(), sinks.cuda() if sink else None, bs, sm,
+                              dist=(r1.cuda(), r2.cuda()))
+    d = (torch.arange(n)[:, None] - torch.arange(n)[None]).double()
+    for h in range(H):
+        sc = q[:, h * dk:(h + 1) * dk].double() @ k[:, h * dk:(h + 1) * dk].double().T * dk ** -0.5 * temp[h].double()
+        pen = r1[h].double() * torch.log1p(r2[h].double() * d.clamp(min=0))
+        sc = (sc - pen).masked_fill(d < 0, float("-inf"))
+        full = torch.cat([sc, sinks[h].double().expand(n, 1)], 1) if sink else sc
+        p = torch.softmax(full, -1)[:, :n]
+        vv = v[:, h * dv:(h + 1) * dv].double()
+        want = p @ vv
+        err = (got[:, h * dv:(h + 1) * dv].double().cpu() - want).abs()
+        # (a score errs by 2^-22 of its own and of the nearest keys' penalty)
+        big = torch.where(p > 1e-12, pen.abs(), 0.0).amax(-1, keepdim=True) + sc.masked_fill(p < 1e-12, 0).abs().amax(-1, keepdim=True)
+        bound = want.abs() * 2.0 ** -8 + (6 * 2.0 ** -9 * p.pow(2).sum(-1, keepdim=True).sqrt() + big * 2.0 ** -22) * vv.abs().max() + 1e-5
+        assert bool((err <= bound).all()), (h, float((err / bound).max()))
