@@ -65,7 +65,7 @@ int ssm_step(const void*, bool, int64_t, const void*, int64_t, const float*, con
 int delta_step(const void*, int64_t, int, int, int, int, int, int, int, const void*, const float*, const float*, const float*,
                float, float*, const int32_t*, const int32_t*, const int32_t*, void*, int, int, int, hipStream_t);
 int tile_plan(const double*, int, const int*, int, const double*, int64_t, int64_t, int64_t, int, int*);
-int grouped_plan(const double*, int, const double*, int, const double*, int64_t, int64_t, int64_t, int64_t, int, int*);
+int grouped_plan(const double*, int, const double*, int, int64_t, int64_t, int64_t, int64_t, int, int*);
 int tile_linear(const void*, int64_t, const void*, const void*, bool, float*, void*, int, int, int, int, int, int, float, float,
                 int, int, int, hipStream_t);
 int tile_grouped(const void*, int64_t, int, const int32_t*, const int32_t*, int, int, const void*, float*, void*, int, int, int, int, float,
@@ -383,10 +383,9 @@ PYBIND11_MODULE(_mixers, m) {
       throw std::invalid_argument("tile_plan: no tile for these sizes");
     return py::make_tuple(best[0], best[1], best[2]);
   });
-  m.def("grouped_plan", [](uintptr_t tiles, int n, uintptr_t quantiles, int n_q, uintptr_t prices, int64_t pairs, int64_t E, int64_t N,
-                           int64_t K, int cus) {
+  m.def("grouped_plan", [](uintptr_t tiles, int n, uintptr_t quantiles, int n_q, int64_t pairs, int64_t E, int64_t N, int64_t K, int cus) {
     int best[2];
-    if (xgm::grouped_plan(P<const double>(tiles), n, P<const double>(quantiles), n_q, P<const double>(prices), pairs, E, N, K, cus, best))
+    if (xgm::grouped_plan(P<const double>(tiles), n, P<const double>(quantiles), n_q, pairs, E, N, K, cus, best))
       throw std::invalid_argument("grouped_plan: no tile for these sizes");
     return py::make_tuple(best[0], best[1]);
   });

@@ -1,9 +1,12 @@
 """Products of many rows (prompt steps) on csrc/mixers/tile_linear.hip: the sizes they run at, and where the library's stay.
 
-`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 4 500 timings on an MI355X (15 weights
-of 768 to 14336 in K and 1088 to 28672 in N, 65 to 8192 rows, cold weights); over these its choice is 1 % slower than the fastest
-of the kernel's forms in the mean and 13 % at most. A product's time steps up with every round of tiles that is begun, so there are
-many sizes: (5, 8), (8, 6), (7, 6), (6, 6), (7, 4) and (5, 4) beside the ten that were there take 2 % off the mean of 144 products of 80 to
+`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 13 900 timings on an MI355X (2 590 products of 52
+weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights); over these its choice is 0.6 % slower than the
+fastest form that was timed in the mean and 19 % at most. A step of 64 of K costs a workgroup its products or, of few rows, its
+reads: weights come from memory, rows from L2, at the rate at which its outstanding loads return (ops.seqmix._rows_cols has the same for a
+few rows). Without that the smallest tiles looked cheaper than they are: us, 224 x 4096 x 4096 27.1 -> 21.9, 768 x 2048 x 8192 50 -> 37, 288 x
+18560 x 4096 75 -> 60; of 483 products, whose plan this changed, the times are 8 % less in the mean, 11 % more at most. A product's time steps up with every round of tiles that is
+begun, so there are many sizes: (5, 8), (8, 6), (7, 6), (6, 6), (7, 4) and (5, 4) beside the ten that were there take 2 % off the mean of 144 products of 80 to
 5000 rows, and, us, cold weights: 2521 x 4096 x 14336 243 -> 213 (256 tiles of 160 x 256, where 192 x 256 left 32 of 256 workgroups out),
 2521 x 2048 x 8192 79 -> 74, 3100 x 6144 x 4096 139 -> 126, 1024 x 18560 x 4096 148 -> 130, 700 x 6144 x 4096 43 -> 38.
 """
@@ -22,14 +25,16 @@ from torch.utils._device import DeviceContext
 from ._native import is_f32, mixers, native_device, on_current_device, stream_ptr
 from .linear import PendingSum, cu_count
 
-# rows and columns of a workgroup's tile / 32 -> us per 64 of K and per tile
-_TILES = {(8, 8): (1.135, 0.02), (7, 8): (1.036, 0.02), (6, 8): (0.910, 0.02), (5, 8): (0.816, 0.02), (4, 8): (0.721, 0.02),
-          (8, 6): (0.937, 0.02), (7, 6): (0.819, 0.61), (6, 6): (0.708, 0.98), (8, 4): (0.705, 0.10), (7, 4): (0.627, 1.11),
-          (6, 4): (0.540, 1.13), (5, 4): (0.480, 1.19), (4, 4): (0.399, 1.62), (3, 4): (0.327, 1.90), (4, 2): (0.254, 1.57),
-          (3, 2): (0.229, 0.46)}
-_LAUNCH, _SUM = 2.19, 3.35                  # us of the launch, and of the one that adds the parts
-_W_BYTES, _PART_BYTES, _OUT_BYTES = 6.25e6, 2.56e6, 2.55e6   # bytes per us: weights, fp32 parts (there and back), the result
-_OVERLAP = 0.31                             # share of the shorter of products and weight stream that stays visible
+# rows and columns of a workgroup's tile / 32 -> us per 64 of K where its products bound it, and per tile
+_TILES = {(8, 8): (1.184, 5.47), (7, 8): (1.130, 3.75), (6, 8): (0.967, 4.90), (5, 8): (0.868, 3.15), (4, 8): (0.883, 1.35),
+          (8, 6): (1.055, 3.27), (7, 6): (0.911, 3.74), (6, 6): (0.790, 3.47), (8, 4): (0.793, 2.94), (7, 4): (0.707, 2.70),
+          (6, 4): (0.648, 2.68), (5, 4): (0.556, 2.47), (4, 4): (0.499, 2.39), (3, 4): (0.410, 3.21), (4, 2): (0.309, 2.69),
+          (3, 2): (0.319, 0.02)}
+# ... and where its reads do: us per 64 of K for 32 rows, for 32 columns (of weights that one row of tiles reads: with n of them n^-1/4 of
+# it), and for the smallest tile besides
+_X_READ, _W_READ, _SMALL = 0.0371, 0.1037, 0.0913
+_SUM, _PART = 4.91, 0.230                    # us of the launch that adds the parts, and for each of them
+_PART_BYTES, _OUT_BYTES = 2.51e6, 2.52e6   # bytes per us: fp32 parts (there and back), the result
 _SPLITS = (1, 2, 3, 4, 6, 8, 12, 16)
 _SPLIT_K, _SPLIT_TILES = 256, 540           # a part's least K; parts of all tiles at most (a bound on the slabs: 2.1 tiles per CU)
 
@@ -45,7 +50,7 @@ def _table(kind: str, *rows):
 
 
 _KEPT: list = []
-_PRICES = _table("d", (_LAUNCH, _SUM, _W_BYTES, _PART_BYTES, _OUT_BYTES, _OVERLAP, _SPLIT_K, _SPLIT_TILES))[0]
+_PRICES = _table("d", (_X_READ, _W_READ, _SMALL, _SUM, _PART, _PART_BYTES, _OUT_BYTES, _SPLIT_K, _SPLIT_TILES))[0]
 _TILE_ROWS = _table("d", *(t + p for t, p in _TILES.items()))[0]
 _SPLIT_ROWS = _table("i", _SPLITS)[0]
 
@@ -57,7 +62,8 @@ def tile_plan(M: int, N: int, K: int, cus: int = 256):
 
 
 # Tiles of the experts' products; offsets of all experts are looked through for a tile's, so there is a bound on their number
-# (their prices are a fit of their own: rows are gathered, and most experts end in a part of a tile)
+# (their prices are a fit of their own: rows are gathered, and most experts end in a part of a tile; with them the weights' reads are a
+# constant, so the time of the tiles alone decides)
 _GROUPED = {(8, 8): (1.098, 0.02), (7, 8): (0.995, 0.63), (6, 8): (0.868, 0.86), (4, 8): (0.694, 1.11), (6, 4): (0.527, 1.55),
             (4, 4): (0.401, 1.88), (3, 4): (0.331, 1.95)}
 GROUPED_EXPERTS_MAX = 64
@@ -74,7 +80,7 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
     of the mean instead, tiles that just hold the mean were taken, and the larger experts' second ones made a round of their own. Cold
     weights, both products, router and shared expert, us: 8 experts of 2 x 2048 x 2048, 300 tokens 131 -> 124; of 2 x 3584 x 4096 256 ->
     241, 400 tokens 290 -> 276 (either product's change alone)."""
-    return mixers().grouped_plan(_GROUPED_ROWS, len(_GROUPED), _QUANTILES, len(_SHARES), _PRICES, pairs, E, N, K, cus)
+    return mixers().grouped_plan(_GROUPED_ROWS, len(_GROUPED), _QUANTILES, len(_SHARES), pairs, E, N, K, cus)
 
 
 def library_better(M: int, N: int, K: int) -> bool:
