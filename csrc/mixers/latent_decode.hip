@@ -11,10 +11,10 @@
 // blocks of 16 rows x 32 columns (1 KB, one DMA instruction) whose 16-byte granules are permuted by row / 4: the fragment
 // reads (S^T = K Q^T) and the transposed ones (O^T += V^T P^T) both spread over all banks.
 //
-// 64 sequences of 1024 keys, 32 heads, R = 256, rd = 32: 17.6 us (37.7 MB of rows) and 8.1 us against 30.6 and, for merge,
+// 64 sequences of 1024 keys, 32 heads, R = 256, rd = 32: 16.0 us (37.7 MB of rows) and 7.8 us against 30.6 and, for merge,
 // expansion product and transpose in three launches, 25.7. The kernel before had one 64-key tile to a workgroup (16 shares),
-// nothing in flight behind it, 33 MB of fp32 shares written and read back, and half of its waves without heads. (R = 512, rd = 64: 30.9
-// where every tile rescaled its 128 accumulators, 28.5 since only those that raise the maximum do. Four slots, or two tiles at a
+// nothing in flight behind it, 33 MB of fp32 shares written and read back, and half of its waves without heads. (R = 512, rd = 64: 29.8
+// where every tile rescaled its 128 accumulators, 27.5 where only those that raise the maximum do. Four slots, or two tiles at a
 // time on eight waves: no faster, one tile takes 7.5 us, most of it one memory latency behind the other.)
 #include "attention_common.h"
 #include "glds.h"

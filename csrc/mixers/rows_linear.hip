@@ -24,11 +24,11 @@
 //   3072 x 768     4.1 /  4.9 /  6.0 /  6.4 -> 3.2 / 3.6 / 4.2 / 4.8     7168 x 4096, gated   13.9 / 17.2 / 18.0 / 21.1 -> 11.0 / 12.8 / 15.6 / 18.2
 //   6176 x 4096   11.5 / 13.3 / 16.7 / 20.5 -> 10.0 / 12.3 / 15.3 / 17.8  10768 x 4096, 64 rows 24.9 -> 22.4; 8192 x 2048, 64 rows 13.3 -> 10.7
 //
-// Measured against the library's product without what follows it, cold weights, us (T = 1 / 17 / 64):
-//   2048 x 2048    5.7 /  7.1 /  8.6 against 11.0 / 11.0 / 11.8      18560 x 4096   28 / 29 / 37 against 67 / 36 / 40
-//   2048 x 8192    9.5 / 11.0 / 13.8 against 12.9 / 13.7 / 22.6      28672 x 4096   39 / 38 / 41 against 64 / 55 / 56
-//   10272 x 2048   9.9 / 10.4 / 13.9 against 16.3 / 14.6 / 15.9      4096 x 14336   21 / 22 / 27 against 26 / 28 / 39
-// (5.8 TB/s of weights at the largest; the smaller ones in parts, as they run where the whole K costs more.)
+// Measured against the library's product without what follows it, each in the form it runs in, cold weights, us (T = 1 / 17 / 64):
+//   2048 x 2048    4.3 /  5.2 /  7.6 against 11.0 / 11.0 / 11.8      18560 x 4096   30 / 30 / 38 against 67 / 36 / 40
+//   2048 x 8192    9.6 / 11.0 / 13.7 against 12.9 / 13.7 / 22.6      28672 x 4096   39 / 38 / 41 against 64 / 55 / 56
+//   10272 x 2048   8.7 /  9.4 / 13.0 against 16.3 / 14.6 / 15.9      4096 x 14336   22 / 23 / 28 against 26 / 28 / 39
+// (5.8 TB/s of weights at the largest; 2048 x 8192, 18560 x 4096 and 4096 x 14336 in parts or tiles of 128, the small ones over the whole K.)
 #include "attention_common.h"
 #include "glds.h"
 #include "glu.h"
