@@ -33,11 +33,12 @@
 // launch and their states are read in place. (With a workgroup per sequence and possible segment, and every sequence's state set aside,
 // 200 single tokens beside 256 of 64 heads took 448 us and 0.9 GB of scratch, now 208 and 34 MB.)
 //
-// Measured, heads of 128 x 64: 2521 ragged tokens of 64 heads 199 -> 78 us (81 traced in a step), 4 x 1024 of 128 276 -> 122, 4001 of 64 96. A chunk of one
-// workgroup is 5 us by itself, 3.9 where two share a unit: 1.9 of vector work (splitting, scales, range checks: 1100 instructions a
-// wave), 0.95 of matrix instructions, 1.2 of LDS reads, the rest waits between its three barriers. A token by itself is 200 vector
-// instructions and one LDS latency (its eight reads go out at once; one behind the other 64 heads, 4001 such tokens 631 -> 605, 8 heads, 257
-// 75 -> 73). No register of a lane is spilled; some 40 scalars that the loop does not hold are lane reads, 2 % of a chunk's instructions.
+// Measured, heads of 128 x 64: 2521 ragged tokens of 64 heads 199 -> 78 us (81 traced in a step), 4 x 1024 of 128 276 -> 122, 4001 of
+// 64 102. A chunk of one workgroup is 5 us by itself, 3.9 where two share a unit: 1.9 of vector work (splitting, scales, range checks:
+// 1100 instructions a wave), 0.95 of matrix instructions, 1.2 of LDS reads, the rest waits between its three barriers. A token by itself
+// is 200 vector instructions and one LDS latency (its eight reads go out at once; one behind the other 64 heads, 4001 such tokens 631 ->
+// 605, 8 heads, 257 75 -> 73). No register of a lane is spilled; some 40 scalars that the loop does not hold are lane reads, 2 % of a
+// chunk's instructions.
 #include "mfma_f32.h"
 
 namespace xgm {

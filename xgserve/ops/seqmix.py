@@ -125,11 +125,12 @@ def _rows_plan(N: int, K: int, gated: bool):
 
 def _rows_cols(T: int, N: int, K: int, gated: bool, wide: bool, S: int) -> int:
     """Weight rows of a workgroup: 128 (`wide`) or 64 of one of S parts of K, or fewer of the whole K, whichever costs less, in units
-    of some 6.5e-5 us: (0.36 rows of x + columns) K and 3600 for the sums of whole ones, rows at 0.14 in wider ones, and for parts that meet
-    38000 + (7000 + 650 S) a tile of 16 rows. Fitted to 1 700 products of 512 to 16384 x 128 to 14336 and up to 64 rows: 0.2 % slower than the faster of
-    both in the mean, 5.5 at most than parts. (Rows at 0.4 in both and 15000 + 25000 a tile: 0.7 %, 20 at most, 3072 x 5120, 64 rows, 17.4
-    us against 14.5.) From K = 12288 on the whole of it gains 4 % at most. Gated products, whose parts are of 128 rows, keep those other prices: whole
-    ones are 0.4 % slower at most and up to 40 % faster. Tiles that leave one round of workgroups only: a second one doubles the time."""
+    of some 6.5e-5 us: (0.36 rows of x + columns) K and 3600 for the sums of whole ones, rows at 0.14 in wider ones, and for parts that
+    meet 38000 + (7000 + 650 S) a tile of 16 rows. Fitted to 1 700 products of 512 to 16384 x 128 to 14336 and up to 64 rows: 0.2 % slower
+    than the faster of both in the mean, 5.5 at most than parts. (Rows at 0.4 in both and 15000 + 25000 a tile: 0.7 %, 20 at most, 3072 x
+    5120, 64 rows, 17.4 us against 14.5.) From K = 12288 on the whole of it gains 4 % at most. Gated products, whose parts are of 128
+    rows, keep those other prices: whole ones are 0.4 % slower at most and up to 40 % faster. Tiles that leave one round of workgroups
+    only: a second one doubles the time."""
     tiles = -(-T // 16)
     if gated:
         whole, parts = 6.4 * tiles, (6.4 * tiles + 128) * K / S + (15000 + 25000 * tiles if S > 1 else 0)
@@ -1638,9 +1639,10 @@ def _ssm_chunks_fill(sm: SeqMeta, T: int) -> bool:
 
 def _ssm_chunk_segments(sm: SeqMeta, T: int, H: int, dk: int, dv: int, cols: int, device):
     """The same for the state-space chunks of 64 tokens (csrc/mixers/ssm_chunk.hip): four to sixteen segments where at most a workgroup
-    per compute unit would run, up to 32 of two chunks each. us whole / in segments, heads of 128 x 64: 4001 tokens of 64 heads 367 / 103 (8), of 128 370 / 191 (4), of 8
-    363 / 42 (32; 16: 48, 8: 75), of 8 whose decays are so strong that tokens run one by one 151 (32; 16: 265; 217 in chunks of 16 tokens), 1531 + 700 + 257 + 33 of 64 145 / 79, 512 of 64 50 / 29; 60 x 1 + 1931 of 16 195 / 43 (16; 8: 48); 1500 + 900 of 128
-    130 / 124, but 300 + 200 36 / 46 and 3 x 800 of 128 102 / 118."""
+    per compute unit would run, up to 32 of two chunks each. us whole / in segments, heads of 128 x 64: 4001 tokens of 64 heads 367 / 103
+    (8), of 128 370 / 191 (4), of 8 363 / 42 (32; 16: 48, 8: 75), of 8 whose decays are so strong that tokens run one by one 151 (32; 16:
+    265; 217 in chunks of 16 tokens), 1531 + 700 + 257 + 33 of 64 145 / 79, 512 of 64 50 / 29; 60 x 1 + 1931 of 16 195 / 43 (16; 8: 48);
+    1500 + 900 of 128 130 / 124, but 300 + 200 36 / 46 and 3 x 800 of 128 102 / 118."""
     chunks = -(-sm.max_q // 64)
     wgs = max(1.0, T / sm.max_q) * H * ((dv + cols - 1) // cols)
     n = min(32, max(4, int(CHUNK_SCAN_FILL_WGS / wgs)), max(16, (chunks + 1) // 2), chunks)

@@ -1,14 +1,15 @@
 """Products of many rows (prompt steps) on csrc/mixers/tile_linear.hip: the sizes they run at, and where the library's stay.
 
-`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 13 900 timings on an MI355X (2 590 products of 52
-weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights); over these its choice is 0.6 % slower than the
-fastest form that was timed in the mean and 19 % at most. A step of 64 of K costs a workgroup its products or, of few rows, its
-reads: weights come from memory, rows from L2, at the rate at which its outstanding loads return (ops.seqmix._rows_cols has the same for a
-few rows). Without that the smallest tiles looked cheaper than they are: us, 224 x 4096 x 4096 27.1 -> 21.9, 768 x 2048 x 8192 50 -> 37, 288 x
-18560 x 4096 75 -> 60; of 483 products, whose plan this changed, the times are 8 % less in the mean, 11 % more at most. A product's time steps up with every round of tiles that is
-begun, so there are many sizes: (5, 8), (8, 6), (7, 6), (6, 6), (7, 4) and (5, 4) beside the ten that were there take 2 % off the mean of 144 products of 80 to
-5000 rows, and, us, cold weights: 2521 x 4096 x 14336 243 -> 213 (256 tiles of 160 x 256, where 192 x 256 left 32 of 256 workgroups out),
-2521 x 2048 x 8192 79 -> 74, 3100 x 6144 x 4096 139 -> 126, 1024 x 18560 x 4096 148 -> 130, 700 x 6144 x 4096 43 -> 38.
+`tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 13 900 timings on an MI355X (2 590 products
+of 52 weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights); over these its choice is 0.6 % slower than the
+fastest form that was timed in the mean and 19 % at most. A step of 64 of K costs a workgroup its products or, of few rows, its reads:
+weights come from memory, rows from L2, at the rate at which its outstanding loads return (ops.seqmix._rows_cols has the same for a few
+rows). Without that the smallest tiles looked cheaper than they are: us, 224 x 4096 x 4096 27.1 -> 21.9, 768 x 2048 x 8192 50 -> 37,
+288 x 18560 x 4096 75 -> 60; of 483 products, whose plan this changed, the times are 8 % less in the mean, 11 % more at most. A
+product's time steps up with every round of tiles that is begun, so there are many sizes: (5, 8), (8, 6), (7, 6), (6, 6), (7, 4) and
+(5, 4) beside the ten that were there take 2 % off the mean of 144 products of 80 to 5000 rows, and, us, cold weights: 2521 x 4096 x
+14336 243 -> 213 (256 tiles of 160 x 256, where 192 x 256 left 32 of 256 workgroups out), 2521 x 2048 x 8192 79 -> 74, 3100 x 6144 x
+4096 139 -> 126, 1024 x 18560 x 4096 148 -> 130, 700 x 6144 x 4096 43 -> 38.
 """
 from __future__ import annotations
 
