@@ -1,4 +1,4 @@
-// The tile and the parts of K of a product on tile_linear.hip: every form of the kernel is priced, the cheapest wins (the first of
+// The tile and the parts of K of a product on tile_linear.h: every form of the kernel is priced, the cheapest wins (the first of
 // equals). Prompt steps rarely have the row count of the one before, so the search runs for every product of nearly every step: in
 // Python it took 20 to 140 us a product, here 2 with the call; a step of a new row count, Dofivik "1b", 80 to 130 rows, 1886 -> 1733 us
 // until its end, Loluzen 1216 -> 1177, Vizonex 1142 -> 1027. The prices and the rules around them are ops/tile_linear.py's.

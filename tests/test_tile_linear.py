@@ -1,4 +1,4 @@
-"""Products of many rows (csrc/mixers/tile_linear.hip): every tile at its edges, parts of K, what follows the product."""
+"""Products of many rows (csrc/mixers/tile_linear.h): every tile at its edges, parts of K, what follows the product."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -78,6 +78,38 @@ def test_gated_tiles(tile, M, F_, K, S, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("K,S", [(192, 1), (256, 1), (320, 1), (384, 1), (448, 1), (704, 2), (1216, 3)])   # K of every ring's length and one more
+def test_tiles_one_after_another(tile, K, S, monkeypatch):
+    """Workgroups that go through many tiles of the result, rows and columns left over, give the bits that one per tile gives."""
+    M, N = 64 * tile[0] + 41, 96 * tile[1] + 24
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device="cuda")
+
+    def results():
+        out = [tl.tile_linear((*tile, S), x, w, b), tl.tile_linear((*tile, S), x, w, b.to(torch.bfloat16), sq.ACT_RELU2),
+               tl.tile_linear((*tile, S), x, w, b, sq.ACT_XIELU, 0.7, 0.9), tl.tile_linear((*tile, S), x, w)]
+        out += [tl.tile_linear((*tile, S), x, w, None, sq.ACT_GLU + k, 2.0, 1.702, tl.PAIR_HALVES)
+                for k in (sq.GLU_GELU_TANH, sq.GLU_CLAMPED, sq.GLU_SILU)]
+        return out + ([tl.tile_parts((*tile, S), x, w).part] if S > 1 else [])
+    got = {}
+    for cus in (1, 3, 1 << 20):
+        monkeypatch.setattr(tl, "cu_count", lambda d, n=cus: n)
+        got[cus] = results()
+    for few, three, own in zip(got[1], got[3], got[1 << 20]):
+        assert torch.equal(few, own) and torch.equal(three, own)
+    _close(got[1][3], x.double() @ w.double().t(), K)
+
+
+def test_results_of_2_31_bytes_a_wave_are_refused():
+    from xgserve.ops._native import mixers
+    with pytest.raises(ValueError):
+        mixers().tile_linear(64, 64, 64, 0, False, 0, 64, 65, 1 << 22, 64, 1, 0, 0, 0.0, 0.0, 4, 4, 256, 0)
+
+
+@pytest.mark.gpu
 def test_prompt_products_take_the_tiles():
     x = torch.randn(300, 2048, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(10304, 2048, device="cuda", dtype=torch.bfloat16) * 2048 ** -0.5
@@ -125,6 +157,27 @@ def test_grouped_tiles(tile, kind, monkeypatch):
         size.index_add_(0, t, wts[t, j, None].double() * (a.abs() @ w2[e].double().abs().t()))
     # the activations are rounded to bf16 (2^-9 of each term of the second product), the sums are fp32
     assert ((got - ref).abs() <= (2.0 ** -9 + F_ * 2.0 ** -23) * size + 1e-5).all(), float(((got - ref).abs() / size).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tl._GROUPED)
+def test_grouped_tiles_one_after_another(tile, monkeypatch):
+    """Workgroups that go through the tiles of several experts give the bits that one per tile gives."""
+    K, F_, W, top, E = 448, 576, 136, 2, 6
+    g = torch.Generator("cuda").manual_seed(tile[1])
+    T = 64 * tile[0] + 77
+    ids = torch.stack([torch.randperm(E, generator=g, device="cuda")[:top] for _ in range(T)]).to(torch.int32)
+    h = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16)
+    w13 = (torch.randn(E, 2 * F_, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    w2 = (torch.randn(E, W, F_, generator=g, device="cuda") * F_ ** -0.5).to(torch.bfloat16)
+    wts = torch.rand(T, top, generator=g, device="cuda")
+    monkeypatch.setattr(sq, "grouped_plan", lambda *a: tile)
+    monkeypatch.setattr(sq, "_experts_on_tiles", lambda *a: True)
+    got = []
+    for cus in (1, 5, 1 << 20):
+        monkeypatch.setattr(sq, "cu_count", lambda d, n=cus: n)
+        got.append(sq.routed_experts(h, w13, w2, ids, wts, sq.GLU_SILU))
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[2])
 
 
 @pytest.mark.gpu

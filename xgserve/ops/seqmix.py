@@ -23,7 +23,8 @@ from .. import tune
 from ._native import is_f32, mixers, native_device, on_current_device, stream_ptr
 from .linear import cu_count
 from .moe import _moe_pf_cfg
-from .tile_linear import GROUPED_EXPERTS_MAX, PAIR_HALVES, forward_only as _forward_only, grouped_plan, tile_linear, tile_plan_of
+from .tile_linear import (COLUMNS_END, GROUPED_EXPERTS_MAX, PAIR_HALVES, forward_only as _forward_only, grouped_plan, tile_linear,
+                          tile_plan_of)
 
 
 @dataclass
@@ -1200,7 +1201,7 @@ ACT_RELU2 = 2   # routed_experts(kind=...): an expert without a gate, W_down rel
 MOE_MFMA = tune.get_bool("moe_mfma", True)
 # XGS_TUNE seq_moe_pf=0: the gated experts of long steps stay on grouped_gemm (A/B and tests)
 SEQ_MOE_PF = tune.get_bool("seq_moe_pf", True)
-# Average rows per expert from which gated experts run on the tiles of tile_linear.hip: up to there most segments fit one tile of 64
+# Average rows per expert from which gated experts run on the tiles of tile_linear.h: up to there most segments fit one tile of 64
 # rows of the weight-streaming products, and experts of less than MOE_TILED_ELEMS gate and up weights stay on those up to where
 # gemm_pf's form would begin. Cold weights, with router and shared expert, us, streamed / tiles: 8 experts of 2 x 3584 x 4096, average
 # 45 228 / 210, 57 246 / 217, 75 290 / 241; of 2 x 2048 x 2048 101 / 104, 103 / 108, 116 / 124, 100 167 / 127.
@@ -1327,7 +1328,7 @@ def _experts_on_tiles(pairs: int, E: int, K: int, F_: int, W: int, T: int) -> bo
     """Whether gated experts of these sizes run on tile_linear's grouped form: enough rows per expert, whole column groups, and what a
     lane's 32-bit byte offset reaches (the rows, an expert's weights, the activations in their sorted layout)."""
     least = MOE_TILED_MIN if 2 * F_ * K >= MOE_TILED_ELEMS else max(MOE_TILED_MIN, MOE_PF_MIN)
-    return pairs >= least * E and E <= GROUPED_EXPERTS_MAX and W % 8 == 0 \
+    return pairs >= least * E and E <= GROUPED_EXPERTS_MAX and W % 8 == 0 and max(2 * F_, W) < COLUMNS_END \
         and max(T * K, 2 * F_ * K, W * F_, _sorted_rows(pairs, E, 16) * F_) < 1 << 31
 
 

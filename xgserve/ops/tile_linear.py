@@ -1,4 +1,4 @@
-"""Products of many rows (prompt steps) on csrc/mixers/tile_linear.hip: the sizes they run at, and where the library's stay.
+"""Products of many rows (prompt steps) on csrc/mixers/tile_linear.h: the sizes they run at, and where the library's stay.
 
 `tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 13 900 timings on an MI355X (2 590 products
 of 52 weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights); over these its choice is 0.6 % slower than the
@@ -40,6 +40,7 @@ _SPLITS = (1, 2, 3, 4, 6, 8, 12, 16)
 _SPLIT_K, _SPLIT_TILES = 256, 540           # a part's least K; parts of all tiles at most (a bound on the slabs: 2.1 tiles per CU)
 
 PAIR_NONE, PAIR_HALVES, PAIR_BLOCKS = 0, 1, 2   # rows of a gated weight: [gate | up], or 16 gate rows, 16 up rows, ...
+COLUMNS_END = 1 << 22                       # 128 rows of fp32 results stay below 2^31 bytes
 TILE_ROWS_MIN = 65                          # (up to 64 rows the weights are streamed past them: rows_linear)
 
 
@@ -128,8 +129,8 @@ def tile_plan_of(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     if ldk != K or K < 64 or K % 64 or N < 8 or N % (32 if pairs == PAIR_BLOCKS else 8) or not w.is_contiguous() or \
             x.stride(1) != 1 or x.stride(0) < K or x.stride(0) % 8 or (x.data_ptr() | w.data_ptr()) % 16:
         return None
-    # (a lane's offsets are 32 bits: of the whole weight, and of a tile's rows; tiles are counted in an int)
-    if 2 * N * K >= 1 << 32 or 512 * x.stride(0) >= 1 << 32 or M * N >= 1 << 40:
+    # (a lane's offsets are 32 bits: of the whole weight, of a tile's rows and of its results; tiles are counted in an int)
+    if 2 * N * K >= 1 << 32 or 512 * x.stride(0) >= 1 << 32 or N >= COLUMNS_END or M * N >= 1 << 40:
         return None
     if bias is not None and not (pairs == PAIR_NONE and bias.device == x.device and bias.dtype in (torch.float32, torch.bfloat16)
                                  and bias.shape == (N,) and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
