@@ -56,6 +56,15 @@ enum { kPairNone = 0, kPairHalves = 1, kPairBlocks = 2 };               // w's r
 // 29, 400 x 18560 x 4096 73 / 77, 1024 x 2048 x 8192 45 / 80; both products of 8 experts of 2 x 3584 x 4096 with 75 rows each 176 / 152,
 // with 250 290 / 270.
 constexpr int kRotateRows = 256;
+// A CU has some 100 requests under way, and what it gets is what their latency leaves: 130 bytes a ns from L2, 60 from the Infinity
+// Cache. Row tiles on the same columns would all ask for the same rows of w at the same time and each wait for memory; so number r of
+// them takes K tiles in the order t ^ r within groups of four (of two where there are two): each fetches a share and finds the others' in
+// L2. For tiles whose loads take longer than their products, up to eight row tiles, weights beyond 24 MB (smaller ones come soon enough
+// and lose by it: 275 x 4096 x 2048, gated, on 128 x 64 12.2 / 12.7). us, without / with: 512 x 6144 x 4096 on 128 x 128
+// 38.5 / 31.3, 512 x 4096 x 4096 on 128 x 64 27.7 / 24.1, 1024 x 2048 x 8192 on 128 x 128 65.4 / 52.9, 1500 x 8192 x 2048 on 192 x 192
+// 59.9 / 54.6, 300 x 18560 x 4096 on 160 x 128 84.6 / 71.0 (in groups of four 78); but 130 x 28672 x 4096, gated, on 128 x 128 66.1 / 67.3,
+// and with more row tiles 2521 x 2048 x 8192 on 192 x 128 79.3 / 81.2, 4001 rows on 256 x 128 104.3 / 107.2.
+constexpr int kStaggerTiles = 8, kStaggerArea = 256 * 192, kStaggerWeights = 12 << 20;
 constexpr int kTileColumns = 1 << 22;   // a wave's 128 rows of fp32 results are less than 2^31 bytes
 
 struct TileArgs {
@@ -73,6 +82,7 @@ struct TileArgs {
   int E, top;
   int64_t w_stride;
   bool rotate;             // column tiles start at different K tiles
+  bool stagger;            // row tiles take them in different orders
 };
 
 // LDS DMA of 16 bytes a lane from a uniform base and a lane's byte offset
@@ -176,6 +186,127 @@ __device__ __forceinline__ void tile_by_act(const TileArgs& a, F f) {
   }
 }
 
+// the same in all lanes, and in a scalar register
+__device__ __forceinline__ int tile_one(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ const char* tile_one(const char* p) {
+  const uint64_t v = reinterpret_cast<uintptr_t>(p);
+  uint64_t u = (uint64_t)(uint32_t)tile_one((int)(v >> 32)) << 32 | (uint32_t)tile_one((int)(uint32_t)v);
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_nop 4" : "+s"(u));   // (a load's base that a vector instruction wrote)
+#endif
+  return reinterpret_cast<const char*>(u);
+}
+// (what follows from it is computed where it is used, and takes no registers before)
+__device__ __forceinline__ int tile_opaque(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+  return v;
+}
+
+// A tile of the result: rows m0 .. hi - 1 (BM of them at most), columns n0 .., part s of K (nk K tiles of 64 from kt_lo on), expert e.
+// K tiles are asked for from number `rot` on and around, in whole groups (up to `whole`) number u ^ off in u's place.
+struct TileAt { int m0, hi, n0, s, kt_lo, nk, rot, whole, off, e; };
+// ... number v of `total` = TN column tiles for every row tile and part: columns of up to 8 row tiles next to each other
+template <int BM, int BN, bool GRP>
+__device__ __forceinline__ TileAt tile_at(const TileArgs& a, int TN, int v) {
+  constexpr bool STAGGER = !GRP && BM * BN < kStaggerArea;
+  TileAt t;
+  int TM = (a.M + BM - 1) / BM, u = v, lo = 0;
+  t.hi = a.M, t.s = t.e = 0;
+  if constexpr (GRP) {   // the experts' tiles one expert after the other
+    for (;; ++t.e) {
+      lo = a.offs[t.e], t.hi = a.offs[t.e + 1], TM = (t.hi - lo + BM - 1) / BM;
+      if (u < TM * TN) break;
+      u -= TM * TN;
+    }
+  } else {
+    t.s = v / (TM * TN), u = v - t.s * TM * TN;
+  }
+  const int GM = TM < 8 ? TM : 8, gid = u / (GM * TN), first = gid * GM;
+  const int gm = TM - first < GM ? TM - first : GM, ug = u - gid * GM * TN, tn = ug / gm;
+  t.m0 = lo + (first + ug - tn * gm) * BM, t.n0 = tn * BN;
+  const int nk_all = a.K / 64;
+  t.kt_lo = t.s * nk_all / a.S;
+  t.nk = (t.s + 1) * nk_all / a.S - t.kt_lo;
+  t.rot = a.rotate ? (unsigned)tn * 37u % (unsigned)t.nk : 0;
+  const int others = !STAGGER || !a.stagger || TM < 2 || TM > kStaggerTiles ? 0 : TM < 3 ? 1 : 3;
+  t.whole = t.nk & ~others, t.off = (ug - tn * gm) & others;
+  return t;
+}
+// the block's place among nb neighbours in that order: neighbours on one XCD
+__device__ __forceinline__ int tile_order(int nb) {
+  const int bid = blockIdx.x, q8 = nb >> 3, r8 = nb & 7, xcd = bid & 7;
+  return (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
+}
+// what a lane asks for of a K tile, from the tile's bases: x pieces wv FM + i, w pieces wv FN + i, 8 rows of 128 bytes each
+template <int FM, int FN, bool PAIR, bool GRP>
+__device__ __forceinline__ void tile_offsets(const TileArgs& a, const TileAt& t, int wv, int lane, uint32_t (&ao)[FM], uint32_t (&wo)[FN]) {
+  const int at = tile_opaque(lane), dr = at >> 3, dj = at & 7, half = a.N / 2;
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    int r = min(8 * (wv * FM + i) + dr, t.hi - 1 - t.m0);
+    if (GRP) r += t.m0;
+    if (GRP && a.rows) r = max(a.rows[r], 0) / a.top;
+    ao[i] = (uint32_t)r * (uint32_t)(2 * a.ld_x) + 16 * (dj ^ dr);
+  }
+#pragma unroll
+  for (int i = 0; i < FN; ++i) {
+    const int p = wv * FN + i;
+    int r;
+    if (PAIR) {
+      const int c = min(t.n0 / 2 + 4 * p + (dr & 3), half - 1);
+      r = a.pairs == kPairHalves ? c + (dr >> 2) * half : 2 * (c & ~15) + (c & 15) + (dr >> 2) * 16;
+    } else {
+      r = min(t.n0 + 8 * p + dr, a.N - 1);
+    }
+    wo[i] = (uint32_t)r * (uint32_t)(2 * a.K) + 16 * (dj ^ ((dr & 3) | ((p & 1) << 2)));
+  }
+}
+
+// Where a wave's results go: a lane holds 8 neighbouring columns of a row (two fragments), or 4 gate and 4 up columns. Through a buffer
+// descriptor of the rows that there are: a lane outside stores nothing, and needs no branch.
+template <bool PAIR>
+struct TileOut {
+  char* dst;
+  uint32_t bytes, place, at, row_bytes, esz, half;   // place: this lane's row and columns from the first; at: with a column group's
+  int cols, g4;
+  // `rows` rows from row `row` on, columns from `col` of the result on
+  __device__ __forceinline__ void start(const TileArgs& a, int s, int row, int rows, int col, int l16, int g) {
+    half = a.N / 2, cols = PAIR ? half : a.N, esz = a.part ? 4 : 2, row_bytes = (uint32_t)(a.part ? a.N : cols) * esz, g4 = g;
+    char* base = a.part ? reinterpret_cast<char*>(a.part) + ((int64_t)s * a.M + row) * row_bytes + col * 4
+                        : reinterpret_cast<char*>(a.out) + (int64_t)row * row_bytes + col * 2;
+    const uint32_t all = (uint32_t)max(0, rows) * row_bytes;   // (the last row ends col columns ahead of so many bytes)
+    dst = const_cast<char*>(tile_one(base)), bytes = tile_one(all > col * esz ? all - col * esz : 0u);
+    place = (uint32_t)tile_opaque(l16) * row_bytes + (PAIR ? 4 : 8) * g4 * esz;
+  }
+  __device__ __forceinline__ void columns(int j, int col) {   // group j, lane 0's first column being `col`
+    at = (PAIR ? 4 : 8) * g4 < cols - col ? place + (PAIR ? 16 : 32) * j * esz : 0x80000000u;   // (a wave's rows are less than 2^31 bytes)
+  }
+  template <int ACT>
+  __device__ __forceinline__ void put(const TileArgs& a, int m, f32x4_t lo, f32x4_t hi, const float (&b)[8]) {
+    typedef __attribute__((ext_vector_type(4))) uint32_t u4;
+    typedef __attribute__((ext_vector_type(2))) uint32_t u2;
+    const uint32_t off = at + 16 * m * row_bytes;
+    const auto to = __builtin_amdgcn_make_buffer_rsrc(dst, 0, bytes, 0x00020000);
+    if constexpr (ACT == kTilePart) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, lo), to, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, hi), to, PAIR ? off + half * 4 : off + 16, 0, 0);
+    } else if constexpr (PAIR) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile_glu<ACT>(a, lo[e], hi[e]);
+      __builtin_amdgcn_raw_buffer_store_b64(u2{xgk::pack2(v[0], v[1]), xgk::pack2(v[2], v[3])}, to, off, 0, 0);
+    } else {
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = tile_act<ACT>(a, lo[e] + b[e]), o[4 + e] = tile_act<ACT>(a, hi[e] + b[4 + e]);
+      const u4 v = {xgk::pack2(o[0], o[1]), xgk::pack2(o[2], o[3]), xgk::pack2(o[4], o[5]), xgk::pack2(o[6], o[7])};
+      __builtin_amdgcn_raw_buffer_store_b128(v, to, off, 0, 0);
+    }
+  }
+};
+
 // f(0) .. f(N - 1), each index a constant
 template <typename F, int... I>
 __device__ __forceinline__ void tile_each(std::integer_sequence<int, I...>, F f) {
@@ -227,78 +358,26 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
     for (int e = 0; e < a.E; ++e) total += (a.offs[e + 1] - a.offs[e] + BM - 1) / BM * TN;
     if ((int)blockIdx.x >= total) return;
   }
-  const int nk_all = a.K / 64, half = a.N / 2;
-  struct Tile { int m0, hi, n0, s, nk; };
-  Tile ld, cur;        // the tile that is loaded, and the one whose products run
-  uint32_t ao[FM], wo[FN], kx, kw;   // what this lane asks for: A pieces wv FM + i, W pieces wv FN + i, 8 rows of 128 bytes each; place in a row
+  TileAt ld, cur;      // the tile that is loaded, and the one whose products run
+  uint32_t ao[FM], wo[FN], kx, kw;   // what this lane asks for; place in a row
+  uint32_t ux, uw;     // ... counted (128 bytes a K tile)
   const char *xb, *wb;
   int done = 0;
-  auto opaque = [](int v) __attribute__((always_inline)) {   // (what follows from it is computed where it is used, and takes no registers before)
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(v));
-#endif
-    return v;
-  };
-  auto one = [](int v) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(v); };   // (the same in all lanes, and in a scalar register)
-  auto one_ptr = [&](const char* p) __attribute__((always_inline)) {
-    const uint64_t v = reinterpret_cast<uintptr_t>(p);
-    uint64_t u = (uint64_t)(uint32_t)one((int)(v >> 32)) << 32 | (uint32_t)one((int)(uint32_t)v);
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_nop 4" : "+s"(u));   // (a load's base that a vector instruction wrote)
-#endif
-    return reinterpret_cast<const char*>(u);
-  };
-  // the tile at place `done` of the order: neighbours on one XCD, columns of up to 8 row tiles next to each other
-  auto place = [&]() __attribute__((always_inline)) {
-    const int nb = min((int)gridDim.x, total - done), bid = blockIdx.x, q8 = nb >> 3, r8 = nb & 7, xcd = bid & 7;
-    const int v = done + (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (bid >> 3);
-    int TM = (a.M + BM - 1) / BM, u = v, lo = 0, e = 0;
-    ld.hi = a.M, ld.s = 0;
-    if constexpr (GRP) {   // the experts' tiles one expert after the other
-      for (;; ++e) {
-        lo = a.offs[e], ld.hi = a.offs[e + 1], TM = (ld.hi - lo + BM - 1) / BM;
-        if (u < TM * TN) break;
-        u -= TM * TN;
-      }
-    } else {
-      ld.s = v / (TM * TN), u = v - ld.s * TM * TN;
-    }
-    const int GM = TM < 8 ? TM : 8, gid = u / (GM * TN), first = gid * GM;
-    const int gm = TM - first < GM ? TM - first : GM, ug = u - gid * GM * TN, tn = ug / gm;
-    ld.m0 = lo + (first + ug - tn * gm) * BM, ld.n0 = tn * BN;
-    const int kt_lo = ld.s * nk_all / a.S;
-    ld.nk = (ld.s + 1) * nk_all / a.S - kt_lo;
-    kx = kw = a.rotate ? (unsigned)tn * 37u % (unsigned)ld.nk * 128u : 0u;
-    const int at = opaque(lane), dr = at >> 3, dj = at & 7;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      int r = min(8 * (wv * FM + i) + dr, ld.hi - 1 - ld.m0);
-      if (GRP) r += ld.m0;
-      if (GRP && a.rows) r = max(a.rows[r], 0) / a.top;
-      ao[i] = (uint32_t)r * (uint32_t)(2 * a.ld_x) + 16 * (dj ^ dr);
-    }
-#pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      const int p = wv * FN + i;
-      int r;
-      if (PAIR) {
-        const int c = min(ld.n0 / 2 + 4 * p + (dr & 3), half - 1);
-        r = a.pairs == kPairHalves ? c + (dr >> 2) * half : 2 * (c & ~15) + (c & 15) + (dr >> 2) * 16;
-      } else {
-        r = min(ld.n0 + 8 * p + dr, a.N - 1);
-      }
-      wo[i] = (uint32_t)r * (uint32_t)(2 * a.K) + 16 * (dj ^ ((dr & 3) | ((p & 1) << 2)));
-    }
-    xb = reinterpret_cast<const char*>(a.x + (GRP ? 0 : (int64_t)ld.m0 * a.ld_x) + kt_lo * 64);
-    wb = reinterpret_cast<const char*>(a.w + (GRP ? e * a.w_stride : 0) + kt_lo * 64);
-    ld.m0 = one(ld.m0), ld.hi = one(ld.hi), ld.n0 = one(ld.n0), ld.s = one(ld.s), ld.nk = one(ld.nk), kx = kw = one(kx);
-    xb = one_ptr(xb), wb = one_ptr(wb);
+  auto k_of = [&](uint32_t u) __attribute__((always_inline)) { return u ^ (u < (uint32_t)ld.whole ? ld.off : 0); };
+  auto place = [&]() __attribute__((always_inline)) {   // the block's next tile
+    ld = tile_at<BM, BN, GRP>(a, TN, done + tile_order(min((int)gridDim.x, total - done)));
+    tile_offsets<FM, FN, PAIR, GRP>(a, ld, wv, lane, ao, wo);
+    xb = tile_one(reinterpret_cast<const char*>(a.x + (GRP ? 0 : (int64_t)ld.m0 * a.ld_x) + ld.kt_lo * 64));
+    wb = tile_one(reinterpret_cast<const char*>(a.w + (GRP ? ld.e * a.w_stride : 0) + ld.kt_lo * 64));
+    ld.m0 = tile_one(ld.m0), ld.hi = tile_one(ld.hi), ld.n0 = tile_one(ld.n0), ld.s = tile_one(ld.s), ld.nk = tile_one(ld.nk);
+    ld.whole = tile_one(ld.whole) * 128, ld.off = tile_one(ld.off) * 128;
+    ux = uw = tile_one(ld.rot) * 128u, kx = kw = k_of(ux);
   };
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t) reinterpret_cast<uintptr_t>((xgk::lds_void_t*)lds));
   const uint32_t lds_a = lds0 + wv * FM * 1024, lds_w = lds0 + RA * ASZ + wv * FN * 1024;
-  auto next = [&](uint32_t& k) __attribute__((always_inline)) {
-    k += 128;
-    if (k == (uint32_t)ld.nk * 128u) k = 0;
+  auto next = [&](uint32_t& k, uint32_t& u) __attribute__((always_inline)) {
+    u = u + 128 == (uint32_t)ld.nk * 128 ? 0 : u + 128;
+    k = k_of(u);
   };
 
   // ---- fragment reads: x row 16 i + l16, W row 32 (i / 2) + 8 (l16 / 4) + l16 % 4 + 4 (i % 2); K half ks
@@ -318,8 +397,8 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
   };
   int sa, sw;          // slots of the K tile at hand
 
-  // ---- results: a lane holds 8 neighbouring columns of a row (two fragments), or 4 gate and 4 up columns
-  Tile old;            // the tile whose results are in the accumulators
+  // ---- results
+  TileAt old;          // the tile whose results are in the accumulators
   constexpr int NB = (16 * FN + 63) / 64;   // lane l holds the biases of the wave's columns l, l + 64: 16 lanes need the same eight
   float bias[NB], b[8];
   const bool biased = !PAIR && a.bias && !a.part;
@@ -335,56 +414,15 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
       bias[i] = a.bias_f32 ? ((const float*)a.bias)[col] : ldf((const bf16*)a.bias + col);
     }
 #pragma unroll
-    for (int i = 0; i < NB; ++i) bias[i] = __int_as_float(opaque(__float_as_int(bias[i])));   // (they are waited for here)
+    for (int i = 0; i < NB; ++i) bias[i] = __int_as_float(tile_opaque(__float_as_int(bias[i])));   // (they are waited for here)
   };
   auto biases_of = [&](int j) __attribute__((always_inline)) {
     if (!biased) return;
-    const int from = opaque(32 * g4) + 4 * (32 * j & 63);
+    const int from = tile_opaque(32 * g4) + 4 * (32 * j & 63);
 #pragma unroll
     for (int e = 0; e < 8; ++e) b[e] = __int_as_float(__builtin_amdgcn_ds_bpermute(from + 4 * e, __float_as_int(bias[32 * j / 64])));
   };
-  // (through buffer descriptors of the wave's rows that there are: a lane outside stores nothing, and needs no branch)
-  const int cols = PAIR ? half : a.N;
-  const uint32_t esz = a.part ? 4 : 2, row_bytes = (uint32_t)(a.part ? a.N : cols) * esz;
-  char* dst = nullptr;
-  uint32_t dst_bytes = 0;
-  uint32_t place_in = 0, col_in = 0;   // bytes from the wave's first row and column: of this lane, and with a column group's
-  auto results_to = [&]() __attribute__((always_inline)) {
-    const int row = old.m0 + wm * 16 * FM, col = PAIR ? old.n0 / 2 + wn * 8 * FN : old.n0 + wn * 16 * FN;
-    char* base = a.part ? reinterpret_cast<char*>(a.part) + ((int64_t)old.s * a.M + row) * row_bytes + col * 4
-                        : reinterpret_cast<char*>(a.out) + (int64_t)row * row_bytes + col * 2;
-    const int rows = max(0, min(old.hi - row, 16 * FM));
-    // (the first column is not the row's: the last row's end is col before the last byte's)
-    const uint32_t bytes = (uint32_t)rows * row_bytes;
-    dst = const_cast<char*>(one_ptr(base)), dst_bytes = one(bytes > col * esz ? bytes - col * esz : 0u);
-    place_in = (uint32_t)opaque(l16) * row_bytes + (PAIR ? 4 : 8) * g4 * esz;
-  };
-  auto columns = [&](int j) __attribute__((always_inline)) {
-    const int col = PAIR ? old.n0 / 2 + wn * 8 * FN + 16 * j : old.n0 + wn * 16 * FN + 32 * j;   // of lane 0
-    col_in = (PAIR ? 4 : 8) * g4 < cols - col ? place_in + (PAIR ? 16 : 32) * j * esz : 0x80000000u;
-  };
-  typedef __attribute__((ext_vector_type(4))) uint32_t u4;
-  typedef __attribute__((ext_vector_type(2))) uint32_t u2;
-  auto emit = [&](auto act_c, int m, f32x4_t lo, f32x4_t hi) __attribute__((always_inline)) {
-    constexpr int ACT = decltype(act_c)::value;
-    const uint32_t at = col_in + 16 * m * row_bytes;   // (a wave's rows are less than 2^31 bytes)
-    const auto to = __builtin_amdgcn_make_buffer_rsrc(dst, 0, dst_bytes, 0x00020000);
-    if constexpr (ACT == kTilePart) {
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, lo), to, at, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, hi), to, PAIR ? at + half * 4 : at + 16, 0, 0);
-    } else if constexpr (PAIR) {
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = tile_glu<ACT>(a, lo[e], hi[e]);
-      __builtin_amdgcn_raw_buffer_store_b64(u2{xgk::pack2(v[0], v[1]), xgk::pack2(v[2], v[3])}, to, at, 0, 0);
-    } else {
-      float o[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = tile_act<ACT>(a, lo[e] + b[e]), o[4 + e] = tile_act<ACT>(a, hi[e] + b[4 + e]);
-      const u4 v = {xgk::pack2(o[0], o[1]), xgk::pack2(o[2], o[3]), xgk::pack2(o[4], o[5]), xgk::pack2(o[6], o[7])};
-      __builtin_amdgcn_raw_buffer_store_b128(v, to, at, 0, 0);
-    }
-  };
+  TileOut<PAIR> out;
 
   // one step: the products of K half KS, and between them the other half's reads and the next loads, one at a time. MODE: loads go out;
   // none are left; the first step of a tile, which takes the last one's results out of the accumulators it starts
@@ -395,7 +433,10 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
     const char* src = KS ? xb + kx : wb + kw;
     const uint32_t at = KS ? lds_a + sa * ASZ : lds_w + (sw == 0 ? RW - 1 : sw - 1) * WSZ;
     f32x4_t lo, hi;
-    if constexpr (MODE == kJoin) results_to();
+    if constexpr (MODE == kJoin) {
+      const int row = old.m0 + wm * 16 * FM;
+      out.start(a, old.s, row, min(old.hi - row, 16 * FM), PAIR ? old.n0 / 2 + wn * 8 * FN : old.n0 + wn * 16 * FN, l16, g4);
+    }
     tile_each<FM * FN>([&](auto q_c) __attribute__((always_inline)) {
       constexpr int q = decltype(q_c)::value, IN = XL ? FN : FM;
       constexpr int o = q / IN, i = o & 1 ? IN - 1 - q % IN : q % IN;   // there and back: the operand at the turn stays
@@ -404,20 +445,20 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
       const uint32_t off = KS ? ao[d >= 0 && d < FM ? d : 0] : wo[d >= 0 && d < FN ? d : 0];
       if constexpr (MODE >= kStart) {
         if (MODE == kJoin && q % (2 * FM) == 0) {
-          columns(n / 2);
+          out.columns(n / 2, PAIR ? old.n0 / 2 + wn * 8 * FN + 8 * n : old.n0 + wn * 16 * FN + 16 * n);
           if (!PAIR) biases_of(n / 2);
         }
         if (MODE == kJoin && q % 2 == 0) lo = TileAcc<m * FN + (n & ~1)>::take(), hi = TileAcc<m * FN + (n | 1)>::take();
         TileAcc<m * FN + n>::first(wf[KS][n], af[KS][m]);
         if (d >= 0 && load) tile_dma(src, off, at + d * 1024);
-        if (MODE == kJoin && q % 2 == 1) emit(act_c, m, lo, hi);
+        if (MODE == kJoin && q % 2 == 1) out.template put<decltype(act_c)::value>(a, m, lo, hi, b);
       } else if constexpr (MODE == kRun && d >= 0) {
         TileAcc<m * FN + n>::mul_dma(wf[KS][n], af[KS][m], src, off, at + d * 1024);
       } else {
         TileAcc<m * FN + n>::mul(wf[KS][n], af[KS][m]);
       }
       if (q % RS == 0 && q / RS < LD) read(q / RS, KS ^ 1, ra, rw);
-      if (MODE != kLast && q == FM * FN - 2) next(KS ? kx : kw);
+      if (MODE != kLast && q == FM * FN - 2) KS ? next(kx, ux) : next(kw, uw);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -436,12 +477,12 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
     if (t + RA >= 0 && (!SHORT || t + RA < ld.nk)) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) tile_dma(xb + kx, ao[i], lds_a + (t + RA) * ASZ + i * 1024);
-      next(kx);
+      next(kx, ux);
     }
     if (SHORT ? t + RW < ld.nk : t < -1) {
 #pragma unroll
       for (int i = 0; i < FN; ++i) tile_dma(wb + kw, wo[i], lds_w + (t + RW) * WSZ + i * 1024);
-      next(kw);
+      next(kw, uw);
     }
   }
   done += gridDim.x;

@@ -103,6 +103,18 @@ def test_tiles_one_after_another(tile, K, S, monkeypatch):
     _close(got[1][3], x.double() @ w.double().t(), K)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [t for t in sorted(tl._TILES) if t[0] * t[1] < 48])
+@pytest.mark.parametrize("tiles,S", [(2, 1), (3, 1), (4, 2), (8, 1), (9, 1)])
+def test_row_tiles_that_take_k_in_other_orders(tile, tiles, S):
+    """Weights beyond 24 MB, groups of two and of four K tiles, K tiles left over behind the last group; around, too (up to 256 rows)."""
+    M, N, K = 32 * tile[0] * tiles - 13, 1544, 8192 + 192
+    g = torch.Generator("cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    _close(tl.tile_linear((*tile, S), x, w), x.double() @ w.double().t(), K)
+
+
 def test_results_of_2_31_bytes_a_wave_are_refused():
     from xgserve.ops._native import mixers
     with pytest.raises(ValueError):
