@@ -1,0 +1,107 @@
+"""The residual sum, its norm and the convolution behind it of prompt rows in one pass (ops.seqmix.norm_conv_rows,
+residual_norm_conv_rows), against fp64.
+
+Tolerance: fp32 arithmetic (a few 2^-24 per term, n 2^-24 relative for a sum of n squares, halved by the root); bf16 results
+rounded once (2^-8)."""
+import pytest
+import torch
+
+from xgserve.ops import seqmix as sq
+
+from _seq_util import record_native
+
+pytestmark = pytest.mark.gpu
+
+
+def meta(lens, ctx, slots):
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    n, first = len(lens), [sum(lens[:i]) for i in range(len(lens) + 1)]
+    one = i32([0])
+    return sq.SeqMeta(n, max(lens), i32(first), i32([q + c for q, c in zip(lens, ctx)]), i32(slots), one, one, one, one), first
+
+
+def close(got, want, terms, scale):
+    bits = 2.0 ** -8 if got.dtype == torch.bfloat16 else 0.0
+    assert bool(((got.double().cpu() - want).abs() <= want.abs() * bits + terms * 2.0 ** -23 * scale).all())
+
+
+def norm(v, eps=1e-5):
+    return v / (v.pow(2).mean(-1, keepdim=True) + eps).sqrt()
+
+
+def conv(r, w, state, lens, first, ctx, slots):
+    """(outputs, rows that have one, carried inputs)"""
+    nh, out, live, new = w.shape[1] - 1, r.clone(), torch.zeros(r.shape[0], dtype=torch.bool), state.double().clone()
+    for q, a, c, s in zip(lens, first, ctx, slots):
+        if s < 0 or q == 0:
+            continue
+        hist = state[s].double() * (torch.arange(-nh, 0)[:, None] + c >= 0)
+        ext = torch.cat([hist, r[a:a + q]])
+        for j in range(nh + 1):
+            out[a:a + q] += w.double()[:, j] * ext[j:j + q]
+        live[a:a + q] = True
+        new[s] = ext[-nh:]
+    return out, live, new
+
+
+# strips of 5 rows (4 taps), up to 33 where there are many rows of few columns; sequences that end at a strip, one row before or behind
+@pytest.mark.parametrize("W,taps,lens,behind", [
+    (4, 4, [1, 2, 3, 4, 5, 6, 0, 9, 10, 11], 0), (2048, 4, [5, 1, 7, 16, 2], 3), (2052, 3, [6, 12, 7, 1, 13], 1), (4096, 2, [7, 1, 8, 14, 15], 0),
+    (64, 4, [4001, 1999, 33, 1], 2), (8, 4, [9000, 7000, 2500, 34, 35], 0), (16, 2, [9000, 7000, 2500, 34, 35], 40)])
+def test_against_fp64(W, taps, lens, behind, monkeypatch):
+    calls = record_native(monkeypatch, sq)
+    g = torch.Generator().manual_seed(W + taps)
+    n = len(lens)
+    ctx, slots = [(0, 7, 1, 2, 0)[i % 5] for i in range(n)], [(-1 if i == 3 else n - 1 - i) for i in range(n)]
+    sm, first = meta(lens, ctx, slots)
+    T = first[-1] + behind
+    x, w, b, a1, a2 = torch.randn(T, W, generator=g), *(torch.randn(W, generator=g) for _ in range(4))
+    y, z = (torch.randn(T, W + 8, generator=g).bfloat16()[:, 4:4 + W] for _ in range(2))
+    yg, zg = (torch.randn(T, W + 8).bfloat16().cuda()[:, 4:4 + W].copy_(t) for t in (y, z))
+    cw, state = torch.randn(W, taps, generator=g), torch.randn(n, taps - 1, W, generator=g)
+    for bias in (b, None):
+        xg, st = x.cuda(), state.cuda()
+        out, h = sq.norm_conv_rows(xg, yg, w.cuda(), 1e-5, 0.7, None if bias is None else bias.cuda(), (cw.cuda(), st), sm, torch.bfloat16)
+        r = norm(0.7 * x.double() + y.double() + (0 if bias is None else bias.double())) * (1 + w.double())
+        want, live, new = conv(r, cw, state, lens, first, ctx, slots)
+        big = float(r.abs().max())
+        assert torch.equal(xg.cpu(), x)
+        close(out, r, W / 2 + 16, big)
+        close(h[live], want[live], W / 2 + 40, big * 8)
+        close(st, new, W / 2 + 16, max(big, 5.0))
+    for f32, z2, s1, s2 in ((True, zg, a1, a2), (False, zg, None, a2), (False, None, a1, None)):
+        xg, st = x.cuda(), state.cuda()
+        out, n32, nact, h = sq.residual_norm_conv_rows(xg, yg, None if s1 is None else s1.cuda(), z2, None, None if s2 is None else s2.cuda(),
+                                                       w.cuda(), 1e-5, torch.bfloat16, (cw.cuda(), st), f32, sm)
+        v = x.double() + (1 if s1 is None else s1.double()) * y.double()
+        if z2 is not None:
+            v = v + (1 if s2 is None else s2.double()) * z.double()
+        r = norm(v) * w.double()
+        want, live, new = conv(r, cw, state, lens, first, ctx, slots)
+        big = float(r.abs().max())
+        close(out, v, 24, float(v.abs().max()) + 30)
+        close(nact, r, W / 2 + 16, big)
+        assert (n32 is not None) == f32
+        if f32:
+            close(n32, r, W / 2 + 16, big)
+        close(h[live], want[live], W / 2 + 40, big * 8)
+        close(st, new, W / 2 + 16, max(big, 5.0))
+    assert calls == ["norm_conv"] * 5
+
+
+def test_others_take_the_separate_kernels(monkeypatch):
+    """More than 4096 columns, fp32 rows, a sum over experts, weights off 16 bytes: in place, by the launches they had."""
+    calls = record_native(monkeypatch, sq)
+    lens, ctx, slots, T = [3, 6], [0, 2], [1, 0], 9
+    sm, _ = meta(lens, ctx, slots)
+
+    def ones(*s):
+        return torch.ones(*s, device="cuda")
+    for W, dtype, off in ((4100, torch.bfloat16, 0), (64, torch.float32, 0), (64, torch.bfloat16, 1)):
+        x, w = ones(T, W), ones(W + 4)[off:off + W]
+        out, h = sq.norm_conv_rows(x, ones(T, W).to(dtype), w, 1e-5, 1.0, None, (ones(W, 4), ones(2, 3, W)), sm, dtype)
+        assert out is x and h.dtype == dtype
+    x = ones(T, 64)
+    assert sq.residual_norm_conv_rows(x, ones(T, 64).bfloat16(), None, None, ones(T, 64), None, ones(64), 1e-5, torch.bfloat16,
+                                      (ones(64, 4), ones(2, 3, 64)), False, sm)[0] is x
+    assert "norm_conv" not in calls

@@ -135,17 +135,17 @@ class DofivikLayer(nn.Module):
             self.norm2, self.canon2 = _p(f(W)), _p(f(W, taps))
 
     def forward(self, x, conv, sm: sq.SeqMeta, lc: LayerCache, rot, block_size, dtype, next_conv):
-        """x: fp32 residual (updated in place and returned). conv: a list of one, this layer's first convolution of x, replaced
-        by the one that the next layer begins with (next_conv: its weights and state, or None)."""
+        """x: fp32 residual; its new rows are returned (in x, or in another tensor). conv: a list of one, this layer's first
+        convolution of x, replaced by the one that the next layer begins with (next_conv: its weights and state, or None)."""
         if self.kind == "latent_attention":
             y = self.mix(conv[0], sm, lc.latent, rot, block_size)
         else:
             y = self.mix(conv[0], sm, lc.delta)
         if self.mlp is not None:
-            h = sq.norm_conv(x, y, self.norm1, self.eps, self.alpha, None, (self.canon2, lc.conv2), sm, dtype)
-            conv[0] = sq.norm_conv(x, self.mlp(h, sm), self.norm2, self.eps, self.alpha, self.mlp.down_b, next_conv, sm, dtype)
+            x, h = sq.norm_conv_rows(x, y, self.norm1, self.eps, self.alpha, None, (self.canon2, lc.conv2), sm, dtype)
+            x, conv[0] = sq.norm_conv_rows(x, self.mlp(h, sm), self.norm2, self.eps, self.alpha, self.mlp.down_b, next_conv, sm, dtype)
         else:
-            conv[0] = sq.norm_conv(x, y, self.norm1, self.eps, self.alpha, None, next_conv, sm, dtype)
+            x, conv[0] = sq.norm_conv_rows(x, y, self.norm1, self.eps, self.alpha, None, next_conv, sm, dtype)
         return x
 
 

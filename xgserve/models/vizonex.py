@@ -152,8 +152,9 @@ class VizonexLayer(nn.Module):
                 GatedMLP(W, mlp["ff"], sq.GLU_GELU_TANH, 0.0, device, dtype)
 
     def forward(self, x, h, n32, nact, sm: sq.SeqMeta, lc: LayerCache, block_size: int, next_norm, next_conv, need_f32: bool):
-        """x: fp32 residual (updated in place); n32 / nact: this block's norm of x (fp32 for routers), h: its convolution.
-        Returns (x, the same three of the next block) (next_conv: its convolution's weights and state, or None)."""
+        """x: fp32 residual; n32 / nact: this block's norm of x (fp32 for routers), h: its convolution.
+        Returns x's new rows (in x, or in another tensor) and the same three of the next block (next_conv: its convolution's
+        weights and state, or None)."""
         y1 = self.mix(h, sm, lc, block_size)
         y2 = y3 = None
         if self.mlp is not None:
@@ -161,8 +162,8 @@ class VizonexLayer(nn.Module):
                 y2, y3 = self.mlp(n32, nact, sm)
             else:
                 y2 = self.mlp(nact, sm)
-        n32, nact, h = sq.residual_norm_conv(x, y1, self.ls1, y2, y3, self.ls2, next_norm, self.eps, nact.dtype, next_conv,
-                                             need_f32, sm)
+        x, n32, nact, h = sq.residual_norm_conv_rows(x, y1, self.ls1, y2, y3, self.ls2, next_norm, self.eps, nact.dtype, next_conv,
+                                                     need_f32, sm)
         return x, h, n32, nact
 
 

@@ -416,6 +416,51 @@ def norm_conv(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float, bia
     return causal_conv_residual(x, conv[0], conv[1], sm, dtype) if conv is not None else None
 
 
+# ---------------------------------------------------------------------------- ... and of prompt rows
+def _conv_rows(x: torch.Tensor, y1, y2, a1, a2, bias, w: torch.Tensor, conv: Optional[tuple], sm: SeqMeta, dtype: torch.dtype) -> bool:
+    """Whether norm_conv.hip takes these rows: bf16 activations and results, up to 4096 columns, and not the single tokens of a step in
+    parts, which row_update takes."""
+    if sm.parts or conv is None or dtype != torch.bfloat16 or not native_device(x):
+        return False
+    (T, W), (cw, state) = x.shape, conv
+    return (T >= 1 and W % 4 == 0 and W <= 4096 and isinstance(y1, torch.Tensor) and (y2 is None or isinstance(y2, torch.Tensor))
+            and all(y is None or (y.dtype == torch.bfloat16 and y.shape == x.shape and y.stride(0) >= W) for y in (y1, y2))
+            and _rows_aligned(y1, y2, x, a1, a2, bias, w, cw, state) and all(
+                t is None or (t.dtype == torch.float32 and t.is_contiguous()) for t in (x, a1, a2, bias, w, cw, state))
+            and cw.shape[0] == W and 2 <= cw.shape[1] <= 4 and state.shape[1:] == (cw.shape[1] - 1, W) and sm.num_seqs < 65535)
+
+
+def _norm_conv(x, y1, y2, a1, a2, bias, alpha, w, off, eps, keep_norm, want_f32, want_act, conv, sm):
+    T, W = x.shape
+    cw, state = conv
+    out, h = torch.empty_like(x), torch.empty(T, W, dtype=torch.bfloat16, device=x.device)
+    n32 = torch.empty_like(x) if want_f32 else None
+    nact = torch.empty_like(h) if want_act else None
+    mixers().norm_conv(x.data_ptr(), y1.data_ptr(), y1.stride(0), _p(y2), y2.stride(0) if y2 is not None else 0, _p(a1), _p(a2),
+                       _p(bias), float(alpha), w.data_ptr(), float(off), float(eps), keep_norm, out.data_ptr(), _p(n32), _p(nact),
+                       cw.data_ptr(), cw.shape[1], state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
+                       _i32(sm.slots).data_ptr(), h.data_ptr(), sm.num_seqs, sm.max_q, T, W, 0, stream_ptr())
+    return out, n32, nact, h
+
+
+def norm_conv_rows(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float, bias: Optional[torch.Tensor],
+                   conv: Optional[tuple], sm: SeqMeta, dtype: torch.dtype):
+    """norm_conv as (new x, convolution or None): x itself, updated, or where the rows of a prompt take both in one pass another
+    tensor (a workgroup there reads rows that belong to its neighbour)."""
+    if _conv_rows(x, y, None, None, None, bias, w, conv, sm, dtype):
+        out, _, _, h = _norm_conv(x, y, None, None, None, bias, alpha, w, 1.0, eps, True, False, False, conv, sm)
+        return out, h
+    return x, norm_conv(x, y, w, eps, alpha, bias, conv, sm, dtype)
+
+
+def residual_norm_conv_rows(x: torch.Tensor, y1, a1: Optional[torch.Tensor], y2, y3, a2: Optional[torch.Tensor], norm_w: torch.Tensor,
+                            eps: float, dtype: torch.dtype, conv: Optional[tuple], need_f32: bool, sm: SeqMeta):
+    """residual_norm_conv as (new x, n fp32 where `need_f32`, n as `dtype`, convolution or None); x as in norm_conv_rows."""
+    if y3 is None and _conv_rows(x, y1, y2, a1, a2, None, norm_w, conv, sm, dtype):
+        return _norm_conv(x, y1, y2, a1, a2, None, 1.0, norm_w, 0.0, eps, False, need_f32, True, conv, sm)
+    return x, *residual_norm_conv(x, y1, a1, y2, y3, a2, norm_w, eps, dtype, conv, need_f32, sm)
+
+
 def residual_norm_conv(x: torch.Tensor, y1, a1: Optional[torch.Tensor], y2, y3: Optional[torch.Tensor],
                        a2: Optional[torch.Tensor], norm_w: torch.Tensor, eps: float, dtype: torch.dtype,
                        conv: Optional[tuple], need_f32: bool, sm: SeqMeta):
