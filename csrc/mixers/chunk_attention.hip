@@ -592,6 +592,44 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(const T* __restrict__ o_a
   }
 }
 
+// The same for many rows: a thread has four value columns of one token's key/value head, whose rows it reads once for all REP heads of
+// that key/value head; the weights are the same for the whole workgroup (scalar loads). us, a thread per head and
+// four columns / now: 4001 rows of 16 heads, 2 x 64 columns 19.0 / 11.0, 2 x 128 32.7 / 12.9.
+template <typename T, int REP>
+__global__ __launch_bounds__(256) void talk_mix_rows_kernel(const T* __restrict__ o_all, const float* __restrict__ talk,
+                                                            const T* __restrict__ gate, int64_t ld_gate, T* __restrict__ out, int T_,
+                                                            int H, int G, int dv, int sh) {
+  const int c = blockIdx.y, t = ((int)blockIdx.x * 256 + (int)threadIdx.x) >> sh, d = 4 * (threadIdx.x & ((1 << sh) - 1));   // 2^sh quads
+  if (t >= T_) return;
+  const T* row = o_all + ((int64_t)t * H * G + c) * dv + d;
+  float acc[REP][4];
+#pragma unroll
+  for (int j = 0; j < REP; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[j][i] = 0.f;
+#pragma unroll 8
+  for (int g = 0; g < H; ++g) {
+    float v[4];
+    ld4(row + (int64_t)g * G * dv, v);
+#pragma unroll
+    for (int j = 0; j < REP; ++j) {
+      const float w = talk[(c * REP + j) * H + g];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][i] += w * v[i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < REP; ++j) {
+    const int h = c * REP + j;
+    if (gate) {
+      const float sg = sigmoid_for<T>(ldf(gate + (int64_t)t * ld_gate + h));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][i] *= sg;
+    }
+    st4(out + ((int64_t)t * H + h) * dv + d, acc[j]);
+  }
+}
+
 // The same from the shares that the keys of single tokens were divided into (masked_attention_combine's, vmode all): merged and mixed
 // in one launch, the merged rows in LDS and fp32. A workgroup has 16 value columns of a token, which belong to one key/value head.
 // Both launches it stands for are latency alone: 17 tokens of 16 heads, 2 x 128 value columns, 5.2 + 7.6 us.
@@ -1046,6 +1084,19 @@ int talk_mix_parts(const float* part_o, const float* part_ml, const int32_t* slo
 void talk_mix(const void* o_all, bool f32, const float* talk, const void* gate, int64_t ld_gate, void* out, int T_, int H,
               int G, int dv, hipStream_t st) {
   if (T_ <= 0) return;
+  const int rep = H / G, quads = dv / 4;
+  if (T_ > 256 && dv % 4 == 0 && quads <= 256 && (quads & (quads - 1)) == 0 && (rep == 2 || rep == 4 || rep == 8) && G <= 65535 &&
+      (int64_t)T_ * quads < (1ll << 31)) {
+    int sh = 0;
+    while (1 << sh < quads) ++sh;
+    const dim3 grid((unsigned)(((int64_t)T_ * quads + 255) / 256), G);
+#define XGM_TM(REP)                                                                                                          \
+  XGM_DISPATCH_T(f32, talk_mix_rows_kernel<T, REP><<<grid, 256, 0, st>>>((const T*)o_all, talk, (const T*)gate, ld_gate, (T*)out, \
+                                                                        T_, H, G, dv, sh);)
+    if (rep == 2) { XGM_TM(2) } else if (rep == 4) { XGM_TM(4) } else { XGM_TM(8) }
+#undef XGM_TM
+    return;
+  }
   // few rows: a wave per 256 value columns (17 rows of 16 heads of 128: 7.5 us against 11.7 with a workgroup per row)
   const int waves = dv % 4 == 0 && T_ <= 256 ? std::min(64, (H * dv / 4 + 63) / 64) : 1;
   XGM_DISPATCH_T(f32, talk_mix_kernel<T><<<dim3(T_, waves), waves > 1 ? 64 : 256, 0, st>>>((const T*)o_all, talk, (const T*)gate,

@@ -125,8 +125,8 @@ __global__ void canon_conv_kernel(const TI* __restrict__ x, int64_t ld_in, const
 // TT + TAPS - 1 rows in flight before it uses the first. The first tile of a sequence, the only one that reads the carried
 // inputs, also writes them back (the last rows are a second read of a few cache lines), so no launch follows.
 // Memory-bound (with silu its arithmetic); against the kernel above without its second launch (5 us), us: 8192 x 2048
-// fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 21.1
-// against 49.0, 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us without silu and loses 5 with it.
+// fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 14.8
+// against 49.0 (23.6 with the general exponential and division), 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us without silu and loses 5 with it.
 template <typename TI, typename TO, int TAPS, int TT>
 __global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, int64_t ld_in, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ state,
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, in
       o[e] = (residual ? v[t + NH][e] : 0.f) + bf[e];
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) o[e] += wf[TAPS * e + j] * v[t + j][e];
-      if (act) o[e] = siluf(o[e]);
+      if (act) o[e] = silu_for<TO>(o[e]);
     }
     if (t0 + t < q) st4(out + (int64_t)(q0 + t0 + t) * W + c, o);   // (no early exit: the loop has to unroll)
   }
@@ -353,6 +353,68 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
     stf(dst + R + 2 * i + 1, v * c + u * s);
   }
   for (int i = rot_dims + threadIdx.x; i < rd; i += blockDim.x) stf(dst + R + i, ldf(kr + i));
+}
+
+// The same in quads (Rq, R, rd and the offsets whole ones, aligned rows; Rq + R up to 1024 NV): a row is loaded once, the query latent's
+// and the key/value latent's statistics meet in one exchange. us, entry by entry and
+// read twice / now: 8192 rows of 768 + 256 23.9 / 12.1, of 1536 + 512 33.7 / 16.7.
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void latent_prep4_kernel(const T* __restrict__ proj, int64_t ld, int off_q, int Rq, int off_kv, int R,
+                                                           int rd, const float* __restrict__ wq, const float* __restrict__ wkv,
+                                                           float eps, const int32_t* __restrict__ positions,
+                                                           const int32_t* __restrict__ slot_mapping, const float* __restrict__ rot,
+                                                           int rot_dims, T* __restrict__ cq, T* __restrict__ cache) {
+  __shared__ float red[8];
+  const int t = blockIdx.x, all = Rq + (off_kv < 0 ? 0 : R), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const T* row = proj + (int64_t)t * ld;
+  const int slot = off_kv < 0 ? -1 : slot_mapping[t];
+  Raw4<T> raw[NV];
+  Raw4<float> wt[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = 4 * (threadIdx.x + 256 * j);
+    if (c >= all) continue;
+    raw[j].load(c < Rq ? row + off_q + c : row + off_kv + (c - Rq));
+    wt[j].load(c < Rq ? wq + c : wkv + (c - Rq));
+  }
+  if (slot >= 0) {   // the shared rotary key
+    T* dst = cache + (int64_t)slot * (R + rd) + R;
+    const T* kr = row + off_kv + R;
+    const float* rt = rot + (int64_t)positions[t] * (rot_dims & ~1);
+    for (int i = threadIdx.x; i < rot_dims >> 1; i += 256) {
+      const float c = rt[2 * i], s = rt[2 * i + 1], u = ldf(kr + 2 * i), v = ldf(kr + 2 * i + 1);
+      stf(dst + 2 * i, u * c - v * s);
+      stf(dst + 2 * i + 1, v * c + u * s);
+    }
+    for (int i = rot_dims + threadIdx.x; i < rd; i += 256) stf(dst + i, ldf(kr + i));
+  }
+  float v[NV][4], sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = 4 * (threadIdx.x + 256 * j);
+    if (c >= all) continue;
+    raw[j].get(v[j]);
+    const float ss = v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
+    if (c < Rq) sq += ss;
+    else sk += ss;
+  }
+  sq = wave_sum(sq), sk = wave_sum(sk);
+  if (lane == 0) red[wave] = sq, red[4 + wave] = sk;
+  __syncthreads();
+  const float r = 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)Rq + eps);
+  const float rk = 1.f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)R + eps);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = 4 * (threadIdx.x + 256 * j);
+    if (c >= all) continue;
+    float w[4];
+    wt[j].get(w);
+    const float f = c < Rq ? r : rk;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[j][e] = v[j][e] * f * w[e];
+    if (c < Rq) st4(cq + (int64_t)t * Rq + c, v[j]);
+    else if (slot >= 0) st4(cache + (int64_t)slot * (R + rd) + (c - Rq), v[j]);
+  }
 }
 
 // ------------------------------------------------------------------ latent attention over the paged latent cache
@@ -906,27 +968,27 @@ __global__ void delta_out_kernel(const float* __restrict__ o, const float* __res
         row[d] * r * nw[h * D + d] * sigmoidf(ldf(gate + (int64_t)t * gate_stride + h * D + d)));
 }
 
-// D = 4 L with L a power of two: four entries per lane, 64 / L heads per wave. Memory-bound: 8192 x 32 x 64 29.8 us
-// (4.5 TB/s) against 73.6 with a wave per head.
+// D = 4 L with L a power of two: four entries per lane, 64 / L heads per wave, `nb` workgroups a row. us, with a wave per
+// head / with sums through LDS, a 64-bit division a thread and the general sigmoid, which the vector units bound / now, by memory (6 TB/s):
+// 8192 x 32 x 64 73.6 / 28.9 / 22.4, 2599 x 64 x 64 - / 18.9 / 14.0.
 template <typename T>
 __global__ __launch_bounds__(256) void delta_out4_kernel(const float* __restrict__ o, const float* __restrict__ nw,
                                                          const T* __restrict__ gate, int64_t gate_stride, float eps,
-                                                         T* __restrict__ out, int64_t quads, int HD, int L) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= quads) return;   // (whole heads: HD is a multiple of 4 L)
-  const int64_t t = 4 * i / HD;
-  const int c = (int)(4 * i - t * HD);
+                                                         T* __restrict__ out, int nb, int HD, int L) {
+  const int64_t t = blockIdx.x / nb;
+  const int c = 4 * ((int)(blockIdx.x % nb) * blockDim.x + threadIdx.x);
+  if (c >= HD) return;   // (whole heads: HD is a multiple of 4 L)
   float v[4], w[4], g[4];
   Raw4<T> gr;
   gr.load(gate + t * gate_stride + c);
   ld4(nw + c, w);
-  ld4(o + 4 * i, v);
+  ld4(o + t * HD + c, v);
   const float ss = seg_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], L);
   const float r = 1.f / sqrtf(ss / (float)(4 * L) + eps);
   gr.get(g);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * sigmoidf(g[e]);
-  st4(out + 4 * i, v);
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * sigmoid_for<T>(g[e]);
+  st4(out + t * HD + c, v);
 }
 
 // ------------------------------------------------------------------ activations
@@ -1080,9 +1142,25 @@ void latent_prep(const void* proj, bool f32, int64_t ld, int off_q, int Rq, int 
                  const float* wkv, float eps, const int32_t* positions, const int32_t* slot_mapping, const float* rot,
                  int rot_dims, void* cq, void* cache, int T_, hipStream_t st) {
   if (T_ <= 0) return;
-  XGM_DISPATCH_T(f32, latent_prep_kernel<T><<<T_, 256, 0, st>>>((const T*)proj, ld, off_q, Rq, off_kv, R, rd, wq, wkv, eps,
-                                                                 positions, slot_mapping, rot, rot_dims, (T*)cq,
-                                                                 (T*)cache);)
+  const int esz = f32 ? 4 : 2, all = Rq + (off_kv < 0 ? 0 : R);
+  const bool vec = Rq % 4 == 0 && off_q % 4 == 0 && ld % 4 == 0 && all <= 4096 &&
+                   (off_kv < 0 || (R > 0 && R % 4 == 0 && off_kv % 4 == 0 && (R + rd) % 4 == 0 && (uintptr_t)cache % (4 * esz) == 0 &&
+                                   (uintptr_t)wkv % 16 == 0)) &&
+                   (uintptr_t)proj % (4 * esz) == 0 && (uintptr_t)cq % (4 * esz) == 0 && (uintptr_t)wq % 16 == 0;
+#define XGM_LP(NV)                                                                                                               \
+  XGM_DISPATCH_T(f32, latent_prep4_kernel<T, NV><<<T_, 256, 0, st>>>((const T*)proj, ld, off_q, Rq, off_kv, R, rd, wq, wkv, eps, \
+                                                                    positions, slot_mapping, rot, rot_dims, (T*)cq, (T*)cache);)
+  if (vec && all <= 1024) {
+    XGM_LP(1)
+  } else if (vec && all <= 2048) {
+    XGM_LP(2)
+  } else if (vec) {
+    XGM_LP(4)
+  } else {
+    XGM_DISPATCH_T(f32, latent_prep_kernel<T><<<T_, 256, 0, st>>>((const T*)proj, ld, off_q, Rq, off_kv, R, rd, wq, wkv, eps,
+                                                                  positions, slot_mapping, rot, rot_dims, (T*)cq, (T*)cache);)
+  }
+#undef XGM_LP
 }
 
 template <typename T, int NR>
@@ -1216,11 +1294,11 @@ void delta_out(const float* o, const float* nw, const void* gate, bool f32, int6
                int T_, int H, int D, hipStream_t st) {
   if (T_ <= 0) return;
   const int esz = f32 ? 4 : 2, L = D / 4;
-  const int64_t quads = (int64_t)T_ * H * L;
-  if (D % 4 == 0 && L >= 1 && L <= 64 && (L & (L - 1)) == 0 && gate_stride % 4 == 0 && quads < (1ll << 38) &&
+  const int nb = (H * L + 255) / 256, nth = nb > 1 ? 256 : (H * L + 63) / 64 * 64;
+  if (D % 4 == 0 && L >= 1 && L <= 64 && (L & (L - 1)) == 0 && gate_stride % 4 == 0 && (int64_t)T_ * nb < (1ll << 31) &&
       (uintptr_t)gate % (4 * esz) == 0 && (((uintptr_t)o | (uintptr_t)nw | (uintptr_t)out) & 15) == 0) {
-    XGM_DISPATCH_T(f32, delta_out4_kernel<T><<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(o, nw, (const T*)gate, gate_stride,
-                                                                                             eps, (T*)out, quads, H * D, L);)
+    XGM_DISPATCH_T(f32, delta_out4_kernel<T><<<(unsigned)T_ * nb, nth, 0, st>>>(o, nw, (const T*)gate, gate_stride, eps, (T*)out, nb,
+                                                                               H * D, L);)
     return;
   }
   XGM_DISPATCH_T(f32, delta_out_kernel<T><<<dim3(T_, (H + 3) / 4), 256, 0, st>>>(o, nw, (const T*)gate, gate_stride, eps, (T*)out, H, D);)

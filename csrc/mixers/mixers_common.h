@@ -81,9 +81,31 @@ __device__ __forceinline__ void add_slabs(const float* p, int64_t slab, int n, f
     }
 }
 
-// sum over the L lanes (a power of two) of an aligned segment of the wave
+// sum over the L lanes (a power of two, the same for all) of an aligned segment of the wave, whose lanes all take part: lanes ^ L / 2, ..,
+// 1 joined in turn by register moves, as wave_sum does it
+template <int CTRL>
+__device__ __forceinline__ float lane_dpp(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+#else
+  return v;
+#endif
+}
 __device__ __forceinline__ float seg_sum(float v, int L) {
-  for (int o = L >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (L > 32) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  }
+  if (L > 16) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  }
+#endif
+  if (L > 8) v += lane_dpp<0x128>(v);                    // row_ror:8
+  if (L > 4) v += lane_dpp<0x1B>(lane_dpp<0x141>(v));    // half rows mirrored (^ 7), quads mirrored (^ 3)
+  if (L > 2) v += lane_dpp<0x4E>(v);
+  if (L > 1) v += lane_dpp<0xB1>(v);
   return v;
 }
 
@@ -117,6 +139,21 @@ __device__ __forceinline__ float relu2f(float z) {
   return r * r;
 }
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }
+
+// The same, and the sigmoid, behind which the result is rounded to T. For bf16 (2^-9) by the exponential and reciprocal instructions, 5
+// instructions instead of 25 (off by 2^-23 of it and |x| 2^-24, of what expf and a division give): launches that a full chip's vector
+// work bounds. Error of the bf16 result against fp64 over x of spread 0.3 to 3: the same to five digits.
+template <typename T>
+__device__ __forceinline__ float sigmoid_for(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (sizeof(T) == 2) return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * x));
+#endif
+  return sigmoidf(x);
+}
+template <typename T>
+__device__ __forceinline__ float silu_for(float x) {
+  return sizeof(T) == 2 ? x * sigmoid_for<T>(x) : siluf(x);
+}
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 }  // namespace xgm

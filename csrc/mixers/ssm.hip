@@ -157,24 +157,25 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 }
 
 // Groups of 4 K L values (L lanes, a power of two): K quads per lane stay in registers between the statistic and the
-// result, 64 / L groups per wave. Memory-bound, us: 2521 x 4096 in 8 groups 18.8 against 47.7 a
-// workgroup per group that reads it twice, 4001 x 16 x 128 12.9 against 34.8.
+// result, 64 / L groups per wave. Memory-bound, us: 2521 x 4096 in 8 groups 13.4 against 47.7 a
+// workgroup per group that reads it twice (18.0 with 64-bit divisions a thread, remainders and the general gate), 4001 x 16 x 128 13.4
+// against 34.8.
 template <typename T, int K>
 __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __restrict__ y, const T* __restrict__ z,
                                                                 int64_t ld_z, const float* __restrict__ w, int wn, float eps,
-                                                                T* __restrict__ out, int64_t groups, int ng, int L,
-                                                                int gate_after) {
-  const int64_t g = ((int64_t)blockIdx.x * 256 + threadIdx.x) / L;
-  if (g >= groups) return;
-  const int64_t t = g / ng;
-  const int gs = 4 * K * L, l = threadIdx.x & (L - 1), c0 = (int)(g - t * ng) * gs + 4 * l;
+                                                                T* __restrict__ out, int inner, int nb, int sh, int gate_after) {
+  // `nb` workgroups a row; a group is 2^sh lanes
+  const int64_t t = blockIdx.x / nb;
+  const int i = (int)(blockIdx.x % nb) * blockDim.x + threadIdx.x, L = 1 << sh, gs = 4 * K * L, l = i & (L - 1), c0 = (i >> sh) * gs + 4 * l;
+  if (c0 >= inner) return;
+  y += t * inner, out += t * inner;
   Raw4<float> yr[K], wr[K];
   Raw4<T> zr[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    yr[k].load(y + g * gs + 4 * (l + L * k));
+    yr[k].load(y + c0 + 4 * L * k);
     if (z) zr[k].load(z + t * ld_z + c0 + 4 * L * k);
-    if (w) wr[k].load(w + (c0 + 4 * L * k) % wn);
+    if (w) wr[k].load(w + (wn == inner ? c0 + 4 * L * k : wn == gs ? 4 * (l + L * k) : (c0 + 4 * L * k) % wn));
   }
   float v[K][4], zs[K][4], ss = 0.f;
 #pragma unroll
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __r
     if (z) zr[k].get(zs[k]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      zs[k][e] = z ? siluf(zs[k][e]) : 1.f;
+      zs[k][e] = z ? silu_for<T>(zs[k][e]) : 1.f;
       if (!gate_after) v[k][e] *= zs[k][e];
       ss += v[k][e] * v[k][e];
     }
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __r
       v[k][e] = v[k][e] * r * wf[e];
       if (gate_after) v[k][e] *= zs[k][e];
     }
-    st4(out + g * gs + 4 * (l + L * k), v[k]);
+    st4(out + c0 + 4 * L * k, v[k]);
   }
 }
 
@@ -226,15 +227,17 @@ void gated_group_norm(const float* y, const void* z, bool f32, int64_t ld_z, con
                       int T_, int inner, int ng, bool gate_after, hipStream_t st) {
   if (T_ <= 0) return;
   const int esz = f32 ? 4 : 2, gsz = inner / ng, L = gsz <= 256 ? gsz / 4 : 64, K = L > 0 ? gsz / (4 * L) : 0;
-  const int64_t groups = (int64_t)T_ * ng;
+  const int lanes = ng * L, nb = (lanes + 255) / 256, block = nb > 1 ? 256 : (lanes + 63) / 64 * 64;
   if (L > 0 && (L & (L - 1)) == 0 && 4 * K * L == gsz && (K == 1 || K == 2 || K == 4) && (!w || wn % 4 == 0) &&
-      (!z || (ld_z % 4 == 0 && (uintptr_t)z % (4 * esz) == 0)) && groups * L < (1ll << 38) &&
+      (!z || (ld_z % 4 == 0 && (uintptr_t)z % (4 * esz) == 0)) && (int64_t)T_ * nb < (1ll << 31) &&
       (((uintptr_t)y | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
-    const unsigned blocks = (unsigned)((groups * L + 255) / 256);
+    int sh = 0;
+    while (1 << sh < L) ++sh;
 #define XGM_GN(KK)                                                                                                         \
   if (K == KK) {                                                                                                           \
-    XGM_DISPATCH_T(f32, gated_group_norm4_kernel<T, KK><<<blocks, 256, 0, st>>>(y, (const T*)z, ld_z, w, wn, eps, (T*)out, \
-                                                                               groups, ng, L, gate_after ? 1 : 0);)        \
+    XGM_DISPATCH_T(f32, gated_group_norm4_kernel<T, KK><<<(unsigned)T_ * nb, block, 0, st>>>(y, (const T*)z, ld_z, w, wn, eps, \
+                                                                                         (T*)out, inner, nb, sh,           \
+                                                                                         gate_after ? 1 : 0);)             \
   }
     XGM_GN(1)
     XGM_GN(2)

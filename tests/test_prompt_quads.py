@@ -1,0 +1,89 @@
+"""Row kernels of prompts in quads (latent projections, heads' maps mixed over many rows, group norms over every size of a lane
+group), against fp64 and on both sides of what they accept.
+
+Tolerance: fp32 arithmetic on exact inputs, a few roundings of 2^-24 per term and, for a norm, of its sum of n squares
+(n 2^-24 relative, halved by the root); bf16 results are rounded once (2^-8)."""
+import pytest
+import torch
+
+from xgserve.ops import seqmix as sq
+
+pytestmark = pytest.mark.gpu
+
+
+def close(got, want, terms, scale):
+    bits = 2.0 ** -8 if got.dtype == torch.bfloat16 else 0.0
+    assert bool(((got.double().cpu() - want).abs() <= want.abs() * bits + terms * 2.0 ** -23 * scale).all())
+
+
+def normed(a, w):
+    return a / (a.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double()
+
+
+@pytest.mark.parametrize("Rq,R,rd,rot_dims,off", [(768, 256, 32, 32, 0), (768, 260, 32, 16, 4), (1536, 512, 64, 64, 0), (4, 4, 4, 2, 0),
+                                                  (2048, 2048, 64, 64, 8), (2048, 2052, 64, 64, 0), (768, 254, 32, 32, 0),
+                                                  (768, 256, 32, 32, 2), (1000, 24, 36, 32, 0), (1000, 28, 36, 32, 0)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_latent_rows(Rq, R, rd, rot_dims, off, dt):
+    g, T, slots = torch.Generator().manual_seed(Rq + R), 5, [3, -1, 0, 6, 5]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    one = i32([0])
+    sm = sq.SeqMeta(1, T, i32([0, T]), i32([T]), one, one, one, i32([4, 0, 9, 2, 7]), i32(slots))
+    proj = torch.randn(T, off + Rq + R + rd + 8, generator=g).to(dt)
+    wq, wk = torch.randn(Rq, generator=g), torch.randn(R, generator=g)
+    rot = sq.build_rot_table(rot_dims, 10000.0, 16, "cpu")
+    p = proj.double()
+    want = normed(p[:, off:off + Rq], wq)
+    k, r = normed(p[:, off + Rq:off + Rq + R], wk), p[:, off + Rq + R:off + Rq + R + rd].clone()
+    cs = rot.double().view(16, -1, 2)[sm.positions.long().cpu()]
+    u, v = r[:, 0:rot_dims:2].clone(), r[:, 1:rot_dims:2].clone()
+    r[:, 0:rot_dims:2], r[:, 1:rot_dims:2] = u * cs[..., 0] - v * cs[..., 1], v * cs[..., 0] + u * cs[..., 1]
+    for own in (True, False):
+        cache = torch.full((7, R + rd), 9.0, dtype=dt, device="cuda")
+        cq = sq.latent_prep(proj.cuda(), off, Rq, off + Rq if own else -1, R, rd, wq.cuda(), wk.cuda() if own else None, 1e-5, rot.cuda(),
+                            rot_dims, sm, cache)
+        close(cq, want, Rq / 2 + 8, float(want.abs().max()))
+        held = torch.full((7, R + rd), 9.0, dtype=torch.float64)
+        for t, s in enumerate(slots):
+            if own and s >= 0:
+                held[s] = torch.cat([k[t], r[t]])
+        close(cache, held, R / 2 + 8, 9.0)
+
+
+@pytest.mark.parametrize("H,G,dv", [(16, 2, 64), (16, 2, 128), (8, 4, 32), (8, 2, 4), (4, 4, 64), (6, 2, 64), (16, 2, 48), (8, 1, 1024)])
+@pytest.mark.parametrize("T", [256, 257, 300])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_mixed_maps_of_many_rows(H, G, dv, T, dt):
+    g = torch.Generator().manual_seed(H * dv)
+    o, talk = torch.randn(T, H * G * dv, generator=g).to(dt), torch.randn(H, H, generator=g)
+    gate = torch.randn(T, H + 3, generator=g).to(dt)
+    wide = o.double().view(T, H, G, dv)[:, :, torch.arange(H) // (H // G)]
+    want = (wide * talk.double().T[None, :, :, None]).sum(1)
+    for gt in (gate, None):
+        got = sq.talk_mix(o.cuda(), talk.cuda(), H, G, dv, gate=None if gt is None else gt.cuda())
+        ref = want if gt is None else want * torch.sigmoid(gt[:, :H].double())[:, :, None]
+        close(got, ref.reshape(T, -1), H + 12, 30.0)
+
+
+@pytest.mark.parametrize("size", [4, 8, 16, 32, 64, 128, 256, 512, 1024])
+@pytest.mark.parametrize("groups", [1, 3, 40])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_group_norms(size, groups, dt):
+    g, T, n = torch.Generator().manual_seed(size), 3, size * groups
+    y, z = torch.randn(T, n, generator=g), (3 * torch.randn(T, n, generator=g)).to(dt)
+    for wn in {size, n}:
+        w = torch.randn(wn, generator=g)
+        got = sq.gated_group_norm(y.cuda(), z.cuda(), w.cuda(), 1e-5, groups, dt)
+        v = (y.double() * z.double() * torch.sigmoid(z.double())).view(T, groups, -1)
+        v = (v / (v.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).view(T, n) * w.double().repeat(n // wn)
+        close(got, v, size / 2 + 16, float(v.abs().max()))
+
+
+def test_gates_behind_which_bf16_follows():
+    """Their error against fp64 is that of the rounding: as with expf and a division, to 1 in 10^4."""
+    x = torch.linspace(-12, 12, 1 << 16).bfloat16()
+    o, w = torch.ones(1, x.numel()), torch.ones(x.numel())
+    got = sq.delta_rule_out(o.cuda(), w.cuda(), x[None].cuda(), 0.0, x.numel() // 4, 4, torch.bfloat16).double().cpu()[0]
+    want = torch.sigmoid(x.double())
+    rounded = torch.sigmoid(x.double()).float().bfloat16().double()
+    assert (got - want).norm() <= 1.0001 * (rounded - want).norm()
