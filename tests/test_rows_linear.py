@@ -205,3 +205,24 @@ def test_whole_tiles(T, N, K, cols, monkeypatch):
         v = z + b.double()
         check(sq.linear_relu2(x, w, b, sm), v.clamp(min=0) ** 2, mag + 8, K, 2 * float(v.abs().max()) + 2)
     assert calls == ["rows_linear"] * (1 if cols < 0 else 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,native", [(1, 128256, 4096, True), (16, 32000, 4096, True), (17, 32000, 4096, False), (3, 32004, 2048, True),
+                                          (2, 32002, 2048, False), (1, 512, 4096, False), (4, 32000, 2112, False)])
+def test_heads_of_few_rows(M, N, K, native, monkeypatch):
+    """lm_head_linear: up to 16 rows on rows_linear where it takes the sizes in one part, the library's product else."""
+    from xgserve.ops.linear import lm_head_linear
+    calls = record_native(monkeypatch, sq)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    got = lm_head_linear(x, w).double()
+    want = x.double() @ w.double().T
+    # one rounding to bf16, and fp32 sums of K products of size 1 / sqrt(K)
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -22 * 5).all())
+    assert ("rows_linear" in calls) == native
+    assert lm_head_linear(x.float(), w.float()).dtype == torch.float32 if M <= 16 else True
+    if M <= 16:
+        xr = x.clone().requires_grad_()
+        assert lm_head_linear(xr, w).grad_fn is not None

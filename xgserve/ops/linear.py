@@ -254,7 +254,9 @@ _MW_TUNED = {
     # 64 rows 170.4 us (hipBLASLt 212), 128 rows 175.5 (237), 192 219.5 (257), 256 267 (299)
     (128256, 4096, MODE_BF16): {128: (1, 0), 192: (1, 6), 256: (1, 6)},
 }
-LM_HEAD_MW_MIN_M = 17  # batch <= 16 keeps the library GEMM (not swept)
+# up to 16 rows run on rows_linear: 1 row of 128256 x 4096 155 us against the library's 175 (gemm_mw 154), of 32000 x 4096 43 against 62,
+# of 152064 x 3584 172 against 229; 16 rows 160 / 176, 41 / 58, 173 / 232
+LM_HEAD_MW_MIN_M = 17
 
 
 def _mw_bucket(M: int) -> int:
@@ -389,10 +391,13 @@ def pf_linear(x: torch.Tensor, w: torch.Tensor, mode: int = MODE_BF16, plan=None
 
 
 def lm_head_linear(h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """bf16 logits h . w^T for the LM head: gemm_mw where the sweep measured a plan for
-    this row bucket (_MW_TUNED, mode bf16), else hipBLASLt."""
+    """bf16 logits h . w^T for the LM head: rows_linear for up to 16 rows that it takes, gemm_mw where the sweep
+    measured a plan for this row bucket (_MW_TUNED, mode bf16), else hipBLASLt."""
     M, K = h.shape
     N = w.shape[0]
+    if M < LM_HEAD_MW_MIN_M:
+        from .seqmix import rows_product   # (which builds on this module)
+        return rows_product(h, w)
     if (h.is_cuda and LM_HEAD_MW_MIN_M <= M <= MW_MAX_M and h.is_contiguous() and w.is_contiguous()
             and _mw_bucket(M) in _MW_TUNED.get((N, K, MODE_BF16), {})):
         return mw_linear(h, w, MODE_BF16)

@@ -193,6 +193,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, sm: Optional[SeqMeta] = None,
     return _prompt_linear(x, w, bias) if bias is None or bias.dtype == x.dtype else F.linear(x, w, bias)
 
 
+def rows_product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x . w^T of a few rows behind no step's metadata: rows_linear where it takes them over the whole K, else torch."""
+    plan = _rows_plan_of(x, w, None, None, False)
+    return _rows_linear(plan, x, w, None, None, ACT_NONE, 0.0, 0.0) if plan is not None else F.linear(x, w)
+
+
 @dataclass
 class Parts:
     """A product whose parts of K have not been added: fp32 [parts, T, N]."""
