@@ -1,5 +1,6 @@
 // Latent attention of a step of single tokens (bf16; one token per sequence):
 //
+//   latent_query_kernel    the heads' W_uk folded into their queries: qabs[h][t] = q[t][h] . W_uk[h]
 //   latent_decode_kernel   attention over the cached latents for 32 heads of one sequence and one share of its window
 //   latent_out_kernel      the shares of a (token, head) merged, gated, and expanded by the head's W_uv into the output row
 //
@@ -21,10 +22,48 @@
 
 namespace xgm {
 using xgk::as_frag;
+using xgk::bf16x8_t;
 using xgk::f32x4_t;
 using xgk::mfma16x16x32;
 
 constexpr int kLatentPages = 2048;   // page table entries of a share in LDS
+
+// qabs[h][t][r] = sum_d q[t][h][d] uk[h][d][r], transposed: a wave has 16 columns r of a head for up to 16 MT tokens, dn = 32 NK. Latency
+// alone (64 rows, 32 heads, dn = 64, R = 256: 2 MB in all), so no LDS and no exchange: every load is on its way at once, W_uk's entry by
+// entry, as its rows run along r, 16 lanes to 32 bytes.
+// The library's batched product took 7.7 us there, a step of 64 (four of them) 701 us with it and 685 with this.
+template <int NK, int MT>
+__global__ __launch_bounds__(256) void latent_query_kernel(const bf16* __restrict__ q, int dq, const bf16* __restrict__ uk,
+                                                           bf16* __restrict__ qabs, int T, int H, int R) {
+  const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4, h = blockIdx.y, t0 = 16 * MT * blockIdx.z;
+  const int r0 = 64 * blockIdx.x + 16 * (threadIdx.x >> 6);   // (R is a multiple of 64)
+  const bf16* w = uk + (int64_t)(h * 32 * NK + 8 * g) * R + r0 + li;
+  bf16 wr[NK][8];
+  uint4 x[MT][NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wr[k][e] = w[(int64_t)(32 * k + e) * R];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+      x[m][k] = xgk::ld16(q + ((int64_t)min(t0 + 16 * m + li, T - 1) * H + h) * dq + 32 * k + 8 * g);
+  bf16x8_t wf[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wf[k][e] = (short)wr[k][e];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < NK; ++k) acc = mfma16x16x32(wf[k], as_frag(x[m][k]), acc);
+    const int t = t0 + 16 * m + li;   // lane: columns 4 g .. of token li
+    if (t < T) *reinterpret_cast<uint2*>(qabs + ((int64_t)h * T + t) * R + r0 + 4 * g) =
+        make_uint2(xgk::pack2(acc[0], acc[1]), xgk::pack2(acc[2], acc[3]));
+  }
+}
 
 struct LatentDecodeArgs {
   const bf16 *qabs, *q, *cache;
@@ -300,5 +339,21 @@ int latent_decode(const void* qabs, const void* q, int dq, int dn, const void* g
 #undef XGM_LD
 #undef XGM_LO
   return -1;
+}
+
+// q: [T, H, dq] rows whose first dn entries are the unrotated ones. Returns -1 for sizes or alignments outside this contract.
+int latent_query(const void* q, int dq, int dn, const void* uk, void* qabs, int T, int H, int R, hipStream_t st) {
+  if (T < 1 || H < 1 || H > 65535 || dq < dn || dq % 8 || (dn != 32 && dn != 64 && dn != 128) || R < 64 || R % 64 || T > 65535 ||
+      ((uintptr_t)q & 15) || ((uintptr_t)uk & 1) || ((uintptr_t)qabs & 7))
+    return -1;
+  const int mt = T <= 16 ? 1 : T <= 32 ? 2 : 4;
+  const dim3 grid(R / 64, H, (T + 16 * mt - 1) / (16 * mt));
+#define XGM_LQ(NK, MT) latent_query_kernel<NK, MT><<<grid, 256, 0, st>>>((const bf16*)q, dq, (const bf16*)uk, (bf16*)qabs, T, H, R);
+#define XGM_LQM(NK) \
+  if (mt == 1) { XGM_LQ(NK, 1) } else if (mt == 2) { XGM_LQ(NK, 2) } else { XGM_LQ(NK, 4) }
+  if (dn == 32) { XGM_LQM(1) } else if (dn == 64) { XGM_LQM(2) } else { XGM_LQM(4) }
+#undef XGM_LQM
+#undef XGM_LQ
+  return 0;
 }
 }  // namespace xgm

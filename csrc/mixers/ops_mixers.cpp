@@ -56,6 +56,7 @@ int gated_linear_scan(const float*, const float*, const float*, const void*, int
                       const void*, bool, int64_t, float*, const int32_t*, const int32_t*, const int32_t*, float*, int, int,
                       int, int, int, float*, int, int, const float*, const float*, hipStream_t);
 int64_t gated_linear_scan_scratch_floats(int, int, int, int, int);
+int latent_query(const void*, int, int, const void*, void*, int, int, int, hipStream_t);
 int latent_decode(const void*, const void*, int, int, const void*, int64_t, const void*, const int32_t*, int, int, const int32_t*,
                   const int32_t*, const int32_t*, const int32_t*, const float*, int, const void*, void*, int, int, int, int, int, float, int,
                   float*, float*, hipStream_t);
@@ -350,10 +351,15 @@ PYBIND11_MODULE(_mixers, m) {
   });
   m.def("gated_linear_scan_scratch_floats",
         [](int T, int ns, int H, int dk, int dv) { return xgm::gated_linear_scan_scratch_floats(T, ns, H, dk, dv); });
+  m.def("latent_query", [](uintptr_t q, int dq, int dn, uintptr_t uk, uintptr_t qabs, int T, int H, int R, uintptr_t st) {
+    check(xgm::latent_query(P<const void>(q), dq, dn, P<const void>(uk), P<void>(qabs), T, H, R, S(st)), "latent_query");
+  });
   m.def("latent_decode", [](uintptr_t qabs, uintptr_t q, int dq, int dn, uintptr_t gate, int64_t gate_stride, uintptr_t cache,
                             uintptr_t bt, int bt_width, int bs, uintptr_t qsl, uintptr_t seq_lens, uintptr_t slots,
                             uintptr_t token_seq, uintptr_t rot, int rot_dims, uintptr_t uv, uintptr_t out, int T, int H, int R, int dv, int window,
-                            float scale, int shares, uintptr_t part_o, uintptr_t part_ml, uintptr_t st) {
+                            float scale, int shares, uintptr_t part_o, uintptr_t part_ml, uintptr_t uk, uintptr_t st) {
+    // uk: the queries in latent space are formed first (into qabs), 0: they are there
+    if (uk) check(xgm::latent_query(P<const void>(q), dq, dn, P<const void>(uk), P<void>(qabs), T, H, R, S(st)), "latent_query");
     check(xgm::latent_decode(P<const void>(qabs), P<const void>(q), dq, dn, P<const void>(gate), gate_stride,
                              P<const void>(cache), P<const int32_t>(bt), bt_width, bs, P<const int32_t>(qsl),
                              P<const int32_t>(seq_lens), P<const int32_t>(slots), P<const int32_t>(token_seq),

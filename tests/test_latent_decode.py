@@ -112,3 +112,21 @@ def test_sequences_without_a_token():
     assert sq._latent_shares(q, uv, R, rd, dv, window, bs, sm, cache) > 0
     got = sq.latent_attention_heads(q, dn, gate, cache, uk, uv, rot, rd, window, 0.1, bs, sm)
     assert torch.equal(got[:3], want) and not bool(got[3].any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dn,rd,R", [(32, 32, 64), (64, 32, 256), (128, 64, 512)])
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 64, 65, 130])
+def test_queries_in_latent_space(dn, rd, R, T):
+    """latent_query: q[t, h, :dn] . uk[h], fp32 sums of dn products (dn 2^-24 of their sizes) rounded once to bf16 (2^-8)."""
+    from xgserve.ops._native import mixers, stream_ptr
+    g, H = torch.Generator().manual_seed(T + R), 5
+    q, uk = torch.randn(T, H, dn + rd, generator=g).bfloat16(), (torch.randn(H, dn, R, generator=g) / dn ** 0.5).bfloat16()
+    qd, ud, out = q.cuda(), uk.cuda(), torch.full((H, T, R), 7.0, dtype=torch.bfloat16, device="cuda")
+    mixers().latent_query(qd.data_ptr(), dn + rd, dn, ud.data_ptr(), out.data_ptr(), T, H, R, stream_ptr())
+    a = q[:, :, :dn].double().transpose(0, 1)
+    want, size = a @ uk.double(), a.abs() @ uk.double().abs()
+    assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + dn * 2.0 ** -24 * size).all())
+    for bad in ((dn, rd, R + 32), (dn + 8, rd, R)):
+        with pytest.raises(ValueError):
+            mixers().latent_query(qd.data_ptr(), sum(bad[:2]), bad[0], ud.data_ptr(), out.data_ptr(), T, H, bad[2], stream_ptr())

@@ -684,8 +684,13 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
                                   sm.qsl.data_ptr(), sm.seq_lens.data_ptr(), sm.slots.data_ptr(), out.data_ptr(), T,
                                   sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
         return out
-    qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
     shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm, cache)
+    fold = (shares and dn in (32, 64, 128) and dq % 8 == 0 and q.is_contiguous() and uk.is_contiguous() and uk.dtype == q.dtype
+            and uk.shape[0] == H * dn and q.data_ptr() % 16 == 0 and uk.device == q.device)   # (latent_query, behind the same call)
+    if fold:
+        qabs = torch.empty(H, T, R, dtype=q.dtype, device=q.device)
+    else:
+        qabs = torch.bmm(q[:, :, :dn].transpose(0, 1), uk.view(H, dn, R))   # [H, T, R]
     if shares:
         assert q.is_contiguous() and cache.is_contiguous() and gate.stride(1) == 1 and cache.shape[-1] == R + dq - dn
         assert cache.dtype == gate.dtype == uv.dtype == q.dtype and uv.is_contiguous()
@@ -696,7 +701,7 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
                                bt.data_ptr(), bt.shape[1], block_size, _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
                                _i32(sm.slots).data_ptr(), _i32(sm.token_seq).data_ptr(), rot.data_ptr(), rot_dims,
                                uv.data_ptr(), out.data_ptr(), T, H, R, dv, int(window), float(scale), shares, part.data_ptr(),
-                               part.data_ptr() + 4 * shares * H * T * R, stream_ptr())
+                               part.data_ptr() + 4 * shares * H * T * R, uk.data_ptr() if fold else 0, stream_ptr())
         return out
     o_lat = latent_attention(qabs, q, dn, gate, cache, rot, rot_dims, window, scale, block_size, sm)
     return heads_to_rows(torch.bmm(o_lat, uv.view(H, dv, R).transpose(1, 2)))   # [H, T, dv] -> rows
