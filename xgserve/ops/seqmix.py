@@ -425,23 +425,38 @@ def norm_conv(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float, bia
 # ---------------------------------------------------------------------------- ... and of prompt rows
 def _conv_rows(x: torch.Tensor, y1, y2, a1, a2, bias, w: torch.Tensor, conv: Optional[tuple], sm: SeqMeta, dtype: torch.dtype) -> bool:
     """Whether norm_conv.hip takes these rows: bf16 activations and results, up to 4096 columns, and not the single tokens of a step in
-    parts, which row_update takes."""
+    parts, which row_update takes. (Plain statements: small eager steps wait for the host.)"""
     if sm.parts or conv is None or dtype != torch.bfloat16 or not native_device(x):
         return False
-    (T, W), (cw, state) = x.shape, conv
-    return (T >= 1 and W % 4 == 0 and W <= 4096 and isinstance(y1, torch.Tensor) and (y2 is None or isinstance(y2, torch.Tensor))
-            and all(y is None or (y.dtype == torch.bfloat16 and y.shape == x.shape and y.stride(0) >= W) for y in (y1, y2))
-            and _rows_aligned(y1, y2, x, a1, a2, bias, w, cw, state) and all(
-                t is None or (t.dtype == torch.float32 and t.is_contiguous()) for t in (x, a1, a2, bias, w, cw, state))
-            and cw.shape[0] == W and 2 <= cw.shape[1] <= 4 and state.shape[1:] == (cw.shape[1] - 1, W) and sm.num_seqs < 65535)
+    shape, (cw, state) = x.shape, conv
+    W, taps = shape[1], cw.shape[1]
+    if W % 4 or W > 4096 or shape[0] < 1 or taps < 2 or taps > 4 or cw.shape[0] != W or sm.num_seqs > 65534:
+        return False
+    if state.shape[1] != taps - 1 or state.shape[2] != W:
+        return False
+    at = 0
+    for t in (x, w, cw, state, a1, a2, bias):
+        if t is not None:
+            if t.dtype != torch.float32 or not t.is_contiguous():
+                return False
+            at |= t.data_ptr()
+    for y in (y1,) if y2 is None else (y1, y2):
+        if not isinstance(y, torch.Tensor) or y.dtype != torch.bfloat16 or y.shape != shape:
+            return False
+        ld, one = y.stride()
+        if one != 1 or ld % 4 or ld < W:
+            return False
+        at |= 2 * y.data_ptr()   # (8 bytes)
+    return at % 16 == 0
 
 
 def _norm_conv(x, y1, y2, a1, a2, bias, alpha, w, off, eps, keep_norm, want_f32, want_act, conv, sm):
     T, W = x.shape
     cw, state = conv
-    out, h = torch.empty_like(x), torch.empty(T, W, dtype=torch.bfloat16, device=x.device)
-    n32 = torch.empty_like(x) if want_f32 else None
-    nact = torch.empty_like(h) if want_act else None
+    dev = x.device
+    out, h = torch.empty(T, W, dtype=torch.float32, device=dev), torch.empty(T, W, dtype=torch.bfloat16, device=dev)
+    n32 = torch.empty(T, W, dtype=torch.float32, device=dev) if want_f32 else None
+    nact = torch.empty(T, W, dtype=torch.bfloat16, device=dev) if want_act else None
     mixers().norm_conv(x.data_ptr(), y1.data_ptr(), y1.stride(0), _p(y2), y2.stride(0) if y2 is not None else 0, _p(a1), _p(a2),
                        _p(bias), float(alpha), w.data_ptr(), float(off), float(eps), keep_norm, out.data_ptr(), _p(n32), _p(nact),
                        cw.data_ptr(), cw.shape[1], state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
