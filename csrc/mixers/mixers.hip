@@ -126,7 +126,8 @@ __global__ void canon_conv_kernel(const TI* __restrict__ x, int64_t ld_in, const
 // inputs, also writes them back (the last rows are a second read of a few cache lines), so no launch follows.
 // Memory-bound (with silu its arithmetic); against the kernel above without its second launch (5 us), us: 8192 x 2048
 // fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 14.8
-// against 49.0 (23.6 with the general exponential and division), 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us without silu and loses 5 with it.
+// against 49.0 (23.6 with the general exponential and division), 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us
+// without silu and loses 5 with it.
 template <typename TI, typename TO, int TAPS, int TT>
 __global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, int64_t ld_in, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ state,
@@ -356,8 +357,8 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
 }
 
 // The same in quads (Rq, R, rd and the offsets whole ones, aligned rows; Rq + R up to 1024 NV): a row is loaded once, the query latent's
-// and the key/value latent's statistics meet in one exchange. us, entry by entry and
-// read twice / now: 8192 rows of 768 + 256 23.9 / 12.1, of 1536 + 512 33.7 / 16.7.
+// and the key/value latent's statistics meet in one exchange. us, entry by entry and read twice / now: 8192 rows of 768 + 256
+// 23.9 / 12.1, of 1536 + 512 33.7 / 16.7.
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void latent_prep4_kernel(const T* __restrict__ proj, int64_t ld, int off_q, int Rq, int off_kv, int R,
                                                            int rd, const float* __restrict__ wq, const float* __restrict__ wkv,
