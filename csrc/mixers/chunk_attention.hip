@@ -622,7 +622,7 @@ __global__ __launch_bounds__(256) void talk_mix_rows_kernel(const T* __restrict_
   for (int j = 0; j < REP; ++j) {
     const int h = c * REP + j;
     if (gate) {
-      const float sg = sigmoid_for<T>(ldf(gate + (int64_t)t * ld_gate + h));
+      const float sg = sigmoidf(ldf(gate + (int64_t)t * ld_gate + h));
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[j][i] *= sg;
     }

@@ -125,9 +125,8 @@ __global__ void canon_conv_kernel(const TI* __restrict__ x, int64_t ld_in, const
 // TT + TAPS - 1 rows in flight before it uses the first. The first tile of a sequence, the only one that reads the carried
 // inputs, also writes them back (the last rows are a second read of a few cache lines), so no launch follows.
 // Memory-bound (with silu its arithmetic); against the kernel above without its second launch (5 us), us: 8192 x 2048
-// fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 14.8
-// against 49.0 (23.6 with the general exponential and division), 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us
-// without silu and loses 5 with it.
+// fp32 -> bf16 22.5 against 32.9 (4.5 TB/s), 2521 x 2048 in four sequences 10.2 against 27.0, 2521 x 6144 bf16 with silu 23.0
+// against 49.0, 4001 x 3072 bf16 -> fp32 14.7 against 46.1. TT = 16 gains 1 us without silu and loses 5 with it.
 template <typename TI, typename TO, int TAPS, int TT>
 __global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, int64_t ld_in, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ state,
@@ -202,7 +201,7 @@ __global__ __launch_bounds__(256) void conv4_kernel(const TI* __restrict__ x, in
       o[e] = (residual ? v[t + NH][e] : 0.f) + bf[e];
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) o[e] += wf[TAPS * e + j] * v[t + j][e];
-      if (act) o[e] = silu_for<TO>(o[e]);
+      if (act) o[e] = siluf(o[e]);
     }
     if (t0 + t < q) st4(out + (int64_t)(q0 + t0 + t) * W + c, o);   // (no early exit: the loop has to unroll)
   }
@@ -970,8 +969,8 @@ __global__ void delta_out_kernel(const float* __restrict__ o, const float* __res
 }
 
 // D = 4 L with L a power of two: four entries per lane, 64 / L heads per wave, `nb` workgroups a row. us, with a wave per
-// head / with sums through LDS, a 64-bit division a thread and the general sigmoid, which the vector units bound / now, by memory (6 TB/s):
-// 8192 x 32 x 64 73.6 / 28.9 / 22.4, 2599 x 64 x 64 - / 18.9 / 14.0.
+// head / with sums through LDS and a 64-bit division a thread / now, bound by the sigmoid's exponential and division: 8192 x 32 x 64
+// 73.6 / 35.5 / 32.0, 2599 x 64 x 64 - / 23.4 / 20.4.
 template <typename T>
 __global__ __launch_bounds__(256) void delta_out4_kernel(const float* __restrict__ o, const float* __restrict__ nw,
                                                          const T* __restrict__ gate, int64_t gate_stride, float eps,
@@ -988,7 +987,7 @@ __global__ __launch_bounds__(256) void delta_out4_kernel(const float* __restrict
   const float r = 1.f / sqrtf(ss / (float)(4 * L) + eps);
   gr.get(g);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * sigmoid_for<T>(g[e]);
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * sigmoidf(g[e]);
   st4(out + t * HD + c, v);
 }
 

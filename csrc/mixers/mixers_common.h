@@ -139,21 +139,6 @@ __device__ __forceinline__ float relu2f(float z) {
   return r * r;
 }
 __device__ __forceinline__ float siluf(float x) { return x / (1.f + expf(-x)); }
-
-// The same, and the sigmoid, behind which the result is rounded to T. For bf16 (2^-9) by the exponential and reciprocal instructions, 5
-// instructions instead of 25 (off by 2^-23 of it and |x| 2^-24, of what expf and a division give): launches that a full chip's vector
-// work bounds. Error of the bf16 result against fp64 over x of spread 0.3 to 3: the same to five digits.
-template <typename T>
-__device__ __forceinline__ float sigmoid_for(float x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if (sizeof(T) == 2) return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * x));
-#endif
-  return sigmoidf(x);
-}
-template <typename T>
-__device__ __forceinline__ float silu_for(float x) {
-  return sizeof(T) == 2 ? x * sigmoid_for<T>(x) : siluf(x);
-}
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 }  // namespace xgm

@@ -157,9 +157,9 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 }
 
 // Groups of 4 K L values (L lanes, a power of two): K quads per lane stay in registers between the statistic and the
-// result, 64 / L groups per wave. Memory-bound, us: 2521 x 4096 in 8 groups 13.4 against 47.7 a
-// workgroup per group that reads it twice (18.0 with 64-bit divisions a thread, remainders and the general gate), 4001 x 16 x 128 13.4
-// against 34.8.
+// result, 64 / L groups per wave. us: 2521 x 4096 in 8 groups, bound by the gate's exponential and
+// division, 18.3 against 47.7 a workgroup per group that reads it twice (23.2 with 64-bit divisions a thread and remainders), without a
+// gate 4001 x 16 x 128 13.4 against 34.8.
 template <typename T, int K>
 __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __restrict__ y, const T* __restrict__ z,
                                                                 int64_t ld_z, const float* __restrict__ w, int wn, float eps,
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __r
     if (z) zr[k].get(zs[k]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      zs[k][e] = z ? silu_for<T>(zs[k][e]) : 1.f;
+      zs[k][e] = z ? siluf(zs[k][e]) : 1.f;
       if (!gate_after) v[k][e] *= zs[k][e];
       ss += v[k][e] * v[k][e];
     }

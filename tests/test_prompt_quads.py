@@ -87,3 +87,31 @@ def test_gates_behind_which_bf16_follows():
     want = torch.sigmoid(x.double())
     rounded = torch.sigmoid(x.double()).float().bfloat16().double()
     assert (got - want).norm() <= 1.0001 * (rounded - want).norm()
+
+
+@pytest.mark.parametrize("T", [3, 300])
+def test_bf16_results_are_those_of_fp32_rounded(T):
+    """The same arithmetic in fp32 for either type of the rows, gates (spread 3) too: a bf16 result is the fp32 one, rounded once."""
+    g = torch.Generator().manual_seed(T)
+
+    def rows(n):
+        return (3 * torch.randn(T, n, generator=g)).bfloat16().cuda()
+
+    def weights(*s):
+        return torch.randn(*s, generator=g).cuda()
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    one, n = i32(0), 2048
+    sm = sq.SeqMeta(1, T, i32(0, T), i32(T), one, one, one, one, one)
+    x, y, cw, cb = rows(n), weights(T, n), weights(n, 4), weights(n)
+    o, talk, gate = rows(16 * 2 * 64), weights(16, 16), rows(16)
+
+    def results(dt):
+        state = torch.zeros(1, 3, n, device="cuda")
+        yield sq.causal_conv(x, cw, cb, state, sm, dt, silu=True)
+        yield sq.delta_rule_out(y, cb, x.to(dt), 1e-5, n // 64, 64, dt)
+        yield sq.gated_group_norm(y, x.to(dt), cb, 1e-5, 8, dt)
+        yield sq.gated_group_norm(y, x.to(dt), cb[:128], 1e-5, n // 128, dt, gate_after=True)
+        yield sq.talk_mix(o.to(dt), talk, 16, 2, 64, gate=gate.to(dt))
+    for got, want in zip(results(torch.bfloat16), results(torch.float32)):
+        assert got.dtype == torch.bfloat16 and want.dtype == torch.float32
+        assert torch.equal(got, want.bfloat16())
