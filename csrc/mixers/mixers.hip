@@ -355,9 +355,10 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
   for (int i = rot_dims + threadIdx.x; i < rd; i += blockDim.x) stf(dst + R + i, ldf(kr + i));
 }
 
-// The same in quads (Rq, R, rd and the offsets whole ones, aligned rows; Rq + R up to 1024 NV): a row is loaded once, the query latent's
-// and the key/value latent's statistics meet in one exchange. us, entry by entry and read twice / now: 8192 rows of 768 + 256
-// 23.9 / 12.1, of 1536 + 512 33.7 / 16.7.
+// The same in quads (Rq, R and the offsets whole ones, aligned rows; Rq + R up to 1024 NV): a row is loaded once, and the query latent's
+// and the key/value latent's statistics meet in one exchange. The entries pass through LDS, where a thread takes every 256th as above: the
+// sums are the same bits. us, entry by entry and read twice / now (in brackets with sums over quads): 8192 rows of 768 + 256 24.0 / 14.7
+// (12.6), of 1536 + 512 41.6 / 21.9 (20.0); 64 rows 4.8 / 3.7 and 5.6 / 4.2.
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void latent_prep4_kernel(const T* __restrict__ proj, int64_t ld, int off_q, int Rq, int off_kv, int R,
                                                            int rd, const float* __restrict__ wq, const float* __restrict__ wkv,
@@ -365,6 +366,7 @@ __global__ __launch_bounds__(256) void latent_prep4_kernel(const T* __restrict__
                                                            const int32_t* __restrict__ slot_mapping, const float* __restrict__ rot,
                                                            int rot_dims, T* __restrict__ cq, T* __restrict__ cache) {
   __shared__ float red[8];
+  __shared__ __attribute__((aligned(16))) T held[1024 * NV];   // [query latent | key/value latent]
   const int t = blockIdx.x, all = Rq + (off_kv < 0 ? 0 : R), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const T* row = proj + (int64_t)t * ld;
   const int slot = off_kv < 0 ? -1 : slot_mapping[t];
@@ -388,15 +390,25 @@ __global__ __launch_bounds__(256) void latent_prep4_kernel(const T* __restrict__
     }
     for (int i = rot_dims + threadIdx.x; i < rd; i += 256) stf(dst + i, ldf(kr + i));
   }
-  float v[NV][4], sq = 0.f, sk = 0.f;
+  float v[NV][4];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int c = 4 * (threadIdx.x + 256 * j);
     if (c >= all) continue;
     raw[j].get(v[j]);
-    const float ss = v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
-    if (c < Rq) sq += ss;
-    else sk += ss;
+    st4(held + c, v[j]);
+  }
+  __syncthreads();
+  float sq = 0.f, sk = 0.f;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < Rq; i += 256) {
+    const float e = ldf(held + i);
+    sq += e * e;
+  }
+#pragma unroll 2
+  for (int i = Rq + threadIdx.x; i < all; i += 256) {
+    const float e = ldf(held + i);
+    sk += e * e;
   }
   sq = wave_sum(sq), sk = wave_sum(sk);
   if (lane == 0) red[wave] = sq, red[4 + wave] = sk;

@@ -50,6 +50,26 @@ def test_latent_rows(Rq, R, rd, rot_dims, off, dt):
         close(cache, held, R / 2 + 8, 9.0)
 
 
+@pytest.mark.parametrize("Rq,R", [(768, 256), (1536, 512), (1024, 512), (100, 12), (4, 4), (1028, 1020), (1000, 28), (2048, 2048), (512, 1536)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_latent_rows_sum_in_one_order(Rq, R, dt):
+    """Rows in quads and rows off their alignment, entry by entry, give the same bits."""
+    g, T, rd = torch.Generator().manual_seed(Rq + R), 130, 32
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    one = i32([0])
+    sm = sq.SeqMeta(1, T, i32([0, T]), i32([T]), one, one, one, i32([0] * T), i32(list(range(T))))
+    row = torch.randn(T, Rq + R + rd, generator=g).to(dt)
+    wq, wk, rot = torch.randn(Rq, generator=g).cuda(), torch.randn(R, generator=g).cuda(), sq.build_rot_table(rd, 1e4, 1, "cuda")
+
+    def prep(off):
+        proj = torch.zeros(T, Rq + R + rd + 4, dtype=dt)
+        proj[:, off:off + row.shape[1]] = row
+        cache = torch.zeros(T, R + rd, dtype=dt, device="cuda")
+        return sq.latent_prep(proj.cuda(), off, Rq, off + Rq, R, rd, wq, wk, 1e-5, rot, rd, sm, cache), cache
+    for got, want in zip(prep(0), prep(1)):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("H,G,dv", [(16, 2, 64), (16, 2, 128), (8, 4, 32), (8, 2, 4), (4, 4, 64), (6, 2, 64), (16, 2, 48), (8, 1, 1024)])
 @pytest.mark.parametrize("T", [256, 257, 300])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
