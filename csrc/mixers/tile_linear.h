@@ -55,16 +55,10 @@ enum { kPairNone = 0, kPairHalves = 1, kPairBlocks = 2 };               // w's r
 // gain more from reading its rows together. us without / with: 128 x 28672 x 4096 57 / 50, 128 x 18560 x 4096 50 / 46, 192 x 4096 x 8192 31 /
 // 29, 400 x 18560 x 4096 73 / 77, 1024 x 2048 x 8192 45 / 80; both products of 8 experts of 2 x 3584 x 4096 with 75 rows each 176 / 152,
 // with 250 290 / 270.
+// All row tiles take K in the same order, so that a row's result does not depend on where it is in the step. (With up to eight of them in
+// orders of their own, each fetching a share of the weight that the others find in L2, a Llama prompt of 512 takes 2042 us instead of
+// 2162, and equal rows differ by a rounding.)
 constexpr int kRotateRows = 256;
-// A CU has some 100 requests under way, and what it gets is what their latency leaves: 130 bytes a ns from L2, 60 from the Infinity
-// Cache. Row tiles on the same columns would all ask for the same rows of w at the same time and each wait for memory; so number r of
-// them takes K tiles in the order t ^ r within groups of four (of two where there are two): each fetches a share and finds the others' in
-// L2. For tiles whose loads take longer than their products, up to eight row tiles, weights beyond 24 MB (smaller ones come soon enough
-// and lose by it: 275 x 4096 x 2048, gated, on 128 x 64 12.2 / 12.7). us, without / with: 512 x 6144 x 4096 on 128 x 128
-// 38.5 / 31.3, 512 x 4096 x 4096 on 128 x 64 27.7 / 24.1, 1024 x 2048 x 8192 on 128 x 128 65.4 / 52.9, 1500 x 8192 x 2048 on 192 x 192
-// 59.9 / 54.6, 300 x 18560 x 4096 on 160 x 128 84.6 / 71.0 (in groups of four 78); but 130 x 28672 x 4096, gated, on 128 x 128 66.1 / 67.3,
-// and with more row tiles 2521 x 2048 x 8192 on 192 x 128 79.3 / 81.2, 4001 rows on 256 x 128 104.3 / 107.2.
-constexpr int kStaggerTiles = 8, kStaggerArea = 256 * 192, kStaggerWeights = 12 << 20;
 constexpr int kTileColumns = 1 << 22;   // a wave's 128 rows of fp32 results are less than 2^31 bytes
 
 struct TileArgs {
@@ -82,7 +76,6 @@ struct TileArgs {
   int E, top;
   int64_t w_stride;
   bool rotate;             // column tiles start at different K tiles
-  bool stagger;            // row tiles take them in different orders
 };
 
 // LDS DMA of 16 bytes a lane from a uniform base and a lane's byte offset
@@ -205,12 +198,11 @@ __device__ __forceinline__ int tile_opaque(int v) {
 }
 
 // A tile of the result: rows m0 .. hi - 1 (BM of them at most), columns n0 .., part s of K (nk K tiles of 64 from kt_lo on), expert e.
-// K tiles are asked for from number `rot` on and around, in whole groups (up to `whole`) number u ^ off in u's place.
-struct TileAt { int m0, hi, n0, s, kt_lo, nk, rot, whole, off, e; };
+// K tiles are asked for from number `rot` on and around: the same for all row tiles, so that equal rows give equal bits.
+struct TileAt { int m0, hi, n0, s, kt_lo, nk, rot, e; };
 // ... number v of `total` = TN column tiles for every row tile and part: columns of up to 8 row tiles next to each other
 template <int BM, int BN, bool GRP>
 __device__ __forceinline__ TileAt tile_at(const TileArgs& a, int TN, int v) {
-  constexpr bool STAGGER = !GRP && BM * BN < kStaggerArea;
   TileAt t;
   int TM = (a.M + BM - 1) / BM, u = v, lo = 0;
   t.hi = a.M, t.s = t.e = 0;
@@ -230,8 +222,6 @@ __device__ __forceinline__ TileAt tile_at(const TileArgs& a, int TN, int v) {
   t.kt_lo = t.s * nk_all / a.S;
   t.nk = (t.s + 1) * nk_all / a.S - t.kt_lo;
   t.rot = a.rotate ? (unsigned)tn * 37u % (unsigned)t.nk : 0;
-  const int others = !STAGGER || !a.stagger || TM < 2 || TM > kStaggerTiles ? 0 : TM < 3 ? 1 : 3;
-  t.whole = t.nk & ~others, t.off = (ug - tn * gm) & others;
   return t;
 }
 // the block's place among nb neighbours in that order: neighbours on one XCD
@@ -360,25 +350,19 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
   }
   TileAt ld, cur;      // the tile that is loaded, and the one whose products run
   uint32_t ao[FM], wo[FN], kx, kw;   // what this lane asks for; place in a row
-  uint32_t ux, uw;     // ... counted (128 bytes a K tile)
   const char *xb, *wb;
   int done = 0;
-  auto k_of = [&](uint32_t u) __attribute__((always_inline)) { return u ^ (u < (uint32_t)ld.whole ? ld.off : 0); };
   auto place = [&]() __attribute__((always_inline)) {   // the block's next tile
     ld = tile_at<BM, BN, GRP>(a, TN, done + tile_order(min((int)gridDim.x, total - done)));
     tile_offsets<FM, FN, PAIR, GRP>(a, ld, wv, lane, ao, wo);
     xb = tile_one(reinterpret_cast<const char*>(a.x + (GRP ? 0 : (int64_t)ld.m0 * a.ld_x) + ld.kt_lo * 64));
     wb = tile_one(reinterpret_cast<const char*>(a.w + (GRP ? ld.e * a.w_stride : 0) + ld.kt_lo * 64));
     ld.m0 = tile_one(ld.m0), ld.hi = tile_one(ld.hi), ld.n0 = tile_one(ld.n0), ld.s = tile_one(ld.s), ld.nk = tile_one(ld.nk);
-    ld.whole = tile_one(ld.whole) * 128, ld.off = tile_one(ld.off) * 128;
-    ux = uw = tile_one(ld.rot) * 128u, kx = kw = k_of(ux);
+    kx = kw = tile_one(ld.rot) * 128u;
   };
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t) reinterpret_cast<uintptr_t>((xgk::lds_void_t*)lds));
   const uint32_t lds_a = lds0 + wv * FM * 1024, lds_w = lds0 + RA * ASZ + wv * FN * 1024;
-  auto next = [&](uint32_t& k, uint32_t& u) __attribute__((always_inline)) {
-    u = u + 128 == (uint32_t)ld.nk * 128 ? 0 : u + 128;
-    k = k_of(u);
-  };
+  auto next = [&](uint32_t& k) __attribute__((always_inline)) { k = k + 128 == (uint32_t)ld.nk * 128 ? 0 : k + 128; };
 
   // ---- fragment reads: x row 16 i + l16, W row 32 (i / 2) + 8 (l16 / 4) + l16 % 4 + 4 (i % 2); K half ks
   const uint8_t* ap = lds + (wm * 16 * FM + l16) * 128;
@@ -458,7 +442,7 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
         TileAcc<m * FN + n>::mul(wf[KS][n], af[KS][m]);
       }
       if (q % RS == 0 && q / RS < LD) read(q / RS, KS ^ 1, ra, rw);
-      if (MODE != kLast && q == FM * FN - 2) KS ? next(kx, ux) : next(kw, uw);
+      if (MODE != kLast && q == FM * FN - 2) KS ? next(kx) : next(kw);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -477,12 +461,12 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const TileArgs a) {
     if (t + RA >= 0 && (!SHORT || t + RA < ld.nk)) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) tile_dma(xb + kx, ao[i], lds_a + (t + RA) * ASZ + i * 1024);
-      next(kx, ux);
+      next(kx);
     }
     if (SHORT ? t + RW < ld.nk : t < -1) {
 #pragma unroll
       for (int i = 0; i < FN; ++i) tile_dma(wb + kw, wo[i], lds_w + (t + RW) * WSZ + i * 1024);
-      next(kw, uw);
+      next(kw);
     }
   }
   done += gridDim.x;

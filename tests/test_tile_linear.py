@@ -104,15 +104,20 @@ def test_tiles_one_after_another(tile, K, S, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", [t for t in sorted(tl._TILES) if t[0] * t[1] < 48])
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
 @pytest.mark.parametrize("tiles,S", [(2, 1), (3, 1), (4, 2), (8, 1), (9, 1)])
-def test_row_tiles_that_take_k_in_other_orders(tile, tiles, S):
-    """Weights beyond 24 MB, groups of two and of four K tiles, K tiles left over behind the last group; around, too (up to 256 rows)."""
+def test_equal_rows_give_equal_bits(tile, tiles, S):
+    """Wherever they are in the step: two to nine tiles of rows, weights beyond 24 MB, K tiles that begin at another place (up to 256 rows)."""
     M, N, K = 32 * tile[0] * tiles - 13, 1544, 8192 + 192
     g = torch.Generator("cuda").manual_seed(M)
-    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    few = torch.randn(7, K, generator=g, device="cuda").to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
-    _close(tl.tile_linear((*tile, S), x, w), x.double() @ w.double().t(), K)
+    at = torch.arange(M, device="cuda") % 7
+    y = tl.tile_linear((*tile, S), few[at], w)
+    assert torch.equal(y, y[:7][at])
+    _close(y[-7:], few[at[-7:]].double() @ w.double().t(), K)
+    glu = tl.tile_linear((*tile, S), few[at], w, None, sq.ACT_GLU + sq.GLU_SILU, 0.0, 1.702, tl.PAIR_HALVES)
+    assert torch.equal(glu, glu[:7][at])
 
 
 def test_results_of_2_31_bytes_a_wave_are_refused():
