@@ -22,9 +22,13 @@ import argparse
 import concurrent.futures as cf
 import hashlib
 import os
+import re
+import shutil
+import struct
 import subprocess
 import sys
 import sysconfig
+import tempfile
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -74,6 +78,63 @@ def _write_stamp(out: Path, stamp: str):
 
 # hipcc -O3 forms packed-fp32 instructions from plain float code by itself; they stay off
 NO_PK_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+
+
+# tile_linear.h's kernels keep their accumulators in registers that their statements name, and nothing tells the compiler that these
+# hold something between two statements. What it made is looked at instead: a register of that file may only be written by a product
+# onto itself (or onto zero), and only be read into a vector register; and nothing may be spilled.
+NAMED_ACCUMULATORS = "tile_linear_kernel"
+_PRODUCT = re.compile(r"v_mfma_\w+ (a\[\d+:\d+\]), v\[\d+:\d+\], v\[\d+:\d+\], (a\[\d+:\d+\]|0)$")
+_TAKE = re.compile(r"v_accvgpr_read_b32 v\d+, a\d+$")
+_ACCUMULATOR = re.compile(r"\ba(\[|\d)")
+
+
+def check_accumulators(listing: str) -> int:
+    """The kernels with named accumulators in a disassembly (llvm-objdump -d); raises where one lets the compiler at them."""
+    kernel, count = None, 0
+    for line in listing.splitlines():
+        if line.endswith(">:"):
+            name = line[line.index("<") + 1:-2]
+            kernel = name if NAMED_ACCUMULATORS in name else None
+            count += kernel is not None
+            continue
+        if kernel is None:
+            continue
+        op = line.split("//")[0].strip()
+        if op.startswith("scratch_"):
+            raise RuntimeError(f"{kernel}: spilled registers ({op})")
+        if _ACCUMULATOR.search(op):
+            m = _PRODUCT.match(op)
+            if not (m and m[2] in (m[1], "0")) and not _TAKE.match(op):
+                raise RuntimeError(f"{kernel}: an accumulator that is not the compiler's to use ({op})")
+    return count
+
+
+def _device_code(library: Path):
+    """The library's code objects for ARCH."""
+    data = library.read_bytes()
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        entry = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, entry)
+            if ARCH.encode() in data[entry + 24:entry + 24 + length]:
+                yield data[at + offset:at + offset + size]
+            entry += 24 + length
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+
+
+def check_library_accumulators(library: Path) -> int:
+    """check_accumulators of all kernels of a built library."""
+    objdump = shutil.which("llvm-objdump") or os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm/bin/llvm-objdump")
+    count = 0
+    for code in _device_code(library):
+        if NAMED_ACCUMULATORS.encode() in code:
+            with tempfile.NamedTemporaryFile(suffix=".elf") as f:
+                f.write(code)
+                f.flush()
+                count += check_accumulators(_run([objdump, "-d", f.name]))
+    return count
 
 
 def build_runtime(force: bool = False, jobs: int = 8, extra=()) -> Path:
@@ -157,6 +218,12 @@ def build_mixers(force: bool = False, jobs: int = 8) -> Path:
     tl = _torch_lib()
     _run(["hipcc", "-shared", f"--offload-arch={ARCH}", "-fPIC", *map(str, objs),
           f"-L{tl}", f"-Wl,-rpath,{tl}", "-lamdhip64", "-o", str(out)])
+    try:
+        if check_library_accumulators(out) == 0:
+            raise RuntimeError(f"no {NAMED_ACCUMULATORS} found in {out.name}")
+    except Exception:
+        out.unlink()
+        raise
     _write_stamp(out, stamp)
     return out
 
