@@ -87,8 +87,9 @@ __device__ __forceinline__ void tile_dma(const void* base, uint32_t off, uint32_
 
 // Accumulator I of a wave: accumulation registers 4 I .. 4 I + 3, by name. (As values of the compiler's they are moved between register
 // files inside the loop, some 100 moves per 64 products, and where a branch joins two ways to write them, behind a product that has
-// not written them yet. Every statement names what it writes, so nothing else lives there; with registers to spare, which the build's
-// metadata shows, nothing passes through either.) There are no waits between products: an accumulator is read again by the same
+// not written them yet. Every statement names what it writes, but the compiler does not know that these registers hold something
+// between two statements: the build looks whether it has put anything of its own there, and fails if so, _build.check_accumulators.)
+// There are no waits between products: an accumulator is read again by the same
 // instruction on the same registers, which takes two wait states at most, and kMfmaApart other products lie between at least.
 //   mul, mul_dma, first   acc += w . x^T; the same and an LDS DMA behind it (M0 is written ahead of the product, which is the wait
 //                         state between the two); acc = w . x^T
@@ -554,8 +555,9 @@ static void tile_launch(const TileArgs& a, int cus, hipStream_t st) {
 }
 
 // K (a part of it) of up to RA tiles: the ring does not turn. Up to five tiles then run on 128 x 128 tiles without one, six on 128 x 64 where
-// those were asked for, and what lies on both sides of that (parts that differ by one tile) on the ring of two. The results are the same
-// bits: every size sums K in the same order. us, as it was with a ring that ends with the tile / now: 700 x 2056 x 256 6.9 / 5.8, 300 x 4096 x
+// those were asked for, and what lies on both sides of that (parts that differ by one tile) on the ring of two. Beyond kRotateRows rows the
+// results are the same bits, as every size then sums K in the same order; up to there a column begins where its tile's number says, which
+// goes by the tile's width. us, as it was with a ring that ends with the tile / now: 700 x 2056 x 256 6.9 / 5.8, 300 x 4096 x
 // 384 6.0 / 5.5, 256 x 2048 x 128 11.4 (256 x 256) / 4.6, but 4096 x 4096 x 128 15.4 (256 x 256) / 17.6: no weight is that narrow.
 constexpr int kShortK = 5;
 enum TileForm { kFormRing, kFormShort, kFormShortNarrow, kFormRing2 };

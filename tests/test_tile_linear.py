@@ -120,6 +120,17 @@ def test_equal_rows_give_equal_bits(tile, tiles, S):
     assert torch.equal(glu, glu[:7][at])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 192, 320, 384, 448, 1024])
+def test_sizes_of_tiles_sum_in_the_same_order(K):
+    """More than 256 rows: every size of the tile gives the same bits, K of a few tiles (forms without a ring) and longer."""
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.randn(300, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(1544, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    got = [tl.tile_linear((*tile, 1), x, w) for tile in sorted(tl._TILES)]
+    assert all(torch.equal(y, got[0]) for y in got)
+
+
 def test_results_of_2_31_bytes_a_wave_are_refused():
     from xgserve.ops._native import mixers
     with pytest.raises(ValueError):
