@@ -570,6 +570,9 @@ static TileForm tile_form(int nk_least, int nk_most, int fm, int fn, int ra) {
 // the launch of one size (-1: there is none); gated products are compiled in tile_gated.hip
 // (a round of workgroups costs the same full or nearly empty: sizes between the powers of two are there for the row counts that
 // leave such a round; 160 x 192 and 128 x 192 were the fastest too rarely, by 1 to 6 %)
+// (96 x 64 with rings of four, which two workgroups of a CU just have: w is asked for one step behind x, so that in rings of three it
+// comes late. us, rings that end with the tile and ask for both at once / of three / of four: 400 x 2048 x 2048 12.1 / 12.6 / 11.5, 298 x
+// 4096 x 4096 28.4 / 29.0 / 24.8, 65 x 16384 x 2048 20.2 / 20.2 / 17.7, in four parts 130 x 2048 x 2048 10.1 / 10.5 / 10.5)
 template <bool PAIR>
 static int tile_launch_size(const TileArgs& a, int fm, int fn, int cus, hipStream_t st) {
   const int nk = a.K / 64, least = nk / a.S, most = (nk + a.S - 1) / a.S;
@@ -597,7 +600,7 @@ static int tile_launch_size(const TileArgs& a, int fm, int fn, int cus, hipStrea
   XGM_TILE(4, 4, 5, 5, 1)
   XGM_TILE(3, 4, 5, 5, 1)
   XGM_TILE(4, 2, 6, 6, 1)
-  XGM_TILE(3, 2, 3, 3, 2)
+  XGM_TILE(3, 2, 4, 4, 2)
 #undef XGM_TILE
   return -1;
 }
