@@ -130,3 +130,24 @@ def test_queries_in_latent_space(dn, rd, R, T):
     for bad in ((dn, rd, R + 32), (dn + 8, rd, R)):
         with pytest.raises(ValueError):
             mixers().latent_query(qd.data_ptr(), sum(bad[:2]), bad[0], ud.data_ptr(), out.data_ptr(), T, H, bad[2], stream_ptr())
+
+
+@pytest.mark.parametrize("fold", [True, False])
+def test_queries_on_both_sides_of_the_line(fold, monkeypatch):
+    """By latent_query up to LATENT_QUERY_MACS multiply-adds of a step's queries, by the library beyond."""
+    T, H, dn, R = 9, 32, 64, 256
+    monkeypatch.setattr(sq, "LATENT_QUERY_MACS", T * H * dn * R - (not fold))
+    real, seen = sq.mixers(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(real, name)
+            return lambda *a: (seen.append(a[-2] != 0) if name == "latent_decode" else None, f(*a))[1]
+    monkeypatch.setattr(sq, "mixers", Spy)
+    test_against_fp64(H, dn, 32, 64, R, 32, [20 + 7 * i for i in range(T)], 64, 16, monkeypatch)
+    assert seen == [fold]
+
+
+def test_large_steps_leave_the_queries_to_the_library():
+    for T, H, dn, R, fold in ((64, 32, 64, 256, True), (64, 32, 128, 512, True), (128, 32, 128, 512, False), (256, 64, 64, 512, False)):
+        assert (T * H * dn * R <= sq.LATENT_QUERY_MACS) == fold

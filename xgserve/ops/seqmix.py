@@ -658,6 +658,12 @@ def _latent_expands(q, dn: int, R: int, dv: int, rot_dims: int, window: int, blo
 # / 42, R = 512 82 / 56 / 48 / 65 / 95; one sequence of 4000 keys, R = 512, in 8 / 16 / 32 / 63 shares 48 / 43 / 49 / 65.
 LATENT_DECODE_WGS, LATENT_DECODE_SHARES = 256, 16
 LATENT_PAGES = 2048     # page table entries of a share
+# Up to so many multiply-adds (T H dn R) the queries come into latent space by latent_query, beyond by the library: every 64 tokens read
+# the whole of uk once more. From the queries to the heads' outputs, us, library / kernel, (H, dn, R) at both sides of the line: (32, 64,
+# 256) 256 rows 34.5 / 28.3, 512 43.2 / 43.4; (64, 64, 512) 80 rows 39.7 / 37.2, 160 60.8 / 62.3; (32, 128, 512) 80 rows 38.1 / 35.8, 128
+# 38.8 / 39.4, 512 92.5 / 104.5; (64, 128, 512) 48 rows 37.9 / 36.6, 64 38.0 / 38.7, 512 175 / 204; (16, 128, 256) 256 rows 32.9 / 26.3,
+# 384 37.1 / 37.6; (32, 32, 128) 512 rows, far below it, 33.7 / 28.2.
+LATENT_QUERY_MACS = 200_000_000
 
 
 def _latent_shares(q, uv, R: int, rd: int, dv: int, window: int, block_size: int, sm: SeqMeta, cache=None) -> int:
@@ -700,8 +706,9 @@ def latent_attention_heads(q: torch.Tensor, dn: int, gate: torch.Tensor, cache: 
                                   sm.num_seqs, sm.max_q, H, int(window), float(scale), stream_ptr())
         return out
     shares = _latent_shares(q, uv, R, dq - dn, dv, window, block_size, sm, cache)
-    fold = (shares and dn in (32, 64, 128) and dq % 8 == 0 and q.is_contiguous() and uk.is_contiguous() and uk.dtype == q.dtype
-            and uk.shape[0] == H * dn and q.data_ptr() % 16 == 0 and uk.device == q.device)   # (latent_query, behind the same call)
+    fold = (shares and dn in (32, 64, 128) and T * H * dn * R <= LATENT_QUERY_MACS and dq % 8 == 0 and q.is_contiguous()
+            and uk.is_contiguous() and uk.dtype == q.dtype and uk.shape[0] == H * dn and q.data_ptr() % 16 == 0
+            and uk.device == q.device)   # (latent_query, behind the same call)
     if fold:
         qabs = torch.empty(H, T, R, dtype=q.dtype, device=q.device)
     else:
