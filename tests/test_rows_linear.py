@@ -226,3 +226,9 @@ def test_heads_of_few_rows(M, N, K, native, monkeypatch):
     if M <= 16:
         xr = x.clone().requires_grad_()
         assert lm_head_linear(xr, w).grad_fn is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,native", [(32768, 1024, True), (32772, 1024, False), (50304, 1024, False), (32772, 1536, True)])
+def test_wide_heads_of_short_rows_stay_with_the_library(N, K, native, monkeypatch):
+    test_heads_of_few_rows(2, N, K, native, monkeypatch)

@@ -255,8 +255,11 @@ _MW_TUNED = {
     (128256, 4096, MODE_BF16): {128: (1, 0), 192: (1, 6), 256: (1, 6)},
 }
 # up to 16 rows run on rows_linear: 1 row of 128256 x 4096 155 us against the library's 175 (gemm_mw 154), of 32000 x 4096 43 against 62,
-# of 152064 x 3584 172 against 229; 16 rows 160 / 176, 41 / 58, 173 / 232
+# of 152064 x 3584 172 against 229; 16 rows 160 / 176, 41 / 58, 173 / 232. Rows of fewer than LM_HEAD_ROWS_MIN_K entries in up to
+# LM_HEAD_ROWS_MAX_N columns (16 rows, library / rows_linear: 32000 x 512 12.8 / 9.9, 32000 x 1280 22.4 / 18.1, but 50304 x 1024 23.6 / 25.1,
+# 50304 x 1280 29.3 / 31.2, 262144 x 512 60.6 / 63.4, 262144 x 1024 101 / 108; from 1536 on 50304 34.1 / 33.2, 262144 150 / 145)
 LM_HEAD_MW_MIN_M = 17
+LM_HEAD_ROWS_MIN_K, LM_HEAD_ROWS_MAX_N = 1536, 32768
 
 
 def _mw_bucket(M: int) -> int:
@@ -395,7 +398,7 @@ def lm_head_linear(h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     measured a plan for this row bucket (_MW_TUNED, mode bf16), else hipBLASLt."""
     M, K = h.shape
     N = w.shape[0]
-    if M < LM_HEAD_MW_MIN_M:
+    if M < LM_HEAD_MW_MIN_M and (K >= LM_HEAD_ROWS_MIN_K or N <= LM_HEAD_ROWS_MAX_N):
         from .seqmix import rows_product   # (which builds on this module)
         return rows_product(h, w)
     if (h.is_cuda and LM_HEAD_MW_MIN_M <= M <= MW_MAX_M and h.is_contiguous() and w.is_contiguous()
