@@ -593,8 +593,11 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(const T* __restrict__ o_a
 }
 
 // The same for many rows: a thread has four value columns of one token's key/value head, whose rows it reads once for all REP heads of
-// that key/value head; the weights are the same for the whole workgroup (scalar loads). us, a thread per head and
-// four columns / now: 4001 rows of 16 heads, 2 x 64 columns 19.0 / 11.0, 2 x 128 32.7 / 12.9.
+// that key/value head; the weights are the same for the whole workgroup (scalar loads). Few workgroups, each with H reads one behind the
+// other: the form above is the faster one while its threads have fewer than 32 reads and there are fewer than 2000 rows. us, a thread per
+// head and four columns / this (H heads, G x dv columns): 16, 2 x 64 257 rows 5.0 / 7.1, 1000 6.6 / 7.5, 2000 11.2 / 10.9, 4001 19.3 /
+// 11.9; 8, 2 x 32 1000 rows 4.3 / 4.5, 2800 5.4 / 4.7; 8, 1 x 256 400 rows 5.7 / 6.0, 2000 11.5 / 8.9; 32 reads and more: 16, 2 x 128 257
+// rows 7.5 / 7.2, 4001 32.5 / 14.2; 32, 8 x 64 257 rows 20.9 / 12.6; 32, 8 x 128 257 rows 40.1 / 14.0.
 template <typename T, int REP>
 __global__ __launch_bounds__(256) void talk_mix_rows_kernel(const T* __restrict__ o_all, const float* __restrict__ talk,
                                                             const T* __restrict__ gate, int64_t ld_gate, T* __restrict__ out, int T_,
@@ -1084,8 +1087,8 @@ int talk_mix_parts(const float* part_o, const float* part_ml, const int32_t* slo
 void talk_mix(const void* o_all, bool f32, const float* talk, const void* gate, int64_t ld_gate, void* out, int T_, int H,
               int G, int dv, hipStream_t st) {
   if (T_ <= 0) return;
-  const int rep = H / G, quads = dv / 4;
-  if (T_ > 256 && dv % 4 == 0 && quads <= 256 && (quads & (quads - 1)) == 0 && (rep == 2 || rep == 4 || rep == 8) && G <= 65535 &&
+  const int rep = H / G, quads = dv / 4, reads = H * ((H * quads + 255) / 256);   // (of a thread of the kernel for few rows)
+  if (T_ > (reads >= 32 ? 256 : 1999) && dv % 4 == 0 && quads <= 256 && (quads & (quads - 1)) == 0 && (rep == 2 || rep == 4 || rep == 8) && G <= 65535 &&
       (int64_t)T_ * quads < (1ll << 31)) {
     int sh = 0;
     while (1 << sh < quads) ++sh;

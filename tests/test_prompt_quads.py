@@ -85,6 +85,17 @@ def test_mixed_maps_of_many_rows(H, G, dv, T, dt):
         close(got, ref.reshape(T, -1), H + 12, 30.0)
 
 
+@pytest.mark.parametrize("H,G,dv", [(16, 2, 64), (8, 4, 32), (8, 2, 4), (8, 1, 256), (4, 4, 64)])
+@pytest.mark.parametrize("T", [1999, 2000, 2049])
+def test_mixed_maps_of_few_reads(H, G, dv, T):
+    """Up to 31 reads a thread the kernel of many rows begins at 2000; both give the same bits."""
+    g = torch.Generator().manual_seed(H * dv)
+    o, talk = torch.randn(T, H * G * dv, generator=g).bfloat16().cuda(), torch.randn(H, H, generator=g).cuda()
+    gate = torch.randn(T, H, generator=g).bfloat16().cuda()
+    few = torch.cat([sq.talk_mix(o[i:i + 1000], talk, H, G, dv, gate=gate[i:i + 1000]) for i in range(0, T, 1000)])
+    assert torch.equal(sq.talk_mix(o, talk, H, G, dv, gate=gate), few)
+
+
 @pytest.mark.parametrize("size", [4, 8, 16, 32, 64, 128, 256, 512, 1024])
 @pytest.mark.parametrize("groups", [1, 3, 40])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
