@@ -18,8 +18,10 @@
 // them (one of rows beyond 2048 columns): the weights that a workgroup loads are four rows' bytes. us, KEEP / the other form, two
 // launches before in brackets: 8192 x 2048 in strips of 8 / 12 / 20 / 28 47.8 / 41.6 / 38.3 / 44.9 (53.5) and 63.2 / 58.2 / 54.0 / 60.2
 // (79.6); 2521 x 2048 in 8 / 12 / 16 19.4 / 17.3 / 19.0 (20.5) and 23.8 / 21.6 / 24.3 (26.6); 8192 x 4096 in 36 87 (108) and 116 (170);
-// 2599 x 4096 in 16 27.6 (37.1) and 36.6 (56.0); 512 x 2048 8.6 (10.8) and 10.3 (14.5); 300 x 4096 11.1 (10.9) and 13.2 (14.7); 96 single
-// tokens of 2048 5.1 (10.6) and 5.3 (14.5).
+// 2599 x 4096 in 16 27.6 (37.1) and 36.6 (56.0); 512 x 2048 8.6 (10.8) and 10.3 (14.5); 96 single tokens of 2048 5.6 (7.1) and 6.1 (8.0),
+// 256 of 4096 10.3 (14.2) and 11.1 (16.8). Rows of 4096 up to some 400 (100 10.9 (9.2) and 13.1 (11.3)), and of 2048 up to 200 (100 8.2 (7.7)
+// and 9.6 (8.7)), are slower than in two launches on the card, but not in a step, which the host launches: 65 rows Dofivik 1b 1140 (1149), 8b
+// 763 (762), Vizonex 1b 834 (866), 8b 720 (725), 200 rows 1163 (1182), 950 (949), 923 (934), 940 (948).
 #include "glds.h"
 #include "mixers_common.h"
 
@@ -221,24 +223,24 @@ __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a
   }
 }
 
-// strip: rows of a strip and its TAPS - 1 before, a multiple of 4 (0: the longest that leaves the chip full). Sequences of up to max_q
-// rows; those without a slot and the rows behind the last one are normed and not convolved. Returns -1 for sizes or alignments outside
-// this contract.
+// Strips, with the TAPS - 1 rows before them, of 8 to 36 rows: the shortest that need no more than the workgroups named above, of `cus` CUs.
+// Sequences of up to max_q rows; those without a slot and the rows behind the last one are normed and not convolved. Returns -1 for sizes
+// or alignments outside this contract.
 int norm_conv(const float* x, const void* y1, int64_t ld1, const void* y2, int64_t ld2, const float* a1, const float* a2,
               const float* bias, float alpha, const float* g, float off, float eps, bool keep_norm, float* x_out, float* n32, void* nact,
               const float* cw, int taps, float* state, const int32_t* qsl, const int32_t* seq_lens, const int32_t* slots, void* h,
-              int ns, int max_q, int T_, int W, int strip, hipStream_t st) {
+              int ns, int max_q, int T_, int W, int cus, hipStream_t st) {
   if (T_ <= 0) return 0;
   auto rows_ok = [&](const void* p, int64_t ld) { return ld % 4 == 0 && ld >= W && (uintptr_t)p % 8 == 0; };
   if (W < 4 || W > 4096 || W % 4 || taps < 2 || taps > 4 || ns < 0 || ns > 65534 || max_q < 0 || !y1 || !rows_ok(y1, ld1) ||
       (y2 && !rows_ok(y2, ld2)) || (keep_norm && (y2 || a1 || a2 || n32 || nact)) || (!keep_norm && bias) || !x_out || x_out == x || !h ||
-      strip < 0 || strip % 4 || (strip && strip < 8) || strip > 256 ||
+      cus < 1 ||
       (((uintptr_t)x | (uintptr_t)x_out | (uintptr_t)a1 | (uintptr_t)a2 | (uintptr_t)bias | (uintptr_t)g | (uintptr_t)n32 | (uintptr_t)cw |
         (uintptr_t)state) & 15) || (((uintptr_t)nact | (uintptr_t)h) & 7))
     return -1;
-  const int fill = W <= 2048 ? 512 : 256;
-  if (!strip)
-    for (strip = 8; strip < 36 && (T_ + strip - taps) / (strip + 1 - taps) > (strip == 8 ? 256 : fill); strip += 4) {}
+  const int64_t fill = W <= 2048 ? 2ll * cus : cus;
+  int strip = 8;
+  while (strip < 36 && (T_ + strip - taps) / (strip + 1 - taps) > (strip == 8 ? cus : fill)) strip += 4;
   const int rows = strip - (taps - 1);
   const NormConvArgs a = {x, (const bf16*)y1, (const bf16*)y2, ld1, ld2, a1, a2, bias, g, cw, alpha, off, eps, state,
                           qsl, seq_lens, slots, x_out, n32, (bf16*)nact, (bf16*)h, T_, W, ns, rows};

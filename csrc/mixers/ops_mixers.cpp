@@ -314,11 +314,11 @@ PYBIND11_MODULE(_mixers, m) {
   m.def("norm_conv", [](uintptr_t x, uintptr_t y1, int64_t ld1, uintptr_t y2, int64_t ld2, uintptr_t a1, uintptr_t a2, uintptr_t bias,
                         float alpha, uintptr_t g, float off, float eps, bool keep_norm, uintptr_t x_out, uintptr_t n32, uintptr_t nact,
                         uintptr_t cw, int taps, uintptr_t state, uintptr_t qsl, uintptr_t seq_lens, uintptr_t slots, uintptr_t h, int ns,
-                        int max_q, int T, int W, int strip, uintptr_t st) {
+                        int max_q, int T, int W, int cus, uintptr_t st) {
     check(xgm::norm_conv(P<const float>(x), P<const void>(y1), ld1, P<const void>(y2), ld2, P<const float>(a1), P<const float>(a2),
                          P<const float>(bias), alpha, P<const float>(g), off, eps, keep_norm, P<float>(x_out), P<float>(n32),
                          P<void>(nact), P<const float>(cw), taps, P<float>(state), P<const int32_t>(qsl), P<const int32_t>(seq_lens),
-                         P<const int32_t>(slots), P<void>(h), ns, max_q, T, W, strip, S(st)),
+                         P<const int32_t>(slots), P<void>(h), ns, max_q, T, W, cus, S(st)),
           "norm_conv");
   });
   m.def("relu2", [](uintptr_t in, bool f32, uintptr_t bias, uintptr_t out, int64_t n, int cols, uintptr_t st) {

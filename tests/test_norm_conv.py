@@ -89,6 +89,46 @@ def test_against_fp64(W, taps, lens, behind, monkeypatch):
     assert calls == ["norm_conv"] * 5
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("W", [8, 2052])
+@pytest.mark.parametrize("strip", [8, 12, 20, 36])
+def test_strips(strip, W, taps, monkeypatch):
+    """Strips of every length, which go by the rows and the CUs: sequences that end with one or two of them, a row before and a row behind,
+    at a start, behind carried inputs and behind fewer of those than there are taps."""
+    rows = strip + 1 - taps
+    lens = [n for k in (1, 2) for n in (k * rows - 1, k * rows, k * rows + 1) for _ in range(3)] + [1, 1, 1]
+    T = sum(lens)
+    # workgroups that strips of this length need, and shorter ones exceed (strips of 8 have one workgroup a CU, as all of wide rows have)
+    wgs = -(-T // rows)
+    cus = wgs if strip == 8 or W > 2048 else -(-wgs // 2)
+    assert strip == 8 or -(-T // (rows - 4)) > (cus if strip == 12 or W > 2048 else 2 * cus)
+    monkeypatch.setattr(sq, "cu_count", lambda d: cus)
+    g, n = torch.Generator().manual_seed(strip + taps), len(lens)
+    ctx, slots = [(0, 7, 1)[i % 3] for i in range(n)], [n - 1 - i for i in range(n)]
+    sm, first = meta(lens, ctx, slots)
+    x, w, a1 = torch.randn(T, W, generator=g), torch.randn(W, generator=g), torch.randn(W, generator=g)
+    y = torch.randn(T, W, generator=g).bfloat16()
+    cw, state = torch.randn(W, taps, generator=g), torch.randn(n, taps - 1, W, generator=g)
+    for keep in (True, False):
+        st = state.cuda()
+        if keep:
+            out, h = sq.norm_conv_rows(x.cuda(), y.cuda(), w.cuda(), 1e-5, 0.7, a1.cuda(), (cw.cuda(), st), sm, torch.bfloat16)
+            r = norm(0.7 * x.double() + y.double() + a1.double()) * (1 + w.double())
+            close(out, r, W / 2 + 16, float(r.abs().max()))
+        else:
+            out, _, nact, h = sq.residual_norm_conv_rows(x.cuda(), y.cuda(), a1.cuda(), None, None, None, w.cuda(), 1e-5, torch.bfloat16,
+                                                         (cw.cuda(), st), False, sm)
+            v = x.double() + a1.double() * y.double()
+            r = norm(v) * w.double()
+            close(out, v, 24, float(v.abs().max()) + 30)
+            close(nact, r, W / 2 + 16, float(r.abs().max()))
+        want, live, new = conv(r, cw, state, lens, first, ctx, slots)
+        big = float(r.abs().max())
+        assert bool(live.all())
+        close(h, want, W / 2 + 40, big * 8)
+        close(st, new, W / 2 + 16, max(big, 5.0))
+
+
 def test_others_take_the_separate_kernels(monkeypatch):
     """More than 4096 columns, fp32 rows, a sum over experts, weights off 16 bytes: in place, by the launches they had."""
     calls = record_native(monkeypatch, sq)

@@ -460,7 +460,7 @@ def _norm_conv(x, y1, y2, a1, a2, bias, alpha, w, off, eps, keep_norm, want_f32,
     mixers().norm_conv(x.data_ptr(), y1.data_ptr(), y1.stride(0), _p(y2), y2.stride(0) if y2 is not None else 0, _p(a1), _p(a2),
                        _p(bias), float(alpha), w.data_ptr(), float(off), float(eps), keep_norm, out.data_ptr(), _p(n32), _p(nact),
                        cw.data_ptr(), cw.shape[1], state.data_ptr(), _i32(sm.qsl).data_ptr(), _i32(sm.seq_lens).data_ptr(),
-                       _i32(sm.slots).data_ptr(), h.data_ptr(), sm.num_seqs, sm.max_q, T, W, 0, stream_ptr())
+                       _i32(sm.slots).data_ptr(), h.data_ptr(), sm.num_seqs, sm.max_q, T, W, cu_count(x.device), stream_ptr())
     return out, n32, nact, h
 
 
