@@ -21,7 +21,9 @@
 // 2599 x 4096 in 16 27.6 (37.1) and 36.6 (56.0); 512 x 2048 8.6 (10.8) and 10.3 (14.5); 96 single tokens of 2048 5.6 (7.1) and 6.1 (8.0),
 // 256 of 4096 10.3 (14.2) and 11.1 (16.8). Rows of 4096 up to some 400 (100 10.9 (9.2) and 13.1 (11.3)), and of 2048 up to 200 (100 8.2 (7.7)
 // and 9.6 (8.7)), are slower than in two launches on the card, but not in a step, which the host launches: 65 rows Dofivik 1b 1140 (1149), 8b
-// 763 (762), Vizonex 1b 834 (866), 8b 720 (725), 200 rows 1163 (1182), 950 (949), 923 (934), 940 (948).
+// 763 (762), Vizonex 1b 834 (866), 8b 720 (725), 200 rows 1163 (1182), 950 (949), 923 (934), 940 (948). Rows of up to 1024 columns have one
+// quad a thread (two, half of them idle, in square brackets): 300 x 1024 6.8 [8.2] (7.5) and 7.6 [9.8] (8.4), 1500 10.8 [12.1] (10.7) and
+// 12.1 [15.1] (13.1), 8192 27.5 [29.0] (29.7) and 34.3 [38.8] (49.3).
 #include "glds.h"
 #include "mixers_common.h"
 
@@ -56,10 +58,10 @@ struct StripOut {
   }
 };
 
-// NTHR threads of two quads of columns each: W <= 8 NTHR
-template <bool KEEP, int TAPS, int NTHR>
+// NTHR threads of NV quads of columns each: W <= 4 NV NTHR
+template <bool KEEP, int TAPS, int NTHR, int NV>
 __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a) {
-  constexpr int NH = TAPS - 1, NW = NTHR / 64, ROWS = 2, DEPTH = 2, NV = 2;
+  constexpr int NH = TAPS - 1, NW = NTHR / 64, ROWS = 2, DEPTH = 2;
   constexpr int AGAIN = (NH + ROWS - 1) / ROWS;   // groups of the last rows
   __shared__ float red[2][ROWS][NW];
   const int s = blockIdx.y, W = a.W;
@@ -247,8 +249,9 @@ int norm_conv(const float* x, const void* y1, int64_t ld1, const void* y2, int64
   const int n = max(1, (max_q + rows - 1) / rows);
   const dim3 grid(n < 65535 ? n : 65535, ns + 1);
 #define XGM_NC(KEEP, TAPS)                                                    \
-  if (W <= 2048) norm_conv_kernel<KEEP, TAPS, 256><<<grid, 256, 0, st>>>(a);  \
-  else norm_conv_kernel<KEEP, TAPS, 512><<<grid, 512, 0, st>>>(a);
+  if (W <= 1024) norm_conv_kernel<KEEP, TAPS, 256, 1><<<grid, 256, 0, st>>>(a);       \
+  else if (W <= 2048) norm_conv_kernel<KEEP, TAPS, 256, 2><<<grid, 256, 0, st>>>(a);  \
+  else norm_conv_kernel<KEEP, TAPS, 512, 2><<<grid, 512, 0, st>>>(a);
 #define XGM_NCT(KEEP)                                                                             \
   if (taps == 4) { XGM_NC(KEEP, 4) } else if (taps == 3) { XGM_NC(KEEP, 3) } else { XGM_NC(KEEP, 2) }
   if (keep_norm) { XGM_NCT(true) } else { XGM_NCT(false) }

@@ -90,7 +90,7 @@ def test_against_fp64(W, taps, lens, behind, monkeypatch):
 
 
 @pytest.mark.parametrize("taps", [2, 3, 4])
-@pytest.mark.parametrize("W", [8, 2052])
+@pytest.mark.parametrize("W", [8, 1024, 1028, 2052])
 @pytest.mark.parametrize("strip", [8, 12, 20, 36])
 def test_strips(strip, W, taps, monkeypatch):
     """Strips of every length, which go by the rows and the CUs: sequences that end with one or two of them, a row before and a row behind,
