@@ -986,10 +986,10 @@ __global__ void delta_out_kernel(const float* __restrict__ o, const float* __res
 template <typename T>
 __global__ __launch_bounds__(256) void delta_out4_kernel(const float* __restrict__ o, const float* __restrict__ nw,
                                                          const T* __restrict__ gate, int64_t gate_stride, float eps,
-                                                         T* __restrict__ out, int nb, int HD, int L) {
-  const int64_t t = blockIdx.x / nb;
+                                                         T* __restrict__ out, int T_, int nb, int HD, int L) {
+  const int64_t t = (int64_t)(blockIdx.x / nb) * blockDim.y + threadIdx.y;
   const int c = 4 * ((int)(blockIdx.x % nb) * blockDim.x + threadIdx.x);
-  if (c >= HD) return;   // (whole heads: HD is a multiple of 4 L)
+  if (c >= HD || t >= T_) return;   // (whole heads: HD is a multiple of 4 L)
   float v[4], w[4], g[4];
   Raw4<T> gr;
   gr.load(gate + t * gate_stride + c);
@@ -1306,11 +1306,12 @@ void delta_out(const float* o, const float* nw, const void* gate, bool f32, int6
                int T_, int H, int D, hipStream_t st) {
   if (T_ <= 0) return;
   const int esz = f32 ? 4 : 2, L = D / 4;
-  const int nb = (H * L + 255) / 256, nth = nb > 1 ? 256 : (H * L + 63) / 64 * 64;
+  const int nb = (H * L + 255) / 256;
+  const dim3 block = row_block(H * L);
   if (D % 4 == 0 && L >= 1 && L <= 64 && (L & (L - 1)) == 0 && gate_stride % 4 == 0 && (int64_t)T_ * nb < (1ll << 31) &&
       (uintptr_t)gate % (4 * esz) == 0 && (((uintptr_t)o | (uintptr_t)nw | (uintptr_t)out) & 15) == 0) {
-    XGM_DISPATCH_T(f32, delta_out4_kernel<T><<<(unsigned)T_ * nb, nth, 0, st>>>(o, nw, (const T*)gate, gate_stride, eps, (T*)out, nb,
-                                                                               H * D, L);)
+    XGM_DISPATCH_T(f32, delta_out4_kernel<T><<<(unsigned)((T_ + block.y - 1) / block.y) * nb, block, 0, st>>>(
+        o, nw, (const T*)gate, gate_stride, eps, (T*)out, T_, nb, H * D, L);)
     return;
   }
   XGM_DISPATCH_T(f32, delta_out_kernel<T><<<dim3(T_, (H + 3) / 4), 256, 0, st>>>(o, nw, (const T*)gate, gate_stride, eps, (T*)out, H, D);)

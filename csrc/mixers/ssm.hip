@@ -163,11 +163,11 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 template <typename T, int K>
 __global__ __launch_bounds__(256) void gated_group_norm4_kernel(const float* __restrict__ y, const T* __restrict__ z,
                                                                 int64_t ld_z, const float* __restrict__ w, int wn, float eps,
-                                                                T* __restrict__ out, int inner, int nb, int sh, int gate_after) {
-  // `nb` workgroups a row; a group is 2^sh lanes
-  const int64_t t = blockIdx.x / nb;
+                                                                T* __restrict__ out, int T_, int inner, int nb, int sh, int gate_after) {
+  // `nb` workgroups a row, or blockDim.y rows a workgroup; a group is 2^sh lanes
+  const int64_t t = (int64_t)(blockIdx.x / nb) * blockDim.y + threadIdx.y;
   const int i = (int)(blockIdx.x % nb) * blockDim.x + threadIdx.x, L = 1 << sh, gs = 4 * K * L, l = i & (L - 1), c0 = (i >> sh) * gs + 4 * l;
-  if (c0 >= inner) return;
+  if (c0 >= inner || t >= T_) return;
   y += t * inner, out += t * inner;
   Raw4<float> yr[K], wr[K];
   Raw4<T> zr[K];
@@ -227,7 +227,8 @@ void gated_group_norm(const float* y, const void* z, bool f32, int64_t ld_z, con
                       int T_, int inner, int ng, bool gate_after, hipStream_t st) {
   if (T_ <= 0) return;
   const int esz = f32 ? 4 : 2, gsz = inner / ng, L = gsz <= 256 ? gsz / 4 : 64, K = L > 0 ? gsz / (4 * L) : 0;
-  const int lanes = ng * L, nb = (lanes + 255) / 256, block = nb > 1 ? 256 : (lanes + 63) / 64 * 64;
+  const int lanes = ng * L, nb = (lanes + 255) / 256;
+  const dim3 block = row_block(lanes);
   if (L > 0 && (L & (L - 1)) == 0 && 4 * K * L == gsz && (K == 1 || K == 2 || K == 4) && (!w || wn % 4 == 0) &&
       (!z || (ld_z % 4 == 0 && (uintptr_t)z % (4 * esz) == 0)) && (int64_t)T_ * nb < (1ll << 31) &&
       (((uintptr_t)y | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
@@ -235,9 +236,8 @@ void gated_group_norm(const float* y, const void* z, bool f32, int64_t ld_z, con
     while (1 << sh < L) ++sh;
 #define XGM_GN(KK)                                                                                                         \
   if (K == KK) {                                                                                                           \
-    XGM_DISPATCH_T(f32, gated_group_norm4_kernel<T, KK><<<(unsigned)T_ * nb, block, 0, st>>>(y, (const T*)z, ld_z, w, wn, eps, \
-                                                                                         (T*)out, inner, nb, sh,           \
-                                                                                         gate_after ? 1 : 0);)             \
+    XGM_DISPATCH_T(f32, gated_group_norm4_kernel<T, KK><<<(unsigned)((T_ + block.y - 1) / block.y) * nb, block, 0, st>>>(      \
+        y, (const T*)z, ld_z, w, wn, eps, (T*)out, T_, inner, nb, sh, gate_after ? 1 : 0);)                                \
   }
     XGM_GN(1)
     XGM_GN(2)

@@ -110,6 +110,20 @@ def test_group_norms(size, groups, dt):
         close(got, v, size / 2 + 16, float(v.abs().max()))
 
 
+@pytest.mark.parametrize("H,D", [(1, 4), (1, 64), (3, 16), (5, 32), (15, 16), (1, 128), (2, 128), (2, 2), (63, 4), (64, 4)])
+@pytest.mark.parametrize("T", [1, 5, 255, 257, 1000])
+def test_rows_of_few_lanes(H, D, T):
+    """Rows of less than a wave share workgroups: any number of them, the last workgroup's in part."""
+    g, n = torch.Generator().manual_seed(H * D + T), H * D
+    y, z, w = torch.randn(T, n, generator=g), torch.randn(T, n, generator=g).bfloat16(), torch.randn(n, generator=g)
+    heads = y.double().view(T, H, D)
+    v = (heads / (heads.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).view(T, n) * w.double()
+    got = sq.delta_rule_out(y.cuda(), w.cuda(), z.cuda(), 1e-5, H, D, torch.bfloat16)
+    close(got, v * torch.sigmoid(z.double()), D / 2 + 16, float(v.abs().max()))
+    got = sq.gated_group_norm(y.cuda(), z.cuda(), w.cuda(), 1e-5, H, torch.bfloat16, gate_after=True)
+    close(got, v * z.double() * torch.sigmoid(z.double()), D / 2 + 24, 4 * float(v.abs().max()))
+
+
 def test_gates_behind_which_bf16_follows():
     """Their error against fp64 is that of the rounding: as with expf and a division, to 1 in 10^4."""
     x = torch.linspace(-12, 12, 1 << 16).bfloat16()
