@@ -63,7 +63,11 @@ template <bool KEEP, int TAPS, int NTHR, int NV>
 __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a) {
   constexpr int NH = TAPS - 1, NW = NTHR / 64, ROWS = 2, DEPTH = 2;
   constexpr int AGAIN = (NH + ROWS - 1) / ROWS;   // groups of the last rows
-  __shared__ float red[2][ROWS][NW];
+  // a row's sum is that of 256 threads, each with every 256th quad: of the two rows of a group twice as many threads take one each
+  constexpr bool SWAP = NTHR > 256;
+  static_assert(!SWAP || NTHR == 256 * ROWS, "rows of a group and threads");
+  __shared__ float red[2][ROWS][SWAP ? 4 : NW];
+  __shared__ __attribute__((aligned(16))) float held[SWAP ? ROWS : 1][SWAP ? 4 * NV * NTHR : 4];
   const int s = blockIdx.y, W = a.W;
   // the rows behind the last sequence are normed as well, and not convolved
   const int q0 = a.qsl[s], q = (s < a.ns ? a.qsl[s + 1] : a.T) - q0, slot = s < a.ns ? a.slots[s] : -1;
@@ -138,6 +142,10 @@ __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a
     const uint32_t vals = (uint32_t)(t1 - t0) * W;
     const StripOut xo = {a.x_out + at0, 4 * vals}, no = {a.n32 + at0, a.n32 ? 4 * vals : 0}, ao = {a.nact + at0, a.nact ? 2 * vals : 0},
                    ho = {a.h + at0, slot >= 0 ? 2 * vals : 0}, so = {st, (uint32_t)(4 * NH * W)};
+    auto add_squares = [](const float (&f)[4], float& sum) __attribute__((always_inline)) {   // (each form as the separate launch rounds it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = KEEP ? sum + f[e] * f[e] : fmaf(f[e], f[e], sum);
+    };
     auto group = [&](int d, int it) __attribute__((always_inline)) {
       const int t = row_of(it);
       float v[ROWS][NV][4], ss[ROWS];
@@ -161,18 +169,37 @@ __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[i][j][e] += s2[j][e] * y[e];
           }
-          if (on[j])
-#pragma unroll
-            for (int e = 0; e < 4; ++e)   // (each as the separate launch rounds it)
-              ss[i] = KEEP ? ss[i] + v[i][j][e] * v[i][j][e] : fmaf(v[i][j][e], v[i][j][e], ss[i]);
+          if constexpr (SWAP) {
+            if (on[j]) st4(held[i] + col[j], v[i][j]);
+          } else if (on[j]) {
+            add_squares(v[i][j], ss[i]);
+          }
         }
       }
       if (it + DEPTH < groups) load(d, it + DEPTH);
+      if constexpr (SWAP) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        xgk::raw_barrier();
+        const int i = wv / 4;
+        float sum = 0.f;
 #pragma unroll
-      for (int i = 0; i < ROWS; ++i) ss[i] = wave_sum(ss[i]);
-      if (lane == 0)
+        for (int j = 0; j < NV * ROWS; ++j) {
+          const int c = 4 * ((int)(threadIdx.x & 255) + 256 * j);
+          float f[4];
+          if (c < W) {
+            ld4(held[i] + c, f);
+            add_squares(f, sum);
+          }
+        }
+        sum = wave_sum(sum);
+        if (lane == 0) red[it & 1][i][wv & 3] = sum;
+      } else {
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) red[it & 1][i][wv] = ss[i];
+        for (int i = 0; i < ROWS; ++i) ss[i] = wave_sum(ss[i]);
+        if (lane == 0)
+#pragma unroll
+          for (int i = 0; i < ROWS; ++i) red[it & 1][i][wv] = ss[i];
+      }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       xgk::raw_barrier();   // (two sets of sums in turn: one barrier between those who write a set and those who still read it)
       float rs[ROWS];
@@ -180,7 +207,7 @@ __global__ __launch_bounds__(NTHR, 2) void norm_conv_kernel(const NormConvArgs a
       for (int i = 0; i < ROWS; ++i) {
         float sum = 0.f;
 #pragma unroll
-        for (int k = 0; k < NW; ++k) sum += red[it & 1][i][k];
+        for (int k = 0; k < (SWAP ? 4 : NW); ++k) sum += red[it & 1][i][k];
         rs[i] = 1.f / sqrtf(sum / (float)W + a.eps);
       }
 #pragma unroll

@@ -129,6 +129,28 @@ def test_strips(strip, W, taps, monkeypatch):
         close(st, new, W / 2 + 16, max(big, 5.0))
 
 
+@pytest.mark.parametrize("W", [64, 1024, 1032, 2048, 2056, 3000, 4096])
+@pytest.mark.parametrize("lens", [[1, 2, 3, 40], [257, 33], [2599]])
+def test_the_bits_of_the_separate_launches(W, lens):
+    """A row's sum is formed in one order, whichever launch forms it (rows of whole 16 bytes; others were summed entry by entry)."""
+    g, n, T = torch.Generator().manual_seed(W + len(lens)), len(lens), sum(lens)
+    sm, _ = meta(lens, [(0, 5)[i % 2] for i in range(n)], list(range(n)))
+    x, w, a1, a2, cw = (torch.randn(*s, generator=g).cuda() for s in ((T, W), (W,), (W,), (W,), (W, 4)))
+    y, z = (torch.randn(T, W, generator=g).bfloat16().cuda() for _ in range(2))
+    state = torch.randn(n, 3, W, generator=g).cuda()
+
+    def both(rows, separate):
+        s1, s2, old = state.clone(), state.clone(), x.clone()
+        got, want = rows(x, s1), separate(old, s2)
+        want = (old, *(want if isinstance(want, tuple) else (want,)), s2)
+        for a, b in zip((*got, s1), want):
+            assert torch.equal(a, b)
+    both(lambda v, s: sq.norm_conv_rows(v, y, w, 1e-5, 0.7, a1, (cw, s), sm, torch.bfloat16),
+         lambda v, s: sq.norm_conv(v, y, w, 1e-5, 0.7, a1, (cw, s), sm, torch.bfloat16))
+    both(lambda v, s: sq.residual_norm_conv_rows(v, y, a1, z, None, a2, w, 1e-5, torch.bfloat16, (cw, s), True, sm),
+         lambda v, s: sq.residual_norm_conv(v, y, a1, z, None, a2, w, 1e-5, torch.bfloat16, (cw, s), True, sm))
+
+
 def test_others_take_the_separate_kernels(monkeypatch):
     """More than 4096 columns, fp32 rows, a sum over experts, weights off 16 bytes: in place, by the launches they had."""
     calls = record_native(monkeypatch, sq)
