@@ -15,15 +15,16 @@
 // writes them.
 //
 // A strip is 8 rows, with those before it, while that leaves a CU without a second workgroup, else as short as leaves two for each of
-// them (one of rows beyond 2048 columns): the weights that a workgroup loads are four rows' bytes. us, KEEP / the other form, two
-// launches before in brackets: 8192 x 2048 in strips of 8 / 12 / 20 / 28 47.8 / 41.6 / 38.3 / 44.9 (53.5) and 63.2 / 58.2 / 54.0 / 60.2
-// (79.6); 2521 x 2048 in 8 / 12 / 16 19.4 / 17.3 / 19.0 (20.5) and 23.8 / 21.6 / 24.3 (26.6); 8192 x 4096 in 36 87 (108) and 116 (170);
-// 2599 x 4096 in 16 27.6 (37.1) and 36.6 (56.0); 512 x 2048 8.6 (10.8) and 10.3 (14.5); 96 single tokens of 2048 5.6 (7.1) and 6.1 (8.0),
-// 256 of 4096 10.3 (14.2) and 11.1 (16.8). Rows of 4096 up to some 400 (100 10.9 (9.2) and 13.1 (11.3)), and of 2048 up to 200 (100 8.2 (7.7)
-// and 9.6 (8.7)), are slower than in two launches on the card, but not in a step, which the host launches: 65 rows Dofivik 1b 1140 (1149), 8b
-// 763 (762), Vizonex 1b 834 (866), 8b 720 (725), 200 rows 1163 (1182), 950 (949), 923 (934), 940 (948). Rows of up to 1024 columns have one
-// quad a thread (two, half of them idle, in square brackets): 300 x 1024 6.8 [8.2] (7.5) and 7.6 [9.8] (8.4), 1500 10.8 [12.1] (10.7) and
-// 12.1 [15.1] (13.1), 8192 27.5 [29.0] (29.7) and 34.3 [38.8] (49.3).
+// them (one of rows beyond 2048 columns): the weights that a workgroup loads are four rows' bytes. us, KEEP / the other form, the two
+// launches in brackets (four sets of rows in turn): 8192 x 2048 in strips of 20 47.8 (57.1) and 63.5 (86.5), 2521 x 2048 in 12 19.2 (21.6)
+// and 28.2 (32.3), 8192 x 4096 in 36 89.3 (110) and 118 (175), 2599 x 4096 in 16 34.0 (38.8) and 45.2 (62.7), 512 x 2048 9.5 (9.7) and 10.4
+// (12.0), 300 x 4096 12.5 (11.5) and 14.2 (14.6), 96 single tokens of 2048 5.4 (7.1) and 5.8 (8.1), 256 of 4096 10.3 (14.1) and 11.2 (16.8).
+// Rows of 2048 up to some 200 (100 8.2 (7.8) and 9.0 (8.7)) and with two branches of 4096 (100 13.1 (11.2)) are slower than in two launches
+// on the card, but not in a step, which the host launches: 65 rows Dofivik 1b 1215 (1221), Vizonex 1b 833 (863), 8b 724 (723), 200 rows 1169
+// (1190), 913 (930), 968 (974). (The caller keeps the two launches for 65 to 699 rows of 4096 with one branch.)
+//
+// Threads have one quad of columns up to 1024 columns (with two, half of them idle: 1500 x 1024 10.8 / 12.1 instead of 12.1 / 15.1), and in
+// strips of 8 rows up to 2048, where a wave's instructions count (512 x 2048 9.5 / 10.4 instead of 9.5 / 11.4); else two.
 #include "glds.h"
 #include "mixers_common.h"
 
@@ -275,9 +276,10 @@ int norm_conv(const float* x, const void* y1, int64_t ld1, const void* y2, int64
                           qsl, seq_lens, slots, x_out, n32, (bf16*)nact, (bf16*)h, T_, W, ns, rows};
   const int n = max(1, (max_q + rows - 1) / rows);
   const dim3 grid(n < 65535 ? n : 65535, ns + 1);
-#define XGM_NC(KEEP, TAPS)                                                    \
-  if (W <= 1024) norm_conv_kernel<KEEP, TAPS, 256, 1><<<grid, 256, 0, st>>>(a);       \
-  else if (W <= 2048) norm_conv_kernel<KEEP, TAPS, 256, 2><<<grid, 256, 0, st>>>(a);  \
+#define XGM_NC(KEEP, TAPS)                                                                          \
+  if (W <= 1024) norm_conv_kernel<KEEP, TAPS, 256, 1><<<grid, 256, 0, st>>>(a);                     \
+  else if (W <= 2048 && strip == 8) norm_conv_kernel<KEEP, TAPS, 512, 1><<<grid, 512, 0, st>>>(a);  \
+  else if (W <= 2048) norm_conv_kernel<KEEP, TAPS, 256, 2><<<grid, 256, 0, st>>>(a);                \
   else norm_conv_kernel<KEEP, TAPS, 512, 2><<<grid, 512, 0, st>>>(a);
 #define XGM_NCT(KEEP)                                                                             \
   if (taps == 4) { XGM_NC(KEEP, 4) } else if (taps == 3) { XGM_NC(KEEP, 3) } else { XGM_NC(KEEP, 2) }

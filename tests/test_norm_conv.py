@@ -167,3 +167,20 @@ def test_others_take_the_separate_kernels(monkeypatch):
     assert sq.residual_norm_conv_rows(x, ones(T, 64).bfloat16(), None, None, ones(T, 64), None, ones(64), 1e-5, torch.bfloat16,
                                       (ones(64, 4), ones(2, 3, 64)), False, sm)[0] is x
     assert "norm_conv" not in calls
+
+
+@pytest.mark.parametrize("W,lens,one", [(4096, [65], False), (4096, [699], False), (4096, [700], True), (4096, [64], True), (2048, [65], True),
+                                        (4096, [1] * 96, True), (2056, [1, 70], False)])
+def test_wide_rows_of_some_hundred_tokens(W, lens, one, monkeypatch):
+    """One branch: in two launches where one is the slower, with the same bits."""
+    calls = record_native(monkeypatch, sq)
+    g, n, T = torch.Generator().manual_seed(W), len(lens), sum(lens)
+    sm, _ = meta(lens, [0] * n, list(range(n)))
+    x, w, cw = (torch.randn(*s, generator=g).cuda() for s in ((T, W), (W,), (W, 4)))
+    y, state = torch.randn(T, W, generator=g).bfloat16().cuda(), torch.zeros(n, 3, W, device="cuda")
+    got = sq.norm_conv_rows(x.clone(), y, w, 1e-5, 0.7, None, (cw, state), sm, torch.bfloat16)
+    assert ("norm_conv" in calls) == one
+    monkeypatch.setattr(sq, "NORM_CONV_WIDE_MIN", 1 << 30 if one else 0)
+    monkeypatch.setattr(sq, "_conv_rows", lambda *a: not one)
+    again = sq.norm_conv_rows(x, y, w, 1e-5, 0.7, None, (cw, torch.zeros_like(state)), sm, torch.bfloat16)
+    assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])

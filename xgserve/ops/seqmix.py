@@ -450,6 +450,12 @@ def _conv_rows(x: torch.Tensor, y1, y2, a1, a2, bias, w: torch.Tensor, conv: Opt
     return at % 16 == 0
 
 
+# Portions' rows of more than 2048 columns with one branch: two launches from 65 rows up to here (us on the card, one / two launches, 4096
+# columns: 65 rows 11.1 / 8.9, 200 12.1 / 10.8, 400 13.0 / 12.2, 700 14.7 / 15.2, 1000 16.4 / 18.0; steps of Dofivik 8b, 100 rows 823 / 817,
+# 300 1104 / 1098, 512 1358 / 1353, 1000 2072 / 2088). Fewer rows wait for the host, which has one launch less (16 rows 660 / 664).
+NORM_CONV_WIDE_MIN = 700
+
+
 def _norm_conv(x, y1, y2, a1, a2, bias, alpha, w, off, eps, keep_norm, want_f32, want_act, conv, sm):
     T, W = x.shape
     cw, state = conv
@@ -468,7 +474,8 @@ def norm_conv_rows(x: torch.Tensor, y, w: torch.Tensor, eps: float, alpha: float
                    conv: Optional[tuple], sm: SeqMeta, dtype: torch.dtype):
     """norm_conv as (new x, convolution or None): x itself, updated, or where the rows of a prompt take both in one pass another
     tensor (a workgroup there reads rows that belong to its neighbour)."""
-    if _conv_rows(x, y, None, None, None, bias, w, conv, sm, dtype):
+    apart = x.shape[1] > 2048 and 64 < x.shape[0] < NORM_CONV_WIDE_MIN and sm.max_q > 1
+    if not apart and _conv_rows(x, y, None, None, None, bias, w, conv, sm, dtype):
         out, _, _, h = _norm_conv(x, y, None, None, None, bias, alpha, w, 1.0, eps, True, False, False, conv, sm)
         return out, h
     return x, norm_conv(x, y, w, eps, alpha, bias, conv, sm, dtype)
