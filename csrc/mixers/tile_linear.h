@@ -572,10 +572,15 @@ static TileForm tile_form(int nk_least, int nk_most, int fm, int fn, int ra) {
 // leave such a round; 160 x 192 and 128 x 192 were the fastest too rarely, by 1 to 6 %)
 // (96 x 64 with rings of four, which two workgroups of a CU just have: w is asked for one step behind x, so that in rings of three it
 // comes late. us, rings that end with the tile and ask for both at once / of three / of four: 400 x 2048 x 2048 12.1 / 12.6 / 11.5, 298 x
-// 4096 x 4096 28.4 / 29.0 / 24.8, 65 x 16384 x 2048 20.2 / 20.2 / 17.7, in four parts 130 x 2048 x 2048 10.1 / 10.5 / 10.5)
+// 4096 x 4096 28.4 / 29.0 / 24.8, 65 x 16384 x 2048 20.2 / 20.2 / 17.7, in four parts 130 x 2048 x 2048 10.1 / 10.5 / 10.5. Four tiles of K, which
+// a ring of four would not turn for, have three slots for x: 93 x 1088 x 2048 in eight parts 11.5 / 9.2)
 template <bool PAIR>
 static int tile_launch_size(const TileArgs& a, int fm, int fn, int cus, hipStream_t st) {
   const int nk = a.K / 64, least = nk / a.S, most = (nk + a.S - 1) / a.S;
+  if (fm == 3 && fn == 2 && least == 4) {
+    tile_launch<PAIR, 3, 2, 3, 4, 2>(a, cus, st);
+    return 0;
+  }
 #define XGM_TILE(FM, FN, RA, RW, OCC)                                                   \
   if (fm == FM && fn == FN) {                                                           \
     const TileForm form = tile_form(least, most, FM, FN, RA);                           \
