@@ -2,12 +2,12 @@
 #include "tile_linear.h"
 
 namespace xgm {
-template <int FM, int FN, int RA, int RW, bool SHORT = false>
+template <int FM, int FN, int RA, int RW, int OCC = 1, bool SHORT = false>
 static void tile_launch_grouped(const TileArgs& a, int cus, hipStream_t st) {
   const int64_t tiles = (int64_t)(a.M / (32 * FM) + a.E) * ((a.N + 32 * FN - 1) / (32 * FN));   // at most
-  const int grid = SHORT || tiles < cus ? (int)tiles : cus;
-  if (a.pairs) tile_linear_kernel<FM, FN, RA, RW, 1, true, true, SHORT><<<grid, 256, 0, st>>>(a);
-  else tile_linear_kernel<FM, FN, RA, RW, 1, false, true, SHORT><<<grid, 256, 0, st>>>(a);
+  const int grid = SHORT || tiles < cus * OCC ? (int)tiles : cus * OCC;
+  if (a.pairs) tile_linear_kernel<FM, FN, RA, RW, OCC, true, true, SHORT><<<grid, 256, 0, st>>>(a);
+  else tile_linear_kernel<FM, FN, RA, RW, OCC, false, true, SHORT><<<grid, 256, 0, st>>>(a);
 }
 
 // Products of the experts' sorted rows (moe_align, moe_ff.hip) with their expert's weights w [E, N, K]: gated (act >= kTileGlu) `out`
@@ -26,7 +26,8 @@ int tile_grouped(const void* x, int64_t ld_x, int x_rows, const int32_t* rows, c
 #define XGM_TILE(FM, FN, RA, RW)                                                \
   else if (fm == FM && fn == FN) {                                              \
     if (K / 64 > RA) tile_launch_grouped<FM, FN, RA, RW>(a, cus, st);           \
-    else tile_launch_grouped<4, 4, 5, 5, true>(a, cus, st);                     \
+    else if (K / 64 > 2) tile_launch_grouped<4, 4, 2, 3, 2>(a, cus, st);        \
+    else tile_launch_grouped<4, 4, 2, 2, 2, true>(a, cus, st);                  \
   }
   if (false) {}
   XGM_TILE(8, 8, 2, 3)

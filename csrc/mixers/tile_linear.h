@@ -11,7 +11,7 @@
 // whose first reader waits for HBM). A K tile is two steps, one per 32 of K. Between the products of a step the other step's fragments
 // are read (into the registers that the step before has used up) and the tiles RA and RW further on asked for, x in the second step and
 // w in the next one's first, in even distances and not beside a read: with all of them in the second step, their addresses computed
-// beside them, a K tile of 256 x 256 took 2670 clocks for 2048 of products, so 2400 (8192 x 4096 x 14336, us: 673 -> 624, of which 5 are
+// beside them, a K tile of 256 x 256 took 2670 clocks for 2048 of products, so 2400 (8192 x 4096 x 14336, us: 673 -> 625, of which 5 are
 // the order of products, row after row there and back, so that the operand at the turn stays: less power). One barrier per K tile. The
 // 16-byte granules of a row are permuted by the row, so that the
 // reads of 16 rows fall on all banks; w's rows are dealt to the fragments in fours, so that a lane ends up with eight neighbouring
@@ -19,10 +19,10 @@
 //
 // Workgroups stay and take tile after tile, and the ring runs through: where a tile has RA tiles of K to go, the loads go over to the
 // next one, and its first step takes the results out of an accumulator right before the product that starts it anew. The stores go
-// through buffer descriptors, which drop what lies outside, so that there is no branch between the products. us, without / with: 8192 x
-// 8192 x 2048 204 / 191, 5000 x 5000 x 448 on 128 x 128 48 / 33.5, 5000 x 5000 x 192 27 / 22.8, 8192 x 28672 x 4096 gated 1327 / 1295 (the
-// gates' vector work is the matrix cores' wait either way); one tile a workgroup, 512 x 6144 x 4096 39.7 / 38.5, 256 x 2048 x 192 12.4 / 10.0.
-// S parts of K fill the chip where the tiles are few; their slabs are added by a second launch. K of up to RA tiles has no ring to run:
+// through buffer descriptors, which drop what lies outside, so that there is no branch between the products. us, without (and
+// with all loads in the second step) / with, on one box: 8192 x 8192 x 2048 228 / 208, 5000 x 5000 x 448 on 128 x 128 60 / 47, 8192 x 28672 x
+// 4096 gated 1336 / 1311 (the gates' vector work is the matrix cores' wait either way); one tile a workgroup, 512 x 6144 x 4096 41.8 / 40.6.
+// S parts of K fill the chip where the tiles are few; their slabs are added by a second launch. K of one or two tiles has no ring to run:
 // all of it is loaded first, a workgroup per tile (SHORT).
 //
 // The grouped form (tile_grouped) walks the tiles of all experts' sorted rows one expert after the other, with the rows of x gathered
@@ -30,10 +30,10 @@
 // grouped_rows.hip or 192 to 288-row ones of gemm_pf (tokens, two experts each): 2 x 3584 x 4096 300 240 -> 152, 700 242 -> 189, 4000
 // 744 -> 631, 8192 1401 -> 1300; 2 x 2048 x 2048 1000 129 -> 85; 32 experts of 2 x 1024 x 2048, four each, 2000 239 -> 194.
 //
-// Measured, cold weights, us, against the library's product without what follows (M x N x K): 128 x 4096 x 14336 34 against 72;
-// 512 x 4096 x 14336 64 against 86; 300 x 10304 x 2048 20 against 24; 2521 x 10304 x 2048 88 against 96; 4001 x 18560 x 4096 438 against 554;
-// gated, 2521 x 16384 x 2048 141 against 192 with its activation, 8192 x 28672 x 4096 1319 against 1404; 8192 x 4096 x 14336 645 against 599
-// (1.49 PFLOP/s at the power limit: the library's has the better of it in long plain products, which stay there).
+// Measured, cold weights, us, against the library's product without what follows (M x N x K), on the same box: 128 x 4096 x 14336 37 against
+// 79; 512 x 4096 x 14336 72 against 95; 300 x 10304 x 2048 23 against 28; 2521 x 10304 x 2048 98 against 105; 4001 x 18560 x 4096 447 against
+// 560; gated, 2521 x 16384 x 2048 140 against 191 with its activation, 8192 x 28672 x 4096 1311 against 1417; 8192 x 4096 x 14336 625 against
+// 615 (1.54 PFLOP/s at the power limit: the library's has the better of it in long plain products, which stay there).
 #pragma once
 
 #include <type_traits>
@@ -155,9 +155,10 @@ __device__ __forceinline__ float tile_act(const TileArgs& a, float v) {
   return ACT == kTileXielu ? xieluf(v, a.p0, a.p1) : ACT == kTileRelu2 ? relu2f(v) : v;
 }
 // glu.h's gates for a bf16 result, whose rounding is 2^-9: the exponential and reciprocal instructions (2^-23 each, and 2^-24 of the
-// exponent from its rounding) instead of expf and a division, 20 instructions an output instead of 45. A tile's gates run on four waves while its matrix cores wait: 8192 x 16384 x 2048
-// 440 -> 405 us, 2521 rows 152 -> 141, 8192 x 28672 x 4096 1381 -> 1319. Error of the result against fp64 over gates and factors of spread
-// 0.3, 1 and 3: 1.649554e-3, 1.660321e-3, 1.654740e-3 (tanh-GELU; the others likewise), the same to seven digits as with those.
+// exponent from its rounding) instead of expf and a division, 20 instructions an output instead of 45. A tile's gates run on four waves while
+// its matrix cores wait: with rings that end with the tile, 8192 x 16384 x 2048 440 -> 405 us, 2521 rows 152 -> 141. Error of the result
+// against fp64 over gates and factors of spread 0.3, 1 and 3: 1.649554e-3, 1.660321e-3, 1.654740e-3 (tanh-GELU; the others likewise), the
+// same to seven digits as with those.
 template <int KIND>
 __device__ __forceinline__ float tile_glu(const TileArgs& a, float g, float u) {
   if (KIND == xgk::kGluClamped) g = fminf(g, a.p0), u = fminf(fmaxf(u, -a.p0), a.p0) + 1.f;
@@ -554,17 +555,27 @@ static void tile_launch(const TileArgs& a, int cus, hipStream_t st) {
   tile_linear_kernel<FM, FN, RA, RW, OCC, PAIR, false, SHORT><<<grid, 256, 0, st>>>(a);
 }
 
-// K (a part of it) of up to RA tiles: the ring does not turn. Up to five tiles then run on 128 x 128 tiles without one, six on 128 x 64 where
-// those were asked for, and what lies on both sides of that (parts that differ by one tile) on the ring of two. Beyond kRotateRows rows the
-// results are the same bits, as every size then sums K in the same order; up to there a column begins where its tile's number says, which
-// goes by the tile's width. us, as it was with a ring that ends with the tile / now: 700 x 2056 x 256 6.9 / 5.8, 300 x 4096 x
-// 384 6.0 / 5.5, 256 x 2048 x 128 11.4 (256 x 256) / 4.6, but 4096 x 4096 x 128 15.4 (256 x 256) / 17.6: no weight is that narrow.
-constexpr int kShortK = 5;
-enum TileForm { kFormRing, kFormShort, kFormShortNarrow, kFormRing2 };
-static TileForm tile_form(int nk_least, int nk_most, int fm, int fn, int ra) {
-  if (nk_least > ra) return kFormRing;
-  if (nk_most <= 6 && fm == 4 && fn == 2) return kFormShortNarrow;
-  return nk_most <= kShortK ? kFormShort : kFormRing2;
+// K (a part of it) of up to RA tiles: the ring of this size does not turn. From three tiles on a ring of two does, on the nearest of three
+// sizes, the smaller ones in two workgroups a CU; one or two are loaded whole, by a workgroup for every tile of the result and two a CU, so
+// that one's stores run beside the other's loads. (Parts of two and of three tiles: the same with three slots.) Beyond kRotateRows rows all
+// sizes give the same bits, as all sum K in the same order; up to there a column begins where its tile's number says, which goes by the
+// tile's width. us, rings that end with the tile / now (in brackets all of K loaded first, a workgroup a CU): 2521 x 2048 x 64
+// 8.1 / 7.3 (9.2), 8192 x 8192 x 128 64 / 51 (79) and gated 48 / 43 (68), 8192 x 8192 x 192 78 / 61 (92), 2521 x 2048 x 256 9.8 / 9.1 (13.4), 300 x
+// 16384 x 256 9.9 / 9.3 (13.4), 300 x 2048 x 192 5.0 / 4.8 (5.9); 32 experts of 128 x 2048, four each, 6000 tokens 170 / 177 (217).
+template <bool PAIR>
+static void tile_launch_short(const TileArgs& a, int fm, int fn, int least, int most, int cus, hipStream_t st) {
+  const int area = fm * fn;
+  if (least > 2) {
+    if (area <= 12) tile_launch<PAIR, 3, 2, 2, 3, 2>(a, cus, st);
+    else if (area <= 28) tile_launch<PAIR, 4, 4, 2, 3, 2>(a, cus, st);
+    else tile_launch<PAIR, 5, 8, 2, 3, 1>(a, cus, st);
+  } else if (most > 2) {
+    tile_launch<PAIR, 4, 4, 3, 3, 1, true>(a, cus, st);
+  } else if (area <= 12) {
+    tile_launch<PAIR, 3, 2, 2, 2, 2, true>(a, cus, st);
+  } else {
+    tile_launch<PAIR, 4, 4, 2, 2, 2, true>(a, cus, st);
+  }
 }
 
 // the launch of one size (-1: there is none); gated products are compiled in tile_gated.hip
@@ -583,11 +594,8 @@ static int tile_launch_size(const TileArgs& a, int fm, int fn, int cus, hipStrea
   }
 #define XGM_TILE(FM, FN, RA, RW, OCC)                                                   \
   if (fm == FM && fn == FN) {                                                           \
-    const TileForm form = tile_form(least, most, FM, FN, RA);                           \
-    if (form == kFormRing) tile_launch<PAIR, FM, FN, RA, RW, OCC>(a, cus, st);          \
-    else if (form == kFormShort) tile_launch<PAIR, 4, 4, 5, 5, 1, true>(a, cus, st);    \
-    else if (form == kFormShortNarrow) tile_launch<PAIR, 4, 2, 6, 6, 1, true>(a, cus, st); \
-    else tile_launch<PAIR, 8, 8, 2, 3, 1>(a, cus, st);                                  \
+    if (least > RA) tile_launch<PAIR, FM, FN, RA, RW, OCC>(a, cus, st);                 \
+    else tile_launch_short<PAIR>(a, FM, FN, least, most, cus, st);                      \
     return 0;                                                                           \
   }
   XGM_TILE(8, 8, 2, 3, 1)

@@ -121,7 +121,7 @@ def test_equal_rows_give_equal_bits(tile, tiles, S):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("K", [64, 192, 320, 384, 448, 1024])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448, 1024])
 def test_sizes_of_tiles_sum_in_the_same_order(K):
     """More than 256 rows: every size of the tile gives the same bits, K of a few tiles (forms without a ring) and longer."""
     g = torch.Generator("cuda").manual_seed(K)
