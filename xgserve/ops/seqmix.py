@@ -92,8 +92,8 @@ _ROWS_PARTS, _ROWS_PART_K = 8, 512
 _ROWS_TICKETS = _ROWS_WGS // 2     # column tiles of a product in parts
 
 # xIELU behind the product of prompt rows up to here: its 25 instructions an element run on four waves there and on a full chip in a
-# launch of their own (8192 x 2048, us, behind / by itself: 300 rows 20.6 / 24.3, 1000 rows 42.9 / 42.0, 2048 rows 85 / 70, 8192 rows 255 / 246). The
-# squared ReLU and the gated activations always go behind (8192 rows: 216 / 253; gated 16384 x 2048, 2521 rows 141 / 192).
+# launch of their own (8192 x 2048, us, behind / by itself: 300 rows 22.7 / 23.9, 1000 rows 42.0 / 42.9, 2048 rows 70.9 / 68.5, 8192 rows 267 /
+# 257). The squared ReLU and the gated activations always go behind (8192 rows: 214 / 263; gated 16384 x 2048, 2521 rows 140 / 191).
 XIELU_BEHIND_MAX = 512
 
 ACT_NONE, ACT_XIELU, ACT_RELU2, ACT_GLU = 0, 1, 2, 3   # ACT_GLU + GLU_...: the gated activations

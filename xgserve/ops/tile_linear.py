@@ -1,8 +1,11 @@
 """Products of many rows (prompt steps) on csrc/mixers/tile_linear.h: the sizes they run at, and where the library's stay.
 
 `tile_plan` prices every tile and split of K of the kernel with a model that was fitted to 13 900 timings on an MI355X (2 590 products
-of 52 weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights); over these its choice is 0.6 % slower than the
-fastest form that was timed in the mean and 19 % at most. A step of 64 of K costs a workgroup its products or, of few rows, its reads:
+of 52 weights of 512 to 18944 in K and 32 to 37888 in N, 65 to 6000 rows, cold weights), of the kernel whose load ring ended with each
+tile of the result. Over these its choice was 0.6 % slower than the fastest form that was timed in the mean and 19 % at most. Of the kernel
+as it is, whose ring runs through the tiles, 144 products of 16 weights were timed (65 to 6000 rows, all forms within half of the cheapest
+price): 0.8 % in the mean, 9 % at most (251 x 4096 x 14336 48.7 us, 44.9 on 256 x 128 in eight parts). The figures that follow are of the
+fit. A step of 64 of K costs a workgroup its products or, of few rows, its reads:
 weights come from memory, rows from L2, at the rate at which its outstanding loads return (ops.seqmix._rows_cols has the same for a few
 rows). Without that the smallest tiles looked cheaper than they are: us, 224 x 4096 x 4096 27.1 -> 21.9, 768 x 2048 x 8192 50 -> 37,
 288 x 18560 x 4096 75 -> 60; of 483 products, whose plan this changed, the times are 8 % less in the mean, 11 % more at most. A
@@ -87,14 +90,15 @@ def grouped_plan(pairs: int, E: int, N: int, K: int, cus: int = 256):
 
 def library_better(M: int, N: int, K: int) -> bool:
     """Whether the library's plain product (nothing behind it) is the faster one (us, library against this kernel): long ones, which run
-    at the card's power limit, where the library's needs less of it, by 0 to 12 % (28672x4096, 8192 rows 1222 against 1307; 4096x4096,
-    4001 rows 91 against 98; 16384x2048, 2048 rows 103 against 117), as long as no columns are left over beside its tiles of 256
-    (10304x2048, 4001 rows 168 against 129; 18560x4096, 2048 rows 344 against 257) and these fill their rounds of the chip to three
-    quarters (0.81 to 1: -14 to 10 %; below, at 0.6, 6144x4096, 3100 rows 169 against 126; 4096x14336, 2521 rows 226 against 213;
-    4096x4096, 5000 rows 137 against 132; up to 1792 rows 4096x14336, 1536 rows 168 against 140; 6144x4096, 700 rows 45 against 38). Its narrow
-    products of few rows are 1 to 2 us faster on the card (2048x2048, 65 rows 8.8 against 10.2, 256 rows 10.2 against 11.4; 4096x4096,
-    256 rows 23.1 against 27.8), and some of middle size by 2 to 9 (6144x4096, 512 rows 38.2 against 40.8; 18560x4096, 400 rows 71
-    against 80), but not in steps. Eager ones of few rows wait for the host, of which the library's call takes 31 us and this kernel's
+    at the card's power limit, where the library's needs less of it, by 1 to 10 % (28672x4096, 8192 rows 1284 against 1370; 4096x4096,
+    4001 rows 95 against 98; 16384x2048, 2048 rows 103 against 115; 6144x4096, 8192 rows 279 against 305; but 4096x4096, 3072 rows 81
+    against 76), as long as no columns are left over beside its tiles of 256
+    (10304x2048, 4001 rows 182 against 146; 18560x4096, 2048 rows 347 against 272) and these fill their rounds of the chip to three
+    quarters (below, at 0.6, 6144x4096, 3100 rows 166 against 126; 4096x14336, 2521 rows 249 against 237;
+    4096x4096, 5000 rows 140 against 129; up to 1792 rows 4096x14336, 1536 rows 188 against 150; 6144x4096, 700 rows 52 against 40). Its narrow
+    products of few rows are up to 1 us faster on the card (2048x2048, 65 rows 9.4 against 9.7, 256 rows 10.7 against 11.5), and some of
+    middle size by as much (6144x4096, 512 rows 38.8 against 40.2), others no longer (4096x4096, 256 rows 23.3 against 22.7; 18560x4096, 400
+    rows 71 against 68), but not in steps. Eager ones of few rows wait for the host, of which the library's call takes 31 us and this kernel's
     10: with the faster of both for every product, 96 rows, Vizonex "1b" 868 -> 1159 us, Dofivik 1300 -> 1507; from 400 rows on within
     1 %. Replayed ones of 96 and 160 rows are up to 2 % slower with it, of 256 rows up to 2 % faster."""
     tiles = -(-M // 256) * (N // 256)
