@@ -81,10 +81,8 @@ __device__ __forceinline__ float row_ror(float v) {
 #endif
 }
 template <typename F>
-__device__ __forceinline__ float wave_join(float v, F f) {
+__device__ __forceinline__ float wave_join_halves(float v, F f) {   // lanes ^ 16 .. 1: within each half of the wave
 #if defined(__HIP_DEVICE_COMPILE__)
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
   const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 #endif
@@ -93,8 +91,27 @@ __device__ __forceinline__ float wave_join(float v, F f) {
   v = f(v, row_ror<2>(v));
   return f(v, row_ror<1>(v));
 }
+template <typename F>
+__device__ __forceinline__ float wave_join(float v, F f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+#endif
+  return wave_join_halves(v, f);
+}
 __device__ __forceinline__ float wave_sum(float v) {
   return wave_join(v, [](float a, float b) { return a + b; });
+}
+
+// The sum of x y, a lane's own product joined to that of lane ^ 32 by a multiply-add, one rounding less. (Where wave_sum(x * y) exchanged
+// through LDS the compiler made that of it, and these sums are the same bits; the halves of the wave may differ by that rounding.)
+__device__ __forceinline__ float wave_sum_products(float x, float y) {
+  float v = x * y;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaf(x, y, __uint_as_float(threadIdx.x & 32 ? a[0] : a[1]));
+#endif
+  return wave_join_halves(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {

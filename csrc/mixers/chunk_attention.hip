@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void masked_attention_combine_kernel(
     const float ls = lane < nsplit ? part_ml[2 * (row0 + lane * step) + 1] : 0.f;
     const float M = wave_max(ms);
     w = ms == -INFINITY ? 0.f : exp2_fast(ms - M);
-    const float L = wave_sum(w * ls);
+    const float L = wave_sum_products(w, ls);
     inv = L > 0.f ? 1.f / L : 0.f;
   }
   if (threadIdx.x < 64) ws[lane] = w;
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(256) void talk_mix_parts_kernel(const float* __rest
     const float ls = lane < nsplit ? part_ml[2 * (row0 + g + lane * step) + 1] : 0.f;
     const float M = wave_max(ms);
     const float w = ms == -INFINITY ? 0.f : exp2_fast(ms - M);
-    const float L = wave_sum(w * ls);
+    const float L = wave_sum_products(w, ls);
     ws[g][lane] = w;
     if (lane == 0) inv[g] = L > 0.f ? 1.f / L : 0.f;
   }

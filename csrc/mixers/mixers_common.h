@@ -10,6 +10,7 @@ using xgk::block_sum;
 using xgk::f2bf;
 using xgk::wave_max;
 using xgk::wave_sum;
+using xgk::wave_sum_products;
 typedef uint16_t bf16;
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p);

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const DeltaStepArgs a) 
   if (lane < QC) st4(&part[1][wave][c], o4);
   __syncthreads();
   const float od = d < D ? part[1][0][d] + part[1][1][d] + part[1][2][d] + part[1][3][d] : 0.f;
-  const float osq = wave_sum(od * od);
+  const float osq = wave_sum_products(od, od);
   if (D > 64) {
     if (lane == 0) redo[wave] = osq;
     __syncthreads();
