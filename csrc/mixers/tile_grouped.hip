@@ -22,7 +22,7 @@ int tile_grouped(const void* x, int64_t ld_x, int x_rows, const int32_t* rows, c
       N >= kTileColumns || x_rows * ld_x * 2 >= (1LL << 32))
     return -1;
   TileArgs a = {(const bf16*)x, (const bf16*)w, nullptr, y, (bf16*)out, ld_x, M, N, K, 1, act, gated ? kPairHalves : kPairNone, p0, p1,
-                false, rows, offs, E, top, (int64_t)N * K, M <= (int64_t)kRotateRows * E};
+                false, rows, offs, E, top, (int64_t)N * K, M <= (int64_t)kRotateRows * E ? 32 * fn : 0};
 #define XGM_TILE(FM, FN, RA, RW)                                                \
   else if (fm == FM && fn == FN) {                                              \
     if (K / 64 > RA) tile_launch_grouped<FM, FN, RA, RW>(a, cus, st);           \

@@ -75,7 +75,7 @@ struct TileArgs {
   const int32_t *rows, *offs;
   int E, top;
   int64_t w_stride;
-  bool rotate;             // column tiles start at different K tiles
+  int rotate;              // groups of so many columns start at different K tiles (0: all at the first)
 };
 
 // LDS DMA of 16 bytes a lane from a uniform base and a lane's byte offset
@@ -223,7 +223,7 @@ __device__ __forceinline__ TileAt tile_at(const TileArgs& a, int TN, int v) {
   const int nk_all = a.K / 64;
   t.kt_lo = t.s * nk_all / a.S;
   t.nk = (t.s + 1) * nk_all / a.S - t.kt_lo;
-  t.rot = a.rotate ? (unsigned)tn * 37u % (unsigned)t.nk : 0;
+  t.rot = a.rotate ? (unsigned)(t.n0 / a.rotate) * 37u % (unsigned)t.nk : 0;
   return t;
 }
 // the block's place among nb neighbours in that order: neighbours on one XCD
@@ -558,20 +558,22 @@ static void tile_launch(const TileArgs& a, int cus, hipStream_t st) {
 // K (a part of it) of up to RA tiles: the ring of this size does not turn. From three tiles on a ring of two does, on the nearest of three
 // sizes, the smaller ones in two workgroups a CU; one or two are loaded whole, by a workgroup for every tile of the result and two a CU, so
 // that one's stores run beside the other's loads. (Parts of two and of three tiles: the same with three slots.) Beyond kRotateRows rows all
-// sizes give the same bits, as all sum K in the same order; up to there a column begins where its tile's number says, which goes by the
-// tile's width. us, rings that end with the tile / now (in brackets all of K loaded first, a workgroup a CU): 2521 x 2048 x 64
+// sizes give the same bits, as all sum K in the same order. Up to there a column begins where the number of its tile says, of the size that
+// was asked for: what runs in its place has columns that fill that one's without a rest. us, rings that end with the tile / now (in brackets all of K loaded first, a workgroup a CU): 2521 x 2048 x 64
 // 8.1 / 7.3 (9.2), 8192 x 8192 x 128 64 / 51 (79) and gated 48 / 43 (68), 8192 x 8192 x 192 78 / 61 (92), 2521 x 2048 x 256 9.8 / 9.1 (13.4), 300 x
 // 16384 x 256 9.9 / 9.3 (13.4), 300 x 2048 x 192 5.0 / 4.8 (5.9); 32 experts of 128 x 2048, four each, 6000 tokens 170 / 177 (217).
 template <bool PAIR>
 static void tile_launch_short(const TileArgs& a, int fm, int fn, int least, int most, int cus, hipStream_t st) {
   const int area = fm * fn;
+  const bool narrow = area <= 12 || (a.rotate && fn % 4);
   if (least > 2) {
-    if (area <= 12) tile_launch<PAIR, 3, 2, 2, 3, 2>(a, cus, st);
-    else if (area <= 28) tile_launch<PAIR, 4, 4, 2, 3, 2>(a, cus, st);
+    if (narrow) tile_launch<PAIR, 3, 2, 2, 3, 2>(a, cus, st);
+    else if (area <= 28 || (a.rotate && fn == 4)) tile_launch<PAIR, 4, 4, 2, 3, 2>(a, cus, st);
     else tile_launch<PAIR, 5, 8, 2, 3, 1>(a, cus, st);
   } else if (most > 2) {
-    tile_launch<PAIR, 4, 4, 3, 3, 1, true>(a, cus, st);
-  } else if (area <= 12) {
+    if (narrow) tile_launch<PAIR, 3, 2, 3, 3, 2, true>(a, cus, st);
+    else tile_launch<PAIR, 4, 4, 3, 3, 1, true>(a, cus, st);
+  } else if (narrow) {
     tile_launch<PAIR, 3, 2, 2, 2, 2, true>(a, cus, st);
   } else {
     tile_launch<PAIR, 4, 4, 2, 2, 2, true>(a, cus, st);

@@ -38,7 +38,7 @@ int tile_linear(const void* x, int64_t ld_x, const void* w, const void* bias, bo
       N >= kTileColumns || (int64_t)N * K * 2 >= (1LL << 32) || 256 * ld_x * 2 >= (1LL << 32))
     return -1;
   TileArgs a = {(const bf16*)x, (const bf16*)w, bias, S > 1 ? part : nullptr, (bf16*)out, ld_x, M, N, K, S, act, pairs, p0, p1, bias_f32,
-                nullptr, nullptr, 0, 1, 0, M <= kRotateRows};
+                nullptr, nullptr, 0, 1, 0, M <= kRotateRows ? 32 * fn : 0};
   if (gated ? tile_launch_gated(a, fm, fn, cus, st) : tile_launch_size<false>(a, fm, fn, cus, st)) return -1;
   if (S > 1 && out) {   // (without a result the slabs are it: the next kernel adds them)
     const int64_t n = (int64_t)M * (gated ? N / 2 : N) / 4;

@@ -131,6 +131,30 @@ def test_sizes_of_tiles_sum_in_the_same_order(K):
     assert all(torch.equal(y, got[0]) for y in got)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(tl._TILES))
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
+@pytest.mark.parametrize("S", [1, 2, 3])
+def test_columns_begin_where_their_size_says(tile, K, S):
+    """Up to 256 rows column tile n of the size that was asked for takes a part's K tiles from number 37 n on and around, whatever size
+    runs in its place: the bits are those of more rows (which begin at the first) with x's and w's K tiles in that order."""
+    nk, width, N = K // 64, 32 * tile[1], 1544
+    if S > nk:
+        pytest.skip("fewer K tiles than parts")
+    g = torch.Generator("cuda").manual_seed(K + S)
+    x = torch.randn(300, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    got = tl.tile_linear((*tile, S), x[:200], w)
+    for n in range(-(-N // width)):
+        order = []
+        for s in range(S):
+            lo, k = s * nk // S, (s + 1) * nk // S - s * nk // S
+            order += [64 * (lo + (37 * n + i) % k) + e for i in range(k) for e in range(64)]
+        cols = slice(width * n, min(width * (n + 1), N))
+        want = tl.tile_linear((4, 4, S), x[:, order].contiguous(), w[cols, order].contiguous())
+        assert torch.equal(got[:, cols], want[:200])
+
+
 def test_results_of_2_31_bytes_a_wave_are_refused():
     from xgserve.ops._native import mixers
     with pytest.raises(ValueError):
